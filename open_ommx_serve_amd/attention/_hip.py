@@ -1,7 +1,8 @@
-"""ctypes binding of ``libommx_hip.so`` (the C ABI declared in ``include/ommx_hip.h``).
+"""ctypes binding of ``libommx_hip.so`` (the C ABI declared in ``include/ommx_hip.h``), and the
+loader of ``_ommx_host``, the native half of the Python launchers (``csrc/ommx_host.cpp``).
 
-The library is built in-tree by ``open_ommx_serve_amd.csrc.build``.  There is no fallback:
-if it is missing or an entry point fails, the caller gets an exception.
+Both are built in-tree by ``open_ommx_serve_amd.csrc.build``.  There is no fallback: if one is
+missing or an entry point fails, the caller gets an exception.
 """
 from __future__ import annotations
 
@@ -14,6 +15,7 @@ import torch
 _LIB_PATH = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
                          "csrc", "libommx_hip.so")
 _lib: Optional[C.CDLL] = None
+_host_module = None
 
 STORE_TABLE_FLOATS = 264
 ABI_VERSION = 8
@@ -98,6 +100,21 @@ def load() -> C.CDLL:
         raise RuntimeError("libommx_hip.so ABI version mismatch; rebuild it")
     _lib = lib
     return lib
+
+
+def host():
+    """The extension module ``_ommx_host``: each launcher in it returns True when it has launched
+    the call and False when the arguments are not in the form it takes."""
+    global _host_module
+    if _host_module is None:
+        load()                        # its checks (presence, ABI version) come first
+        try:
+            from ..csrc import _ommx_host
+        except ImportError as exc:
+            raise RuntimeError(f"the _ommx_host extension cannot be loaded ({exc}): build it with "
+                               "`python -m open_ommx_serve_amd.csrc.build`") from exc
+        _host_module = _ommx_host
+    return _host_module
 
 
 def exported_symbols():

@@ -22,14 +22,13 @@ import torch
 
 from . import _hip
 
-_CU_COUNT = {}
+_native = None             # the extension module, once the first call has loaded it
 
 
-def _cu_count(device: torch.device) -> int:
-    key = str(device)
-    if key not in _CU_COUNT:
-        _CU_COUNT[key] = int(torch.cuda.get_device_properties(device).multi_processor_count)
-    return _CU_COUNT[key]
+def _load_native():
+    global _native
+    _native = _hip.host()
+    return _native
 
 
 MAX_KV_SPLITS = 512
@@ -51,39 +50,9 @@ def auto_num_kv_splits(max_seq_len: int, batch: int, kv_heads: int, n_cu: int = 
     for the others the count is chosen so that their rounding leaves no split empty.  At most 512,
     the number of partial states the combine kernel keeps on chip.  Splits are whole K groups
     (``group_tokens``), so longer groups mean coarser steps."""
-    wgs_per_split = max(1, int(batch) * max(1, int(kv_heads) // 4))
-    gt = max(32, int(group_tokens))
-    step_tokens = max(64, gt)
-    steps = max(1, (int(max_seq_len) + step_tokens - 1) // step_tokens)
-    groups = max(1, (int(max_seq_len) + gt - 1) // gt)
-    equal = int(batch) == 1 or (mean_seq_len is not None and float(mean_seq_len) >= 0.9 * float(max_seq_len))
-    rounds = 1 if equal else 2
-
-    def count(res: int) -> int:
-        want = max(1, min(MAX_KV_SPLITS, (rounds * res * int(n_cu)) // wgs_per_split))
-        if not equal and int(batch) > 1 and (steps + min(want, steps) - 1) // min(want, steps) > 16:
-            # long splits of requests of different length: four rounds even out better (3-6 % on
-            # 96-128 requests of 1K..16K tokens), the start-up they add is small against 16 steps
-            want = max(1, min(MAX_KV_SPLITS, (4 * res * int(n_cu)) // wgs_per_split))
-        return want
-
-    res = max(1, int(resident))
-    want = count(res)
-    if res >= 3 and steps < 4 * want:
-        # a third resident workgroup pays only while every wave keeps four steps or more: below that
-        # the start-up of the extra waves costs more than their overlap returns (one request of 64K
-        # tokens: 27.7 us with 256 splits of four steps, 28.9 us with 384 of fewer than three)
-        res = 2
-        want = count(res)
-    if want >= 2 * steps:          # plenty of idle units: splits of one K group
-        return int(min(want, groups))
-    if res >= 3:
-        # the kernel deals the groups out evenly whatever the count: fill the chip
-        return int(max(1, min(want, groups)))
-    target = max(1, min(want, steps))
-    # equal whole steps per split, no empty split: the slowest wave sets the kernel's time
-    steps_per_split = (steps + target - 1) // target
-    return int((steps + steps_per_split - 1) // steps_per_split)
+    mean = -1.0 if mean_seq_len is None else float(mean_seq_len)
+    return _hip.host().auto_num_kv_splits(int(max_seq_len), int(batch), int(kv_heads), int(n_cu),
+                                          int(group_tokens), mean, int(resident))
 
 
 def make_attn_logits(batch: int, q_heads: int, num_kv_splits: int, head_dim: int, device) -> torch.Tensor:
@@ -142,6 +111,14 @@ def ommx_paged_decode_attention_canonical(
     f16 operands of the matrix-core kernel cannot carry: the output is finite but off, and
     ``_force_reference_kernel=True`` serves such a cache.
     """
+    if (_native or _load_native()).decode(
+            q, k_base, k_scale, k_zp, k_oidx, k_oval, v_main, v_scale, v_zp, k_tail, v_tail, b_tail_len,
+            o, lse, req_to_token, req_to_group, b_seq_len, sm_scale, page_size, logit_cap,
+            k_outliers_per_vector, k_format, combinadic_read, bitmap_read, k_obmp, k_fp4_mapscale,
+            k_fp4_mapcenter, kv_outlier_map, kv_int8_scale, num_kv_splits, max_seq_len, max_tail_len,
+            attn_logits, packed_start_offset, seg_group_base, _force_reference_kernel, mean_seq_len, err_flag):
+        return
+    # The native launcher has refused: say what is wrong, or bring the arguments into its form.
     pages, ngroups = int(k_base.shape[0]), int(k_scale.shape[0])
     ps = int(page_size)
     if pages == 0 or ngroups == 0:
@@ -270,7 +247,7 @@ def ommx_paged_decode_attention_canonical(
         bitmap_read = to == "bitmap"
         k_obmp, k_oidx = (plane, k_oidx) if bitmap_read else (k_obmp, plane)
     # which index plane the kernels read (paged_decode.py:945-968 bitmap, :843-913 relidx7)
-    k_index, index_repr = (k_obmp, _hip.INDEX_BITMAP) if bitmap_read else (k_oidx, _hip.INDEX_RELIDX7)
+    k_index = k_obmp if bitmap_read else k_oidx
     if k > 0 and (k_index.dtype != torch.uint8 or tuple(k_index.shape[:3]) != tuple(k_scale.shape)
                   or int(k_index.shape[-1]) != ((group_tokens + 7) // 8 if bitmap_read else (7 * k + 7) // 8)):
         raise ValueError("outlier index plane must be u8 [group_slots, Hkv, D, group_tokens/8 (bitmap) "
@@ -300,67 +277,30 @@ def ommx_paged_decode_attention_canonical(
                              f"stride; got {tuple(k_tail.shape)} / {tuple(v_tail.shape)}")
 
     _hip.require_gpu(q.device)
-    if max_seq_len is not None:
-        max_seq = max(1, int(max_seq_len))
-    elif num_kv_splits is None and int(b_seq_len.numel()) > 0:
-        lens = b_seq_len.tolist()                      # the one host sync of this path
-        max_seq = max(1, max(lens))
+    if max_seq_len is None and num_kv_splits is None:
+        lens = b_seq_len.tolist() if int(b_seq_len.numel()) > 0 else [1]   # the one host sync of this path
+        max_seq_len = max(lens)
         if mean_seq_len is None:
             mean_seq_len = sum(lens) / len(lens)
-    else:
-        max_seq = int(b_seq_len.max().item()) if int(b_seq_len.numel()) > 0 else 1
-    # the serving-recipe kernel keeps three workgroups per compute unit resident with up to 4 q heads
-    # per kv head (two with 8, and so do the other kernels); it also serves the call in one launch
-    tuned = D == 128 and Hq // Hkv <= 4 and k == 6
-    general4 = bitmap_read and 1 <= k <= 6 and ((D == 128 and Hq // Hkv <= 4) or      # (7, 8 outliers: two resident)
-                                                (D == 64 and Hq // Hkv <= 2 and Hkv % 2 == 0))
-    lean = ((tuned or general4) and group_tokens == 32 and group_channels == 32
-            and not scale_bf16 and not v_bf16 and not _force_reference_kernel)
-    if num_kv_splits is None:
-        # (at head_dim 64 a wave of that kernel takes a pair of kv heads)
-        paired = D == 64 and bitmap_read and 1 <= k <= 8 and Hq // Hkv <= 4 and Hkv % 2 == 0 and not (
-            scale_bf16 or v_bf16 or _force_reference_kernel) and group_tokens == 32 and group_channels == 32
-        num_kv_splits = auto_num_kv_splits(max_seq, B, Hkv // 2 if paired else Hkv, _cu_count(q.device),
-                                           Hq // Hkv, group_tokens, mean_seq_len, resident=3 if lean else 2)
-    S = max(1, int(num_kv_splits))
-    if attn_logits is None:
-        attn_logits = make_attn_logits(B, Hq, S, D, q.device)
-    else:
+    S = None if num_kv_splits is None else max(1, int(num_kv_splits))
+    if attn_logits is not None:
         if attn_logits.dtype != torch.float32 or attn_logits.dim() != 4 \
-                or tuple(attn_logits.shape[:2]) != (B, Hq) or int(attn_logits.shape[2]) < S \
+                or tuple(attn_logits.shape[:2]) != (B, Hq) or int(attn_logits.shape[2]) < (S or 1) \
                 or int(attn_logits.shape[3]) < D + 1 or attn_logits.stride(-1) != 1:
-            raise ValueError(f"attn_logits must be fp32 [B={B}, Hq={Hq}, >= {S}, >= {D + 1}] "
+            raise ValueError(f"attn_logits must be fp32 [B={B}, Hq={Hq}, >= {S or 'splits'}, >= {D + 1}] "
                              f"with unit inner stride; got {tuple(attn_logits.shape)}")
     if err_flag is not None and (err_flag.dtype != torch.int32 or err_flag.device != q.device):
         raise ValueError("err_flag must be an int32 tensor on the device of q")
-    lib = _hip.load()
-    stream = _hip.current_stream_ptr(q.device)
-    splitkv = lib.ommx_decode_splitkv_ref if _force_reference_kernel else lib.ommx_decode_splitkv
-    tail_args = ((k_tail.data_ptr(), v_tail.data_ptr(), k_tail.stride(0), k_tail.stride(1), k_tail.stride(2),
-                  v_tail.stride(0), v_tail.stride(1), v_tail.stride(2), b_tail_len.data_ptr())
-                 if has_tail else (None, None, 0, 0, 0, 0, 0, 0, None))
-    planes = (k_base.data_ptr(), k_scale.data_ptr(), k_zp.data_ptr(),
-              _hip.ptr(k_fp4_mapscale) if use_map else None, _hip.ptr(k_fp4_mapcenter) if use_map else None,
-              _hip.ptr(k_index) if k > 0 else None, _hip.ptr(k_oval) if k > 0 else None,
-              v_main.data_ptr(), v_scale.data_ptr(), v_zp.data_ptr(),
-              req_to_token.data_ptr(), req_to_token.stride(0),
-              req_to_group.data_ptr(), req_to_group.stride(0),
-              1 if req_to_token.dtype == torch.int64 else 0,
-              b_seq_len.data_ptr(),
-              attn_logits.data_ptr(), attn_logits.stride(0), attn_logits.stride(1), attn_logits.stride(2))
-    shape = (B, Hq, Hkv, D, ps, k, index_repr, 1 if scale_bf16 else 0, group_tokens, group_channels,
-             1 if v_bf16 else 0, S, float(sm_scale), float(logit_cap), off, gbase,
-             pages, ngroups, _hip.ptr(err_flag), stream)
-    with torch.cuda.device(q.device):
-        rc = splitkv(q.data_ptr(), q.stride(0), q.stride(1), *planes, *shape)
-        _hip.check(rc, "ommx_decode_splitkv")
-        rc = lib.ommx_decode_combine(
-            attn_logits.data_ptr(), attn_logits.stride(0), attn_logits.stride(1), attn_logits.stride(2),
-            q.data_ptr(), q.stride(0), q.stride(1), *tail_args[:8], tail_args[8], b_seq_len.data_ptr(),
-            o.data_ptr(), o.stride(0), o.stride(1), lse.data_ptr(), lse.stride(0),
-            B, Hq, Hkv, D, S, group_tokens, int(k_tail.shape[1]) if has_tail else 0,
-            float(sm_scale), float(logit_cap), stream)
-        _hip.check(rc, "ommx_decode_combine")
+    if not _native.decode(
+            q, k_base, k_scale, k_zp, k_oidx, k_oval, v_main, v_scale, v_zp, k_tail, v_tail, b_tail_len,
+            o, lse, req_to_token, req_to_group, b_seq_len, float(sm_scale), ps, float(logit_cap), k, kfmt,
+            False, bool(bitmap_read), k_obmp, k_fp4_mapscale, k_fp4_mapcenter, use_map, bool(kv_int8_scale),
+            S, None if max_seq_len is None else int(max_seq_len),
+            None if max_tail_len is None else int(max_tail_len), attn_logits, off, gbase,
+            bool(_force_reference_kernel), None if mean_seq_len is None else float(mean_seq_len), err_flag):
+        raise ValueError("the decode launcher refused these arguments"
+                         + (f": attn_logits {tuple(attn_logits.shape)} is too small for the split count"
+                            if attn_logits is not None else ""))
 
 
 def merge_attention_states(o_parts: torch.Tensor, lse_parts: torch.Tensor, *, valid_lens=None,
