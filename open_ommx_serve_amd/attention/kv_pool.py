@@ -30,7 +30,7 @@ import torch
 from . import _hip
 from .kv_store_ops import gather_tails, ring_slot, write_tokens
 from .kv_window import CANONICAL_GROUP_TOKENS, WindowSpec
-from .pack import index_plane_bytes, raise_for_store_errors, store_pack_into
+from .pack import index_plane_bytes, raise_for_store_errors, store_pack_into, store_table
 
 _FALSE = {"0", "false", "off", "no"}
 
@@ -200,17 +200,21 @@ class MultiSeqKVPool:
         self.wide_steps = False      # a packed K step above 2^15 was seen: decode on the plain kernel
         self._dbuf: Optional[Dict[str, object]] = None
         self._planes_cache: Optional[dict] = None
+        self._host = _hip.host()
+        # what every store launch of this pool is told (argument order of the native launchers)
+        self._recipe = (self.k, self.gt, self.gc, self.outlier_repr, self.outlier_select, self.use_pow2,
+                        self.kv_int8_scale, "i2")
+        self._store_planes = {
+            "k_base": self.k_base, "k_scale": self.k_scale, "k_zp": self.k_zp,
+            "k_fp4_mapscale": self.k_fp4_mapscale, "k_fp4_mapcenter": self.k_fp4_mapcenter,
+            "k_obmp": self.k_obmp, "k_oidx": self.k_oidx, "k_oval": self.k_oval, "k_crank": self.k_crank,
+            "_k_obmp_scratch": self.k_obmp if self.outlier_repr == "combinadic" else None,
+            "v_main": self.v_main, "v_scale": self.v_scale, "v_zp": self.v_zp}
 
     # ── ring address mapping ───────────────────────────────────────────────────────
 
     def _ring_slot_host(self, pos: int) -> int:
         return ring_slot(pos, self._ring_sink, self._ring_rec) if self.kv_ring else int(pos)
-
-    def _ring_slot_dev(self, pos: torch.Tensor) -> torch.Tensor:
-        if not self.kv_ring:
-            return pos
-        rel = (pos - self._ring_sink) % self._ring_rec + self._ring_sink
-        return torch.where(pos < self._ring_sink, pos, rel)
 
     def check_errors(self) -> None:
         """Read the device error bits (host sync) and raise what the reference would have."""
@@ -241,14 +245,6 @@ class MultiSeqKVPool:
 
     # ── write path ───────────────────────────────────────────────────────────────
 
-    def _planes_for_store(self) -> dict:
-        return {"k_base": self.k_base, "k_scale": self.k_scale, "k_zp": self.k_zp,
-                "k_fp4_mapscale": self.k_fp4_mapscale, "k_fp4_mapcenter": self.k_fp4_mapcenter,
-                "k_obmp": self.k_obmp, "k_oidx": self.k_oidx, "k_oval": self.k_oval,
-                "k_crank": self.k_crank,
-                "_k_obmp_scratch": self.k_obmp if self.outlier_repr == "combinadic" else None,
-                "v_main": self.v_main, "v_scale": self.v_scale, "v_zp": self.v_zp}
-
     def _as_rows(self, t: torch.Tensor, what: str) -> torch.Tensor:
         if t.device != self.device:
             t = t.to(self.device)
@@ -270,8 +266,7 @@ class MultiSeqKVPool:
         if not self.kv_ring:
             if s + T > self.max_seq_len:
                 raise RuntimeError(f"MultiSeqKVPool req {r} capacity {self.max_seq_len} exceeded")
-            self.k_hist[r, s:s + T] = K.to(torch.bfloat16)
-            self.v_hist[r, s:s + T] = V.to(torch.bfloat16)
+            self._write_rows(r, K, V, s, 0, 0)
             self.seq_len[r] = s + T
             return self.regroup(r)
         if s != 0:
@@ -279,26 +274,29 @@ class MultiSeqKVPool:
                 f"ring append_block expects a fresh request slot (seq_len==0); chunked prefill "
                 f"under the ring is unsupported (it cannot retain unpacked rows across chunks). "
                 f"Reset pool slot {r} before each prefill block.")
-        Kb, Vb = K.to(torch.bfloat16), V.to(torch.bfloat16)
+        K, V = K.to(torch.bfloat16), V.to(torch.bfloat16)
         self.seq_len[r] = T
         target = self.window.num_groups(T)
+        sink = self.window.sink_tokens
         if target > 0:
-            sink = self.window.sink_tokens
-            self._pack_block_into_pool(r, Kb[sink:sink + target * self.gt],
-                                       Vb[sink:sink + target * self.gt], 0, target)
+            self._pack_block_into_pool(r, K, V, 0, target, row0=sink)
             self.packed_groups[r] = target
         # only the live rows enter the ring: sink, and [boundary - gt, T)
-        boundary = self.window.boundary(T)
-        sink_tokens = self.window.sink_tokens
-        lo = max(sink_tokens, boundary - self.gt)
-        parts = [torch.arange(0, min(sink_tokens, T), device=self.device)]
-        if lo < T:
-            parts.append(torch.arange(lo, T, device=self.device))
-        live = torch.cat(parts).to(torch.long)
-        slots = self._ring_slot_dev(live)
-        self.k_hist[r].index_copy_(0, slots, Kb.index_select(0, live))
-        self.v_hist[r].index_copy_(0, slots, Vb.index_select(0, live))
+        lo = max(sink, self.window.boundary(T) - self.gt)
+        self._write_rows(r, K, V, 0, min(sink, T), min(lo, T))
         return target
+
+    def _write_rows(self, req: int, K: torch.Tensor, V: torch.Tensor, pos0: int, n_head: int, lo: int) -> None:
+        """Rows ``[0, n_head)`` and ``[lo, T)`` of a block into request ``req``'s history at their ring
+        slots (the block starts at absolute position ``pos0``), one launch."""
+        if K.stride(-1) != 1:
+            K = K.contiguous()
+        if V.stride(-1) != 1:
+            V = V.contiguous()
+        if not self._host.rows_write(K, V, self.k_hist, self.v_hist, req, pos0, n_head, lo, self._ring_sink,
+                                     self._ring_rec):
+            raise ValueError(f"K / V rows {tuple(K.shape)} / {tuple(V.shape)} do not fit the history of request "
+                             f"{req} at position {pos0}")
 
     def append(self, req: int, k: torch.Tensor, v: torch.Tensor) -> int:
         """One decode step's K/V row ``[H, D]`` for request ``req`` (kv_pool.py:370-381)."""
@@ -306,9 +304,8 @@ class MultiSeqKVPool:
         s = self.seq_len[r]
         if not self.kv_ring and s >= self.max_seq_len:
             raise RuntimeError(f"MultiSeqKVPool req {r} capacity {self.max_seq_len} exceeded")
-        slot = self._ring_slot_host(s)
-        self.k_hist[r, slot] = k.reshape(self.H, self.D).to(self.device, torch.bfloat16)
-        self.v_hist[r, slot] = v.reshape(self.H, self.D).to(self.device, torch.bfloat16)
+        self._write_rows(r, self._as_rows(k.reshape(1, self.H, self.D), "k"),
+                         self._as_rows(v.reshape(1, self.H, self.D), "v"), s, 0, 0)
         self.seq_len[r] = s + 1
         return self.regroup(r)
 
@@ -317,6 +314,13 @@ class MultiSeqKVPool:
         if t.dtype != torch.bfloat16 or t.device != self.device:
             t = t.to(self.device, torch.bfloat16)
         return t if t.stride(-1) == 1 else t.contiguous()
+
+    def _upload(self, *rows: List[int]) -> torch.Tensor:
+        """int64 ``[len(rows), n]`` on the device, filled by a launch that carries the numbers."""
+        out = torch.empty(len(rows), len(rows[0]), dtype=torch.int64, device=self.device)
+        if not self._host.upload(out, [x for row in rows for x in row]):
+            raise ValueError("pool slots and lengths must be ints")
+        return out
 
     def _advance_host_and_pack(self, slots: Sequence[int]) -> int:
         pend: List[Tuple[int, int, int]] = []
@@ -343,8 +347,7 @@ class MultiSeqKVPool:
         for r in slots:
             if not self.kv_ring and self.seq_len[r] >= self.max_seq_len:
                 raise RuntimeError(f"MultiSeqKVPool req {r} capacity {self.max_seq_len} exceeded")
-        meta = torch.tensor([slots, [self.seq_len[r] for r in slots]], dtype=torch.int64).to(
-            self.device, non_blocking=True)
+        meta = self._upload(slots, [self.seq_len[r] for r in slots])
         write_tokens(self.k_hist, self.v_hist, meta[1], self._bf16_batch(K, B), self._bf16_batch(V, B),
                      self._ring_sink, self._ring_rec, slots=meta[0], err_flag=self.err_flag)
         return self._advance_host_and_pack(slots)
@@ -374,6 +377,12 @@ class MultiSeqKVPool:
         The launch reads the source rows in place (``src_rows`` = flat history rows through
         the ring map) and writes to each request's own page / group slots.
         """
+        pairs = [x for (r, g0, g1) in pend for g in range(g0, g1) for x in (r, g)]
+        if self._host.pack_groups(self.k_hist, self.v_hist, self._store_planes, pairs, self.ps, self._ring_sink,
+                                  self._ring_rec, self.window.sink_tokens, self.G_per_seq, self.err_flag,
+                                  store_table(self.k_hist.device), *self._recipe):
+            return
+        # ranks instead of positions: the index lists go through the general entry
         gt, ppg, sink = self.gt, self.pages_per_group, self.window.sink_tokens
         src: List[int] = []
         pages: List[int] = []
@@ -387,14 +396,15 @@ class MultiSeqKVPool:
                 pages.extend(r * self.P_per_seq + g * ppg + i for i in range(ppg))
         idx = torch.tensor(src + pages + groups, dtype=torch.int32).to(self.device, non_blocking=True)
         n_s, n_p = len(src), len(pages)
-        flat_k = self.k_hist.view(self.num_seqs * self.S_ring, self.H, self.D)
-        flat_v = self.v_hist.view(self.num_seqs * self.S_ring, self.H, self.D)
-        store_pack_into(flat_k, flat_v, self._planes_for_store(), outliers_per_vector=self.k,
+        self._store(self.k_hist.view(-1, self.H, self.D), self.v_hist.view(-1, self.H, self.D), n_s,
+                    src_rows=idx[:n_s], dst_pages=idx[n_s:n_s + n_p], dst_groups=idx[n_s + n_p:])
+
+    def _store(self, K: torch.Tensor, V: torch.Tensor, num_tokens: int, **tables) -> None:
+        store_pack_into(K, V, self._store_planes, outliers_per_vector=self.k,
                         outlier_repr=self.outlier_repr, outlier_select=self.outlier_select,
                         use_pow2=self.use_pow2, kv_int8_scale=self.kv_int8_scale,
-                        group_tokens=self.gt, group_channels=self.gc,
-                        page_size=self.ps, src_rows=idx[:n_s], dst_pages=idx[n_s:n_s + n_p],
-                        dst_groups=idx[n_s + n_p:], err_flag=self.err_flag, num_tokens=n_s)
+                        group_tokens=self.gt, group_channels=self.gc, page_size=self.ps,
+                        err_flag=self.err_flag, num_tokens=num_tokens, **tables)
 
     def regroup(self, req: int) -> int:
         """Pack request ``req``'s newly completed groups (kv_pool.py:637-652)."""
@@ -412,28 +422,26 @@ class MultiSeqKVPool:
         if self.kv_ring:
             self._regroup_pack_batched_device([(r, g0, g1)])
             return
-        sink = self.window.sink_tokens
-        t0, t1 = sink + g0 * self.gt, sink + g1 * self.gt
-        self._pack_block_into_pool(r, self.k_hist[r, t0:t1], self.v_hist[r, t0:t1], g0, g1)
+        self._pack_block_into_pool(r, self.k_hist[r], self.v_hist[r], g0, g1,
+                                   row0=self.window.sink_tokens + g0 * self.gt)
 
-    def _pack_block_into_pool(self, req: int, K_blk: torch.Tensor, V_blk: torch.Tensor,
-                              g0: int, g1: int) -> None:
-        """Pack a source block of exactly ``(g1-g0)*gt`` tokens into request ``req``'s group /
+    def _pack_block_into_pool(self, req: int, K: torch.Tensor, V: torch.Tensor, g0: int, g1: int,
+                              row0: int = 0) -> None:
+        """Pack the ``(g1-g0)*gt`` tokens from row ``row0`` of a source block into request ``req``'s group /
         page slots ``[g0, g1)`` with one store launch (kv_pool.py:677-734)."""
         r = int(req)
         n_tok = (g1 - g0) * self.gt
-        if int(K_blk.shape[0]) != n_tok or int(V_blk.shape[0]) != n_tok:
-            raise ValueError(f"source block must hold {n_tok} tokens; got {int(K_blk.shape[0])}")
+        if row0 + n_tok > int(K.shape[0]) or row0 + n_tok > int(V.shape[0]):
+            raise ValueError(f"source block must hold {n_tok} tokens from row {row0}; got {int(K.shape[0])}")
         gp0 = r * self.G_per_seq + g0
         pp0 = r * self.P_per_seq + g0 * self.pages_per_group
-        store_pack_into(K_blk, V_blk, self._planes_for_store(), outliers_per_vector=self.k,
-                        outlier_repr=self.outlier_repr, outlier_select=self.outlier_select,
-                        use_pow2=self.use_pow2, kv_int8_scale=self.kv_int8_scale,
-                        group_tokens=self.gt, group_channels=self.gc,
-                        page_size=self.ps,
-                        dst_pages=self._req_to_token.view(-1)[pp0:pp0 + (g1 - g0) * self.pages_per_group],
-                        dst_groups=self._req_to_group.view(-1)[gp0:gp0 + (g1 - g0)],
-                        err_flag=self.err_flag)
+        if self._host.store_pack(K, V, self._store_planes, self.ps, None, self._req_to_token, self._req_to_group,
+                                 self.err_flag, n_tok, store_table(K.device), row0, pp0, gp0, *self._recipe):
+            return
+        rows = slice(row0, row0 + n_tok)
+        self._store(K[rows], V[rows], n_tok,
+                    dst_pages=self._req_to_token.view(-1)[pp0:pp0 + (g1 - g0) * self.pages_per_group],
+                    dst_groups=self._req_to_group.view(-1)[gp0:gp0 + (g1 - g0)])
 
     # ── read path ────────────────────────────────────────────────────────────────
 
@@ -503,7 +511,7 @@ class MultiSeqKVPool:
         vt = torch.empty_like(kt)
         b_tail = torch.zeros(B, dtype=torch.int32, device=dev)
         if B:
-            meta = torch.tensor([slots, [self.seq_len[r] for r in slots]], dtype=torch.int64).to(dev)
+            meta = self._upload(slots, [self.seq_len[r] for r in slots])
             self._gather(kt, vt, seq=meta[1], slots=meta[0], b_tail=b_tail)
         return kt, vt, b_tail
 
@@ -576,8 +584,7 @@ class MultiSeqKVPool:
         slots = [int(s) for s in slots]
         B = len(slots)
         d = self._decode_buffers(B)
-        meta = torch.tensor([slots, [self.seq_len[r] for r in slots]], dtype=torch.int64).to(
-            self.device, non_blocking=True)
+        meta = self._upload(slots, [self.seq_len[r] for r in slots])
         d["sel"].copy_(meta[0])
         self._gather(d["kt"], d["vt"], seq=meta[1], slots=d["sel"], b_tail=d["b_tail"], b_seq=d["b_seq"])
         max_pg = max([self.packed_groups[r] for r in slots], default=0)
@@ -591,8 +598,7 @@ class MultiSeqKVPool:
         slots = [int(s) for s in slots]
         B = len(slots)
         d = self._decode_buffers(B)
-        meta = torch.tensor([slots, [self.seq_len[r] for r in slots]], dtype=torch.int64).to(
-            self.device, non_blocking=True)
+        meta = self._upload(slots, [self.seq_len[r] for r in slots])
         d["rows"].copy_(meta[0])
         d["sel"].copy_(meta[0])
         d["seq_dev"].copy_(meta[1])

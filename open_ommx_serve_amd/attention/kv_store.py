@@ -21,7 +21,7 @@ from . import _hip
 from .kv_pool import _env_flag, check_serving_recipe
 from .kv_store_ops import gather_tail, ring_slot, write_token
 from .kv_window import CANONICAL_GROUP_TOKENS, WindowSpec
-from .pack import index_plane_bytes, raise_for_store_errors, store_pack_into
+from .pack import index_plane_bytes, raise_for_store_errors, store_pack_into, store_table
 
 
 class CanonicalKVStore:
@@ -146,17 +146,21 @@ class CanonicalKVStore:
         self.v_tail_buf = z(1, self.tail_cap, self.H, self.D, dtype=bf, device=dev)
         self.err_flag = torch.zeros(1, dtype=torch.int32, device=dev)
         self.wide_steps = False      # a packed K step above 2^15 was seen: decode on the plain kernel
+        self._host = _hip.host()
+        # what every store launch of this cache is told (argument order of the native launchers)
+        self._recipe = (self.k, self.gt, self.gc, self.outlier_repr, self.outlier_select, self.use_pow2,
+                        self.kv_int8_scale, self.v_format)
+        self._store_planes = {
+            "k_base": self.k_base, "k_scale": self.k_scale, "k_zp": self.k_zp,
+            "k_fp4_mapscale": self.k_fp4_mapscale, "k_fp4_mapcenter": self.k_fp4_mapcenter,
+            "k_obmp": self.k_obmp, "k_oidx": self.k_oidx, "k_oval": self.k_oval, "k_crank": self.k_crank,
+            "_k_obmp_scratch": self.k_obmp if self.outlier_repr == "combinadic" else None,
+            "v_main": self.v_main, "v_scale": self.v_scale, "v_zp": self.v_zp}
 
     # ── ring address mapping (kv_store.py:301-327) ────────────────────────────────────
 
     def _ring_slot_host(self, pos: int) -> int:
         return ring_slot(pos, self._ring_sink, self._ring_rec) if self.kv_ring else int(pos)
-
-    def _ring_slot_dev(self, pos: torch.Tensor) -> torch.Tensor:
-        if not self.kv_ring:
-            return pos
-        rel = (pos - self._ring_sink) % self._ring_rec + self._ring_sink
-        return torch.where(pos < self._ring_sink, pos, rel)
 
     def check_errors(self) -> None:
         """Read the device error bits (host sync) and raise what the reference would have."""
@@ -193,9 +197,7 @@ class CanonicalKVStore:
         """Stash one decode step's K/V row ``[H, D]`` (kv_store.py:349-357)."""
         if not self.kv_ring and self.seq_len >= self.kv_cap:
             raise RuntimeError(f"CanonicalKVStore capacity {self.kv_cap} exceeded (seq_len)")
-        slot = self._ring_slot_host(self.seq_len)
-        self.k_hist[slot] = k.reshape(self.H, self.D).to(self.device, torch.bfloat16)
-        self.v_hist[slot] = v.reshape(self.H, self.D).to(self.device, torch.bfloat16)
+        self._write_rows(k.reshape(1, self.H, self.D), v.reshape(1, self.H, self.D), self.seq_len, 0, 0)
         self.seq_len += 1
 
     def write_token(self, pos: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> None:
@@ -233,13 +235,10 @@ class CanonicalKVStore:
     def append_block(self, K: torch.Tensor, V: torch.Tensor) -> None:
         """Stash a prefill block ``[T, H, D]`` and pack its completed groups (kv_store.py:429-490)."""
         T = int(K.shape[0])
-        Kb = K.to(self.device, torch.bfloat16)
-        Vb = V.to(self.device, torch.bfloat16)
         if not self.kv_ring:
             if self.seq_len + T > self.kv_cap:
                 raise RuntimeError("CanonicalKVStore capacity exceeded (block)")
-            self.k_hist[self.seq_len:self.seq_len + T] = Kb
-            self.v_hist[self.seq_len:self.seq_len + T] = Vb
+            self._write_rows(K, V, self.seq_len, 0, 0)
             self.seq_len += T
             self.maybe_regroup()
             return
@@ -247,23 +246,25 @@ class CanonicalKVStore:
             raise RuntimeError(
                 "ring append_block expects a fresh sequence (seq_len==0); chunked prefill under "
                 "the ring is not supported. Reset the store before each prefill block.")
+        K, V = K.to(self.device, torch.bfloat16), V.to(self.device, torch.bfloat16)
         self.seq_len = T
         target = self.window.num_groups(T)
+        sink = self.window.sink_tokens
         if target > 0:
-            sink = self.window.sink_tokens
-            self._pack_block_into_planes(Kb[sink:sink + target * self.gt],
-                                         Vb[sink:sink + target * self.gt], 0, target)
+            self._pack_block_into_planes(K, V, 0, target, row0=sink)
             self.packed_groups = target
-        boundary = self.window.boundary(T)
-        sink_tokens = self.window.sink_tokens
-        lo = max(sink_tokens, boundary - self.gt)
-        parts = [torch.arange(0, min(sink_tokens, T), device=self.device)]
-        if lo < T:
-            parts.append(torch.arange(lo, T, device=self.device))
-        live = torch.cat(parts).to(torch.long)
-        slots = self._ring_slot_dev(live)
-        self.k_hist.index_copy_(0, slots, Kb.index_select(0, live))
-        self.v_hist.index_copy_(0, slots, Vb.index_select(0, live))
+        lo = max(sink, self.window.boundary(T) - self.gt)
+        self._write_rows(K, V, 0, min(sink, T), min(lo, T))
+
+    def _write_rows(self, K: torch.Tensor, V: torch.Tensor, pos0: int, n_head: int, lo: int) -> None:
+        """Rows ``[0, n_head)`` and ``[lo, T)`` of a block into the history at their ring slots (the block
+        starts at absolute position ``pos0``), one launch."""
+        K, V = (t if t.dtype == torch.float32 and t.device == self.device else t.to(self.device, torch.bfloat16)
+                for t in (K, V))
+        K, V = (t if t.stride(-1) == 1 else t.contiguous() for t in (K, V))
+        if not self._host.rows_write(K, V, self.k_hist.unsqueeze(0), self.v_hist.unsqueeze(0), 0, pos0, n_head, lo,
+                                     self._ring_sink, self._ring_rec):
+            raise ValueError(f"K / V rows {tuple(K.shape)} / {tuple(V.shape)} do not fit the history at position {pos0}")
 
     def maybe_regroup(self) -> int:
         """Pack any newly completed groups; returns how many (kv_store.py:492-526)."""
@@ -279,31 +280,33 @@ class CanonicalKVStore:
         self.packed_groups = target
         return n
 
-    def _planes_for_store(self) -> dict:
-        return {"k_base": self.k_base, "k_scale": self.k_scale, "k_zp": self.k_zp,
-                "k_fp4_mapscale": self.k_fp4_mapscale, "k_fp4_mapcenter": self.k_fp4_mapcenter,
-                "k_obmp": self.k_obmp, "k_oidx": self.k_oidx, "k_oval": self.k_oval,
-                "k_crank": self.k_crank,
-                "_k_obmp_scratch": self.k_obmp if self.outlier_repr == "combinadic" else None,
-                "v_main": self.v_main, "v_scale": self.v_scale, "v_zp": self.v_zp}
-
     def _regroup_pack_range(self, g0: int, g1: int) -> None:
-        sink = self.window.sink_tokens
-        t0, t1 = sink + g0 * self.gt, sink + g1 * self.gt
-        if self.kv_ring:
-            rows = torch.tensor([self._ring_slot_host(t) for t in range(t0, t1)], dtype=torch.int32).to(
-                self.device, non_blocking=True)
-            self._pack_block_into_planes(self.k_hist, self.v_hist, g0, g1, src_rows=rows)
-        else:
-            self._pack_block_into_planes(self.k_hist[t0:t1], self.v_hist[t0:t1], g0, g1)
+        row0 = self.window.sink_tokens + g0 * self.gt
+        if not self.kv_ring:
+            self._pack_block_into_planes(self.k_hist, self.v_hist, g0, g1, row0=row0)
+            return
+        pairs = [x for g in range(g0, g1) for x in (0, g)]
+        if self._host.pack_groups(self.k_hist.unsqueeze(0), self.v_hist.unsqueeze(0), self._store_planes, pairs,
+                                  self.ps, self._ring_sink, self._ring_rec, self.window.sink_tokens, self.G_cap,
+                                  self.err_flag, store_table(self.k_hist.device), *self._recipe):
+            return
+        rows = torch.tensor([self._ring_slot_host(t) for t in range(row0, row0 + (g1 - g0) * self.gt)],
+                            dtype=torch.int32).to(self.device, non_blocking=True)
+        self._pack_block_into_planes(self.k_hist, self.v_hist, g0, g1, src_rows=rows)
 
-    def _pack_block_into_planes(self, K_blk: torch.Tensor, V_blk: torch.Tensor, g0: int, g1: int,
+    def _pack_block_into_planes(self, K: torch.Tensor, V: torch.Tensor, g0: int, g1: int, *, row0: int = 0,
                                 src_rows: Optional[torch.Tensor] = None) -> None:
-        """Pack ``(g1-g0)*gt`` tokens into group slots ``[g0, g1)`` with one store launch
-        (kv_store.py:551-610)."""
+        """Pack ``(g1-g0)*gt`` tokens (rows from ``row0`` on, or ``src_rows``) into group slots ``[g0, g1)``
+        with one store launch (kv_store.py:551-610)."""
         n_tok = (g1 - g0) * self.gt
         ppg = self.pages_per_group
-        store_pack_into(K_blk, V_blk, self._planes_for_store(), outliers_per_vector=self.k,
+        if self._host.store_pack(K, V, self._store_planes, self.ps, src_rows, self._req_to_token_full,
+                                 self._req_to_group_full, self.err_flag, n_tok, store_table(K.device), row0,
+                                 g0 * ppg, g0, *self._recipe):
+            return
+        if src_rows is None:
+            K, V = K[row0:row0 + n_tok], V[row0:row0 + n_tok]
+        store_pack_into(K, V, self._store_planes, outliers_per_vector=self.k,
                         outlier_repr=self.outlier_repr, outlier_select=self.outlier_select,
                         use_pow2=self.use_pow2, kv_int8_scale=self.kv_int8_scale,
                         group_tokens=self.gt, group_channels=self.gc, v_format=self.v_format,

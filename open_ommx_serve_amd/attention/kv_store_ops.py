@@ -47,6 +47,9 @@ def write_tokens(k_hist: torch.Tensor, v_hist: torch.Tensor, pos: torch.Tensor, 
     (last dim contiguous); ``pos``: int64 ``[B]`` on the device; ``recent`` is the sliding span
     of the ring (0: whole history).  ``pos_next`` (may be ``pos``) receives ``pos + 1``.
     """
+    if _hip.host().ring_write(k_hist, v_hist, pos, k, v, sink, recent, slots, pos_next, err_flag):
+        return
+    # the native launcher has refused: say what is wrong, or bring the arguments into its form
     _check_hist(k_hist, v_hist)
     if k_hist.dim() != 4:
         raise ValueError("k_hist must be [num_slots, rows, H, D]")
@@ -65,13 +68,8 @@ def write_tokens(k_hist: torch.Tensor, v_hist: torch.Tensor, pos: torch.Tensor, 
     if slots is None and B > N:
         raise ValueError(f"{B} requests but only {N} history slots")
     _hip.require_gpu(dev)
-    lib = _hip.load()
-    _hip.check(lib.ommx_ring_write(
-        k.data_ptr(), v.data_ptr(), k.stride(0), k.stride(1), v.stride(0), v.stride(1),
-        k_hist.data_ptr(), v_hist.data_ptr(), k_hist.stride(0), rows,
-        _hip.ptr(slots), pos.data_ptr(), _hip.ptr(pos_next),
-        B, H, D, int(sink), int(recent), _hip.ptr(err_flag), _hip.current_stream_ptr(dev)),
-        "ommx_ring_write")
+    if not _hip.host().ring_write(k_hist, v_hist, pos, k, v, int(sink), int(recent), slots, pos_next, err_flag):
+        raise ValueError("the ring-write launcher refused these arguments")
 
 
 def write_token(k_hist: torch.Tensor, v_hist: torch.Tensor, pos: torch.Tensor, k: torch.Tensor,
@@ -104,6 +102,11 @@ def gather_tails(k_hist: torch.Tensor, v_hist: torch.Tensor, k_tail: torch.Tenso
     step that appends and decodes before the host packs passes 1: the boundary is then the one
     the host has packed for, and the rows since come from the ring.
     """
+    wsink = sink if window_sink is None else window_sink
+    if _hip.host().tail_gather(k_hist, v_hist, k_tail, v_tail, recent_span, seq, tail_idx, slots, b_tail_len,
+                               b_seq_len, wsink, window_recent, group_tokens, packed_lag, err_flag):
+        return
+    # the native launcher has refused: say what is wrong, or bring the arguments into its form
     _check_hist(k_hist, v_hist)
     if k_hist.dim() != 4:
         raise ValueError("k_hist must be [num_slots, rows, H, D]")
@@ -128,14 +131,10 @@ def gather_tails(k_hist: torch.Tensor, v_hist: torch.Tensor, k_tail: torch.Tenso
     if slots is None and B > N:
         raise ValueError(f"{B} requests but only {N} history slots")
     _hip.require_gpu(dev)
-    lib = _hip.load()
-    wsink = int(sink if window_sink is None else window_sink)
-    _hip.check(lib.ommx_tail_gather(
-        k_hist.data_ptr(), v_hist.data_ptr(), k_hist.stride(0), rows,
-        _hip.ptr(slots), _hip.ptr(seq), _hip.ptr(tail_idx),
-        k_tail.data_ptr(), v_tail.data_ptr(), _hip.ptr(b_tail_len), _hip.ptr(b_seq_len),
-        B, T, H, D, wsink, int(window_recent), int(group_tokens), int(recent_span),
-        int(packed_lag), _hip.ptr(err_flag), _hip.current_stream_ptr(dev)), "ommx_tail_gather")
+    if not _hip.host().tail_gather(k_hist, v_hist, k_tail, v_tail, int(recent_span), seq, tail_idx, slots,
+                                   b_tail_len, b_seq_len, int(wsink), int(window_recent), int(group_tokens),
+                                   int(packed_lag), err_flag):
+        raise ValueError("the tail-gather launcher refused these arguments")
 
 
 def gather_tail(k_hist: torch.Tensor, v_hist: torch.Tensor, indices: torch.Tensor,

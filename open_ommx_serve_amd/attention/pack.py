@@ -25,7 +25,7 @@ OUTLIER_REPRS = ("relidx7", "combinadic", "bitmap")
 
 _FP4_MAGNITUDES = (0.0, 0.5, 1.0, 1.5, 2.0, 3.0, 4.0, 6.0)
 _table_host: Optional[torch.Tensor] = None
-_table_dev: Dict[str, torch.Tensor] = {}
+_table_dev: Dict[torch.device, torch.Tensor] = {}
 
 
 # -- decision tables ----------------------------------------------------------------------
@@ -83,16 +83,18 @@ def measure_store_table() -> torch.Tensor:
 
 def store_table(device: torch.device) -> torch.Tensor:
     """Device copy of the decision table (measured once per process, cached per device)."""
+    known = _table_dev.get(device)
+    if known is not None:
+        return known
     global _table_host
     if _table_host is None:
         _table_host = measure_store_table()
     device = torch.device(device)
     if device.type == "cuda" and device.index is None:
         device = torch.device("cuda", torch.cuda.current_device())
-    key = str(device)
-    if key not in _table_dev:
-        _table_dev[key] = _table_host.to(device)    # first use on a device uploads (not capturable)
-    return _table_dev[key]
+    if device not in _table_dev:
+        _table_dev[device] = _table_host.to(device)    # first use on a device uploads (not capturable)
+    return _table_dev[device]
 
 
 # -- launch -------------------------------------------------------------------------------
@@ -126,6 +128,13 @@ def store_pack_into(K: torch.Tensor, V: torch.Tensor, planes: Dict[str, Any], *,
     can afford to.  Launches on the current stream.  ``outlier_repr`` names the index plane
     that is written: ``planes["k_obmp"]`` (``"bitmap"``) or ``planes["k_oidx"]`` (``"relidx7"``).
     """
+    if K.is_cuda and _hip.host().store_pack(
+            K, V, planes, page_size, src_rows, dst_pages, dst_groups, err_flag, num_tokens, store_table(K.device),
+            0, 0, 0, outliers_per_vector, group_tokens, group_channels, outlier_repr, outlier_select, use_pow2,
+            kv_int8_scale, v_format):
+        return
+    # The native launcher has refused: say what is wrong, bring the arguments into its form, or take the
+    # combinadic way (bitmask first, ranks from it).
     _check_rows("K", K)
     _check_rows("V", V)
     if K.dtype != V.dtype or K.device != V.device:
@@ -165,19 +174,13 @@ def store_pack_into(K: torch.Tensor, V: torch.Tensor, planes: Dict[str, Any], *,
     want_dt = torch.int8 if mode == _hip.SCALE_POW2_INT8 else torch.bfloat16
     if planes["k_scale"].dtype != want_dt or planes["v_scale"].dtype != want_dt:
         raise ValueError(f"k_scale / v_scale planes must be {want_dt} for this recipe")
-    lib = _hip.load()
-    with torch.cuda.device(K.device):
-        rc = lib.ommx_store_pack(
-            K.data_ptr(), V.data_ptr(), 1 if K.dtype == torch.float32 else 0,
-            K.stride(0), K.stride(1), V.stride(0), V.stride(1),
-            _hip.ptr(src_rows), T, H, D, int(page_size), k, index_repr, 1 if sel == "abs" else 0, mode,
-            gt, gc, 1 if v_bf16 else 0, _hip.ptr(dst_pages), _hip.ptr(dst_groups), store_table(K.device).data_ptr(),
-            planes["k_base"].data_ptr(), planes["k_scale"].data_ptr(), planes["k_zp"].data_ptr(),
-            _hip.ptr(planes.get("k_fp4_mapscale")), _hip.ptr(planes.get("k_fp4_mapcenter")),
-            _hip.ptr(index_plane), _hip.ptr(planes.get("k_oval")),
-            planes["v_main"].data_ptr(), planes["v_scale"].data_ptr(), planes["v_zp"].data_ptr(),
-            _hip.ptr(err_flag), _hip.current_stream_ptr(K.device))
-    _hip.check(rc, "ommx_store_pack")
+    target = dict(planes, k_obmp=index_plane) if combinadic else planes
+    if not _hip.host().store_pack(
+            K, V, target, int(page_size), src_rows, dst_pages, dst_groups, err_flag, T, store_table(K.device), 0, 0, 0,
+            k, gt, gc, "bitmap" if index_repr == _hip.INDEX_BITMAP else "relidx7", sel, bool(use_pow2),
+            bool(kv_int8_scale), "bf16" if v_bf16 else "i2"):
+        raise ValueError(f"the store launcher refused these arguments: K {tuple(K.shape)}, V {tuple(V.shape)}, "
+                         f"{T} tokens, {k} outliers, group_tokens={gt}, group_channels={gc}")
     if combinadic and T >= gt:
         convert_index_plane(index_plane, planes["k_crank"], group_tokens=gt, k=k, src_repr="bitmap",
                             dst_repr="combinadic", groups=dst_groups, n_groups=T // gt, err_flag=err_flag)
@@ -421,17 +424,31 @@ def ommx_pack_kv_canonical_block(
     if Vd.stride(-1) != 1:
         Vd = Vd.contiguous()
     G, pages = T // gt, T // int(page_size)
-    planes = alloc_planes(pages, G, H, D, page_size=int(page_size), outliers_per_vector=k, device=dev,
-                          outlier_repr=repr_l, kv_outlier_map=bool(kv_outlier_map),
-                          int8_scale=bool(use_pow2) and bool(kv_int8_scale),
-                          group_tokens=gt, group_channels=gc, v_format=vfmt)
-    err = torch.zeros(1, dtype=torch.int32, device=dev)
-    if T > 0:
-        store_pack_into(Kd, Vd, planes, outliers_per_vector=k, page_size=int(page_size), err_flag=err,
-                        outlier_repr=repr_l, outlier_select=outlier_select,
-                        use_pow2=bool(use_pow2), kv_int8_scale=bool(kv_int8_scale),
-                        group_tokens=gt, group_channels=gc, v_format=vfmt)
-    raise_for_store_errors(int(err.item()))
+    mode = (bool(use_pow2), bool(kv_int8_scale))
+    sel = str(outlier_select).lower()
+    packed = T > 0 and repr_l != "combinadic" and _hip.host().pack_block(
+        Kd, Vd, int(page_size), bool(kv_outlier_map), store_table(dev), k, gt, gc, repr_l, sel, *mode, vfmt)
+    if packed:
+        (bits, k_base, k_scale, k_zp, k_index, k_oval, k_ms, k_mc, v_main, v_scale, v_zp, to_token, to_group) = packed
+        planes = {"k_base": k_base, "k_scale": k_scale, "k_zp": k_zp, "k_oidx": None, "k_crank": None, "k_obmp": None,
+                  "k_oval": k_oval, "k_fp4_mapscale": k_ms, "k_fp4_mapcenter": k_mc,
+                  "v_main": v_main, "v_scale": v_scale, "v_zp": v_zp}
+        planes["k_obmp" if repr_l == "bitmap" else "k_oidx"] = k_index
+    else:
+        planes = alloc_planes(pages, G, H, D, page_size=int(page_size), outliers_per_vector=k, device=dev,
+                              outlier_repr=repr_l, kv_outlier_map=bool(kv_outlier_map), int8_scale=all(mode),
+                              group_tokens=gt, group_channels=gc, v_format=vfmt)
+        err = torch.zeros(1, dtype=torch.int32, device=dev)
+        if T > 0:
+            store_pack_into(Kd, Vd, planes, outliers_per_vector=k, page_size=int(page_size), err_flag=err,
+                            outlier_repr=repr_l, outlier_select=outlier_select,
+                            use_pow2=mode[0], kv_int8_scale=mode[1],
+                            group_tokens=gt, group_channels=gc, v_format=vfmt)
+        bits = int(err.item())
+        to_token = torch.arange(pages, dtype=torch.int32, device=dev).reshape(1, pages)
+        to_group = torch.arange(G, dtype=torch.int32, device=dev).reshape(1, G)
+    if bits:
+        raise_for_store_errors(bits)
 
     def _to(t):
         return t.to(device) if t is not None else None
@@ -446,10 +463,9 @@ def ommx_pack_kv_canonical_block(
         out["k_field_bytes"] = int(planes["k_crank"].shape[-1])
     out.update({name: _to(planes[name]) for name in ("v_main", "v_scale", "v_zp")})
     out.update(
-        req_to_token=torch.arange(pages, dtype=torch.int32, device=device).reshape(1, pages),
-        req_to_group=torch.arange(G, dtype=torch.int32, device=device).reshape(1, G),
+        req_to_token=_to(to_token), req_to_group=_to(to_group),
         head_dim=D, n_kv_heads=H, num_tokens=T, n_groups=G, page_size=int(page_size),
-        outliers_per_vector=k, outlier_repr=repr_l, outlier_select=str(outlier_select).lower(),
+        outliers_per_vector=k, outlier_repr=repr_l, outlier_select=sel,
         group_tokens=gt, group_channels=gc, k_format=kfmt, v_format=vfmt,
         k_base_bits=2, oval_bits=4, use_pow2=bool(use_pow2),
         kv_outlier_map=bool(kv_outlier_map and k > 0),

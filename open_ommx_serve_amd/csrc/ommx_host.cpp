@@ -15,12 +15,16 @@
 #include <c10/hip/HIPGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <algorithm>
 #include <atomic>
+#include <initializer_list>
+#include <vector>
 
 #include "../../include/ommx_hip.h"
+#include "ommx_internal.h"
 
 namespace {
 
@@ -98,7 +102,7 @@ int auto_splits(int64_t max_seq, int64_t batch, int64_t kv_heads, int64_t n_cu, 
     return static_cast<int>((steps + per - 1) / per);
 }
 
-PyObject* py_auto_splits(PyObject*, PyObject* const* a, Py_ssize_t n) {
+PyObject* py_auto_num_kv_splits(PyObject*, PyObject* const* a, Py_ssize_t n) {
     bool ok = n == 7;
     if (!ok) { PyErr_SetString(PyExc_TypeError, "auto_num_kv_splits takes 7 arguments"); return nullptr; }
     const int64_t max_seq = as_int(a[0], ok), batch = as_int(a[1], ok), heads = as_int(a[2], ok),
@@ -271,13 +275,376 @@ PyObject* py_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Py_RETURN_TRUE;
 }
 
+// ── stores ─────────────────────────────────────────────────────────────────────────────────────
+
+hipStream_t stream_of(c10::Device dev) { return c10::hip::getCurrentHIPStream(dev.index()).stream(); }
+bool is_index(const at::Tensor* t, c10::Device dev, at::ScalarType type, int64_t n) {
+    return !t || (t->scalar_type() == type && t->is_contiguous() && t->numel() >= n && t->device() == dev);
+}
+
+// [T, H, D] rows of bf16 or fp32 with a contiguous last axis
+bool is_rows(const at::Tensor& t) {
+    return t.dim() == 3 && (t.scalar_type() == at::kBFloat16 || t.scalar_type() == at::kFloat) && t.stride(2) == 1;
+}
+
+struct Recipe {
+    int64_t k, gt, gc;
+    bool bitmap, abs, v_bf16;
+    int mode;
+};
+// (outliers, group_tokens, group_channels, outlier_repr, outlier_select, use_pow2, kv_int8_scale, v_format)
+bool read_recipe(PyObject* const* a, Recipe& r) {
+    bool ok = true;
+    r.k = as_int(a[0], ok); r.gt = as_int(a[1], ok); r.gc = as_int(a[2], ok);
+    r.bitmap = is_word(a[3], "bitmap");
+    if (!r.bitmap && !is_word(a[3], "relidx7")) return false;
+    r.abs = is_word(a[4], "abs");
+    if (!r.abs && !is_word(a[4], "signed")) return false;
+    const bool pow2 = as_bool(a[5], ok), int8 = as_bool(a[6], ok);
+    r.mode = !pow2 ? OMMX_SCALE_BF16 : (int8 ? OMMX_SCALE_POW2_INT8 : OMMX_SCALE_POW2_BF16);
+    r.v_bf16 = is_word(a[7], "bf16");
+    if (!r.v_bf16 && !is_word(a[7], "i2")) return false;
+    return ok && r.k >= 0 && r.k <= 16 && is_group_size(r.gt) && is_group_size(r.gc);
+}
+
+struct Planes {
+    const at::Tensor *k_base = nullptr, *k_scale = nullptr, *k_zp = nullptr, *ms = nullptr, *mc = nullptr,
+                     *index = nullptr, *oval = nullptr, *v_main = nullptr, *v_scale = nullptr, *v_zp = nullptr;
+};
+PyObject* g_names[11];      // interned keys of a plane dict
+enum { N_KBASE, N_KSCALE, N_KZP, N_MS, N_MC, N_OBMP, N_OIDX, N_OVAL, N_VMAIN, N_VSCALE, N_VZP };
+
+bool read_planes(PyObject* d, const Recipe& r, Planes& p) {
+    if (!PyDict_Check(d)) return false;
+    bool ok = true;
+    auto get = [&](int name) -> const at::Tensor* {
+        PyObject* o = PyDict_GetItem(d, g_names[name]);      // borrowed
+        return !o || o == Py_None ? nullptr : as_tensor(o, ok);
+    };
+    p = {get(N_KBASE), get(N_KSCALE), get(N_KZP), get(N_MS), get(N_MC), get(r.bitmap ? N_OBMP : N_OIDX),
+         get(N_OVAL), get(N_VMAIN), get(N_VSCALE), get(N_VZP)};
+    if (!ok || !p.k_base || !p.k_scale || !p.k_zp || !p.v_main || !p.v_scale || !p.v_zp) return false;
+    if (r.k > 0 && (!p.index || p.index->dim() < 1 ||
+                    p.index->size(-1) != (r.bitmap ? (r.gt + 7) / 8 : (7 * r.k + 7) / 8)))
+        return false;
+    const at::ScalarType step = r.mode == OMMX_SCALE_POW2_INT8 ? at::kChar : at::kBFloat16;
+    return (p.v_main->scalar_type() == at::kBFloat16) == r.v_bf16 && p.k_scale->scalar_type() == step &&
+           p.v_scale->scalar_type() == step;
+}
+
+int launch_store(const at::Tensor& K, const at::Tensor& V, int64_t row0, const Planes& p, const Recipe& r, int64_t T, int64_t ps,
+                 const int32_t* src, const int32_t* pages, const int32_t* groups, const at::Tensor& table,
+                 int32_t* err, bool err_words, hipStream_t stream) {
+    auto from = [row0](const at::Tensor& t) {
+        return static_cast<const char*>(t.data_ptr()) + row0 * t.stride(0) * static_cast<int64_t>(t.element_size());
+    };
+    return ommx::store_pack(
+        from(K), from(V), K.scalar_type() == at::kFloat, K.stride(0), K.stride(1), V.stride(0), V.stride(1),
+        src, T, K.size(1), K.size(2), ps, r.k, r.bitmap ? OMMX_INDEX_BITMAP : OMMX_INDEX_RELIDX7, r.abs, r.mode, r.gt,
+        r.gc, r.v_bf16, pages, groups, table.data_ptr<float>(), data<uint8_t>(p.k_base), data(p.k_scale),
+        data<uint16_t>(p.k_zp), data<uint16_t>(p.ms), data<uint16_t>(p.mc), data<uint8_t>(p.index),
+        data<uint8_t>(p.oval), data<uint8_t>(p.v_main), data(p.v_scale), data<uint16_t>(p.v_zp), err, err_words,
+        stream);
+}
+
+// (K, V, planes, page_size, src_rows, dst_pages, dst_groups, err_flag, num_tokens, table, row0, page0, group0, recipe x 8);
+// without src_rows the tokens are the rows row0, row0 + 1, ...; the tables are read from entry page0 / group0 on
+PyObject* py_store_pack(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 21) { PyErr_SetString(PyExc_TypeError, "store_pack: wrong number of arguments"); return nullptr; }
+    bool ok = true;
+    const at::Tensor *K = as_tensor(a[0], ok), *V = as_tensor(a[1], ok), *src = as_tensor_or_none(a[4], ok),
+                     *pages = as_tensor_or_none(a[5], ok), *groups = as_tensor_or_none(a[6], ok),
+                     *err = as_tensor_or_none(a[7], ok), *table = as_tensor(a[9], ok);
+    const int64_t ps = as_int(a[3], ok), row0 = as_int(a[10], ok), page0 = as_int(a[11], ok), group0 = as_int(a[12], ok);
+    Recipe r;
+    Planes p;
+    if (!ok || !read_recipe(a + 13, r) || !read_planes(a[2], r, p) || !is_rows(*K) || !is_rows(*V) || ps < 1 ||
+        K->scalar_type() != V->scalar_type() || K->device() != V->device() || !K->is_cuda())
+        Py_RETURN_FALSE;
+    const c10::Device dev = K->device();
+    const int64_t T = a[8] != Py_None ? as_int(a[8], ok) : (src ? src->numel() : K->size(0));
+    if (!ok || T < 0 || row0 < 0 || page0 < 0 || group0 < 0 || (!src && row0 + T > K->size(0)) ||
+        !is_index(src, dev, at::kInt, T) || !is_index(pages, dev, at::kInt, page0 + T / ps) ||
+        !is_index(groups, dev, at::kInt, group0 + T / r.gt))
+        Py_RETURN_FALSE;
+    c10::hip::HIPGuard guard(dev.index());
+    hipStream_t stream = stream_of(dev);
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = launch_store(*K, *V, row0, p, r, T, ps, data<int32_t>(src), pages ? data<int32_t>(pages) + page0 : nullptr,
+                      groups ? data<int32_t>(groups) + group0 : nullptr, *table, data<int32_t>(err), false, stream);
+    Py_END_ALLOW_THREADS
+    if (failed(rc, "ommx_store_pack")) return nullptr;
+    Py_RETURN_TRUE;
+}
+
+// (K, V, page_size, kv_outlier_map, table, recipe x 8) -> (error bits, k_base, k_scale, k_zp, k_index, k_oval,
+// k_mapscale, k_mapcenter, v_main, v_scale, v_zp, req_to_token, req_to_group), or False.  Packs a block into planes
+// of its own with identity tables and waits for it: the error bits come back through host memory that the
+// kernel writes only when there is something to report, so the wait is the one host stop and nothing is copied.
+PyObject* py_pack_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 13) { PyErr_SetString(PyExc_TypeError, "pack_block: wrong number of arguments"); return nullptr; }
+    bool ok = true;
+    const at::Tensor *K = as_tensor(a[0], ok), *V = as_tensor(a[1], ok), *table = as_tensor(a[4], ok);
+    const int64_t ps = as_int(a[2], ok);
+    const bool own_map = as_bool(a[3], ok);
+    Recipe r;
+    if (!ok || !read_recipe(a + 5, r) || !is_rows(*K) || !is_rows(*V) || K->sizes() != V->sizes() || ps < 1 ||
+        K->scalar_type() != V->scalar_type() || K->device() != V->device() || !K->is_cuda() || K->size(0) < 1 ||
+        K->size(0) % ps || K->size(0) % r.gt || K->size(2) % r.gc)
+        Py_RETURN_FALSE;
+    const c10::Device dev = K->device();
+    c10::hip::HIPGuard guard(dev.index());
+    hipStream_t stream = stream_of(dev);
+    const int64_t T = K->size(0), H = K->size(1), D = K->size(2), G = T / r.gt, P = T / ps;
+    auto make = [&](at::IntArrayRef shape, at::ScalarType type) {
+        return at::empty(shape, at::TensorOptions().dtype(type).device(dev));
+    };
+    const at::ScalarType step = r.mode == OMMX_SCALE_POW2_INT8 ? at::kChar : at::kBFloat16;
+    enum { KBASE, KSCALE, KZP, INDEX, OVAL, MS, MC, VMAIN, VSCALE, VZP, TOK, GRP, COUNT };
+    at::Tensor t[COUNT];
+    t[KBASE] = make({P, ps, H, D / 4}, at::kByte);
+    t[KSCALE] = make({G, H, D}, step);
+    t[KZP] = make({G, H, D}, at::kBFloat16);
+    if (r.k > 0) {
+        t[INDEX] = make({G, H, D, r.bitmap ? (r.gt + 7) / 8 : (7 * r.k + 7) / 8}, at::kByte);
+        t[OVAL] = make({G, H, D, (r.k + 1) / 2}, at::kByte);
+        if (own_map) {
+            t[MS] = make({G, H, D}, at::kBFloat16);
+            t[MC] = make({G, H, D}, at::kBFloat16);
+        }
+    }
+    t[VMAIN] = r.v_bf16 ? make({P, ps, H, D}, at::kBFloat16) : make({P, ps, H, D / 4}, at::kByte);
+    t[VSCALE] = make({P, ps, H, D / r.gc}, step);
+    t[VZP] = make({P, ps, H, D / r.gc}, at::kBFloat16);
+    t[TOK] = make({1, P}, at::kInt);
+    t[GRP] = make({1, G}, at::kInt);
+    at::Tensor flags = at::empty({OMMX_STORE_ERR_WORDS}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+    int32_t* words = flags.data_ptr<int32_t>();
+    std::fill(words, words + OMMX_STORE_ERR_WORDS, 0);
+    auto opt = [&](int i) { return t[i].defined() ? &t[i] : nullptr; };
+    const Planes p{&t[KBASE], &t[KSCALE], &t[KZP], opt(MS), opt(MC), opt(INDEX), opt(OVAL), &t[VMAIN], &t[VSCALE],
+                   &t[VZP]};
+    int rc;
+    hipError_t waited = hipSuccess;
+    Py_BEGIN_ALLOW_THREADS
+    rc = launch_store(*K, *V, 0, p, r, T, ps, nullptr, nullptr, nullptr, *table, words, true, stream);
+    if (rc == 0) rc = ommx::identity_tables(t[TOK].data_ptr<int32_t>(), P, t[GRP].data_ptr<int32_t>(), G, stream);
+    if (rc == 0) waited = hipStreamSynchronize(stream);
+    Py_END_ALLOW_THREADS
+    if (failed(rc, "ommx_store_pack")) return nullptr;
+    if (waited != hipSuccess) {
+        PyErr_Format(PyExc_RuntimeError, "ommx_store_pack: %s", hipGetErrorString(waited));
+        return nullptr;
+    }
+    long bits = 0;
+    for (int i = 0; i < OMMX_STORE_ERR_WORDS; ++i) bits |= (words[i] ? 1L : 0L) << i;
+    PyObject* out = PyTuple_New(1 + COUNT);
+    PyTuple_SET_ITEM(out, 0, PyLong_FromLong(bits));
+    for (int i = 0; i < COUNT; ++i) {
+        if (!t[i].defined()) { Py_INCREF(Py_None); PyTuple_SET_ITEM(out, 1 + i, Py_None); }
+        else PyTuple_SET_ITEM(out, 1 + i, THPVariable_Wrap(std::move(t[i])));
+    }
+    return out;
+}
+
+// ── bf16 row history ───────────────────────────────────────────────────────────────────────────
+
+bool is_history(const at::Tensor& k, const at::Tensor& v) {
+    return k.dim() == 4 && k.sizes() == v.sizes() && k.scalar_type() == at::kBFloat16 &&
+           v.scalar_type() == at::kBFloat16 && k.is_contiguous() && v.is_contiguous() && k.is_cuda();
+}
+
+// (k_hist, v_hist, pos, k, v, sink, span, slots, pos_next, err_flag)
+PyObject* py_ring_write(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 10) { PyErr_SetString(PyExc_TypeError, "ring_write: wrong number of arguments"); return nullptr; }
+    bool ok = true;
+    const at::Tensor *kh = as_tensor(a[0], ok), *vh = as_tensor(a[1], ok), *pos = as_tensor(a[2], ok),
+                     *k = as_tensor(a[3], ok), *v = as_tensor(a[4], ok), *slots = as_tensor_or_none(a[7], ok),
+                     *next = as_tensor_or_none(a[8], ok), *err = as_tensor_or_none(a[9], ok);
+    const int64_t sink = as_int(a[5], ok), span = as_int(a[6], ok);
+    if (!ok || !is_history(*kh, *vh) || k->dim() != 3 || k->sizes() != v->sizes()) Py_RETURN_FALSE;
+    const c10::Device dev = kh->device();
+    const int64_t B = k->size(0), N = kh->size(0), rows = kh->size(1), H = kh->size(2), D = kh->size(3);
+    if (k->size(1) != H || k->size(2) != D || k->scalar_type() != at::kBFloat16 ||
+        v->scalar_type() != at::kBFloat16 || k->stride(2) != 1 || v->stride(2) != 1 ||
+        !is_index(pos, dev, at::kLong, B) || !is_index(slots, dev, at::kLong, B) ||
+        !is_index(next, dev, at::kLong, B) || (!slots && B > N))
+        Py_RETURN_FALSE;
+    c10::hip::HIPGuard guard(dev.index());
+    hipStream_t stream = stream_of(dev);
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = ommx_ring_write(data<uint16_t>(k), data<uint16_t>(v), k->stride(0), k->stride(1), v->stride(0), v->stride(1),
+                         data<uint16_t>(kh), data<uint16_t>(vh), kh->stride(0), rows, data<int64_t>(slots),
+                         data<int64_t>(pos), data<int64_t>(next), B, H, D, sink, span, data<int32_t>(err), stream);
+    Py_END_ALLOW_THREADS
+    if (failed(rc, "ommx_ring_write")) return nullptr;
+    Py_RETURN_TRUE;
+}
+
+// (k_hist, v_hist, k_tail, v_tail, span, seq, tail_idx, slots, b_tail_len, b_seq_len, window_sink, window_recent,
+//  group_tokens, packed_lag, err_flag)
+PyObject* py_tail_gather(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 15) { PyErr_SetString(PyExc_TypeError, "tail_gather: wrong number of arguments"); return nullptr; }
+    bool ok = true;
+    const at::Tensor *kh = as_tensor(a[0], ok), *vh = as_tensor(a[1], ok), *kt = as_tensor(a[2], ok),
+                     *vt = as_tensor(a[3], ok), *seq = as_tensor_or_none(a[5], ok),
+                     *idx = as_tensor_or_none(a[6], ok), *slots = as_tensor_or_none(a[7], ok),
+                     *bt = as_tensor_or_none(a[8], ok), *bs = as_tensor_or_none(a[9], ok),
+                     *err = as_tensor_or_none(a[14], ok);
+    const int64_t span = as_int(a[4], ok), wsink = as_int(a[10], ok), recent = as_int(a[11], ok),
+                  gt = as_int(a[12], ok), lag = as_int(a[13], ok);
+    if (!ok || !is_history(*kh, *vh) || kt->dim() != 4 || kt->sizes() != vt->sizes() || !seq == !idx) Py_RETURN_FALSE;
+    const c10::Device dev = kh->device();
+    const int64_t B = kt->size(0), T = kt->size(1), N = kh->size(0), rows = kh->size(1), H = kh->size(2), D = kh->size(3);
+    if (kt->size(2) != H || kt->size(3) != D || kt->scalar_type() != at::kBFloat16 ||
+        vt->scalar_type() != at::kBFloat16 || !kt->is_contiguous() || !vt->is_contiguous() ||
+        !is_index(seq, dev, at::kLong, B) || !is_index(idx, dev, at::kLong, B * T) ||
+        !is_index(slots, dev, at::kLong, B) || !is_index(bt, dev, at::kInt, B) || !is_index(bs, dev, at::kInt, B) ||
+        (!slots && B > N))
+        Py_RETURN_FALSE;
+    c10::hip::HIPGuard guard(dev.index());
+    hipStream_t stream = stream_of(dev);
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = ommx_tail_gather(data<uint16_t>(kh), data<uint16_t>(vh), kh->stride(0), rows, data<int64_t>(slots),
+                          data<int64_t>(seq), data<int64_t>(idx), data<uint16_t>(kt), data<uint16_t>(vt),
+                          data<int32_t>(bt), data<int32_t>(bs), B, T, H, D, wsink, recent, gt, span, lag,
+                          data<int32_t>(err), stream);
+    Py_END_ALLOW_THREADS
+    if (failed(rc, "ommx_tail_gather")) return nullptr;
+    Py_RETURN_TRUE;
+}
+
+// (K, V, k_hist, v_hist, request, pos0, n_head, lo, sink, span): rows [0, n_head) and [lo, T) of a block into the
+// history of one request
+PyObject* py_rows_write(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 10) { PyErr_SetString(PyExc_TypeError, "rows_write: wrong number of arguments"); return nullptr; }
+    bool ok = true;
+    const at::Tensor *K = as_tensor(a[0], ok), *V = as_tensor(a[1], ok), *kh = as_tensor(a[2], ok),
+                     *vh = as_tensor(a[3], ok);
+    const int64_t req = as_int(a[4], ok), pos0 = as_int(a[5], ok), head = as_int(a[6], ok), lo = as_int(a[7], ok),
+                  sink = as_int(a[8], ok), span = as_int(a[9], ok);
+    if (!ok || !is_history(*kh, *vh) || !is_rows(*K) || !is_rows(*V) || K->sizes() != V->sizes() ||
+        K->device() != kh->device() || V->device() != kh->device())
+        Py_RETURN_FALSE;
+    const int64_t T = K->size(0), rows = kh->size(1), H = kh->size(2), D = kh->size(3);
+    // every slot has to lie inside the history: below the ring's end, or the block's last position without a ring
+    if (K->size(1) != H || K->size(2) != D || D % 8 || req < 0 || req >= kh->size(0) || pos0 < 0 || head < 0 ||
+        lo < head || lo > T || sink < 0 || span < 0 || (span > 0 ? sink + span : pos0 + T) > rows)
+        Py_RETURN_FALSE;
+    const c10::Device dev = kh->device();
+    c10::hip::HIPGuard guard(dev.index());
+    hipStream_t stream = stream_of(dev);
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = ommx::rows_write(K->data_ptr(), V->data_ptr(), K->scalar_type() == at::kFloat, V->scalar_type() == at::kFloat,
+                          K->stride(0), K->stride(1), V->stride(0), V->stride(1),
+                          data<uint16_t>(kh) + req * kh->stride(0), data<uint16_t>(vh) + req * vh->stride(0), pos0,
+                          head, lo, T, H, D, sink, span, stream);
+    Py_END_ALLOW_THREADS
+    if (failed(rc, "rows_write")) return nullptr;
+    Py_RETURN_TRUE;
+}
+
+bool read_ints(PyObject* list, std::vector<int64_t>& out) {
+    if (!PyList_Check(list)) return false;
+    bool ok = true;
+    const Py_ssize_t n = PyList_GET_SIZE(list);
+    out.reserve(n);
+    for (Py_ssize_t i = 0; i < n; ++i) out.push_back(as_int(PyList_GET_ITEM(list, i), ok));
+    return ok;
+}
+
+// (k_hist, v_hist, planes, pairs [r0, g0, r1, g1, ...], page_size, hist sink, hist span, window_sink, groups_per_seq,
+//  err_flag, table, recipe x 8): packs group g of request r for every pair, the rows read in place from the history
+PyObject* py_pack_groups(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 19) { PyErr_SetString(PyExc_TypeError, "pack_groups: wrong number of arguments"); return nullptr; }
+    bool ok = true;
+    const at::Tensor *kh = as_tensor(a[0], ok), *vh = as_tensor(a[1], ok), *err = as_tensor_or_none(a[9], ok),
+                     *table = as_tensor(a[10], ok);
+    const int64_t ps = as_int(a[4], ok), sink = as_int(a[5], ok), span = as_int(a[6], ok), wsink = as_int(a[7], ok),
+                  per_seq = as_int(a[8], ok);
+    Recipe r;
+    Planes p;
+    std::vector<int64_t> pairs64;
+    if (!ok || !is_history(*kh, *vh) || !read_recipe(a + 11, r) || !read_planes(a[2], r, p) || ps < 1 || r.gt % ps ||
+        !read_ints(a[3], pairs64) || pairs64.empty() || pairs64.size() % 2)
+        Py_RETURN_FALSE;
+    const int64_t count = static_cast<int64_t>(pairs64.size()) / 2, ppg = r.gt / ps, N = kh->size(0), rows = kh->size(1);
+    for (int64_t i = 0; i < count; ++i) {
+        const int64_t req = pairs64[2 * i], g = pairs64[2 * i + 1];
+        if (req < 0 || req >= N || g < 0 || g >= per_seq || (span == 0 && wsink + (g + 1) * r.gt > rows)) Py_RETURN_FALSE;
+    }
+    if (span > 0 && sink + span > rows) Py_RETURN_FALSE;
+    const std::vector<int32_t> pairs(pairs64.begin(), pairs64.end());
+    const c10::Device dev = kh->device();
+    c10::hip::HIPGuard guard(dev.index());
+    hipStream_t stream = stream_of(dev);
+    // index tables: stream-ordered scratch, given back to torch's allocator when this call returns
+    c10::DataPtr scratch = c10::GetAllocator(c10::DeviceType::CUDA)->allocate(count * (r.gt + ppg + 1) * sizeof(int32_t));
+    int32_t *src = static_cast<int32_t*>(scratch.get()), *pages = src + count * r.gt, *groups = pages + count * ppg;
+    const at::Tensor K = kh->view({N * rows, kh->size(2), kh->size(3)}), V = vh->view({N * rows, kh->size(2), kh->size(3)});
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = ommx::pack_list(pairs.data(), count, src, pages, groups, r.gt, ppg, rows, sink, span, wsink, per_seq,
+                         per_seq * ppg, stream);
+    if (rc == 0)
+        rc = launch_store(K, V, 0, p, r, count * r.gt, ps, src, pages, groups, *table, data<int32_t>(err), false, stream);
+    Py_END_ALLOW_THREADS
+    if (failed(rc, "ommx_store_pack")) return nullptr;
+    Py_RETURN_TRUE;
+}
+
+// (dst, values): a contiguous int64 or int32 tensor on the GPU filled from a list of ints, by a launch
+PyObject* py_upload(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 2) { PyErr_SetString(PyExc_TypeError, "upload: wrong number of arguments"); return nullptr; }
+    bool ok = true;
+    const at::Tensor* dst = as_tensor(a[0], ok);
+    std::vector<int64_t> values;
+    if (!ok || !dst->is_cuda() || !dst->is_contiguous() || !read_ints(a[1], values) ||
+        dst->numel() != static_cast<int64_t>(values.size()) ||
+        (dst->scalar_type() != at::kLong && dst->scalar_type() != at::kInt))
+        Py_RETURN_FALSE;
+    c10::hip::HIPGuard guard(dst->device().index());
+    hipStream_t stream = stream_of(dst->device());
+    int rc;
+    if (dst->scalar_type() == at::kLong) {
+        rc = ommx::upload_words(static_cast<int32_t*>(dst->data_ptr()), reinterpret_cast<const int32_t*>(values.data()),
+                                static_cast<int>(2 * values.size()), stream);
+    } else {
+        const std::vector<int32_t> words(values.begin(), values.end());
+        rc = ommx::upload_words(static_cast<int32_t*>(dst->data_ptr()), words.data(), static_cast<int>(words.size()), stream);
+    }
+    if (failed(rc, "upload")) return nullptr;
+    Py_RETURN_TRUE;
+}
+
+// C++ exceptions (out of memory among them) become the Python exceptions torch raises for them.
+template <PyObject* (*F)(PyObject*, PyObject* const*, Py_ssize_t)>
+PyObject* guarded(PyObject* self, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    return F(self, a, n);
+    END_HANDLE_TH_ERRORS
+}
+
+#define OMMX_FAST(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(guarded<py_##name>)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
-    {"auto_num_kv_splits", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_auto_splits)), METH_FASTCALL, nullptr},
-    {"decode", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_decode)), METH_FASTCALL, nullptr},
+    OMMX_FAST(auto_num_kv_splits),
+    OMMX_FAST(decode), OMMX_FAST(store_pack), OMMX_FAST(pack_block), OMMX_FAST(pack_groups), OMMX_FAST(ring_write),
+    OMMX_FAST(tail_gather), OMMX_FAST(rows_write), OMMX_FAST(upload),
     {nullptr, nullptr, 0, nullptr},
 };
+#undef OMMX_FAST
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_ommx_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__ommx_host(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__ommx_host(void) {
+    const char* names[] = {"k_base", "k_scale", "k_zp", "k_fp4_mapscale", "k_fp4_mapcenter", "k_obmp",
+                           "k_oidx", "k_oval", "v_main", "v_scale", "v_zp"};
+    for (int i = 0; i < 11; ++i)
+        if (!(g_names[i] = PyUnicode_InternFromString(names[i]))) return nullptr;
+    return PyModule_Create(&module);
+}

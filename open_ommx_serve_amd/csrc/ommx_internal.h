@@ -1,0 +1,40 @@
+// Entry points of libommx_hip.so that only the native half of the Python launchers uses: not part of the
+// C ABI.  Plain C++ (no device code), so that the host module can include it.
+#pragma once
+#include <stdint.h>
+
+#define OMMX_STORE_ERR_WORDS 16
+
+namespace ommx {
+
+// ommx_store_pack (the C ABI documents the arguments) with one more choice: err_words, err_flag is an array of
+// OMMX_STORE_ERR_WORDS host-visible ints, one per error bit.
+int store_pack(const void* K, const void* V, int in_dtype, int64_t k_ts, int64_t k_hs, int64_t v_ts, int64_t v_hs,
+               const int32_t* src_rows, int T, int H, int D, int page_size, int k_outliers, int index_repr,
+               int select_abs, int scale_mode, int group_tokens, int group_channels, int v_bf16,
+               const int32_t* dst_pages, const int32_t* dst_groups, const float* table, uint8_t* k_base,
+               void* k_scale, uint16_t* k_zp, uint16_t* k_ms, uint16_t* k_mc, uint8_t* k_index, uint8_t* k_oval,
+               uint8_t* v_main, void* v_scale, uint16_t* v_zp, int32_t* err_flag, bool err_words, void* stream);
+
+// req_to_token[i] = i for i < n_pages and req_to_group[i] = i for i < n_groups, one launch.
+int identity_tables(int32_t* req_to_token, int n_pages, int32_t* req_to_group, int n_groups, void* stream);
+
+// Rows [0, n_head) and [lo, T) of a K/V block [T, H, D] (fp32 or bf16, last axis contiguous) into the history
+// [hist_rows, H, D] of one request, at the ring slots of the absolute positions pos0 + row; rounds fp32 as
+// torch does.  The caller has checked that every slot lies inside the history.
+int rows_write(const void* K, const void* V, bool k_f32, bool v_f32, int64_t k_ts, int64_t k_hs, int64_t v_ts,
+               int64_t v_hs, uint16_t* k_hist, uint16_t* v_hist, int64_t pos0, int n_head, int lo, int T, int H,
+               int D, int sink, int span, void* stream);
+
+// Up to kUploadWords 32-bit words from the host to dst inside a kernel's own argument block: no staging buffer, no
+// copy engine, nothing to keep alive after the call.
+constexpr int kUploadWords = 960;
+int upload_words(int32_t* dst, const int32_t* host_words, int n, void* stream);
+
+// Index tables of one store launch that packs `n` groups of a pool, from (request, group) pairs in host memory:
+// src_rows[n * gt] flat history rows through the ring map, dst_pages[n * ppg], dst_groups[n].
+int pack_list(const int32_t* host_pairs, int n, int32_t* src_rows, int32_t* dst_pages, int32_t* dst_groups, int gt,
+              int ppg, int hist_rows, int sink, int span, int window_sink, int groups_per_seq, int pages_per_seq,
+              void* stream);
+
+}  // namespace ommx

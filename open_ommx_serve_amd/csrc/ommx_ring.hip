@@ -15,6 +15,7 @@
 //
 // Both kernels are pure row copies (H*D bf16 per row), 16 bytes per thread when rows are
 // 16-byte aligned, one workgroup per row.
+#include "ommx_internal.h"
 #include "ommx_ring_args.h"
 
 namespace ommx {
@@ -127,6 +128,128 @@ int launch_tail_gather(const RingArgs& a, const int64_t* seq, const int64_t* tai
     const int threads = (a.H * a.D / (vec ? 8 : 1)) >= 256 ? 256 : 128;
     hipLaunchKernelGGL(tail_gather_kernel, dim3(T, B), dim3(threads), 0, st, a, seq, tail_idx,
                        k_tail, v_tail, T, recent, gt, lag, b_tail_len, b_seq_len, vec);
+    return 0;
+}
+
+// ---- prompt blocks ---------------------------------------------------------------------------
+// One workgroup per row, K and V together.  A row is H*D elements; a thread moves eight of them (16 bytes of
+// bf16) per turn.  Bound by HBM for long blocks, by the launch for the ring's few live rows; replaces one
+// torch copy per tensor (whole history) or nine small index launches (ring).
+template <bool F32>
+__device__ __forceinline__ void put8(uint16_t* dst, const void* src, int64_t at, bool vec) {
+    if constexpr (F32) {
+        const float* p = static_cast<const float*>(src) + at;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) dst[i] = f32_to_bf16_any(p[i]);
+    } else {
+        const uint16_t* p = static_cast<const uint16_t*>(src) + at;
+        if (vec) *reinterpret_cast<uint4*>(dst) = *reinterpret_cast<const uint4*>(p);
+        else
+#pragma unroll
+            for (int i = 0; i < 8; ++i) dst[i] = p[i];
+    }
+}
+
+struct BlockRows {
+    const void *K, *V;
+    int k_f32, v_f32, k_vec, v_vec;
+    int64_t k_ts, k_hs, v_ts, v_hs;
+    uint16_t *k_hist, *v_hist;
+    int64_t pos0;
+    int n_head, lo, H, D, sink, span;
+};
+
+__global__ void __launch_bounds__(256) rows_write_kernel(BlockRows a) {
+    const int row = static_cast<int>(blockIdx.x) < a.n_head ? blockIdx.x : a.lo + (blockIdx.x - a.n_head);
+    const int64_t at = ring_slot(a.pos0 + row, a.sink, a.span) * static_cast<int64_t>(a.H * a.D);
+    const int per_head = a.D / 8;
+    for (int i = threadIdx.x; i < a.H * per_head; i += blockDim.x) {
+        const int h = i / per_head, c = (i % per_head) * 8;
+        const int64_t k_at = row * a.k_ts + h * a.k_hs + c, v_at = row * a.v_ts + h * a.v_hs + c;
+        const int64_t to = at + h * a.D + c;
+        if (a.k_f32) put8<true>(a.k_hist + to, a.K, k_at, false); else put8<false>(a.k_hist + to, a.K, k_at, a.k_vec);
+        if (a.v_f32) put8<true>(a.v_hist + to, a.V, v_at, false); else put8<false>(a.v_hist + to, a.V, v_at, a.v_vec);
+    }
+}
+
+int rows_write(const void* K, const void* V, bool k_f32, bool v_f32, int64_t k_ts, int64_t k_hs, int64_t v_ts,
+               int64_t v_hs, uint16_t* k_hist, uint16_t* v_hist, int64_t pos0, int n_head, int lo, int T, int H,
+               int D, int sink, int span, void* stream) {
+    if (D % 8 || n_head < 0 || lo < n_head || lo > T) { set_error("rows_write: bad shape"); return -1; }
+    const int rows = n_head + (T - lo);
+    if (rows == 0) return 0;
+    const bool dst_ok = aligned16(k_hist) && aligned16(v_hist);
+    const BlockRows a{K, V, k_f32, v_f32, dst_ok && aligned16(K) && k_ts % 8 == 0 && k_hs % 8 == 0,
+                      dst_ok && aligned16(V) && v_ts % 8 == 0 && v_hs % 8 == 0, k_ts, k_hs, v_ts, v_hs, k_hist,
+                      v_hist, pos0, n_head, lo, H, D, sink, span};
+    hipLaunchKernelGGL(rows_write_kernel, dim3(rows), dim3(H * D / 8 > 64 ? 128 : 64), 0,
+                       static_cast<hipStream_t>(stream), a);
+    if (hipGetLastError() != hipSuccess) { set_error("rows_write: launch failed"); return -2; }
+    return 0;
+}
+
+// ---- small host-to-device blocks through the kernel argument buffer ----------------------------
+// A host-to-device copy of a few hundred bytes of pageable memory costs 10-15 us of host time and waits for its
+// staging; a launch that carries the words as its arguments costs 2 us and leaves nothing behind.
+struct Words { int32_t w[kUploadWords]; };
+
+__global__ void __launch_bounds__(256) upload_words_kernel(int32_t* dst, int n, Words words) {
+    for (int i = threadIdx.x; i < n; i += 256) dst[i] = words.w[i];
+}
+
+int upload_words(int32_t* dst, const int32_t* host_words, int n, void* stream) {
+    Words w;
+    for (int done = 0; done < n; done += kUploadWords) {
+        const int m = n - done < kUploadWords ? n - done : kUploadWords;
+        for (int i = 0; i < m; ++i) w.w[i] = host_words[done + i];
+        hipLaunchKernelGGL(upload_words_kernel, dim3(1), dim3(256), 0, static_cast<hipStream_t>(stream),
+                           dst + done, m, w);
+    }
+    if (hipGetLastError() != hipSuccess) { set_error("upload_words: launch failed"); return -2; }
+    return 0;
+}
+
+__global__ void __launch_bounds__(256) identity_tables_kernel(int32_t* a, int na, int32_t* b, int nb) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < na) a[i] = i;
+    if (i < nb) b[i] = i;
+}
+
+int identity_tables(int32_t* req_to_token, int n_pages, int32_t* req_to_group, int n_groups, void* stream) {
+    const int n = n_pages > n_groups ? n_pages : n_groups;
+    if (n <= 0) return 0;
+    hipLaunchKernelGGL(identity_tables_kernel, dim3((n + 255) / 256), dim3(256), 0, static_cast<hipStream_t>(stream),
+                       req_to_token, n_pages, req_to_group, n_groups);
+    if (hipGetLastError() != hipSuccess) { set_error("identity_tables: launch failed"); return -2; }
+    return 0;
+}
+
+// One workgroup per group of the list.
+constexpr int kPackPairs = kUploadWords / 2;
+__global__ void __launch_bounds__(128) pack_list_kernel(int32_t* src_rows, int32_t* dst_pages, int32_t* dst_groups,
+                                                        int gt, int ppg, int hist_rows, int sink, int span,
+                                                        int window_sink, int groups_per_seq, int pages_per_seq,
+                                                        Words pairs) {
+    const int n = blockIdx.x, r = pairs.w[2 * n], g = pairs.w[2 * n + 1], t = threadIdx.x;
+    if (t < gt)
+        src_rows[n * gt + t] = r * hist_rows + static_cast<int32_t>(ring_slot(window_sink + g * gt + t, sink, span));
+    if (t < ppg) dst_pages[n * ppg + t] = r * pages_per_seq + g * ppg + t;
+    if (t == 0) dst_groups[n] = r * groups_per_seq + g;
+}
+
+int pack_list(const int32_t* host_pairs, int n, int32_t* src_rows, int32_t* dst_pages, int32_t* dst_groups, int gt,
+              int ppg, int hist_rows, int sink, int span, int window_sink, int groups_per_seq, int pages_per_seq,
+              void* stream) {
+    if (gt > 128 || ppg > gt) { set_error("pack_list: bad group size"); return -1; }
+    Words w;
+    for (int done = 0; done < n; done += kPackPairs) {
+        const int m = n - done < kPackPairs ? n - done : kPackPairs;
+        for (int i = 0; i < 2 * m; ++i) w.w[i] = host_pairs[2 * done + i];
+        hipLaunchKernelGGL(pack_list_kernel, dim3(m), dim3(128), 0, static_cast<hipStream_t>(stream),
+                           src_rows + done * gt, dst_pages + done * ppg, dst_groups + done, gt, ppg, hist_rows, sink,
+                           span, window_sink, groups_per_seq, pages_per_seq, w);
+    }
+    if (hipGetLastError() != hipSuccess) { set_error("pack_list: launch failed"); return -2; }
     return 0;
 }
 

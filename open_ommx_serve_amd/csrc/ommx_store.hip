@@ -442,7 +442,7 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
         else reinterpret_cast<uint16_t*>(a.v_scale)[vidx] = st.bits;
         a.v_zp[vidx] = zp_b;
     }
-    if (err && a.err) atomicOr(a.err, err);
+    if (err && a.err) report_store_bits(a, err);
 }
 
 }  // namespace ommx
@@ -467,17 +467,15 @@ extern "C" void ommx_store_default_table(float* t) {
     }
 }
 
-extern "C" int ommx_store_pack(const void* K, const void* V, int in_dtype,
-                               int64_t k_ts, int64_t k_hs, int64_t v_ts, int64_t v_hs,
-                               const int32_t* src_rows, int T, int H, int D, int page_size,
-                               int k_outliers, int index_repr, int select_abs, int scale_mode,
-                               int group_tokens, int group_channels, int v_bf16,
-                               const int32_t* dst_pages,
-                               const int32_t* dst_groups, const float* table,
-                               uint8_t* k_base, void* k_scale, uint16_t* k_zp,
-                               uint16_t* k_ms, uint16_t* k_mc, uint8_t* k_index,
-                               uint8_t* k_oval, uint8_t* v_main, void* v_scale,
-                               uint16_t* v_zp, int32_t* err_flag, void* stream) {
+int ommx::store_pack(const void* K, const void* V, int in_dtype,
+                     int64_t k_ts, int64_t k_hs, int64_t v_ts, int64_t v_hs,
+                     const int32_t* src_rows, int T, int H, int D, int page_size,
+                     int k_outliers, int index_repr, int select_abs, int scale_mode,
+                     int group_tokens, int group_channels, int v_bf16,
+                     const int32_t* dst_pages, const int32_t* dst_groups, const float* table,
+                     uint8_t* k_base, void* k_scale, uint16_t* k_zp, uint16_t* k_ms, uint16_t* k_mc,
+                     uint8_t* k_index, uint8_t* k_oval, uint8_t* v_main, void* v_scale, uint16_t* v_zp,
+                     int32_t* err_flag, bool err_words, void* stream) {
     using namespace ommx;
     const int gt = group_tokens, gc = group_channels;
     if (!(gt == 16 || gt == 32 || gt == 64 || gt == 128) || !(gc == 16 || gc == 32 || gc == 64 || gc == 128)) {
@@ -510,7 +508,7 @@ extern "C" int ommx_store_pack(const void* K, const void* V, int in_dtype,
                 static_cast<int8_t*>(v_scale), v_zp,
                 err_flag, H, D, page_size, k_outliers,
                 (reinterpret_cast<uintptr_t>(V) % 16 == 0 && v_ts % 8 == 0 && v_hs % 8 == 0) ? 1 : 0,
-                index_repr, select_abs ? 1 : 0, scale_mode, gt, gc, v_bf16 ? 1 : 0};
+                index_repr, select_abs ? 1 : 0, scale_mode, gt, gc, v_bf16 ? 1 : 0, err_words ? 1 : 0};
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (gt != 32 || gc != 32 || k_outliers > 8 || 32 % page_size || v_bf16) {   // everything but the 32x32 recipe
         if (launch_store_generic(a, T, in_dtype, st) != 0) {
@@ -533,4 +531,21 @@ extern "C" int ommx_store_pack(const void* K, const void* V, int in_dtype,
         hipLaunchKernelGGL((store_pack_kernel<false, false, 2>), grid, block, shm, st, a);
     if (hipGetLastError() != hipSuccess) { set_error("ommx_store_pack: launch failed"); return -2; }
     return 0;
+}
+
+extern "C" int ommx_store_pack(const void* K, const void* V, int in_dtype,
+                               int64_t k_ts, int64_t k_hs, int64_t v_ts, int64_t v_hs,
+                               const int32_t* src_rows, int T, int H, int D, int page_size,
+                               int k_outliers, int index_repr, int select_abs, int scale_mode,
+                               int group_tokens, int group_channels, int v_bf16,
+                               const int32_t* dst_pages,
+                               const int32_t* dst_groups, const float* table,
+                               uint8_t* k_base, void* k_scale, uint16_t* k_zp,
+                               uint16_t* k_ms, uint16_t* k_mc, uint8_t* k_index,
+                               uint8_t* k_oval, uint8_t* v_main, void* v_scale,
+                               uint16_t* v_zp, int32_t* err_flag, void* stream) {
+    return ommx::store_pack(K, V, in_dtype, k_ts, k_hs, v_ts, v_hs, src_rows, T, H, D, page_size, k_outliers,
+                            index_repr, select_abs, scale_mode, group_tokens, group_channels, v_bf16, dst_pages,
+                            dst_groups, table, k_base, k_scale, k_zp, k_ms, k_mc, k_index, k_oval, v_main,
+                            v_scale, v_zp, err_flag, false, stream);
 }

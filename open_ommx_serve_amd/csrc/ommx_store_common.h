@@ -3,6 +3,7 @@
 // in the reference packer's order; the including files are compiled with -ffp-contract=off.
 #pragma once
 #include "ommx_common.h"
+#include "ommx_internal.h"
 
 namespace ommx {
 
@@ -33,7 +34,16 @@ struct StoreArgs {
                             // 2 bf16((max - min) / 3) as it comes, bf16 plane (pack.py:459-463, 586-590)
     int gt, gc;             // tokens per K vector, channels per V vector (32 and 32 in the tuned kernel)
     int v_bf16;             // V is kept as bf16 rows [pages, ps, H, D]; v_scale = 1, v_zp = 0 (pack.py:596-602)
+    int err_words;          // err is an array of OMMX_STORE_ERR_WORDS ints in host memory, one per bit, instead of one
+                            // word of bits: the bus has no atomic OR, a store of 1 per bit needs none
 };
+
+// The bits a thread has found, into the caller's flag.  Reached on an error (or a noted wide step) only.
+__device__ __forceinline__ void report_store_bits(const StoreArgs& a, int bits) {
+    if (!a.err_words) { atomicOr(a.err, bits); return; }
+    for (int i = 0; i < OMMX_STORE_ERR_WORDS; ++i)
+        if ((bits >> i) & 1) *reinterpret_cast<volatile int32_t*>(a.err + i) = 1;
+}
 
 
 template <bool F32>

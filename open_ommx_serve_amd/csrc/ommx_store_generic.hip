@@ -242,7 +242,7 @@ __global__ void __launch_bounds__(256) store_generic_kernel(StoreArgs a) {
         else reinterpret_cast<uint16_t*>(a.v_scale)[vidx] = st.bits;
         a.v_zp[vidx] = zp_b;
     }
-    if (err && a.err) atomicOr(a.err, err);
+    if (err && a.err) report_store_bits(a, err);
 }
 
 template <bool F32, int GT>

@@ -1,0 +1,67 @@
+"""The launches behind the native half of the Python launchers, at the sizes where they can go
+wrong: row blocks of one row up to several workgroups, fp32 and strided sources, ring and whole
+history; uploads around the block that one launch carries; group lists longer than one launch."""
+import pytest
+import torch
+
+import oracle.ommx_oracle as O
+from open_ommx_serve_amd.attention import MultiSeqKVPool, WindowSpec, _hip
+from open_ommx_serve_amd.attention.kv_store_ops import ring_slot
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+RECIPE = dict(outliers_per_vector=6, outlier_repr="bitmap", use_pow2=True)
+
+
+def _block(T, H, D, dtype, seed, strided=False):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    t = torch.randn(T, H, 2 * D if strided else D, generator=g, device=DEV).to(dtype)
+    return t[..., D // 2:D // 2 + D] if strided else t
+
+
+@pytest.mark.parametrize("ring", [False, True])
+@pytest.mark.parametrize("T", [1, 7, 8, 9, 39, 71, 72, 73, 200, 1033])
+@pytest.mark.parametrize("dtype,strided", [(torch.bfloat16, False), (torch.float32, False), (torch.bfloat16, True)])
+def test_block_rows_reach_their_history_slots(ring, T, dtype, strided):
+    H, D, win = 2, 128, WindowSpec()
+    pool = MultiSeqKVPool(D, H, 3, 1100, window=win, device=DEV, kv_ring=ring, **RECIPE)
+    K, V = _block(T, H, D, dtype, 1, strided), _block(T, H, D, dtype, 2, strided)
+    assert pool.append_block(1, K, V) == win.num_groups(T)
+    live = range(T) if not ring else [*range(min(8, T)), *range(min(T, max(8, win.boundary(T) - 32)), T)]
+    for p in live:
+        slot = ring_slot(p, pool._ring_sink, pool._ring_rec) if ring else p
+        assert torch.equal(pool.k_hist[1, slot], K[p].to(torch.bfloat16)), p
+        assert torch.equal(pool.v_hist[1, slot], V[p].to(torch.bfloat16)), p
+    assert not pool.k_hist[0].any() and not pool.k_hist[2].any()
+    if win.num_groups(T):
+        edge = win.boundary(T)
+        want = O.pack_kv(K[8:edge].to(torch.bfloat16).cpu(), V[8:edge].to(torch.bfloat16).cpu())
+        got = pool.request_planes(1)
+        for n in ("k_base", "k_scale", "k_obmp", "k_oval", "v_main", "v_scale"):
+            assert torch.equal(got[n].cpu(), want[n]), n
+
+
+@pytest.mark.parametrize("n", [1, 479, 480, 481, 960, 961, 2000])
+@pytest.mark.parametrize("dtype", [torch.int64, torch.int32])
+def test_uploads_of_one_launch_and_more(n, dtype):
+    values = [(-1) ** i * (i * 7919 % 2000003) for i in range(n)]
+    out = torch.full((n + 1,), -5, dtype=dtype, device=DEV)
+    assert _hip.host().upload(out[:n], values)
+    assert out.tolist() == values + [-5]
+    assert not _hip.host().upload(out, values)              # a list of another length is refused
+
+
+@pytest.mark.parametrize("ring", [False, True])
+def test_groups_of_many_requests_complete_in_one_step(ring):
+    """490 requests complete a group in the same step: the group list takes two launches."""
+    B, H, D, win = 490, 1, 32, WindowSpec()
+    pool = MultiSeqKVPool(D, H, B, 80, window=win, device=DEV, kv_ring=ring, **RECIPE)
+    K, V = _block(73 * B, H, D, torch.bfloat16, 3).view(73, B, H, D), _block(73 * B, H, D, torch.bfloat16, 4).view(73, B, H, D)
+    for r in range(B):
+        pool.append_block(r, K[:71, r], V[:71, r])
+    assert pool.append_decode_batched(range(B), K[71], V[71]) == B
+    for r in (0, 1, 479, 480, 489):
+        want = O.pack_kv(K[8:40, r].cpu(), V[8:40, r].cpu())
+        got = pool.request_planes(r)
+        for n in ("k_base", "k_scale", "k_obmp", "k_oval", "v_main", "v_scale"):
+            assert torch.equal(got[n].cpu(), want[n]), (r, n)
