@@ -310,7 +310,8 @@ class MultiSeqKVPool:
         return self.regroup(r)
 
     def _bf16_batch(self, t: torch.Tensor, B: int) -> torch.Tensor:
-        t = t.reshape(B, self.H, self.D)
+        if t.dim() != 3 or int(t.shape[1]) != self.H or int(t.shape[0]) != B:
+            t = t.reshape(B, self.H, self.D)
         if t.dtype != torch.bfloat16 or t.device != self.device:
             t = t.to(self.device, torch.bfloat16)
         return t if t.stride(-1) == 1 else t.contiguous()
@@ -323,18 +324,22 @@ class MultiSeqKVPool:
         return out
 
     def _advance_host_and_pack(self, slots: Sequence[int]) -> int:
+        # (WindowSpec.num_groups in place: this runs per request, layer and step)
+        kept, gt = self.window.sink_tokens + self.window.recent_window, self.gt
+        seq, packed = self.seq_len, self.packed_groups
         pend: List[Tuple[int, int, int]] = []
         total = 0
         for r in slots:
-            self.seq_len[r] += 1
-            target = self.window.num_groups(self.seq_len[r])
-            if target > self.packed_groups[r]:
-                pend.append((r, self.packed_groups[r], target))
-                total += target - self.packed_groups[r]
+            n = seq[r] + 1
+            seq[r] = n
+            target = (n - kept) // gt
+            if target > packed[r]:
+                pend.append((r, packed[r], target))
+                total += target - packed[r]
         if pend:
             self._regroup_pack_batched_device(pend)
             for r, _g0, g1 in pend:
-                self.packed_groups[r] = g1
+                packed[r] = g1
         return total
 
     def append_decode_batched(self, slots: Sequence[int], K: torch.Tensor, V: torch.Tensor) -> int:
@@ -350,6 +355,17 @@ class MultiSeqKVPool:
         meta = self._upload(slots, [self.seq_len[r] for r in slots])
         write_tokens(self.k_hist, self.v_hist, meta[1], self._bf16_batch(K, B), self._bf16_batch(V, B),
                      self._ring_sink, self._ring_rec, slots=meta[0], err_flag=self.err_flag)
+        return self._advance_host_and_pack(slots)
+
+    def append_decode_rows(self, slots: Sequence[int], rows: torch.Tensor, cols: torch.Tensor, K: torch.Tensor,
+                           V: torch.Tensor) -> int:
+        """``append_decode_batched`` for a caller that already holds the slots and write positions on the
+        device (int64 ``[B]``): every layer of a model writes at the same ones."""
+        if not self.kv_ring:
+            for r in slots:
+                if self.seq_len[r] >= self.max_seq_len:
+                    raise RuntimeError(f"MultiSeqKVPool req {r} capacity {self.max_seq_len} exceeded")
+        self.append_decode_captured(rows, cols, K, V)
         return self._advance_host_and_pack(slots)
 
     def append_decode_captured(self, rows: torch.Tensor, cols: torch.Tensor, K: torch.Tensor,
@@ -589,6 +605,18 @@ class MultiSeqKVPool:
         self._gather(d["kt"], d["vt"], seq=meta[1], slots=d["sel"], b_tail=d["b_tail"], b_seq=d["b_seq"])
         max_pg = max([self.packed_groups[r] for r in slots], default=0)
         return self._bundle(d["sel"], d["b_seq"], d["b_tail"], d["kt"], d["vt"], max(1, max_pg * self.gt))
+
+    def decode_into(self, q: torch.Tensor, out: torch.Tensor, rows: torch.Tensor, seq: torch.Tensor,
+                    b_seq_len: torch.Tensor, tables: Tuple[torch.Tensor, torch.Tensor], *, sm_scale: float,
+                    max_seq_len: int, mean_seq_len: Optional[float] = None) -> bool:
+        """Decode ``q [B, Hq, D]`` over this pool into ``out`` (bf16 or fp32): the tail rows are read in
+        place from the history at the device lengths ``seq`` (int64) of the slots ``rows``, so there is no
+        gather launch; ``b_seq_len`` (int32) are the packed lengths, ``tables`` the page / group rows of
+        the slots.  False when the native launcher does not take the arguments (nothing is done then)."""
+        return self._host.decode_pool(q, self._store_planes, self.k_hist, self.v_hist, rows, seq, b_seq_len,
+                                      tables[0], tables[1], out, sm_scale, self.ps, max_seq_len, mean_seq_len,
+                                      self._ring_sink, self._ring_rec, self.window.sink_tokens,
+                                      self.window.recent_window, self.wide_steps, self.err_flag, *self._recipe)
 
     # ── device decode path ───────────────────────────────────────────────────────────
 

@@ -147,6 +147,7 @@ class CanonicalKVStore:
         self.err_flag = torch.zeros(1, dtype=torch.int32, device=dev)
         self.wide_steps = False      # a packed K step above 2^15 was seen: decode on the plain kernel
         self._host = _hip.host()
+        self._k_hist4, self._v_hist4 = self.k_hist.unsqueeze(0), self.v_hist.unsqueeze(0)
         # what every store launch of this cache is told (argument order of the native launchers)
         self._recipe = (self.k, self.gt, self.gc, self.outlier_repr, self.outlier_select, self.use_pow2,
                         self.kv_int8_scale, self.v_format)
@@ -203,6 +204,10 @@ class CanonicalKVStore:
     def write_token(self, pos: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> None:
         """Write one K/V row at the absolute position held in the device tensor ``pos``
         ([1] int64); launch-only, ``seq_len`` is not touched (kv_store.py:361-385)."""
+        if self._host.ring_write(self._k_hist4, self._v_hist4, pos, k.reshape(1, self.H, self.D),
+                                 v.reshape(1, self.H, self.D), self._ring_sink, self._ring_rec, None, None,
+                                 self.err_flag):
+            return
         kb = k.reshape(self.H, self.D)
         vb = v.reshape(self.H, self.D)
         if kb.dtype != torch.bfloat16 or kb.device != self.device:
@@ -262,7 +267,7 @@ class CanonicalKVStore:
         K, V = (t if t.dtype == torch.float32 and t.device == self.device else t.to(self.device, torch.bfloat16)
                 for t in (K, V))
         K, V = (t if t.stride(-1) == 1 else t.contiguous() for t in (K, V))
-        if not self._host.rows_write(K, V, self.k_hist.unsqueeze(0), self.v_hist.unsqueeze(0), 0, pos0, n_head, lo,
+        if not self._host.rows_write(K, V, self._k_hist4, self._v_hist4, 0, pos0, n_head, lo,
                                      self._ring_sink, self._ring_rec):
             raise ValueError(f"K / V rows {tuple(K.shape)} / {tuple(V.shape)} do not fit the history at position {pos0}")
 
@@ -286,7 +291,7 @@ class CanonicalKVStore:
             self._pack_block_into_planes(self.k_hist, self.v_hist, g0, g1, row0=row0)
             return
         pairs = [x for g in range(g0, g1) for x in (0, g)]
-        if self._host.pack_groups(self.k_hist.unsqueeze(0), self.v_hist.unsqueeze(0), self._store_planes, pairs,
+        if self._host.pack_groups(self._k_hist4, self._v_hist4, self._store_planes, pairs,
                                   self.ps, self._ring_sink, self._ring_rec, self.window.sink_tokens, self.G_cap,
                                   self.err_flag, store_table(self.k_hist.device), *self._recipe):
             return
@@ -344,6 +349,16 @@ class CanonicalKVStore:
         out.update(self._meta())
         out["err_flag"], out["force_reference_kernel"] = self.err_flag, self.wide_steps
         return out
+
+    def decode_into(self, q: torch.Tensor, out: torch.Tensor, seq: torch.Tensor, b_seq_len: torch.Tensor, *,
+                    sm_scale: float, max_seq_len: int) -> bool:
+        """Decode ``q [1, Hq, D]`` over this cache into ``out`` (bf16 or fp32), the tail rows read in place
+        from the history at the device length ``seq`` (int64 ``[1]``); ``b_seq_len`` (int32) is the packed
+        length.  False when the native launcher does not take the arguments (nothing is done then)."""
+        return self._host.decode_pool(q, self._store_planes, self._k_hist4, self._v_hist4, None, seq, b_seq_len,
+                                      self._req_to_token_full, self._req_to_group_full, out, sm_scale, self.ps,
+                                      max_seq_len, None, self._ring_sink, self._ring_rec, self.window.sink_tokens,
+                                      self.window.recent_window, self.wide_steps, self.err_flag, *self._recipe)
 
     def decode_planes_full(self) -> dict:
         """Full-capacity, fixed-address plane dict (kv_store.py:651-676)."""

@@ -61,7 +61,7 @@ def _compile(src: str, extra) -> str:
 
 
 def _compile_host() -> str:
-    """Host C++ only (no kernel in it); ``-isystem``: warnings of torch's own headers are not ours."""
+    """Host C++ only (no kernel in it; HIP's own headers ask g++ for the platform macro); ``-isystem``: warnings of torch's own headers are not ours."""
     from torch.utils.cpp_extension import include_paths
     obj = os.path.join(HERE, "ommx_host.o")
     inc = [f"-isystem{p}" for p in (*include_paths("cuda"), sysconfig.get_paths()["include"])]

@@ -3,6 +3,7 @@
 #include <string>
 
 #include "ommx_decode_args.h"
+#include "ommx_internal.h"
 #include "ommx_ring_args.h"
 
 namespace ommx {
@@ -167,6 +168,43 @@ extern "C" int ommx_decode_combine(
         return -1;
     }
     if (hipGetLastError() != hipSuccess) { set_error("ommx_decode_combine: launch failed"); return -2; }
+    return 0;
+}
+
+int ommx::decode_combine_hist(const float* attn_logits, int64_t al_b, int64_t al_h, int64_t al_s, const uint16_t* q,
+                              int64_t q_b, int64_t q_h, const HistTail& t, void* o, bool o_bf16, int64_t o_b,
+                              int64_t o_h, float* lse, int64_t lse_b, int B, int Hq, int Hkv, int D, int num_splits,
+                              int group_tokens, float sm_scale, float logit_cap, void* stream) {
+    const char* where = "decode_combine_hist";
+    if (B <= 0 || Hkv <= 0 || Hq % Hkv || num_splits < 1 || num_splits > 512 || !(D == 64 || D == 128) ||
+        group_tokens < 16 || group_tokens > 128 || t.rows <= 0 || t.win_sink < 0 || t.win_recent < 0) {
+        set_error2(where, "bad shape");
+        return -1;
+    }
+    const int most = t.win_recent + group_tokens - 1;      // rows past the sink
+    if (t.ring_span > 0 && (t.ring_sink != t.win_sink || t.ring_span < most || t.ring_sink + t.ring_span > t.rows)) {
+        set_error2(where, "the ring does not hold the window");
+        return -1;
+    }
+    if (!attn_logits || !o || !lse || !q || !t.k || !t.v || !t.seq ||
+        ((reinterpret_cast<uintptr_t>(t.k) | reinterpret_cast<uintptr_t>(t.v)) & 15) || t.stride_req % 8) {
+        set_error2(where, "null or misaligned pointer");
+        return -1;
+    }
+    const int64_t row = static_cast<int64_t>(Hkv) * D;
+    CombineArgs a{attn_logits, al_b, al_h, al_s, q, q_b, q_h, t.k, t.v, t.stride_req, row, D, t.stride_req, row, D,
+                  nullptr, nullptr, o_bf16 ? nullptr : static_cast<float*>(o), o_b, o_h, lse, lse_b, B, Hq, Hkv,
+                  num_splits, sm_scale, logit_cap, group_tokens, t.win_sink + most};
+    a.o16 = o_bf16 ? static_cast<uint16_t*>(o) : nullptr;
+    a.hist_seq = t.seq;
+    a.hist_slots = t.slots;
+    a.hist_rows = t.rows;
+    a.ring_sink = t.ring_span > 0 ? t.ring_sink : 0;
+    a.ring_span = t.ring_span;
+    a.win_sink = t.win_sink;
+    a.win_recent = t.win_recent;
+    if (launch_combine(a, D, static_cast<hipStream_t>(stream)) != 0) { set_error2(where, "unsupported shape"); return -1; }
+    if (hipGetLastError() != hipSuccess) { set_error2(where, "launch failed"); return -2; }
     return 0;
 }
 

@@ -44,7 +44,13 @@ __device__ __forceinline__ float wave64_max(float v) {
 
 // NT threads per workgroup, at most MAXS splits: 1024 / 256 in general, 512 / 64 when many
 // (request, head) pairs with few splits each fill the chip (fewer idle lanes per workgroup).
-template <int D, int Q, int NT = 1024, int MAXS = 256>
+__device__ __forceinline__ void put_out(const CombineArgs& a, int64_t at, float v) {
+    if (a.o16) a.o16[at] = f32_to_bf16_any(v);
+    else a.o[at] = v;
+}
+
+// HIST: the tail rows lie in a row history instead of a gathered buffer.
+template <int D, int Q, bool HIST, int NT = 1024, int MAXS = 256>
 __global__ void __launch_bounds__(NT) combine_kernel(CombineArgs a) {
     constexpr int CH = D / Q;            // channels of this workgroup (one of Q pieces of the head)
     constexpr int NSG = NT / CH;         // split groups: thread (d, sg) owns splits sg, sg + NSG, ...
@@ -64,13 +70,10 @@ __global__ void __launch_bounds__(NT) combine_kernel(CombineArgs a) {
     const int d = cq * CH + dl;          // this thread's channel of the head
     const int kvh = h / (a.Hq / a.Hkv);
     const float* base = a.al + b * a.al_b + (int64_t)h * a.al_h;
-    // the two scalars that everything after the split loads waits for: requested first
-    const int L = a.seq[b];
-    // a length outside the tail buffer (when the caller has said how many rows it holds) is held
-    // inside it, so that no row address leaves the buffer whatever b_tail_len contains
-    int tail = a.tail ? a.tail[b] : 0;
-    tail = max(tail, 0);
-    if (a.T > 0) tail = min(tail, a.T);
+    // what everything after the split loads waits for: requested first
+    TailRows<HIST> rows;
+    rows.init(a, b);
+    const int tail = rows.n;
 
     // ---- all loads of the split part --------------------------------------------------
     // They depend on the arguments only, so they go out before anything is read from
@@ -98,7 +101,6 @@ __global__ void __launch_bounds__(NT) combine_kernel(CombineArgs a) {
     // (the reference recomputes its rounding here, paged_decode.py:2407-2410).
     float my_lse = -INFINITY;
     if (tid < MAXS && tid < a.S) my_lse = base[(int64_t)tid * a.al_s + D];
-    (void)L;
 
     if (tid < D) s_q[tid] = __uint_as_float(q_raw << 16);
     if (tid < MAXS) {
@@ -116,17 +118,17 @@ __global__ void __launch_bounds__(NT) combine_kernel(CombineArgs a) {
     uint32_t vv[PER];
     auto load_rows = [&](int r0, int last) {
         ku = *reinterpret_cast<const uint4*>(
-            a.kt + b * a.kt_b + (int64_t)(r0 + min(row, last)) * a.kt_t + (int64_t)kvh * a.kt_h +
+            a.kt + rows.k_base + (int64_t)rows.row(r0 + min(row, last)) * a.kt_t + (int64_t)kvh * a.kt_h +
             (part * 8) % D);
 #pragma unroll
         for (int i = 0; i < PER; ++i)
-            vv[i] = a.vt[b * a.vt_b + (int64_t)(r0 + min(sg + NSG * i, last)) * a.vt_t +
+            vv[i] = a.vt[rows.v_base + (int64_t)rows.row(r0 + min(sg + NSG * i, last)) * a.vt_t +
                          (int64_t)kvh * a.vt_h + d];
     };
     // When the caller has said how many rows the tail buffers hold, the first chunk is asked for
     // here, with the split loads and before the tail length has arrived (its uses below wait for
     // it): rows past the tail are addressable, and neither their logits nor their V are used.
-    const bool early = a.T > 0 && a.tail != nullptr;
+    const bool early = a.T > 0 && (HIST || a.tail != nullptr);
     if (early) load_rows(0, min(ROWS, a.T) - 1);
     for (int r0 = 0; r0 < tail; r0 += ROWS) {
         const int nr = min(ROWS, tail - r0);
@@ -205,7 +207,7 @@ __global__ void __launch_bounds__(NT) combine_kernel(CombineArgs a) {
             W += w;
             A = fmaf(w, TA / TL, A);
         }
-        a.o[b * a.o_b + (int64_t)h * a.o_h + d] = W > 0.0f ? A / W : 0.0f;
+        put_out(a, b * a.o_b + (int64_t)h * a.o_h + d, W > 0.0f ? A / W : 0.0f);
         if (d == 0) a.lse[b * a.lse_b + h] = W > 0.0f ? n_max + __logf(W) : -INFINITY;
     }
 }
@@ -231,7 +233,7 @@ __device__ __forceinline__ float wave_sum_f32(float v) {
 // EARLY: the tail rows of the first pass are asked for before the split part and held in registers
 // (32 more: one workgroup per compute unit instead of two, which pays while the grid is no larger
 // than the chip).
-template <int D, int R, bool EARLY>
+template <int D, int R, bool EARLY, bool HIST>
 __global__ void __launch_bounds__(512) combine_grouped_kernel(CombineArgs a) {
     constexpr int NT = 512, MAXS = 64;
     constexpr int ROWS = 128;              // tail rows per pass (two per thread of the logit layout)
@@ -248,12 +250,9 @@ __global__ void __launch_bounds__(512) combine_grouped_kernel(CombineArgs a) {
     const int lane = tid & 63, wave = tid >> 6;
     const int h0 = kvh * R;
     const float* base = a.al + b * a.al_b + (int64_t)h0 * a.al_h;
-    const int L = a.seq[b];
-    // a length outside the tail buffer (when the caller has said how many rows it holds) is held
-    // inside it, so that no row address leaves the buffer whatever b_tail_len contains
-    int tail = a.tail ? a.tail[b] : 0;
-    tail = max(tail, 0);
-    if (a.T > 0) tail = min(tail, a.T);
+    TailRows<HIST> rows;
+    rows.init(a, b);
+    const int tail = rows.n;
 
     // ---- split weights: wave r, lane s ----------------------------------------------------
     if (a.q) {
@@ -265,7 +264,6 @@ __global__ void __launch_bounds__(512) combine_grouped_kernel(CombineArgs a) {
             s_q[r][2 * c2 + 1] = __uint_as_float(w & 0xFFFF0000u);
         }
     }
-    (void)L;
     if (wave < R) {
         const bool valid = lane < a.S;          // an empty split's lse is -inf
         const float my_lse = valid ? base[(int64_t)wave * a.al_h + (int64_t)lane * a.al_s + D] : -INFINITY;
@@ -293,7 +291,7 @@ __global__ void __launch_bounds__(512) combine_grouped_kernel(CombineArgs a) {
 #pragma unroll
             for (int c8 = 0; c8 < CHP / 8; ++c8) kk[h2][c8] = uint4{0u, 0u, 0u, 0u};
             if (t < nr) {
-                const uint16_t* kp = a.kt + b * a.kt_b + (int64_t)(r0 + t) * a.kt_t +
+                const uint16_t* kp = a.kt + rows.k_base + (int64_t)rows.row(r0 + t) * a.kt_t +
                                      (int64_t)kvh * a.kt_h + part * CHP;
 #pragma unroll
                 for (int c8 = 0; c8 < CHP / 8; ++c8) kk[h2][c8] = reinterpret_cast<const uint4*>(kp)[c8];
@@ -306,7 +304,7 @@ __global__ void __launch_bounds__(512) combine_grouped_kernel(CombineArgs a) {
                 vv[i] = 0u;
                 if (t < nr)
                     vv[i] = *reinterpret_cast<const uint32_t*>(
-                        a.vt + b * a.vt_b + (int64_t)(r0 + t) * a.vt_t + (int64_t)kvh * a.vt_h + 2 * dp);
+                        a.vt + rows.v_base + (int64_t)rows.row(r0 + t) * a.vt_t + (int64_t)kvh * a.vt_h + 2 * dp);
             }
         }
     };
@@ -420,7 +418,7 @@ __global__ void __launch_bounds__(512) combine_grouped_kernel(CombineArgs a) {
             } else {
                 for (int t = rg; t < nr; t += NRG) {
                     const uint32_t vw = *reinterpret_cast<const uint32_t*>(
-                        a.vt + b * a.vt_b + (int64_t)(r0 + t) * a.vt_t + (int64_t)kvh * a.vt_h + 2 * dp);
+                        a.vt + rows.v_base + (int64_t)rows.row(r0 + t) * a.vt_t + (int64_t)kvh * a.vt_h + 2 * dp);
                     const float v0 = __uint_as_float(vw << 16), v1 = __uint_as_float(vw & 0xFFFF0000u);
 #pragma unroll
                     for (int r = 0; r < R; ++r) {
@@ -464,13 +462,14 @@ __global__ void __launch_bounds__(512) combine_grouped_kernel(CombineArgs a) {
                 W += w;
                 Av = fmaf(w, TA / TL, Av);
             }
-            a.o[b * a.o_b + (int64_t)(h0 + r) * a.o_h + d] = W > 0.0f ? Av / W : 0.0f;
+            put_out(a, b * a.o_b + (int64_t)(h0 + r) * a.o_h + d, W > 0.0f ? Av / W : 0.0f);
             if (d == 0) a.lse[b * a.lse_b + h0 + r] = W > 0.0f ? n_max + __logf(W) : -INFINITY;
         }
     }
 }
 
-int launch_combine(const CombineArgs& a, int D, hipStream_t st) {
+template <bool HIST>
+static int launch_combine_rows(const CombineArgs& a, int D, hipStream_t st) {
     if (a.S > 512) return -1;
     // Pieces per head.  At batch 1 the kernel is latency bound and 2 pieces measured best (1.4 us
     // per step at 64K less than one, the same as four, 0.5 us less than eight); with many
@@ -487,8 +486,8 @@ int launch_combine(const CombineArgs& a, int D, hipStream_t st) {
         const bool early = a.B * a.Hkv <= 320;       // about one workgroup per compute unit
 #define OMMX_GROUPED(DD, RR)                                                                              \
         do {                                                                                              \
-            if (early) hipLaunchKernelGGL((combine_grouped_kernel<DD, RR, true>), g2, dim3(512), 0, st, a);  \
-            else hipLaunchKernelGGL((combine_grouped_kernel<DD, RR, false>), g2, dim3(512), 0, st, a);       \
+            if (early) hipLaunchKernelGGL((combine_grouped_kernel<DD, RR, true, HIST>), g2, dim3(512), 0, st, a);  \
+            else hipLaunchKernelGGL((combine_grouped_kernel<DD, RR, false, HIST>), g2, dim3(512), 0, st, a);       \
         } while (0)
         if (D == 128 && R == 4) OMMX_GROUPED(128, 4);
         else if (D == 128) OMMX_GROUPED(128, 8);
@@ -500,21 +499,25 @@ int launch_combine(const CombineArgs& a, int D, hipStream_t st) {
     }
     if (a.S > 256) {        // 257..512 splits: the same kernel with twice the split slots per thread
         const dim3 g1(a.B, a.Hq, split2 ? 2 : 1);
-        if (D == 128 && split2) hipLaunchKernelGGL((combine_kernel<128, 2, 1024, 512>), g1, dim3(1024), 0, st, a);
-        else if (D == 128) hipLaunchKernelGGL((combine_kernel<128, 1, 1024, 512>), g1, dim3(1024), 0, st, a);
-        else if (D == 64 && split2) hipLaunchKernelGGL((combine_kernel<64, 2, 1024, 512>), g1, dim3(1024), 0, st, a);
-        else if (D == 64) hipLaunchKernelGGL((combine_kernel<64, 1, 1024, 512>), g1, dim3(1024), 0, st, a);
+        if (D == 128 && split2) hipLaunchKernelGGL((combine_kernel<128, 2, HIST, 1024, 512>), g1, dim3(1024), 0, st, a);
+        else if (D == 128) hipLaunchKernelGGL((combine_kernel<128, 1, HIST, 1024, 512>), g1, dim3(1024), 0, st, a);
+        else if (D == 64 && split2) hipLaunchKernelGGL((combine_kernel<64, 2, HIST, 1024, 512>), g1, dim3(1024), 0, st, a);
+        else if (D == 64) hipLaunchKernelGGL((combine_kernel<64, 1, HIST, 1024, 512>), g1, dim3(1024), 0, st, a);
         else return -1;
         return 0;
     }
-    if (D == 128 && split2) hipLaunchKernelGGL((combine_kernel<128, 2>), grid, dim3(1024), 0, st, a);
-    else if (D == 128 && small) hipLaunchKernelGGL((combine_kernel<128, 1, 512, 64>), grid, dim3(512), 0, st, a);
-    else if (D == 128) hipLaunchKernelGGL((combine_kernel<128, 1>), grid, dim3(1024), 0, st, a);
-    else if (D == 64 && split2) hipLaunchKernelGGL((combine_kernel<64, 2>), grid, dim3(1024), 0, st, a);
-    else if (D == 64 && small) hipLaunchKernelGGL((combine_kernel<64, 1, 512, 64>), grid, dim3(512), 0, st, a);
-    else if (D == 64) hipLaunchKernelGGL((combine_kernel<64, 1>), grid, dim3(1024), 0, st, a);
+    if (D == 128 && split2) hipLaunchKernelGGL((combine_kernel<128, 2, HIST>), grid, dim3(1024), 0, st, a);
+    else if (D == 128 && small) hipLaunchKernelGGL((combine_kernel<128, 1, HIST, 512, 64>), grid, dim3(512), 0, st, a);
+    else if (D == 128) hipLaunchKernelGGL((combine_kernel<128, 1, HIST>), grid, dim3(1024), 0, st, a);
+    else if (D == 64 && split2) hipLaunchKernelGGL((combine_kernel<64, 2, HIST>), grid, dim3(1024), 0, st, a);
+    else if (D == 64 && small) hipLaunchKernelGGL((combine_kernel<64, 1, HIST, 512, 64>), grid, dim3(512), 0, st, a);
+    else if (D == 64) hipLaunchKernelGGL((combine_kernel<64, 1, HIST>), grid, dim3(1024), 0, st, a);
     else return -1;
     return 0;
+}
+
+int launch_combine(const CombineArgs& a, int D, hipStream_t st) {
+    return a.hist_seq ? launch_combine_rows<true>(a, D, st) : launch_combine_rows<false>(a, D, st);
 }
 
 }  // namespace ommx

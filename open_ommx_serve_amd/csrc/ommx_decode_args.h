@@ -71,6 +71,54 @@ struct CombineArgs {
     int gt;                          // tokens per K group: the splits are rounded to it
     int T;                           // rows every request's tail buffer holds (0: not told): rows below it
                                      // may be read before b_tail_len has arrived
+    uint16_t* o16;                   // bf16 output in place of o (same strides); NULL: fp32 into o
+    // Tail rows read in place from the row history instead of a gathered buffer: kt / vt are the histories, kt_b
+    // the elements between two requests' histories, and the rows follow from the sequence length (TailRows below).
+    const int64_t* hist_seq;         // NULL: gathered buffer
+    const int64_t* hist_slots;       // NULL: request b uses history b
+    int hist_rows, ring_sink, ring_span, win_sink, win_recent;
+};
+
+// The bf16 rows of one request: how many, and where row t of them lies (elements from the K / V base pointers).
+// Gathered buffer: rows 0, 1, ... of the request.  History: positions [0, min(sink, seq)) ++ [boundary, seq)
+// (kv_pool.py:1080-1097) through the ring map of kv_store.py:301-327; the sliding part starts at ring offset
+// `turn`, so a row costs one conditional subtraction instead of a remainder.
+template <bool HIST>
+struct TailRows {
+    int n, n_sink, turn, span, sink, cap;
+    int64_t k_base, v_base;
+
+    __device__ __forceinline__ void init(const CombineArgs& a, int b) {
+        if constexpr (!HIST) {
+            // a length outside the tail buffer (when the caller has said how many rows it holds) is held
+            // inside it, so that no row address leaves the buffer whatever b_tail_len contains
+            n = a.tail ? a.tail[b] : 0;
+            n = max(n, 0);
+            if (a.T > 0) n = min(n, a.T);
+            k_base = b * a.kt_b;
+            v_base = b * a.vt_b;
+            return;
+        }
+        const int seq = static_cast<int>(a.hist_seq[b]), slot = a.hist_slots ? static_cast<int>(a.hist_slots[b]) : b;
+        k_base = slot * a.kt_b;
+        v_base = slot * a.vt_b;
+        const int extra = seq - a.win_sink - a.win_recent;
+        n_sink = min(seq, a.win_sink);
+        const int boundary = extra <= 0 ? n_sink : a.win_sink + extra / a.gt * a.gt;
+        n = min(max(0, n_sink + max(seq - boundary, 0)), a.T);
+        sink = a.ring_sink;
+        span = a.ring_span;
+        cap = a.hist_rows;
+        turn = span > 0 && boundary >= sink ? (boundary - sink) % span : boundary - sink;
+    }
+    __device__ __forceinline__ int row(int t) const {
+        if constexpr (!HIST) return t;
+        if (t < n_sink) return t;              // (the ring pins the window's sink rows: ring_sink == win_sink, or no ring)
+        int r = turn + (t - n_sink);
+        if (span > 0 && r >= span) r -= span;
+        r += sink;
+        return min(max(r, 0), cap - 1);
+    }
 };
 
 int launch_decode_ref(const DecodeArgs& a, int D, int R, hipStream_t st);

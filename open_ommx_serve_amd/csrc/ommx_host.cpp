@@ -20,6 +20,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cstring>
 #include <initializer_list>
 #include <vector>
 
@@ -62,6 +63,8 @@ bool failed(int rc, const char* what) {
     PyErr_Format(PyExc_RuntimeError, "%s failed (rc=%d): %s", what, rc, ommx_last_error());
     return true;
 }
+
+hipStream_t stream_of(c10::Device dev) { return c10::hip::getCurrentHIPStream(dev.index()).stream(); }
 
 int cu_count(int device) {
     static std::atomic<int> known[64];
@@ -127,157 +130,206 @@ bool is_shape3(const at::Tensor& t, int64_t a, int64_t b, int64_t c) {
 }
 bool on(const at::Tensor* t, c10::Device d) { return t && t->device() == d; }
 
+// One decode call: what both Python entries below fill in.
+struct DecodeCall {
+    const at::Tensor *q = nullptr, *k_base = nullptr, *k_scale = nullptr, *k_zp = nullptr, *k_index = nullptr,
+                     *k_oval = nullptr, *v_main = nullptr, *v_scale = nullptr, *v_zp = nullptr, *k_tail = nullptr,
+                     *v_tail = nullptr, *b_tail = nullptr, *o = nullptr, *lse = nullptr, *rt = nullptr, *rg = nullptr,
+                     *seq = nullptr, *ms = nullptr, *mc = nullptr, *ws = nullptr, *err = nullptr;
+    double sm_scale = 1, cap = 0, mean = -1;             // mean < 0: not given
+    int64_t ps = 16, k = 0, splits = 0, max_seq = -1, max_tail = 1, off = 0, gbase = 0;   // splits 0 / max_seq < 0: not given
+    bool bitmap = false, want_map = false, int8 = false, force = false;
+    // tail rows read in place from the row history (k_tail / v_tail are [requests, rows, Hkv, D] then)
+    const at::Tensor *hist_seq = nullptr, *hist_slots = nullptr;
+    int64_t ring_sink = 0, ring_span = 0, win_sink = 0, win_recent = 0;
+};
+
+// Checks the call and launches it: 1 launched, 0 refused (nothing done), -1 a launch failed (exception set).
+int run_decode(const DecodeCall& c) {
+    const at::Tensor &q = *c.q, &k_base = *c.k_base, &k_scale = *c.k_scale, &v_main = *c.v_main, &v_scale = *c.v_scale;
+    // geometry of the planes
+    if (q.dim() != 3 || k_base.dim() != 4 || k_scale.dim() != 3 || v_main.dim() != 4 || v_scale.dim() != 4 ||
+        c.v_zp->dim() != 4 || c.ps < 1)
+        return 0;
+    const c10::Device dev = q.device();
+    if (!dev.is_cuda()) return 0;
+    const int64_t ps = c.ps, k = c.k, pages = k_base.size(0), slots = k_scale.size(0), B = q.size(0), Hq = q.size(1),
+                  Hkv = k_base.size(2), D = k_base.size(3) * 4;
+    const int64_t gt = (pages == 0 || slots == 0) ? 32 : pages * ps / slots;
+    const bool v_bf16 = v_main.scalar_type() == at::kBFloat16;
+    const int64_t v_width = v_bf16 ? v_main.size(3) : v_main.size(3) * 4, per_row = v_scale.size(3);
+    const int64_t gc = per_row == 0 ? 32 : v_width / per_row;
+    if (!is_group_size(gt) || !is_group_size(gc) || v_width % gc || B < 1 || Hkv < 1 || Hq < Hkv || Hq % Hkv ||
+        v_width != D || (D != 64 && D != 128) || q.size(2) != D || gt % ps || pages > INT32_MAX || slots > INT32_MAX)
+        return 0;
+    const int64_t R = Hq / Hkv;
+    if (R != 1 && R != 2 && R != 4 && R != 8) return 0;
+    for (const at::Tensor* t : {c.k_base, c.v_main, c.v_scale, c.v_zp})
+        if (!t->is_contiguous() || t->size(0) != pages || t->size(1) != ps || t->size(2) != Hkv) return 0;
+    if (!is_shape3(k_scale, slots, Hkv, D) || !is_shape3(*c.k_zp, slots, Hkv, D) ||
+        c.k_zp->scalar_type() != at::kBFloat16 || !is_shape3(*c.o, B, Hq, D))
+        return 0;
+    const at::ScalarType st = k_scale.scalar_type();
+    const bool scale_bf16 = st == at::kBFloat16;
+    if (st != v_scale.scalar_type() || (st != at::kChar && !scale_bf16) || scale_bf16 == c.int8) return 0;
+    if (q.scalar_type() != at::kBFloat16 || q.stride(2) != 1) return 0;
+
+    // lengths, tables, outputs
+    if (c.seq->numel() < B || !c.seq->is_contiguous() || c.seq->scalar_type() != at::kInt) return 0;
+    if (c.b_tail && (c.b_tail->numel() < B || !c.b_tail->is_contiguous() || c.b_tail->scalar_type() != at::kInt)) return 0;
+    const at::Tensor &rt = *c.rt, &rg = *c.rg;
+    if (rt.dim() != 2 || rg.dim() != 2 || rt.size(0) < B || rg.size(0) < B || rt.scalar_type() != rg.scalar_type() ||
+        (rt.scalar_type() != at::kInt && rt.scalar_type() != at::kLong) || rt.stride(1) != 1 || rg.stride(1) != 1)
+        return 0;
+    const bool hist = c.hist_seq != nullptr;
+    const bool o_bf16 = c.o->scalar_type() == at::kBFloat16;
+    if ((c.o->scalar_type() != at::kFloat && !(hist && o_bf16)) || c.o->stride(2) != 1) return 0;
+    if (!c.lse && !hist) return 0;
+    if (c.lse && (c.lse->dim() != 2 || c.lse->size(0) != B || c.lse->size(1) != Hq ||
+                  c.lse->scalar_type() != at::kFloat || c.lse->stride(1) != 1 || !on(c.lse, dev)))
+        return 0;
+    for (const at::Tensor* t : {c.k_base, c.k_scale, c.v_main, c.o, c.rt, c.rg, c.seq})
+        if (!on(t, dev)) return 0;
+    if (c.off < 0 || c.off >= ps || c.gbase < 0) return 0;
+
+    // outliers
+    const bool own_map = c.want_map && k > 0;
+    if (k < 0 || k > 16 || (c.bitmap && k > 8)) return 0;
+    if (k > 0) {
+        const int64_t index_bytes = c.bitmap ? (gt + 7) / 8 : (7 * k + 7) / 8;
+        for (const at::Tensor* t : {c.k_oval, c.k_index})
+            if (!t || t->scalar_type() != at::kByte || t->dim() != 4 || t->size(0) != slots || t->size(1) != Hkv ||
+                t->size(2) != D || t->size(3) != (t == c.k_oval ? (k + 1) / 2 : index_bytes) || !t->is_contiguous())
+                return 0;
+    }
+    if (own_map && (!c.ms || !c.mc)) return 0;
+    for (const at::Tensor* t : {c.ms, c.mc})
+        if (t && (!t->is_contiguous() ||
+                  (own_map && (t->scalar_type() != at::kBFloat16 || !is_shape3(*t, slots, Hkv, D)))))
+            return 0;
+    if (!k_scale.is_contiguous() || !c.k_zp->is_contiguous()) return 0;
+
+    // tail
+    const at::Tensor *kt = c.k_tail, *vt = c.v_tail;
+    bool tail = false;
+    if (hist) {
+        if (!kt || !vt || kt->dim() != 4 || kt->sizes() != vt->sizes() || kt->size(2) != Hkv || kt->size(3) != D ||
+            kt->scalar_type() != at::kBFloat16 || vt->scalar_type() != at::kBFloat16 || !kt->is_contiguous() ||
+            !vt->is_contiguous() || !on(kt, dev) || !on(vt, dev) || c.hist_seq->scalar_type() != at::kLong ||
+            !c.hist_seq->is_contiguous() || c.hist_seq->numel() < B || !on(c.hist_seq, dev) || c.gbase != 0)
+            return 0;
+        if (c.hist_slots ? (c.hist_slots->scalar_type() != at::kLong || !c.hist_slots->is_contiguous() ||
+                            c.hist_slots->numel() < B || !on(c.hist_slots, dev))
+                         : kt->size(0) < B)
+            return 0;
+    } else if (c.gbase == 0 && kt && vt && c.b_tail) {
+        if (kt->dim() != 4) return 0;
+        tail = kt->size(1) > 0 && c.max_tail > 0;
+        if (tail && (kt->scalar_type() != at::kBFloat16 || vt->scalar_type() != at::kBFloat16 || kt->stride(3) != 1 ||
+                     vt->dim() != 4 || vt->stride(3) != 1 || kt->sizes() != vt->sizes() || kt->size(0) < B ||
+                     kt->size(2) != Hkv || kt->size(3) != D))
+            return 0;
+    }
+    if (c.err && (c.err->scalar_type() != at::kInt || !on(c.err, dev))) return 0;
+
+    // splits and the workspace of their partial states
+    if (c.splits == 0 && c.max_seq < 0) return 0;
+    int64_t S = c.splits;
+    if (S == 0) {
+        // The serving-recipe kernel keeps three workgroups per compute unit resident with up to 4 q heads per
+        // kv head (two with 8, and so do the other kernels); at head_dim 64 one of its waves takes a pair of kv heads.
+        const bool plain_planes = gt == 32 && gc == 32 && !scale_bf16 && !v_bf16 && !c.force;
+        const bool lean = plain_planes && ((D == 128 && R <= 4 && k == 6) ||
+                                           (c.bitmap && k >= 1 && k <= 6 && ((D == 128 && R <= 4) ||
+                                                                             (D == 64 && R <= 2 && Hkv % 2 == 0))));
+        const bool paired = plain_planes && D == 64 && c.bitmap && k >= 1 && k <= 8 && R <= 4 && Hkv % 2 == 0;
+        S = auto_splits(c.max_seq, B, paired ? Hkv / 2 : Hkv, cu_count(dev.index()), gt, c.mean, lean ? 3 : 2);
+    }
+    if (c.ws && (c.ws->scalar_type() != at::kFloat || c.ws->dim() != 4 || c.ws->size(0) != B || c.ws->size(1) != Hq ||
+                 c.ws->size(2) < S || c.ws->size(3) < D + 1 || c.ws->stride(3) != 1))
+        return 0;
+
+    c10::hip::HIPGuard guard(dev.index());
+    hipStream_t stream = stream_of(dev);
+    int64_t al_b = Hq * (S + 1) * (D + 1), al_h = (S + 1) * (D + 1), al_s = D + 1;
+    c10::DataPtr scratch;
+    float *al, *lse = data<float>(c.lse);
+    if (c.ws && c.lse) {
+        al = c.ws->data_ptr<float>();
+        al_b = c.ws->stride(0); al_h = c.ws->stride(1); al_s = c.ws->stride(2);
+    } else {
+        scratch = c10::GetAllocator(c10::DeviceType::CUDA)->allocate(static_cast<size_t>(B * (al_b + Hq)) * sizeof(float));
+        al = static_cast<float*>(scratch.get());
+        if (!lse) lse = al + B * al_b;
+    }
+    const uint16_t* qp = data<const uint16_t>(c.q);
+    int rc, rc2 = 0;
+    Py_BEGIN_ALLOW_THREADS
+    rc = (c.force ? ommx_decode_splitkv_ref : ommx_decode_splitkv)(
+        qp, q.stride(0), q.stride(1), data<uint8_t>(c.k_base), data(c.k_scale), data<uint16_t>(c.k_zp),
+        own_map ? data<uint16_t>(c.ms) : nullptr, own_map ? data<uint16_t>(c.mc) : nullptr,
+        k > 0 ? data<uint8_t>(c.k_index) : nullptr, k > 0 ? data<uint8_t>(c.k_oval) : nullptr, data<uint8_t>(c.v_main),
+        data(c.v_scale), data<uint16_t>(c.v_zp), data(c.rt), rt.stride(0), data(c.rg), rg.stride(0),
+        rt.scalar_type() == at::kLong, data<int32_t>(c.seq), al, al_b, al_h, al_s, B, Hq, Hkv, D, ps, k,
+        c.bitmap ? OMMX_INDEX_BITMAP : OMMX_INDEX_RELIDX7, scale_bf16, gt, gc, v_bf16, S, c.sm_scale, c.cap, c.off,
+        c.gbase, pages, slots, data<int32_t>(c.err), stream);
+    if (rc == 0 && hist) {
+        const ommx::HistTail t{data<uint16_t>(kt), data<uint16_t>(vt), kt->stride(0), static_cast<int>(kt->size(1)),
+                               data<int64_t>(c.hist_seq), data<int64_t>(c.hist_slots), static_cast<int>(c.ring_sink),
+                               static_cast<int>(c.ring_span), static_cast<int>(c.win_sink), static_cast<int>(c.win_recent)};
+        rc2 = ommx::decode_combine_hist(al, al_b, al_h, al_s, qp, q.stride(0), q.stride(1), t, data(c.o), o_bf16,
+                                        c.o->stride(0), c.o->stride(1), lse, c.lse ? c.lse->stride(0) : Hq, B, Hq, Hkv,
+                                        D, S, gt, c.sm_scale, c.cap, stream);
+    } else if (rc == 0) {
+        rc2 = ommx_decode_combine(
+            al, al_b, al_h, al_s, qp, q.stride(0), q.stride(1), tail ? data<uint16_t>(kt) : nullptr,
+            tail ? data<uint16_t>(vt) : nullptr, tail ? kt->stride(0) : 0, tail ? kt->stride(1) : 0,
+            tail ? kt->stride(2) : 0, tail ? vt->stride(0) : 0, tail ? vt->stride(1) : 0, tail ? vt->stride(2) : 0,
+            tail ? data<int32_t>(c.b_tail) : nullptr, data<int32_t>(c.seq), data<float>(c.o), c.o->stride(0),
+            c.o->stride(1), lse, c.lse->stride(0), B, Hq, Hkv, D, S, gt, tail ? kt->size(1) : 0, c.sm_scale, c.cap,
+            stream);
+    }
+    Py_END_ALLOW_THREADS
+    return failed(rc, "ommx_decode_splitkv") || failed(rc2, "ommx_decode_combine") ? -1 : 1;
+}
+
+PyObject* answer(int rc) {
+    if (rc < 0) return nullptr;
+    return PyBool_FromLong(rc);
+}
+
+// The arguments of ommx_paged_decode_attention_canonical, in the order of DecodeArg.
 PyObject* py_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != A_COUNT) { PyErr_SetString(PyExc_TypeError, "decode: wrong number of arguments"); return nullptr; }
     bool ok = true;
-    const at::Tensor *q = as_tensor(a[A_Q], ok), *k_base = as_tensor(a[A_KBASE], ok),
-                     *k_scale = as_tensor(a[A_KSCALE], ok), *k_zp = as_tensor(a[A_KZP], ok),
-                     *k_oidx = as_tensor_or_none(a[A_KOIDX], ok), *k_oval = as_tensor_or_none(a[A_KOVAL], ok),
-                     *v_main = as_tensor(a[A_VMAIN], ok), *v_scale = as_tensor(a[A_VSCALE], ok),
-                     *v_zp = as_tensor(a[A_VZP], ok), *k_tail = as_tensor_or_none(a[A_KTAIL], ok),
-                     *v_tail = as_tensor_or_none(a[A_VTAIL], ok), *b_tail = as_tensor_or_none(a[A_BTAIL], ok),
-                     *o = as_tensor(a[A_O], ok), *lse = as_tensor(a[A_LSE], ok), *rt = as_tensor(a[A_RT], ok),
-                     *rg = as_tensor(a[A_RG], ok), *seq = as_tensor(a[A_SEQ], ok),
-                     *k_obmp = as_tensor_or_none(a[A_KOBMP], ok), *ms = as_tensor_or_none(a[A_MS], ok),
-                     *mc = as_tensor_or_none(a[A_MC], ok), *ws = as_tensor_or_none(a[A_WS], ok),
-                     *err = as_tensor_or_none(a[A_ERR], ok);
-    const double sm_scale = as_double(a[A_SM], ok), cap = as_double(a[A_CAP], ok);
-    const int64_t ps = as_int(a[A_PS], ok), k = as_int(a[A_KOUT], ok), off = as_int(a[A_OFF], ok),
-                  gbase = as_int(a[A_GBASE], ok);
-    const bool bitmap = as_bool(a[A_BITMAP], ok), int8 = as_bool(a[A_INT8], ok), force = as_bool(a[A_FORCE], ok);
-    const bool combinadic = as_bool(a[A_COMBI], ok), want_map = as_bool(a[A_MAP], ok);
-    const int64_t given_splits = a[A_SPLITS] == Py_None ? 0 : as_int(a[A_SPLITS], ok);
-    const int64_t max_seq = a[A_MAXSEQ] == Py_None ? -1 : std::max<int64_t>(1, as_int(a[A_MAXSEQ], ok));
-    const int64_t max_tail = a[A_MAXTAIL] == Py_None ? 1 : as_int(a[A_MAXTAIL], ok);
-    const double mean = a[A_MEAN] == Py_None ? -1.0 : as_double(a[A_MEAN], ok);
-    ok = ok && !combinadic && (is_word(a[A_KFMT], "i2f4") || is_word(a[A_KFMT], "itf4"));
-    if (!ok) Py_RETURN_FALSE;
-
-    // geometry of the planes
-    if (q->dim() != 3 || k_base->dim() != 4 || k_scale->dim() != 3 || v_main->dim() != 4 || v_scale->dim() != 4 ||
-        v_zp->dim() != 4 || ps < 1)
-        Py_RETURN_FALSE;
-    const c10::Device dev = q->device();
-    if (!dev.is_cuda()) Py_RETURN_FALSE;
-    const int64_t pages = k_base->size(0), slots = k_scale->size(0), B = q->size(0), Hq = q->size(1),
-                  Hkv = k_base->size(2), D = k_base->size(3) * 4;
-    const int64_t gt = (pages == 0 || slots == 0) ? 32 : pages * ps / slots;
-    const bool v_bf16 = v_main->scalar_type() == at::kBFloat16;
-    const int64_t v_width = v_bf16 ? v_main->size(3) : v_main->size(3) * 4, per_row = v_scale->size(3);
-    const int64_t gc = per_row == 0 ? 32 : v_width / per_row;
-    if (!is_group_size(gt) || !is_group_size(gc) || v_width % gc || B < 1 || Hkv < 1 || Hq < Hkv || Hq % Hkv ||
-        v_width != D || (D != 64 && D != 128) || q->size(2) != D || gt % ps || pages > INT32_MAX || slots > INT32_MAX)
-        Py_RETURN_FALSE;
-    const int64_t R = Hq / Hkv;
-    if (R != 1 && R != 2 && R != 4 && R != 8) Py_RETURN_FALSE;
-    for (const at::Tensor* t : {k_base, v_main, v_scale, v_zp})
-        if (!t->is_contiguous() || t->size(0) != pages || t->size(1) != ps || t->size(2) != Hkv) Py_RETURN_FALSE;
-    if (!is_shape3(*k_scale, slots, Hkv, D) || !is_shape3(*k_zp, slots, Hkv, D) ||
-        k_zp->scalar_type() != at::kBFloat16 || !is_shape3(*o, B, Hq, D) || lse->dim() != 2 || lse->size(0) != B ||
-        lse->size(1) != Hq)
-        Py_RETURN_FALSE;
-    const at::ScalarType st = k_scale->scalar_type();
-    const bool scale_bf16 = st == at::kBFloat16;
-    if (st != v_scale->scalar_type() || (st != at::kChar && !scale_bf16) || scale_bf16 == int8) Py_RETURN_FALSE;
-    if (q->scalar_type() != at::kBFloat16 || q->stride(2) != 1) Py_RETURN_FALSE;
-
-    // lengths, tables, outputs
-    if (seq->numel() < B || !seq->is_contiguous() || seq->scalar_type() != at::kInt) Py_RETURN_FALSE;
-    if (b_tail && (b_tail->numel() < B || !b_tail->is_contiguous() || b_tail->scalar_type() != at::kInt)) Py_RETURN_FALSE;
-    if (rt->dim() != 2 || rg->dim() != 2 || rt->size(0) < B || rg->size(0) < B ||
-        rt->scalar_type() != rg->scalar_type() || (rt->scalar_type() != at::kInt && rt->scalar_type() != at::kLong) ||
-        rt->stride(1) != 1 || rg->stride(1) != 1)
-        Py_RETURN_FALSE;
-    if (o->scalar_type() != at::kFloat || lse->scalar_type() != at::kFloat || o->stride(2) != 1 || lse->stride(1) != 1)
-        Py_RETURN_FALSE;
-    for (const at::Tensor* t : {k_base, k_scale, v_main, o, lse, rt, rg, seq})
-        if (!on(t, dev)) Py_RETURN_FALSE;
-    if (off < 0 || off >= ps || gbase < 0) Py_RETURN_FALSE;
-
-    // outliers
-    const at::Tensor* k_index = bitmap ? k_obmp : k_oidx;
-    const bool own_map = want_map && k > 0;
-    if (k < 0 || k > 16 || (bitmap && k > 8)) Py_RETURN_FALSE;
-    if (k > 0) {
-        const int64_t index_bytes = bitmap ? (gt + 7) / 8 : (7 * k + 7) / 8;
-        for (const at::Tensor* t : {k_oval, k_index})
-            if (!t || t->scalar_type() != at::kByte || t->dim() != 4 || t->size(0) != slots || t->size(1) != Hkv ||
-                t->size(2) != D || t->size(3) != (t == k_oval ? (k + 1) / 2 : index_bytes) || !t->is_contiguous())
-                Py_RETURN_FALSE;
+    DecodeCall c;
+    c.q = as_tensor(a[A_Q], ok); c.k_base = as_tensor(a[A_KBASE], ok); c.k_scale = as_tensor(a[A_KSCALE], ok);
+    c.k_zp = as_tensor(a[A_KZP], ok); c.k_oval = as_tensor_or_none(a[A_KOVAL], ok);
+    c.v_main = as_tensor(a[A_VMAIN], ok); c.v_scale = as_tensor(a[A_VSCALE], ok); c.v_zp = as_tensor(a[A_VZP], ok);
+    c.k_tail = as_tensor_or_none(a[A_KTAIL], ok); c.v_tail = as_tensor_or_none(a[A_VTAIL], ok);
+    c.b_tail = as_tensor_or_none(a[A_BTAIL], ok); c.o = as_tensor(a[A_O], ok); c.lse = as_tensor(a[A_LSE], ok);
+    c.rt = as_tensor(a[A_RT], ok); c.rg = as_tensor(a[A_RG], ok); c.seq = as_tensor(a[A_SEQ], ok);
+    c.ms = as_tensor_or_none(a[A_MS], ok); c.mc = as_tensor_or_none(a[A_MC], ok);
+    c.ws = as_tensor_or_none(a[A_WS], ok); c.err = as_tensor_or_none(a[A_ERR], ok);
+    c.sm_scale = as_double(a[A_SM], ok); c.cap = as_double(a[A_CAP], ok);
+    c.ps = as_int(a[A_PS], ok); c.k = as_int(a[A_KOUT], ok); c.off = as_int(a[A_OFF], ok); c.gbase = as_int(a[A_GBASE], ok);
+    c.bitmap = as_bool(a[A_BITMAP], ok); c.int8 = as_bool(a[A_INT8], ok); c.force = as_bool(a[A_FORCE], ok);
+    c.want_map = as_bool(a[A_MAP], ok);
+    if (a[A_SPLITS] != Py_None) {
+        c.splits = as_int(a[A_SPLITS], ok);
+        if (c.splits < 1) ok = false;
     }
-    if (own_map && (!ms || !mc)) Py_RETURN_FALSE;
-    for (const at::Tensor* t : {ms, mc})
-        if (t && (!t->is_contiguous() ||
-                  (own_map && (t->scalar_type() != at::kBFloat16 || !is_shape3(*t, slots, Hkv, D)))))
-            Py_RETURN_FALSE;
-    if (!k_scale->is_contiguous() || !k_zp->is_contiguous()) Py_RETURN_FALSE;
-
-    // tail
-    const bool tail = gbase == 0 && k_tail && v_tail && b_tail && k_tail->dim() == 4 && k_tail->size(1) > 0 && max_tail > 0;
-    if (gbase == 0 && k_tail && v_tail && b_tail && k_tail->dim() != 4) Py_RETURN_FALSE;
-    if (tail && (k_tail->scalar_type() != at::kBFloat16 || v_tail->scalar_type() != at::kBFloat16 ||
-                 k_tail->stride(3) != 1 || v_tail->dim() != 4 || v_tail->stride(3) != 1 ||
-                 k_tail->sizes() != v_tail->sizes() || k_tail->size(0) < B || k_tail->size(2) != Hkv ||
-                 k_tail->size(3) != D))
-        Py_RETURN_FALSE;
-    if (err && (err->scalar_type() != at::kInt || !on(err, dev))) Py_RETURN_FALSE;
-
-    // splits and the workspace of their partial states
-    if (given_splits < 0 || (a[A_SPLITS] == Py_None && max_seq < 0)) Py_RETURN_FALSE;
-    int64_t S = std::max<int64_t>(1, given_splits);
-    if (a[A_SPLITS] == Py_None) {
-        // The serving-recipe kernel keeps three workgroups per compute unit resident with up to 4 q heads per
-        // kv head (two with 8, and so do the other kernels); at head_dim 64 one of its waves takes a pair of kv heads.
-        const bool plain_planes = gt == 32 && gc == 32 && !scale_bf16 && !v_bf16 && !force;
-        const bool lean = plain_planes && ((D == 128 && R <= 4 && k == 6) ||
-                                           (bitmap && k >= 1 && k <= 6 && ((D == 128 && R <= 4) ||
-                                                                           (D == 64 && R <= 2 && Hkv % 2 == 0))));
-        const bool paired = plain_planes && D == 64 && bitmap && k >= 1 && k <= 8 && R <= 4 && Hkv % 2 == 0;
-        S = auto_splits(max_seq, B, paired ? Hkv / 2 : Hkv, cu_count(dev.index()), gt, mean, lean ? 3 : 2);
-    }
-    if (ws && (ws->scalar_type() != at::kFloat || ws->dim() != 4 || ws->size(0) != B || ws->size(1) != Hq ||
-               ws->size(2) < S || ws->size(3) < D + 1 || ws->stride(3) != 1))
-        Py_RETURN_FALSE;
-
-    c10::hip::HIPGuard guard(dev.index());
-    hipStream_t stream = c10::hip::getCurrentHIPStream(dev.index()).stream();
-    int64_t al_b = Hq * (S + 1) * (D + 1), al_h = (S + 1) * (D + 1), al_s = D + 1;
-    c10::DataPtr scratch;
-    float* al;
-    if (ws) {
-        al = ws->data_ptr<float>();
-        al_b = ws->stride(0); al_h = ws->stride(1); al_s = ws->stride(2);
-    } else {
-        scratch = c10::GetAllocator(c10::DeviceType::CUDA)->allocate(static_cast<size_t>(B * al_b) * sizeof(float));
-        al = static_cast<float*>(scratch.get());
-    }
-    const uint16_t* qp = data<const uint16_t>(q);
-    int rc, rc2 = 0;
-    Py_BEGIN_ALLOW_THREADS
-    rc = (force ? ommx_decode_splitkv_ref : ommx_decode_splitkv)(
-        qp, q->stride(0), q->stride(1), data<uint8_t>(k_base), data(k_scale), data<uint16_t>(k_zp),
-        own_map ? data<uint16_t>(ms) : nullptr, own_map ? data<uint16_t>(mc) : nullptr,
-        k > 0 ? data<uint8_t>(k_index) : nullptr, k > 0 ? data<uint8_t>(k_oval) : nullptr, data<uint8_t>(v_main),
-        data(v_scale), data<uint16_t>(v_zp), data(rt), rt->stride(0), data(rg), rg->stride(0),
-        rt->scalar_type() == at::kLong, data<int32_t>(seq), al, al_b, al_h, al_s, B, Hq, Hkv, D, ps, k,
-        bitmap ? OMMX_INDEX_BITMAP : OMMX_INDEX_RELIDX7, scale_bf16, gt, gc, v_bf16, S, sm_scale, cap, off, gbase,
-        pages, slots, data<int32_t>(err), stream);
-    if (rc == 0)
-        rc2 = ommx_decode_combine(
-            al, al_b, al_h, al_s, qp, q->stride(0), q->stride(1), tail ? data<uint16_t>(k_tail) : nullptr,
-            tail ? data<uint16_t>(v_tail) : nullptr, tail ? k_tail->stride(0) : 0, tail ? k_tail->stride(1) : 0,
-            tail ? k_tail->stride(2) : 0, tail ? v_tail->stride(0) : 0, tail ? v_tail->stride(1) : 0,
-            tail ? v_tail->stride(2) : 0, tail ? data<int32_t>(b_tail) : nullptr, data<int32_t>(seq),
-            data<float>(o), o->stride(0), o->stride(1), data<float>(lse), lse->stride(0), B, Hq, Hkv, D, S, gt,
-            tail ? k_tail->size(1) : 0, sm_scale, cap, stream);
-    Py_END_ALLOW_THREADS
-    if (failed(rc, "ommx_decode_splitkv") || failed(rc2, "ommx_decode_combine")) return nullptr;
-    Py_RETURN_TRUE;
+    if (a[A_MAXSEQ] != Py_None) c.max_seq = std::max<int64_t>(1, as_int(a[A_MAXSEQ], ok));
+    if (a[A_MAXTAIL] != Py_None) c.max_tail = as_int(a[A_MAXTAIL], ok);
+    if (a[A_MEAN] != Py_None) c.mean = as_double(a[A_MEAN], ok);
+    c.k_index = as_tensor_or_none(a[c.bitmap ? A_KOBMP : A_KOIDX], ok);
+    const bool combinadic = as_bool(a[A_COMBI], ok);
+    if (!ok || combinadic || (!is_word(a[A_KFMT], "i2f4") && !is_word(a[A_KFMT], "itf4"))) Py_RETURN_FALSE;
+    return answer(run_decode(c));
 }
 
 // ── stores ─────────────────────────────────────────────────────────────────────────────────────
 
-hipStream_t stream_of(c10::Device dev) { return c10::hip::getCurrentHIPStream(dev.index()).stream(); }
 bool is_index(const at::Tensor* t, c10::Device dev, at::ScalarType type, int64_t n) {
     return !t || (t->scalar_type() == type && t->is_contiguous() && t->numel() >= n && t->device() == dev);
 }
@@ -312,6 +364,7 @@ struct Planes {
                      *index = nullptr, *oval = nullptr, *v_main = nullptr, *v_scale = nullptr, *v_zp = nullptr;
 };
 PyObject* g_names[11];      // interned keys of a plane dict
+PyObject* g_bitmap;
 enum { N_KBASE, N_KSCALE, N_KZP, N_MS, N_MC, N_OBMP, N_OIDX, N_OVAL, N_VMAIN, N_VSCALE, N_VZP };
 
 bool read_planes(PyObject* d, const Recipe& r, Planes& p) {
@@ -597,26 +650,54 @@ PyObject* py_pack_groups(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Py_RETURN_TRUE;
 }
 
-// (dst, values): a contiguous int64 or int32 tensor on the GPU filled from a list of ints, by a launch
+// (q, planes, k_hist, v_hist, slots, seq, b_seq_len, req_to_token, req_to_group, out, sm_scale, page_size, max_seq_len,
+//  mean_seq_len, ring sink, ring span, window sink, window recent, plain kernel, err_flag, recipe x 8): decode over a
+// pool's planes with the tail rows read in place from its history; out bf16 or fp32
+PyObject* py_decode_pool(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 28) { PyErr_SetString(PyExc_TypeError, "decode_pool: wrong number of arguments"); return nullptr; }
+    bool ok = true;
+    DecodeCall c;
+    Recipe r;
+    Planes p;
+    // a cache of ranks keeps the bitmask beside them as what the kernels read
+    PyObject* recipe[8];
+    std::copy(a + 20, a + 28, recipe);
+    if (is_word(recipe[3], "combinadic")) recipe[3] = g_bitmap;
+    if (!read_recipe(recipe, r) || !read_planes(a[1], r, p)) Py_RETURN_FALSE;
+    c.q = as_tensor(a[0], ok); c.k_tail = as_tensor(a[2], ok); c.v_tail = as_tensor(a[3], ok);
+    c.hist_slots = as_tensor_or_none(a[4], ok); c.hist_seq = as_tensor(a[5], ok); c.seq = as_tensor(a[6], ok);
+    c.rt = as_tensor(a[7], ok); c.rg = as_tensor(a[8], ok); c.o = as_tensor(a[9], ok);
+    c.sm_scale = as_double(a[10], ok); c.ps = as_int(a[11], ok); c.max_seq = std::max<int64_t>(1, as_int(a[12], ok));
+    if (a[13] != Py_None) c.mean = as_double(a[13], ok);
+    c.ring_sink = as_int(a[14], ok); c.ring_span = as_int(a[15], ok); c.win_sink = as_int(a[16], ok);
+    c.win_recent = as_int(a[17], ok); c.force = as_bool(a[18], ok); c.err = as_tensor_or_none(a[19], ok);
+    if (!ok) Py_RETURN_FALSE;
+    c.k_base = p.k_base; c.k_scale = p.k_scale; c.k_zp = p.k_zp; c.k_index = p.index; c.k_oval = p.oval;
+    c.v_main = p.v_main; c.v_scale = p.v_scale; c.v_zp = p.v_zp; c.ms = p.ms; c.mc = p.mc;
+    c.k = r.k; c.bitmap = r.bitmap; c.want_map = p.ms != nullptr; c.int8 = r.mode == OMMX_SCALE_POW2_INT8;
+    return answer(run_decode(c));
+}
+
+// (dst, values, n64 = all or none): a contiguous GPU tensor filled from a list of ints by a launch.  int64 and int32
+// tensors take one entry per value; an int32 tensor with n64 given holds n64 int64 values first, then int32 ones.
 PyObject* py_upload(PyObject*, PyObject* const* a, Py_ssize_t n) {
-    if (n != 2) { PyErr_SetString(PyExc_TypeError, "upload: wrong number of arguments"); return nullptr; }
+    if (n != 2 && n != 3) { PyErr_SetString(PyExc_TypeError, "upload: wrong number of arguments"); return nullptr; }
     bool ok = true;
     const at::Tensor* dst = as_tensor(a[0], ok);
     std::vector<int64_t> values;
-    if (!ok || !dst->is_cuda() || !dst->is_contiguous() || !read_ints(a[1], values) ||
-        dst->numel() != static_cast<int64_t>(values.size()) ||
-        (dst->scalar_type() != at::kLong && dst->scalar_type() != at::kInt))
+    if (!ok || !dst->is_cuda() || !dst->is_contiguous() || !read_ints(a[1], values)) Py_RETURN_FALSE;
+    const int64_t count = static_cast<int64_t>(values.size());
+    const bool wide = dst->scalar_type() == at::kLong;
+    if (!wide && dst->scalar_type() != at::kInt) Py_RETURN_FALSE;
+    const int64_t n64 = n == 3 ? as_int(a[2], ok) : (wide ? count : 0);
+    if (!ok || n64 < 0 || n64 > count || (wide && n64 != count) || dst->numel() * (wide ? 2 : 1) != count + n64)
         Py_RETURN_FALSE;
+    std::vector<int32_t> words(static_cast<size_t>(count + n64));
+    std::memcpy(words.data(), values.data(), static_cast<size_t>(n64) * 8);
+    std::copy(values.begin() + n64, values.end(), words.begin() + 2 * n64);
     c10::hip::HIPGuard guard(dst->device().index());
-    hipStream_t stream = stream_of(dst->device());
-    int rc;
-    if (dst->scalar_type() == at::kLong) {
-        rc = ommx::upload_words(static_cast<int32_t*>(dst->data_ptr()), reinterpret_cast<const int32_t*>(values.data()),
-                                static_cast<int>(2 * values.size()), stream);
-    } else {
-        const std::vector<int32_t> words(values.begin(), values.end());
-        rc = ommx::upload_words(static_cast<int32_t*>(dst->data_ptr()), words.data(), static_cast<int>(words.size()), stream);
-    }
+    const int rc = ommx::upload_words(static_cast<int32_t*>(dst->data_ptr()), words.data(),
+                                      static_cast<int>(words.size()), stream_of(dst->device()));
     if (failed(rc, "upload")) return nullptr;
     Py_RETURN_TRUE;
 }
@@ -632,7 +713,7 @@ PyObject* guarded(PyObject* self, PyObject* const* a, Py_ssize_t n) {
 #define OMMX_FAST(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(guarded<py_##name>)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
     OMMX_FAST(auto_num_kv_splits),
-    OMMX_FAST(decode), OMMX_FAST(store_pack), OMMX_FAST(pack_block), OMMX_FAST(pack_groups), OMMX_FAST(ring_write),
+    OMMX_FAST(decode), OMMX_FAST(decode_pool), OMMX_FAST(store_pack), OMMX_FAST(pack_block), OMMX_FAST(pack_groups), OMMX_FAST(ring_write),
     OMMX_FAST(tail_gather), OMMX_FAST(rows_write), OMMX_FAST(upload),
     {nullptr, nullptr, 0, nullptr},
 };
@@ -646,5 +727,6 @@ PyMODINIT_FUNC PyInit__ommx_host(void) {
                            "k_oidx", "k_oval", "v_main", "v_scale", "v_zp"};
     for (int i = 0; i < 11; ++i)
         if (!(g_names[i] = PyUnicode_InternFromString(names[i]))) return nullptr;
+    if (!(g_bitmap = PyUnicode_InternFromString("bitmap"))) return nullptr;
     return PyModule_Create(&module);
 }

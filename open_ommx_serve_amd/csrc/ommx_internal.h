@@ -37,4 +37,20 @@ int pack_list(const int32_t* host_pairs, int n, int32_t* src_rows, int32_t* dst_
               int ppg, int hist_rows, int sink, int span, int window_sink, int groups_per_seq, int pages_per_seq,
               void* stream);
 
+// Split combine with the tail rows read in place from a bf16 row history [requests, rows, Hkv, D]: positions
+// [0, min(win_sink, seq)) ++ [boundary, seq) of every request through the ring map, boundary being what
+// ommx_tail_gather computes without a lag.  Saves the gather launch and the gathered copy.  o is fp32, or bf16
+// rounded as torch does.
+struct HistTail {
+    const uint16_t *k, *v;
+    int64_t stride_req;             // elements between the histories of two requests
+    int rows;
+    const int64_t *seq, *slots;     // device: [B] lengths, [B] history of each request (NULL: b)
+    int ring_sink, ring_span, win_sink, win_recent;
+};
+int decode_combine_hist(const float* attn_logits, int64_t al_b, int64_t al_h, int64_t al_s, const uint16_t* q,
+                        int64_t q_b, int64_t q_h, const HistTail& tail, void* o, bool o_bf16, int64_t o_b, int64_t o_h,
+                        float* lse, int64_t lse_b, int B, int Hq, int Hkv, int D, int num_splits, int group_tokens,
+                        float sm_scale, float logit_cap, void* stream);
+
 }  // namespace ommx

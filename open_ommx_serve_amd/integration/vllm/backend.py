@@ -34,8 +34,7 @@ import torch
 from ...attention.kv_store import CanonicalKVStore
 from ...attention.reference_op import ommx_paged_decode
 from .config import OMMXServingConfig, resolve_serving_config
-from .metadata import (STEP_ROUTE_UNCLASSIFIED, OMMXBatchedStepManager, OMMXStepManager,
-                       detect_full_prefill, detect_step_route)
+from .metadata import STEP_ROUTE_UNCLASSIFIED, OMMXBatchedStepManager, OMMXStepManager, StepShape
 
 try:                                                     # engine present: real bases
     from vllm.v1.attention.backends.flash_attn import (FlashAttentionBackend as _BackendBase,
@@ -135,12 +134,13 @@ class OMMXCanonicalMetadataBuilder(_BuilderBase):
         """Route decisions of one step (``backend.py:1080-1151``)."""
         s = _STATE
         s.last_common = common
-        B, uniform = detect_step_route(common)
+        shape = StepShape.of_step(common)
+        B, uniform = shape.batch, shape.batch >= 1 and shape.one_token_each
         st = s.step
         st["B"], st["uniform"] = int(B), bool(uniform)
         if B == STEP_ROUTE_UNCLASSIFIED and (s.graph or s.batched_graph):
             raise RuntimeError("OMMX refuses graph replay with unclassified batch metadata")
-        st["full_prefill"] = detect_full_prefill(common)
+        st["full_prefill"] = shape.whole_sequences
         if s.graph and B > 1:
             raise RuntimeError(
                 "OMMX_ATTN_GRAPH supports one request only; restart with OMMX_ATTN_GRAPH=0 and "
@@ -161,7 +161,7 @@ class OMMXCanonicalMetadataBuilder(_BuilderBase):
                 raise RuntimeError("OMMX refuses to decode with stale KV metadata: "
                                    f"{s.manager.dead_reason}")
         if in_batched and s.bmanager is not None:
-            s.bmanager.on_build(common)
+            s.bmanager.on_build(common, shape=shape if shape.lengths is not None else None)
             if s.bmanager.dead:
                 raise RuntimeError("OMMX refuses to serve this step from the batched pool: "
                                    f"{s.bmanager.dead_reason}")
@@ -303,14 +303,15 @@ class OMMXCanonicalImpl(_ImplBase):
             bounds = list(range(B + 1))
         else:
             raise RuntimeError(f"batched write: cannot map {n} tokens to {B} requests")
-        uniform = n == B and all(bounds[i + 1] - bounds[i] == 1 for i in range(B))
-        if uniform and not any(int(mgr.seq_lens[i]) - 1 <= 0 for i in range(B)):
-            for i, slot in enumerate(mgr.slots):
-                if int(pool.seq_len[slot]) != int(mgr.seq_lens[i]) - 1:
+        uniform = n == B and (mgr.is_uniform_decode or all(bounds[i + 1] - bounds[i] == 1 for i in range(B)))
+        if uniform and min(mgr.seq_lens) > 1:
+            for slot, seq in zip(mgr.slots, mgr.seq_lens):
+                if pool.seq_len[slot] != seq - 1:
                     raise RuntimeError(
                         f"batched write: slot {slot} holds {pool.seq_len[slot]} tokens but the "
-                        f"scheduler reports {mgr.seq_lens[i]} after this step")
-            pool.append_decode_batched(mgr.slots, key, value)
+                        f"scheduler reports {seq} after this step")
+            step = mgr.step_on_device(pool)
+            pool.append_decode_rows(mgr.slots, step.sel, step.col, key, value)
             return
         for i in range(B):
             slot = mgr.slots[i]
@@ -427,6 +428,12 @@ class OMMXCanonicalImpl(_ImplBase):
         layer._ommx_ws_cache = ws
         return ws
 
+    def _reads_what_was_stored(self) -> bool:
+        """Whether the decode reads the index plane that the store wrote, which is every configuration
+        but the A/B overrides."""
+        cfg = self._ommx_cfg()
+        return cfg.bitmap_read is None and cfg.combinadic_read is None
+
     def _decode(self, layer, q, out, bundle, max_seq_len) -> None:
         B = int(q.shape[0])
         ws = self._ommx_ws(layer, B, max_seq_len, q.device)
@@ -450,6 +457,12 @@ class OMMXCanonicalImpl(_ImplBase):
                                f"{getattr(mgr, 'dead_reason', None) or 'no prefill reached it'}")
         ws = getattr(layer, "_ommx_single_ws", None)
         T = mgr.max_tail_cap
+        # outside graph capture the split count may follow the actual length
+        if self._reads_what_was_stored() and store.decode_into(
+                q[:1], out[:1], mgr.seq_dev, mgr.b_seq_len, sm_scale=self.scale,
+                max_seq_len=mgr.max_seq_len if _STATE.graph else max(1, mgr.cur_packed)):
+            _STATE.fires["single"] += 1
+            return
         if ws is None:
             ws = {"kt": torch.zeros(1, T, store.H, store.D, dtype=torch.bfloat16, device=q.device)}
             ws["vt"] = torch.zeros_like(ws["kt"])
@@ -470,6 +483,14 @@ class OMMXCanonicalImpl(_ImplBase):
         if pool is None:
             raise RuntimeError("[ommx] batched decode before any write reached this layer's pool")
         B = len(mgr.slots)
+        # (a pool that is not at the scheduler's lengths is read at its own, below)
+        in_step = self._reads_what_was_stored() and [pool.seq_len[x] for x in mgr.slots] == mgr.seq_lens
+        step = mgr.step_on_device(pool) if in_step else None
+        if step is not None and pool.decode_into(
+                q[:B], out[:B], step.sel, step.cur, step.packed, step.tables, sm_scale=self.scale,
+                max_seq_len=step.max_packed, mean_seq_len=step.mean_packed):
+            _STATE.fires["batched"] += 1
+            return
         bundle = pool.decode_inputs_batched(mgr.slots)
         self._decode(layer, q[:B], out, bundle, bundle["max_seq_len"])
         _STATE.fires["batched"] += 1
