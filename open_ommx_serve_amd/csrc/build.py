@@ -30,6 +30,7 @@ SOURCES = {
     "ommx_ring.hip": [],
     "ommx_merge.hip": [],
     "ommx_index.hip": [],
+    "ommx_prefill.hip": [],
     "ommx_capi.hip": [],
 }
 COMMON = ["-O3", "-fPIC", "-std=c++17", f"--offload-arch={ARCH}",

@@ -678,6 +678,42 @@ PyObject* py_decode_pool(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return answer(run_decode(c));
 }
 
+// (q, k, v, out, starts, scale): causal attention of prompt rows, out fp32 or bf16
+PyObject* py_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 6) { PyErr_SetString(PyExc_TypeError, "prefill: wrong number of arguments"); return nullptr; }
+    bool ok = true;
+    const at::Tensor *q = as_tensor(a[0], ok), *k = as_tensor(a[1], ok), *v = as_tensor(a[2], ok), *o = as_tensor(a[3], ok);
+    std::vector<int64_t> starts;
+    const double scale = as_double(a[5], ok);
+    if (!ok || !read_ints(a[4], starts) || starts.size() < 2 || starts[0] < 0 || !q->is_cuda()) Py_RETURN_FALSE;
+    for (size_t i = 1; i < starts.size(); ++i)
+        if (starts[i] < starts[i - 1]) Py_RETURN_FALSE;
+    for (const at::Tensor* t : {q, k, v, o})
+        if (t->dim() != 3 || t->stride(2) != 1 || t->device() != q->device() || t->size(0) < starts.back()) Py_RETURN_FALSE;
+    const int64_t Hq = q->size(1), Hkv = k->size(1), D = q->size(2);
+    if (k->size(2) != D || v->size(2) != D || v->size(1) != Hkv || o->size(1) != Hq || o->size(2) != D ||
+        (D != 64 && D != 128) || Hkv < 1 || Hq % Hkv || !(scale > 0))
+        Py_RETURN_FALSE;
+    for (const at::Tensor* t : {q, k, v, o}) {
+        const bool is16 = t->scalar_type() == at::kBFloat16;
+        if ((!is16 && (t != o || t->scalar_type() != at::kFloat)) || t->stride(0) % 8 || t->stride(1) % 8 ||
+            (reinterpret_cast<uintptr_t>(t->data_ptr()) & 15))
+            Py_RETURN_FALSE;
+    }
+    if (starts.back() == starts[0]) Py_RETURN_TRUE;
+    c10::hip::HIPGuard guard(q->device().index());
+    hipStream_t stream = stream_of(q->device());
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = ommx::prefill_attention(data<uint16_t>(q), q->stride(0), q->stride(1), data<uint16_t>(k), k->stride(0),
+                                 k->stride(1), data<uint16_t>(v), v->stride(0), v->stride(1), data(o),
+                                 o->scalar_type() == at::kBFloat16, o->stride(0), o->stride(1), starts.data(),
+                                 static_cast<int>(starts.size()) - 1, Hq, Hkv, D, scale, stream);
+    Py_END_ALLOW_THREADS
+    if (failed(rc, "prefill_attention")) return nullptr;
+    Py_RETURN_TRUE;
+}
+
 // (dst, values, n64 = all or none): a contiguous GPU tensor filled from a list of ints by a launch.  int64 and int32
 // tensors take one entry per value; an int32 tensor with n64 given holds n64 int64 values first, then int32 ones.
 PyObject* py_upload(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -714,7 +750,7 @@ PyObject* guarded(PyObject* self, PyObject* const* a, Py_ssize_t n) {
 PyMethodDef methods[] = {
     OMMX_FAST(auto_num_kv_splits),
     OMMX_FAST(decode), OMMX_FAST(decode_pool), OMMX_FAST(store_pack), OMMX_FAST(pack_block), OMMX_FAST(pack_groups), OMMX_FAST(ring_write),
-    OMMX_FAST(tail_gather), OMMX_FAST(rows_write), OMMX_FAST(upload),
+    OMMX_FAST(tail_gather), OMMX_FAST(rows_write), OMMX_FAST(upload), OMMX_FAST(prefill),
     {nullptr, nullptr, 0, nullptr},
 };
 #undef OMMX_FAST

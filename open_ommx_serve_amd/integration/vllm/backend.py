@@ -31,6 +31,7 @@ from typing import Any, Callable, Dict, Optional
 
 import torch
 
+from ...attention import _hip
 from ...attention.kv_store import CanonicalKVStore
 from ...attention.reference_op import ommx_paged_decode
 from .config import OMMXServingConfig, resolve_serving_config
@@ -186,11 +187,13 @@ class OMMXCanonicalMetadataBuilder(_BuilderBase):
 # ── per-layer implementation ─────────────────────────────────────────────────────────────
 
 def causal_prefill_attention(query, key, value, q_start, scale, n_rep):
-    """Causal attention of each request over its own rows of a full-prefill step, fp32 math on
-    the device through torch (a library call; prefill is outside the decode path).
-    ``query [n, Hq, D]``, ``key`` / ``value [n, Hkv, D]``, ``q_start`` cumulative row offsets;
-    returns fp32 ``[n, Hq, D]``."""
+    """Causal attention of each request over its own rows of a full-prefill step, softmax weights of fp32
+    precision.  ``query [n, Hq, D]``, ``key`` / ``value [n, Hkv, D]``, ``q_start`` cumulative row offsets;
+    returns fp32 ``[n, Hq, D]``.  bf16 rows of head_dim 64 or 128 take the HIP kernel; anything
+    else goes through torch's attention in fp32."""
     out = torch.empty(query.shape, dtype=torch.float32, device=query.device)
+    if _prefill_into(query, key, value, q_start, scale, out):
+        return out
     for i in range(len(q_start) - 1):
         t0, t1 = int(q_start[i]), int(q_start[i + 1])
         if t1 <= t0:
@@ -201,6 +204,11 @@ def causal_prefill_attention(query, key, value, q_start, scale, n_rep):
         o = torch.nn.functional.scaled_dot_product_attention(q, k, v, is_causal=True, scale=scale)
         out[t0:t1] = o[0].transpose(0, 1)
     return out
+
+
+def _prefill_into(query, key, value, q_start, scale, out) -> bool:
+    """The HIP kernel writing ``out`` (fp32 or bf16) in place; False when it does not take the rows."""
+    return query.is_cuda and _hip.host().prefill(query, key, value, out, [int(x) for x in q_start], float(scale))
 
 
 class OMMXCanonicalImpl(_ImplBase):
@@ -377,6 +385,9 @@ class OMMXCanonicalImpl(_ImplBase):
         k = key.reshape(-1, self.num_kv_heads, D)
         v = value.reshape(-1, self.num_kv_heads, D)
         t0 = int(q_start[0])
+        if type(self).prefill_attention is causal_prefill_attention and _prefill_into(q, k, v, q_start, self.scale, out):
+            _STATE.fires["prefill"] += 1
+            return
         res = type(self).prefill_attention(q[t0:n], k[t0:n], v[t0:n], [x - t0 for x in q_start],
                                            self.scale, self.num_heads // self.num_kv_heads)
         out[t0:n].copy_(res)

@@ -1,0 +1,62 @@
+"""The prompt-attention kernel against causal softmax in fp64: request lengths around the 32-row
+wave, the 64-key and the 128-row tile, empty requests, rows that start past zero, every head
+grouping, both output types, and a batch whose tile list takes more than one launch."""
+import pytest
+import torch
+
+from open_ommx_serve_amd.attention import _hip
+from open_ommx_serve_amd.integration.vllm.backend import causal_prefill_attention
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _rows(n, H, D, seed):
+    return torch.randn(n, H, D, generator=torch.Generator(device=DEV).manual_seed(seed), device=DEV).to(torch.bfloat16)
+
+
+def _reference(q, k, v, starts, scale):
+    out = torch.full(q.shape, float("nan"), dtype=torch.float64, device=DEV)
+    rep = q.shape[1] // k.shape[1]
+    for a, b in zip(starts, starts[1:]):
+        Q, K, V = (t[a:b].double().transpose(0, 1).contiguous() for t in (q, k, v))
+        K, V = K.repeat_interleave(rep, 0), V.repeat_interleave(rep, 0)
+        s = Q @ K.transpose(1, 2).contiguous() * scale
+        s = s.masked_fill(torch.ones(b - a, b - a, dtype=torch.bool, device=DEV).triu(1), -float("inf"))
+        out[a:b] = (s.softmax(-1) @ V).transpose(0, 1)
+    return out
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("hq,hkv", [(4, 4), (8, 2), (8, 1), (6, 2)])
+@pytest.mark.parametrize("starts", [
+    [0, 1], [0, 31, 63, 64], [0, 32, 97], [2, 65, 65, 129], [0, 127, 255], [0, 128, 257], [0, 700], [5, 6, 390]])
+def test_prompt_attention_matches_causal_softmax(D, hq, hkv, starts):
+    n = starts[-1] + 3
+    q, k, v = _rows(n, hq, D, 1), _rows(n, hkv, D, 2), _rows(n, hkv, D, 3)
+    k[:, :, :3] *= 12
+    want = _reference(q, k, v, starts, D ** -0.5)
+    out = torch.full((n, hq, D), 7.0, device=DEV)
+    assert _hip.host().prefill(q, k, v, out, starts, D ** -0.5)
+    live = slice(starts[0], starts[-1])
+    assert (out[live].double() - want[live]).abs().max().item() <= 1e-5
+    assert bool((out[:starts[0]] == 7).all()) and bool((out[starts[-1]:] == 7).all())     # other rows untouched
+    half = torch.empty(n, hq, D, dtype=torch.bfloat16, device=DEV)
+    assert _hip.host().prefill(q, k, v, half, starts, D ** -0.5)
+    assert torch.equal(half[live], out[live].to(torch.bfloat16))
+
+
+def test_more_tiles_than_one_launch_lists():
+    starts = [*range(0, 330 * 3 + 1, 3)]                       # 330 requests of three rows
+    q, k, v = _rows(starts[-1], 2, 64, 4), _rows(starts[-1], 1, 64, 5), _rows(starts[-1], 1, 64, 6)
+    got = causal_prefill_attention(q, k, v, starts, 0.125, 2)
+    assert (got.double() - _reference(q, k, v, starts, 0.125)).abs().max().item() <= 1e-5
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.float32, 128), (torch.bfloat16, 96)])
+def test_rows_the_kernel_does_not_take_still_run(dtype, D):
+    q, k, v = (_rows(70, h, D, h).to(dtype) for h in (4, 2, 2))
+    out = torch.empty(70, 4, D, device=DEV)
+    assert not _hip.host().prefill(q, k, v, out, [0, 70], D ** -0.5)
+    got = causal_prefill_attention(q, k, v, [0, 70], D ** -0.5, 2)
+    assert (got.double() - _reference(q, k, v, [0, 70], D ** -0.5)).abs().max().item() <= 2e-5
