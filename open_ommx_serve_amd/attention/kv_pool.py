@@ -365,7 +365,9 @@ class MultiSeqKVPool:
             for r in slots:
                 if self.seq_len[r] >= self.max_seq_len:
                     raise RuntimeError(f"MultiSeqKVPool req {r} capacity {self.max_seq_len} exceeded")
-        self.append_decode_captured(rows, cols, K, V)
+        if not self._host.ring_write(self.k_hist, self.v_hist, cols, K, V, self._ring_sink, self._ring_rec, rows,
+                                     None, self.err_flag):
+            self.append_decode_captured(rows, cols, K, V)
         return self._advance_host_and_pack(slots)
 
     def append_decode_captured(self, rows: torch.Tensor, cols: torch.Tensor, K: torch.Tensor,

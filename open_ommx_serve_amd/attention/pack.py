@@ -429,7 +429,7 @@ def ommx_pack_kv_canonical_block(
     packed = T > 0 and repr_l != "combinadic" and _hip.host().pack_block(
         Kd, Vd, int(page_size), bool(kv_outlier_map), store_table(dev), k, gt, gc, repr_l, sel, *mode, vfmt)
     if packed:
-        (bits, k_base, k_scale, k_zp, k_index, k_oval, k_ms, k_mc, v_main, v_scale, v_zp, to_token, to_group) = packed
+        (flags, k_base, k_scale, k_zp, k_index, k_oval, k_ms, k_mc, v_main, v_scale, v_zp, to_token, to_group) = packed
         planes = {"k_base": k_base, "k_scale": k_scale, "k_zp": k_zp, "k_oidx": None, "k_crank": None, "k_obmp": None,
                   "k_oval": k_oval, "k_fp4_mapscale": k_ms, "k_fp4_mapcenter": k_mc,
                   "v_main": v_main, "v_scale": v_scale, "v_zp": v_zp}
@@ -444,14 +444,16 @@ def ommx_pack_kv_canonical_block(
                             outlier_repr=repr_l, outlier_select=outlier_select,
                             use_pow2=mode[0], kv_int8_scale=mode[1],
                             group_tokens=gt, group_channels=gc, v_format=vfmt)
-        bits = int(err.item())
+        raise_for_store_errors(int(err.item()))
         to_token = torch.arange(pages, dtype=torch.int32, device=dev).reshape(1, pages)
         to_group = torch.arange(G, dtype=torch.int32, device=dev).reshape(1, G)
-    if bits:
-        raise_for_store_errors(bits)
+    target = torch.device(device)
+    stays = target.type == "cuda" and dev.index == (torch.cuda.current_device() if target.index is None else target.index)
+    if packed and not stays:
+        raise_for_store_errors(_hip.host().block_errors(flags, Kd))
 
     def _to(t):
-        return t.to(device) if t is not None else None
+        return t if stays or t is None else t.to(device)
 
     out = {name: _to(planes[name]) for name in (
         "k_base", "k_scale", "k_zp", "k_oidx", "k_oval", "k_crank", "k_obmp",
@@ -470,6 +472,8 @@ def ommx_pack_kv_canonical_block(
         k_base_bits=2, oval_bits=4, use_pow2=bool(use_pow2),
         kv_outlier_map=bool(kv_outlier_map and k > 0),
         kv_int8_scale=bool(use_pow2) and bool(kv_int8_scale))
+    if packed and stays:                 # the dict above was put together while the kernel ran
+        raise_for_store_errors(_hip.host().block_errors(flags, Kd))
     return out
 
 

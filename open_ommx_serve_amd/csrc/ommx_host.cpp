@@ -11,6 +11,8 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/EmptyTensor.h>
+#include <ATen/hip/impl/HIPCachingAllocatorMasqueradingAsCUDA.h>
 #include <c10/core/Allocator.h>
 #include <c10/hip/HIPGuard.h>
 #include <c10/hip/HIPStream.h>
@@ -22,6 +24,7 @@
 #include <atomic>
 #include <cstring>
 #include <initializer_list>
+#include <mutex>
 #include <vector>
 
 #include "../../include/ommx_hip.h"
@@ -431,10 +434,34 @@ PyObject* py_store_pack(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Py_RETURN_TRUE;
 }
 
-// (K, V, page_size, kv_outlier_map, table, recipe x 8) -> (error bits, k_base, k_scale, k_zp, k_index, k_oval,
-// k_mapscale, k_mapcenter, v_main, v_scale, v_zp, req_to_token, req_to_group), or False.  Packs a block into planes
-// of its own with identity tables and waits for it: the error bits come back through host memory that the
-// kernel writes only when there is something to report, so the wait is the one host stop and nothing is copied.
+// Host-visible error words of block packing, OMMX_STORE_ERR_WORDS ints each.  A call takes a block and gives it back
+// when it has been read; at most kKeptFlags idle ones are kept (more go back to torch's pinned allocator).
+constexpr size_t kKeptFlags = 16;
+struct FlagPool {
+    std::mutex lock;
+    std::vector<at::Tensor> idle;
+};
+FlagPool& flag_pool() {
+    static FlagPool* const pool = new FlagPool;      // never destroyed: the runtime may be gone before static destructors
+    return *pool;
+}
+at::Tensor take_flags() {
+    at::Tensor t;
+    {
+        FlagPool& pool = flag_pool();
+        std::lock_guard<std::mutex> hold(pool.lock);
+        if (!pool.idle.empty()) { t = std::move(pool.idle.back()); pool.idle.pop_back(); }
+    }
+    if (!t.defined()) t = at::empty({OMMX_STORE_ERR_WORDS}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+    std::fill_n(t.data_ptr<int32_t>(), OMMX_STORE_ERR_WORDS, 0);
+    return t;
+}
+
+// (K, V, page_size, kv_outlier_map, table, recipe x 8) -> (flags, k_base, k_scale, k_zp, k_index, k_oval, k_mapscale,
+// k_mapcenter, v_main, v_scale, v_zp, req_to_token, req_to_group), or False.  Launches the packing of a block into planes
+// of its own with identity tables.  The caller does its own work and then asks block_errors(flags), the one host
+// stop: the error bits come back through host memory that the kernel writes only when there is something to
+// report, so nothing is copied.
 PyObject* py_pack_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != 13) { PyErr_SetString(PyExc_TypeError, "pack_block: wrong number of arguments"); return nullptr; }
     bool ok = true;
@@ -450,12 +477,15 @@ PyObject* py_pack_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
     c10::hip::HIPGuard guard(dev.index());
     hipStream_t stream = stream_of(dev);
     const int64_t T = K->size(0), H = K->size(1), D = K->size(2), G = T / r.gt, P = T / ps;
+    c10::Allocator* const allocator = c10::hip::HIPCachingAllocatorMasqueradingAsCUDA::get();
+    // (a dozen tensors: taken from the allocator directly, the dispatcher would cost a microsecond for each)
     auto make = [&](at::IntArrayRef shape, at::ScalarType type) {
-        return at::empty(shape, at::TensorOptions().dtype(type).device(dev));
+        return at::detail::empty_generic(shape, allocator, c10::DispatchKeySet(c10::DispatchKey::CUDA), type, std::nullopt);
     };
     const at::ScalarType step = r.mode == OMMX_SCALE_POW2_INT8 ? at::kChar : at::kBFloat16;
-    enum { KBASE, KSCALE, KZP, INDEX, OVAL, MS, MC, VMAIN, VSCALE, VZP, TOK, GRP, COUNT };
+    enum { FLAGS, KBASE, KSCALE, KZP, INDEX, OVAL, MS, MC, VMAIN, VSCALE, VZP, TOK, GRP, COUNT };
     at::Tensor t[COUNT];
+    t[FLAGS] = take_flags();
     t[KBASE] = make({P, ps, H, D / 4}, at::kByte);
     t[KSCALE] = make({G, H, D}, step);
     t[KZP] = make({G, H, D}, at::kBFloat16);
@@ -472,33 +502,49 @@ PyObject* py_pack_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
     t[VZP] = make({P, ps, H, D / r.gc}, at::kBFloat16);
     t[TOK] = make({1, P}, at::kInt);
     t[GRP] = make({1, G}, at::kInt);
-    at::Tensor flags = at::empty({OMMX_STORE_ERR_WORDS}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
-    int32_t* words = flags.data_ptr<int32_t>();
-    std::fill(words, words + OMMX_STORE_ERR_WORDS, 0);
     auto opt = [&](int i) { return t[i].defined() ? &t[i] : nullptr; };
-    const Planes p{&t[KBASE], &t[KSCALE], &t[KZP], opt(MS), opt(MC), opt(INDEX), opt(OVAL), &t[VMAIN], &t[VSCALE],
-                   &t[VZP]};
+    const Planes p{&t[KBASE], &t[KSCALE], &t[KZP], opt(MS), opt(MC), opt(INDEX), opt(OVAL), &t[VMAIN], &t[VSCALE], &t[VZP]};
     int rc;
-    hipError_t waited = hipSuccess;
     Py_BEGIN_ALLOW_THREADS
-    rc = launch_store(*K, *V, 0, p, r, T, ps, nullptr, nullptr, nullptr, *table, words, true, stream);
+    rc = launch_store(*K, *V, 0, p, r, T, ps, nullptr, nullptr, nullptr, *table, t[FLAGS].data_ptr<int32_t>(), true, stream);
     if (rc == 0) rc = ommx::identity_tables(t[TOK].data_ptr<int32_t>(), P, t[GRP].data_ptr<int32_t>(), G, stream);
-    if (rc == 0) waited = hipStreamSynchronize(stream);
     Py_END_ALLOW_THREADS
     if (failed(rc, "ommx_store_pack")) return nullptr;
+    PyObject* out = PyTuple_New(COUNT);
+    for (int i = 0; i < COUNT; ++i) {
+        if (!t[i].defined()) { Py_INCREF(Py_None); PyTuple_SET_ITEM(out, i, Py_None); }
+        else PyTuple_SET_ITEM(out, i, THPVariable_Wrap(std::move(t[i])));
+    }
+    return out;
+}
+
+// (flags, tensor of the packing device): waits for the current stream of that device and returns the error bits
+PyObject* py_block_errors(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    bool ok = n == 2;
+    const at::Tensor *flags = ok ? as_tensor(a[0], ok) : nullptr, *on_dev = ok ? as_tensor(a[1], ok) : nullptr;
+    if (!ok || flags->numel() != OMMX_STORE_ERR_WORDS || flags->scalar_type() != at::kInt || !on_dev->is_cuda()) {
+        PyErr_SetString(PyExc_TypeError, "block_errors: flags of pack_block and a GPU tensor expected");
+        return nullptr;
+    }
+    c10::hip::HIPGuard guard(on_dev->device().index());
+    hipStream_t stream = stream_of(on_dev->device());
+    hipError_t waited;
+    Py_BEGIN_ALLOW_THREADS
+    waited = hipStreamSynchronize(stream);
+    Py_END_ALLOW_THREADS
     if (waited != hipSuccess) {
         PyErr_Format(PyExc_RuntimeError, "ommx_store_pack: %s", hipGetErrorString(waited));
         return nullptr;
     }
+    const int32_t* words = flags->data_ptr<int32_t>();
     long bits = 0;
     for (int i = 0; i < OMMX_STORE_ERR_WORDS; ++i) bits |= (words[i] ? 1L : 0L) << i;
-    PyObject* out = PyTuple_New(1 + COUNT);
-    PyTuple_SET_ITEM(out, 0, PyLong_FromLong(bits));
-    for (int i = 0; i < COUNT; ++i) {
-        if (!t[i].defined()) { Py_INCREF(Py_None); PyTuple_SET_ITEM(out, 1 + i, Py_None); }
-        else PyTuple_SET_ITEM(out, 1 + i, THPVariable_Wrap(std::move(t[i])));
+    {
+        FlagPool& pool = flag_pool();
+        std::lock_guard<std::mutex> hold(pool.lock);
+        if (pool.idle.size() < kKeptFlags) pool.idle.push_back(*flags);
     }
-    return out;
+    return PyLong_FromLong(bits);
 }
 
 // ── bf16 row history ───────────────────────────────────────────────────────────────────────────
@@ -749,7 +795,7 @@ PyObject* guarded(PyObject* self, PyObject* const* a, Py_ssize_t n) {
 #define OMMX_FAST(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(guarded<py_##name>)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
     OMMX_FAST(auto_num_kv_splits),
-    OMMX_FAST(decode), OMMX_FAST(decode_pool), OMMX_FAST(store_pack), OMMX_FAST(pack_block), OMMX_FAST(pack_groups), OMMX_FAST(ring_write),
+    OMMX_FAST(decode), OMMX_FAST(decode_pool), OMMX_FAST(store_pack), OMMX_FAST(pack_block), OMMX_FAST(block_errors), OMMX_FAST(pack_groups), OMMX_FAST(ring_write),
     OMMX_FAST(tail_gather), OMMX_FAST(rows_write), OMMX_FAST(upload), OMMX_FAST(prefill),
     {nullptr, nullptr, 0, nullptr},
 };

@@ -260,8 +260,10 @@ class OMMXCanonicalImpl(_ImplBase):
             return
         s, st = _STATE, _STATE.step
         cfg = self._ommx_cfg()
-        key = key.reshape(n, self.num_kv_heads, self.head_size)
-        value = value.reshape(n, self.num_kv_heads, self.head_size)
+        if key.dim() != 3:
+            key = key.reshape(n, self.num_kv_heads, self.head_size)
+        if value.dim() != 3:
+            value = value.reshape(n, self.num_kv_heads, self.head_size)
         if st["B"] == STEP_ROUTE_UNCLASSIFIED and not st["batched_write"]:
             raise RuntimeError(
                 "[ommx] cannot classify this step: the metadata exposed no readable per-request "
@@ -350,10 +352,10 @@ class OMMXCanonicalImpl(_ImplBase):
     def forward(self, layer, query, key, value, kv_cache=None, attn_metadata=None, output=None,
                 output_scale=None, output_block_scale=None):
         H, D = self.num_heads, self.head_size
-        q = query.reshape(-1, H, D)
+        q = query if query.dim() == 3 else query.reshape(-1, H, D)
         if output is None:
             output = torch.empty_like(query)
-        out = output.view(-1, H, D)
+        out = output if output.dim() == 3 else output.view(-1, H, D)
         st = _STATE.step
         if st["B"] == STEP_ROUTE_UNCLASSIFIED:
             raise RuntimeError("[ommx] unclassified step: request count unknown, refusing to "
@@ -498,7 +500,7 @@ class OMMXCanonicalImpl(_ImplBase):
         in_step = self._reads_what_was_stored() and [pool.seq_len[x] for x in mgr.slots] == mgr.seq_lens
         step = mgr.step_on_device(pool) if in_step else None
         if step is not None and pool.decode_into(
-                q[:B], out[:B], step.sel, step.cur, step.packed, step.tables, sm_scale=self.scale,
+                q if q.shape[0] == B else q[:B], out if out.shape[0] == B else out[:B], step.sel, step.cur, step.packed, step.tables, sm_scale=self.scale,
                 max_seq_len=step.max_packed, mean_seq_len=step.mean_packed):
             _STATE.fires["batched"] += 1
             return
