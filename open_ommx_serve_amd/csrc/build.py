@@ -22,6 +22,7 @@ HOST_MODULE = os.path.join(HERE, "_ommx_host" + sysconfig.get_config_var("EXT_SU
 ARCH = "gfx950"
 SOURCES = {
     "ommx_store.hip": ["-ffp-contract=off"],
+    "ommx_store_long.hip": ["-ffp-contract=off"],
     "ommx_store_generic.hip": ["-ffp-contract=off"],
     "ommx_decode_ref.hip": [],
     "ommx_decode.hip": [],

@@ -510,17 +510,20 @@ int ommx::store_pack(const void* K, const void* V, int in_dtype,
                 (reinterpret_cast<uintptr_t>(V) % 16 == 0 && v_ts % 8 == 0 && v_hs % 8 == 0) ? 1 : 0,
                 index_repr, select_abs ? 1 : 0, scale_mode, gt, gc, v_bf16 ? 1 : 0, err_words ? 1 : 0};
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (gt != 32 || gc != 32 || k_outliers > 8 || 32 % page_size || v_bf16) {   // everything but the 32x32 recipe
-        if (launch_store_generic(a, T, in_dtype, st) != 0) {
-            set_error("ommx_store_pack: no kernel for this recipe");
-            return -1;
+    const bool tuned = k_outliers == 6 && !select_abs && scale_mode == 0 && k_ms && D == 128 && gt == 32 && gc == 32 &&
+                       32 % page_size == 0 && !v_bf16 && in_dtype == 0;   // the serving recipe
+    if (!tuned) {
+        int rc = launch_store_long(a, T, in_dtype, st);
+        if (rc == 1 && (gt != 32 || gc != 32 || k_outliers > 8 || 32 % page_size || v_bf16))
+            rc = launch_store_generic(a, T, in_dtype, st);   // everything but 32x32 recipes
+        if (rc < 0) { set_error("ommx_store_pack: no kernel for this recipe"); return -1; }
+        if (rc == 0) {
+            if (hipGetLastError() != hipSuccess) { set_error("ommx_store_pack: launch failed"); return -2; }
+            return 0;
         }
-        if (hipGetLastError() != hipSuccess) { set_error("ommx_store_pack: launch failed"); return -2; }
-        return 0;
     }
     const dim3 grid(T / 32, H), block(D);
     const size_t shm = 32 * (size_t)D + 4 * (size_t)D + (index_repr ? 8 * (size_t)D : 0);
-    const bool tuned = k_outliers == 6 && !select_abs && scale_mode == 0 && k_ms && D == 128;   // the serving recipe
     if (in_dtype == 1)
         hipLaunchKernelGGL((store_pack_kernel<true, false, 2>), grid, block, shm, st, a);
     else if (tuned && index_repr == 0)

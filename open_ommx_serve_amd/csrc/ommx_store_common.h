@@ -128,6 +128,7 @@ __device__ __forceinline__ uint32_t int2_code_fused(float w, float inv_scale, fl
     return __builtin_amdgcn_cvt_pk_u8_f32(fminf(__builtin_fmaf(w, inv_scale, c), 3.0f), 0u, 0u);
 }
 
+int launch_store_long(const StoreArgs& a, int T, int in_dtype, hipStream_t st);
 int launch_store_generic(const StoreArgs& a, int T, int in_dtype, hipStream_t st);
 
 }  // namespace ommx

@@ -1,0 +1,73 @@
+"""The store kernel of the signed power-of-two recipes beside the serving one, bit for bit against
+the oracle: every vector length it is built for, heads narrower and wider than the tuned one, both
+outlier counts and maps, blocks of heavy ties (the outlier sets of the two ends then overlap), constant
+vectors, permuted destinations, and what it reports."""
+import numpy as np
+import pytest
+import torch
+
+import oracle.ommx_oracle as O
+from conftest import bits_of
+from open_ommx_serve_amd.attention import ommx_pack_kv_canonical_block
+from open_ommx_serve_amd.attention.pack import alloc_planes, store_pack_into
+from open_ommx_serve_amd.synth import synth_kv
+
+pytestmark = pytest.mark.gpu
+ZERO_SIGN_FREE = ("k_zp", "v_zp", "k_fp4_mapcenter")
+
+
+def _names(recipe):
+    names = ["k_base", "k_scale", "k_zp", "k_oval", "v_main", "v_scale", "v_zp",
+             "k_obmp" if recipe["outlier_repr"] == "bitmap" else "k_oidx"]
+    return names + (["k_fp4_mapscale", "k_fp4_mapcenter"] if recipe.get("kv_outlier_map", True) else [])
+
+
+def _same(got, want, names):
+    for n in names:
+        a, b = got[n], want[n]
+        if n in ZERO_SIGN_FREE:                       # (a zero's sign is open where zeros of both signs tie)
+            a, b = a.float().cpu() + 0.0, b.float().cpu() + 0.0
+        assert np.array_equal(bits_of(a), bits_of(b)), n
+
+
+@pytest.mark.parametrize("gt,gc,D,k,repr_,own_map", [
+    (32, 32, 64, 6, "bitmap", True), (32, 32, 128, 6, "relidx7", False), (32, 32, 32, 10, "relidx7", True),
+    (64, 64, 128, 6, "relidx7", False), (64, 32, 64, 10, "bitmap", True), (64, 64, 256, 6, "bitmap", True),
+    (128, 128, 128, 10, "relidx7", True), (128, 64, 64, 6, "bitmap", False), (128, 128, 256, 10, "bitmap", False),
+    (128, 32, 96, 10, "relidx7", True)])
+def test_long_group_store_is_bit_exact(gt, gc, D, k, repr_, own_map):
+    T, H = 4 * gt, 3
+    K, V = synth_kv(T, H, D, seed=gt + D + k, sparse_frac=0.01)
+    g = torch.Generator().manual_seed(gt)
+    few = torch.tensor([-3.0, -1.0, 1.0, 0.0, -0.0, 0.5, -0.5, 2.0])
+    K[:gt] = few[torch.randint(0, len(few), (gt, H, D), generator=g)].to(torch.bfloat16)      # heavy ties
+    K[gt:2 * gt, 0] = 1.5                                                                     # constant vectors
+    K[gt:2 * gt, 1] = few[torch.randint(2, 5, (gt, D), generator=g)].to(torch.bfloat16)       # hardly two values
+    V[:gt, :, :gc] = -2.25
+    recipe = dict(outliers_per_vector=k, outlier_repr=repr_, outlier_select="signed", use_pow2=True,
+                  kv_outlier_map=own_map, group_tokens=gt, group_channels=gc)
+    want = O.pack_kv(K, V, **recipe)
+    _same(ommx_pack_kv_canonical_block(K.cuda(), V.cuda(), **recipe), want, _names(recipe))
+
+    # the same block through a source permutation into permuted slots
+    rows = torch.randperm(T, generator=g)
+    pages, groups = torch.randperm(T // 16, generator=g), torch.randperm(T // gt, generator=g)
+    planes = alloc_planes(T // 16, T // gt, H, D, outliers_per_vector=k, outlier_repr=repr_, kv_outlier_map=own_map,
+                          group_tokens=gt, group_channels=gc, device="cuda")
+    shuffled_k, shuffled_v = torch.empty_like(K), torch.empty_like(V)
+    shuffled_k[rows], shuffled_v[rows] = K, V
+    store_pack_into(shuffled_k.cuda(), shuffled_v.cuda(), planes, src_rows=rows.int().cuda(),
+                    dst_pages=pages.int().cuda(), dst_groups=groups.int().cuda(), outliers_per_vector=k,
+                    outlier_repr=repr_, group_tokens=gt, group_channels=gc)
+    _same({n: planes[n][(pages if n in ("k_base", "v_main", "v_scale", "v_zp") else groups).cuda()]
+           for n in _names(recipe)}, want, _names(recipe))
+
+
+@pytest.mark.parametrize("gt,k", [(32, 10), (64, 6), (128, 10)])
+@pytest.mark.parametrize("where,error", [("K", ValueError), ("V", ValueError)])
+def test_long_group_store_reports_values_that_are_not_finite(gt, k, where, error):
+    K, V = synth_kv(2 * gt, 2, 128, seed=5)
+    (K if where == "K" else V)[gt + 3, 1, 77] = float("inf")
+    with pytest.raises(error):
+        ommx_pack_kv_canonical_block(K.cuda(), V.cuda(), outliers_per_vector=k, outlier_repr="relidx7",
+                                     outlier_select="signed", use_pow2=True, group_tokens=gt)
