@@ -4,14 +4,15 @@
 // Same planes and the same arithmetic as ommx_store_generic.hip (reference attention/pack.py:419-623), which
 // keeps the recipes left over (other outlier counts, largest-magnitude selection, bf16 steps, fp32 rows, bf16 V).
 //
-// One workgroup of D threads packs one (K group, kv head), thread d owning channel d, as in ommx_store.hip.  What
-// bounds it is the number of vector instructions, and the selection is most of them: the general kernel runs
-// `k` passes of 5 instructions per element over the vector (64 tokens, 6 outliers: 1920); here one pass through
-// two sorted networks of depth k/2 + 1 (max / median of three on keys that hold the ordered bf16 value and the
-// tie breaker) takes k + 7 an element and leaves the extremes of what stays as their last ranks.  The outliers come out of
-// the network by rank and are wanted by position: each thread sorts them through its own few bytes of LDS.
-// Measured, 8128 tokens x 8 heads: "low-bit lever" (64 x 64, 6 outliers) and "paper-kv" (128 x 128, 10) at the
-// figures beside launch_store_long.
+// One workgroup of 2 D threads packs one (K group, kv head): the first D threads own one channel each and do K, the
+// others take the V vectors meanwhile.  The K tile comes in by 16-byte loads through LDS, and both passes over a
+// channel (selection, codes) are loops that read it there: held in registers and unrolled, 128 tokens overrun the
+// register file, and a straight-line body of 20-30 KB that every wave runs once is bound by instruction
+// fetch.  Selection is what remains: the general kernel runs k passes of 5 instructions per element over
+// the vector (64 tokens, 6 outliers: 1920); here one pass through two sorted networks of depth k/2 + 1
+// (max / median of three on keys that hold the ordered bf16 value and the tie breaker) takes k + 7 an
+// element and leaves the extremes of what stays as its last ranks.  The outliers come out of the network by
+// rank and are wanted by position: each thread sorts them through its own few bytes of LDS.
 #include <limits.h>
 
 #include "ommx_store_common.h"
@@ -43,72 +44,60 @@ __device__ __forceinline__ void keep_smallest(int (&t)[N], int key) {
     t[0] = min(t[0], key);
 }
 
+// k_vec: K rows allow 16-byte loads
 template <int GT, int GC, int KH>
-__global__ void __launch_bounds__(256) store_long_kernel(StoreArgs a) {
+__global__ void __launch_bounds__(512) store_long_kernel(StoreArgs a, int k_vec) {
     constexpr int K = 2 * KH, MW = GT / 32, TIE = GT - 1;      // GT is a power of two: the tie breaker is its low bits
     constexpr int SORT = K <= 8 ? 8 : 12;                      // LDS bytes per thread and sorted list
     constexpr int NVAL = K / 2, NIDX = (7 * K + 7) / 8;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int D = a.D, H = a.H, pieces = D >> 5;
-    uint8_t* const s_codes = smem;                             // [GT][D] one code per byte
-    uint8_t* const s_pos = smem + GT * D;                      // [D][SORT] positions, then FP4 codes, by slot
+    uint16_t* const s_k = reinterpret_cast<uint16_t*>(smem);   // [GT][D] the K tile
+    uint8_t* const s_codes = smem + 2 * GT * D;                // [GT][D] one code per byte
+    uint8_t* const s_pos = s_codes + GT * D;                   // [D][SORT] positions, then FP4 codes, by slot
     uint8_t* const s_fp4 = s_pos + SORT * D;
     uint8_t* const s_oval = s_fp4 + SORT * D;                  // [D][NVAL] as in memory
     uint8_t* const s_oidx = s_oval + 8 * D;                    // [D][bytes of the index plane] as in memory
-    const int g = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+    const int g = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, NT = 2 * D;
     const int nidx = a.idx_repr == 0 ? GT / 8 : NIDX;
     const int64_t gs = a.dst_groups ? a.dst_groups[g] : g;
     const float* __restrict__ tab = a.table;
     int err = 0;
+    auto src_row = [&](int i) -> int64_t { return a.src_rows ? a.src_rows[g * GT + i] : (int64_t)g * GT + i; };
+    auto phys_row = [&](int tok) {
+        const int lp = tok / a.ps;
+        const int64_t page = a.dst_pages ? a.dst_pages[lp] : lp;
+        return page * a.ps + (tok % a.ps);
+    };
+
+    if (k_vec) {
+        const int per_row = D / 8;
+#pragma unroll 4
+        for (int i = tid; i < GT * per_row; i += NT) {
+            const int r = i / per_row, c = i % per_row;
+            const uint16_t* src = static_cast<const uint16_t*>(a.K) + src_row(r) * a.k_ts + (int64_t)h * a.k_hs + 8 * c;
+            *reinterpret_cast<uint4*>(s_k + r * D + 8 * c) = *reinterpret_cast<const uint4*>(src);
+        }
+    } else {
+        for (int i = tid; i < GT * D; i += NT)
+            s_k[i] = static_cast<const uint16_t*>(a.K)[src_row(i / D) * a.k_ts + (int64_t)h * a.k_hs + i % D];
+    }
+    __syncthreads();
 
     // ------------------------------------------------------------------ K vector
-    {
+    if (tid < D) {
         const int d = tid;
-        // The vector is walked 32 tokens at a time, and read again (from L2) by the pass that forms the codes: held
-        // whole, 128 tokens and their keys overrun the registers, and the unrolled passes the instruction cache.
-        auto load32 = [&](int c, float (&w)[32]) {
-            typedef const __attribute__((address_space(1))) char* gptr;
-            const uint32_t off = static_cast<uint32_t>(d) * 2u;
-            if (a.src_rows) {
-#pragma unroll
-                for (int i = 0; i < 32; ++i) {
-                    const uint64_t row = reinterpret_cast<uint64_t>(a.K) + static_cast<uint64_t>(
-                        (static_cast<int64_t>(a.src_rows[g * GT + 32 * c + i]) * a.k_ts + (int64_t)h * a.k_hs) * 2);
-                    w[i] = bf16_to_f32(*reinterpret_cast<const __attribute__((address_space(1))) uint16_t*>(reinterpret_cast<gptr>(row) + off));
-                }
-                return;
-            }
-            uint64_t row = reinterpret_cast<uint64_t>(a.K) + static_cast<uint64_t>(
-                (static_cast<int64_t>(g * GT + 32 * c) * a.k_ts + (int64_t)h * a.k_hs) * 2);
-            const uint64_t stride = static_cast<uint64_t>(a.k_ts * 2);
-#pragma unroll
-            for (int i = 0; i < 32; ++i) {
-                w[i] = bf16_to_f32(*reinterpret_cast<const __attribute__((address_space(1))) uint16_t*>(reinterpret_cast<gptr>(row) + off));
-                row += stride;
-                asm volatile("" : "+s"(row));        // a scalar address per row, the channel as one shared 32-bit offset
-            }
-        };
-
-        auto one = [&](int i) {                      // token i of the vector, for the rare passes
-            const int64_t r = a.src_rows ? a.src_rows[g * GT + i] : (int64_t)g * GT + i;
-            return bf16_to_f32(static_cast<const uint16_t*>(a.K)[r * a.k_ts + (int64_t)h * a.k_hs + d]);
-        };
+        auto one = [&](int i) { return bf16_to_f32(s_k[i * D + d]); };       // token i of this thread's channel
 
         // (adding +0 turns -0 into +0: they tie in the reference's sorts)
         int t[KH + 1], b[KH + 1];
 #pragma unroll
         for (int j = 0; j <= KH; ++j) { t[j] = INT_MIN; b[j] = INT_MAX; }
-#pragma unroll 1
-        for (int c = 0; c < MW; ++c) {
-            float w[32];
-            load32(c, w);
-            const int hi = 32 * (MW - 1 - c), lo = 32 * c;
-#pragma unroll
-            for (int i = 0; i < 32; ++i) {
-                const int ob = ordered_pair_half(__float_as_uint(w[i] + 0.0f));
-                keep_largest(t, ob | (31 - i) | hi);       // equal values: the lower position first
-                keep_smallest(b, ob | i | lo);
-            }
+#pragma unroll 8
+        for (int i = 0; i < GT; ++i) {
+            const int ob = ordered_pair_half(__float_as_uint(one(i) + 0.0f));
+            keep_largest(t, ob | (TIE - i));           // equal values: the lower position first
+            keep_smallest(b, ob | i);
         }
 #pragma unroll
         for (int j = 0; j <= KH; ++j) asm volatile("" : "+v"(t[j]), "+v"(b[j]));
@@ -190,19 +179,13 @@ __global__ void __launch_bounds__(256) store_long_kernel(StoreArgs a) {
         }
         const float zc = -zp * st.inv;
         const bool fused_k = st.inv_ok && fabsf(zc) < INFINITY;
+        if (fused_k) {
+#pragma unroll 8
+            for (int i = 0; i < GT; ++i) s_codes[i * D + d] = static_cast<uint8_t>(int2_code_fused(one(i), st.inv, zc));
+        } else {
 #pragma unroll 1
-        for (int c = 0; c < MW; ++c) {
-            float w[32];
-            load32(c, w);
-            uint8_t* const out = s_codes + 32 * c * D + d;
-            if (fused_k) {
-#pragma unroll
-                for (int i = 0; i < 32; ++i) out[i * D] = static_cast<uint8_t>(int2_code_fused(w[i], st.inv, zc));
-            } else {
-#pragma unroll 1
-                for (int i = 0; i < 32; ++i)
-                    out[i * D] = static_cast<uint8_t>(int2_code(one(32 * c + i) - zp, st.scale, st.inv, st.inv_ok));
-            }
+            for (int i = 0; i < GT; ++i)
+                s_codes[i * D + d] = static_cast<uint8_t>(int2_code(one(i) - zp, st.scale, st.inv, st.inv_ok));
         }
 
         // FP4 codes of the chosen lanes by slot = rank of their position.  |mapped| is largest at the extreme
@@ -262,26 +245,86 @@ __global__ void __launch_bounds__(256) store_long_kernel(StoreArgs a) {
             for (int q = 0; q < NIDX; ++q)
                 s_oidx[d * NIDX + q] = static_cast<uint8_t>(q < 8 ? lo >> (8 * q) : hi >> (8 * (q - 8)));
         }
+    } else {
+        // -------------------------------------------- V vectors (pack.py:604-623)
+        const int ngv = D / GC;
+        for (int it = tid - D; it < GT * ngv; it += D) {
+            const int tk = it / ngv, j = it % ngv, tok = g * GT + tk;
+            const int64_t prow = phys_row(tok);
+            const int64_t row = a.src_rows ? a.src_rows[tok] : tok;
+            const uint16_t* const vp = static_cast<const uint16_t*>(a.V) + row * a.v_ts + (int64_t)h * a.v_hs + GC * j;
+            // eight channels a turn, read again (from L1 / L2) by the second pass
+            auto eight = [&](int q) {
+                if (a.v_vec) return reinterpret_cast<const uint4*>(vp)[q];
+                const uint16_t* e = vp + 8 * q;
+                return uint4{e[0] | (static_cast<uint32_t>(e[1]) << 16), e[2] | (static_cast<uint32_t>(e[3]) << 16),
+                             e[4] | (static_cast<uint32_t>(e[5]) << 16), e[6] | (static_cast<uint32_t>(e[7]) << 16)};
+            };
+            typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+            u16x2 e2 = {0, 0};                    // largest exponent field: all ones when a value is not finite
+            float mn = bf16_to_f32(vp[0]), mx = mn;
+#pragma unroll 4
+            for (int q = 0; q < GC / 8; ++q) {
+                const uint4 u = eight(q);
+                const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const float lo = __uint_as_float(w[c] << 16), hi = __uint_as_float(w[c] & 0xFFFF0000u);
+                    mn = fminf(fminf(mn, lo), hi);
+                    mx = fmaxf(fmaxf(mx, lo), hi);
+                    e2 = __builtin_elementwise_max(e2, __builtin_bit_cast(u16x2, w[c] & 0x7F807F80u));
+                }
+            }
+            if (e2[0] == 0x7F80 || e2[1] == 0x7F80) err |= OMMX_ERR_NONFINITE_V;
+            const Step st = make_step(__fdiv_rn(fmaxf(mx - mn, 1e-8f), 3.0f), 0, tab);
+            if (!st.in_range) err |= OMMX_ERR_EXP_RANGE;
+            if (st.e > 15) err |= OMMX_NOTE_WIDE_STEP;
+            const uint16_t zp_b = f32_to_bf16_rne(mn);
+            const float zp = bf16_to_f32(zp_b), zc = -zp * st.inv;
+            const bool fused = st.inv_ok && fabsf(zc) < INFINITY;
+            uint16_t* const dst = reinterpret_cast<uint16_t*>(a.v_main + (prow * H + h) * (D / 4) + j * (GC / 4));
+#pragma unroll 4
+            for (int q = 0; q < GC / 8; ++q) {
+                const uint4 u = eight(q);
+                const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+                uint32_t bits = 0;
+                if (fused) {
+#pragma unroll
+                    for (int f = 0; f < 2; ++f) {
+                        uint32_t four = 0;
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) {
+                            const uint32_t x = w[2 * f + (c >> 1)];
+                            const float v = __uint_as_float((c & 1) ? x & 0xFFFF0000u : x << 16);
+                            four = __builtin_amdgcn_cvt_pk_u8_f32(fminf(__builtin_fmaf(v, st.inv, zc), 3.0f), c, four);
+                        }
+                        bits |= __builtin_amdgcn_udot4(four, 0x40100401u, 0u, false) << (8 * f);
+                    }
+                } else {
+#pragma unroll 1
+                    for (int c = 0; c < 8; ++c)
+                        bits |= int2_code(bf16_to_f32(vp[8 * q + c]) - zp, st.scale, st.inv, st.inv_ok) << (2 * c);
+                }
+                dst[q] = static_cast<uint16_t>(bits);
+            }
+            const int64_t vidx = (prow * H + h) * ngv + j;
+            a.v_scale[vidx] = static_cast<int8_t>(st.e);
+            a.v_zp[vidx] = zp_b;
+        }
     }
     __syncthreads();
 
     {   // D frames of NVAL / nidx bytes each, contiguous in memory: whole dwords
         const int64_t obase = (gs * H + h) * (int64_t)D * NVAL;
-        for (int wd = tid; wd < D * NVAL / 4; wd += D)
+        for (int wd = tid; wd < D * NVAL / 4; wd += NT)
             reinterpret_cast<uint32_t*>(a.k_oval + obase)[wd] = reinterpret_cast<const uint32_t*>(s_oval)[wd];
         const int64_t ibase = (gs * H + h) * (int64_t)D * nidx;
-        for (int wd = tid; wd < D * nidx / 4; wd += D)
+        for (int wd = tid; wd < D * nidx / 4; wd += NT)
             reinterpret_cast<uint32_t*>(a.k_obmp + ibase)[wd] = reinterpret_cast<const uint32_t*>(s_oidx)[wd];
     }
 
-    auto phys_row = [&](int tok) {
-        const int lp = tok / a.ps;
-        const int64_t page = a.dst_pages ? a.dst_pages[lp] : lp;
-        return page * a.ps + (tok % a.ps);
-    };
-
     // ------------------------------------------------- k_base rows: 8 bytes = 32 channels a piece
-    for (int it = tid; it < GT * pieces; it += D) {
+    for (int it = tid; it < GT * pieces; it += NT) {
         const int tk = it / pieces, j = it % pieces;
         uint64_t kb8 = 0;
         const uint4* cr = reinterpret_cast<const uint4*>(s_codes + tk * D + 32 * j);
@@ -296,77 +339,17 @@ __global__ void __launch_bounds__(256) store_long_kernel(StoreArgs a) {
         reinterpret_cast<uint64_t*>(a.k_base)[(phys_row(g * GT + tk) * H + h) * pieces + j] = kb8;
     }
 
-    // ------------------------------------------------- V vectors (pack.py:604-623)
-    const int ngv = D / GC;
-    for (int it = tid; it < GT * ngv; it += D) {
-        const int tk = it / ngv, j = it % ngv, tok = g * GT + tk;
-        const int64_t prow = phys_row(tok);
-        const int64_t row = a.src_rows ? a.src_rows[tok] : tok;
-        const uint16_t* const vp = static_cast<const uint16_t*>(a.V) + row * a.v_ts + (int64_t)h * a.v_hs + GC * j;
-        uint32_t raw[GC / 2];
-        if (a.v_vec) {
-#pragma unroll
-            for (int q = 0; q < GC / 8; ++q) {
-                const uint4 u = reinterpret_cast<const uint4*>(vp)[q];
-                raw[4 * q] = u.x; raw[4 * q + 1] = u.y; raw[4 * q + 2] = u.z; raw[4 * q + 3] = u.w;
-            }
-        } else {
-#pragma unroll
-            for (int c = 0; c < GC / 2; ++c) raw[c] = vp[2 * c] | (static_cast<uint32_t>(vp[2 * c + 1]) << 16);
-        }
-        auto val = [&](int c) { return __uint_as_float((c & 1) ? raw[c >> 1] & 0xFFFF0000u : raw[c >> 1] << 16); };
-        typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-        u16x2 e2 = {0, 0};                        // largest exponent field: all ones when a value is not finite
-        float mn = val(0), mx = val(0);
-#pragma unroll
-        for (int c = 0; c < GC; ++c) {
-            if (c) { mn = fminf(mn, val(c)); mx = fmaxf(mx, val(c)); }
-            if (!(c & 1)) e2 = __builtin_elementwise_max(e2, __builtin_bit_cast(u16x2, raw[c >> 1] & 0x7F807F80u));
-        }
-#pragma unroll
-        for (int c = 0; c < GC / 2; ++c) asm volatile("" : "+v"(raw[c]));       // unpacked again below, not kept unpacked
-        if (e2[0] == 0x7F80 || e2[1] == 0x7F80) err |= OMMX_ERR_NONFINITE_V;
-        const Step st = make_step(__fdiv_rn(fmaxf(mx - mn, 1e-8f), 3.0f), 0, tab);
-        if (!st.in_range) err |= OMMX_ERR_EXP_RANGE;
-        if (st.e > 15) err |= OMMX_NOTE_WIDE_STEP;
-        const uint16_t zp_b = f32_to_bf16_rne(mn);
-        const float zp = bf16_to_f32(zp_b), zc = -zp * st.inv;
-        const bool fused = st.inv_ok && fabsf(zc) < INFINITY;
-        uint32_t* const dst = reinterpret_cast<uint32_t*>(a.v_main + (prow * H + h) * (D / 4) + j * (GC / 4));
-#pragma unroll
-        for (int wd = 0; wd < GC / 16; ++wd) {
-            uint32_t bits = 0;
-            if (fused) {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    uint32_t four = 0;
-#pragma unroll
-                    for (int c = 0; c < 4; ++c)
-                        four = __builtin_amdgcn_cvt_pk_u8_f32(fminf(__builtin_fmaf(val(16 * wd + 4 * q + c), st.inv, zc), 3.0f), c, four);
-                    bits |= __builtin_amdgcn_udot4(four, 0x40100401u, 0u, false) << (8 * q);
-                }
-            } else {
-#pragma unroll 1
-                for (int c = 0; c < 16; ++c) {
-                    const uint16_t e16 = vp[16 * wd + c];
-                    bits |= int2_code(bf16_to_f32(e16) - zp, st.scale, st.inv, st.inv_ok) << (2 * c);
-                }
-            }
-            dst[wd] = bits;
-        }
-        const int64_t vidx = (prow * H + h) * ngv + j;
-        a.v_scale[vidx] = static_cast<int8_t>(st.e);
-        a.v_zp[vidx] = zp_b;
-    }
     if (err && a.err) report_store_bits(a, err);
 }
 
 template <int GT, int GC>
 int launch_k(const StoreArgs& a, int T, hipStream_t st) {
-    const dim3 grid(T / GT, a.H), block(a.D);
-    const size_t shm = static_cast<size_t>(a.D) * (GT + 2 * 12 + 8 + 16);
-    if (a.kout == 6) hipLaunchKernelGGL((store_long_kernel<GT, GC, 3>), grid, block, shm, st, a);
-    else hipLaunchKernelGGL((store_long_kernel<GT, GC, 5>), grid, block, shm, st, a);
+    const dim3 grid(T / GT, a.H), block(2 * a.D);
+    const size_t shm = static_cast<size_t>(a.D) * (3 * GT + 2 * 12 + 8 + 16);
+    if (shm > 64 * 1024) return 1;           // 128 tokens of a 256-channel head: the general kernel
+    const int k_vec = reinterpret_cast<uintptr_t>(a.K) % 16 == 0 && a.k_ts % 8 == 0 && a.k_hs % 8 == 0;
+    if (a.kout == 6) hipLaunchKernelGGL((store_long_kernel<GT, GC, 3>), grid, block, shm, st, a, k_vec);
+    else hipLaunchKernelGGL((store_long_kernel<GT, GC, 5>), grid, block, shm, st, a, k_vec);
     return 0;
 }
 template <int GT>
