@@ -101,9 +101,11 @@ def ommx_paged_decode_attention_canonical(
     (``paged_decode.py:2856-2887``).  ``seg_group_base > 0`` emits the un-merged state of a
     group-range segment without the tail (``:2892-2902``).
 
-    ``mean_seq_len`` (not in the reference's signature) is a hint for the automatic split count
-    only: a caller that passes ``max_seq_len`` to avoid the host sync may also say how long the
-    requests are on average, see :func:`auto_num_kv_splits`.  ``err_flag`` (not in the reference's
+    With neither ``num_kv_splits`` nor a workspace given, a batch with work for every SIMD is dealt out
+    in equal shares by the kernels themselves, whatever the lengths; otherwise every request gets
+    ``num_kv_splits``, or :func:`auto_num_kv_splits`, splits.  ``mean_seq_len`` (not in the reference's
+    signature) is a hint for the latter only: a caller that passes ``max_seq_len`` to avoid the host sync
+    may also say how long the requests are on average.  ``err_flag`` (not in the reference's
     signature either): an int32 device tensor that receives ``_hip.ERR_TABLE_RANGE`` when a page id
     or group slot of the tables lies outside the planes (the kernels clamp such an entry, so nothing
     is read out of bounds; the reference leaves these checks to the pools, ``kv_pool.py:526-550``),

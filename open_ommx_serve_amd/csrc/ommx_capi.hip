@@ -89,46 +89,69 @@ static const char* check_decode(OMMX_DECODE_PARAMS) {
 }
 
 static DecodeArgs make_decode_args(OMMX_DECODE_PARAMS) {
-    (void)D; (void)stream;
-    return DecodeArgs{q, q_stride_b, q_stride_h, k_base, static_cast<const int8_t*>(k_scale), k_zp, k_ms, k_mc,
+    (void)stream;
+    DecodeArgs a{q, q_stride_b, q_stride_h, k_base, static_cast<const int8_t*>(k_scale), k_zp, k_ms, k_mc,
                       k_index, k_oval, v_main, static_cast<const int8_t*>(v_scale), v_zp, req_to_token, rt_stride,
                       req_to_group, rg_stride, table_i64, b_seq_len, attn_logits, al_stride_b, al_stride_h,
                       al_stride_s, B, Hq, Hkv, page_size, k_outliers, num_splits, sm_scale, logit_cap,
                       packed_start_offset, seg_group_base, index_repr, scale_bf16 ? 1 : 0,
                       group_tokens, group_channels, v_bf16 ? 1 : 0, num_pages, num_group_slots, err_flag};
+    a.sl = attn_logits + D;
+    a.sl_b = al_stride_b;
+    a.sl_h = al_stride_h;
+    a.sl_s = al_stride_s;
+    return a;
 }
 
 static void set_error2(const char* where, const char* what) { g_error = std::string(where) + ": " + what; }
 
 }  // namespace ommx
 
-extern "C" int ommx_decode_splitkv(OMMX_DECODE_PARAMS) {
-    using namespace ommx;
-    if (const char* bad = check_decode(OMMX_DECODE_ARGS)) { set_error2("ommx_decode_splitkv", bad); return -1; }
-    const DecodeArgs a = make_decode_args(OMMX_DECODE_ARGS);
+int ommx::decode_splitkv(OMMX_DECODE_PARAMS, bool plain, const StateLse* lse, const Shares* shares) {
+    const char* where = plain ? "ommx_decode_splitkv_ref" : "ommx_decode_splitkv";
+    if (const char* bad = check_decode(OMMX_DECODE_ARGS)) { set_error2(where, bad); return -1; }
+    DecodeArgs a = make_decode_args(OMMX_DECODE_ARGS);
+    if (lse) { a.sl = lse->p; a.sl_b = lse->b; a.sl_h = lse->h; a.sl_s = lse->s; }
+    if (shares) {
+        if (plain || shares->few < B || shares->all < shares->few || !shares->count) {
+            set_error2(where, "bad share counts");
+            return -1;
+        }
+        a.shares = shares->all;
+        a.shares_few = shares->few;
+        a.singles = shares->singles;
+        a.share_count = shares->count;
+    }
+    const int R = Hq / Hkv;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    int rc = launch_decode_gqa4(a, D, Hq / Hkv, st);
-    if (rc == 1) rc = launch_decode_fast(a, D, Hq / Hkv, st);
-    if (rc == 1) rc = launch_decode_ref(a, D, Hq / Hkv, st);      // shapes the matrix-core kernel leaves out
-    if (rc != 0) { set_error("ommx_decode_splitkv: no kernel for this shape"); return -1; }
-    if (hipGetLastError() != hipSuccess) { set_error("ommx_decode_splitkv: launch failed"); return -2; }
+    int rc = 1;
+    if (!plain) {
+        rc = launch_decode_gqa4(a, D, R, st);
+        if (rc == 1) rc = launch_decode_fast(a, D, R, st);
+        if (rc == 1 && shares) return 1;                  // (the plain kernel knows fixed splits only)
+    }
+    if (rc == 1) rc = launch_decode_ref(a, D, R, st);     // shapes the matrix-core kernels leave out
+    if (rc != 0) { set_error2(where, "no kernel for this shape"); return -1; }
+    if (hipGetLastError() != hipSuccess) { set_error2(where, "launch failed"); return -2; }
     return 0;
+}
+
+extern "C" int ommx_decode_splitkv(OMMX_DECODE_PARAMS) {
+    return ommx::decode_splitkv(OMMX_DECODE_ARGS, false, nullptr, nullptr);
 }
 
 // Same operator through the plain fp32 kernel only (cross-check entry used by tests).
 extern "C" int ommx_decode_splitkv_ref(OMMX_DECODE_PARAMS) {
-    using namespace ommx;
-    if (const char* bad = check_decode(OMMX_DECODE_ARGS)) { set_error2("ommx_decode_splitkv_ref", bad); return -1; }
-    const DecodeArgs a = make_decode_args(OMMX_DECODE_ARGS);
-    if (launch_decode_ref(a, D, Hq / Hkv, static_cast<hipStream_t>(stream)) != 0) {
-        set_error("ommx_decode_splitkv_ref: unsupported shape");
-        return -1;
-    }
-    if (hipGetLastError() != hipSuccess) { set_error("ommx_decode_splitkv_ref: launch failed"); return -2; }
-    return 0;
+    return ommx::decode_splitkv(OMMX_DECODE_ARGS, true, nullptr, nullptr);
 }
 
-extern "C" int ommx_decode_combine(
+// What the combine knows of the shares: each request's number of states, on the device, and how many an even deal gives.
+static void set_shares(ommx::CombineArgs& a, const ommx::Shares* shares) {
+    a.share_count = shares ? shares->count : nullptr;
+    a.sure = shares ? std::min(a.S, shares->each) : a.S;
+}
+
+int ommx::decode_combine(
     const float* attn_logits, int64_t al_stride_b, int64_t al_stride_h, int64_t al_stride_s,
     const uint16_t* q, int64_t q_stride_b, int64_t q_stride_h,
     const uint16_t* k_tail, const uint16_t* v_tail,
@@ -137,8 +160,7 @@ extern "C" int ommx_decode_combine(
     const int32_t* b_tail_len, const int32_t* b_seq_len,
     float* o, int64_t o_stride_b, int64_t o_stride_h, float* lse, int64_t lse_stride_b,
     int B, int Hq, int Hkv, int D, int num_splits, int group_tokens, int tail_rows, float sm_scale,
-    float logit_cap, void* stream) {
-    using namespace ommx;
+    float logit_cap, const StateLse* states, const Shares* shares, void* stream) {
     if (B <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv || num_splits < 1 || !(D == 64 || D == 128) ||
         group_tokens < 16 || group_tokens > 128 || (group_tokens & (group_tokens - 1)) || tail_rows < 0) {
         set_error("ommx_decode_combine: bad shape");
@@ -163,6 +185,11 @@ extern "C" int ommx_decode_combine(
                   vt_stride_b, vt_stride_t, vt_stride_h, b_tail_len, b_seq_len,
                   o, o_stride_b, o_stride_h, lse, lse_stride_b, B, Hq, Hkv, num_splits,
                   sm_scale, logit_cap, group_tokens, b_tail_len ? tail_rows : 0};
+    set_shares(a, shares);
+    a.sl = states ? states->p : attn_logits + D;
+    a.sl_b = states ? states->b : al_stride_b;
+    a.sl_h = states ? states->h : al_stride_h;
+    a.sl_s = states ? states->s : al_stride_s;
     if (launch_combine(a, D, static_cast<hipStream_t>(stream)) != 0) {
         set_error("ommx_decode_combine: unsupported head_dim");
         return -1;
@@ -171,10 +198,27 @@ extern "C" int ommx_decode_combine(
     return 0;
 }
 
+extern "C" int ommx_decode_combine(
+    const float* attn_logits, int64_t al_stride_b, int64_t al_stride_h, int64_t al_stride_s,
+    const uint16_t* q, int64_t q_stride_b, int64_t q_stride_h,
+    const uint16_t* k_tail, const uint16_t* v_tail,
+    int64_t kt_stride_b, int64_t kt_stride_t, int64_t kt_stride_h,
+    int64_t vt_stride_b, int64_t vt_stride_t, int64_t vt_stride_h,
+    const int32_t* b_tail_len, const int32_t* b_seq_len,
+    float* o, int64_t o_stride_b, int64_t o_stride_h, float* lse, int64_t lse_stride_b,
+    int B, int Hq, int Hkv, int D, int num_splits, int group_tokens, int tail_rows, float sm_scale,
+    float logit_cap, void* stream) {
+    return ommx::decode_combine(attn_logits, al_stride_b, al_stride_h, al_stride_s, q, q_stride_b, q_stride_h, k_tail,
+                                v_tail, kt_stride_b, kt_stride_t, kt_stride_h, vt_stride_b, vt_stride_t, vt_stride_h,
+                                b_tail_len, b_seq_len, o, o_stride_b, o_stride_h, lse, lse_stride_b, B, Hq, Hkv, D,
+                                num_splits, group_tokens, tail_rows, sm_scale, logit_cap, nullptr, nullptr, stream);
+}
+
 int ommx::decode_combine_hist(const float* attn_logits, int64_t al_b, int64_t al_h, int64_t al_s, const uint16_t* q,
                               int64_t q_b, int64_t q_h, const HistTail& t, void* o, bool o_bf16, int64_t o_b,
                               int64_t o_h, float* lse, int64_t lse_b, int B, int Hq, int Hkv, int D, int num_splits,
-                              int group_tokens, float sm_scale, float logit_cap, void* stream) {
+                              int group_tokens, float sm_scale, float logit_cap, const StateLse& states,
+                              const Shares* shares, void* stream) {
     const char* where = "decode_combine_hist";
     if (B <= 0 || Hkv <= 0 || Hq % Hkv || num_splits < 1 || num_splits > 512 || !(D == 64 || D == 128) ||
         group_tokens < 16 || group_tokens > 128 || t.rows <= 0 || t.win_sink < 0 || t.win_recent < 0) {
@@ -196,6 +240,11 @@ int ommx::decode_combine_hist(const float* attn_logits, int64_t al_b, int64_t al
                   nullptr, nullptr, o_bf16 ? nullptr : static_cast<float*>(o), o_b, o_h, lse, lse_b, B, Hq, Hkv,
                   num_splits, sm_scale, logit_cap, group_tokens, t.win_sink + most};
     a.o16 = o_bf16 ? static_cast<uint16_t*>(o) : nullptr;
+    set_shares(a, shares);
+    a.sl = states.p;
+    a.sl_b = states.b;
+    a.sl_h = states.h;
+    a.sl_s = states.s;
     a.hist_seq = t.seq;
     a.hist_slots = t.slots;
     a.hist_rows = t.rows;

@@ -49,8 +49,9 @@ __device__ __forceinline__ void put_out(const CombineArgs& a, int64_t at, float 
     else a.o[at] = v;
 }
 
-// HIST: the tail rows lie in a row history instead of a gathered buffer.
-template <int D, int Q, bool HIST, int NT = 1024, int MAXS = 256>
+// HIST: the tail rows lie in a row history instead of a gathered buffer.  SHARED: the number of states is the
+// request's own.
+template <int D, int Q, bool HIST, bool SHARED, int NT = 1024, int MAXS = 256>
 __global__ void __launch_bounds__(NT) combine_kernel(CombineArgs a) {
     constexpr int CH = D / Q;            // channels of this workgroup (one of Q pieces of the head)
     constexpr int NSG = NT / CH;         // split groups: thread (d, sg) owns splits sg, sg + NSG, ...
@@ -80,8 +81,11 @@ __global__ void __launch_bounds__(NT) combine_kernel(CombineArgs a) {
     // memory; one pointer per thread, advanced by NSG split slots per load.  (A uniform trip
     // count and a clamped last address keep the loads free of per-lane branches, so they
     // are all in flight together.)
+    // With shares the number of states is itself read from memory, one memory latency (0.7 us) later than everything
+    // else: what an even deal gives every request goes out before it is here (the slots exist; what an unused one
+    // holds is dropped below), the states beyond that once the weights are there.
     float pv[NSP];
-    const int n_i = (a.S + NSG - 1) / NSG;
+    const int n_i = (a.sure + NSG - 1) / NSG;
     {
         const float* p = base + (int64_t)sg * a.al_s + d;
         const int64_t step = NSG * a.al_s;
@@ -95,12 +99,14 @@ __global__ void __launch_bounds__(NT) combine_kernel(CombineArgs a) {
             }
         }
     }
-    const uint32_t q_raw = (a.q && tid < D) ? a.q[b * a.q_sb + (int64_t)h * a.q_sh + tid] : 0u;
     // Every split wrote its state, an empty one with lse = -inf (paged_decode.py:2262-2284), so the
     // weights follow from the lse column alone, whatever rule dealt the tokens out to the splits
     // (the reference recomputes its rounding here, paged_decode.py:2407-2410).
     float my_lse = -INFINITY;
-    if (tid < MAXS && tid < a.S) my_lse = base[(int64_t)tid * a.al_s + D];
+    if (tid < MAXS && tid < a.S) my_lse = a.sl[b * a.sl_b + (int64_t)h * a.sl_h + (int64_t)tid * a.sl_s];
+    const uint32_t q_raw = (a.q && tid < D) ? a.q[b * a.q_sb + (int64_t)h * a.q_sh + tid] : 0u;
+    const int S = SHARED ? min(max(a.share_count[b], 1), a.S) : a.S;
+    if (SHARED && tid >= S) my_lse = -INFINITY;
 
     if (tid < D) s_q[tid] = __uint_as_float(q_raw << 16);
     if (tid < MAXS) {
@@ -188,6 +194,18 @@ __global__ void __launch_bounds__(NT) combine_kernel(CombineArgs a) {
             acc = w[k] > 0.0f ? fmaf(w[k], pv[4 * i4 + k], acc) : acc;
         }
     }
+    if (SHARED) {
+        for (int i = n_i; i * NSG < S; i += 4) {
+            float v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = base[(int64_t)min(sg + NSG * (i + u), S - 1) * a.al_s + d];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const float w = i + u < NSP ? s_wT[sg][i + u] : 0.0f;
+                acc = w > 0.0f ? fmaf(w, v[u], acc) : acc;
+            }
+        }
+    }
     s_acc[sg][dl] = acc;
     s_tacc[sg][dl] = t_acc;
     if (dl == 0) { s_w[sg] = wsum; s_tl[sg] = t_l; }
@@ -233,7 +251,7 @@ __device__ __forceinline__ float wave_sum_f32(float v) {
 // EARLY: the tail rows of the first pass are asked for before the split part and held in registers
 // (32 more: one workgroup per compute unit instead of two, which pays while the grid is no larger
 // than the chip).
-template <int D, int R, bool EARLY, bool HIST>
+template <int D, int R, bool EARLY, bool HIST, bool SHARED>
 __global__ void __launch_bounds__(512) combine_grouped_kernel(CombineArgs a) {
     constexpr int NT = 512, MAXS = 64;
     constexpr int ROWS = 128;              // tail rows per pass (two per thread of the logit layout)
@@ -250,6 +268,8 @@ __global__ void __launch_bounds__(512) combine_grouped_kernel(CombineArgs a) {
     const int lane = tid & 63, wave = tid >> 6;
     const int h0 = kvh * R;
     const float* base = a.al + b * a.al_b + (int64_t)h0 * a.al_h;
+    // (the states of this request: its own number when the work was dealt out in shares)
+    const int S = SHARED ? min(max(a.share_count[b], 1), a.S) : a.S;
     TailRows<HIST> rows;
     rows.init(a, b);
     const int tail = rows.n;
@@ -265,8 +285,8 @@ __global__ void __launch_bounds__(512) combine_grouped_kernel(CombineArgs a) {
         }
     }
     if (wave < R) {
-        const bool valid = lane < a.S;          // an empty split's lse is -inf
-        const float my_lse = valid ? base[(int64_t)wave * a.al_h + (int64_t)lane * a.al_s + D] : -INFINITY;
+        float my_lse = lane < a.S ? a.sl[b * a.sl_b + (int64_t)(h0 + wave) * a.sl_h + (int64_t)lane * a.sl_s] : -INFINITY;
+        if (lane >= S) my_lse = -INFINITY;    // an empty split's lse is -inf, an unused slot holds anything
         const float g_max = wave_max_f32(my_lse);
         const float g_safe = (g_max == -INFINITY) ? 0.0f : g_max;
         const float w = my_lse == -INFINITY ? 0.0f : __expf(my_lse - g_safe);
@@ -322,13 +342,13 @@ __global__ void __launch_bounds__(512) combine_grouped_kernel(CombineArgs a) {
             const int r = i / D, d = i % D;
             const float* p = base + (int64_t)r * a.al_h + d;
             float acc = 0.0f;
-            for (int s0 = 0; s0 < a.S; s0 += 8) {
+            for (int s0 = 0; s0 < S; s0 += 8) {
                 float v[8];
 #pragma unroll
-                for (int u = 0; u < 8; ++u) v[u] = p[(int64_t)min(s0 + u, a.S - 1) * a.al_s];
+                for (int u = 0; u < 8; ++u) v[u] = p[(int64_t)min(s0 + u, S - 1) * a.al_s];
 #pragma unroll
                 for (int u = 0; u < 8; ++u) {
-                    const float w = s0 + u < a.S ? s_w[r][s0 + u] : 0.0f;
+                    const float w = s0 + u < S ? s_w[r][s0 + u] : 0.0f;
                     acc = w > 0.0f ? fmaf(w, v[u], acc) : acc;
                 }
             }
@@ -468,7 +488,7 @@ __global__ void __launch_bounds__(512) combine_grouped_kernel(CombineArgs a) {
     }
 }
 
-template <bool HIST>
+template <bool HIST, bool SHARED>
 static int launch_combine_rows(const CombineArgs& a, int D, hipStream_t st) {
     if (a.S > 512) return -1;
     // Pieces per head.  At batch 1 the kernel is latency bound and 2 pieces measured best (1.4 us
@@ -486,8 +506,8 @@ static int launch_combine_rows(const CombineArgs& a, int D, hipStream_t st) {
         const bool early = a.B * a.Hkv <= 320;       // about one workgroup per compute unit
 #define OMMX_GROUPED(DD, RR)                                                                              \
         do {                                                                                              \
-            if (early) hipLaunchKernelGGL((combine_grouped_kernel<DD, RR, true, HIST>), g2, dim3(512), 0, st, a);  \
-            else hipLaunchKernelGGL((combine_grouped_kernel<DD, RR, false, HIST>), g2, dim3(512), 0, st, a);       \
+            if (early) hipLaunchKernelGGL((combine_grouped_kernel<DD, RR, true, HIST, SHARED>), g2, dim3(512), 0, st, a);  \
+            else hipLaunchKernelGGL((combine_grouped_kernel<DD, RR, false, HIST, SHARED>), g2, dim3(512), 0, st, a);       \
         } while (0)
         if (D == 128 && R == 4) OMMX_GROUPED(128, 4);
         else if (D == 128) OMMX_GROUPED(128, 8);
@@ -499,25 +519,27 @@ static int launch_combine_rows(const CombineArgs& a, int D, hipStream_t st) {
     }
     if (a.S > 256) {        // 257..512 splits: the same kernel with twice the split slots per thread
         const dim3 g1(a.B, a.Hq, split2 ? 2 : 1);
-        if (D == 128 && split2) hipLaunchKernelGGL((combine_kernel<128, 2, HIST, 1024, 512>), g1, dim3(1024), 0, st, a);
-        else if (D == 128) hipLaunchKernelGGL((combine_kernel<128, 1, HIST, 1024, 512>), g1, dim3(1024), 0, st, a);
-        else if (D == 64 && split2) hipLaunchKernelGGL((combine_kernel<64, 2, HIST, 1024, 512>), g1, dim3(1024), 0, st, a);
-        else if (D == 64) hipLaunchKernelGGL((combine_kernel<64, 1, HIST, 1024, 512>), g1, dim3(1024), 0, st, a);
+        if (D == 128 && split2) hipLaunchKernelGGL((combine_kernel<128, 2, HIST, SHARED, 1024, 512>), g1, dim3(1024), 0, st, a);
+        else if (D == 128) hipLaunchKernelGGL((combine_kernel<128, 1, HIST, SHARED, 1024, 512>), g1, dim3(1024), 0, st, a);
+        else if (D == 64 && split2) hipLaunchKernelGGL((combine_kernel<64, 2, HIST, SHARED, 1024, 512>), g1, dim3(1024), 0, st, a);
+        else if (D == 64) hipLaunchKernelGGL((combine_kernel<64, 1, HIST, SHARED, 1024, 512>), g1, dim3(1024), 0, st, a);
         else return -1;
         return 0;
     }
-    if (D == 128 && split2) hipLaunchKernelGGL((combine_kernel<128, 2, HIST>), grid, dim3(1024), 0, st, a);
-    else if (D == 128 && small) hipLaunchKernelGGL((combine_kernel<128, 1, HIST, 512, 64>), grid, dim3(512), 0, st, a);
-    else if (D == 128) hipLaunchKernelGGL((combine_kernel<128, 1, HIST>), grid, dim3(1024), 0, st, a);
-    else if (D == 64 && split2) hipLaunchKernelGGL((combine_kernel<64, 2, HIST>), grid, dim3(1024), 0, st, a);
-    else if (D == 64 && small) hipLaunchKernelGGL((combine_kernel<64, 1, HIST, 512, 64>), grid, dim3(512), 0, st, a);
-    else if (D == 64) hipLaunchKernelGGL((combine_kernel<64, 1, HIST>), grid, dim3(1024), 0, st, a);
+    if (D == 128 && split2) hipLaunchKernelGGL((combine_kernel<128, 2, HIST, SHARED>), grid, dim3(1024), 0, st, a);
+    else if (D == 128 && small) hipLaunchKernelGGL((combine_kernel<128, 1, HIST, SHARED, 512, 64>), grid, dim3(512), 0, st, a);
+    else if (D == 128) hipLaunchKernelGGL((combine_kernel<128, 1, HIST, SHARED>), grid, dim3(1024), 0, st, a);
+    else if (D == 64 && split2) hipLaunchKernelGGL((combine_kernel<64, 2, HIST, SHARED>), grid, dim3(1024), 0, st, a);
+    else if (D == 64 && small) hipLaunchKernelGGL((combine_kernel<64, 1, HIST, SHARED, 512, 64>), grid, dim3(512), 0, st, a);
+    else if (D == 64) hipLaunchKernelGGL((combine_kernel<64, 1, HIST, SHARED>), grid, dim3(1024), 0, st, a);
     else return -1;
     return 0;
 }
 
 int launch_combine(const CombineArgs& a, int D, hipStream_t st) {
-    return a.hist_seq ? launch_combine_rows<true>(a, D, st) : launch_combine_rows<false>(a, D, st);
+    if (a.share_count)
+        return a.hist_seq ? launch_combine_rows<true, true>(a, D, st) : launch_combine_rows<false, true>(a, D, st);
+    return a.hist_seq ? launch_combine_rows<true, false>(a, D, st) : launch_combine_rows<false, false>(a, D, st);
 }
 
 }  // namespace ommx

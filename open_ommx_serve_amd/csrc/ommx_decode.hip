@@ -36,6 +36,7 @@
 //            heads, only softmax and the A operands double.
 #include <type_traits>
 
+#include "ommx_decode_shares.h"
 #include "ommx_decode_util.h"
 
 namespace ommx {
@@ -123,10 +124,12 @@ __global__ void __launch_bounds__(256, 2) decode_splitkv_mfma_kernel(DecodeArgs 
     const int hg = HR == 8 ? (kq & 1) : 0;
     const int Hkv = a.Hkv;
     const int waves = blockDim.x >> 6;
-    const int kvh = blockIdx.y * waves + wave;
+    // (shares: the head groups vary fastest, so that the shares nobody needs are dispatched last)
+    const bool dealt = ORDER >= 1 && a.shares > 0;
+    const int kvh = (dealt ? blockIdx.x : blockIdx.y) * waves + wave;
     const int heads = PARTIAL ? a.Hq / Hkv : HR;      // q heads this kv head really serves
     const int qh0 = kvh * heads;          // first of this wave's q heads
-    const int sp = blockIdx.x;
+    int sp = blockIdx.x, S = a.S;
     // Requests are served longest first: workgroups are dispatched in grid order, so the ones that
     // start last, when most compute units have run dry, belong to the shortest requests.
     // blockIdx.z is the rank of the request by (length descending, index ascending); every wave
@@ -134,7 +137,11 @@ __global__ void __launch_bounds__(256, 2) decode_splitkv_mfma_kernel(DecodeArgs 
     // above its own; up to 256 (four keys per lane) by a radix select of the key of that rank,
     // one bit per round (the serving recipe's instantiations only); more keep the grid order.
     int b = blockIdx.z, L;
-    if (ORDER >= 1 && a.B > 1 && a.B <= 64) {
+    if (dealt) {
+        shares::Share mine;
+        if (!shares::find_share<(32 << GTS), ORDER == 2 ? 4 : 1>(a, blockIdx.y, lane, mine)) return;
+        b = mine.b; L = mine.L; sp = static_cast<int>(mine.sp); S = static_cast<int>(mine.n);
+    } else if (ORDER >= 1 && a.B > 1 && a.B <= 64) {
         const int my_len = lane < a.B ? a.seq[lane] : 0;
         const uint32_t key = (static_cast<uint32_t>(my_len) << 6) | (63u - lane);   // distinct per lane
         int rank = 0;
@@ -189,7 +196,7 @@ __global__ void __launch_bounds__(256, 2) decode_splitkv_mfma_kernel(DecodeArgs 
     static_assert(GTS == 0 || IDX == 1, "longer groups are read through position streams");
     static_assert(KO == 6 || (KO == 10 && IDX == 1), "10 outliers: position streams only");
     if (L < 0) { L = 0; report_table_range(a.err, true); }      // a negative length: nothing packed, reported
-    const int per = ((((L + a.S - 1) / a.S) + GT - 1) / GT) * GT;
+    const int per = ((((L + S - 1) / S) + GT - 1) / GT) * GT;
     const int n_begin = per * sp;
     const int n_end = min(n_begin + per, L);
     const float c_log2e = 1.4426950408889634f;
@@ -329,7 +336,7 @@ __global__ void __launch_bounds__(256, 2) decode_splitkv_mfma_kernel(DecodeArgs 
             float* dst = a.al + b * a.al_b + (int64_t)(qh0 + r) * a.al_h + (int64_t)sp * a.al_s;
             dst[lane] = 0.0f;
             dst[64 + lane] = 0.0f;
-            if (lane == 0) dst[D] = -INFINITY;
+            if (lane == 0) a.sl[b * a.sl_b + (int64_t)(qh0 + r) * a.sl_h + (int64_t)sp * a.sl_s] = -INFINITY;
         }
         return;
     }
@@ -824,10 +831,9 @@ __global__ void __launch_bounds__(256, 2) decode_splitkv_mfma_kernel(DecodeArgs 
         }
     }
     if (j < 4 && kq < HR / 4 && 4 * kq + j < heads) {     // lane 16*hg + r holds head 4*hg + r
-        float* dst = a.al + b * a.al_b + (int64_t)(qh0 + 4 * kq + j) * a.al_h + (int64_t)sp * a.al_s;
         const float lt = j == 0 ? l_tot[0] : (j == 1 ? l_tot[1] : (j == 2 ? l_tot[2] : l_tot[3]));
         const float mt = j == 0 ? m_run[0] : (j == 1 ? m_run[1] : (j == 2 ? m_run[2] : m_run[3]));
-        dst[D] = lt > 0.0f ? (mt + log2f(lt)) * 0.6931471805599453f : -INFINITY;
+        a.sl[b * a.sl_b + (int64_t)(qh0 + 4 * kq + j) * a.sl_h + (int64_t)sp * a.sl_s] = lt > 0.0f ? (mt + log2f(lt)) * 0.6931471805599453f : -INFINITY;
     }
 }
 
@@ -848,7 +854,10 @@ int launch_decode_fast(const DecodeArgs& a, int Dh, int R, hipStream_t st) {
     // the kernel reads q two channels at a time
     if ((reinterpret_cast<uintptr_t>(a.q) & 3) || (a.q_sb & 1) || (a.q_sh & 1)) return 1;
     const int waves = (a.Hkv % 4 == 0) ? 4 : ((a.Hkv % 2 == 0) ? 2 : 1);    // one wave per kv head
-    const dim3 grid(a.S, a.Hkv / waves, a.B), block(64 * waves);
+    // shares: one request per lane, or four in the serving recipe's instantiations
+    if (a.shares > 0 && a.B > (a.kout == 6 && !longer && R >= 4 ? 256 : 64)) return 1;
+    const dim3 grid = a.shares > 0 ? dim3(a.Hkv / waves, a.shares) : dim3(a.S, a.Hkv / waves, a.B);
+    const dim3 block(64 * waves);
     const size_t shm = (size_t)waves * (R <= 4 ? (a.kout > 0 ? LdsMap<4>::END : LdsMap<4>::DT)
                                                : (a.kout > 0 ? LdsMap<8>::END : LdsMap<8>::DT));
     const bool own_map = a.k_ms != nullptr;

@@ -26,6 +26,16 @@ struct DecodeArgs {
     // OR-ed into *err (may be NULL).  0 = extent not given: ids are used as they are.
     int n_pages, n_gslots;
     int32_t* err;
+    // Where the lse of a state goes: attn_logits' column D of the C ABI, or a plane of its own (the caller's workspace
+    // has rows of D + 1; in a workspace of our own the rows are D floats, aligned, and the merge reads the lse of all
+    // states of a head from a few cache lines).
+    float* sl; int64_t sl_b, sl_h, sl_s;
+    // Work dealt out in shares instead of a fixed number of splits per request (ommx_decode_shares.h): workgroups along
+    // x with a third resident workgroup per compute unit and without, the most groups of a batch that get a share
+    // each, and where the kernel leaves the number of shares of every request (at most S) for the combine.
+    // shares 0: fixed splits.
+    int shares, shares_few, singles;
+    int32_t* share_count;
     // set by the launcher of the serving-recipe kernel only: head_dim is 64 and Hkv counts PAIRS of kv
     // heads (the planes of two neighbouring 64-channel heads read like one 128-channel head)
     int half;
@@ -71,12 +81,15 @@ struct CombineArgs {
     int gt;                          // tokens per K group: the splits are rounded to it
     int T;                           // rows every request's tail buffer holds (0: not told): rows below it
                                      // may be read before b_tail_len has arrived
+    const float* sl; int64_t sl_b, sl_h, sl_s;      // lse of the states, as in DecodeArgs
     uint16_t* o16;                   // bf16 output in place of o (same strides); NULL: fp32 into o
     // Tail rows read in place from the row history instead of a gathered buffer: kt / vt are the histories, kt_b
     // the elements between two requests' histories, and the rows follow from the sequence length (TailRows below).
     const int64_t* hist_seq;         // NULL: gathered buffer
     const int64_t* hist_slots;       // NULL: request b uses history b
     int hist_rows, ring_sink, ring_span, win_sink, win_recent;
+    const int32_t* share_count;      // states of every request (at most S); NULL: S each
+    int sure;                        // state slots to read before share_count is here (S without it)
 };
 
 // The bf16 rows of one request: how many, and where row t of them lies (elements from the K / V base pointers).

@@ -38,6 +38,7 @@
 //   P.V      A = (1 + code/4 | 1 + code/16) * 2^e_v as f16 for 8 tokens of one channel, B = p (f16).
 #include <type_traits>
 
+#include "ommx_decode_shares.h"
 #include "ommx_decode_util.h"
 
 namespace ommx {
@@ -150,14 +151,19 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
     const int j = lane & 15, kq = lane >> 4;
     const int Hkv = a.Hkv;
     const int waves = blockDim.x >> 6;
-    const int kvh = blockIdx.y * waves + wave;
+    // (shares: the head groups vary fastest, so that the shares nobody needs are dispatched last)
+    const bool dealt = ORDER >= 1 && a.shares > 0;
+    const int kvh = (dealt ? blockIdx.x : blockIdx.y) * waves + wave;
     const int heads = PARTIAL ? a.Hq / Hkv : NH;
     const int qh0 = kvh * heads;
     const int r_half = max(heads >> 1, 1);            // head_dim 64: q heads per kv head of the pair
-    const int Dout = half ? 64 : D;                   // channels of an output state
-    const int sp = blockIdx.x;
+    uint32_t sp = blockIdx.x, S = static_cast<uint32_t>(a.S);
     int b = ORDER == 0 ? 0 : static_cast<int>(blockIdx.z), L;      // ORDER 0 is launched for one request only
-    if (ORDER >= 1 && a.B > 1 && a.B <= 64) {
+    if (dealt) {
+        shares::Share mine;
+        if (!shares::find_share<32, ORDER == 2 ? 4 : 1>(a, blockIdx.y, lane, mine)) return;
+        b = mine.b; L = mine.L; sp = mine.sp; S = mine.n;
+    } else if (ORDER >= 1 && a.B > 1 && a.B <= 64) {
         const int my_len = lane < a.B ? a.seq[lane] : 0;
         const uint32_t key = (static_cast<uint32_t>(my_len) << 6) | (63u - lane);
         int rank = 0;
@@ -193,11 +199,11 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
     // and channels 2*lane, 2*lane+1 of every head (for the channel pass)
     uint32_t qw[16], qraw[NH];      // qraw: channels 2*lane, 2*lane+1 of every head, for the thresholds below
     {
-        const int slot = min(j & (NH - 1), heads - 1);
-        // head_dim 64: the head's 64 channels are the pair's channels 64 * (slot / r_half) .. + 63
-        const bool q_real = !half || (kq >> 1) == slot / r_half;
+        const int hs = min(j & (NH - 1), heads - 1);
+        // head_dim 64: the head's 64 channels are the pair's channels 64 * (hs / r_half) .. + 63
+        const bool q_real = !half || (kq >> 1) == hs / r_half;
         const uint32_t* qh = reinterpret_cast<const uint32_t*>(
-            a.q + b * a.q_sb + (int64_t)(qh0 + slot) * a.q_sh + (half ? 32 * (kq & 1) : 32 * kq));
+            a.q + b * a.q_sb + (int64_t)(qh0 + hs) * a.q_sh + (half ? 32 * (kq & 1) : 32 * kq));
 #pragma unroll
         for (int i = 0; i < 16; ++i) qw[i] = q_real ? qh[i] : 0u;
 #pragma unroll
@@ -240,7 +246,7 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
     // G >= S.  (One 32-bit division; the combine weighs the states by their lse, -inf for an
     // empty split, so it need not know this rule.)
     if (L < 0) { L = 0; report_table_range(a.err, true); }      // a negative length: nothing packed, reported
-    const uint32_t G = static_cast<uint32_t>(L + 31) >> 5, S = static_cast<uint32_t>(a.S);
+    const uint32_t G = static_cast<uint32_t>(L + 31) >> 5;
     const uint32_t g_each = G / S, g_more = G - g_each * S;
     const uint32_t g_first = static_cast<uint32_t>(sp) * g_each + min(static_cast<uint32_t>(sp), g_more);
     const uint32_t g_count = g_each + (static_cast<uint32_t>(sp) < g_more ? 1u : 0u);
@@ -252,7 +258,7 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
             float* dst = a.al + b * a.al_b + (int64_t)(qh0 + r) * a.al_h + (int64_t)sp * a.al_s;
             dst[lane] = 0.0f;
             if (!half) dst[64 + lane] = 0.0f;
-            if (lane == 0) dst[Dout] = -INFINITY;
+            if (lane == 0) a.sl[b * a.sl_b + (int64_t)(qh0 + r) * a.sl_h + (int64_t)sp * a.sl_s] = -INFINITY;
         }
         return;
     }
@@ -967,7 +973,7 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
         if (x == 0 && kqe == (NH == 8 ? (h >> 2) : 0)) {
             const int hr = h & 3;
             const float mt = hr == 0 ? m_run[0] : (hr == 1 ? m_run[1] : (hr == 2 ? m_run[2] : m_run[3]));
-            dst[Dout] = l_tot > 0.0f ? (mt + log2f(l_tot)) * 0.6931471805599453f : -INFINITY;
+            a.sl[b * a.sl_b + (int64_t)(qh0 + h) * a.sl_h + (int64_t)sp * a.sl_s] = l_tot > 0.0f ? (mt + log2f(l_tot)) * 0.6931471805599453f : -INFINITY;
         }
     }
 }
@@ -1002,7 +1008,10 @@ int launch_decode_gqa4(const DecodeArgs& a_in, int Dh, int R, hipStream_t st) {
     const bool general = a.half || a.kout != 6;
     if (general && a.idx_repr != 0) return 1;       // the general form reads bitmaps only
     const int waves = (a.Hkv % 4 == 0) ? 4 : ((a.Hkv % 2 == 0) ? 2 : 1);
-    const dim3 grid(a.S, a.Hkv / waves, a.B), block(64 * waves);
+    // shares: the orders below hold up to 64 requests (one per lane), or 256 (four)
+    if (a.shares > 0 && a.B > (nh < 4 && !general ? 64 : 256)) return 1;
+    const dim3 grid = a.shares > 0 ? dim3(a.Hkv / waves, a.shares) : dim3(a.S, a.Hkv / waves, a.B);
+    const dim3 block(64 * waves);
     const size_t shm = (size_t)waves * (nh == 8 ? LdsMap<8>::LDS_WAVE : LdsMap<4>::LDS_WAVE);
     const bool own_map = a.k_ms != nullptr;
     const int order = a.B == 1 ? 0 : (a.B > 64 && a.B <= 256 ? 2 : 1);

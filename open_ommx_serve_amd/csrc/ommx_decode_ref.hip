@@ -241,7 +241,7 @@ __global__ void __launch_bounds__(256) decode_splitkv_ref_kernel(DecodeArgs a) {
         const float l = s_p[8 + r];
         float* dst = a.al + b * a.al_b + (int64_t)(kvh * R + r) * a.al_h + (int64_t)sp * a.al_s;
         dst[d] = l > 0.0f ? s / l : 0.0f;
-        if (d == 0) dst[D] = l > 0.0f ? s_p[r] + __logf(l) : -INFINITY;
+        if (d == 0) a.sl[b * a.sl_b + (int64_t)(kvh * R + r) * a.sl_h + (int64_t)sp * a.sl_s] = l > 0.0f ? s_p[r] + __logf(l) : -INFINITY;
     }
 }
 

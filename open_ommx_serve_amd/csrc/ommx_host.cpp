@@ -235,64 +235,103 @@ int run_decode(const DecodeCall& c) {
     }
     if (c.err && (c.err->scalar_type() != at::kInt || !on(c.err, dev))) return 0;
 
-    // splits and the workspace of their partial states
     if (c.splits == 0 && c.max_seq < 0) return 0;
-    int64_t S = c.splits;
-    if (S == 0) {
-        // The serving-recipe kernel keeps three workgroups per compute unit resident with up to 4 q heads per
-        // kv head (two with 8, and so do the other kernels); at head_dim 64 one of its waves takes a pair of kv heads.
-        const bool plain_planes = gt == 32 && gc == 32 && !scale_bf16 && !v_bf16 && !c.force;
-        const bool lean = plain_planes && ((D == 128 && R <= 4 && k == 6) ||
-                                           (c.bitmap && k >= 1 && k <= 6 && ((D == 128 && R <= 4) ||
-                                                                             (D == 64 && R <= 2 && Hkv % 2 == 0))));
-        const bool paired = plain_planes && D == 64 && c.bitmap && k >= 1 && k <= 8 && R <= 4 && Hkv % 2 == 0;
-        S = auto_splits(c.max_seq, B, paired ? Hkv / 2 : Hkv, cu_count(dev.index()), gt, c.mean, lean ? 3 : 2);
-    }
-    if (c.ws && (c.ws->scalar_type() != at::kFloat || c.ws->dim() != 4 || c.ws->size(0) != B || c.ws->size(1) != Hq ||
-                 c.ws->size(2) < S || c.ws->size(3) < D + 1 || c.ws->stride(3) != 1))
-        return 0;
+    // The serving-recipe kernel keeps three workgroups per compute unit resident with up to 4 q heads per
+    // kv head (two with 8, and so do the other kernels); at head_dim 64 one of its waves takes a pair of kv heads.
+    const bool plain_planes = gt == 32 && gc == 32 && !scale_bf16 && !v_bf16 && !c.force;
+    const bool lean = plain_planes && ((D == 128 && R <= 4 && k == 6) ||
+                                       (c.bitmap && k >= 1 && k <= 6 && ((D == 128 && R <= 4) ||
+                                                                         (D == 64 && R <= 2 && Hkv % 2 == 0))));
+    const bool paired = plain_planes && D == 64 && c.bitmap && k >= 1 && k <= 8 && R <= 4 && Hkv % 2 == 0;
+    const int64_t wave_heads = paired ? Hkv / 2 : Hkv;           // waves that one share of the tokens takes
 
     c10::hip::HIPGuard guard(dev.index());
     hipStream_t stream = stream_of(dev);
-    int64_t al_b = Hq * (S + 1) * (D + 1), al_h = (S + 1) * (D + 1), al_s = D + 1;
-    c10::DataPtr scratch;
-    float *al, *lse = data<float>(c.lse);
-    if (c.ws && c.lse) {
-        al = c.ws->data_ptr<float>();
-        al_b = c.ws->stride(0); al_h = c.ws->stride(1); al_s = c.ws->stride(2);
-    } else {
-        scratch = c10::GetAllocator(c10::DeviceType::CUDA)->allocate(static_cast<size_t>(B * (al_b + Hq)) * sizeof(float));
-        al = static_cast<float*>(scratch.get());
-        if (!lse) lse = al + B * al_b;
-    }
+    c10::Allocator* const allocator = c10::GetAllocator(c10::DeviceType::CUDA);
     const uint16_t* qp = data<const uint16_t>(c.q);
-    int rc, rc2 = 0;
-    Py_BEGIN_ALLOW_THREADS
-    rc = (c.force ? ommx_decode_splitkv_ref : ommx_decode_splitkv)(
-        qp, q.stride(0), q.stride(1), data<uint8_t>(c.k_base), data(c.k_scale), data<uint16_t>(c.k_zp),
-        own_map ? data<uint16_t>(c.ms) : nullptr, own_map ? data<uint16_t>(c.mc) : nullptr,
-        k > 0 ? data<uint8_t>(c.k_index) : nullptr, k > 0 ? data<uint8_t>(c.k_oval) : nullptr, data<uint8_t>(c.v_main),
-        data(c.v_scale), data<uint16_t>(c.v_zp), data(c.rt), rt.stride(0), data(c.rg), rg.stride(0),
-        rt.scalar_type() == at::kLong, data<int32_t>(c.seq), al, al_b, al_h, al_s, B, Hq, Hkv, D, ps, k,
-        c.bitmap ? OMMX_INDEX_BITMAP : OMMX_INDEX_RELIDX7, scale_bf16, gt, gc, v_bf16, S, c.sm_scale, c.cap, c.off,
-        c.gbase, pages, slots, data<int32_t>(c.err), stream);
-    if (rc == 0 && hist) {
-        const ommx::HistTail t{data<uint16_t>(kt), data<uint16_t>(vt), kt->stride(0), static_cast<int>(kt->size(1)),
-                               data<int64_t>(c.hist_seq), data<int64_t>(c.hist_slots), static_cast<int>(c.ring_sink),
-                               static_cast<int>(c.ring_span), static_cast<int>(c.win_sink), static_cast<int>(c.win_recent)};
-        rc2 = ommx::decode_combine_hist(al, al_b, al_h, al_s, qp, q.stride(0), q.stride(1), t, data(c.o), o_bf16,
-                                        c.o->stride(0), c.o->stride(1), lse, c.lse ? c.lse->stride(0) : Hq, B, Hq, Hkv,
-                                        D, S, gt, c.sm_scale, c.cap, stream);
-    } else if (rc == 0) {
-        rc2 = ommx_decode_combine(
+    auto combine = [&](const float* al, int64_t al_b, int64_t al_h, int64_t al_s, float* lse, int64_t S, const ommx::StateLse* states,
+                       const ommx::Shares* dealt) {
+        if (hist) {
+            const ommx::HistTail t{data<uint16_t>(kt), data<uint16_t>(vt), kt->stride(0), static_cast<int>(kt->size(1)),
+                                   data<int64_t>(c.hist_seq), data<int64_t>(c.hist_slots), static_cast<int>(c.ring_sink),
+                                   static_cast<int>(c.ring_span), static_cast<int>(c.win_sink), static_cast<int>(c.win_recent)};
+            return ommx::decode_combine_hist(al, al_b, al_h, al_s, qp, q.stride(0), q.stride(1), t, data(c.o), o_bf16,
+                                             c.o->stride(0), c.o->stride(1), lse, c.lse ? c.lse->stride(0) : Hq, B, Hq,
+                                             Hkv, D, S, gt, c.sm_scale, c.cap, *states, dealt, stream);
+        }
+        return ommx::decode_combine(
             al, al_b, al_h, al_s, qp, q.stride(0), q.stride(1), tail ? data<uint16_t>(kt) : nullptr,
             tail ? data<uint16_t>(vt) : nullptr, tail ? kt->stride(0) : 0, tail ? kt->stride(1) : 0,
             tail ? kt->stride(2) : 0, tail ? vt->stride(0) : 0, tail ? vt->stride(1) : 0, tail ? vt->stride(2) : 0,
             tail ? data<int32_t>(c.b_tail) : nullptr, data<int32_t>(c.seq), data<float>(c.o), c.o->stride(0),
             c.o->stride(1), lse, c.lse->stride(0), B, Hq, Hkv, D, S, gt, tail ? kt->size(1) : 0, c.sm_scale, c.cap,
-            stream);
+            states, dealt, stream);
+    };
+    // (the argument list that the split-KV entries share; the state strides and the split count come first)
+#define OMMX_SPLITKV_ARGS(AL, AL_B, AL_H, AL_S, SPLITS)                                                                  \
+    qp, q.stride(0), q.stride(1), data<uint8_t>(c.k_base), data(c.k_scale), data<uint16_t>(c.k_zp),                      \
+        own_map ? data<uint16_t>(c.ms) : nullptr, own_map ? data<uint16_t>(c.mc) : nullptr,                              \
+        k > 0 ? data<uint8_t>(c.k_index) : nullptr, k > 0 ? data<uint8_t>(c.k_oval) : nullptr, data<uint8_t>(c.v_main),  \
+        data(c.v_scale), data<uint16_t>(c.v_zp), data(c.rt), rt.stride(0), data(c.rg), rg.stride(0),                     \
+        rt.scalar_type() == at::kLong, data<int32_t>(c.seq), AL, AL_B, AL_H, AL_S, B, Hq, Hkv, D, ps, k,                 \
+        c.bitmap ? OMMX_INDEX_BITMAP : OMMX_INDEX_RELIDX7, scale_bf16, gt, gc, v_bf16, SPLITS, c.sm_scale, c.cap, c.off, \
+        c.gbase, pages, slots, data<int32_t>(c.err), stream
+
+    int rc = 1, rc2 = 0;
+    if (c.splits == 0 && !c.ws && !c.force && B > 1) {
+        // Several requests and nobody asked for a split count: the kernels deal the groups out in equal shares, as many
+        // as are resident at once (a wave per kv head and share).  One request gets at most 256 of them (its states
+        // are merged on chip), 64 with many (request, head) pairs, where the combine's small form serves, and no
+        // more than four times its even part, which bounds the workspace.
+        const int64_t fit = cu_count(dev.index()) * 4 / wave_heads;
+        // (max_seq bounds how many groups there can be; were it too small, the shares would be longer, nothing else)
+        const int64_t longest = std::max<int64_t>(1, (c.max_seq + gt - 1) / gt);
+        const int64_t shares = std::min({int64_t{2048}, fit * (lean ? 3 : 2), B * longest}), few = std::min(shares, fit * 2);
+        const int64_t most = std::min({int64_t{B * Hq >= 256 ? 64 : (shares > 256 * B && longest > 512 ? 512 : 256)}, longest,
+                                       std::max<int64_t>(8, 4 * shares / B)});
+        // A batch of fewer groups than one and a half waves per SIMD is left to fixed splits: no wave gets more than
+        // one step either way, and those need not find their share (0.3 us, and as much again in the combine).
+        if (few >= B && 2 * B * longest > 3 * fit) {
+            const int64_t n = B * Hq * most, singles = paired ? 2 * fit : fit;
+            c10::DataPtr scratch = allocator->allocate(static_cast<size_t>(n * (D + 1) + B * Hq + B) * sizeof(float));
+            float *al = static_cast<float*>(scratch.get()), *lse = c.lse ? data<float>(c.lse) : al + n * (D + 1);
+            const ommx::StateLse states{al + n * D, Hq * most, most, 1};
+            const ommx::Shares dealt{static_cast<int>(shares), static_cast<int>(few), static_cast<int>(singles),
+                                     static_cast<int>((std::min(shares, B * longest > singles ? B * longest / 2 : shares) + B - 1) / B),
+                                     reinterpret_cast<int32_t*>(al + n * (D + 1) + B * Hq)};
+            Py_BEGIN_ALLOW_THREADS
+            rc = ommx::decode_splitkv(OMMX_SPLITKV_ARGS(al, Hq * most * D, most * D, D, most), false, &states, &dealt);
+            if (rc == 0) rc2 = combine(al, Hq * most * D, most * D, D, lse, most, &states, &dealt);
+            Py_END_ALLOW_THREADS
+        }
     }
-    Py_END_ALLOW_THREADS
+    if (rc == 1) {
+        int64_t S = c.splits;
+        if (S == 0) S = auto_splits(c.max_seq, B, wave_heads, cu_count(dev.index()), gt, c.mean, lean ? 3 : 2);
+        if (c.ws && (c.ws->scalar_type() != at::kFloat || c.ws->dim() != 4 || c.ws->size(0) != B || c.ws->size(1) != Hq ||
+                     c.ws->size(2) < S || c.ws->size(3) < D + 1 || c.ws->stride(3) != 1))
+            return 0;
+        const int64_t n = B * Hq * S;
+        int64_t al_b = Hq * S * D, al_h = S * D, al_s = D;
+        c10::DataPtr scratch;
+        float *al, *lse = data<float>(c.lse);
+        ommx::StateLse states;
+        if (c.ws && c.lse) {
+            al = c.ws->data_ptr<float>();
+            al_b = c.ws->stride(0); al_h = c.ws->stride(1); al_s = c.ws->stride(2);
+            states = {al + D, al_b, al_h, al_s};
+        } else {
+            scratch = allocator->allocate(static_cast<size_t>(n * (D + 1) + B * Hq) * sizeof(float));
+            al = static_cast<float*>(scratch.get());
+            states = {al + n * D, Hq * S, S, 1};
+            if (!lse) lse = al + n * (D + 1);
+        }
+        Py_BEGIN_ALLOW_THREADS
+        rc = ommx::decode_splitkv(OMMX_SPLITKV_ARGS(al, al_b, al_h, al_s, S), c.force, &states, nullptr);
+        if (rc == 0) rc2 = combine(al, al_b, al_h, al_s, lse, S, &states, nullptr);
+        Py_END_ALLOW_THREADS
+    }
+#undef OMMX_SPLITKV_ARGS
     return failed(rc, "ommx_decode_splitkv") || failed(rc2, "ommx_decode_combine") ? -1 : 1;
 }
 

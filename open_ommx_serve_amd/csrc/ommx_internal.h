@@ -37,6 +37,16 @@ int pack_list(const int32_t* host_pairs, int n, int32_t* src_rows, int32_t* dst_
               int ppg, int hist_rows, int sink, int span, int window_sink, int groups_per_seq, int pages_per_seq,
               void* stream);
 
+// Where the log-sum-exp of the split states lies when it is not column D of the states.
+struct StateLse { float* p; int64_t b, h, s; };
+
+// The packed groups of the whole batch dealt out in equal pieces (csrc/ommx_decode_shares.h) instead of num_splits per
+// request: at most `all` of them (`few`, if a third resident workgroup per compute unit does not pay), at most
+// num_splits for one request, single groups while the batch has no more than `singles`.  `each` is about what one of B requests of the same length gets;
+// count int32[B] receives
+// the number of pieces of every request, which the combine entries take.
+struct Shares { int all, few, singles, each; int32_t* count; };
+
 // Split combine with the tail rows read in place from a bf16 row history [requests, rows, Hkv, D]: positions
 // [0, min(win_sink, seq)) ++ [boundary, seq) of every request through the ring map, boundary being what
 // ommx_tail_gather computes without a lag.  Saves the gather launch and the gathered copy.  o is fp32, or bf16
@@ -51,7 +61,32 @@ struct HistTail {
 int decode_combine_hist(const float* attn_logits, int64_t al_b, int64_t al_h, int64_t al_s, const uint16_t* q,
                         int64_t q_b, int64_t q_h, const HistTail& tail, void* o, bool o_bf16, int64_t o_b, int64_t o_h,
                         float* lse, int64_t lse_b, int B, int Hq, int Hkv, int D, int num_splits, int group_tokens,
-                        float sm_scale, float logit_cap, void* stream);
+                        float sm_scale, float logit_cap, const StateLse& states, const Shares* shares, void* stream);
+
+// ommx_decode_splitkv / _ref (plain) with these choices (either may be NULL).  Returns 1, with nothing done, when shares
+// are asked for and no kernel with shares serves the call.
+#define OMMX_DECODE_DECL                                                                            \
+    const uint16_t* q, int64_t q_stride_b, int64_t q_stride_h, const uint8_t* k_base,               \
+    const void* k_scale, const uint16_t* k_zp, const uint16_t* k_ms, const uint16_t* k_mc,          \
+    const uint8_t* k_index, const uint8_t* k_oval, const uint8_t* v_main, const void* v_scale,      \
+    const uint16_t* v_zp, const void* req_to_token, int64_t rt_stride, const void* req_to_group,    \
+    int64_t rg_stride, int table_i64, const int32_t* b_seq_len, float* attn_logits,                 \
+    int64_t al_stride_b, int64_t al_stride_h, int64_t al_stride_s, int B, int Hq, int Hkv, int D,   \
+    int page_size, int k_outliers, int index_repr, int scale_bf16, int group_tokens,                \
+    int group_channels, int v_bf16, int num_splits, float sm_scale, float logit_cap,                \
+    int packed_start_offset, int seg_group_base, int num_pages, int num_group_slots,                \
+    int32_t* err_flag, void* stream
+int decode_splitkv(OMMX_DECODE_DECL, bool plain, const StateLse* lse, const Shares* shares);
+#undef OMMX_DECODE_DECL
+
+// ommx_decode_combine with the lse of the states elsewhere (NULL: column D) and the shares they come from (NULL:
+// num_splits states per request; else at most that many).
+int decode_combine(const float* attn_logits, int64_t al_b, int64_t al_h, int64_t al_s, const uint16_t* q, int64_t q_b,
+                   int64_t q_h, const uint16_t* k_tail, const uint16_t* v_tail, int64_t kt_b, int64_t kt_t, int64_t kt_h,
+                   int64_t vt_b, int64_t vt_t, int64_t vt_h, const int32_t* b_tail_len, const int32_t* b_seq_len,
+                   float* o, int64_t o_b, int64_t o_h, float* lse, int64_t lse_b, int B, int Hq, int Hkv, int D,
+                   int num_splits, int group_tokens, int tail_rows, float sm_scale, float logit_cap,
+                   const StateLse* states, const Shares* shares, void* stream);
 
 // Causal attention of B requests' prompt rows over their own K/V, rows host_starts[b] .. host_starts[b + 1] of
 // q [n, Hq, D], k / v [n, Hkv, D] (bf16, head_dim 64 or 128, 16-byte aligned rows, strides in elements); o fp32 or
