@@ -772,12 +772,13 @@ PyObject* py_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const double scale = as_double(a[5], ok);
     if (!ok || !read_ints(a[4], starts) || starts.size() < 2 || starts[0] < 0 || !q->is_cuda()) Py_RETURN_FALSE;
     for (size_t i = 1; i < starts.size(); ++i)
-        if (starts[i] < starts[i - 1]) Py_RETURN_FALSE;
+        if (starts[i] < starts[i - 1] || starts[i] - starts[i - 1] > ommx::kPrefillMaxRows) Py_RETURN_FALSE;
     for (const at::Tensor* t : {q, k, v, o})
         if (t->dim() != 3 || t->stride(2) != 1 || t->device() != q->device() || t->size(0) < starts.back()) Py_RETURN_FALSE;
     const int64_t Hq = q->size(1), Hkv = k->size(1), D = q->size(2);
     if (k->size(2) != D || v->size(2) != D || v->size(1) != Hkv || o->size(1) != Hq || o->size(2) != D ||
-        (D != 64 && D != 128) || Hkv < 1 || Hq % Hkv || !(scale > 0))
+        (D != 64 && D != 128) || Hkv < 1 || Hq % Hkv || !(scale > 0) ||
+        std::max(k->stride(0), v->stride(0)) >= ommx::kPrefillMaxStride)
         Py_RETURN_FALSE;
     for (const at::Tensor* t : {q, k, v, o}) {
         const bool is16 = t->scalar_type() == at::kBFloat16;

@@ -90,7 +90,10 @@ int decode_combine(const float* attn_logits, int64_t al_b, int64_t al_h, int64_t
 
 // Causal attention of B requests' prompt rows over their own K/V, rows host_starts[b] .. host_starts[b + 1] of
 // q [n, Hq, D], k / v [n, Hkv, D] (bf16, head_dim 64 or 128, 16-byte aligned rows, strides in elements); o fp32 or
-// bf16.  Weights of fp32 precision (csrc/ommx_prefill.hip).
+// bf16.  Weights of fp32 precision (csrc/ommx_prefill.hip).  A 64-key tile of K and of V is addressed by 32-bit byte
+// offsets, which bounds their row strides; a bit per tile of the longest request fits the kernel's LDS.
+constexpr int64_t kPrefillMaxStride = 1 << 24;
+constexpr int kPrefillMaxRows = 1 << 18;
 int prefill_attention(const uint16_t* q, int64_t q_t, int64_t q_h, const uint16_t* k, int64_t k_t, int64_t k_h,
                       const uint16_t* v, int64_t v_t, int64_t v_h, void* o, bool o_bf16, int64_t o_t, int64_t o_h,
                       const int64_t* host_starts, int B, int Hq, int Hkv, int D, float scale, void* stream);

@@ -3,23 +3,30 @@
 // Grouped-query heads, any number of requests per launch, head_dim 64 or 128.
 //
 // Precision is that of an fp32 softmax: q.k of bf16 operands is exact in the fp32 accumulator, the weights
-// p = exp2(s - m) are fp32, and they enter P.V whole: p is cut into three bf16 pieces (8 + 8 + 8 bits,
-// by truncation, so p = p0 + p1 + p2 exactly) that go through three matrix instructions against the
-// same V operand.
+// p = exp2(s - m) are fp32 and enter P.V as two f16 pieces (11 bits, then the remainder rounded to 11: within
+// 2^-23 of the weight) against V times 2^8 in f16, which is exact for every bf16 of magnitude 2^-22 to 256
+// and zero.  A 64-key tile with any other V element is left out and follows after the loop with the weights in three
+// bf16 pieces and V as it is.  Against fp64, 4096 rows with K outliers: relative error 9.3e-7, the library's
+// fp32 attention 1.2e-6 (three bf16 pieces throughout: the same, with a third more PV instructions).
 //
-// Layout.  A workgroup is four waves = 128 query rows of one q head; a wave owns 32 rows and walks the keys
-// 64 at a time with mfma_f32_32x32x16_bf16.  Scores are formed transposed, S^T = K.Q^T, so a lane
+// Layout.  A group of four waves = 128 query rows of one q head; a wave owns 32 rows and walks the keys
+// 64 at a time with mfma_f32_32x32x16.  Scores are formed transposed, S^T = K.Q^T, so a lane
 // holds 32 scores of ONE query row: maximum and sum are register work plus one exchange with the
 // other half of the wave.  The accumulator rows a lane holds (8j + 4*half + 0..3) are, in this order, what
 // the B operand of O^T = V^T.P^T wants for a 16-key block once V^T lists its keys in the same order,
-// so the weights never pass through LDS.  K rows and transposed V go to LDS, double buffered (64 KB,
-// two workgroups per compute unit), 16-byte chunks XOR-swizzled by row: reads of eight rows hit eight
-// different bank groups, and so do the transposing writes.  The next tile's rows are requested before a
-// tile is worked on.
+// so the weights never pass through LDS.  K rows and transposed V are double buffered in LDS (70 KB); the next tile's
+// rows are requested before a tile is worked on, through buffers that end with the request.
 //
-// Bound: matrix instructions, four units (one QK, three PV) where a bf16-weight kernel has two: 4096 tokens of
-// 32 heads are 275 GFLOP issued, 0.11 ms at the card's peak rate.  The library's fp32 attention took
-// 2.45 ms for them plus 0.1 ms of widening and repeating its inputs.
+// Bound: matrix instructions and vector instructions share a SIMD's time (next to a wave that issues matrix
+// instructions back to back another one keeps about half its vector rate).  4096 tokens of 32 heads:
+// 200 K clocks of matrix instructions (82 us at 2.4 GHz) and 220 K of vector ones in 377 K.  Two groups of waves in one
+// workgroup, one half a tile behind the other so that the matrix phase of one meets the vector phase of
+// the other, share the staged tiles as well: 264 -> 191 us (same box).  In lockstep, without the shift, the eight
+// waves took 210 us, as two workgroups of four 233 us; any register spilled in the loop costs more than
+// all of this, because its reload waits for the loads on their way (285 us).  Short prompts are latency: one group
+// per workgroup, two workgroups per compute unit (see prefill_attention).  The library's fp32 attention took 2.45 ms.
+#include <algorithm>
+
 #include "ommx_common.h"
 #include "ommx_internal.h"
 
@@ -28,9 +35,13 @@ namespace ommx {
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
 struct PrefillArgs {
     const uint16_t *q, *k, *v;
@@ -47,36 +58,66 @@ constexpr int QROWS = 128, KEYS = 64;
 constexpr int kTilesPerLaunch = kUploadWords / 3;
 struct TileList { int32_t w[kUploadWords]; };
 
-__device__ __forceinline__ f32x16 mfma32(u32x4 a, u32x4 b, f32x16 c) {
+__device__ __forceinline__ f32x16 mfma_bf16(u32x4 a, u32x4 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x16 mfma_f16(u32x4 a, u32x4 b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
 }
 __device__ __forceinline__ float other_half(float v) { return __shfl_xor(v, 32); }
 // high halves of two words: elements 0 and 1 of a packed bf16 pair, truncated
 __device__ __forceinline__ uint32_t hi_pair(float lo, float hi) {
     return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
 }
+// x less one half of a packed f16 pair, one instruction (the compiler converts first)
+__device__ __forceinline__ float minus_low(float x, f16x2 h) {
+    float r;
+    asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(x));
+    return r;
+}
+__device__ __forceinline__ float minus_high(float x, f16x2 h) {
+    float r;
+    asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(x));
+    return r;
+}
+__device__ __forceinline__ u32x4 load16(__amdgpu_buffer_rsrc_t rows, uint32_t at) {
+    return __builtin_amdgcn_raw_buffer_load_b128(rows, at, 0, 0);
+}
 
 // the running maximum is refreshed when a score (base 2) exceeds it by this: any bound that keeps
 // exp2 in range serves an online softmax, and most tiles then rescale nothing
 constexpr float MAX_SLACK = 8.0f;
+// weights are carried times 2^6 (at most 2^14 with the slack): the second f16 piece of a weight stays
+// accurate to 2^-31 of the largest.  V is carried times 2^8 and divided by it at the end.
+constexpr float P_SHIFT = 6.0f, V_GAIN = 256.0f;
+// a bf16 value times 2^8 is exactly an f16 when its magnitude bits are 0 or in this range (2^-22 to 256)
+constexpr unsigned short V_LOW = (104 + 1) << 7, V_HIGH = ((104 + 31) << 7) - 1;
 
-template <int D>
-__global__ void __launch_bounds__(256, 2) prefill_kernel(PrefillArgs a, TileList tiles) {
+// LDS rows are 16 bytes longer than their data: eight neighbouring rows start in different bank groups, and every
+// operand read is one lane address plus an immediate offset (an XOR swizzle kept 36 addresses in registers)
+constexpr int k_stride(int D) { return 2 * D + 16; }
+constexpr int V_STRIDE = 2 * KEYS + 16;
+
+template <int D, int GROUPS>
+__global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a, TileList tiles) {
     constexpr int KB = D / 16;           // 16-channel blocks of QK
     constexpr int DB = D / 32;           // 32-channel blocks of the output
     constexpr int CHUNKS = D / 8;        // 16-byte chunks of a K row
-    constexpr int K_BYTES = KEYS * D * 2, V_BYTES = D * KEYS * 2;
+    constexpr int KS = k_stride(D), VS = V_STRIDE;
     constexpr int KLOADS = KEYS * CHUNKS / 256;
-    extern __shared__ __attribute__((aligned(16))) uint8_t sm[];        // two buffers of K_BYTES + V_BYTES
+    __shared__ __attribute__((aligned(16))) uint8_t s_k[2][KEYS * KS], s_v[2][D * VS];
+    __shared__ uint32_t s_inexact[kPrefillMaxRows / KEYS / 32];          // bit per tile: some V element is no f16
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int col = lane & 31, half = lane >> 5;
+    const int col = lane & 31, half = lane >> 5, group = GROUPS == 2 ? wave >> 2 : 0;
     const int t0 = tiles.w[3 * blockIdx.y], len = tiles.w[3 * blockIdx.y + 1], q0 = tiles.w[3 * blockIdx.y + 2];
     // (neighbouring workgroups take neighbouring kv heads, so with 8 kv heads an XCD keeps to one)
-    const int kvh = blockIdx.x % a.Hkv, h = kvh * a.R + blockIdx.x / a.Hkv;
+    const int kvh = blockIdx.x % a.Hkv, part = blockIdx.x / a.Hkv;
+    const bool pair = GROUPS == 2 && a.R % 2 == 0;          // the groups take two q heads, else two row blocks of one
+    const int h = kvh * a.R + (pair ? 2 * part + group : part);
     const uint16_t* const kp = a.k + t0 * a.k_t + kvh * a.k_h;
     const uint16_t* const vp = a.v + t0 * a.v_t + kvh * a.v_h;
 
-    const int row_first = q0 + 32 * wave, row = row_first + col;         // of this wave, of this lane
+    const int row_first = q0 + 32 * (wave & 3) + (pair ? 0 : QROWS * group), row = row_first + col;   // of this wave, of this lane
     u32x4 qf[KB];
     {
         const uint16_t* qp = a.q + (t0 + min(row, len - 1)) * a.q_t + h * a.q_h + 8 * half;
@@ -88,138 +129,237 @@ __global__ void __launch_bounds__(256, 2) prefill_kernel(PrefillArgs a, TileList
     for (int d = 0; d < DB; ++d)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[d][r] = 0.0f;
-    float m = -INFINITY, l = 0.0f;
+    float m = -INFINITY, l = 0.0f;       // m: running maximum less P_SHIFT
 
-    const int n_tiles = (min(len, q0 + QROWS) + KEYS - 1) / KEYS;
+    // key tiles of the workgroup and of this wave (causal; a wave whose rows are past the end has none)
+    const int n_tiles = (min(len, q0 + (pair ? QROWS : GROUPS * QROWS)) + KEYS - 1) / KEYS;
+    const int n_mine = row_first < len ? min(n_tiles, (row_first + 31) / KEYS + 1) : 0;
 
-    // ---- staging: thread -> chunk tid % CHUNKS of K rows, and channels 8*d8.. of four neighbouring V rows
-    const int kc = tid % CHUNKS, kr = tid / CHUNKS;
-    const int d8 = tid % CHUNKS, kg = tid / CHUNKS;
-    constexpr int VGROUPS = KEYS / 4;                       // groups of four keys
-    const bool v_mine = kg < VGROUPS;                       // head_dim 64: half of the threads
-    u32x4 kn[KLOADS], vn[4];
-    auto request = [&](int k0) {
-#pragma unroll
-        for (int i = 0; i < KLOADS; ++i) {
-            const int key = min(k0 + kr + i * (256 / CHUNKS), len - 1);
-            kn[i] = *reinterpret_cast<const u32x4*>(kp + key * a.k_t + 8 * kc);
-        }
-        if (v_mine) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int key = min(k0 + 4 * kg + i, len - 1);
-                vn[i] = *reinterpret_cast<const u32x4*>(vp + key * a.v_t + 8 * d8);
-            }
-        }
+    // ---- staging.  The first group brings V: channels 8*d8.. of four neighbouring rows per thread, sixteen lanes write a
+    // whole row of transposed V (head_dim 64: half of the threads).  The second group brings K: chunk kc of rows kr, ...
+    const int st = tid & 255;
+    const int kc = st % CHUNKS, kr = st / CHUNKS;
+    const int kg = st % (KEYS / 4), d8 = st / (KEYS / 4);
+    const uint32_t k_row = static_cast<uint32_t>(a.k_t) * 2, v_row = static_cast<uint32_t>(a.v_t) * 2;
+    const uint32_t k_at = kr * k_row + 16 * kc, v_at = 4 * kg * v_row + 16 * d8;
+    u32x4 nx[GROUPS == 2 ? 4 : 8];       // rows on their way: V, K behind it (two groups: either)
+    u32x4* const nk = nx + (GROUPS == 2 ? 0 : 4);
+    // The rows of a tile as a buffer that ends with the request's last row: loads beyond it return zeros.
+    auto tile_rows = [&](const uint16_t* p, int64_t stride, int t) {
+        const int rows = min(len - t * KEYS, KEYS);
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p + t * KEYS * stride), 0,
+                                                 (rows - 1) * static_cast<int>(stride) * 2 + 2 * D, 0x00027000);
     };
-    auto stage = [&](uint8_t* buf) {
+    auto request_k = [&](int t) {
+        if (t >= n_tiles) return;
+        const auto rows = tile_rows(kp, a.k_t, t);
 #pragma unroll
-        for (int i = 0; i < KLOADS; ++i) {
-            const int r = kr + i * (256 / CHUNKS);
-            *reinterpret_cast<u32x4*>(buf + r * (2 * D) + 16 * (kc ^ (r & 7))) = kn[i];
-        }
-        if (v_mine) {
-            // keys 4kg..4kg+3 are block kg / 4, half kg & 1 of it, first or second four slots of that chunk
-            const int chunk = 2 * (kg >> 2) + (kg & 1), part = (kg >> 1) & 1;
+        for (int i = 0; i < KLOADS; ++i) nk[i] = load16(rows, k_at + i * (256 / CHUNKS) * k_row);
+    };
+    auto request_v = [&](int t) {
+        if (t >= n_tiles || d8 >= CHUNKS) return;
+        const auto rows = tile_rows(vp, a.v_t, t);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) nx[i] = load16(rows, v_at + i * v_row);
+    };
+    auto write_v = [&](int buf, const u32x4* f) {
+        // keys 4kg..4kg+3 are block kg / 4, half kg & 1 of it, first or second four slots of that chunk
+        uint8_t* const at = s_v[buf] + 8 * d8 * VS + 16 * (2 * (kg >> 2) + (kg & 1)) + 8 * ((kg >> 1) & 1);
+#pragma unroll
+        for (int w = 0; w < 4; ++w)
+#pragma unroll
+            for (int odd = 0; odd < 2; ++odd) {
+                const uint32_t sel = odd ? 0x07060302u : 0x05040100u;
+                *reinterpret_cast<u32x2*>(at + (2 * w + odd) * VS) =
+                    u32x2{__builtin_amdgcn_perm(f[1][w], f[0][w], sel), __builtin_amdgcn_perm(f[3][w], f[2][w], sel)};
+            }
+    };
+    auto stage_k = [&](int t) {
+        if (t >= n_tiles) return;
+#pragma unroll
+        for (int i = 0; i < KLOADS; ++i)
+            *reinterpret_cast<u32x4*>(s_k[t & 1] + (kr + i * (256 / CHUNKS)) * KS + 16 * kc) = nk[i];
+    };
+    auto stage_v = [&](int t) {
+        if (d8 >= CHUNKS) return;
+        // V * 2^8 as f16: the exponent field shifted down by 104, three more mantissa bits; zero stays zero
+        u16x2 low = {0xFFFF, 0xFFFF}, high = {0, 0};
+        u32x4 f[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
             for (int w = 0; w < 4; ++w) {
-#pragma unroll
-                for (int odd = 0; odd < 2; ++odd) {
-                    const uint32_t sel = odd ? 0x07060302u : 0x05040100u;
-                    const u32x2 four = {__builtin_amdgcn_perm(vn[1][w], vn[0][w], sel),
-                                        __builtin_amdgcn_perm(vn[3][w], vn[2][w], sel)};
-                    const int d = 8 * d8 + 2 * w + odd;
-                    *reinterpret_cast<u32x2*>(buf + K_BYTES + d * (2 * KEYS) + 16 * (chunk ^ (d & 7) ^ (d8 & 7)) + 8 * part) = four;
-                }
+                const uint32_t x = nx[i][w];
+                const u16x2 mag = __builtin_bit_cast(u16x2, x & 0x7FFF7FFFu);
+                low = __builtin_elementwise_min(low, mag - static_cast<unsigned short>(1));      // zero wraps to the top
+                high = __builtin_elementwise_max(high, mag);
+                const u16x2 bias = {104 << 7, 104 << 7};
+                f[i][w] = (x & 0x80008000u) | __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(mag, bias) << 3);
             }
+        if (min(low[0], low[1]) < V_LOW - 1 || max(high[0], high[1]) > V_HIGH) atomicOr(&s_inexact[t >> 5], 1u << (t & 31));
+        write_v(t & 1, f);
+    };
+    auto inexact = [&](int t) { return (__builtin_amdgcn_readfirstlane(s_inexact[t >> 5]) >> (t & 31)) & 1u; };
+
+    f32x16 s[2];                 // scores of the tile, transposed: lane's row is the query
+    u32x4 p0[4], p1[4];          // their weights in two f16 pieces, by 16-key block
+
+    auto v_operand = [&](int buf, int b, int d) {
+        return *reinterpret_cast<const u32x4*>(s_v[buf] + (32 * d + col) * VS + 32 * b + 16 * half);
+    };
+    auto scores = [&](int buf) {
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[g][r] = 0.0f;
+        u32x4 kf[2][2][2];
+        auto read = [&](int kb2) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                kf[kb2 & 1][i >> 1][i & 1] =
+                    *reinterpret_cast<const u32x4*>(s_k[buf] + (32 * (i & 1) + col) * KS + 32 * (2 * kb2 + (i >> 1)) + 16 * half);
+        };
+        read(0);
+#pragma unroll
+        for (int kb2 = 0; kb2 < KB / 2; ++kb2) {
+            if (kb2 + 1 < KB / 2) read(kb2 + 1);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s[i & 1] = mfma_bf16(kf[kb2 & 1][i >> 1][i & 1], qf[2 * kb2 + (i >> 1)], s[i & 1]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    auto mask = [&](int t) {
+        const int k0 = t * KEYS;
+        if (k0 + KEYS - 1 <= row_first) return;
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                if (k0 + 32 * g + 8 * (r >> 2) + 4 * half + (r & 3) > row) s[g][r] = -INFINITY;
+    };
+    // O^T += V^T.P^T of one tile
+    auto add_pv = [&](int t) {
+        if (inexact(t)) return;              // (follows after the loop)
+        u32x4 vf[2][DB];                     // operands one block ahead, no further: registers
+#pragma unroll
+        for (int d = 0; d < DB; ++d) vf[0][d] = v_operand(t & 1, 0, d);
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+#pragma unroll
+            for (int d = 0; d < DB; ++d)
+                if (b < 3) vf[(b + 1) & 1][d] = v_operand(t & 1, b + 1, d);
+#pragma unroll
+            for (int d = 0; d < DB; ++d) acc[d] = mfma_f16(vf[b & 1][d], p0[b], acc[d]);
+#pragma unroll
+            for (int d = 0; d < DB; ++d) acc[d] = mfma_f16(vf[b & 1][d], p1[b], acc[d]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    // vector phase: staging, then the online softmax of one row per lane
+    auto vector_phase = [&](int t) {
+        if (GROUPS == 1 || !group) { stage_v(t); request_v(t + 1); }
+        if (GROUPS == 1) { stage_k(t + 1); request_k(t + 2); }
+        else if (group) { stage_k(t + 2); request_k(t + 3); }
+        mask(t);
+        float mx = s[0][0];
+#pragma unroll
+        for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[0][r]);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[1][r]);
+        mx = fmaf(fmaxf(mx, other_half(mx)), a.scale_log2, -P_SHIFT);      // (the scale is positive)
+        if (__any(mx > m + MAX_SLACK)) {
+            const float m_new = fmaxf(m, mx);
+            const float shrink = __builtin_amdgcn_exp2f(m - m_new);       // 0 on the first tile
+            m = m_new;
+            l *= shrink;
+#pragma unroll
+            for (int d = 0; d < DB; ++d)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[d][r] *= shrink;
+        }
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float x = __builtin_amdgcn_exp2f(fmaf(s[b >> 1][8 * (b & 1) + 2 * i], a.scale_log2, -m));
+                const float y = __builtin_amdgcn_exp2f(fmaf(s[b >> 1][8 * (b & 1) + 2 * i + 1], a.scale_log2, -m));
+                l += x;
+                l += y;
+                const f16x2 hi = __builtin_convertvector((f32x2{x, y}), f16x2);
+                const f32x2 rest = {minus_low(x, hi), minus_high(y, hi)};
+                p0[b][i] = __builtin_bit_cast(uint32_t, hi);
+                p1[b][i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(rest, f16x2));
+            }
+        if (GROUPS == 2) {        // all of it here: the compiler would move the weights behind the barrier, to their use
+#pragma unroll
+            for (int b = 0; b < 4; ++b) asm volatile("" : "+v"(p0[b]), "+v"(p1[b]));
+            asm volatile("" : "+v"(l));
         }
     };
 
-    request(0);
-    stage(sm);
+    if (tid < kPrefillMaxRows / KEYS / 32) s_inexact[tid] = 0;
+    if (GROUPS == 1 || group) { request_k(0); stage_k(0); request_k(1); }
+    if (GROUPS == 1 || !group) request_v(0);
     __syncthreads();
-    for (int t = 0; t < n_tiles; ++t) {
-        const int k0 = t * KEYS;
-        uint8_t* const buf = sm + (t & 1) * (K_BYTES + V_BYTES);
-        if (t + 1 < n_tiles) request(k0 + KEYS);
-        if (row_first < len && k0 <= row_first + 31) {
-            // ---------------------------------------------------------------- S^T = K.Q^T
-            f32x16 s[2];
-#pragma unroll
-            for (int g = 0; g < 2; ++g) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) s[g][r] = 0.0f;
-                const int key = 32 * g + col;
-#pragma unroll
-                for (int kb = 0; kb < KB; ++kb) {
-                    const u32x4 kf = *reinterpret_cast<const u32x4*>(buf + key * (2 * D) + 16 * ((2 * kb + half) ^ (key & 7)));
-                    s[g] = mfma32(kf, qf[kb], s[g]);
-                }
-            }
-            // ---------------------------------------------------------------- online softmax of one row
-            if (k0 + KEYS - 1 > row_first) {
-#pragma unroll
-                for (int g = 0; g < 2; ++g)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        if (k0 + 32 * g + 8 * (r >> 2) + 4 * half + (r & 3) > row) s[g][r] = -INFINITY;
-            }
-            float mx = s[0][0];
-#pragma unroll
-            for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[0][r]);
-#pragma unroll
-            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[1][r]);
-            mx = fmaxf(mx, other_half(mx)) * a.scale_log2;      // (the scale is positive)
-            if (__any(mx > m + MAX_SLACK)) {
-                const float m_new = fmaxf(m, mx);
-                const float shrink = __builtin_amdgcn_exp2f(m - m_new);       // 0 on the first tile
-                m = m_new;
-                l *= shrink;
-#pragma unroll
-                for (int d = 0; d < DB; ++d)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) acc[d][r] *= shrink;
-            }
-#pragma unroll
-            for (int g = 0; g < 2; ++g)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    s[g][r] = __builtin_amdgcn_exp2f(fmaf(s[g][r], a.scale_log2, -m));
-                    l += s[g][r];
-                }
-            // ---------------------------------------------------------------- O^T += V^T.P^T
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                u32x4 p0, p1, p2;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const float x = s[b >> 1][8 * (b & 1) + 2 * i], y = s[b >> 1][8 * (b & 1) + 2 * i + 1];
-                    const float x1 = x - __uint_as_float(__float_as_uint(x) & 0xFFFF0000u);
-                    const float y1 = y - __uint_as_float(__float_as_uint(y) & 0xFFFF0000u);
-                    const float x2 = x1 - __uint_as_float(__float_as_uint(x1) & 0xFFFF0000u);
-                    const float y2 = y1 - __uint_as_float(__float_as_uint(y1) & 0xFFFF0000u);
-                    p0[i] = hi_pair(x, y);
-                    p1[i] = hi_pair(x1, y1);
-                    p2[i] = hi_pair(x2, y2);
-                }
-#pragma unroll
-                for (int d = 0; d < DB; ++d) {
-                    const int ch = 32 * d + col;
-                    const u32x4 vf = *reinterpret_cast<const u32x4*>(
-                        buf + K_BYTES + ch * (2 * KEYS) + 16 * ((2 * b + half) ^ (ch & 7) ^ ((ch >> 3) & 7)));
-                    acc[d] = mfma32(vf, p0, acc[d]);
-                    acc[d] = mfma32(vf, p1, acc[d]);
-                    acc[d] = mfma32(vf, p2, acc[d]);
-                }
-            }
-        }
-        if (t + 1 < n_tiles) stage(sm + ((t + 1) & 1) * (K_BYTES + V_BYTES));
+    if (group) {                  // one phase behind the first group
+        stage_k(1);
+        request_k(2);
         __syncthreads();
+    }
+    scores(0);
+    if (GROUPS == 2) __syncthreads();
+    for (int t = 0; t < n_tiles; ++t) {
+        vector_phase(t);
+        __syncthreads();
+        add_pv(t);
+        if (t + 1 < n_tiles) scores((t + 1) & 1);
+        else asm volatile("" : "=v"(s[0]), "=v"(s[1]));           // (keeps the scores out of the loop's registers)
+        if (GROUPS == 2 && (!group || t + 1 < n_tiles)) __syncthreads();
+    }
+
+    // Tiles whose V is not exact in f16: scores once more, weights against the final maximum in three bf16 pieces
+    // (8 + 8 + 8 bits by truncation, their sum is the weight), V as it is.
+    __syncthreads();
+    for (int w = 0; w <= (n_tiles - 1) >> 5; ++w) {
+        for (uint32_t left = __builtin_amdgcn_readfirstlane(s_inexact[w]); left; left &= left - 1) {
+            const int t = 32 * w + __builtin_ctz(left);
+            if (GROUPS == 1 || group) {
+                request_k(t);
+                stage_k(t);
+            }
+            if ((GROUPS == 1 || !group) && d8 < CHUNKS) {
+                request_v(t);
+                write_v(t & 1, nx);
+            }
+            __syncthreads();
+            if (t < n_mine) {
+                scores(t & 1);
+                mask(t);
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    float x[8];
+#pragma unroll
+                    for (int i = 0; i < 8; ++i)
+                        x[i] = __builtin_amdgcn_exp2f(fmaf(s[b >> 1][8 * (b & 1) + i], a.scale_log2, -m)) * V_GAIN;
+#pragma unroll
+                    for (int n = 0; n < 3; ++n) {
+                        u32x4 p;
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) p[i] = hi_pair(x[2 * i], x[2 * i + 1]);
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) x[i] -= __uint_as_float(__float_as_uint(x[i]) & 0xFFFF0000u);
+#pragma unroll
+                        for (int d = 0; d < DB; ++d) acc[d] = mfma_bf16(v_operand(t & 1, b, d), p, acc[d]);
+                    }
+                }
+            }
+            __syncthreads();
+        }
     }
 
     if (row >= len) return;
     l += other_half(l);
-    const float inv = 1.0f / l;
+    const float inv = 1.0f / (l * V_GAIN);
     const int64_t at = (t0 + row) * a.o_t + h * a.o_h;
 #pragma unroll
     for (int d = 0; d < DB; ++d)
@@ -239,9 +379,11 @@ __global__ void __launch_bounds__(256, 2) prefill_kernel(PrefillArgs a, TileList
 }
 
 template <int D>
-void launch(const PrefillArgs& a, const TileList& list, int n, hipStream_t st) {
-    const size_t shm = 2 * (2 * KEYS * D * 2);
-    hipLaunchKernelGGL((prefill_kernel<D>), dim3(a.Hkv * a.R, n), dim3(256), shm, st, a, list);
+void launch(const PrefillArgs& a, const TileList& list, int n, bool two_groups, hipStream_t st) {
+    if (two_groups)
+        hipLaunchKernelGGL((prefill_kernel<D, 2>), dim3(a.R % 2 ? a.Hkv * a.R : a.Hkv * a.R / 2, n), dim3(512), 0, st, a, list);
+    else
+        hipLaunchKernelGGL((prefill_kernel<D, 1>), dim3(a.Hkv * a.R, n), dim3(256), 0, st, a, list);
 }
 
 }  // namespace
@@ -255,6 +397,9 @@ int prefill_attention(const uint16_t* q, int64_t q_t, int64_t q_h, const uint16_
                reinterpret_cast<uintptr_t>(o)) & 15) ||
              (q_t | q_h | k_t | k_h | v_t | v_h | o_t | o_h) % 8)
         bad = "prefill_attention: rows must be 16-byte aligned";
+    else if (k_t >= kPrefillMaxStride || v_t >= kPrefillMaxStride) bad = "prefill_attention: K / V rows too far apart";
+    for (int b = 0; b < B && !bad; ++b)
+        if (host_starts[b + 1] - host_starts[b] > kPrefillMaxRows) bad = "prefill_attention: request too long";
     if (bad) { set_error(bad); return -1; }
     const PrefillArgs a{q, k, v, q_t, q_h, k_t, k_h, v_t, v_h, o_bf16 ? nullptr : static_cast<float*>(o),
                         o_bf16 ? static_cast<uint16_t*>(o) : nullptr, o_t, o_h, Hkv, Hq / Hkv,
@@ -265,15 +410,27 @@ int prefill_attention(const uint16_t* q, int64_t q_t, int64_t q_h, const uint16_
         const int64_t n = host_starts[b + 1] - host_starts[b];
         if (n > most) most = static_cast<int>(n);
     }
+    // Two wave groups per workgroup pay when the tiles are long and fill the chip: they halve the vector work of staging
+    // and overlap matrix and vector work, but a workgroup is twice as large and runs half a tile longer.  One group -> two
+    // groups, us, 32 q / 8 kv heads: 4096 rows 246 -> 208, 2048 80.5 -> 79.3, 8 x 1024 141 -> 137; 1024 38.5 -> 42.1
+    // (half the chip), 16 x 512 95 -> 126 (five key tiles a workgroup on average), 100 rows 9.8 -> 13.0.
+    int64_t groups = 0, key_tiles = 0;
+    for (int b = 0; b < B; ++b)
+        for (int64_t q0 = 0, len = host_starts[b + 1] - host_starts[b]; q0 < len; q0 += QROWS) {
+            ++groups;
+            key_tiles += (std::min(len, q0 + QROWS) + KEYS - 1) / KEYS;
+        }
+    const bool two_groups = groups * Hq >= 2 * 256 && key_tiles >= 8 * groups;
     TileList list;
     int n = 0;
     hipStream_t st = static_cast<hipStream_t>(stream);
     auto flush = [&]() {
         if (n == 0) return;
-        if (D == 128) launch<128>(a, list, n, st); else launch<64>(a, list, n, st);
+        if (D == 128) launch<128>(a, list, n, two_groups, st); else launch<64>(a, list, n, two_groups, st);
         n = 0;
     };
-    for (int q0 = (most - 1) / QROWS * QROWS; q0 >= 0; q0 -= QROWS)
+    const int step = two_groups && a.R % 2 ? 2 * QROWS : QROWS;
+    for (int q0 = (most - 1) / step * step; q0 >= 0; q0 -= step)
         for (int b = 0; b < B; ++b) {
             const int len = static_cast<int>(host_starts[b + 1] - host_starts[b]);
             if (q0 >= len) continue;

@@ -60,3 +60,61 @@ def test_rows_the_kernel_does_not_take_still_run(dtype, D):
     assert not _hip.host().prefill(q, k, v, out, [0, 70], D ** -0.5)
     got = causal_prefill_attention(q, k, v, [0, 70], D ** -0.5, 2)
     assert (got.double() - _reference(q, k, v, [0, 70], D ** -0.5)).abs().max().item() <= 2e-5
+
+
+@pytest.mark.parametrize("D,hq,hkv,starts", [
+    (128, 64, 8, [0, 1025]), (128, 96, 32, [3, 1412]), (64, 64, 16, [0, 1024, 1090, 2300]), (128, 64, 64, [0, 1087])])
+def test_long_prompts_in_two_wave_groups(D, hq, hkv, starts):
+    """Enough long tiles for the two-group kernel: groups on two q heads and (odd or single q heads) on two row blocks."""
+    n = starts[-1] + 3
+    q, k, v = _rows(n, hq, D, 1), _rows(n, hkv, D, 2), _rows(n, hkv, D, 3)
+    k[:, :, :3] *= 12
+    out = torch.full((n, hq, D), 7.0, device=DEV)
+    assert _hip.host().prefill(q, k, v, out, starts, D ** -0.5)
+    live = slice(starts[0], starts[-1])
+    for h in range(0, hq, hq // hkv):
+        heads = slice(h, h + hq // hkv)
+        kv = slice(h // (hq // hkv), h // (hq // hkv) + 1)
+        want = _reference(q[:, heads], k[:, kv], v[:, kv], starts, D ** -0.5)
+        assert (out[live, heads].double() - want[live]).abs().max().item() <= 1e-5
+    assert bool((out[:starts[0]] == 7).all()) and bool((out[starts[-1]:] == 7).all())
+
+
+@pytest.mark.parametrize("hq,hkv,n", [(4, 2, 201), (64, 8, 1025)])       # one wave group, two
+@pytest.mark.parametrize("case", ["tiny", "huge", "some", "edges"])
+def test_values_that_are_no_f16(case, hq, hkv, n):
+    """V elements outside 2^-22..256 take their tile through the three-piece path."""
+    D = 128
+    q, k, v = _rows(n, hq, D, 1), _rows(n, hkv, D, 2), _rows(n, hkv, D, 3)
+    if case == "tiny":
+        v *= 2.0 ** -40
+    elif case == "huge":
+        v *= 2.0 ** 20
+    elif case == "some":
+        v[70, :, 5], v[n - 1, :, 127], v[64, 0, 0] = 1e4, 2.0 ** -30, 0.0
+    else:       # the last values on either side of both ends
+        top = torch.tensor([0x4380, 0x437F, 0x3480, 0x347F, 0x0001, -0x7F00 - 0x80 + 0x4380], dtype=torch.int16, device=DEV)
+        v[5, :, :6] = top.view(torch.bfloat16)
+        v[130, :, 6:10] = top[1:3].repeat(2).view(torch.bfloat16)          # a tile with exact ends only
+    out = torch.empty(n, hq, D, device=DEV)
+    assert _hip.host().prefill(q, k, v, out, [0, n], D ** -0.5)
+    rep = hq // hkv
+    for h in range(0, hq, rep):
+        want = _reference(q[:, h:h + rep], k[:, h // rep:h // rep + 1], v[:, h // rep:h // rep + 1], [0, n], D ** -0.5)
+        # fp32 sums of up to n weights, relative to the largest value of the channel
+        bound = 2e-6 * v[:, h // rep].double().abs().amax(0)
+        assert bool(((out[:, h:h + rep].double() - want).abs() <= bound + 1e-44).all())
+
+
+def test_an_infinite_value_stays_with_its_tile():
+    n, D = 1025, 128
+    q, k, v = _rows(n, 64, D, 1), _rows(n, 8, D, 2), _rows(n, 8, D, 3)
+    clean = torch.empty(n, 64, D, device=DEV)
+    assert _hip.host().prefill(q, k, v, clean, [0, n], D ** -0.5)
+    v[400, :, 9] = float("inf")
+    out = torch.empty(n, 64, D, device=DEV)
+    assert _hip.host().prefill(q, k, v, out, [0, n], D ** -0.5)
+    assert torch.equal(out[:384], clean[:384])                             # rows before the 64-key tile of row 400
+    assert not bool(torch.isfinite(out[400:, :, 9]).any())                 # (inf, or NaN where a piece of the weight is 0)
+    other = torch.arange(D, device=DEV) != 9
+    assert (out[:, :, other] - clean[:, :, other]).abs().max().item() <= 1e-5
