@@ -429,7 +429,7 @@ bool read_planes(PyObject* d, const Recipe& r, Planes& p) {
 
 int launch_store(const at::Tensor& K, const at::Tensor& V, int64_t row0, const Planes& p, const Recipe& r, int64_t T, int64_t ps,
                  const int32_t* src, const int32_t* pages, const int32_t* groups, const at::Tensor& table,
-                 int32_t* err, bool err_words, hipStream_t stream) {
+                 int32_t* err, bool err_words, int32_t* own_pages, int32_t* own_groups, hipStream_t stream) {
     auto from = [row0](const at::Tensor& t) {
         return static_cast<const char*>(t.data_ptr()) + row0 * t.stride(0) * static_cast<int64_t>(t.element_size());
     };
@@ -439,7 +439,7 @@ int launch_store(const at::Tensor& K, const at::Tensor& V, int64_t row0, const P
         r.gc, r.v_bf16, pages, groups, table.data_ptr<float>(), data<uint8_t>(p.k_base), data(p.k_scale),
         data<uint16_t>(p.k_zp), data<uint16_t>(p.ms), data<uint16_t>(p.mc), data<uint8_t>(p.index),
         data<uint8_t>(p.oval), data<uint8_t>(p.v_main), data(p.v_scale), data<uint16_t>(p.v_zp), err, err_words,
-        stream);
+        own_pages, own_groups, stream);
 }
 
 // (K, V, planes, page_size, src_rows, dst_pages, dst_groups, err_flag, num_tokens, table, row0, page0, group0, recipe x 8);
@@ -467,7 +467,8 @@ PyObject* py_store_pack(PyObject*, PyObject* const* a, Py_ssize_t n) {
     int rc;
     Py_BEGIN_ALLOW_THREADS
     rc = launch_store(*K, *V, row0, p, r, T, ps, data<int32_t>(src), pages ? data<int32_t>(pages) + page0 : nullptr,
-                      groups ? data<int32_t>(groups) + group0 : nullptr, *table, data<int32_t>(err), false, stream);
+                      groups ? data<int32_t>(groups) + group0 : nullptr, *table, data<int32_t>(err), false, nullptr, nullptr,
+                      stream);
     Py_END_ALLOW_THREADS
     if (failed(rc, "ommx_store_pack")) return nullptr;
     Py_RETURN_TRUE;
@@ -545,8 +546,8 @@ PyObject* py_pack_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const Planes p{&t[KBASE], &t[KSCALE], &t[KZP], opt(MS), opt(MC), opt(INDEX), opt(OVAL), &t[VMAIN], &t[VSCALE], &t[VZP]};
     int rc;
     Py_BEGIN_ALLOW_THREADS
-    rc = launch_store(*K, *V, 0, p, r, T, ps, nullptr, nullptr, nullptr, *table, t[FLAGS].data_ptr<int32_t>(), true, stream);
-    if (rc == 0) rc = ommx::identity_tables(t[TOK].data_ptr<int32_t>(), P, t[GRP].data_ptr<int32_t>(), G, stream);
+    rc = launch_store(*K, *V, 0, p, r, T, ps, nullptr, nullptr, nullptr, *table, t[FLAGS].data_ptr<int32_t>(), true,
+                      t[TOK].data_ptr<int32_t>(), t[GRP].data_ptr<int32_t>(), stream);
     Py_END_ALLOW_THREADS
     if (failed(rc, "ommx_store_pack")) return nullptr;
     PyObject* out = PyTuple_New(COUNT);
@@ -729,7 +730,8 @@ PyObject* py_pack_groups(PyObject*, PyObject* const* a, Py_ssize_t n) {
     rc = ommx::pack_list(pairs.data(), count, src, pages, groups, r.gt, ppg, rows, sink, span, wsink, per_seq,
                          per_seq * ppg, stream);
     if (rc == 0)
-        rc = launch_store(K, V, 0, p, r, count * r.gt, ps, src, pages, groups, *table, data<int32_t>(err), false, stream);
+        rc = launch_store(K, V, 0, p, r, count * r.gt, ps, src, pages, groups, *table, data<int32_t>(err), false, nullptr, nullptr,
+                      stream);
     Py_END_ALLOW_THREADS
     if (failed(rc, "ommx_store_pack")) return nullptr;
     Py_RETURN_TRUE;

@@ -8,16 +8,15 @@
 namespace ommx {
 
 // ommx_store_pack (the C ABI documents the arguments) with one more choice: err_words, err_flag is an array of
-// OMMX_STORE_ERR_WORDS host-visible ints, one per error bit.
+// OMMX_STORE_ERR_WORDS host-visible ints, one per error bit; and, for a block of its own, the identity tables
+// own_pages[T / page_size] and own_groups[T / group_tokens] (both or neither) filled by the same launch.
 int store_pack(const void* K, const void* V, int in_dtype, int64_t k_ts, int64_t k_hs, int64_t v_ts, int64_t v_hs,
                const int32_t* src_rows, int T, int H, int D, int page_size, int k_outliers, int index_repr,
                int select_abs, int scale_mode, int group_tokens, int group_channels, int v_bf16,
                const int32_t* dst_pages, const int32_t* dst_groups, const float* table, uint8_t* k_base,
                void* k_scale, uint16_t* k_zp, uint16_t* k_ms, uint16_t* k_mc, uint8_t* k_index, uint8_t* k_oval,
-               uint8_t* v_main, void* v_scale, uint16_t* v_zp, int32_t* err_flag, bool err_words, void* stream);
-
-// req_to_token[i] = i for i < n_pages and req_to_group[i] = i for i < n_groups, one launch.
-int identity_tables(int32_t* req_to_token, int n_pages, int32_t* req_to_group, int n_groups, void* stream);
+               uint8_t* v_main, void* v_scale, uint16_t* v_zp, int32_t* err_flag, bool err_words, int32_t* own_pages,
+               int32_t* own_groups, void* stream);
 
 // Rows [0, n_head) and [lo, T) of a K/V block [T, H, D] (fp32 or bf16, last axis contiguous) into the history
 // [hist_rows, H, D] of one request, at the ring slots of the absolute positions pos0 + row; rounds fp32 as

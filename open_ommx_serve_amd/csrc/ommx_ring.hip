@@ -209,21 +209,6 @@ int upload_words(int32_t* dst, const int32_t* host_words, int n, void* stream) {
     return 0;
 }
 
-__global__ void __launch_bounds__(256) identity_tables_kernel(int32_t* a, int na, int32_t* b, int nb) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < na) a[i] = i;
-    if (i < nb) b[i] = i;
-}
-
-int identity_tables(int32_t* req_to_token, int n_pages, int32_t* req_to_group, int n_groups, void* stream) {
-    const int n = n_pages > n_groups ? n_pages : n_groups;
-    if (n <= 0) return 0;
-    hipLaunchKernelGGL(identity_tables_kernel, dim3((n + 255) / 256), dim3(256), 0, static_cast<hipStream_t>(stream),
-                       req_to_token, n_pages, req_to_group, n_groups);
-    if (hipGetLastError() != hipSuccess) { set_error("identity_tables: launch failed"); return -2; }
-    return 0;
-}
-
 // One workgroup per group of the list.
 constexpr int kPackPairs = kUploadWords / 2;
 __global__ void __launch_bounds__(128) pack_list_kernel(int32_t* src_rows, int32_t* dst_pages, int32_t* dst_groups,

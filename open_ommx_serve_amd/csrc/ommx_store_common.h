@@ -36,7 +36,17 @@ struct StoreArgs {
     int v_bf16;             // V is kept as bf16 rows [pages, ps, H, D]; v_scale = 1, v_zp = 0 (pack.py:596-602)
     int err_words;          // err is an array of OMMX_STORE_ERR_WORDS ints in host memory, one per bit, instead of one
                             // word of bits: the bus has no atomic OR, a store of 1 per bit needs none
+    int32_t *own_pages, *own_groups;      // with a block of its own: its identity tables, written on the way instead of by a
+                                          // launch of their own (4096-token block, whole call: 33.4 -> 31.9 us)
 };
+
+// Entries of the identity tables that belong to K group g: the pages that begin in it, and its own.
+__device__ __forceinline__ void write_own_tables(const StoreArgs& a, int g, int tid) {
+    if (!a.own_groups || blockIdx.y != 0) return;
+    const int first = (g * a.gt + a.ps - 1) / a.ps, end = ((g + 1) * a.gt + a.ps - 1) / a.ps;
+    for (int p = first + tid; p < end; p += blockDim.x) a.own_pages[p] = p;
+    if (tid == 0) a.own_groups[g] = g;
+}
 
 // The bits a thread has found, into the caller's flag.  Reached on an error (or a noted wide step) only.
 __device__ __forceinline__ void report_store_bits(const StoreArgs& a, int bits) {

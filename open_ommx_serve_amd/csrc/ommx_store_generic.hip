@@ -242,6 +242,7 @@ __global__ void __launch_bounds__(256) store_generic_kernel(StoreArgs a) {
         else reinterpret_cast<uint16_t*>(a.v_scale)[vidx] = st.bits;
         a.v_zp[vidx] = zp_b;
     }
+    write_own_tables(a, g, tid);
     if (err && a.err) report_store_bits(a, err);
 }
 

@@ -339,6 +339,7 @@ __global__ void __launch_bounds__(512) store_long_kernel(StoreArgs a, int k_vec)
         reinterpret_cast<uint64_t*>(a.k_base)[(phys_row(g * GT + tk) * H + h) * pieces + j] = kb8;
     }
 
+    write_own_tables(a, g, tid);
     if (err && a.err) report_store_bits(a, err);
 }
 

@@ -5,7 +5,7 @@ import pytest
 import torch
 
 import oracle.ommx_oracle as O
-from open_ommx_serve_amd.attention import MultiSeqKVPool, WindowSpec, _hip
+from open_ommx_serve_amd.attention import MultiSeqKVPool, WindowSpec, _hip, ommx_pack_kv_canonical_block
 from open_ommx_serve_amd.attention.kv_store_ops import ring_slot
 
 pytestmark = pytest.mark.gpu
@@ -65,3 +65,15 @@ def test_groups_of_many_requests_complete_in_one_step(ring):
         got = pool.request_planes(r)
         for n in ("k_base", "k_scale", "k_obmp", "k_oval", "v_main", "v_scale"):
             assert torch.equal(got[n].cpu(), want[n]), (r, n)
+
+
+@pytest.mark.parametrize("gt,ps", [(32, 16), (32, 32), (32, 64), (64, 16), (128, 256), (16, 64)])
+@pytest.mark.parametrize("groups", [2, 6, 34])
+def test_a_block_carries_identity_tables(gt, ps, groups):
+    """Each store kernel writes the tables of its block: pages shorter and longer than a group."""
+    T, gc = 2 * gt * ps // 16 * groups, 32 if gt < 64 else gt
+    K, V = _block(T, 2, 128, torch.bfloat16, 5), _block(T, 2, 128, torch.bfloat16, 6)
+    out = ommx_pack_kv_canonical_block(K, V, outliers_per_vector=6, page_size=ps, device=DEV, outlier_select="signed",
+                                       use_pow2=True, group_tokens=gt, group_channels=gc)
+    assert torch.equal(out["req_to_token"], torch.arange(T // ps, dtype=torch.int32, device=DEV)[None])
+    assert torch.equal(out["req_to_group"], torch.arange(T // gt, dtype=torch.int32, device=DEV)[None])
