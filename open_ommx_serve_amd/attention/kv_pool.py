@@ -278,12 +278,14 @@ class MultiSeqKVPool:
         self.seq_len[r] = T
         target = self.window.num_groups(T)
         sink = self.window.sink_tokens
-        if target > 0:
-            self._pack_block_into_pool(r, K, V, 0, target, row0=sink)
-            self.packed_groups[r] = target
         # only the live rows enter the ring: sink, and [boundary - gt, T)
-        lo = max(sink, self.window.boundary(T) - self.gt)
-        self._write_rows(r, K, V, 0, min(sink, T), min(lo, T))
+        live = (min(sink, T), min(max(sink, self.window.boundary(T) - self.gt), T))
+        if target > 0:
+            written = self._pack_block_into_pool(r, K, V, 0, target, row0=sink, live=live)
+            self.packed_groups[r] = target
+            if written:
+                return target
+        self._write_rows(r, K, V, 0, *live)
         return target
 
     def _write_rows(self, req: int, K: torch.Tensor, V: torch.Tensor, pos0: int, n_head: int, lo: int) -> None:
@@ -444,22 +446,28 @@ class MultiSeqKVPool:
                                    row0=self.window.sink_tokens + g0 * self.gt)
 
     def _pack_block_into_pool(self, req: int, K: torch.Tensor, V: torch.Tensor, g0: int, g1: int,
-                              row0: int = 0) -> None:
+                              row0: int = 0, live: Optional[Tuple[int, int]] = None) -> bool:
         """Pack the ``(g1-g0)*gt`` tokens from row ``row0`` of a source block into request ``req``'s group /
-        page slots ``[g0, g1)`` with one store launch (kv_pool.py:677-734)."""
+        page slots ``[g0, g1)`` with one store launch (kv_pool.py:677-734).  ``live = (n_head, lo)``: the same
+        launch may write the block's rows ``[0, n_head)`` and ``[lo, T)`` into the ring; True when it has."""
         r = int(req)
         n_tok = (g1 - g0) * self.gt
         if row0 + n_tok > int(K.shape[0]) or row0 + n_tok > int(V.shape[0]):
             raise ValueError(f"source block must hold {n_tok} tokens from row {row0}; got {int(K.shape[0])}")
         gp0 = r * self.G_per_seq + g0
         pp0 = r * self.P_per_seq + g0 * self.pages_per_group
-        if self._host.store_pack(K, V, self._store_planes, self.ps, None, self._req_to_token, self._req_to_group,
-                                 self.err_flag, n_tok, store_table(K.device), row0, pp0, gp0, *self._recipe):
-            return
+        call = (K, V, self._store_planes, self.ps, None, self._req_to_token, self._req_to_group, self.err_flag, n_tok,
+                store_table(K.device), row0, pp0, gp0, *self._recipe)
+        if live is not None and self._host.store_pack(*call, self.k_hist, self.v_hist, r, *live, self._ring_sink,
+                                                      self._ring_rec):
+            return True
+        if self._host.store_pack(*call):
+            return False
         rows = slice(row0, row0 + n_tok)
         self._store(K[rows], V[rows], n_tok,
                     dst_pages=self._req_to_token.view(-1)[pp0:pp0 + (g1 - g0) * self.pages_per_group],
                     dst_groups=self._req_to_group.view(-1)[gp0:gp0 + (g1 - g0)])
+        return False
 
     # ── read path ────────────────────────────────────────────────────────────────
 

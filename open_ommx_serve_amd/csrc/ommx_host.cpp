@@ -429,7 +429,7 @@ bool read_planes(PyObject* d, const Recipe& r, Planes& p) {
 
 int launch_store(const at::Tensor& K, const at::Tensor& V, int64_t row0, const Planes& p, const Recipe& r, int64_t T, int64_t ps,
                  const int32_t* src, const int32_t* pages, const int32_t* groups, const at::Tensor& table,
-                 int32_t* err, bool err_words, int32_t* own_pages, int32_t* own_groups, hipStream_t stream) {
+                 int32_t* err, const ommx::StoreExtras& extras, hipStream_t stream) {
     auto from = [row0](const at::Tensor& t) {
         return static_cast<const char*>(t.data_ptr()) + row0 * t.stride(0) * static_cast<int64_t>(t.element_size());
     };
@@ -438,14 +438,40 @@ int launch_store(const at::Tensor& K, const at::Tensor& V, int64_t row0, const P
         src, T, K.size(1), K.size(2), ps, r.k, r.bitmap ? OMMX_INDEX_BITMAP : OMMX_INDEX_RELIDX7, r.abs, r.mode, r.gt,
         r.gc, r.v_bf16, pages, groups, table.data_ptr<float>(), data<uint8_t>(p.k_base), data(p.k_scale),
         data<uint16_t>(p.k_zp), data<uint16_t>(p.ms), data<uint16_t>(p.mc), data<uint8_t>(p.index),
-        data<uint8_t>(p.oval), data<uint8_t>(p.v_main), data(p.v_scale), data<uint16_t>(p.v_zp), err, err_words,
-        own_pages, own_groups, stream);
+        data<uint8_t>(p.oval), data<uint8_t>(p.v_main), data(p.v_scale), data<uint16_t>(p.v_zp), err, extras, stream);
+}
+
+bool is_history(const at::Tensor& k, const at::Tensor& v) {
+    return k.dim() == 4 && k.sizes() == v.sizes() && k.scalar_type() == at::kBFloat16 &&
+           v.scalar_type() == at::kBFloat16 && k.is_contiguous() && v.is_contiguous() && k.is_cuda();
+}
+
+// (k_hist, v_hist, req, n_head, lo, sink, span) at `a`: rows [0, n_head) and [lo, T) of K / V into a request's history
+bool read_block_rows(const at::Tensor& K, const at::Tensor& V, PyObject* const* a, int64_t pos0, ommx::BlockRows& out) {
+    bool ok = true;
+    const at::Tensor *kh = as_tensor(a[0], ok), *vh = as_tensor(a[1], ok);
+    const int64_t req = as_int(a[2], ok), head = as_int(a[3], ok), lo = as_int(a[4], ok), sink = as_int(a[5], ok),
+                  span = as_int(a[6], ok);
+    if (!ok || !is_history(*kh, *vh) || !is_rows(K) || !is_rows(V) || K.sizes() != V.sizes() ||
+        K.device() != kh->device() || V.device() != kh->device())
+        return false;
+    const int64_t T = K.size(0), rows = kh->size(1), H = kh->size(2), D = kh->size(3);
+    // every slot has to lie inside the history: below the ring's end, or the block's last position without a ring
+    if (K.size(1) != H || K.size(2) != D || D % 8 || req < 0 || req >= kh->size(0) || pos0 < 0 || head < 0 ||
+        lo < head || lo > T || sink < 0 || span < 0 || (span > 0 ? sink + span : pos0 + T) > rows)
+        return false;
+    out = ommx::block_rows(K.data_ptr(), V.data_ptr(), K.scalar_type() == at::kFloat, V.scalar_type() == at::kFloat,
+                           K.stride(0), K.stride(1), V.stride(0), V.stride(1),
+                           data<uint16_t>(kh) + req * kh->stride(0), data<uint16_t>(vh) + req * vh->stride(0), pos0,
+                           head, lo, T, H, D, sink, span);
+    return true;
 }
 
 // (K, V, planes, page_size, src_rows, dst_pages, dst_groups, err_flag, num_tokens, table, row0, page0, group0, recipe x 8);
 // without src_rows the tokens are the rows row0, row0 + 1, ...; the tables are read from entry page0 / group0 on
+// Seven more arguments (see read_block_rows): rows of the same bf16 block copied into a request's history by the same launch.
 PyObject* py_store_pack(PyObject*, PyObject* const* a, Py_ssize_t n) {
-    if (n != 21) { PyErr_SetString(PyExc_TypeError, "store_pack: wrong number of arguments"); return nullptr; }
+    if (n != 21 && n != 28) { PyErr_SetString(PyExc_TypeError, "store_pack: wrong number of arguments"); return nullptr; }
     bool ok = true;
     const at::Tensor *K = as_tensor(a[0], ok), *V = as_tensor(a[1], ok), *src = as_tensor_or_none(a[4], ok),
                      *pages = as_tensor_or_none(a[5], ok), *groups = as_tensor_or_none(a[6], ok),
@@ -462,13 +488,21 @@ PyObject* py_store_pack(PyObject*, PyObject* const* a, Py_ssize_t n) {
         !is_index(src, dev, at::kInt, T) || !is_index(pages, dev, at::kInt, page0 + T / ps) ||
         !is_index(groups, dev, at::kInt, group0 + T / r.gt))
         Py_RETURN_FALSE;
+    ommx::StoreExtras extras;
+    ommx::BlockRows rows;
+    if (n == 28) {
+        // (rows that come out of the history itself: not while it is being written)
+        if (T == 0 || K->scalar_type() != at::kBFloat16 || !read_block_rows(*K, *V, a + 21, 0, rows)) Py_RETURN_FALSE;
+        for (PyObject* hist : {a[21], a[22]})
+            if (K->is_alias_of(THPVariable_Unpack(hist)) || V->is_alias_of(THPVariable_Unpack(hist))) Py_RETURN_FALSE;
+        extras.rows = &rows;
+    }
     c10::hip::HIPGuard guard(dev.index());
     hipStream_t stream = stream_of(dev);
     int rc;
     Py_BEGIN_ALLOW_THREADS
     rc = launch_store(*K, *V, row0, p, r, T, ps, data<int32_t>(src), pages ? data<int32_t>(pages) + page0 : nullptr,
-                      groups ? data<int32_t>(groups) + group0 : nullptr, *table, data<int32_t>(err), false, nullptr, nullptr,
-                      stream);
+                      groups ? data<int32_t>(groups) + group0 : nullptr, *table, data<int32_t>(err), extras, stream);
     Py_END_ALLOW_THREADS
     if (failed(rc, "ommx_store_pack")) return nullptr;
     Py_RETURN_TRUE;
@@ -546,8 +580,8 @@ PyObject* py_pack_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const Planes p{&t[KBASE], &t[KSCALE], &t[KZP], opt(MS), opt(MC), opt(INDEX), opt(OVAL), &t[VMAIN], &t[VSCALE], &t[VZP]};
     int rc;
     Py_BEGIN_ALLOW_THREADS
-    rc = launch_store(*K, *V, 0, p, r, T, ps, nullptr, nullptr, nullptr, *table, t[FLAGS].data_ptr<int32_t>(), true,
-                      t[TOK].data_ptr<int32_t>(), t[GRP].data_ptr<int32_t>(), stream);
+    rc = launch_store(*K, *V, 0, p, r, T, ps, nullptr, nullptr, nullptr, *table, t[FLAGS].data_ptr<int32_t>(),
+                      {true, t[TOK].data_ptr<int32_t>(), t[GRP].data_ptr<int32_t>()}, stream);
     Py_END_ALLOW_THREADS
     if (failed(rc, "ommx_store_pack")) return nullptr;
     PyObject* out = PyTuple_New(COUNT);
@@ -588,11 +622,6 @@ PyObject* py_block_errors(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 // ── bf16 row history ───────────────────────────────────────────────────────────────────────────
-
-bool is_history(const at::Tensor& k, const at::Tensor& v) {
-    return k.dim() == 4 && k.sizes() == v.sizes() && k.scalar_type() == at::kBFloat16 &&
-           v.scalar_type() == at::kBFloat16 && k.is_contiguous() && v.is_contiguous() && k.is_cuda();
-}
 
 // (k_hist, v_hist, pos, k, v, sink, span, slots, pos_next, err_flag)
 PyObject* py_ring_write(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -661,27 +690,16 @@ PyObject* py_tail_gather(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyObject* py_rows_write(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != 10) { PyErr_SetString(PyExc_TypeError, "rows_write: wrong number of arguments"); return nullptr; }
     bool ok = true;
-    const at::Tensor *K = as_tensor(a[0], ok), *V = as_tensor(a[1], ok), *kh = as_tensor(a[2], ok),
-                     *vh = as_tensor(a[3], ok);
-    const int64_t req = as_int(a[4], ok), pos0 = as_int(a[5], ok), head = as_int(a[6], ok), lo = as_int(a[7], ok),
-                  sink = as_int(a[8], ok), span = as_int(a[9], ok);
-    if (!ok || !is_history(*kh, *vh) || !is_rows(*K) || !is_rows(*V) || K->sizes() != V->sizes() ||
-        K->device() != kh->device() || V->device() != kh->device())
-        Py_RETURN_FALSE;
-    const int64_t T = K->size(0), rows = kh->size(1), H = kh->size(2), D = kh->size(3);
-    // every slot has to lie inside the history: below the ring's end, or the block's last position without a ring
-    if (K->size(1) != H || K->size(2) != D || D % 8 || req < 0 || req >= kh->size(0) || pos0 < 0 || head < 0 ||
-        lo < head || lo > T || sink < 0 || span < 0 || (span > 0 ? sink + span : pos0 + T) > rows)
-        Py_RETURN_FALSE;
-    const c10::Device dev = kh->device();
-    c10::hip::HIPGuard guard(dev.index());
-    hipStream_t stream = stream_of(dev);
+    const at::Tensor *K = as_tensor(a[0], ok), *V = as_tensor(a[1], ok);
+    const int64_t pos0 = as_int(a[5], ok);
+    PyObject* const rest[] = {a[2], a[3], a[4], a[6], a[7], a[8], a[9]};
+    ommx::BlockRows rows;
+    if (!ok || !read_block_rows(*K, *V, rest, pos0, rows)) Py_RETURN_FALSE;
+    c10::hip::HIPGuard guard(K->device().index());
+    hipStream_t stream = stream_of(K->device());
     int rc;
     Py_BEGIN_ALLOW_THREADS
-    rc = ommx::rows_write(K->data_ptr(), V->data_ptr(), K->scalar_type() == at::kFloat, V->scalar_type() == at::kFloat,
-                          K->stride(0), K->stride(1), V->stride(0), V->stride(1),
-                          data<uint16_t>(kh) + req * kh->stride(0), data<uint16_t>(vh) + req * vh->stride(0), pos0,
-                          head, lo, T, H, D, sink, span, stream);
+    rc = ommx::rows_write(rows, stream);
     Py_END_ALLOW_THREADS
     if (failed(rc, "rows_write")) return nullptr;
     Py_RETURN_TRUE;
@@ -730,8 +748,7 @@ PyObject* py_pack_groups(PyObject*, PyObject* const* a, Py_ssize_t n) {
     rc = ommx::pack_list(pairs.data(), count, src, pages, groups, r.gt, ppg, rows, sink, span, wsink, per_seq,
                          per_seq * ppg, stream);
     if (rc == 0)
-        rc = launch_store(K, V, 0, p, r, count * r.gt, ps, src, pages, groups, *table, data<int32_t>(err), false, nullptr, nullptr,
-                      stream);
+        rc = launch_store(K, V, 0, p, r, count * r.gt, ps, src, pages, groups, *table, data<int32_t>(err), {}, stream);
     Py_END_ALLOW_THREADS
     if (failed(rc, "ommx_store_pack")) return nullptr;
     Py_RETURN_TRUE;

@@ -7,23 +7,46 @@
 
 namespace ommx {
 
-// ommx_store_pack (the C ABI documents the arguments) with one more choice: err_words, err_flag is an array of
-// OMMX_STORE_ERR_WORDS host-visible ints, one per error bit; and, for a block of its own, the identity tables
-// own_pages[T / page_size] and own_groups[T / group_tokens] (both or neither) filled by the same launch.
+// Rows of a prompt block and their places in the history of one request (ommx_rows.h copies them).
+struct BlockRows {
+    const void *K, *V;
+    int k_f32, v_f32, k_vec, v_vec;
+    int64_t k_ts, k_hs, v_ts, v_hs;
+    uint16_t *k_hist, *v_hist;
+    int64_t pos0;
+    int n_head, lo, H, D, sink, span;
+    int rows;               // [0, n_head) and [lo, T) of the block
+};
+
+inline bool rows_aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+inline BlockRows block_rows(const void* K, const void* V, bool k_f32, bool v_f32, int64_t k_ts, int64_t k_hs, int64_t v_ts,
+                            int64_t v_hs, uint16_t* k_hist, uint16_t* v_hist, int64_t pos0, int n_head, int lo, int T,
+                            int H, int D, int sink, int span) {
+    const bool dst_ok = rows_aligned16(k_hist) && rows_aligned16(v_hist);
+    return {K, V, k_f32, v_f32, dst_ok && rows_aligned16(K) && k_ts % 8 == 0 && k_hs % 8 == 0,
+            dst_ok && rows_aligned16(V) && v_ts % 8 == 0 && v_hs % 8 == 0, k_ts, k_hs, v_ts, v_hs, k_hist, v_hist, pos0,
+            n_head, lo, H, D, sink, span, n_head + (T - lo)};
+}
+
+// What a store launch of the native launchers does besides packing.
+struct StoreExtras {
+    bool err_words = false;               // err_flag is an array of OMMX_STORE_ERR_WORDS host-visible ints, one per error bit
+    int32_t *own_pages = nullptr, *own_groups = nullptr;      // identity tables [T / page_size], [T / group_tokens] to
+                                                              // fill (both or neither)
+    const BlockRows* rows = nullptr;      // bf16 rows to copy into the history (head_dim a multiple of 8, every slot inside it)
+};
+
+// ommx_store_pack (the C ABI documents the arguments) with extras.
 int store_pack(const void* K, const void* V, int in_dtype, int64_t k_ts, int64_t k_hs, int64_t v_ts, int64_t v_hs,
                const int32_t* src_rows, int T, int H, int D, int page_size, int k_outliers, int index_repr,
                int select_abs, int scale_mode, int group_tokens, int group_channels, int v_bf16,
                const int32_t* dst_pages, const int32_t* dst_groups, const float* table, uint8_t* k_base,
                void* k_scale, uint16_t* k_zp, uint16_t* k_ms, uint16_t* k_mc, uint8_t* k_index, uint8_t* k_oval,
-               uint8_t* v_main, void* v_scale, uint16_t* v_zp, int32_t* err_flag, bool err_words, int32_t* own_pages,
-               int32_t* own_groups, void* stream);
+               uint8_t* v_main, void* v_scale, uint16_t* v_zp, int32_t* err_flag, const StoreExtras& extras,
+               void* stream);
 
-// Rows [0, n_head) and [lo, T) of a K/V block [T, H, D] (fp32 or bf16, last axis contiguous) into the history
-// [hist_rows, H, D] of one request, at the ring slots of the absolute positions pos0 + row; rounds fp32 as
-// torch does.  The caller has checked that every slot lies inside the history.
-int rows_write(const void* K, const void* V, bool k_f32, bool v_f32, int64_t k_ts, int64_t k_hs, int64_t v_ts,
-               int64_t v_hs, uint16_t* k_hist, uint16_t* v_hist, int64_t pos0, int n_head, int lo, int T, int H,
-               int D, int sink, int span, void* stream);
+// The rows in one launch; fp32 is rounded as torch does.  The caller has checked that every slot lies inside the history.
+int rows_write(const BlockRows& rows, void* stream);
 
 // Up to kUploadWords 32-bit words from the host to dst inside a kernel's own argument block: no staging buffer, no
 // copy engine, nothing to keep alive after the call.

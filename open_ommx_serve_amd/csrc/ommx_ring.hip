@@ -15,15 +15,10 @@
 //
 // Both kernels are pure row copies (H*D bf16 per row), 16 bytes per thread when rows are
 // 16-byte aligned, one workgroup per row.
-#include "ommx_internal.h"
 #include "ommx_ring_args.h"
+#include "ommx_rows.h"
 
 namespace ommx {
-
-__device__ __forceinline__ int64_t ring_slot(int64_t pos, int sink, int span) {
-    if (span <= 0 || pos < sink) return pos;
-    return sink + (pos - sink) % span;
-}
 
 // Copies n_elem bf16 from src (rows of D contiguous elements, head stride hs) to a dense row.
 __device__ __forceinline__ void copy_row_in(uint16_t* dst, const uint16_t* src, int64_t hs,
@@ -132,57 +127,15 @@ int launch_tail_gather(const RingArgs& a, const int64_t* seq, const int64_t* tai
 }
 
 // ---- prompt blocks ---------------------------------------------------------------------------
-// One workgroup per row, K and V together.  A row is H*D elements; a thread moves eight of them (16 bytes of
-// bf16) per turn.  Bound by HBM for long blocks, by the launch for the ring's few live rows; replaces one
-// torch copy per tensor (whole history) or nine small index launches (ring).
-template <bool F32>
-__device__ __forceinline__ void put8(uint16_t* dst, const void* src, int64_t at, bool vec) {
-    if constexpr (F32) {
-        const float* p = static_cast<const float*>(src) + at;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) dst[i] = f32_to_bf16_any(p[i]);
-    } else {
-        const uint16_t* p = static_cast<const uint16_t*>(src) + at;
-        if (vec) *reinterpret_cast<uint4*>(dst) = *reinterpret_cast<const uint4*>(p);
-        else
-#pragma unroll
-            for (int i = 0; i < 8; ++i) dst[i] = p[i];
-    }
-}
+// One workgroup per row (ommx_rows.h).  Bound by HBM for long blocks, by the launch for a few rows; replaces one torch copy
+// per tensor (whole history) or nine small index launches (ring).  A prompt that completes groups carries its live rows
+// in the store launch instead.
+__global__ void __launch_bounds__(256) rows_write_kernel(BlockRows a) { copy_block_row<true>(a, blockIdx.x); }
 
-struct BlockRows {
-    const void *K, *V;
-    int k_f32, v_f32, k_vec, v_vec;
-    int64_t k_ts, k_hs, v_ts, v_hs;
-    uint16_t *k_hist, *v_hist;
-    int64_t pos0;
-    int n_head, lo, H, D, sink, span;
-};
-
-__global__ void __launch_bounds__(256) rows_write_kernel(BlockRows a) {
-    const int row = static_cast<int>(blockIdx.x) < a.n_head ? blockIdx.x : a.lo + (blockIdx.x - a.n_head);
-    const int64_t at = ring_slot(a.pos0 + row, a.sink, a.span) * static_cast<int64_t>(a.H * a.D);
-    const int per_head = a.D / 8;
-    for (int i = threadIdx.x; i < a.H * per_head; i += blockDim.x) {
-        const int h = i / per_head, c = (i % per_head) * 8;
-        const int64_t k_at = row * a.k_ts + h * a.k_hs + c, v_at = row * a.v_ts + h * a.v_hs + c;
-        const int64_t to = at + h * a.D + c;
-        if (a.k_f32) put8<true>(a.k_hist + to, a.K, k_at, false); else put8<false>(a.k_hist + to, a.K, k_at, a.k_vec);
-        if (a.v_f32) put8<true>(a.v_hist + to, a.V, v_at, false); else put8<false>(a.v_hist + to, a.V, v_at, a.v_vec);
-    }
-}
-
-int rows_write(const void* K, const void* V, bool k_f32, bool v_f32, int64_t k_ts, int64_t k_hs, int64_t v_ts,
-               int64_t v_hs, uint16_t* k_hist, uint16_t* v_hist, int64_t pos0, int n_head, int lo, int T, int H,
-               int D, int sink, int span, void* stream) {
-    if (D % 8 || n_head < 0 || lo < n_head || lo > T) { set_error("rows_write: bad shape"); return -1; }
-    const int rows = n_head + (T - lo);
-    if (rows == 0) return 0;
-    const bool dst_ok = aligned16(k_hist) && aligned16(v_hist);
-    const BlockRows a{K, V, k_f32, v_f32, dst_ok && aligned16(K) && k_ts % 8 == 0 && k_hs % 8 == 0,
-                      dst_ok && aligned16(V) && v_ts % 8 == 0 && v_hs % 8 == 0, k_ts, k_hs, v_ts, v_hs, k_hist,
-                      v_hist, pos0, n_head, lo, H, D, sink, span};
-    hipLaunchKernelGGL(rows_write_kernel, dim3(rows), dim3(H * D / 8 > 64 ? 128 : 64), 0,
+int rows_write(const BlockRows& a, void* stream) {
+    if (a.D % 8 || a.n_head < 0 || a.lo < a.n_head || a.rows < a.n_head) { set_error("rows_write: bad shape"); return -1; }
+    if (a.rows == 0) return 0;
+    hipLaunchKernelGGL(rows_write_kernel, dim3(a.rows), dim3(a.H * a.D / 8 > 64 ? 128 : 64), 0,
                        static_cast<hipStream_t>(stream), a);
     if (hipGetLastError() != hipSuccess) { set_error("rows_write: launch failed"); return -2; }
     return 0;

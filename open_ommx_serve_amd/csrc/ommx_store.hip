@@ -41,6 +41,7 @@ template <bool F32, bool FAST6, int IDXT>
 __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_kernel(StoreArgs a) {
     static_assert(!(F32 && FAST6), "the tuned path reads bf16 input");
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    if (copied_row(a)) return;
     // head_dim 128 is compiled in for the tuned instantiations (their launch checks it): row offsets
     // of the code tile become instruction immediates
     const int D = FAST6 ? 128 : a.D;
@@ -476,7 +477,7 @@ int ommx::store_pack(const void* K, const void* V, int in_dtype,
                      const int32_t* dst_pages, const int32_t* dst_groups, const float* table,
                      uint8_t* k_base, void* k_scale, uint16_t* k_zp, uint16_t* k_ms, uint16_t* k_mc,
                      uint8_t* k_index, uint8_t* k_oval, uint8_t* v_main, void* v_scale, uint16_t* v_zp,
-                     int32_t* err_flag, bool err_words, int32_t* own_pages, int32_t* own_groups, void* stream) {
+                     int32_t* err_flag, const StoreExtras& extras, void* stream) {
     using namespace ommx;
     const int gt = group_tokens, gc = group_channels;
     if (!(gt == 16 || gt == 32 || gt == 64 || gt == 128) || !(gc == 16 || gc == 32 || gc == 64 || gc == 128)) {
@@ -509,7 +510,8 @@ int ommx::store_pack(const void* K, const void* V, int in_dtype,
                 static_cast<int8_t*>(v_scale), v_zp,
                 err_flag, H, D, page_size, k_outliers,
                 (reinterpret_cast<uintptr_t>(V) % 16 == 0 && v_ts % 8 == 0 && v_hs % 8 == 0) ? 1 : 0,
-                index_repr, select_abs ? 1 : 0, scale_mode, gt, gc, v_bf16 ? 1 : 0, err_words ? 1 : 0, own_pages, own_groups};
+                index_repr, select_abs ? 1 : 0, scale_mode, gt, gc, v_bf16 ? 1 : 0, extras.err_words ? 1 : 0,
+                extras.own_pages, extras.own_groups, T / gt, extras.rows ? *extras.rows : BlockRows{}};
     hipStream_t st = static_cast<hipStream_t>(stream);
     const bool tuned = k_outliers == 6 && !select_abs && scale_mode == 0 && k_ms && D == 128 && gt == 32 && gc == 32 &&
                        32 % page_size == 0 && !v_bf16 && in_dtype == 0;   // the serving recipe
@@ -523,7 +525,7 @@ int ommx::store_pack(const void* K, const void* V, int in_dtype,
             return 0;
         }
     }
-    const dim3 grid(T / 32, H), block(D);
+    const dim3 grid(store_grid_x(a), H), block(D);
     const size_t shm = 32 * (size_t)D + 4 * (size_t)D + (index_repr ? 8 * (size_t)D : 0);
     if (in_dtype == 1)
         hipLaunchKernelGGL((store_pack_kernel<true, false, 2>), grid, block, shm, st, a);
@@ -551,5 +553,5 @@ extern "C" int ommx_store_pack(const void* K, const void* V, int in_dtype,
     return ommx::store_pack(K, V, in_dtype, k_ts, k_hs, v_ts, v_hs, src_rows, T, H, D, page_size, k_outliers,
                             index_repr, select_abs, scale_mode, group_tokens, group_channels, v_bf16, dst_pages,
                             dst_groups, table, k_base, k_scale, k_zp, k_ms, k_mc, k_index, k_oval, v_main,
-                            v_scale, v_zp, err_flag, false, nullptr, nullptr, stream);
+                            v_scale, v_zp, err_flag, {}, stream);
 }

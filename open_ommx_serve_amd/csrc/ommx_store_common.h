@@ -3,7 +3,7 @@
 // in the reference packer's order; the including files are compiled with -ffp-contract=off.
 #pragma once
 #include "ommx_common.h"
-#include "ommx_internal.h"
+#include "ommx_rows.h"
 
 namespace ommx {
 
@@ -38,7 +38,19 @@ struct StoreArgs {
                             // word of bits: the bus has no atomic OR, a store of 1 per bit needs none
     int32_t *own_pages, *own_groups;      // with a block of its own: its identity tables, written on the way instead of by a
                                           // launch of their own (4096-token block, whole call: 33.4 -> 31.9 us)
+    int groups;             // T / gt; workgroups beyond them copy rows into the history (bf16), H rows per blockIdx.x
+    BlockRows rows;
 };
+
+// Live rows of a prompt ride along with its packed groups: workgroups behind the last group copy a row each while that
+// one is still being packed.  True when the workgroup had no group.
+__device__ __forceinline__ bool copied_row(const StoreArgs& a) {
+    if (static_cast<int>(blockIdx.x) < a.groups) return false;
+    const int n = (static_cast<int>(blockIdx.x) - a.groups) * a.H + static_cast<int>(blockIdx.y);
+    if (n < a.rows.rows) copy_block_row<false>(a.rows, n);
+    return true;
+}
+inline unsigned store_grid_x(const StoreArgs& a) { return a.groups + (a.rows.rows + a.H - 1) / a.H; }
 
 // Entries of the identity tables that belong to K group g: the pages that begin in it, and its own.
 __device__ __forceinline__ void write_own_tables(const StoreArgs& a, int g, int tid) {

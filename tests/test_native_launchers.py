@@ -77,3 +77,34 @@ def test_a_block_carries_identity_tables(gt, ps, groups):
                                        use_pow2=True, group_tokens=gt, group_channels=gc)
     assert torch.equal(out["req_to_token"], torch.arange(T // ps, dtype=torch.int32, device=DEV)[None])
     assert torch.equal(out["req_to_group"], torch.arange(T // gt, dtype=torch.int32, device=DEV)[None])
+
+
+@pytest.mark.parametrize("recipe", [
+    dict(outliers_per_vector=6, outlier_repr="bitmap"),
+    dict(outliers_per_vector=6, outlier_repr="relidx7", group_tokens=64, group_channels=64, kv_outlier_map=False),
+    dict(outliers_per_vector=4, outlier_repr="relidx7", group_tokens=128, group_channels=32)])
+@pytest.mark.parametrize("H", [1, 3, 8])
+@pytest.mark.parametrize("extra", [0, 1, 31, 127])
+def test_live_rows_ride_along_with_the_groups(recipe, H, extra):
+    """One launch of each store kernel packs the groups and copies the ring's rows: the same as two launches."""
+    recipe = dict(recipe)
+    gt = recipe.pop("group_tokens", 32)
+    win = WindowSpec(page_size=16, group_tokens=gt)
+    T = 40 + 3 * gt + extra
+    K, V = _block(T, H, 128, torch.bfloat16, 7), _block(T, H, 128, torch.bfloat16, 8)
+    pools = [MultiSeqKVPool(128, H, 2, T, window=win, device=DEV, kv_ring=True, use_pow2=True, **recipe) for _ in range(2)]
+    for p in pools:
+        for t in p.pool_planes().values():
+            if torch.is_tensor(t) and t.dtype != torch.int32:
+                t.view(torch.uint8).zero_()
+    one, two = pools
+    launches = []
+    inner = two._pack_block_into_pool
+    two._pack_block_into_pool = lambda *a, live=None, **kw: launches.append(inner(*a, **kw))       # without the rows
+    assert one.append_block(1, K, V) == two.append_block(1, K, V) == win.num_groups(T) > 0
+    assert launches == [False]
+    assert torch.equal(one.k_hist, two.k_hist) and torch.equal(one.v_hist, two.v_hist)
+    assert one.k_hist[1].any() and not one.k_hist[0].any()
+    for n, t in one.pool_planes().items():
+        if torch.is_tensor(t):
+            assert torch.equal(t.view(torch.uint8), two.pool_planes()[n].view(torch.uint8)), n
