@@ -4,9 +4,32 @@
 // ommx_gpu_serve/attention/paged_decode.py:1657-2284 (production branch), used as the
 // on-device cross-check of the tuned kernel and for head shapes the tuned kernel does
 // not cover.
+//
+// Bound by the vector instructions and waits around its loads at five to seven waves per SIMD.  The outlier frames of a
+// channel come in whole dwords and are walked in registers (byte by byte from memory, each slot waited for its
+// own: 64-channel heads, 40001 tokens, 128 -> 109 us with 6-outlier streams of 32 tokens, 100 -> 89 us with 10 of 128).
+// Asking for the frames and the V codes at the top of a tile costs the registers of two waves: 110 and 133 us.
 #include "ommx_decode_args.h"
 
 namespace ommx {
+
+// Up to 16 bytes of a plane at any byte address, read as the aligned dwords that hold them and no others.
+struct Frame {
+    uint32_t w[5];
+    int sh;
+    __device__ __forceinline__ void load(const uint8_t* p, int n) {
+        const uintptr_t at = reinterpret_cast<uintptr_t>(p);
+        const uint32_t* q = reinterpret_cast<const uint32_t*>(at & ~static_cast<uintptr_t>(3));
+        sh = 8 * static_cast<int>(at & 3);
+        const int last = (static_cast<int>(at & 3) + n - 1) >> 2, most = (n + 6) >> 2;      // (most: uniform)
+#pragma unroll
+        for (int j = 0; j < 5; ++j) w[j] = j < most ? q[min(j, last)] : 0u;
+    }
+    __device__ __forceinline__ uint64_t word(int i) const {          // bytes 8i .. 8i + 7; those past n are not meant
+        const uint64_t lo = (static_cast<uint64_t>(w[2 * i + 1]) << 32) | w[2 * i];
+        return sh == 0 ? lo : (lo >> sh) | (static_cast<uint64_t>(w[2 * i + 2]) << (64 - sh));
+    }
+};
 
 template <int D, int R>
 __global__ void __launch_bounds__(256) decode_splitkv_ref_kernel(DecodeArgs a) {
@@ -61,6 +84,18 @@ __global__ void __launch_bounds__(256) decode_splitkv_ref_kernel(DecodeArgs a) {
             }
             gidx_u[u] = (gslot * a.Hkv + kvh) * D;
         }
+        // outlier frame of this thread's channel
+        const int nval = (a.kout + 1) >> 1;
+        const int nidx = a.idx_repr == 0 ? (gt + 7) / 8 : relidx7_bytes(a.kout);
+        const bool own_map = a.k_ms != nullptr, splices = a.kout > 0 && tid < D;
+        Frame ix, ov;
+        uint16_t ms_b = 0, mc_b = 0;
+        auto load_frame = [&](int u) {
+            const int64_t fr = gidx_u[u] + tid;
+            ix.load(a.k_obmp + fr * nidx, nidx);
+            ov.load(a.k_oval + fr * nval, nval);
+            if (own_map) { ms_b = a.k_ms[fr]; mc_b = a.k_mc[fr]; }
+        };
         for (int i = tid; i < nsub * D; i += 256) {
             const int u = i / D, d = i % D;
             s_sc[i] = a.scale_bf16
@@ -101,36 +136,32 @@ __global__ void __launch_bounds__(256) decode_splitkv_ref_kernel(DecodeArgs a) {
         }
         __syncthreads();
 
-        if (a.kout > 0 && tid < D) {   // outlier splice: thread = channel
-            const int nval = (a.kout + 1) >> 1;
-            const int nidx = a.idx_repr == 0 ? (gt + 7) / 8 : relidx7_bytes(a.kout);
-            const bool own_map = a.k_ms != nullptr;
+        if (splices) {   // outlier splice: thread = channel
             for (int u = 0; u < nsub; ++u) {
                 if ((g_first + u) * gt >= n_end) break;
-                const int64_t fr = gidx_u[u] + tid;
+                load_frame(u);
                 // tile-local index of group position 0 (negative when the group began before the tile)
                 const int base = (g_first + u) * gt - n0;
-                const uint8_t* ip = a.k_obmp + fr * nidx;
-                const uint8_t* ov = a.k_oval + fr * nval;
                 // dedicated map: level / map_scale + centre; else the base scale and zero point
-                const float ms = own_map ? bf16_to_f32(a.k_ms[fr]) : 0.0f;
-                const float mc = own_map ? bf16_to_f32(a.k_mc[fr]) : 0.0f;
-                int byte_i = 0, bit0 = 0;           // bitmap walk state: next byte, bit offset of the current one
-                uint32_t cur = 0;
+                const float ms = bf16_to_f32(ms_b), mc = bf16_to_f32(mc_b);
+                uint64_t lo = ix.word(0), hi = ix.word(1), nibbles = ov.word(0);
+                if (a.idx_repr == 0) {              // (bitmaps of 2 to 16 bytes: nothing behind them)
+                    if (nidx < 8) lo &= (1ull << (8 * nidx)) - 1;
+                    if (nidx <= 8) hi = 0;
+                }
                 for (int sl = 0; sl < a.kout; ++sl) {
                     int pos;
                     if (a.idx_repr == 0) {          // next set bit, ascending
-                        while (cur == 0 && byte_i < nidx) { cur = ip[byte_i]; bit0 = 8 * byte_i; ++byte_i; }
-                        if (cur == 0) break;
-                        pos = bit0 + __ffs(cur) - 1;
-                        cur &= cur - 1;
+                        if (lo) { pos = __builtin_ctzll(lo); lo &= lo - 1; }
+                        else if (hi) { pos = 64 + __builtin_ctzll(hi); hi &= hi - 1; }
+                        else break;
                     } else {                        // 7-bit field sl of the stream
-                        const int bit = 7 * sl;
-                        const uint32_t two = static_cast<uint32_t>(ip[bit >> 3]) |
-                            ((bit >> 3) + 1 < nidx ? static_cast<uint32_t>(ip[(bit >> 3) + 1]) << 8 : 0u);
-                        pos = (two >> (bit & 7)) & 127;
+                        pos = static_cast<int>(lo & 127u);
+                        lo = (lo >> 7) | (hi << 57);
+                        hi >>= 7;
                     }
-                    const uint32_t code = (ov[sl >> 1] >> (4 * (sl & 1))) & 0xFu;
+                    const uint32_t code = static_cast<uint32_t>(nibbles) & 0xFu;
+                    nibbles >>= 4;
                     const int tl = base + pos;
                     if (tl < 0 || tl >= 32) continue;
                     float lvl = fp4_level(code & 7u);
