@@ -300,6 +300,17 @@ def test_other_group_sizes(hq, hkv, D, recipe):
         _check(_run(case, num_kv_splits=S), want, f"{recipe} S{S}")
 
 
+@pytest.mark.parametrize("gt,rep,k", [
+    (gt, rep, k) for gt, rep, most in ((16, "bitmap", 8), (32, "bitmap", 8), (128, "bitmap", 8), (64, "relidx7", 16),
+                                       (128, "relidx7", 16)) for k in range(1, most + 1)])     # (a bitmap has at most 8)
+def test_outlier_frames_of_every_width_on_the_plain_kernel(gt, rep, k):
+    """Index frames of 1 to 16 bytes and code frames of 1 to 8, at every byte offset within a dword."""
+    case = build_decode_case([40 + 3 * gt], q_heads=2, kv_heads=1, head_dim=64, seed=70 + k, permute_tables=True,
+                             sparse_frac=0.02, group_tokens=gt, group_channels=min(gt, 64), outliers_per_vector=k,
+                             outlier_repr=rep)
+    _check(_run(case, num_kv_splits=2, ref_kernel=True), _oracle(case), f"k={k}")
+
+
 @pytest.mark.parametrize("kw", [dict(), dict(group_tokens=64, group_channels=64, outlier_repr="relidx7")])
 def test_bf16_v_rows(kw):
     """v_format="bf16": P.V from unquantised bf16 rows (pack.py:596-602, dequant :766-769)."""
