@@ -12,8 +12,11 @@
 
 #include <ATen/ATen.h>
 #include <ATen/EmptyTensor.h>
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/hip/impl/HIPCachingAllocatorMasqueradingAsCUDA.h>
 #include <c10/core/Allocator.h>
+#include <c10/core/GradMode.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
@@ -60,6 +63,29 @@ bool is_word(PyObject* o, const char* w) { return PyUnicode_Check(o) && PyUnicod
 bool is_group_size(int64_t g) { return g == 16 || g == 32 || g == 64 || g == 128; }
 template <class T = void>
 T* data(const at::Tensor* t) { return t ? static_cast<T*>(t->data_ptr()) : nullptr; }
+
+// Whether nobody but the caller has a part in a call on these tensors.  A tracer, a transform (vmap, grad, forward
+// mode, functionalisation), a dispatch or function mode, a tensor subclass and autograd all work in torch's
+// dispatcher, which a launcher here goes past: they would miss its result or take it for a constant.  So what the
+// dispatcher would look at for this call is held against the keys of an ordinary one.
+bool plain_call(PyObject* const* a, Py_ssize_t n) {
+    using c10::DispatchKey;
+    static const c10::DispatchKeySet ordinary{
+        DispatchKey::CPU, DispatchKey::CUDA, DispatchKey::AutogradCPU, DispatchKey::AutogradCUDA,
+        DispatchKey::ADInplaceOrView, DispatchKey::BackendSelect, DispatchKey::AutocastCPU, DispatchKey::AutocastCUDA};
+    if (at::impl::torch_function_mode_enabled()) return false;
+    const c10::impl::LocalDispatchKeySet tls = c10::impl::tls_local_dispatch_key_set();
+    const bool grad = c10::GradMode::is_enabled();
+    for (Py_ssize_t i = 0; i < n; ++i) {
+        if (a[i] == Py_None) continue;
+        if (!THPVariable_CheckExact(a[i])) return false;
+        const at::Tensor& t = THPVariable_Unpack(a[i]);
+        if (!ordinary.isSupersetOf((t.key_set() | tls.included_) - tls.excluded_) || (grad && t.requires_grad()) ||
+            t._fw_grad(0).defined())
+            return false;
+    }
+    return true;
+}
 
 bool failed(int rc, const char* what) {
     if (rc == 0) return false;
@@ -339,6 +365,9 @@ PyObject* answer(int rc) {
     if (rc < 0) return nullptr;
     return PyBool_FromLong(rc);
 }
+
+// (tensors or None ...)
+PyObject* py_plain(PyObject*, PyObject* const* a, Py_ssize_t n) { return PyBool_FromLong(plain_call(a, n)); }
 
 // The arguments of ommx_paged_decode_attention_canonical, in the order of DecodeArg.
 PyObject* py_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -853,7 +882,7 @@ PyObject* guarded(PyObject* self, PyObject* const* a, Py_ssize_t n) {
 
 #define OMMX_FAST(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(guarded<py_##name>)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
-    OMMX_FAST(auto_num_kv_splits),
+    OMMX_FAST(auto_num_kv_splits), OMMX_FAST(plain),
     OMMX_FAST(decode), OMMX_FAST(decode_pool), OMMX_FAST(store_pack), OMMX_FAST(pack_block), OMMX_FAST(block_errors), OMMX_FAST(pack_groups), OMMX_FAST(ring_write),
     OMMX_FAST(tail_gather), OMMX_FAST(rows_write), OMMX_FAST(upload), OMMX_FAST(prefill),
     {nullptr, nullptr, 0, nullptr},
