@@ -622,7 +622,10 @@ class MultiSeqKVPool:
         """Decode ``q [B, Hq, D]`` over this pool into ``out`` (bf16 or fp32): the tail rows are read in
         place from the history at the device lengths ``seq`` (int64) of the slots ``rows``, so there is no
         gather launch; ``b_seq_len`` (int32) are the packed lengths, ``tables`` the page / group rows of
-        the slots.  False when the native launcher does not take the arguments (nothing is done then)."""
+        the slots.  False when the native launcher does not take the arguments (nothing is done then), or
+        the call is traced, transformed or differentiated."""
+        if torch.compiler.is_compiling():
+            return False
         return self._host.decode_pool(q, self._store_planes, self.k_hist, self.v_hist, rows, seq, b_seq_len,
                                       tables[0], tables[1], out, sm_scale, self.ps, max_seq_len, mean_seq_len,
                                       self._ring_sink, self._ring_rec, self.window.sink_tokens,

@@ -354,7 +354,10 @@ class CanonicalKVStore:
                     sm_scale: float, max_seq_len: int) -> bool:
         """Decode ``q [1, Hq, D]`` over this cache into ``out`` (bf16 or fp32), the tail rows read in place
         from the history at the device length ``seq`` (int64 ``[1]``); ``b_seq_len`` (int32) is the packed
-        length.  False when the native launcher does not take the arguments (nothing is done then)."""
+        length.  False when the native launcher does not take the arguments (nothing is done then), or
+        the call is traced, transformed or differentiated."""
+        if torch.compiler.is_compiling():
+            return False
         return self._host.decode_pool(q, self._store_planes, self._k_hist4, self._v_hist4, None, seq, b_seq_len,
                                       self._req_to_token_full, self._req_to_group_full, out, sm_scale, self.ps,
                                       max_seq_len, None, self._ring_sink, self._ring_rec, self.window.sink_tokens,

@@ -785,9 +785,11 @@ PyObject* py_pack_groups(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 // (q, planes, k_hist, v_hist, slots, seq, b_seq_len, req_to_token, req_to_group, out, sm_scale, page_size, max_seq_len,
 //  mean_seq_len, ring sink, ring span, window sink, window recent, plain kernel, err_flag, recipe x 8): decode over a
-// pool's planes with the tail rows read in place from its history; out bf16 or fp32
+// pool's planes with the tail rows read in place from its history; out bf16 or fp32.  An observed call is refused.
 PyObject* py_decode_pool(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != 28) { PyErr_SetString(PyExc_TypeError, "decode_pool: wrong number of arguments"); return nullptr; }
+    PyObject* const rows[] = {a[0], a[9]};
+    if (!plain_call(rows, 2)) Py_RETURN_FALSE;
     bool ok = true;
     DecodeCall c;
     Recipe r;
@@ -811,9 +813,10 @@ PyObject* py_decode_pool(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return answer(run_decode(c));
 }
 
-// (q, k, v, out, starts, scale): causal attention of prompt rows, out fp32 or bf16
+// (q, k, v, out, starts, scale): causal attention of prompt rows, out fp32 or bf16.  An observed call is refused.
 PyObject* py_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != 6) { PyErr_SetString(PyExc_TypeError, "prefill: wrong number of arguments"); return nullptr; }
+    if (!plain_call(a, 4)) Py_RETURN_FALSE;
     bool ok = true;
     const at::Tensor *q = as_tensor(a[0], ok), *k = as_tensor(a[1], ok), *v = as_tensor(a[2], ok), *o = as_tensor(a[3], ok);
     std::vector<int64_t> starts;

@@ -190,7 +190,7 @@ def causal_prefill_attention(query, key, value, q_start, scale, n_rep):
     """Causal attention of each request over its own rows of a full-prefill step, softmax weights of fp32
     precision.  ``query [n, Hq, D]``, ``key`` / ``value [n, Hkv, D]``, ``q_start`` cumulative row offsets;
     returns fp32 ``[n, Hq, D]``.  bf16 rows of head_dim 64 or 128 take the HIP kernel; anything
-    else goes through torch's attention in fp32."""
+    else, and a call that is traced, transformed or differentiated, goes through torch's attention in fp32."""
     out = torch.empty(query.shape, dtype=torch.float32, device=query.device)
     if _prefill_into(query, key, value, q_start, scale, out):
         return out
@@ -208,7 +208,8 @@ def causal_prefill_attention(query, key, value, q_start, scale, n_rep):
 
 def _prefill_into(query, key, value, q_start, scale, out) -> bool:
     """The HIP kernel writing ``out`` (fp32 or bf16) in place; False when it does not take the rows."""
-    return query.is_cuda and _hip.host().prefill(query, key, value, out, [int(x) for x in q_start], float(scale))
+    return (query.is_cuda and not torch.compiler.is_compiling()
+            and _hip.host().prefill(query, key, value, out, [int(x) for x in q_start], float(scale)))
 
 
 class OMMXCanonicalImpl(_ImplBase):

@@ -7,8 +7,9 @@ from torch._subclasses.fake_tensor import FakeTensorMode
 from torch.fx.experimental.proxy_tensor import make_fx
 from torch.overrides import TorchFunctionMode
 
-from open_ommx_serve_amd.attention import _hip
+from open_ommx_serve_amd.attention import MultiSeqKVPool, _hip
 from open_ommx_serve_amd.attention import reference_op as R
+from open_ommx_serve_amd.integration.vllm.backend import causal_prefill_attention
 from open_ommx_serve_amd.synth import build_decode_case
 
 
@@ -95,3 +96,72 @@ def test_a_traced_decode_holds_the_op():
     assert "ommx_gpu_serve::paged_decode" in str(traced.graph)
     other = q.flip(0).contiguous()
     assert torch.equal(traced(other), decode(other)) and not torch.equal(decode(other), decode(q))
+
+
+def _prompt(n=70, D=64):
+    g = torch.Generator(device="cuda").manual_seed(3)
+    return [torch.randn(n, h, D, generator=g, device="cuda").to(torch.bfloat16) for h in (4, 2, 2)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("which", ["q", "k", "v", "qkv"])
+def test_prompt_attention_has_its_gradient(which):
+    rows = _prompt()
+    w = torch.randn(70, 4, 64, device="cuda")
+    leaves = [t.clone().requires_grad_("qkv"[i] in which) for i, t in enumerate(rows)]
+    out = causal_prefill_attention(*leaves, [0, 30, 70], 0.125, 2)
+    (out * w).sum().backward()
+    exact = [t.double().requires_grad_() for t in rows]
+    q, k, v = (t.transpose(0, 1) for t in exact)
+    total = 0
+    for a, b in ((0, 30), (30, 70)):
+        s = q[:, a:b] @ k[:, a:b].repeat_interleave(2, 0).transpose(1, 2).contiguous() * 0.125
+        s = s.masked_fill(torch.ones(b - a, b - a, dtype=torch.bool, device="cuda").triu(1), -float("inf"))
+        total = total + (s.softmax(-1) @ v[:, a:b].repeat_interleave(2, 0) * w[a:b].transpose(0, 1)).sum()
+    total.backward()
+    for leaf, want in zip(leaves, exact):
+        if not leaf.requires_grad:
+            assert leaf.grad is None
+            continue
+        # the gradient is rounded to bf16: 2^-9 of an element, next to fp32 sums of 70 terms
+        assert (leaf.grad.double() - want.grad).abs().max() <= 2.0 ** -8 * want.grad.abs().max()
+    with torch.no_grad():
+        assert _hip.host().prefill(*leaves, torch.empty_like(w), [0, 30, 70], 0.125)
+
+
+@pytest.mark.gpu
+def test_prompt_attention_under_a_tracer_and_fake_tensors():
+    q, k, v = _prompt()
+    traced = torch.jit.trace(lambda q: causal_prefill_attention(q, k, v, [0, 70], 0.125, 2), (q,), check_trace=False)
+    other = q.flip(0).contiguous()
+    want = causal_prefill_attention(other, k, v, [0, 70], 0.125, 2)
+    assert (traced(other) - want).abs().max() <= 1e-5
+    with FakeTensorMode() as mode:
+        out = causal_prefill_attention(*(mode.from_tensor(t) for t in (q, k, v)), [0, 70], 0.125, 2)
+    assert out.shape == q.shape and out.dtype == torch.float32
+
+
+@pytest.mark.gpu
+def test_a_pool_decode_leaves_observed_calls_to_the_op():
+    win_rows = 200
+    pool = MultiSeqKVPool(128, 2, 1, win_rows, outliers_per_vector=6, outlier_repr="bitmap", use_pow2=True)
+    g = torch.Generator(device="cuda").manual_seed(4)
+    K, V, q = (torch.randn(n, h, 128, generator=g, device="cuda").to(torch.bfloat16)
+               for n, h in ((150, 2), (150, 2), (1, 8)))
+    pool.append_block(0, K, V)
+    rows, seq = torch.tensor([0], device="cuda"), torch.tensor([150], device="cuda")
+    packed = torch.tensor([pool.window.packed_len(150)], dtype=torch.int32, device="cuda")
+    tables = (pool.pool_planes()["req_to_token"], pool.pool_planes()["req_to_group"])
+    out = torch.empty(1, 8, 128, device="cuda")
+
+    def decode(q, out):
+        return pool.decode_into(q, out, rows, seq, packed, tables, sm_scale=0.09, max_seq_len=150)
+
+    assert decode(q, out)
+    kept = out.clone()
+    out.fill_(5.0)
+    assert not decode(q.clone().requires_grad_(), out) and not decode(q, torch.empty_like(out).requires_grad_())
+    assert bool((out == 5.0).all())
+    with torch.no_grad():
+        assert decode(q.clone().requires_grad_(), out)
+    assert torch.equal(out, kept)
