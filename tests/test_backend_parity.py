@@ -252,3 +252,34 @@ def test_ring_history_and_the_other_index_planes_through_the_backend(graph, outl
     assert eng.state.manager.kv_ring and not eng.state.manager.dead
     st.check_errors()
     BK.reset_worker_state()
+
+
+def test_layers_on_two_streams_each_read_the_step():
+    """Layer 0 runs on a side stream that is busy, layer 1 meanwhile on the current one: what the step uploads for
+    one must not be what the other reads.  The same outputs as one stream gives."""
+    def outputs(side):
+        eng = _Engine(400, graph=False, batched=True, max_num_seqs=3)
+        reqs = [_Request(11, 150, 160, 100), _Request(25, 97, 110, 200)]
+        eng.step(reqs, check=False)
+        got = []
+        for _ in range(4):
+            reqs.reverse()                                  # other slots, lengths and tables every step
+            eng.builder.build(0, NS(seq_lens_cpu=[r.seq + 1 for r in reqs], query_start_loc_cpu=[0, 1, 2],
+                                    block_table_tensor=torch.tensor([[r.key, r.key + 1] for r in reqs])))
+            rows = [[torch.stack([t[r.seq] for r, t in zip(reqs, ts)]).to(DEV) for ts in (
+                [r.q for r in reqs], [r.K[l] for r in reqs], [r.V[l] for r in reqs])] for l in range(LAYERS)]
+            outs = [torch.empty(2, HQ, D, device=DEV) for _ in range(LAYERS)]
+            torch.cuda.synchronize()
+            for l, (layer, impl, (q, k, v)) in enumerate(zip(eng.layers, eng.impls, rows)):
+                with torch.cuda.stream(side if l == 0 else None):
+                    if l == 0 and side is not None:
+                        torch.cuda._sleep(2_000_000)        # about a millisecond
+                    impl.do_kv_cache_update(layer, k, v)
+                    impl.forward(layer, q, k, v, None, None, outs[l])
+            torch.cuda.synchronize()
+            got += outs
+            for r in reqs:
+                r.seq += 1
+        return torch.stack(got)
+
+    assert torch.equal(outputs(torch.cuda.Stream()), outputs(None))

@@ -295,6 +295,48 @@ def test_identity_is_required_unless_the_unsafe_hatch_is_set(monkeypatch):
         _bmgr(graph=False, strict=True)[0].on_build(_md([5, 6], [4, 4]))
 
 
+def test_each_stream_has_its_own_block_and_tables_of_a_step(monkeypatch):
+    """A layer on another stream is not ordered behind the first layer's upload: nothing may be handed over."""
+    m, _ = _bmgr(graph=False)
+    pool = NS(k_hist=NS(device=torch.device("cpu")), _req_to_token=torch.arange(40).view(4, 10),
+              _req_to_group=torch.arange(20).view(4, 5))
+    now, uploads = [1], []
+
+    def upload(block, values, n64):
+        uploads.append(now[0])
+        block[:2 * n64].view(torch.int64).copy_(torch.tensor(values[:n64]))
+        block[2 * n64:].copy_(torch.tensor(values[n64:], dtype=torch.int32))
+        return True
+
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: now[0], raising=False)
+    monkeypatch.setattr("open_ommx_serve_amd.integration.vllm.metadata._hip.host", lambda: NS(upload=upload))
+
+    def memory(step):
+        return {t.untyped_storage().data_ptr() for t in (*step[:4], *step.tables)}
+
+    def at(stream):
+        now[0] = stream
+        step = m.step_on_device(pool)
+        assert step.sel.tolist() == m.slots and step.cur.tolist() == m.seq_lens
+        assert step.packed.tolist() == [m.window.packed_len(x) for x in m.seq_lens]
+        assert torch.equal(step.tables[0], pool._req_to_token[step.sel])
+        return step
+
+    m.on_build(_md([200, 90], [11, 12]))
+    one, two = at(1), at(2)
+    assert memory(one).isdisjoint(memory(two))
+    assert at(1) is one and at(2) is two and uploads == [1, 2]
+    m.on_build(_md([201, 91], [11, 12]))
+    again = at(2)                              # the same memory, but written on that stream
+    assert memory(again) == memory(two) and uploads == [1, 2, 2]
+    assert memory(at(1)) == memory(one) and uploads == [1, 2, 2, 1]
+    m.on_build(_md([92, 202], [12, 11]))       # rows change places: other slots, other table rows
+    assert at(1).tables[0].tolist() != one.tables[0].tolist()
+    for stream in range(3, 40):                # bounded however many streams come
+        at(stream)
+    assert len(m._stream_blocks) <= 8
+
+
 # ── config and route decisions ───────────────────────────────────────────────────────────
 
 def test_config_defaults_are_the_serving_recipe_and_env_knobs_apply(monkeypatch):
