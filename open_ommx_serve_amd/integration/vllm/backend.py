@@ -261,9 +261,9 @@ class OMMXCanonicalImpl(_ImplBase):
             return
         s, st = _STATE, _STATE.step
         cfg = self._ommx_cfg()
-        if key.dim() != 3:
+        if key.shape[1:] != (self.num_kv_heads, self.head_size):
             key = key.reshape(n, self.num_kv_heads, self.head_size)
-        if value.dim() != 3:
+        if value.shape[1:] != (self.num_kv_heads, self.head_size):
             value = value.reshape(n, self.num_kv_heads, self.head_size)
         if st["B"] == STEP_ROUTE_UNCLASSIFIED and not st["batched_write"]:
             raise RuntimeError(
@@ -353,10 +353,10 @@ class OMMXCanonicalImpl(_ImplBase):
     def forward(self, layer, query, key, value, kv_cache=None, attn_metadata=None, output=None,
                 output_scale=None, output_block_scale=None):
         H, D = self.num_heads, self.head_size
-        q = query if query.dim() == 3 else query.reshape(-1, H, D)
+        q = query if query.shape[1:] == (H, D) else query.reshape(-1, H, D)
         if output is None:
             output = torch.empty_like(query)
-        out = output if output.dim() == 3 else output.view(-1, H, D)
+        out = output if output.shape[1:] == (H, D) else output.view(-1, H, D)
         st = _STATE.step
         if st["B"] == STEP_ROUTE_UNCLASSIFIED:
             raise RuntimeError("[ommx] unclassified step: request count unknown, refusing to "

@@ -399,3 +399,34 @@ def test_builder_route_decisions():
     assert BK.OMMXCanonicalBackend.get_builder_cls() is BK.OMMXCanonicalMetadataBuilder
     assert BK.OMMXCanonicalBackend.get_supported_kernel_block_sizes() == [16]
     BK.reset_worker_state()
+
+
+@pytest.mark.parametrize("form", ["[n, H, D]", "[n, H*D]", "[n, 1, H*D]", "[1, n, H*D]", "[1, n, H, D]", "[n, D, H]"])
+def test_rows_are_taken_in_any_form_that_reshapes(form):
+    """The engine's rows come flat, with a batch axis or by head; a rank of three alone does not say which."""
+    n, HQ, HKV, D = 5, 4, 2, 64
+
+    def shaped(t):
+        n, H, D = t.shape
+        return t.reshape({"[n, H, D]": (n, H, D), "[n, H*D]": (n, H * D), "[n, 1, H*D]": (n, 1, H * D),
+                          "[1, n, H*D]": (1, n, H * D), "[1, n, H, D]": (1, n, H, D), "[n, D, H]": (n, D, H)}[form])
+
+    g = torch.Generator().manual_seed(1)
+    q, k, v = (torch.randn(n, h, D, generator=g).to(torch.bfloat16) for h in (HQ, HKV, HKV))
+    BK.reset_worker_state(graph=False, batched=False, batched_graph=False)
+    BK.OMMXCanonicalMetadataBuilder().build(0, _md([n], [3], q=[0, n]))
+    impl = BK.OMMXCanonicalImpl(HQ, D, None, HKV)
+    want, out = torch.empty(n, HQ, D), shaped(torch.empty(n, HQ, D))
+    impl.forward(NS(), q, k, v, None, None, want)
+    assert impl.forward(NS(), shaped(q), shaped(k), shaped(v), None, None, out) is out
+    assert torch.equal(out.reshape(n, HQ, D), want)
+    got = impl.forward(NS(), shaped(q), shaped(k), shaped(v))
+    assert got.shape == shaped(q).shape and torch.equal(got.reshape(n, HQ, D), want.to(torch.bfloat16))
+    if not form.startswith("[1"):               # (the rows of a write are counted on the first axis)
+        kept = []
+        store = NS(append_block=lambda K, V: kept.append((K, V)), window=WindowSpec(), seq_len=n)
+        impl._ommx_reset = lambda *a: store
+        BK._STATE.manager = NS(register=lambda *a: None)
+        impl.do_kv_cache_update(NS(), shaped(k), shaped(v))
+        assert torch.equal(kept[0][0], k) and torch.equal(kept[0][1], v)
+    BK.reset_worker_state()
