@@ -3,11 +3,16 @@
 // Grouped-query heads, any number of requests per launch, head_dim 64 or 128.
 //
 // Precision is that of an fp32 softmax: q.k of bf16 operands is exact in the fp32 accumulator, the weights
-// p = exp2(s - m) are fp32 and enter P.V as two f16 pieces (11 bits, then the remainder rounded to 11: within
-// 2^-23 of the weight) against V times 2^8 in f16, which is exact for every bf16 of magnitude 2^-22 to 256
-// and zero.  A 64-key tile with any other V element is left out and follows after the loop with the weights in three
-// bf16 pieces and V as it is.  Against fp64, 4096 rows with K outliers: relative error 9.3e-7, the library's
-// fp32 attention 1.2e-6 (three bf16 pieces throughout: the same, with a third more PV instructions).
+// p = exp2(s - m) are fp32 and enter P.V times 2^8 as two f16 pieces (11 bits, then the remainder rounded to 11) against
+// V times 2^8 in f16, which is exact for every bf16 of magnitude 2^-22 to 256 and zero.  Two pieces hold a weight to
+// 2^-23 of itself down to 2^-10 of the row's largest, and to 2^-33 of the largest below.  A 64-key tile with any other
+// V element is left out of the loop and follows in a second pass, with the weights in three bf16 pieces (all 24 bits)
+// and V as it is.  The second pass also takes every tile where the small weights of some row are all that counts (its
+// largest ones met a V of next to nothing: an attention sink), which the sums at the end of the loop show; both passes
+// together take 2.1 times as long.  Relative error against fp64, and that of the library's fp32 attention: 4096 rows
+// with K outliers 7.0e-7 and 1.2e-6; 4096, 700 and 100 plain rows 2.9e-7, 1.9e-7, 1.4e-7 and 4.8e-7, 2.5e-7, 1.5e-7;
+// one key of V = 0 that outweighs every other 2^16 or 2^24 times 7.2e-7, 8.9e-7 and 1.1e-6, 1.4e-6 (without the second
+// pass and at 2^6 instead of 2^8 6.6e-6, 1.6e-3).
 //
 // Layout.  A group of four waves = 128 query rows of one q head; a wave owns 32 rows and walks the keys
 // 64 at a time with mfma_f32_32x32x16.  Scores are formed transposed, S^T = K.Q^T, so a lane
@@ -84,12 +89,20 @@ __device__ __forceinline__ u32x4 load16(__amdgpu_buffer_rsrc_t rows, uint32_t at
     return __builtin_amdgcn_raw_buffer_load_b128(rows, at, 0, 0);
 }
 
-// the running maximum is refreshed when a score (base 2) exceeds it by this: any bound that keeps
-// exp2 in range serves an online softmax, and most tiles then rescale nothing
-constexpr float MAX_SLACK = 8.0f;
-// weights are carried times 2^6 (at most 2^14 with the slack): the second f16 piece of a weight stays
-// accurate to 2^-31 of the largest.  V is carried times 2^8 and divided by it at the end.
-constexpr float P_SHIFT = 6.0f, V_GAIN = 256.0f;
+// The running maximum is refreshed when a score (base 2) exceeds it by the slack: any bound that keeps
+// exp2 in range serves an online softmax, and most tiles then rescale nothing.
+// Weights are carried times 2^8, at most 2^15.75 with the slack, within f16.  More would leave less to the second pass,
+// but the shift is part of exp2's argument, which is rounded to 24 bits: at 2^9 and above plain short rows are less exact
+// than the library's (1.6e-7, at 2^12 2.0e-7, against 1.5e-7), and the smaller slack rescales more tiles (4096 rows 199
+// against 194 us).  The gain as a factor of its own costs 6 % (mixed-precision or plain multiplications).
+// V is carried times 2^8 and divided by it at the end.
+constexpr float P_SHIFT = 8.0f, MAX_SLACK = 7.75f, V_GAIN = 256.0f;
+// In the second pass the sums so far and its weights are carried times this: a V of 2^100 is still in range.
+constexpr float LATE_GAIN = 1.0f / 16384;
+// Rows whose largest sum is below this times sqrt(n) times the largest V go through the second pass.  The pieces are off
+// by 2^-25 at most, 2^-25.8 on average, so n of them leave sqrt(n) * 2^-25.8 of a V of average size, about a quarter of the
+// largest, in a sum about a third of the row's largest: 2^-21.3 of it at the line.
+constexpr float AGAIN_BELOW = 1.0f / 32;
 // a bf16 value times 2^8 is exactly an f16 when its magnitude bits are 0 or in this range (2^-22 to 256)
 constexpr unsigned short V_LOW = (104 + 1) << 7, V_HIGH = ((104 + 31) << 7) - 1;
 
@@ -107,6 +120,7 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
     constexpr int KLOADS = KEYS * CHUNKS / 256;
     __shared__ __attribute__((aligned(16))) uint8_t s_k[2][KEYS * KS], s_v[2][D * VS];
     __shared__ uint32_t s_inexact[kPrefillMaxRows / KEYS / 32];          // bit per tile: some V element is no f16
+    __shared__ uint32_t s_top, s_again;              // largest |V| of the other tiles; a row wants all tiles again
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, half = lane >> 5, group = GROUPS == 2 ? wave >> 2 : 0;
     const int t0 = tiles.w[3 * blockIdx.y], len = tiles.w[3 * blockIdx.y + 1], q0 = tiles.w[3 * blockIdx.y + 2];
@@ -142,6 +156,7 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
     const int kg = st % (KEYS / 4), d8 = st / (KEYS / 4);
     const uint32_t k_row = static_cast<uint32_t>(a.k_t) * 2, v_row = static_cast<uint32_t>(a.v_t) * 2;
     const uint32_t k_at = kr * k_row + 16 * kc, v_at = 4 * kg * v_row + 16 * d8;
+    u16x2 v_top = {0, 0};                // largest |V| this thread has staged
     u32x4 nx[GROUPS == 2 ? 4 : 8];       // rows on their way: V, K behind it (two groups: either)
     u32x4* const nk = nx + (GROUPS == 2 ? 0 : 4);
     // The rows of a tile as a buffer that ends with the request's last row: loads beyond it return zeros.
@@ -197,6 +212,7 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
                 f[i][w] = (x & 0x80008000u) | __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(mag, bias) << 3);
             }
         if (min(low[0], low[1]) < V_LOW - 1 || max(high[0], high[1]) > V_HIGH) atomicOr(&s_inexact[t >> 5], 1u << (t & 31));
+        else v_top = __builtin_elementwise_max(v_top, high);
         write_v(t & 1, f);
     };
     auto inexact = [&](int t) { return (__builtin_amdgcn_readfirstlane(s_inexact[t >> 5]) >> (t & 31)) & 1u; };
@@ -277,19 +293,20 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
 #pragma unroll
                 for (int r = 0; r < 16; ++r) acc[d][r] *= shrink;
         }
+        float tile_l = 0.0f;      // (of its own: next to a large weight small ones would be rounded off one by one)
 #pragma unroll
         for (int b = 0; b < 4; ++b)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const float x = __builtin_amdgcn_exp2f(fmaf(s[b >> 1][8 * (b & 1) + 2 * i], a.scale_log2, -m));
                 const float y = __builtin_amdgcn_exp2f(fmaf(s[b >> 1][8 * (b & 1) + 2 * i + 1], a.scale_log2, -m));
-                l += x;
-                l += y;
+                tile_l += x + y;
                 const f16x2 hi = __builtin_convertvector((f32x2{x, y}), f16x2);
                 const f32x2 rest = {minus_low(x, hi), minus_high(y, hi)};
                 p0[b][i] = __builtin_bit_cast(uint32_t, hi);
                 p1[b][i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(rest, f16x2));
             }
+        l += tile_l;
         if (GROUPS == 2) {        // all of it here: the compiler would move the weights behind the barrier, to their use
 #pragma unroll
             for (int b = 0; b < 4; ++b) asm volatile("" : "+v"(p0[b]), "+v"(p1[b]));
@@ -298,6 +315,7 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
     };
 
     if (tid < kPrefillMaxRows / KEYS / 32) s_inexact[tid] = 0;
+    if (tid == 0) s_top = s_again = 0;
     if (GROUPS == 1 || group) { request_k(0); stage_k(0); request_k(1); }
     if (GROUPS == 1 || !group) request_v(0);
     __syncthreads();
@@ -317,49 +335,79 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
         if (GROUPS == 2 && (!group || t + 1 < n_tiles)) __syncthreads();
     }
 
-    // Tiles whose V is not exact in f16: scores once more, weights against the final maximum in three bf16 pieces
-    // (8 + 8 + 8 bits by truncation, their sum is the weight), V as it is.
-    __syncthreads();
-    for (int w = 0; w <= (n_tiles - 1) >> 5; ++w) {
-        for (uint32_t left = __builtin_amdgcn_readfirstlane(s_inexact[w]); left; left &= left - 1) {
-            const int t = 32 * w + __builtin_ctz(left);
-            if (GROUPS == 1 || group) {
-                request_k(t);
-                stage_k(t);
-            }
-            if ((GROUPS == 1 || !group) && d8 < CHUNKS) {
-                request_v(t);
-                write_v(t & 1, nx);
-            }
-            __syncthreads();
-            if (t < n_mine) {
-                scores(t & 1);
-                mask(t);
+    // Second pass over tiles whose V is not exact in f16: scores once more, weights against the final maximum in three bf16
+    // pieces (8 + 8 + 8 bits by truncation, their sum is the weight), V as it is.
+    float gain = V_GAIN;
+    auto second_pass = [&](auto tiles_of, float keep) {
+        bool first = true;
+        for (int w = 0; w <= (n_tiles - 1) >> 5; ++w)
+            for (uint32_t left = tiles_of(w); left; left &= left - 1) {
+                const int t = 32 * w + __builtin_ctz(left);
+                if (GROUPS == 1 || group) {
+                    request_k(t);
+                    stage_k(t);
+                }
+                if ((GROUPS == 1 || !group) && d8 < CHUNKS) {
+                    request_v(t);
+                    write_v(t & 1, nx);
+                }
+                if (first) {
 #pragma unroll
-                for (int b = 0; b < 4; ++b) {
-                    float x[8];
+                    for (int d = 0; d < DB; ++d)
 #pragma unroll
-                    for (int i = 0; i < 8; ++i)
-                        x[i] = __builtin_amdgcn_exp2f(fmaf(s[b >> 1][8 * (b & 1) + i], a.scale_log2, -m)) * V_GAIN;
+                        for (int r = 0; r < 16; ++r) acc[d][r] *= keep;
+                    gain = V_GAIN * LATE_GAIN;
+                    first = false;
+                }
+                __syncthreads();
+                if (t < n_mine) {
+                    scores(t & 1);
+                    mask(t);
 #pragma unroll
-                    for (int n = 0; n < 3; ++n) {
-                        u32x4 p;
+                    for (int b = 0; b < 4; ++b) {
+                        float x[8];
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) p[i] = hi_pair(x[2 * i], x[2 * i + 1]);
+                        for (int i = 0; i < 8; ++i)
+                            x[i] = __builtin_amdgcn_exp2f(fmaf(s[b >> 1][8 * (b & 1) + i], a.scale_log2, -m)) * (V_GAIN * LATE_GAIN);
 #pragma unroll
-                        for (int i = 0; i < 8; ++i) x[i] -= __uint_as_float(__float_as_uint(x[i]) & 0xFFFF0000u);
+                        for (int n = 0; n < 3; ++n) {
+                            u32x4 p;
 #pragma unroll
-                        for (int d = 0; d < DB; ++d) acc[d] = mfma_bf16(v_operand(t & 1, b, d), p, acc[d]);
+                            for (int i = 0; i < 4; ++i) p[i] = hi_pair(x[2 * i], x[2 * i + 1]);
+#pragma unroll
+                            for (int i = 0; i < 8; ++i) x[i] -= __uint_as_float(__float_as_uint(x[i]) & 0xFFFF0000u);
+#pragma unroll
+                            for (int d = 0; d < DB; ++d) acc[d] = mfma_bf16(v_operand(t & 1, b, d), p, acc[d]);
+                        }
                     }
                 }
+                __syncthreads();
             }
-            __syncthreads();
-        }
+    };
+    for (int i = 32; i; i >>= 1)
+        v_top = __builtin_elementwise_max(v_top, __builtin_bit_cast(u16x2, __shfl_xor(__builtin_bit_cast(int, v_top), i)));
+    if (lane == 0) atomicMax(&s_top, static_cast<uint32_t>(max(v_top[0], v_top[1])));
+    __syncthreads();
+    second_pass([&](int w) -> uint32_t { return __builtin_amdgcn_readfirstlane(s_inexact[w]); }, LATE_GAIN);
+
+    // Rows whose sums are small against V: see AGAIN_BELOW.
+    {
+        float most = 0.0f;
+#pragma unroll
+        for (int d = 0; d < DB; ++d)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) most = fmaxf(most, fabsf(acc[d][r]));
+        most = fmaxf(most, other_half(most));
+        const float top = __uint_as_float(s_top << 16) * gain * AGAIN_BELOW;
+        if (row < len && most * most < top * top * static_cast<float>(row + 1)) s_again = 1;
     }
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(s_again))
+        second_pass([&](int w) { return n_tiles - 32 * w >= 32 ? ~0u : (1u << (n_tiles - 32 * w)) - 1; }, 0.0f);
 
     if (row >= len) return;
     l += other_half(l);
-    const float inv = 1.0f / (l * V_GAIN);
+    const float inv = 1.0f / (l * gain);
     const int64_t at = (t0 + row) * a.o_t + h * a.o_h;
 #pragma unroll
     for (int d = 0; d < DB; ++d)

@@ -1,6 +1,8 @@
 """The prompt-attention kernel against causal softmax in fp64: request lengths around the 32-row
 wave, the 64-key and the 128-row tile, empty requests, rows that start past zero, every head
 grouping, both output types, and a batch whose tile list takes more than one launch."""
+import math
+
 import pytest
 import torch
 
@@ -118,3 +120,25 @@ def test_an_infinite_value_stays_with_its_tile():
     assert not bool(torch.isfinite(out[400:, :, 9]).any())                 # (inf, or NaN where a piece of the weight is 0)
     other = torch.arange(D, device=DEV) != 9
     assert (out[:, :, other] - clean[:, :, other]).abs().max().item() <= 1e-5
+
+
+@pytest.mark.parametrize("D,hq,hkv,n", [(128, 4, 2, 100), (64, 4, 4, 700), (128, 64, 8, 1025), (64, 96, 32, 1412)])
+@pytest.mark.parametrize("gap", [12, 16, 20, 24])
+@pytest.mark.parametrize("sink_v", [0.0, 2.0 ** -12])
+def test_rows_made_of_small_weights(D, hq, hkv, n, gap, sink_v):
+    """A key with next to no V that outweighs every other 2^gap times: the output is the small weights' share."""
+    q, k, v = _rows(n, hq, D, 1), _rows(n, hkv, D, 2), _rows(n, hkv, D, 3)
+    scale = D ** -0.5
+    q[:, :, 0], k[:, :, 0], k[0] = 8.0, 0.0, 0.0
+    k[0, :, 0] = gap * math.log(2.0) / (8.0 * scale)
+    v[0] *= sink_v
+    v[n // 2, :, 3] = 1e-9 if gap == 20 else 0.5                # with and without a tile of its own path
+    out = torch.empty(n, hq, D, device=DEV)
+    assert _hip.host().prefill(q, k, v, out, [0, n], scale)
+    rep = hq // hkv
+    for h in range(0, hq, rep):
+        want = _reference(q[:, h:h + rep], k[:, h // rep:h // rep + 1], v[:, h // rep:h // rep + 1], [0, n], scale)[1:]
+        err = (out[1:, h:h + rep].double() - want).norm(dim=-1) / want.norm(dim=-1)
+        # Scores of up to 2^5 are rounded to 2^-20 twice (the sum, exp2's argument), which moves a weight by
+        # ln 2 of that; 2^-21 is left of the split; fp32 sums of up to 1412 terms add less than 2^-20.
+        assert err.max().item() <= 2.0 ** -18, (h, err.max().item())
