@@ -121,6 +121,7 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
     __shared__ __attribute__((aligned(16))) uint8_t s_k[2][KEYS * KS], s_v[2][D * VS];
     __shared__ uint32_t s_inexact[kPrefillMaxRows / KEYS / 32];          // bit per tile: some V element is no f16
     __shared__ uint32_t s_top, s_again;              // largest |V| of the other tiles; a row wants all tiles again
+    __shared__ int s_first[3][D], s_special;         // first row with +inf, -inf, NaN in a channel of V; whether there is one
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, half = lane >> 5, group = GROUPS == 2 ? wave >> 2 : 0;
     const int t0 = tiles.w[3 * blockIdx.y], len = tiles.w[3 * blockIdx.y + 1], q0 = tiles.w[3 * blockIdx.y + 2];
@@ -214,6 +215,26 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
         if (min(low[0], low[1]) < V_LOW - 1 || max(high[0], high[1]) > V_HIGH) atomicOr(&s_inexact[t >> 5], 1u << (t & 31));
         else v_top = __builtin_elementwise_max(v_top, high);
         write_v(t & 1, f);
+    };
+    // Elements of V that are no number are taken out of the staged rows, where a weight of zero (a row before them, a
+    // piece of a weight) would turn them into NaN, and noted: every row from theirs on gets them in the end.
+    auto take_special = [&](int t) {
+        u16x2 high = {0, 0};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int w = 0; w < 4; ++w) high = __builtin_elementwise_max(high, __builtin_bit_cast(u16x2, nx[i][w] & 0x7FFF7FFFu));
+        if (max(high[0], high[1]) < 0x7F80) return;
+        s_special = 1;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const uint32_t x = nx[i][e >> 1] >> (16 * (e & 1)) & 0xFFFFu;
+                if ((x & 0x7FFFu) < 0x7F80u) continue;
+                atomicMin(&s_first[x == 0x7F80u ? 0 : (x == 0xFF80u ? 1 : 2)][8 * d8 + e], t * KEYS + 4 * kg + i);
+                nx[i][e >> 1] &= e & 1 ? 0x0000FFFFu : 0xFFFF0000u;
+            }
     };
     auto inexact = [&](int t) { return (__builtin_amdgcn_readfirstlane(s_inexact[t >> 5]) >> (t & 31)) & 1u; };
 
@@ -315,7 +336,8 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
     };
 
     if (tid < kPrefillMaxRows / KEYS / 32) s_inexact[tid] = 0;
-    if (tid == 0) s_top = s_again = 0;
+    if (tid < D) s_first[0][tid] = s_first[1][tid] = s_first[2][tid] = INT32_MAX;
+    if (tid == 0) s_top = s_again = s_special = 0;
     if (GROUPS == 1 || group) { request_k(0); stage_k(0); request_k(1); }
     if (GROUPS == 1 || !group) request_v(0);
     __syncthreads();
@@ -349,6 +371,7 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
                 }
                 if ((GROUPS == 1 || !group) && d8 < CHUNKS) {
                     request_v(t);
+                    take_special(t);
                     write_v(t & 1, nx);
                 }
                 if (first) {
@@ -405,6 +428,7 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
     if (__builtin_amdgcn_readfirstlane(s_again))
         second_pass([&](int w) { return n_tiles - 32 * w >= 32 ? ~0u : (1u << (n_tiles - 32 * w)) - 1; }, 0.0f);
 
+    const bool special = __builtin_amdgcn_readfirstlane(s_special);
     if (row >= len) return;
     l += other_half(l);
     const float inv = 1.0f / (l * gain);
@@ -417,6 +441,13 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
             float v[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) v[i] = acc[d][4 * r4 + i] * inv;
+            if (special)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if (row >= s_first[0][ch + i]) v[i] += INFINITY;
+                    if (row >= s_first[1][ch + i]) v[i] -= INFINITY;
+                    if (row >= s_first[2][ch + i]) v[i] = NAN;
+                }
             if (a.o16)
                 *reinterpret_cast<u32x2*>(a.o16 + at + ch) =
                     u32x2{f32_to_bf16_any(v[0]) | (static_cast<uint32_t>(f32_to_bf16_any(v[1])) << 16),

@@ -142,3 +142,28 @@ def test_rows_made_of_small_weights(D, hq, hkv, n, gap, sink_v):
         # Scores of up to 2^5 are rounded to 2^-20 twice (the sum, exp2's argument), which moves a weight by
         # ln 2 of that; 2^-21 is left of the split; fp32 sums of up to 1412 terms add less than 2^-20.
         assert err.max().item() <= 2.0 ** -18, (h, err.max().item())
+
+
+@pytest.mark.parametrize("D,hq,hkv,starts", [(64, 4, 2, [0, 201]), (128, 4, 4, [3, 90, 300]), (128, 64, 8, [0, 1025])])
+def test_values_that_are_no_numbers_reach_the_rows_from_theirs_on(D, hq, hkv, starts):
+    n, inf = starts[-1], float("inf")
+    q, k, v = _rows(n, hq, D, 1), _rows(n, hkv, D, 2), _rows(n, hkv, D, 3)
+    clean = torch.zeros(n, hq, D, device=DEV)
+    assert _hip.host().prefill(q, k, v, clean, starts, D ** -0.5)
+    want = clean.clone()
+    t0 = starts[-2]
+    v[t0 + 70, :, 9], v[t0 + 75, :, 9] = inf, inf
+    v[t0 + 64, :, D - 1], v[t0 + 130, :, D - 1] = -inf, inf
+    v[t0, 0, 0] = float("nan")
+    v[t0 + 127, :, 33], v[t0 + 128, :, 33] = float("nan"), -inf
+    want[t0 + 70:, :, 9] = inf
+    want[t0 + 64:t0 + 130, :, D - 1] = -inf
+    want[t0 + 130:, :, D - 1] = float("nan")
+    want[t0:, :hq // hkv, 0] = float("nan")
+    want[t0 + 127:, :, 33] = float("nan")
+    for dtype in (torch.float32, torch.bfloat16):
+        out = torch.zeros(n, hq, D, dtype=dtype, device=DEV)
+        assert _hip.host().prefill(q, k, v, out, starts, D ** -0.5)
+        # (tiles with such a value take the path of three bf16 pieces: fp32 sums in another order)
+        torch.testing.assert_close(out.float(), want.to(dtype).float(), rtol=2.0 ** -7 if dtype == torch.bfloat16 else 0,
+                                   atol=1e-5, equal_nan=True)
