@@ -87,6 +87,11 @@ bool plain_call(PyObject* const* a, Py_ssize_t n) {
     return true;
 }
 
+// A tensor that a launch has written: autograd has to know that what it saved of it is gone.
+void written(const at::Tensor& t) {
+    if (!t.is_inference()) t.unsafeGetTensorImpl()->bump_version();
+}
+
 bool failed(int rc, const char* what) {
     if (rc == 0) return false;
     PyErr_Format(PyExc_RuntimeError, "%s failed (rc=%d): %s", what, rc, ommx_last_error());
@@ -358,7 +363,10 @@ int run_decode(const DecodeCall& c) {
         Py_END_ALLOW_THREADS
     }
 #undef OMMX_SPLITKV_ARGS
-    return failed(rc, "ommx_decode_splitkv") || failed(rc2, "ommx_decode_combine") ? -1 : 1;
+    if (failed(rc, "ommx_decode_splitkv") || failed(rc2, "ommx_decode_combine")) return -1;
+    written(*c.o);
+    if (c.lse) written(*c.lse);
+    return 1;
 }
 
 PyObject* answer(int rc) {
@@ -848,6 +856,7 @@ PyObject* py_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                  static_cast<int>(starts.size()) - 1, Hq, Hkv, D, scale, stream);
     Py_END_ALLOW_THREADS
     if (failed(rc, "prefill_attention")) return nullptr;
+    written(*o);
     Py_RETURN_TRUE;
 }
 

@@ -75,7 +75,7 @@ def test_an_ordinary_call_is_plain():
         assert plain(t)
 
 
-def _case():
+def _case(**kw):
     case = build_decode_case([300, 150], seed=5)
     planes = dict(case.planes) | {"outliers_per_vector": case.outliers_per_vector, "page_size": case.page_size,
                                   "k_format": "i2f4", "outlier_repr": "bitmap", "kv_outlier_map": True,
@@ -85,7 +85,7 @@ def _case():
         return R.ommx_paged_decode(q, planes, case.k_tail, case.v_tail, case.b_tail_len, case.b_seq_len,
                                    sm_scale=case.sm_scale, req_to_token=case.req_to_token,
                                    req_to_group=case.req_to_group, max_seq_len=300,
-                                   max_tail_len=int(case.k_tail.shape[1]))[0]
+                                   max_tail_len=int(case.k_tail.shape[1]), **kw)[0]
     return case.q, decode
 
 
@@ -163,3 +163,23 @@ def test_a_pool_decode_leaves_observed_calls_to_the_op():
     with torch.no_grad():
         assert decode(q.clone().requires_grad_(), out)
     assert torch.equal(out, kept)
+
+
+@pytest.mark.gpu
+def test_a_tensor_written_by_a_launch_is_a_new_version():
+    """Autograd refuses a backward pass whose saved tensor has been overwritten since."""
+    def overwritten(shape, write):
+        t, x = torch.ones(shape, device="cuda"), torch.ones(shape, device="cuda", requires_grad=True)
+        loss = (x * t).sum()
+        with torch.no_grad():
+            write(t)
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            loss.backward()
+        with torch.inference_mode():
+            write(torch.ones(shape, device="cuda"))
+
+    q, _ = _case()
+    overwritten(q.shape, lambda t: _case(out=t)[1](q))
+    overwritten(q.shape[:2], lambda t: _case(lse_out=t)[1](q))
+    rows = _prompt()
+    overwritten(rows[0].shape, lambda t: _hip.host().prefill(*rows, t, [0, 70], 0.125))
