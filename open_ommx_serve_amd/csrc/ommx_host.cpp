@@ -92,6 +92,17 @@ void written(const at::Tensor& t) {
     if (!t.is_inference()) t.unsafeGetTensorImpl()->bump_version();
 }
 
+// Whether the memory that two tensors span has bytes in common (strides are never negative).
+bool share_memory(const at::Tensor& a, const at::Tensor& b) {
+    auto end = [](const at::Tensor& t) {
+        int64_t last = 0;
+        for (int64_t d = 0; d < t.dim(); ++d) last += (t.size(d) - 1) * t.stride(d);
+        return static_cast<const char*>(t.data_ptr()) + (last + 1) * static_cast<int64_t>(t.element_size());
+    };
+    if (a.numel() == 0 || b.numel() == 0) return false;
+    return static_cast<const char*>(a.data_ptr()) < end(b) && static_cast<const char*>(b.data_ptr()) < end(a);
+}
+
 bool failed(int rc, const char* what) {
     if (rc == 0) return false;
     PyErr_Format(PyExc_RuntimeError, "%s failed (rc=%d): %s", what, rc, ommx_last_error());
@@ -207,6 +218,9 @@ int run_decode(const DecodeCall& c) {
     const bool scale_bf16 = st == at::kBFloat16;
     if (st != v_scale.scalar_type() || (st != at::kChar && !scale_bf16) || scale_bf16 == c.int8) return 0;
     if (q.scalar_type() != at::kBFloat16 || q.stride(2) != 1) return 0;
+
+    // (the workgroups of the merge that writes a row's halves both read all of it)
+    if (c.hist_seq && share_memory(*c.o, q)) return 0;
 
     // lengths, tables, outputs
     if (c.seq->numel() < B || !c.seq->is_contiguous() || c.seq->scalar_type() != at::kInt) return 0;
@@ -821,7 +835,8 @@ PyObject* py_decode_pool(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return answer(run_decode(c));
 }
 
-// (q, k, v, out, starts, scale): causal attention of prompt rows, out fp32 or bf16.  An observed call is refused.
+// (q, k, v, out, starts, scale): causal attention of prompt rows, out fp32 or bf16.  An observed call is refused, and
+// so is an output that lies in the inputs (the caller's way through rows of its own serves it).
 PyObject* py_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != 6) { PyErr_SetString(PyExc_TypeError, "prefill: wrong number of arguments"); return nullptr; }
     if (!plain_call(a, 4)) Py_RETURN_FALSE;
@@ -845,6 +860,9 @@ PyObject* py_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
             (reinterpret_cast<uintptr_t>(t->data_ptr()) & 15))
             Py_RETURN_FALSE;
     }
+    // K and V are read by workgroups that end later; a workgroup reads its own rows of q before it writes them
+    const bool in_place = o->data_ptr() == q->data_ptr() && o->scalar_type() == q->scalar_type() && o->strides() == q->strides();
+    if (share_memory(*o, *k) || share_memory(*o, *v) || (!in_place && share_memory(*o, *q))) Py_RETURN_FALSE;
     if (starts.back() == starts[0]) Py_RETURN_TRUE;
     c10::hip::HIPGuard guard(q->device().index());
     hipStream_t stream = stream_of(q->device());

@@ -283,3 +283,19 @@ def test_layers_on_two_streams_each_read_the_step():
         return torch.stack(got)
 
     assert torch.equal(outputs(torch.cuda.Stream()), outputs(None))
+
+
+@pytest.mark.parametrize("batched", [False, True])
+def test_a_decode_step_writes_over_its_query(batched):
+    """The output may be the query's own memory: a copy in between, as the halves of a row are written separately."""
+    eng = _Engine(400, graph=False, batched=batched, max_num_seqs=2)
+    reqs = [_Request(11, 150, 160, 100), _Request(25, 97, 110, 200)][:2 if batched else 1]
+    eng.step(reqs, check=False)
+    eng.builder.build(0, NS(seq_lens_cpu=[r.seq + 1 for r in reqs], query_start_loc_cpu=list(range(len(reqs) + 1)),
+                            block_table_tensor=torch.tensor([[r.key, r.key + 1] for r in reqs])))
+    q, k, v = (torch.stack([t[r.seq] for r, t in zip(reqs, ts)]).to(DEV).to(torch.bfloat16) for ts in (
+        [r.q for r in reqs], [r.K[0] for r in reqs], [r.V[0] for r in reqs]))
+    eng.impls[0].do_kv_cache_update(eng.layers[0], k, v)
+    want = eng.impls[0].forward(eng.layers[0], q, k, v, None, None, torch.empty_like(q)).clone()
+    eng.impls[0].forward(eng.layers[0], q, k, v, None, None, q)
+    assert torch.equal(q, want)

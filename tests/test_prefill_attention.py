@@ -2,11 +2,13 @@
 wave, the 64-key and the 128-row tile, empty requests, rows that start past zero, every head
 grouping, both output types, and a batch whose tile list takes more than one launch."""
 import math
+from types import SimpleNamespace as NS
 
 import pytest
 import torch
 
 from open_ommx_serve_amd.attention import _hip
+from open_ommx_serve_amd.integration.vllm import backend
 from open_ommx_serve_amd.integration.vllm.backend import causal_prefill_attention
 
 pytestmark = pytest.mark.gpu
@@ -167,3 +169,27 @@ def test_values_that_are_no_numbers_reach_the_rows_from_theirs_on(D, hq, hkv, st
         # (tiles with such a value take the path of three bf16 pieces: fp32 sums in another order)
         torch.testing.assert_close(out.float(), want.to(dtype).float(), rtol=2.0 ** -7 if dtype == torch.bfloat16 else 0,
                                    atol=1e-5, equal_nan=True)
+
+
+@pytest.mark.parametrize("where", ["q", "k", "v", "fused", "shifted q"])
+def test_an_output_in_the_memory_of_the_inputs(where):
+    n, H, D = 700, 4, 64
+    fused = _rows(n, 4 * H, D, 1)
+    q, k, v = fused[:, :H], fused[:, H:2 * H], fused[:, 2 * H:3 * H]
+    q, k, v = (t if where == "fused" else t.contiguous() for t in (q, k, v))
+    if where == "shifted q":
+        q = torch.cat([q, q[:1]])[:n]
+        out = q.as_strided((n - 1, H, D), q.stride(), H * D)
+        q, k, v = q[:n - 1], k[:n - 1], v[:n - 1]
+    else:
+        out = fused[:, 3 * H:] if where == "fused" else {"q": q, "k": k, "v": v}[where]
+    n = out.shape[0]
+    want = torch.empty(n, H, D, dtype=torch.bfloat16, device=DEV)
+    assert _hip.host().prefill(q, k, v, want, [0, n], 0.125)
+    impl = backend.OMMXCanonicalImpl(H, D, 0.125, H)
+    backend.reset_worker_state(graph=False, batched=False, batched_graph=False)
+    backend.OMMXCanonicalMetadataBuilder().build(0, NS(seq_lens_cpu=[n], query_start_loc_cpu=[0, n],
+                                                       block_table_tensor=torch.tensor([[3, 4]])))
+    impl.forward(NS(), q, k, v, None, None, out)
+    backend.reset_worker_state()
+    assert torch.equal(out, want)
