@@ -741,11 +741,20 @@ PyObject* py_tail_gather(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyObject* py_rows_write(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != 10) { PyErr_SetString(PyExc_TypeError, "rows_write: wrong number of arguments"); return nullptr; }
     bool ok = true;
-    const at::Tensor *K = as_tensor(a[0], ok), *V = as_tensor(a[1], ok);
+    const at::Tensor *K = as_tensor(a[0], ok), *V = as_tensor(a[1], ok), *kh = as_tensor(a[2], ok), *vh = as_tensor(a[3], ok);
     const int64_t pos0 = as_int(a[5], ok);
     PyObject* const rest[] = {a[2], a[3], a[4], a[6], a[7], a[8], a[9]};
     ommx::BlockRows rows;
-    if (!ok || !read_block_rows(*K, *V, rest, pos0, rows)) Py_RETURN_FALSE;
+    if (!ok) Py_RETURN_FALSE;
+    at::Tensor copies[2];
+    if (K->is_alias_of(*kh) || K->is_alias_of(*vh) || V->is_alias_of(*kh) || V->is_alias_of(*vh)) {
+        // rows of the history itself: a launch writes them in no order
+        copies[0] = K->clone();
+        copies[1] = V->clone();
+        K = &copies[0];
+        V = &copies[1];
+    }
+    if (!read_block_rows(*K, *V, rest, pos0, rows)) Py_RETURN_FALSE;
     c10::hip::HIPGuard guard(K->device().index());
     hipStream_t stream = stream_of(K->device());
     int rc;

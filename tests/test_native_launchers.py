@@ -108,3 +108,19 @@ def test_live_rows_ride_along_with_the_groups(recipe, H, extra):
     for n, t in one.pool_planes().items():
         if torch.is_tensor(t):
             assert torch.equal(t.view(torch.uint8), two.pool_planes()[n].view(torch.uint8)), n
+
+
+@pytest.mark.parametrize("ring", [False, True])
+def test_a_block_may_come_out_of_the_history_it_goes_to(ring):
+    """Rows that overlap the slots they are written to: as from a copy of them."""
+    H, D, T = 2, 128, 150
+    pools = [MultiSeqKVPool(D, H, 2, 160, device=DEV, kv_ring=ring, **RECIPE) for _ in range(2)]
+    for p in pools:
+        for h, seed in ((p.k_hist, 9), (p.v_hist, 10)):
+            h.copy_(_block(h.shape[0] * h.shape[1], H, D, torch.bfloat16, seed).view(h.shape))
+    first = pools[0].k_hist.shape[1] - 60                    # from the first request's slots into the second's
+    for p, own in zip(pools, (True, False)):
+        K, V = (h.view(-1, H, D)[first:first + T] for h in (p.k_hist, p.v_hist))
+        p.append_block(1, K if own else K.clone(), V if own else V.clone())
+    for name in ("k_hist", "v_hist", "k_base", "k_scale", "v_main", "v_scale"):
+        assert torch.equal(getattr(pools[0], name), getattr(pools[1], name)), name
