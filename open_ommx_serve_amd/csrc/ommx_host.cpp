@@ -13,7 +13,9 @@
 #include <ATen/ATen.h>
 #include <ATen/EmptyTensor.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/core/CachingHostAllocator.h>
 #include <ATen/hip/impl/HIPCachingAllocatorMasqueradingAsCUDA.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/Allocator.h>
 #include <c10/core/GradMode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
@@ -634,6 +636,9 @@ PyObject* py_pack_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
     rc = launch_store(*K, *V, 0, p, r, T, ps, nullptr, nullptr, nullptr, *table, t[FLAGS].data_ptr<int32_t>(),
                       {true, t[TOK].data_ptr<int32_t>(), t[GRP].data_ptr<int32_t>()}, stream);
     Py_END_ALLOW_THREADS
+    // Should the caller never ask for the errors, the block must not be handed on before the kernel is through with it.
+    at::getHostAllocator(c10::DeviceType::CUDA)->record_event(t[FLAGS].data_ptr(), t[FLAGS].storage().data_ptr().get_context(),
+                                                              c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index()).unwrap());
     if (failed(rc, "ommx_store_pack")) return nullptr;
     PyObject* out = PyTuple_New(COUNT);
     for (int i = 0; i < COUNT; ++i) {

@@ -7,6 +7,7 @@ import torch
 import oracle.ommx_oracle as O
 from open_ommx_serve_amd.attention import MultiSeqKVPool, WindowSpec, _hip, ommx_pack_kv_canonical_block
 from open_ommx_serve_amd.attention.kv_store_ops import ring_slot
+from open_ommx_serve_amd.attention.pack import store_table
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -124,3 +125,23 @@ def test_a_block_may_come_out_of_the_history_it_goes_to(ring):
         p.append_block(1, K if own else K.clone(), V if own else V.clone())
     for name in ("k_hist", "v_hist", "k_base", "k_scale", "v_main", "v_scale"):
         assert torch.equal(getattr(pools[0], name), getattr(pools[1], name)), name
+
+
+def test_error_words_nobody_asks_for_stay_until_the_kernel_is_through():
+    """The block goes back to torch's pinned allocator, which must not hand it on while a kernel may write to it."""
+    K, V = _block(128, 2, 128, torch.bfloat16, 11), _block(128, 2, 128, torch.bfloat16, 12)
+
+    def launch():
+        return _hip.host().pack_block(K, V, 16, True, store_table(K.device), 6, 32, 32, "bitmap", "signed", True, True, "i2")[0]
+
+    held = [launch() for _ in range(20)]                     # (more than are kept idle)
+    torch.cuda.synchronize()
+    torch.cuda._sleep(20_000_000)                            # some ten milliseconds
+    flags = launch()
+    at, words = flags.data_ptr(), flags.numel()
+    del flags
+    others = [torch.empty(words, dtype=torch.int32, pin_memory=True) for _ in range(4)]
+    assert not torch.cuda.current_stream().query()           # (still asleep: the test means something)
+    assert at not in [t.data_ptr() for t in others]
+    torch.cuda.synchronize()
+    del held
