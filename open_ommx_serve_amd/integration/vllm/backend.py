@@ -256,15 +256,15 @@ class OMMXCanonicalImpl(_ImplBase):
     # ── write ────────────────────────────────────────────────────────────────────
 
     def do_kv_cache_update(self, layer, key, value, kv_cache=None, slot_mapping=None) -> None:
-        n = int(key.shape[0])
+        rows = key.shape
+        n = int(rows[0])
         if n == 0:
             return
         s, st = _STATE, _STATE.step
         cfg = self._ommx_cfg()
-        if key.shape[1:] != (self.num_kv_heads, self.head_size):
-            key = key.reshape(n, self.num_kv_heads, self.head_size)
-        if value.shape[1:] != (self.num_kv_heads, self.head_size):
-            value = value.reshape(n, self.num_kv_heads, self.head_size)
+        H, D = self.num_kv_heads, self.head_size
+        if len(rows) != 3 or rows[1] != H or rows[2] != D or value.shape != rows:
+            key, value = key.reshape(n, H, D), value.reshape(n, H, D)
         if st["B"] == STEP_ROUTE_UNCLASSIFIED and not st["batched_write"]:
             raise RuntimeError(
                 "[ommx] cannot classify this step: the metadata exposed no readable per-request "
@@ -353,10 +353,11 @@ class OMMXCanonicalImpl(_ImplBase):
     def forward(self, layer, query, key, value, kv_cache=None, attn_metadata=None, output=None,
                 output_scale=None, output_block_scale=None):
         H, D = self.num_heads, self.head_size
-        q = query if query.shape[1:] == (H, D) else query.reshape(-1, H, D)
         if output is None:
             output = torch.empty_like(query)
-        out = output if output.shape[1:] == (H, D) else output.view(-1, H, D)
+        rows, q, out = query.shape, query, output
+        if len(rows) != 3 or rows[1] != H or rows[2] != D or output.shape != rows:
+            q, out = query.reshape(-1, H, D), output.view(-1, H, D)
         st = _STATE.step
         if st["B"] == STEP_ROUTE_UNCLASSIFIED:
             raise RuntimeError("[ommx] unclassified step: request count unknown, refusing to "

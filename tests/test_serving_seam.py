@@ -298,7 +298,7 @@ def test_identity_is_required_unless_the_unsafe_hatch_is_set(monkeypatch):
 def test_each_stream_has_its_own_block_and_tables_of_a_step(monkeypatch):
     """A layer on another stream is not ordered behind the first layer's upload: nothing may be handed over."""
     m, _ = _bmgr(graph=False)
-    pool = NS(k_hist=NS(device=torch.device("cpu")), _req_to_token=torch.arange(40).view(4, 10),
+    pool = NS(k_hist=torch.empty(1), _req_to_token=torch.arange(40).view(4, 10),
               _req_to_group=torch.arange(20).view(4, 5))
     now, uploads = [1], []
 
@@ -308,8 +308,9 @@ def test_each_stream_has_its_own_block_and_tables_of_a_step(monkeypatch):
         block[2 * n64:].copy_(torch.tensor(values[n64:], dtype=torch.int32))
         return True
 
-    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: now[0], raising=False)
-    monkeypatch.setattr("open_ommx_serve_amd.integration.vllm.metadata._hip.host", lambda: NS(upload=upload))
+    seam = "open_ommx_serve_amd.integration.vllm.metadata."
+    monkeypatch.setattr(seam + "_current_stream", lambda index: now[0])
+    monkeypatch.setattr(seam + "_hip.host", lambda: NS(upload=upload))
 
     def memory(step):
         return {t.untyped_storage().data_ptr() for t in (*step[:4], *step.tables)}
