@@ -24,12 +24,14 @@
 //
 // Bound: matrix instructions and vector instructions share a SIMD's time (next to a wave that issues matrix
 // instructions back to back another one keeps about half its vector rate).  4096 tokens of 32 heads:
-// 200 K clocks of matrix instructions (82 us at 2.4 GHz) and 220 K of vector ones in 377 K.  Two groups of waves in one
-// workgroup, one half a tile behind the other so that the matrix phase of one meets the vector phase of
-// the other, share the staged tiles as well: 264 -> 191 us (same box).  In lockstep, without the shift, the eight
-// waves took 210 us, as two workgroups of four 233 us; any register spilled in the loop costs more than
-// all of this, because its reload waits for the loads on their way (285 us).  Short prompts are latency: one group
-// per workgroup, two workgroups per compute unit (see prefill_attention).  The library's fp32 attention took 2.45 ms.
+// 203 K clocks of matrix instructions (85 us at 2.4 GHz) and 203 K of vector ones in 363 K (rocprofv3 counters).  That is
+// 191 to 200 us from box to box (HIP events around launches back to back; the kernel trace of rocprofv3 has 204 at least
+// and 207 on average).  Two groups of waves in one workgroup, one half a tile behind the other so that the matrix phase of
+// one meets the vector phase of the other, share the staged tiles as well: 264 -> 191 us (events, one box, with two pieces
+// and no second pass).  In lockstep, without the shift, the eight waves took 210 us, as two workgroups of four 233 us; any
+// register spilled in the loop costs more than all of this, because its reload waits for the loads on their way (285 us).
+// Short prompts are latency: one group per workgroup, two workgroups per compute unit (see prefill_attention).  The
+// library's fp32 attention took 2.45 ms.
 #include <algorithm>
 
 #include "ommx_common.h"
@@ -93,8 +95,9 @@ __device__ __forceinline__ u32x4 load16(__amdgpu_buffer_rsrc_t rows, uint32_t at
 // exp2 in range serves an online softmax, and most tiles then rescale nothing.
 // Weights are carried times 2^8, at most 2^15.75 with the slack, within f16.  More would leave less to the second pass,
 // but the shift is part of exp2's argument, which is rounded to 24 bits: at 2^9 and above plain short rows are less exact
-// than the library's (1.6e-7, at 2^12 2.0e-7, against 1.5e-7), and the smaller slack rescales more tiles (4096 rows 199
-// against 194 us).  The gain as a factor of its own costs 6 % (mixed-precision or plain multiplications).
+// than the library's (1.6e-7, at 2^12 2.0e-7, against 1.5e-7), and the smaller slack rescales more tiles (4096 rows, at
+// 2^8 and 2^12: 2 % and 3.5 % above 2^6 without the second pass).  The gain as a factor of its own costs 5 to 7 % (plain
+// multiplications, mixed-precision fused ones).
 // V is carried times 2^8 and divided by it at the end.
 constexpr float P_SHIFT = 8.0f, MAX_SLACK = 7.75f, V_GAIN = 256.0f;
 // In the second pass the sums so far and its weights are carried times this: a V of 2^100 is still in range.
