@@ -26,7 +26,6 @@ import os
 from typing import Dict, List, Optional, Sequence, Tuple
 
 import torch
-from torch.compiler import is_compiling
 
 from . import _hip
 from .kv_store_ops import gather_tails, ring_slot, write_tokens
@@ -625,8 +624,6 @@ class MultiSeqKVPool:
         gather launch; ``b_seq_len`` (int32) are the packed lengths, ``tables`` the page / group rows of
         the slots.  False when the native launcher does not take the arguments (nothing is done then), or
         the call is traced, transformed or differentiated."""
-        if is_compiling():
-            return False
         return self._host.decode_pool(q, self._store_planes, self.k_hist, self.v_hist, rows, seq, b_seq_len,
                                       tables[0], tables[1], out, sm_scale, self.ps, max_seq_len, mean_seq_len,
                                       self._ring_sink, self._ring_rec, self.window.sink_tokens,

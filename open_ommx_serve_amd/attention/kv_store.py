@@ -16,7 +16,6 @@ from __future__ import annotations
 from typing import Optional, Tuple
 
 import torch
-from torch.compiler import is_compiling
 
 from . import _hip
 from .kv_pool import _env_flag, check_serving_recipe
@@ -357,8 +356,6 @@ class CanonicalKVStore:
         from the history at the device length ``seq`` (int64 ``[1]``); ``b_seq_len`` (int32) is the packed
         length.  False when the native launcher does not take the arguments (nothing is done then), or
         the call is traced, transformed or differentiated."""
-        if is_compiling():
-            return False
         return self._host.decode_pool(q, self._store_planes, self._k_hist4, self._v_hist4, None, seq, b_seq_len,
                                       self._req_to_token_full, self._req_to_group_full, out, sm_scale, self.ps,
                                       max_seq_len, None, self._ring_sink, self._ring_rec, self.window.sink_tokens,

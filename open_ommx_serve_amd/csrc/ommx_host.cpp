@@ -390,6 +390,18 @@ PyObject* answer(int rc) {
     return PyBool_FromLong(rc);
 }
 
+// (a, b, heads, head_dim): whether both are [rows, heads, head_dim]
+PyObject* py_rows_fit(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    bool ok = n == 4;
+    const at::Tensor *x = ok ? as_tensor(a[0], ok) : nullptr, *y = ok ? as_tensor(a[1], ok) : nullptr;
+    if (!ok) { PyErr_SetString(PyExc_TypeError, "rows_fit: two tensors, heads and head_dim expected"); return nullptr; }
+    const int64_t H = as_int(a[2], ok), D = as_int(a[3], ok);
+    auto fits = [&](const at::Tensor& t) {
+        return !t.unsafeGetTensorImpl()->has_symbolic_sizes_strides() && t.dim() == 3 && t.size(1) == H && t.size(2) == D;
+    };
+    return PyBool_FromLong(ok && fits(*x) && fits(*y));
+}
+
 // (tensors or None ...)
 PyObject* py_plain(PyObject*, PyObject* const* a, Py_ssize_t n) { return PyBool_FromLong(plain_call(a, n)); }
 
@@ -926,7 +938,7 @@ PyObject* guarded(PyObject* self, PyObject* const* a, Py_ssize_t n) {
 
 #define OMMX_FAST(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(guarded<py_##name>)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
-    OMMX_FAST(auto_num_kv_splits), OMMX_FAST(plain),
+    OMMX_FAST(auto_num_kv_splits), OMMX_FAST(plain), OMMX_FAST(rows_fit),
     OMMX_FAST(decode), OMMX_FAST(decode_pool), OMMX_FAST(store_pack), OMMX_FAST(pack_block), OMMX_FAST(block_errors), OMMX_FAST(pack_groups), OMMX_FAST(ring_write),
     OMMX_FAST(tail_gather), OMMX_FAST(rows_write), OMMX_FAST(upload), OMMX_FAST(prefill),
     {nullptr, nullptr, 0, nullptr},

@@ -256,14 +256,13 @@ class OMMXCanonicalImpl(_ImplBase):
     # ── write ────────────────────────────────────────────────────────────────────
 
     def do_kv_cache_update(self, layer, key, value, kv_cache=None, slot_mapping=None) -> None:
-        rows = key.shape
-        n = int(rows[0])
+        n = int(key.shape[0])
         if n == 0:
             return
         s, st = _STATE, _STATE.step
         cfg = self._ommx_cfg()
         H, D = self.num_kv_heads, self.head_size
-        if len(rows) != 3 or rows[1] != H or rows[2] != D or value.shape != rows:
+        if not _hip.host().rows_fit(key, value, H, D):
             key, value = key.reshape(n, H, D), value.reshape(n, H, D)
         if st["B"] == STEP_ROUTE_UNCLASSIFIED and not st["batched_write"]:
             raise RuntimeError(
