@@ -25,9 +25,9 @@
 // Bound: matrix instructions and vector instructions share a SIMD's time (next to a wave that issues matrix
 // instructions back to back another one keeps about half its vector rate).  4096 tokens of 32 heads:
 // 203 K clocks of matrix instructions (85 us at 2.4 GHz) and 203 K of vector ones in 363 K (rocprofv3 counters).  That is
-// 191 to 200 us from box to box (HIP events around launches back to back; the kernel trace of rocprofv3 has 204 at least
+// 191 to 200 us from card to card (HIP events around launches back to back; the kernel trace of rocprofv3 has 204 at least
 // and 207 on average).  Two groups of waves in one workgroup, one half a tile behind the other so that the matrix phase of
-// one meets the vector phase of the other, share the staged tiles as well: 264 -> 191 us (events, one box, with two pieces
+// one meets the vector phase of the other, share the staged tiles as well: 264 -> 191 us (events, one card, with two pieces
 // and no second pass).  In lockstep, without the shift, the eight waves took 210 us, as two workgroups of four 233 us; any
 // register spilled in the loop costs more than all of this, because its reload waits for the loads on their way (285 us).
 // Short prompts are latency: one group per workgroup, two workgroups per compute unit (see prefill_attention).  The
