@@ -1,6 +1,8 @@
 // Tuned split-KV decode kernel for gfx950: head_dim 128, 1, 2, 4 or 8 q heads per kv head, 6 (or
 // 0) outliers per K vector of 32 tokens; with the position-stream index plane also K vectors of
 // 64 / 128 tokens (6 outliers, or 10 with 128 tokens) and V vectors of 64 / 128 channels.
+// ommx_decode_gqa4.hip takes most of these shapes first; what is left here is the recipe without outliers, and
+// planes that kernel does not address (4 GiB and more, or of an extent that the caller has not given).
 // Same operator as ommx_gpu_serve/attention/paged_decode.py:1255-2284.
 //
 // Work decomposition.  A wavefront owns one kv head (and all 4 or 8 of its q heads) of one

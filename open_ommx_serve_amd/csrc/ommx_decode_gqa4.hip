@@ -1,9 +1,10 @@
 // Split-KV decode kernel for gfx950, serving shape: head_dim 128, 1, 2, 4 or 8 q heads per kv head,
 // 6 outliers per K vector of 32 tokens (either index plane, either outlier map), INT2 V with
 // 32-channel vectors, int8 exponents; in a general form (GEN) also 1..8 outliers on the bitmap
-// plane and head_dim 64 with 1, 2 or 4 q heads per kv head.  Same operator as
+// plane and head_dim 64 with 1, 2 or 4 q heads per kv head; and (GTS) K vectors of 64 or 128 tokens on
+// the position-stream plane with 4 or 8 q heads per kv head, 6 outliers or 10 of 128.  Same operator as
 // ommx_gpu_serve/attention/paged_decode.py:1255-2284; the other shapes of the matrix-core path
-// (longer groups, no outliers) stay on the kernel in ommx_decode.hip.
+// (no outliers, planes of 4 GiB and more or of unknown extent) stay on the kernel in ommx_decode.hip.
 //
 // A wavefront owns one kv head (and its q heads) of one split and walks it 64 tokens at a time;
 // a workgroup is 4 waves = 4 neighbouring kv heads.  Measured on MI355X this operator is bound
@@ -23,7 +24,7 @@
 // takes four accumulators, and two workgroups fit a compute unit (190 registers, 14.1 KB of LDS
 // per wave); everything up to the logits is the same code.
 // Arithmetic: exact 16-bit operands, fp32 accumulation, as in ommx_decode.hip.
-//   A (QK)   q * 2^(10-2m) as f16 in pair order, m = 1..4 fixed per channel pair; this one operand
+//   A (QK)   q * 2^(10-2m) as f16 in pair order, m = 2..4 (3 or 4 with longer groups) fixed per channel pair; this one operand
 //            set serves the base codes, the outlier tile and the bias columns.
 //   K base   B = (1 + code*2^(2m-10)) * 2^e as f16: the 2-bit code is dropped into mantissa bits
 //            [2m+1:2m] of a per-(group, channel) pattern that carries the exponent, one and-or per
@@ -57,26 +58,27 @@ constexpr int KT_ROW = 40;                          // bytes per staged K code r
 constexpr int VT_COL = 68;                          // dwords per V dword column (64 used)
 constexpr int PT_ROW = 72;                          // halfwords per row of the f16 [row][64 tokens] arrays
 constexpr int OFF_TILE = 0;                         // [32 tokens][TILE_ROW] f16 outlier deltas of one group
-constexpr int OFF_KT = OFF_TILE + 32 * TILE_ROW;    // [64 tokens][KT_ROW] K code rows
-constexpr int OFF_MAG = OFF_KT + 64 * KT_ROW;       // [2 groups][128] f16 2^e, channels (p, p+8) adjacent
-constexpr int OFF_ZPP = OFF_MAG + 512;              // same order, f16 zero points over the A scale
-// after QK the same bytes hold what P.V needs
-constexpr int OFF_VT = OFF_KT;                      // [8 dword columns][VT_COL] V code dwords
-constexpr int OFF_PT = OFF_VT + 8 * VT_COL * 4;     // [NH heads][PT_ROW] f16 softmax weights
-// what follows the weights depends on the number of q heads per kv head (NH = 4 or 8)
-template <int NH>
+// The rest depends on the number of q heads per kv head (NH = 4 or 8) and, with groups longer than 32 tokens, on one
+// more row of the tile: where the outliers of the group's other tokens go.
+template <int NH, bool LONG>
 struct LdsMap {
+    static constexpr int OFF_KT = OFF_TILE + (LONG ? 33 : 32) * TILE_ROW;    // [64 tokens][KT_ROW] K code rows
+    static constexpr int OFF_MAG = OFF_KT + 64 * KT_ROW;       // [2 groups][128] f16 2^e, channels (p, p+8) adjacent
+    static constexpr int OFF_ZPP = OFF_MAG + 512;              // same order, f16 zero points over the A scale
+    // after QK the same bytes hold what P.V needs
+    static constexpr int OFF_VT = OFF_KT;                      // [8 dword columns][VT_COL] V code dwords
+    static constexpr int OFF_PT = OFF_VT + 8 * VT_COL * 4;     // [NH heads][PT_ROW] f16 softmax weights
     static constexpr int OFF_VZ = OFF_PT + NH * PT_ROW * 2;    // [4 channel groups][PT_ROW] f16 V zero points
     static constexpr int OFF_VS = OFF_VZ + 4 * PT_ROW * 2;     // [4 channel groups][PT_ROW] f16 2^e_v
     static constexpr int OFF_STAGE_END = (OFF_VS + 4 * PT_ROW * 2 > OFF_ZPP + 512) ? OFF_VS + 4 * PT_ROW * 2 : OFF_ZPP + 512;
     static constexpr int OFF_LC = OFF_STAGE_END;               // [32 tokens][NH heads] f32 logit corrections of one group
     static constexpr int OFF_ZERO = OFF_LC + 32 * NH * 4;      // 128 B of zeros, never written again
     static constexpr int OFF_ONES = OFF_ZERO + 128;            // 128 B of f16 1.0, never written again
-    static constexpr int LDS_WAVE = OFF_ONES + 128;            // 13376 (4 heads) / 14464 (8 heads)
+    static constexpr int LDS_WAVE = OFF_ONES + 128;            // 13376 (4 heads) / 14464 (8 heads), LONG 272 more
     static_assert(OFF_KT % 16 == 0 && OFF_PT % 16 == 0 && OFF_VZ % 16 == 0 && OFF_LC % 16 == 0, "b128 alignment");
 };
-static_assert(3 * 4 * LdsMap<4>::LDS_WAVE <= 160 * 1024, "4 heads: three workgroups per compute unit");
-static_assert(2 * 4 * LdsMap<8>::LDS_WAVE <= 160 * 1024, "8 heads: two workgroups per compute unit");
+static_assert(3 * 4 * LdsMap<4, true>::LDS_WAVE <= 160 * 1024, "4 heads: three workgroups per compute unit");
+static_assert(2 * 4 * LdsMap<8, true>::LDS_WAVE <= 160 * 1024, "8 heads: two workgroups per compute unit");
 
 // One f16 carries 11 bits: rounding an outlier delta d costs up to |d| * 2^-11, i.e. up to
 // |d| * max|q| * 2^-11 * sm_scale on a logit.  A delta with |d| * max|q| >= BIG_DELTA * 16
@@ -89,7 +91,7 @@ constexpr float BIG_DELTA = 2.0f;
 constexpr float BIG_DELTA_SM_SCALE = 0.08838834764831845f;
 // the running maximum of the online softmax is refreshed when a logit (base 2) exceeds it by this
 constexpr float MAX_SLACK = 8.0f;
-// The base operand (1 + code*2^(2m-10)) * 2^e carries a constant A*2^e per channel, up to 2^8 times
+// The base operand (1 + code*2^(2m-10)) * 2^e carries a constant A*2^e per channel, up to 2^6 times
 // the signal, which the bias MFMA takes out again: two large sums that cancel in fp32.  From steps
 // of 2^EXACT_STEP_EXP on (values a hundred or more wide inside one vector) that shows on the logits, and
 // the step's two groups take the operand code*2^(2m-10+e) instead (one packed subtraction more per operand
@@ -100,14 +102,21 @@ constexpr int EXACT_STEP_EXP = 5;
 constexpr int MAX_STEP_EXP = 15;
 
 // K pair p of a code dword: channels p (low half) and p+8 (high half) as f16 with the 2-bit
-// code at mantissa bits [2m+1:2m], m = k_pos(p) in 1..4, where the element reads
-// (1 + code * 2^(2m-10)) * 2^e; the A operand of that channel carries q * 2^(10-2m).  Four
-// positions, so that only pairs 0 (up two bits) and 5..7 (down six) need a shift.
-__host__ __device__ constexpr int k_pos(int p) { return p == 0 ? 1 : (p <= 4 ? p : p - 3); }
-template <int P>
-__device__ __forceinline__ uint32_t k_pair(uint32_t w, uint32_t w_up2, uint32_t w_dn6, uint32_t magic) {
-    const uint32_t sh = P == 0 ? w_up2 : (P <= 4 ? w : w_dn6);
-    return (sh & (0x00030003u << (2 * k_pos(P)))) | magic;
+// code at mantissa bits [2m+1:2m], m = k_pos(p), where the element reads
+// (1 + code * 2^(2m-10)) * 2^e; the A operand of that channel carries q * 2^(10-2m).  Positions 2..4, so that
+// only pairs 0, 1 (up four bits) and 5..7 (down six) need a shift; m = 1 (pair 1 unshifted) would carry a constant
+// four times as large through the sums, and the error of the logits with it.  Longer groups have larger steps and
+// fewer roundings elsewhere (their outliers are often exact): they take positions 3 and 4, two more shifts a dword.
+template <bool LONG>
+__host__ __device__ constexpr int k_pos(int p) {
+    if (LONG) return p <= 1 ? p + 3 : p == 2 ? 3 : p <= 4 ? p : p == 5 ? 3 : 4;
+    return p <= 1 ? p + 2 : (p <= 4 ? p : p - 3);
+}
+template <int P, bool LONG>
+__device__ __forceinline__ uint32_t k_pair(uint32_t w, uint32_t w_up, uint32_t w_dn6, uint32_t magic) {
+    const uint32_t sh = LONG ? (P <= 1 ? w_up : P == 2 ? w << 2 : P <= 4 ? w : P <= 6 ? w >> 4 : w_dn6)
+                             : (P <= 1 ? w_up : P <= 4 ? w : w_dn6);
+    return (sh & (0x00030003u << (2 * k_pos<LONG>(P)))) | magic;
 }
 // V channel y of a merged dword (token a in the low 16 bits, token b in the high 16 bits) as
 // f16 (1 + c/16) * 2^e (even y, code at mantissa bits [7:6]) or (1 + c/4) * 2^e (odd y, bits
@@ -129,18 +138,33 @@ __device__ __forceinline__ uint32_t pk_u16(uint32_t lo, uint32_t hi) { return (l
 // head_dim 64 (a.half): the planes of two neighbouring 64-channel kv heads read exactly like one
 // 128-channel head, so a wave takes the pair as one head whose q heads are those of both, each
 // zero on the other one's channels, and writes each q head only its own half of the output.
-template <int IDX, bool OWN_MAP, bool PARTIAL, int ORDER, int NH = 4, bool GEN = false, int KSLOTS = 6>
+// GTS: K groups of 32 << GTS tokens (position streams; V vectors then 32, 64 or 128 channels wide), 6 outliers, or
+// 10 with 128 tokens (KSLOTS).  The 64 tokens of a step lie in one group then, whose parameters are held once, and
+// each 32-token half of the step walks all of the group's outliers: the ones that lie elsewhere go to a row of the
+// tile that nobody reads, which costs their instructions (10 outliers per 128 tokens walked four times are 40 a step
+// and channel pair, against 24 in a 32-token recipe) but no branch.  The work is dealt out in those 64-token steps:
+// whole groups of 128 left a batch of 342 groups on 172 of 256 resident workgroups, four serial steps each.  Whole
+// call, ommx_decode.hip's kernel on whole groups -> this one: 128 tokens and 10 outliers, 4 requests of 2 to 20 K
+// 45.9 -> 34.7 us, one of 64 K 47.1 -> 40.0, 8 of 4 to 16 K with 64 q heads 84.7 -> 52.6; 64 tokens and 6 outliers,
+// 64 K 36.8 -> 32.3, 1.1 K 15.5 -> 14.5.
+template <int IDX, bool OWN_MAP, bool PARTIAL, int ORDER, int NH = 4, bool GEN = false, int KSLOTS = 6, int GTS = 0>
 __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : OMMX_GQA4_WAVES) decode_gqa4_kernel(DecodeArgs a) {
     static_assert(NH == 4 || (NH == 8 && !PARTIAL), "4 heads (or fewer, PARTIAL) or exactly 8");
     static_assert(!GEN || IDX == 0, "the general form reads bitmaps");
     // outlier slots walked per vector: the general form walks 4 or 8 whatever a.kout is (loads and
     // arithmetic of all slots go out together; only the writes of the slots beyond a.kout are skipped)
-    constexpr int KMAX = GEN ? KSLOTS : 6;
-    static_assert(KMAX == 4 || KMAX == 6 || KMAX == 8, "outlier slots");
-    const int kout = GEN ? a.kout : 6;
+    constexpr int KMAX = KSLOTS;
+    static_assert(GEN ? KMAX == 4 || KMAX == 6 || KMAX == 8 : KMAX == 6 || (KMAX == 10 && GTS == 2), "outlier slots");
+    static_assert(GTS == 0 || (IDX == 1 && !GEN && !PARTIAL), "longer groups are read through position streams");
+    constexpr bool LONG = GTS > 0;
+    constexpr int GT_SH = 5 + GTS;                    // log2 of the tokens per K group
+    constexpr int UNIT_SH = LONG ? 6 : 5;             // log2 of the tokens that the work is dealt out in
+    constexpr int NG = LONG ? 1 : 2;                  // groups (parameter sets) a step reads
+    const int kout = GEN ? a.kout : KMAX;
     const bool half = GEN && a.half;
-    using Lds = LdsMap<NH>;
-    constexpr int OFF_VZ = Lds::OFF_VZ, OFF_VS = Lds::OFF_VS, OFF_LC = Lds::OFF_LC, OFF_ZERO = Lds::OFF_ZERO,
+    using Lds = LdsMap<NH, LONG>;
+    constexpr int OFF_KT = Lds::OFF_KT, OFF_MAG = Lds::OFF_MAG, OFF_ZPP = Lds::OFF_ZPP, OFF_VT = Lds::OFF_VT,
+                  OFF_PT = Lds::OFF_PT, OFF_VZ = Lds::OFF_VZ, OFF_VS = Lds::OFF_VS, OFF_LC = Lds::OFF_LC, OFF_ZERO = Lds::OFF_ZERO,
                   OFF_ONES = Lds::OFF_ONES, LDS_WAVE = Lds::LDS_WAVE;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem_all[];
     const int lane = threadIdx.x & 63;
@@ -161,7 +185,7 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
     int b = ORDER == 0 ? 0 : static_cast<int>(blockIdx.z), L;      // ORDER 0 is launched for one request only
     if (dealt) {
         shares::Share mine;
-        if (!shares::find_share<32, ORDER == 2 ? 4 : 1>(a, blockIdx.y, lane, mine)) return;
+        if (!shares::find_share<(1 << UNIT_SH), ORDER == 2 ? 4 : 1>(a, blockIdx.y, lane, mine)) return;
         b = mine.b; L = mine.L; sp = mine.sp; S = mine.n;
     } else if (ORDER >= 1 && a.B > 1 && a.B <= 64) {
         const int my_len = lane < a.B ? a.seq[lane] : 0;
@@ -214,8 +238,8 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
             qraw[r] = (!half || (lane >> 5) == sl / r_half) ? w : 0u;
         }
     }
-    // The A operands are q * 2^(10-2m) as f16, up to q * 2^8: a query element of 256 or more would not
-    // fit.  When the wave's largest |q| reaches 2^7 the whole query is taken divided by a power of two
+    // The A operands are q * 2^(10-2m) as f16, up to q * 2^6, and partly scaled up again below: large query elements would
+    // not fit.  When the wave's largest |q| reaches 2^7 the whole query is taken divided by a power of two
     // (exact) that brings it below, and the softmax scale carries the factor back; 0 for ordinary queries.
     int q_down = 0;
     {
@@ -241,17 +265,17 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
             qraw[r] = (__float_as_uint(lo) >> 16) | (__float_as_uint(hi) & 0xFFFF0000u);
         }
     }
-    // The 32-token groups are dealt out evenly: every split takes G/S groups and the first G%S
-    // splits one more, so no two splits differ by more than one group and none is empty while
+    // The 32-token groups (64-token pieces of longer ones) are dealt out evenly: every split takes G/S of them and
+    // the first G%S splits one more, so no two splits differ by more than one group and none is empty while
     // G >= S.  (One 32-bit division; the combine weighs the states by their lse, -inf for an
     // empty split, so it need not know this rule.)
     if (L < 0) { L = 0; report_table_range(a.err, true); }      // a negative length: nothing packed, reported
-    const uint32_t G = static_cast<uint32_t>(L + 31) >> 5;
+    const uint32_t G = static_cast<uint32_t>(L + (1 << UNIT_SH) - 1) >> UNIT_SH;
     const uint32_t g_each = G / S, g_more = G - g_each * S;
     const uint32_t g_first = static_cast<uint32_t>(sp) * g_each + min(static_cast<uint32_t>(sp), g_more);
     const uint32_t g_count = g_each + (static_cast<uint32_t>(sp) < g_more ? 1u : 0u);
-    const int n_begin = static_cast<int>(g_first << 5);
-    const int n_end = min(static_cast<int>((g_first + g_count) << 5), L);
+    const int n_begin = static_cast<int>(g_first << UNIT_SH);
+    const int n_end = min(static_cast<int>((g_first + g_count) << UNIT_SH), L);
 
     if (n_begin >= n_end) {       // an empty split: the state of nothing attended
         for (int r = 0; r < heads; ++r) {
@@ -268,22 +292,23 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
     const int last = n_end - 1;
     const int ps_sh = __ffs(a.ps) - 1, ps_mask = a.ps - 1;
     const int tsh = a.i64 ? 3 : 2;
-    const int tok_off = a.gbase * 32 + a.off;
+    const int tok_off = (a.gbase << GT_SH) + a.off;
     const char* const rt_b = static_cast<const char*>(a.rt) + ((b * a.rt_s) << tsh);
     const char* const rg_b = static_cast<const char*>(a.rg) + ((b * a.rg_s + a.gbase) << tsh);
     const uint8_t* const kb_head = a.k_base + kvh * 32;
     const uint8_t* const vb_head = a.v_main + kvh * 32;
-    const int8_t* const vs_head = a.v_scale + kvh * 4;
-    const uint16_t* const vz_head = a.v_zp + kvh * 4;
+    const int vv_sh = !LONG || a.gc == 32 ? 2 : a.gc == 64 ? 1 : 0;     // log2 of the V vectors per token
+    const int8_t* const vs_head = a.v_scale + (kvh << vv_sh);
+    const uint16_t* const vz_head = a.v_zp + (kvh << vv_sh);
 
-    int pg1, ps1, gsl[2];
+    int pg1, ps1, gsl[NG];
     auto fetch_tables = [&](int n) {
         const int p = min(n + lane, last) + tok_off;
         pg1 = *reinterpret_cast<const int*>(rt_b + ((uint32_t)(p >> ps_sh) << tsh));
         ps1 = p & ps_mask;
 #pragma unroll
-        for (int g = 0; g < 2; ++g) {
-            const int gi = min((n + 32 * g) >> 5, last >> 5);
+        for (int g = 0; g < NG; ++g) {
+            const int gi = min((n + 32 * g) >> GT_SH, last >> GT_SH);
             gsl[g] = *reinterpret_cast<const int*>(rg_b + ((uint32_t)gi << tsh));
         }
     };
@@ -305,13 +330,24 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
     auto fetch_v = [&]() {          // a row of v_scale is an eighth, a row of v_zp a quarter of a code row
         vr[0] = *reinterpret_cast<const u32x4*>(at(vb_head, vro));
         vr[1] = *reinterpret_cast<const u32x4*>(at(vb_head, vro + 16));
-        vsc = *reinterpret_cast<const uint32_t*>(at(vs_head, vro >> 3));
-        vzp = *reinterpret_cast<const u32x2*>(at(vz_head, vro >> 2));
+        if (vv_sh == 2) {
+            vsc = *reinterpret_cast<const uint32_t*>(at(vs_head, vro >> 3));
+            vzp = *reinterpret_cast<const u32x2*>(at(vz_head, vro >> 2));
+        } else if (vv_sh == 1) {        // (spread over the four 32-channel quarters where they are used)
+            vsc = *reinterpret_cast<const uint16_t*>(at(vs_head, vro >> 4));
+            vzp[0] = *reinterpret_cast<const uint32_t*>(at(vz_head, vro >> 3));
+        } else {
+            vsc = *reinterpret_cast<const uint8_t*>(at(vs_head, vro >> 5));
+            vzp[0] = *reinterpret_cast<const uint16_t*>(at(vz_head, vro >> 4));
+        }
     };
     // channel pair (2*lane, 2*lane+1) parameters of both groups
-    uint32_t g_sc[2], g_zp[2], g_ms[2] = {0, 0}, g_mc[2] = {0, 0};
-    u32x2 g_bm[2], g_ov[2];
-    uint32_t g_bx[2] = {0, 0};
+    uint32_t g_sc[NG], g_zp[NG], g_ms[NG] = {}, g_mc[NG] = {};
+    u32x2 g_bm[NG], g_ov[NG];
+    uint32_t g_bx[NG] = {};
+    // 10 outliers: 18 index bytes and 10 nibble bytes per lane start at a multiple of 2; the aligned dwords that
+    // cover them are loaded and shifted into place when they are used
+    uint32_t g_ix10[5] = {}, g_ov10[3] = {};
     const uint32_t kvh_s = __builtin_amdgcn_readfirstlane(kvh);
     auto fetch_params_g = [&](int g) {
         // (the lane number goes through an opaque copy: otherwise plane pointer + lane offset is kept
@@ -328,14 +364,22 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
             g_ms[g] = *reinterpret_cast<const uint32_t*>(at(a.k_ms, 2 * ch));
             g_mc[g] = *reinterpret_cast<const uint32_t*>(at(a.k_mc, 2 * ch));
         }
-        if constexpr (IDX == 0) {
+        if constexpr (KMAX == 10) {
+            const uint32_t* ixp = reinterpret_cast<const uint32_t*>(at(a.k_obmp, 9 * gidx + ((18 * lane_b) & ~3u)));
+#pragma unroll
+            for (int i = 0; i < 5; ++i) g_ix10[i] = ixp[i];
+            const uint32_t* ovp = reinterpret_cast<const uint32_t*>(at(a.k_oval, 5 * gidx + ((10 * lane_b) & ~3u)));
+#pragma unroll
+            for (int i = 0; i < 3; ++i) g_ov10[i] = ovp[i];
+        } else if constexpr (IDX == 0) {
             g_bm[g] = *reinterpret_cast<const u32x2*>(at(a.k_obmp, 4 * ch));
         } else {
             const uint32_t* ixp = reinterpret_cast<const uint32_t*>(at(a.k_obmp, 6 * ch));
             g_bm[g] = u32x2{ixp[0], ixp[1]};
             g_bx[g] = ixp[2];
         }
-        if constexpr (!GEN) {
+        if constexpr (KMAX == 10) {
+        } else if constexpr (!GEN) {
             // 3 nibble bytes per channel: the two dwords that hold the pair's six bytes
             const uint32_t* ovp = reinterpret_cast<const uint32_t*>(at(a.k_oval, 3 * gidx + 4 * ((3 * lane_b) / 2)));
             g_ov[g] = u32x2{ovp[0], ovp[1]};
@@ -366,7 +410,7 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
 #pragma unroll
             for (int rr = 0; rr < 4; ++rr) {
                 const int cl = 16 * (ks >> 1) + 4 * (ks & 1) + rr;
-                const float qs = static_cast<float>(1 << (10 - 2 * k_pos(4 * (ks & 1) + rr))) * q_mul;
+                const float qs = static_cast<float>(1 << (10 - 2 * k_pos<LONG>(4 * (ks & 1) + rr))) * q_mul;
                 aq[ks][rr] = pack_f16x2(qs * q_at(cl), qs * q_at(cl + 8));
             }
         }
@@ -381,8 +425,8 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
     auto first_fetch = [&]() {
         // in the order the first step needs them: K rows, the group parameters, then V
         fetch_k();
-        fetch_params_g(0);
-        fetch_params_g(1);
+#pragma unroll
+        for (int g = 0; g < NG; ++g) fetch_params_g(g);
         fetch_v();
         fetch_tables(n_begin + 64);
         asm volatile("" ::: "memory");
@@ -418,8 +462,8 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
     // halfword slot of channel c0 in the pair-ordered arrays; channel c0 + 1 sits two slots on
     const uint32_t hw0 = ((c0 >> 4) * 8u + (y0 & 7u)) * 2u + (y0 >> 3);
     // 2^-(10-2m) of the two channels: what their zero points and tile entries are scaled by
-    const float cs0 = 1.0f / static_cast<float>(1 << (10 - 2 * k_pos(int(y0 & 7u))));
-    const float cs1 = 1.0f / static_cast<float>(1 << (10 - 2 * k_pos(int((y0 + 1u) & 7u))));
+    const float cs0 = 1.0f / static_cast<float>(1 << (10 - 2 * k_pos<LONG>(int(y0 & 7u))));
+    const float cs1 = 1.0f / static_cast<float>(1 << (10 - 2 * k_pos<LONG>(int((y0 + 1u) & 7u))));
     // per channel: the |tile entry| from which its f16 rounding matters (infinite for q = 0)
     float big_thr[2];
 #pragma unroll
@@ -455,7 +499,7 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
             typedef short s16x2e __attribute__((ext_vector_type(2)));
             const s16x2e top2 = __builtin_elementwise_max(
                 __builtin_bit_cast(s16x2e, __builtin_amdgcn_perm(0u, g_sc[0], 0x010C000Cu)),
-                __builtin_bit_cast(s16x2e, __builtin_amdgcn_perm(0u, g_sc[1], 0x010C000Cu)));
+                __builtin_bit_cast(s16x2e, __builtin_amdgcn_perm(0u, g_sc[NG - 1], 0x010C000Cu)));
             const short e_top = top2[0] > top2[1] ? top2[0] : top2[1];
             // (a scaled-down query means operands near the top of f16: the same cancellation, the same remedy)
             exact_step = __any(e_top >= EXACT_STEP_EXP * 256) != 0 || q_down != 0;
@@ -470,7 +514,7 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
             uint16_t* mg = reinterpret_cast<uint16_t*>(sm + OFF_MAG) + hw0;
             uint16_t* zp = reinterpret_cast<uint16_t*>(sm + OFF_ZPP) + hw0;
 #pragma unroll
-            for (int g = 0; g < 2; ++g) {
+            for (int g = 0; g < NG; ++g) {
                 // f16 2^e of both channels: (e + 15) << 10 per half, e a signed byte held at -15 or
                 // above (a step below 2^-14 is immaterial next to the f16 operands of the others)
                 const uint32_t e2 = __builtin_amdgcn_perm(0u, g_sc[g], 0x010C000Cu);       // (e1 << 8, e0 << 8)
@@ -502,7 +546,38 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
             if (g == 1 && !g1_live) break;
+            const int pg = LONG ? 0 : g;           // the group's parameter set
             float* lc = reinterpret_cast<float*>(sm + OFF_LC);
+            // (both halves of a step read the same group here: without these copies the compiler would carry what the
+            // halves have in common, positions and levels, in registers that are not there)
+            if constexpr (LONG) {
+                if (g == 1) {
+                    asm volatile("" : "+v"(g_sc[0]), "+v"(g_zp[0]), "+v"(g_ms[0]), "+v"(g_mc[0]));
+                    if constexpr (KMAX == 10) {
+#pragma unroll
+                        for (int i = 0; i < 5; ++i) asm volatile("" : "+v"(g_ix10[i]));
+#pragma unroll
+                        for (int i = 0; i < 3; ++i) asm volatile("" : "+v"(g_ov10[i]));
+                    } else {
+                        asm volatile("" : "+v"(g_bm[0]), "+v"(g_ov[0]), "+v"(g_bx[0]));
+                    }
+                }
+            }
+            // LONG: what flips the upper bits of every 7-bit position so that those of this half's tokens read below 32
+            uint32_t flip[3] = {0, 0, 0};
+            if constexpr (LONG) {
+                const uint32_t piece = (static_cast<uint32_t>(n0 >> 5) + g) & ((1u << GTS) - 1);      // uniform
+                // ones at bits 5, 12, 19, ... (bit 0 of a piece number) and 6, 13, 20, ... (bit 1)
+#pragma unroll
+                for (int i = 0; i < 3; ++i) {
+                    uint32_t one = 0, two = 0;
+                    for (int s7 = 0; s7 < KMAX; ++s7) {
+                        if ((7 * s7 + 5) >> 5 == i) one |= 1u << ((7 * s7 + 5) & 31);
+                        if ((7 * s7 + 6) >> 5 == i) two |= 1u << ((7 * s7 + 6) & 31);
+                    }
+                    flip[i] = ((piece & 1u) ? one : 0u) ^ ((piece & 2u) ? two : 0u);
+                }
+            }
             // The channel pass of a group in two halves, so that the code bytes of both channels are on their
             // way before either channel's entries need them: positions and code reads, then entries and scatter.
             // The base MFMA takes every position of the K rows as it is stored; the tile entry of an
@@ -512,16 +587,34 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
             auto walk_read = [&](auto U, int (&pos)[KMAX], uint32_t (&cb)[KMAX]) {
                 constexpr int u = decltype(U)::value;
                 uint32_t bm = 0, ix_lo = 0, ix_hi = 0;
-                if constexpr (IDX == 0) {
-                    bm = g_bm[g][u];
+                uint32_t ixw[3] = {0, 0, 0};             // 10 outliers: the channel's 70 index bits
+                if constexpr (KMAX == 10) {
+                    // the lane's bytes start 0 or 2 bytes into the loaded dwords; channel 1's stream 9 bytes on
+                    const uint32_t sh = ((lane & 1) ? 16u : 0u) + (u ? 8u : 0u);
+#pragma unroll
+                    for (int i = 0; i < 3; ++i)
+                        ixw[i] = (i == 2 && u) ? g_ix10[4] >> sh : __builtin_amdgcn_alignbit(g_ix10[i + 1 + 2 * u], g_ix10[i + 2 * u], sh);
+#pragma unroll
+                    for (int i = 0; i < 3; ++i) ixw[i] ^= flip[i];
+                } else if constexpr (IDX == 0) {
+                    bm = g_bm[pg][u];
                 } else {
-                    ix_lo = u ? __builtin_amdgcn_alignbit(g_bx[g], g_bm[g][1], 16) : g_bm[g][0];
-                    ix_hi = u ? (g_bx[g] >> 16) : g_bm[g][1];
+                    ix_lo = u ? __builtin_amdgcn_alignbit(g_bx[pg], g_bm[pg][1], 16) : g_bm[pg][0];
+                    ix_hi = u ? (g_bx[pg] >> 16) : g_bm[pg][1];
+                    if constexpr (LONG) { ix_lo ^= flip[0]; ix_hi ^= flip[1]; }
                 }
                 const uint8_t* kt = sm + kt_lane + g * 32 * KT_ROW;
 #pragma unroll
                 for (int sidx = 0; sidx < KMAX; ++sidx) {
-                    if constexpr (IDX == 0) {
+                    if constexpr (LONG) {
+                        // (the position with the half's own bits flipped to zero: below 32 when it lies here)
+                        constexpr uint32_t PM = (1u << GT_SH) - 1;
+                        const int bit = 7 * sidx, wi = bit >> 5, bo = bit & 31;
+                        const uint32_t lo = KMAX == 10 ? ixw[wi] : (wi ? ix_hi : ix_lo);
+                        const uint32_t hi = KMAX == 10 ? ixw[wi < 2 ? wi + 1 : 2] : ix_hi;
+                        const uint32_t f = (bo + GT_SH <= 32 ? (lo >> bo) : __builtin_amdgcn_alignbit(hi, lo, bo)) & PM;
+                        pos[sidx] = static_cast<int>(min(f, 32u));
+                    } else if constexpr (IDX == 0) {
                         pos[sidx] = __builtin_ctz(bm) & 31;
                         if (sidx < KMAX - 1) bm &= bm - 1;
                     } else {
@@ -534,8 +627,8 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
             };
             auto walk_write = [&](auto U, const int (&pos)[KMAX], const uint32_t (&cb)[KMAX], float (&dls)[KMAX]) {
                 constexpr int u = decltype(U)::value;
-                const float zp = __uint_as_float(u ? (g_zp[g] & 0xFFFF0000u) : (g_zp[g] << 16));
-                const int e = static_cast<int8_t>((g_sc[g] >> (8 * u)) & 0xFFu);
+                const float zp = __uint_as_float(u ? (g_zp[pg] & 0xFFFF0000u) : (g_zp[pg] << 16));
+                const int e = static_cast<int8_t>((g_sc[pg] >> (8 * u)) & 0xFFu);
                 const float s = __uint_as_float(static_cast<uint32_t>(e + 127) << 23);
                 // everything below is in units of the channel's A scale: tile entry =
                 // (outlier - zp - code * 2^e) / 2^(10-2m) = level * a1 + b1 (less 3 * sc for code 3)
@@ -543,22 +636,38 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
                 const float sc = s * cs;
                 float a1, b1;
                 if (OWN_MAP) {
-                    const float ms = __uint_as_float(u ? (g_ms[g] & 0xFFFF0000u) : (g_ms[g] << 16));
-                    const float mc = __uint_as_float(u ? (g_mc[g] & 0xFFFF0000u) : (g_mc[g] << 16));
+                    const float ms = __uint_as_float(u ? (g_ms[pg] & 0xFFFF0000u) : (g_ms[pg] << 16));
+                    const float mc = __uint_as_float(u ? (g_mc[pg] & 0xFFFF0000u) : (g_mc[pg] << 16));
                     a1 = cs * __builtin_amdgcn_rcpf(ms);
                     b1 = cs * (mc - zp);
                 } else {
                     a1 = sc;
                     b1 = 0.0f;
                 }
-                const uint64_t ov64 = (static_cast<uint64_t>(g_ov[g][1]) << 32) | g_ov[g][0];
+                float lv[KMAX < 8 ? 8 : KMAX];
+                if constexpr (KMAX == 10) {
+                    // the lane's bytes start 0 or 2 bytes into the loaded dwords; channel u: bytes 5u .. 5u+4
+                    const uint32_t sh = ((lane & 1) ? 16u : 0u) + (u ? 8u : 0u);
+                    const uint32_t o0 = __builtin_amdgcn_alignbit(g_ov10[1 + u], g_ov10[u], sh);
+                    const uint32_t o1 = u ? g_ov10[2] >> sh : __builtin_amdgcn_alignbit(g_ov10[2], g_ov10[1], sh);
+                    const f32x2 l01 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(o0, 1.0f, 0);
+                    const f32x2 l23 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(o0, 1.0f, 1);
+                    const f32x2 l45 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(o0, 1.0f, 2);
+                    const f32x2 l67 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(o0, 1.0f, 3);
+                    const f32x2 l89 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(o1, 1.0f, 0);
+                    lv[0] = l01[0]; lv[1] = l01[1]; lv[2] = l23[0]; lv[3] = l23[1]; lv[4] = l45[0]; lv[5] = l45[1];
+                    lv[6] = l67[0]; lv[7] = l67[1]; lv[8] = l89[0]; lv[9] = l89[1];
+                } else {
+                const uint64_t ov64 = (static_cast<uint64_t>(g_ov[pg][1]) << 32) | g_ov[pg][0];
                 const uint32_t nib = GEN ? static_cast<uint32_t>(ov64 >> (nib_sh + 8 * kbytes * u))
                                          : static_cast<uint32_t>(ov64 >> (nib_sh + 24 * u)) & 0xFFFFFFu;
                 const f32x2 l01 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(nib, 1.0f, 0);
                 const f32x2 l23 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(nib, 1.0f, 1);
                 const f32x2 l45 = KMAX > 4 ? __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(nib, 1.0f, 2) : f32x2{0.0f, 0.0f};
                 const f32x2 l67 = KMAX > 6 ? __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(nib, 1.0f, 3) : f32x2{0.0f, 0.0f};
-                const float lv[8] = {l01[0], l01[1], l23[0], l23[1], l45[0], l45[1], l67[0], l67[1]};
+                lv[0] = l01[0]; lv[1] = l01[1]; lv[2] = l23[0]; lv[3] = l23[1]; lv[4] = l45[0]; lv[5] = l45[1];
+                lv[6] = l67[0]; lv[7] = l67[1];
+                }
                 uint16_t* dt = reinterpret_cast<uint16_t*>(sm + OFF_TILE) + hw0 + 2 * u;      // pair order, like MAG
                 float dl_max = 0.0f;
 #pragma unroll
@@ -585,7 +694,7 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
                 for (int sidx = 0; sidx < KMAX; ++sidx) {
                     if (GEN && sidx >= kout) continue;
                     const float dl = dls[sidx];
-                    if (fabsf(dl) >= big_thr[u]) {
+                    if (fabsf(dl) >= big_thr[u] && (!LONG || pos[sidx] < 32)) {
                         const float lo = (dl - static_cast<float>(static_cast<_Float16>(dl))) * un;
 #pragma unroll
                         for (int r = 0; r < NH; ++r)
@@ -597,19 +706,33 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
             int pos0[KMAX], pos1[KMAX];
             uint32_t cb0[KMAX], cb1[KMAX];
             float dls0[KMAX], dls1[KMAX];
-            // (the general form has fewer registers to spare: one channel after the other there)
+            // (the general form and longer groups have fewer registers to spare: one channel after the other there)
+            constexpr bool ONE_BY_ONE = GEN || LONG;
             walk_read(std::integral_constant<int, 0>{}, pos0, cb0);
-            if constexpr (!GEN) walk_read(std::integral_constant<int, 1>{}, pos1, cb1);
+            if constexpr (!ONE_BY_ONE) walk_read(std::integral_constant<int, 1>{}, pos1, cb1);
             const float dlm0 = walk_write(std::integral_constant<int, 0>{}, pos0, cb0, dls0);
-            if constexpr (GEN) walk_read(std::integral_constant<int, 1>{}, pos1, cb1);
+            // (longer groups: the first channel's residuals before the second's walk, whose entries take its registers)
+            constexpr bool SOON = LONG;
+            bool res_any = false;
+            if constexpr (SOON) {
+                res_any = __any(dlm0 >= big_thr[0]) != 0;
+                if (res_any) residuals(std::integral_constant<int, 0>{}, pos0, dls0);
+            }
+            if constexpr (ONE_BY_ONE) walk_read(std::integral_constant<int, 1>{}, pos1, cb1);
             const float dlm1 = walk_write(std::integral_constant<int, 1>{}, pos1, cb1, dls1);
-            const bool res_any = __any(dlm0 >= big_thr[0] || dlm1 >= big_thr[1]) != 0;
-            if (__builtin_expect(res_any, 0)) {
-                residuals(std::integral_constant<int, 0>{}, pos0, dls0);
-                residuals(std::integral_constant<int, 1>{}, pos1, dls1);
+            if constexpr (SOON) {
+                const bool res1 = __any(dlm1 >= big_thr[1]) != 0;
+                if (res1) residuals(std::integral_constant<int, 1>{}, pos1, dls1);
+                res_any |= res1;
+            } else {
+                res_any = __any(dlm0 >= big_thr[0] || dlm1 >= big_thr[1]) != 0;
+                if (__builtin_expect(res_any, 0)) {
+                    residuals(std::integral_constant<int, 0>{}, pos0, dls0);
+                    residuals(std::integral_constant<int, 1>{}, pos1, dls1);
+                }
             }
             lds_fence();
-            if (more) fetch_params_g(g);
+            if (more && (!LONG || g == 1)) fetch_params_g(pg);
             // both 16-token blocks of the group go through the eight k-steps together (two independent
             // accumulation chains): tile rows (read, clear), then the base codes
             f32x4 d[2] = {f32x4{0, 0, 0, 0}, f32x4{0, 0, 0, 0}};
@@ -627,7 +750,7 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
                     d[t2] = mfma_f16(aq[ks], bt, d[t2]);
                 }
             }
-            const u32x4* mg = reinterpret_cast<const u32x4*>(sm + OFF_MAG + g * 256 + kq * 64);
+            const u32x4* mg = reinterpret_cast<const u32x4*>(sm + OFF_MAG + pg * 256 + kq * 64);
             auto base_mfmas = [&](auto EX) {
                 // EX: the operand without its constant, code * 2^(2m-10+e) = pattern - 2^e
                 auto op = [&](uint32_t pat, uint32_t mag) {
@@ -638,23 +761,25 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
                 for (int hf = 0; hf < 2; ++hf) {          // code dword: channels 16*hf .. 16*hf+15 of the quarter
                     uint32_t w[2], wu[2], wd[2];
 #pragma unroll
-                    for (int t2 = 0; t2 < 2; ++t2) { w[t2] = kw[t2][hf]; wu[t2] = w[t2] << 2; wd[t2] = w[t2] >> 6; }
+                    for (int t2 = 0; t2 < 2; ++t2) { w[t2] = kw[t2][hf]; wu[t2] = w[t2] << (LONG ? 6 : 4); wd[t2] = w[t2] >> 6; }
                     const u32x4 ma = mg[2 * hf], mb = mg[2 * hf + 1];
 #pragma unroll
                     for (int t2 = 0; t2 < 2; ++t2)
-                        d[t2] = mfma_f16(aq[2 * hf], u32x4{op(k_pair<0>(w[t2], wu[t2], wd[t2], ma[0]), ma[0]), op(k_pair<1>(w[t2], wu[t2], wd[t2], ma[1]), ma[1]),
-                                                           op(k_pair<2>(w[t2], wu[t2], wd[t2], ma[2]), ma[2]), op(k_pair<3>(w[t2], wu[t2], wd[t2], ma[3]), ma[3])}, d[t2]);
+                        d[t2] = mfma_f16(aq[2 * hf], u32x4{op(k_pair<0, LONG>(w[t2], wu[t2], wd[t2], ma[0]), ma[0]), op(k_pair<1, LONG>(w[t2], wu[t2], wd[t2], ma[1]), ma[1]),
+                                                           op(k_pair<2, LONG>(w[t2], wu[t2], wd[t2], ma[2]), ma[2]), op(k_pair<3, LONG>(w[t2], wu[t2], wd[t2], ma[3]), ma[3])}, d[t2]);
 #pragma unroll
                     for (int t2 = 0; t2 < 2; ++t2)
-                        d[t2] = mfma_f16(aq[2 * hf + 1], u32x4{op(k_pair<4>(w[t2], wu[t2], wd[t2], mb[0]), mb[0]), op(k_pair<5>(w[t2], wu[t2], wd[t2], mb[1]), mb[1]),
-                                                               op(k_pair<6>(w[t2], wu[t2], wd[t2], mb[2]), mb[2]), op(k_pair<7>(w[t2], wu[t2], wd[t2], mb[3]), mb[3])}, d[t2]);
+                        d[t2] = mfma_f16(aq[2 * hf + 1], u32x4{op(k_pair<4, LONG>(w[t2], wu[t2], wd[t2], mb[0]), mb[0]), op(k_pair<5, LONG>(w[t2], wu[t2], wd[t2], mb[1]), mb[1]),
+                                                               op(k_pair<6, LONG>(w[t2], wu[t2], wd[t2], mb[2]), mb[2]), op(k_pair<7, LONG>(w[t2], wu[t2], wd[t2], mb[3]), mb[3])}, d[t2]);
                 }
             };
             if (__builtin_expect(exact_step, 0)) {
                 base_mfmas(std::true_type{});
                 // the bias MFMA must not take the constant out a second time: its 2^e column of this group reads zeros
-                lds_fence();
-                reinterpret_cast<uint32_t*>(sm + OFF_MAG + g * 256)[lane] = 0u;
+                if (!LONG || g == 1 || !g1_live) {
+                    lds_fence();
+                    reinterpret_cast<uint32_t*>(sm + OFF_MAG + pg * 256)[lane] = 0u;
+                }
             } else {
                 base_mfmas(std::false_type{});
             }
@@ -683,7 +808,7 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
         // bias columns: 0 zp(g0) 1 zp(g1) 2 2^e(g0) 3 2^e(g1); other columns repeat them
         f32x4 dbias = {0, 0, 0, 0};
         {
-            const int src = ((j & 2) ? OFF_MAG : OFF_ZPP) + (j & 1) * 256 + kq * 64;
+            const int src = ((j & 2) ? OFF_MAG : OFF_ZPP) + (LONG ? 0 : (j & 1) * 256) + kq * 64;
             const u32x4* bp = reinterpret_cast<const u32x4*>(sm + src);
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) dbias = mfma_f16(aq[ks], bp[ks], dbias);
@@ -698,6 +823,14 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
             for (int c = 0; c < 8; ++c) vt[c * VT_COL] = vr[c >> 2][c & 3];
             typedef short s16x2 __attribute__((ext_vector_type(2)));
             typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+            if (LONG && vv_sh == 1) {
+                vsc = __builtin_amdgcn_perm(0u, vsc, 0x01010000u);
+                vzp = u32x2{__builtin_amdgcn_perm(0u, vzp[0], 0x01000100u), __builtin_amdgcn_perm(0u, vzp[0], 0x03020302u)};
+            } else if (LONG && vv_sh == 0) {
+                vsc = __builtin_amdgcn_perm(0u, vsc, 0x00000000u);
+                vzp[0] = __builtin_amdgcn_perm(0u, vzp[0], 0x01000100u);
+                vzp[1] = vzp[0];
+            }
             // a V step above 2^MAX_STEP_EXP (a signed exponent byte of 16 or more) is held there and reported
             if (__builtin_expect(__any((((vsc & 0x7F7F7F7Fu) + 0x70707070u) & ~vsc & 0x80808080u) != 0u) != 0, 0)) over_step = true;
             uint16_t* vs16 = reinterpret_cast<uint16_t*>(sm + OFF_VS) + lane;
@@ -778,13 +911,11 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
                 for (int i = 0; i < 4; ++i) { acc[0][i] *= al; acc[1][i] *= al; accz[i] *= al; }
             }
             {
-                const uint32_t p01 = pack_f16x2(__builtin_amdgcn_exp2f(pe[0]), __builtin_amdgcn_exp2f(pe[1]));
-                const uint32_t p23 = pack_f16x2(__builtin_amdgcn_exp2f(pe[2]), __builtin_amdgcn_exp2f(pe[3]));
-                uint16_t* pt = reinterpret_cast<uint16_t*>(sm + OFF_PT) + lane;
-                pt[0] = static_cast<uint16_t>(p01);
-                pt[PT_ROW] = static_cast<uint16_t>(p01 >> 16);
-                pt[2 * PT_ROW] = static_cast<uint16_t>(p23);
-                pt[3 * PT_ROW] = static_cast<uint16_t>(p23 >> 16);
+                // (to the nearest f16: the pairwise conversion cuts off, which costs half an instruction less a
+                // weight and shifts every lse by -2.4e-4 and with it the share of the bf16 tail)
+                _Float16* pt = reinterpret_cast<_Float16*>(sm + OFF_PT) + lane;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) pt[r * PT_ROW] = static_cast<_Float16>(__builtin_amdgcn_exp2f(pe[r]));
             }
         } else {
             // the lane owns tokens n0 + 32g + 16(kq >> 1) + j, g = 0, 1, and heads 4(kq & 1)..+3.  Every quad
@@ -861,16 +992,12 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
                 }
             }
             {
-                uint16_t* pt = reinterpret_cast<uint16_t*>(sm + OFF_PT) + 4 * (kq & 1) * PT_ROW + tk;
+                _Float16* pt = reinterpret_cast<_Float16*>(sm + OFF_PT) + 4 * (kq & 1) * PT_ROW + tk;
 #pragma unroll
-                for (int g = 0; g < 2; ++g) {
-                    const uint32_t p01 = pack_f16x2(__builtin_amdgcn_exp2f(pe[g][0]), __builtin_amdgcn_exp2f(pe[g][1]));
-                    const uint32_t p23 = pack_f16x2(__builtin_amdgcn_exp2f(pe[g][2]), __builtin_amdgcn_exp2f(pe[g][3]));
-                    pt[32 * g] = static_cast<uint16_t>(p01);
-                    pt[32 * g + PT_ROW] = static_cast<uint16_t>(p01 >> 16);
-                    pt[32 * g + 2 * PT_ROW] = static_cast<uint16_t>(p23);
-                    pt[32 * g + 3 * PT_ROW] = static_cast<uint16_t>(p23 >> 16);
-                }
+                for (int g = 0; g < 2; ++g)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        pt[32 * g + r * PT_ROW] = static_cast<_Float16>(__builtin_amdgcn_exp2f(pe[g][r]));
             }
         }
         lds_fence();
@@ -984,7 +1111,16 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
 int launch_decode_gqa4(const DecodeArgs& a_in, int Dh, int R, hipStream_t st) {
     DecodeArgs a = a_in;
     a.half = 0;
-    if (a.scale_bf16 || a.v_bf16 || a.gt != 32 || a.gc != 32 || a.kout < 1 || a.kout > 8) return 1;
+    if (a.scale_bf16 || a.v_bf16) return 1;
+    // K groups of 64 / 128 tokens with position streams: 6 outliers, or 10 of 128; V vectors of 32, 64 or 128 channels
+    const bool longer = a.gt == 64 || a.gt == 128;
+    if (longer) {
+        if (a.idx_repr != 1 || !(a.kout == 6 || (a.kout == 10 && a.gt == 128)) || Dh != 128 || !(R == 4 || R == 8) ||
+            !(a.gc == 32 || a.gc == 64 || a.gc == 128))
+            return 1;
+    } else if (a.gt != 32 || a.gc != 32 || a.kout < 1 || a.kout > 8) {
+        return 1;
+    }
     if ((reinterpret_cast<uintptr_t>(a.q) & 3) || (a.q_sb & 1) || (a.q_sh & 1)) return 1;
     int nh;                                   // q heads of a wave's (pair of) kv head(s)
     if (Dh == 128 && (R == 1 || R == 2 || R == 4 || R == 8)) {
@@ -998,21 +1134,22 @@ int launch_decode_gqa4(const DecodeArgs& a_in, int Dh, int R, hipStream_t st) {
     }
     {
         // the kernel addresses a plane by 32-bit byte offsets: it takes planes whose extents are given and
-        // below 4 GiB (code rows: pages * page size * kv heads * 32 B; the widest group plane has 6 B per channel)
+        // below 4 GiB (code rows: pages * page size * kv heads * 32 B; the widest group plane has 9 B per channel)
         const uint64_t lim = 0xFFFFFF00ull;
         if (a.n_pages <= 0 || a.n_gslots <= 0) return 1;
         if (static_cast<uint64_t>(a.n_pages) * static_cast<uint64_t>(a.ps) >= (1ull << 24)) return 1;
         if (static_cast<uint64_t>(a.n_pages) * a.ps * a.Hkv * 32ull > lim) return 1;
-        if (static_cast<uint64_t>(a.n_gslots) * a.Hkv * D * 6ull > lim) return 1;
+        if (static_cast<uint64_t>(a.n_gslots) * a.Hkv * D * (longer ? 9ull : 6ull) > lim) return 1;
     }
-    const bool general = a.half || a.kout != 6;
+    const bool general = a.half || (a.kout != 6 && !longer);
     if (general && a.idx_repr != 0) return 1;       // the general form reads bitmaps only
     const int waves = (a.Hkv % 4 == 0) ? 4 : ((a.Hkv % 2 == 0) ? 2 : 1);
     // shares: the orders below hold up to 64 requests (one per lane), or 256 (four)
-    if (a.shares > 0 && a.B > (nh < 4 && !general ? 64 : 256)) return 1;
+    if (a.shares > 0 && a.B > (longer || (nh < 4 && !general) ? 64 : 256)) return 1;
     const dim3 grid = a.shares > 0 ? dim3(a.Hkv / waves, a.shares) : dim3(a.S, a.Hkv / waves, a.B);
     const dim3 block(64 * waves);
-    const size_t shm = (size_t)waves * (nh == 8 ? LdsMap<8>::LDS_WAVE : LdsMap<4>::LDS_WAVE);
+    const size_t shm = (size_t)waves * (longer ? (nh == 8 ? LdsMap<8, true>::LDS_WAVE : LdsMap<4, true>::LDS_WAVE)
+                                              : (nh == 8 ? LdsMap<8, false>::LDS_WAVE : LdsMap<4, false>::LDS_WAVE));
     const bool own_map = a.k_ms != nullptr;
     const int order = a.B == 1 ? 0 : (a.B > 64 && a.B <= 256 ? 2 : 1);
 #define OMMX_GO(IDX, MAP, PART, ORD, NH, GEN) \
@@ -1029,6 +1166,28 @@ int launch_decode_gqa4(const DecodeArgs& a_in, int Dh, int R, hipStream_t st) {
         else if (order == 2) OMMX_GO(IDX, MAP, PART, 2, NH, false);  \
         else OMMX_GO(IDX, MAP, PART, 1, NH, false);                  \
     } while (0)
+#define OMMX_GO_LONG(MAP, NH, KO, GTS)                                                                                         \
+    do {                                                                                                                       \
+        if (order == 0) hipLaunchKernelGGL((decode_gqa4_kernel<1, MAP, false, 0, NH, false, KO, GTS>), grid, block, shm, st, a); \
+        else hipLaunchKernelGGL((decode_gqa4_kernel<1, MAP, false, 1, NH, false, KO, GTS>), grid, block, shm, st, a);            \
+    } while (0)
+    if (longer) {
+        switch ((nh == 8 ? 8 : 0) | (own_map ? 4 : 0) | (a.gt == 64 ? 0 : a.kout == 6 ? 1 : 2)) {
+            case 0: OMMX_GO_LONG(false, 4, 6, 1); break;
+            case 1: OMMX_GO_LONG(false, 4, 6, 2); break;
+            case 2: OMMX_GO_LONG(false, 4, 10, 2); break;
+            case 4: OMMX_GO_LONG(true, 4, 6, 1); break;
+            case 5: OMMX_GO_LONG(true, 4, 6, 2); break;
+            case 6: OMMX_GO_LONG(true, 4, 10, 2); break;
+            case 8: OMMX_GO_LONG(false, 8, 6, 1); break;
+            case 9: OMMX_GO_LONG(false, 8, 6, 2); break;
+            case 10: OMMX_GO_LONG(false, 8, 10, 2); break;
+            case 12: OMMX_GO_LONG(true, 8, 6, 1); break;
+            case 13: OMMX_GO_LONG(true, 8, 6, 2); break;
+            default: OMMX_GO_LONG(true, 8, 10, 2); break;
+        }
+        return 0;
+    }
     if (general) {
         // one instantiation per (outlier map, head layout): outlier count, head count and head_dim at run time
         if (nh == 8) { if (own_map) OMMX_GO_GEN(true, false, 8); else OMMX_GO_GEN(false, false, 8); }
@@ -1051,6 +1210,7 @@ int launch_decode_gqa4(const DecodeArgs& a_in, int Dh, int R, hipStream_t st) {
     }
 #undef OMMX_GO
 #undef OMMX_GO_GEN
+#undef OMMX_GO_LONG
 #undef OMMX_GO_ORD
     return 0;
 }

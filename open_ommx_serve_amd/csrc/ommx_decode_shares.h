@@ -48,8 +48,9 @@ struct Share {
 
 // Clocks a wave spends on g groups (a step is two; a lone group costs 0.7 of one, the start-up about one),
 // next to one other wave on its SIMD and next to two: 11 700 and 15 900 a step, here in hundreds.
+template <int GT>
 __device__ __forceinline__ uint32_t wave_cost(uint32_t g, bool third) {
-    return ((g >> 1) * 10u + (g & 1u) * 7u + 10u) * (third ? 159u : 117u);
+    return ((GT == 32 ? (g >> 1) * 10u + (g & 1u) * 7u : g * 10u) + 10u) * (third ? 159u : 117u);
 }
 
 // The share `f` of the batch; false when the batch has fewer.  GT: tokens per group, PER_LANE: requests per lane
@@ -103,7 +104,7 @@ __device__ __forceinline__ bool find_share(const DecodeArgs& a, uint32_t f, int 
     uint32_t g = smallest(a.shares_few, g0);
     if (a.shares > a.shares_few && g > g0) {
         const uint32_t g3 = smallest(a.shares, g0);
-        if (wave_cost(g3, true) < wave_cost(g, false)) g = g3;
+        if (wave_cost<GT>(g3, true) < wave_cost<GT>(g, false)) g = g3;
         else deal(g);
     }
     if (f >= lane_top(incl[PER_LANE - 1])) return false;

@@ -286,9 +286,16 @@ int run_decode(const DecodeCall& c) {
     // The serving-recipe kernel keeps three workgroups per compute unit resident with up to 4 q heads per
     // kv head (two with 8, and so do the other kernels); at head_dim 64 one of its waves takes a pair of kv heads.
     const bool plain_planes = gt == 32 && gc == 32 && !scale_bf16 && !v_bf16 && !c.force;
-    const bool lean = plain_planes && ((D == 128 && R <= 4 && k == 6) ||
-                                       (c.bitmap && k >= 1 && k <= 6 && ((D == 128 && R <= 4) ||
-                                                                         (D == 64 && R <= 2 && Hkv % 2 == 0))));
+    // K groups of 64 / 128 tokens: the same kernel takes them in pieces of 64 tokens (the plane extents that it
+    // addresses are looked at again at the launch; were they too large, the other kernels would serve pieces of groups
+    // with the same numbers).
+    const bool pieces = gt >= 64 && !scale_bf16 && !v_bf16 && !c.force && D == 128 && R >= 4 && gc >= 32 && !c.bitmap &&
+                        (k == 6 || (k == 10 && gt == 128));
+    const int64_t unit = pieces ? 64 : gt;                       // tokens that a share is made of
+    const bool lean = (pieces && R == 4) ||
+                      (plain_planes && ((D == 128 && R <= 4 && k == 6) ||
+                                        (c.bitmap && k >= 1 && k <= 6 && ((D == 128 && R <= 4) ||
+                                                                          (D == 64 && R <= 2 && Hkv % 2 == 0)))));
     const bool paired = plain_planes && D == 64 && c.bitmap && k >= 1 && k <= 8 && R <= 4 && Hkv % 2 == 0;
     const int64_t wave_heads = paired ? Hkv / 2 : Hkv;           // waves that one share of the tokens takes
 
@@ -332,7 +339,7 @@ int run_decode(const DecodeCall& c) {
         // more than four times its even part, which bounds the workspace.
         const int64_t fit = cu_count(dev.index()) * 4 / wave_heads;
         // (max_seq bounds how many groups there can be; were it too small, the shares would be longer, nothing else)
-        const int64_t longest = std::max<int64_t>(1, (c.max_seq + gt - 1) / gt);
+        const int64_t longest = std::max<int64_t>(1, (c.max_seq + unit - 1) / unit);
         const int64_t shares = std::min({int64_t{2048}, fit * (lean ? 3 : 2), B * longest}), few = std::min(shares, fit * 2);
         const int64_t most = std::min({int64_t{B * Hq >= 256 ? 64 : (shares > 256 * B && longest > 512 ? 512 : 256)}, longest,
                                        std::max<int64_t>(8, 4 * shares / B)});
@@ -354,7 +361,7 @@ int run_decode(const DecodeCall& c) {
     }
     if (rc == 1) {
         int64_t S = c.splits;
-        if (S == 0) S = auto_splits(c.max_seq, B, wave_heads, cu_count(dev.index()), gt, c.mean, lean ? 3 : 2);
+        if (S == 0) S = auto_splits(c.max_seq, B, wave_heads, cu_count(dev.index()), unit, c.mean, lean ? 3 : 2);
         if (c.ws && (c.ws->scalar_type() != at::kFloat || c.ws->dim() != 4 || c.ws->size(0) != B || c.ws->size(1) != Hq ||
                      c.ws->size(2) < S || c.ws->size(3) < D + 1 || c.ws->stride(3) != 1))
             return 0;

@@ -341,6 +341,24 @@ def test_longer_groups_on_the_matrix_core_kernel(gt, gc, k, hq, own_map):
         assert (got[0] - ref[0]).abs().max().item() <= MAX_ABS
 
 
+@pytest.mark.parametrize("gt,gc,k,hq,own_map", [(64, 64, 6, 32, False), (128, 64, 6, 64, True), (128, 128, 10, 32, True),
+                                                (128, 32, 10, 64, False)])
+def test_longer_groups_cut_into_pieces(gt, gc, k, hq, own_map):
+    """The kernel takes a longer group in pieces of 64 tokens and walks the group's outliers once per 32: lengths that
+    end a piece after 1, 31, 32, 33, 63 and 64 tokens, in every quarter of a group, dealt out piece by piece, and
+    steps of 2^5 and more (the operand without its constant, once per half of a piece)."""
+    lens = [2 * gt + n for n in (1, 31, 32, 33, 63, 64, gt - 31, gt - 1, gt)]
+    for more in (dict(sparse_frac=0.005), dict(sparse_frac=0.02, sparse_gain=40.0, outlier_gain=150.0)):
+        case = build_decode_case([n + 48 for n in [3 * gt] * len(lens)], q_heads=hq, kv_heads=8, seed=83,
+                                 permute_tables=True, group_tokens=gt, group_channels=gc, outliers_per_vector=k,
+                                 outlier_repr="relidx7", kv_outlier_map=own_map, **more)
+        case.b_seq_len.copy_(torch.tensor(lens, dtype=torch.int32))
+        case.extra["packed_lens"] = lens
+        want = _oracle(case)
+        for S in (None, 1, 3 * gt // 64):
+            _check(_run(case, num_kv_splits=S), want, f"gt{gt} gc{gc} k{k} S{S}")
+
+
 def test_randomised_recipes_against_the_oracle():
     """Forty random draws over the whole recipe space the kernels accept (group sizes, outlier
     count, index plane, outlier map, step mode, V format, head shapes, table dtype, splits,
