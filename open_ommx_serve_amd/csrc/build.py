@@ -27,6 +27,7 @@ SOURCES = {
     "ommx_decode_ref.hip": [],
     "ommx_decode.hip": [],
     "ommx_decode_gqa4.hip": [],
+    "ommx_decode_gqa4_tail.hip": [],
     "ommx_combine.hip": [],
     "ommx_ring.hip": [],
     "ommx_merge.hip": [],
@@ -74,7 +75,7 @@ def _compile_host() -> str:
 
 def build(verbose: bool = True) -> str:
     from torch.utils.cpp_extension import library_paths
-    with ThreadPoolExecutor(max_workers=4) as ex:
+    with ThreadPoolExecutor(max_workers=8) as ex:
         host = ex.submit(_compile_host)
         objs = list(ex.map(lambda kv: _compile(*kv), SOURCES.items()))
         host_obj = host.result()

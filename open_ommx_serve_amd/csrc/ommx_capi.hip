@@ -13,7 +13,8 @@ static thread_local std::string g_error;
 void set_error(const char* msg) { g_error = msg; }
 
 int launch_decode_fast(const DecodeArgs& a, int D, int R, hipStream_t st);
-int launch_decode_gqa4(const DecodeArgs& a, int D, int R, hipStream_t st);
+int launch_decode_gqa4(const DecodeArgs& a, int D, int R, const DecodeTail* tail, hipStream_t st);
+int launch_decode_gqa4_tail(const DecodeArgs& a, int D, int R, const DecodeTail* tail, hipStream_t st);
 
 }  // namespace ommx
 
@@ -107,7 +108,9 @@ static void set_error2(const char* where, const char* what) { g_error = std::str
 
 }  // namespace ommx
 
-int ommx::decode_splitkv(OMMX_DECODE_PARAMS, bool plain, const StateLse* lse, const Shares* shares) {
+int ommx::decode_splitkv(OMMX_DECODE_PARAMS, bool plain, const StateLse* lse, const Shares* shares, const DecodeTail* tail,
+                         bool* tail_done) {
+    if (tail_done) *tail_done = false;
     const char* where = plain ? "ommx_decode_splitkv_ref" : "ommx_decode_splitkv";
     if (const char* bad = check_decode(OMMX_DECODE_ARGS)) { set_error2(where, bad); return -1; }
     DecodeArgs a = make_decode_args(OMMX_DECODE_ARGS);
@@ -126,7 +129,8 @@ int ommx::decode_splitkv(OMMX_DECODE_PARAMS, bool plain, const StateLse* lse, co
     hipStream_t st = static_cast<hipStream_t>(stream);
     int rc = 1;
     if (!plain) {
-        rc = launch_decode_gqa4(a, D, R, st);
+        rc = tail ? launch_decode_gqa4_tail(a, D, R, tail, st) : launch_decode_gqa4(a, D, R, nullptr, st);
+        if (rc == 0 && tail_done) *tail_done = tail != nullptr;
         if (rc == 1) rc = launch_decode_fast(a, D, R, st);
         if (rc == 1 && shares) return 1;                  // (the plain kernel knows fixed splits only)
     }
@@ -137,12 +141,12 @@ int ommx::decode_splitkv(OMMX_DECODE_PARAMS, bool plain, const StateLse* lse, co
 }
 
 extern "C" int ommx_decode_splitkv(OMMX_DECODE_PARAMS) {
-    return ommx::decode_splitkv(OMMX_DECODE_ARGS, false, nullptr, nullptr);
+    return ommx::decode_splitkv(OMMX_DECODE_ARGS, false, nullptr, nullptr, nullptr, nullptr);
 }
 
 // Same operator through the plain fp32 kernel only (cross-check entry used by tests).
 extern "C" int ommx_decode_splitkv_ref(OMMX_DECODE_PARAMS) {
-    return ommx::decode_splitkv(OMMX_DECODE_ARGS, true, nullptr, nullptr);
+    return ommx::decode_splitkv(OMMX_DECODE_ARGS, true, nullptr, nullptr, nullptr, nullptr);
 }
 
 // What the combine knows of the shares: each request's number of states, on the device, and how many an even deal gives.

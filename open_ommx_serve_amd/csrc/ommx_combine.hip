@@ -11,6 +11,8 @@
 // parts of the row).  combine_grouped_kernel (further down): one workgroup per (request, kv head)
 // for large batches, where the tail rows are most of the bytes and are read once for all the
 // q heads of the kv head.
+#include <algorithm>
+
 #include "ommx_decode_args.h"
 
 namespace ommx {
@@ -486,6 +488,128 @@ __global__ void __launch_bounds__(512) combine_grouped_kernel(CombineArgs a) {
             if (d == 0) a.lse[b * a.lse_b + h0 + r] = W > 0.0f ? n_max + __logf(W) : -INFINITY;
         }
     }
+}
+
+// The merge when the tail rows are among the states (ommx_decode_tail.h): o = sum w_i o_i / sum w_i over `slots` states
+// of every (request, q head), w_i = exp(lse_i - max).  A workgroup takes CH channels of one head, LPR lanes a state
+// (four channels each); every wave reads all the lse and works the maximum and the sum of weights out for itself, so
+// that between the one round of loads and the output lie one exchange through LDS and no other wait.
+// An unused slot has lse -inf, and what it holds is not multiplied.
+struct FoldArgs {
+    const float* al; int64_t al_b, al_h, al_s;
+    const float* sl; int64_t sl_b, sl_h, sl_s;
+    float* o; uint16_t* o16; int64_t o_b, o_h;
+    float* lse; int64_t lse_b;
+    int slots, sure;
+};
+template <int D, int Q, int NT>
+__global__ void __launch_bounds__(NT) fold_kernel(FoldArgs a) {
+    constexpr int CH = D / Q, LPR = CH / 4, ROWS = NT / LPR, NW = NT / 64;
+    constexpr int FIRST = 6;                       // states per thread of the first round of loads, upper bound
+    constexpr int NL = 9;                          // 512 splits and the tail's parts, 64 a register
+    static_assert(LPR == 16 || LPR == 32, "lane layout of the sums");
+    __shared__ float s_acc[NW][CH];
+    const int b = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int c4 = tid % LPR, row = tid / LPR;
+    const float* const base = a.al + b * a.al_b + (int64_t)h * a.al_h + blockIdx.z * CH + 4 * c4;
+    const float* const sl = a.sl + b * a.sl_b + (int64_t)h * a.sl_h;
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    const int N = a.slots;
+    const int n_first = min((a.sure + ROWS - 1) / ROWS, FIRST);
+    f32x4 v[FIRST];
+    float my[FIRST], all[NL];
+#pragma unroll
+    for (int i = 0; i < FIRST; ++i) {
+        v[i] = f32x4{0, 0, 0, 0};
+        my[i] = -INFINITY;
+        if (i < n_first) {
+            const int s = min(row + ROWS * i, N - 1);
+            v[i] = *reinterpret_cast<const f32x4*>(base + (int64_t)s * a.al_s);
+            my[i] = sl[(int64_t)s * a.sl_s];
+        }
+    }
+    float top = -INFINITY;
+#pragma unroll
+    for (int k = 0; k < NL; ++k) {
+        all[k] = -INFINITY;
+        if (64 * k < N) {
+            all[k] = sl[(int64_t)min(64 * k + lane, N - 1) * a.sl_s];
+            if (64 * k + lane >= N) all[k] = -INFINITY;
+        }
+        top = fmaxf(top, all[k]);
+    }
+    top = wave64_max(top);
+    const float safe = top == -INFINITY ? 0.0f : top;
+    f32x4 acc = {0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < FIRST; ++i) {
+        if (i < n_first) {
+            const float w = my[i] == -INFINITY || row + ROWS * i >= N ? 0.0f : __expf(my[i] - safe);
+            if (w > 0.0f) acc += w * v[i];
+        }
+    }
+    for (int s = row + ROWS * n_first; s < N; s += ROWS) {
+        const float l = sl[(int64_t)s * a.sl_s];
+        const float w = l == -INFINITY ? 0.0f : __expf(l - safe);
+        if (w > 0.0f) acc += w * *reinterpret_cast<const f32x4*>(base + (int64_t)s * a.al_s);
+    }
+    float W = 0.0f;
+#pragma unroll
+    for (int k = 0; k < NL; ++k)
+        if (64 * k < N) W += all[k] == -INFINITY ? 0.0f : __expf(all[k] - safe);
+    W = row16_sum(W);
+    {
+        auto at = [&](int l) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, W), l)); };
+        W = (at(0) + at(16)) + (at(32) + at(48));
+    }
+    auto fold32 = [](float x, float y) {         // sums over the lanes 32 apart: x's in the lower half, y's in the upper
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    };
+    float lo = fold32(acc[0], acc[2]), hi = fold32(acc[1], acc[3]);
+    const int c = 4 * c4 + 2 * (lane >> 5);
+    if constexpr (LPR == 32) {
+        s_acc[wave][c] = lo;
+        s_acc[wave][c + 1] = hi;
+    } else {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(lo), __float_as_uint(hi), false, false);
+        s_acc[wave][c + ((lane >> 4) & 1)] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+    __syncthreads();
+    if (tid < CH) {
+        float A = 0.0f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) A += s_acc[w][tid];
+        const float out = W > 0.0f ? A / W : 0.0f;
+        const int64_t to = b * a.o_b + (int64_t)h * a.o_h + blockIdx.z * CH + tid;
+        if (a.o16) a.o16[to] = f32_to_bf16_any(out);
+        else a.o[to] = out;
+        if (tid == 0 && blockIdx.z == 0) a.lse[b * a.lse_b + h] = W > 0.0f ? top + __logf(W) : -INFINITY;
+    }
+}
+
+int fold_states(const float* al, int64_t al_b, int64_t al_h, int64_t al_s, const StateLse& states, int slots, int sure,
+                void* o, bool o_bf16, int64_t o_b, int64_t o_h, float* lse, int64_t lse_b, int B, int Hq, int D,
+                void* stream) {
+    if (B <= 0 || Hq <= 0 || slots < 1 || slots > 512 + kTailParts || (D != 64 && D != 128) || !al || !o || !lse || !states.p ||
+        (reinterpret_cast<uintptr_t>(al) & 15) || al_b % 4 || al_h % 4 || al_s % 4) {
+        set_error("fold_states: bad shape or misaligned states");
+        return -1;
+    }
+    const FoldArgs a{al, al_b, al_h, al_s, states.p, states.b, states.h, states.s, o_bf16 ? nullptr : static_cast<float*>(o),
+                     o_bf16 ? static_cast<uint16_t*>(o) : nullptr, o_b, o_h, lse, lse_b, slots, std::min(std::max(sure, 1), slots)};
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    // Few heads: two workgroups each, as many lanes as the states keep busy.
+    const bool halves = D == 128 && B * Hq <= 512, few = slots <= 96;
+    const dim3 grid(B, Hq, halves ? 2 : 1);
+    if (halves && few) hipLaunchKernelGGL((fold_kernel<128, 2, 256>), grid, dim3(256), 0, st, a);
+    else if (halves) hipLaunchKernelGGL((fold_kernel<128, 2, 1024>), grid, dim3(1024), 0, st, a);
+    else if (D == 128 && few) hipLaunchKernelGGL((fold_kernel<128, 1, 256>), grid, dim3(256), 0, st, a);
+    else if (D == 128) hipLaunchKernelGGL((fold_kernel<128, 1, 1024>), grid, dim3(1024), 0, st, a);
+    else if (few) hipLaunchKernelGGL((fold_kernel<64, 1, 256>), grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((fold_kernel<64, 1, 1024>), grid, dim3(1024), 0, st, a);
+    if (hipGetLastError() != hipSuccess) { set_error("fold_states: launch failed"); return -2; }
+    return 0;
 }
 
 template <bool HIST, bool SHARED>

@@ -1,6 +1,7 @@
 // Argument block and small helpers shared by the decode kernels.
 #pragma once
 #include "ommx_common.h"
+#include "ommx_internal.h"
 
 namespace ommx {
 
@@ -39,6 +40,10 @@ struct DecodeArgs {
     // set by the launcher of the serving-recipe kernel only: head_dim is 64 and Hkv counts PAIRS of kv
     // heads (the planes of two neighbouring 64-channel heads read like one 128-channel head)
     int half;
+    // The tail rows attended by this launch (ommx_decode_tail.h): that many slices of the grid, 0 none.  Slices of x
+    // behind the splits, or of y in front of the shares.
+    int t_slices;
+    DecodeTail t;
 };
 
 // 7-bit position streams (pack.py:128-164): position s of a frame at bits [7s, 7s+7)
@@ -101,7 +106,9 @@ struct TailRows {
     int n, n_sink, turn, span, sink, cap;
     int64_t k_base, v_base;
 
-    __device__ __forceinline__ void init(const CombineArgs& a, int b) {
+    // A: CombineArgs or DecodeTail
+    template <class A>
+    __device__ __forceinline__ void init(const A& a, int b) {
         if constexpr (!HIST) {
             // a length outside the tail buffer (when the caller has said how many rows it holds) is held
             // inside it, so that no row address leaves the buffer whatever b_tail_len contains

@@ -40,6 +40,7 @@
 #include <type_traits>
 
 #include "ommx_decode_shares.h"
+#include "ommx_decode_tail.h"
 #include "ommx_decode_util.h"
 
 namespace ommx {
@@ -47,6 +48,15 @@ namespace ommx {
 namespace {
 
 using namespace decode_util;
+
+// The kernels that also attend the tail rows are compiled apart (ommx_decode_gqa4_tail.hip): the tail's code beside the
+// splits' costs a launch that does not need it 0.3 to 1 % (registers, spilled scalars).
+#ifndef OMMX_GQA4_LAUNCH
+#define OMMX_GQA4_LAUNCH launch_decode_gqa4
+constexpr bool TAIL = false;
+#else
+constexpr bool TAIL = true;
+#endif
 
 #ifndef OMMX_GQA4_WAVES
 #define OMMX_GQA4_WAVES 3          // waves per SIMD the register budget is set for
@@ -181,12 +191,30 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
     const int heads = PARTIAL ? a.Hq / Hkv : NH;
     const int qh0 = kvh * heads;
     const int r_half = max(heads >> 1, 1);            // head_dim 64: q heads per kv head of the pair
+    if (TAIL) {
+        // slices of the grid that attend the bf16 tail rows (head_dim 64: of either kv head of the pair)
+        const int slice = dealt ? static_cast<int>(blockIdx.y) : static_cast<int>(blockIdx.x) - a.S;
+        if (slice >= 0 && slice < a.t_slices) {
+            const int part = slice & (kTailParts - 1), rest = slice / kTailParts;
+            const int tb = dealt ? (half ? rest >> 1 : rest) : static_cast<int>(blockIdx.z);
+            const int sub = half ? rest & 1 : 0;
+            if (GEN && half) tail::attend_part<NH, 64>(a, sm, tb, 2 * kvh + sub, heads >> 1, part, lane);
+            else tail::attend_part<NH, 128>(a, sm, tb, kvh, heads, part, lane);
+            return;
+        }
+    }
     uint32_t sp = blockIdx.x, S = static_cast<uint32_t>(a.S);
     int b = ORDER == 0 ? 0 : static_cast<int>(blockIdx.z), L;      // ORDER 0 is launched for one request only
     if (dealt) {
         shares::Share mine;
-        if (!shares::find_share<(1 << UNIT_SH), ORDER == 2 ? 4 : 1>(a, blockIdx.y, lane, mine)) return;
+        if (!shares::find_share<(1 << UNIT_SH), ORDER == 2 ? 4 : 1>(a, blockIdx.y - (TAIL ? a.t_slices : 0), lane, mine)) return;
         b = mine.b; L = mine.L; sp = mine.sp; S = mine.n;
+        if (TAIL && sp == 0) {
+            // the merge then goes by the lse alone: the slots this request does not use say that nothing was attended
+            for (int r = 0; r < heads; ++r)
+                for (uint32_t s = S + lane; s < static_cast<uint32_t>(a.S); s += 64)
+                    a.sl[b * a.sl_b + (int64_t)(qh0 + r) * a.sl_h + (int64_t)s * a.sl_s] = -INFINITY;
+        }
     } else if (ORDER >= 1 && a.B > 1 && a.B <= 64) {
         const int my_len = lane < a.B ? a.seq[lane] : 0;
         const uint32_t key = (static_cast<uint32_t>(my_len) << 6) | (63u - lane);
@@ -1108,7 +1136,7 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
 }  // namespace
 
 // Returns 0 when launched, 1 when the shape belongs to another kernel.
-int launch_decode_gqa4(const DecodeArgs& a_in, int Dh, int R, hipStream_t st) {
+int OMMX_GQA4_LAUNCH(const DecodeArgs& a_in, int Dh, int R, const DecodeTail* tail, hipStream_t st) {
     DecodeArgs a = a_in;
     a.half = 0;
     if (a.scale_bf16 || a.v_bf16) return 1;
@@ -1146,7 +1174,12 @@ int launch_decode_gqa4(const DecodeArgs& a_in, int Dh, int R, hipStream_t st) {
     const int waves = (a.Hkv % 4 == 0) ? 4 : ((a.Hkv % 2 == 0) ? 2 : 1);
     // shares: the orders below hold up to 64 requests (one per lane), or 256 (four)
     if (a.shares > 0 && a.B > (longer || (nh < 4 && !general) ? 64 : 256)) return 1;
-    const dim3 grid = a.shares > 0 ? dim3(a.Hkv / waves, a.shares) : dim3(a.S, a.Hkv / waves, a.B);
+    a.t_slices = 0;
+    if (TAIL) {
+        a.t = *tail;
+        a.t_slices = kTailParts * (a.half ? 2 : 1) * (a.shares > 0 ? a.B : 1);
+    }
+    const dim3 grid = a.shares > 0 ? dim3(a.Hkv / waves, a.t_slices + a.shares) : dim3(a.S + a.t_slices, a.Hkv / waves, a.B);
     const dim3 block(64 * waves);
     const size_t shm = (size_t)waves * (longer ? (nh == 8 ? LdsMap<8, true>::LDS_WAVE : LdsMap<4, true>::LDS_WAVE)
                                               : (nh == 8 ? LdsMap<8, false>::LDS_WAVE : LdsMap<4, false>::LDS_WAVE));

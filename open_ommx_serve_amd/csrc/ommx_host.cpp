@@ -191,6 +191,14 @@ struct DecodeCall {
     int64_t ring_sink = 0, ring_span = 0, win_sink = 0, win_recent = 0;
 };
 
+// Whether the history's ring holds every row that the window can ask for (what the merge over a history checks too).
+bool hist_window_fits(const DecodeCall& c, int64_t gt, int64_t rows) {
+    const int64_t most = c.win_recent + gt - 1;
+    return c.win_sink >= 0 && c.win_recent >= 0 && rows > 0 &&
+           (c.ring_span <= 0 ||
+            (c.ring_sink == c.win_sink && c.ring_span >= most && c.ring_sink + c.ring_span <= rows));
+}
+
 // Checks the call and launches it: 1 launched, 0 refused (nothing done), -1 a launch failed (exception set).
 int run_decode(const DecodeCall& c) {
     const at::Tensor &q = *c.q, &k_base = *c.k_base, &k_scale = *c.k_scale, &v_main = *c.v_main, &v_scale = *c.v_scale;
@@ -321,6 +329,44 @@ int run_decode(const DecodeCall& c) {
             c.o->stride(1), lse, c.lse->stride(0), B, Hq, Hkv, D, S, gt, tail ? kt->size(1) : 0, c.sm_scale, c.cap,
             states, dealt, stream);
     };
+    // The tail rows as states of their own, attended by the split-KV launch: while the launch leaves the wave slots
+    // for them free (they are few, and short beside a split).  Rows must be readable 16 bytes at a time.
+    auto rows16 = [&](const at::Tensor* t) {
+        return reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0 && t->stride(0) % 8 == 0 && t->stride(1) % 8 == 0 &&
+               t->stride(2) % 8 == 0;
+    };
+    const int64_t tail_waves = ommx::kTailParts * B * Hkv, all_waves = int64_t{cu_count(dev.index())} * 4 * (lean ? 3 : 2);
+    const bool tail_rows = (hist || tail) && !c.ws && !c.force && rows16(kt) && rows16(vt) &&
+                           (!hist || hist_window_fits(c, gt, kt->size(1)));
+    ommx::DecodeTail tl{};
+    if (tail_rows) {
+        tl = {data<uint16_t>(kt), data<uint16_t>(vt), kt->stride(0), kt->stride(1), kt->stride(2), vt->stride(0),
+              vt->stride(1), vt->stride(2), nullptr, static_cast<int>(kt->size(1)), nullptr, nullptr, 0, 0, 0, 0, 0,
+              static_cast<int>(gt)};
+        if (hist) {
+            tl.hist_seq = data<int64_t>(c.hist_seq);
+            tl.hist_slots = data<int64_t>(c.hist_slots);
+            tl.hist_rows = static_cast<int>(kt->size(1));
+            tl.ring_sink = c.ring_span > 0 ? static_cast<int>(c.ring_sink) : 0;
+            tl.ring_span = static_cast<int>(c.ring_span);
+            tl.win_sink = static_cast<int>(c.win_sink);
+            tl.win_recent = static_cast<int>(c.win_recent);
+            tl.T = static_cast<int>(c.win_sink + c.win_recent + gt - 1);
+        } else {
+            tl.tail = data<int32_t>(c.b_tail);
+        }
+    }
+    bool tail_done = false;
+    // the merge of either kind: `al` and `states` as the splits have them, `front` slots for the tail before them
+    auto merge = [&](float* al, int64_t al_b, int64_t al_h, int64_t al_s, float* lse, int64_t S, const ommx::StateLse& states,
+                     const ommx::Shares* dealt) {
+        if (!tail_done) return combine(al, al_b, al_h, al_s, lse, S, &states, dealt);
+        ommx::StateLse all = states;
+        all.p -= ommx::kTailParts * states.s;
+        return ommx::fold_states(al - ommx::kTailParts * al_s, al_b, al_h, al_s, all, S + ommx::kTailParts,
+                                 ommx::kTailParts + (dealt ? std::min<int>(S, dealt->each) : S), data(c.o), o_bf16,
+                                 c.o->stride(0), c.o->stride(1), lse, c.lse ? c.lse->stride(0) : Hq, B, Hq, D, stream);
+    };
     // (the argument list that the split-KV entries share; the state strides and the split count come first)
 #define OMMX_SPLITKV_ARGS(AL, AL_B, AL_H, AL_S, SPLITS)                                                                  \
     qp, q.stride(0), q.stride(1), data<uint8_t>(c.k_base), data(c.k_scale), data<uint16_t>(c.k_zp),                      \
@@ -340,22 +386,31 @@ int run_decode(const DecodeCall& c) {
         const int64_t fit = cu_count(dev.index()) * 4 / wave_heads;
         // (max_seq bounds how many groups there can be; were it too small, the shares would be longer, nothing else)
         const int64_t longest = std::max<int64_t>(1, (c.max_seq + unit - 1) / unit);
-        const int64_t shares = std::min({int64_t{2048}, fit * (lean ? 3 : 2), B * longest}), few = std::min(shares, fit * 2);
+        int64_t shares = std::min({int64_t{2048}, fit * (lean ? 3 : 2), B * longest});
+        const int64_t few = std::min(shares, fit * 2);
+        // (a few tail waves: the third workgroup of some compute units is theirs)
+        if (tail_rows && 16 * tail_waves <= all_waves) shares = std::min(shares, std::max(few, (all_waves - tail_waves) / wave_heads));
         const int64_t most = std::min({int64_t{B * Hq >= 256 ? 64 : (shares > 256 * B && longest > 512 ? 512 : 256)}, longest,
                                        std::max<int64_t>(8, 4 * shares / B)});
         // A batch of fewer groups than one and a half waves per SIMD is left to fixed splits: no wave gets more than
         // one step either way, and those need not find their share (0.3 us, and as much again in the combine).
-        if (few >= B && 2 * B * longest > 3 * fit) {
-            const int64_t n = B * Hq * most, singles = paired ? 2 * fit : fit;
+        if (few >= B && B * longest > fit) {
+            const int64_t singles = paired ? 2 * fit : fit;
+            // (about as many shares as there are: each group one, or half as many and each request's last)
+            const int64_t used = std::min(shares, B * longest > singles ? B * longest / 2 + B : B * longest);
+            const bool with_tail = tail_rows && used * wave_heads + tail_waves <= all_waves;
+            const int64_t front = with_tail ? ommx::kTailParts : 0, row = most + front, n = B * Hq * row;
             c10::DataPtr scratch = allocator->allocate(static_cast<size_t>(n * (D + 1) + B * Hq + B) * sizeof(float));
             float *al = static_cast<float*>(scratch.get()), *lse = c.lse ? data<float>(c.lse) : al + n * (D + 1);
-            const ommx::StateLse states{al + n * D, Hq * most, most, 1};
+            const ommx::StateLse states{al + n * D + front, Hq * row, row, 1};
             const ommx::Shares dealt{static_cast<int>(shares), static_cast<int>(few), static_cast<int>(singles),
                                      static_cast<int>((std::min(shares, B * longest > singles ? B * longest / 2 : shares) + B - 1) / B),
                                      reinterpret_cast<int32_t*>(al + n * (D + 1) + B * Hq)};
+            al += front * D;
             Py_BEGIN_ALLOW_THREADS
-            rc = ommx::decode_splitkv(OMMX_SPLITKV_ARGS(al, Hq * most * D, most * D, D, most), false, &states, &dealt);
-            if (rc == 0) rc2 = combine(al, Hq * most * D, most * D, D, lse, most, &states, &dealt);
+            rc = ommx::decode_splitkv(OMMX_SPLITKV_ARGS(al, Hq * row * D, row * D, D, most), false, &states, &dealt,
+                                      with_tail ? &tl : nullptr, &tail_done);
+            if (rc == 0) rc2 = merge(al, Hq * row * D, row * D, D, lse, most, states, &dealt);
             Py_END_ALLOW_THREADS
         }
     }
@@ -365,8 +420,9 @@ int run_decode(const DecodeCall& c) {
         if (c.ws && (c.ws->scalar_type() != at::kFloat || c.ws->dim() != 4 || c.ws->size(0) != B || c.ws->size(1) != Hq ||
                      c.ws->size(2) < S || c.ws->size(3) < D + 1 || c.ws->stride(3) != 1))
             return 0;
-        const int64_t n = B * Hq * S;
-        int64_t al_b = Hq * S * D, al_h = S * D, al_s = D;
+        const bool with_tail = tail_rows && S * wave_heads * B + tail_waves <= all_waves;
+        const int64_t front = with_tail ? ommx::kTailParts : 0, row = S + front, n = B * Hq * row;
+        int64_t al_b = Hq * row * D, al_h = row * D, al_s = D;
         c10::DataPtr scratch;
         float *al, *lse = data<float>(c.lse);
         ommx::StateLse states;
@@ -377,12 +433,14 @@ int run_decode(const DecodeCall& c) {
         } else {
             scratch = allocator->allocate(static_cast<size_t>(n * (D + 1) + B * Hq) * sizeof(float));
             al = static_cast<float*>(scratch.get());
-            states = {al + n * D, Hq * S, S, 1};
+            states = {al + n * D + front, Hq * row, row, 1};
             if (!lse) lse = al + n * (D + 1);
+            al += front * D;
         }
         Py_BEGIN_ALLOW_THREADS
-        rc = ommx::decode_splitkv(OMMX_SPLITKV_ARGS(al, al_b, al_h, al_s, S), c.force, &states, nullptr);
-        if (rc == 0) rc2 = combine(al, al_b, al_h, al_s, lse, S, &states, nullptr);
+        rc = ommx::decode_splitkv(OMMX_SPLITKV_ARGS(al, al_b, al_h, al_s, S), c.force, &states, nullptr,
+                                  with_tail ? &tl : nullptr, &tail_done);
+        if (rc == 0) rc2 = merge(al, al_b, al_h, al_s, lse, S, states, nullptr);
         Py_END_ALLOW_THREADS
     }
 #undef OMMX_SPLITKV_ARGS

@@ -85,8 +85,27 @@ int decode_combine_hist(const float* attn_logits, int64_t al_b, int64_t al_h, in
                         float* lse, int64_t lse_b, int B, int Hq, int Hkv, int D, int num_splits, int group_tokens,
                         float sm_scale, float logit_cap, const StateLse& states, const Shares* shares, void* stream);
 
-// ommx_decode_splitkv / _ref (plain) with these choices (either may be NULL).  Returns 1, with nothing done, when shares
-// are asked for and no kernel with shares serves the call.
+// The bf16 tail rows as kTailParts more states of every (request, q head), attended by the split-KV launch itself: slots
+// 0 .. kTailParts - 1 of the state rows, in front of the splits' own (attn_logits and the lse plane point behind them).
+// Gathered rows (tail lengths) or rows of a history (seq), as above.  K and V rows 16-byte aligned.
+constexpr int kTailParts = 4;
+struct DecodeTail {
+    const uint16_t *kt, *vt;
+    int64_t kt_b, kt_t, kt_h, vt_b, vt_t, vt_h;
+    const int32_t* tail;            // gathered: rows of every request, at most T (0: not told)
+    int T;
+    const int64_t *hist_seq, *hist_slots;
+    int hist_rows, ring_sink, ring_span, win_sink, win_recent, gt;
+};
+
+// o and lse of every (request, q head) from its `slots` states (rows of D floats, lse plane beside them): the merge when
+// the tail rows are among the states.  `sure`: how many slots are read before their lse is known.
+int fold_states(const float* al, int64_t al_b, int64_t al_h, int64_t al_s, const StateLse& states, int slots, int sure,
+                void* o, bool o_bf16, int64_t o_b, int64_t o_h, float* lse, int64_t lse_b, int B, int Hq, int D,
+                void* stream);
+
+// ommx_decode_splitkv / _ref (plain) with these choices (each may be NULL).  Returns 1, with nothing done, when shares
+// are asked for and no kernel with shares serves the call.  *tail_done tells whether the launch attends the tail.
 #define OMMX_DECODE_DECL                                                                            \
     const uint16_t* q, int64_t q_stride_b, int64_t q_stride_h, const uint8_t* k_base,               \
     const void* k_scale, const uint16_t* k_zp, const uint16_t* k_ms, const uint16_t* k_mc,          \
@@ -98,7 +117,8 @@ int decode_combine_hist(const float* attn_logits, int64_t al_b, int64_t al_h, in
     int group_channels, int v_bf16, int num_splits, float sm_scale, float logit_cap,                \
     int packed_start_offset, int seg_group_base, int num_pages, int num_group_slots,                \
     int32_t* err_flag, void* stream
-int decode_splitkv(OMMX_DECODE_DECL, bool plain, const StateLse* lse, const Shares* shares);
+int decode_splitkv(OMMX_DECODE_DECL, bool plain, const StateLse* lse, const Shares* shares, const DecodeTail* tail,
+                   bool* tail_done);
 #undef OMMX_DECODE_DECL
 
 // ommx_decode_combine with the lse of the states elsewhere (NULL: column D) and the shares they come from (NULL:

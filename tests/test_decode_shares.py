@@ -93,3 +93,29 @@ def test_shares_over_a_row_history(lens):
     assert pool.decode_into(q, out, torch.arange(B, device="cuda"), torch.tensor(lens, device="cuda"), d["b_seq_len"],
                             (d["req_to_token"], d["req_to_group"]), sm_scale=D ** -0.5, max_seq_len=d["max_seq_len"])
     assert (out.float() - want).abs().max().item() <= 2.0 ** -8 * want.abs().max().item() + 1e-4
+
+
+@pytest.mark.parametrize("hq,hkv,D,kw,recent", [
+    (32, 8, 128, {}, 32), (64, 8, 128, {}, 32), (4, 4, 128, {}, 130), (8, 1, 128, dict(outlier_repr="relidx7"), 32),
+    (32, 8, 64, {}, 32), (8, 8, 64, {}, 150), (16, 4, 128, dict(group_tokens=128, group_channels=64, outlier_repr="relidx7"), 32),
+])
+def test_tail_rows_beside_the_splits(hq, hkv, D, kw, recent):
+    """The tail in four parts as states of its own: no rows, fewer rows than parts, parts of one and of two blocks of 16
+    and one row more, several passes of 32; one request (fixed splits) and many (shares); rows that cannot be read 16
+    bytes at a time, and a launch whose splits leave no room, take the other merge."""
+    win = WindowSpec(recent_window=recent, group_tokens=kw.get("group_tokens", 32))
+    for seqs in ([2000], [2000, 900, 3000, 700, 2500, 1500]):
+        case = build_decode_case(seqs, q_heads=hq, kv_heads=hkv, head_dim=D, seed=91, permute_tables=True,
+                                 sparse_frac=0.005, window=win, **kw)
+        T = case.k_tail.shape[1]
+        for lens in ([0, 1, 3, 15, 16, 17], [31, 32, 33, 63, 64, 65], [T, T - 1, 70, 128, 129, 2]):
+            lens = [min(n, T) for n in lens][:len(seqs)]
+            case.b_tail_len.copy_(torch.tensor(lens, dtype=torch.int32))
+            want = _oracle(case)
+            longest = max(case.b_seq_len.tolist())
+            _close(_run(case, max_seq_len=longest), want, f"tails {lens}")
+            _close(_run(case, max_seq_len=longest, num_kv_splits=400), want, f"tails {lens}, 400 splits")
+        odd = torch.empty(case.v_tail.numel() + 1, dtype=case.v_tail.dtype, device=case.v_tail.device)[1:].view_as(case.v_tail)
+        odd.copy_(case.v_tail)
+        case.v_tail = odd
+        _close(_run(case, max_seq_len=longest), want, "V rows at an odd address")
