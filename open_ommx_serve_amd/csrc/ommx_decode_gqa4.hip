@@ -145,7 +145,7 @@ __device__ __forceinline__ uint32_t pk_u16(uint32_t lo, uint32_t hi) { return (l
 // first, 2 up to 256 (radix select); see ommx_decode.hip.
 // NH: q heads per kv head the matrix rows and columns are laid out for, 4 or 8.
 // GEN: the general form of the recipe: 1..8 outliers per vector (a.kout, bitmap plane only), and
-// head_dim 64 (a.half): the planes of two neighbouring 64-channel kv heads read exactly like one
+// head_dim 64 (a.half, or HALF when nothing else is general): the planes of two neighbouring 64-channel kv heads read exactly like one
 // 128-channel head, so a wave takes the pair as one head whose q heads are those of both, each
 // zero on the other one's channels, and writes each q head only its own half of the output.
 // GTS: K groups of 32 << GTS tokens (position streams; V vectors then 32, 64 or 128 channels wide), 6 outliers, or
@@ -157,7 +157,7 @@ __device__ __forceinline__ uint32_t pk_u16(uint32_t lo, uint32_t hi) { return (l
 // call, ommx_decode.hip's kernel on whole groups -> this one: 128 tokens and 10 outliers, 4 requests of 2 to 20 K
 // 45.9 -> 34.7 us, one of 64 K 47.1 -> 40.0, 8 of 4 to 16 K with 64 q heads 84.7 -> 52.6; 64 tokens and 6 outliers,
 // 64 K 36.8 -> 32.3, 1.1 K 15.5 -> 14.5.
-template <int IDX, bool OWN_MAP, bool PARTIAL, int ORDER, int NH = 4, bool GEN = false, int KSLOTS = 6, int GTS = 0>
+template <int IDX, bool OWN_MAP, bool PARTIAL, int ORDER, int NH = 4, bool GEN = false, int KSLOTS = 6, int GTS = 0, bool HALF = false>
 __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : OMMX_GQA4_WAVES) decode_gqa4_kernel(DecodeArgs a) {
     static_assert(NH == 4 || (NH == 8 && !PARTIAL), "4 heads (or fewer, PARTIAL) or exactly 8");
     static_assert(!GEN || IDX == 0, "the general form reads bitmaps");
@@ -171,7 +171,7 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
     constexpr int UNIT_SH = LONG ? 6 : 5;             // log2 of the tokens that the work is dealt out in
     constexpr int NG = LONG ? 1 : 2;                  // groups (parameter sets) a step reads
     const int kout = GEN ? a.kout : KMAX;
-    const bool half = GEN && a.half;
+    const bool half = GEN ? a.half != 0 : HALF;
     using Lds = LdsMap<NH, LONG>;
     constexpr int OFF_KT = Lds::OFF_KT, OFF_MAG = Lds::OFF_MAG, OFF_ZPP = Lds::OFF_ZPP, OFF_VT = Lds::OFF_VT,
                   OFF_PT = Lds::OFF_PT, OFF_VZ = Lds::OFF_VZ, OFF_VS = Lds::OFF_VS, OFF_LC = Lds::OFF_LC, OFF_ZERO = Lds::OFF_ZERO,
@@ -198,8 +198,8 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
             const int part = slice & (kTailParts - 1), rest = slice / kTailParts;
             const int tb = dealt ? (half ? rest >> 1 : rest) : static_cast<int>(blockIdx.z);
             const int sub = half ? rest & 1 : 0;
-            if (GEN && half) tail::attend_part<NH, 64>(a, sm, tb, 2 * kvh + sub, heads >> 1, part, lane);
-            else tail::attend_part<NH, 128>(a, sm, tb, kvh, heads, part, lane);
+            if ((GEN || HALF) && half) tail::attend_part<NH, 64>(a, sm, tb, 2 * kvh + sub, heads >> 1, part, lane);
+            else if (!HALF) tail::attend_part<NH, 128>(a, sm, tb, kvh, heads, part, lane);
             return;
         }
     }
@@ -500,7 +500,7 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
 #pragma unroll
         for (int r = 0; r < NH; ++r)
             qm = fmaxf(qm, fabsf(__uint_as_float(u ? (qraw[r] & 0xFFFF0000u) : (qraw[r] << 16))));
-        big_thr[u] = ((GEN ? (kout < 6 ? 0.5f : 0.75f) : 1.0f) * BIG_DELTA * 16.0f * BIG_DELTA_SM_SCALE) * (u ? cs1 : cs0) *
+        big_thr[u] = ((GEN || HALF ? (kout < 6 ? 0.5f : 0.75f) : 1.0f) * BIG_DELTA * 16.0f * BIG_DELTA_SM_SCALE) * (u ? cs1 : cs0) *
                      __builtin_amdgcn_rcpf(qm * sm_scale);
     }
     const uint32_t kt_lane = OFF_KT + (c0 >> 2);                   // code byte of the channel pair (4 channels a byte), row 0
@@ -1219,6 +1219,25 @@ int OMMX_GQA4_LAUNCH(const DecodeArgs& a_in, int Dh, int R, const DecodeTail* ta
             case 13: OMMX_GO_LONG(true, 8, 6, 2); break;
             default: OMMX_GO_LONG(true, 8, 10, 2); break;
         }
+        return 0;
+    }
+    // head_dim 64 with 6 outliers, up to 64 requests: the same form with all of that known at compile time (the general
+    // one walks one channel after the other, looks its slot count up and searches its share over 256 requests: 1 request of
+    // 1 K 10.4 -> 8.8 us, 2 of 12 K 19.1 -> 17.1, 8 of 8 K 27.9 -> 25.1, kernel alone)
+    if (a.half && a.kout == 6 && order < 2) {
+#define OMMX_GO_HALF(MAP, PART, ORD, NH) \
+    hipLaunchKernelGGL((decode_gqa4_kernel<0, MAP, PART, ORD, NH, false, 6, 0, true>), grid, block, shm, st, a)
+        switch ((nh == 8 ? 4 : 0) | (order ? 2 : 0) | (own_map ? 1 : 0)) {
+            case 0: OMMX_GO_HALF(false, true, 0, 4); break;
+            case 1: OMMX_GO_HALF(true, true, 0, 4); break;
+            case 2: OMMX_GO_HALF(false, true, 1, 4); break;
+            case 3: OMMX_GO_HALF(true, true, 1, 4); break;
+            case 4: OMMX_GO_HALF(false, false, 0, 8); break;
+            case 5: OMMX_GO_HALF(true, false, 0, 8); break;
+            case 6: OMMX_GO_HALF(false, false, 1, 8); break;
+            default: OMMX_GO_HALF(true, false, 1, 8); break;
+        }
+#undef OMMX_GO_HALF
         return 0;
     }
     if (general) {
