@@ -288,6 +288,24 @@ class MultiSeqKVPool:
         self._write_rows(r, K, V, 0, *live)
         return target
 
+    def append_prompts(self, slots: Sequence[int], starts: Sequence[int], K: torch.Tensor, V: torch.Tensor) -> bool:
+        """``reset_slot`` and ``append_block`` of several requests in two launches: rows ``starts[i] .. starts[i + 1]``
+        of ``K`` / ``V`` ``[n, H, D]`` are the whole prompt of slot ``slots[i]``.  False, with nothing done, when the
+        rows or the pool are not of the kind that the launches take (a ring, rows that are not bf16, a prompt longer
+        than the history)."""
+        lens = [b - a for a, b in zip(starts, starts[1:])]
+        if self.kv_ring or max(lens) > self.max_seq_len:
+            return False
+        groups = [self.window.num_groups(n) for n in lens]
+        if not self._host.pack_prompts(self.k_hist, self.v_hist, self._store_planes, K, V, list(slots), list(starts),
+                                       groups, self.ps, self.window.sink_tokens, self.G_per_seq, self.err_flag,
+                                       store_table(self.k_hist.device), *self._recipe):
+            return False
+        for r, n, g in zip(slots, lens, groups):
+            self.seq_len[r] = n
+            self.packed_groups[r] = g
+        return True
+
     def _write_rows(self, req: int, K: torch.Tensor, V: torch.Tensor, pos0: int, n_head: int, lo: int) -> None:
         """Rows ``[0, n_head)`` and ``[lo, T)`` of a block into request ``req``'s history at their ring
         slots (the block starts at absolute position ``pos0``), one launch."""

@@ -896,6 +896,62 @@ PyObject* py_pack_groups(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Py_RETURN_TRUE;
 }
 
+// (k_hist, v_hist, planes, K, V, slots [B], starts [B + 1], groups [B], page_size, window_sink, groups_per_seq, err_flag,
+//  table, recipe x 8): rows starts[i] .. starts[i + 1] of K / V are the whole prompt of a fresh request in slot slots[i] of a
+// history without a ring: the rows are copied and the first groups[i] groups packed, two launches for all requests.
+PyObject* py_pack_prompts(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 21) { PyErr_SetString(PyExc_TypeError, "pack_prompts: wrong number of arguments"); return nullptr; }
+    bool ok = true;
+    const at::Tensor *kh = as_tensor(a[0], ok), *vh = as_tensor(a[1], ok), *K = as_tensor(a[3], ok), *V = as_tensor(a[4], ok),
+                     *err = as_tensor_or_none(a[11], ok), *table = as_tensor(a[12], ok);
+    const int64_t ps = as_int(a[8], ok), wsink = as_int(a[9], ok), per_seq = as_int(a[10], ok);
+    Recipe r;
+    Planes p;
+    std::vector<int64_t> slots, starts, groups;
+    if (!ok || !is_history(*kh, *vh) || !read_recipe(a + 13, r) || !read_planes(a[2], r, p) || ps < 1 || r.gt % ps || wsink < 0 ||
+        !read_ints(a[5], slots) || !read_ints(a[6], starts) || !read_ints(a[7], groups) || !is_rows(*K) || !is_rows(*V) ||
+        K->scalar_type() != at::kBFloat16 || V->scalar_type() != at::kBFloat16 || K->sizes() != V->sizes() ||
+        K->device() != kh->device() || V->device() != kh->device() || K->is_alias_of(*kh) || K->is_alias_of(*vh) ||
+        V->is_alias_of(*kh) || V->is_alias_of(*vh))
+        Py_RETURN_FALSE;
+    const int64_t B = static_cast<int64_t>(slots.size()), N = kh->size(0), rows = kh->size(1), H = kh->size(2), D = kh->size(3);
+    if (B < 1 || B > ommx::kPromptsPerLaunch || static_cast<int64_t>(starts.size()) != B + 1 ||
+        static_cast<int64_t>(groups.size()) != B || starts[0] < 0 || starts.back() > K->size(0) || K->size(1) != H || K->size(2) != D)
+        Py_RETURN_FALSE;
+    std::vector<bool> taken(static_cast<size_t>(N), false);
+    std::vector<ommx::PromptRow> prompts(static_cast<size_t>(B));
+    int64_t total = 0;
+    for (int64_t i = 0; i < B; ++i) {
+        const int64_t len = starts[i + 1] - starts[i], slot = slots[i];
+        if (len < 1 || len > rows || slot < 0 || slot >= N || taken[slot] || groups[i] < 0 || groups[i] > per_seq ||
+            (groups[i] > 0 && wsink + groups[i] * r.gt > len))
+            Py_RETURN_FALSE;
+        taken[slot] = true;
+        prompts[i] = {static_cast<int32_t>(starts[i]), static_cast<int32_t>(starts[i + 1]), static_cast<int32_t>(slot),
+                      static_cast<int32_t>(total)};
+        total += groups[i];
+    }
+    if (N * per_seq * (r.gt / ps) > INT32_MAX) Py_RETURN_FALSE;
+    const c10::Device dev = kh->device();
+    c10::hip::HIPGuard guard(dev.index());
+    hipStream_t stream = stream_of(dev);
+    const int64_t T = total * r.gt;
+    // index tables: stream-ordered scratch, given back to torch's allocator when this call returns
+    c10::DataPtr scratch = c10::GetAllocator(c10::DeviceType::CUDA)->allocate((T + T / ps + total + 1) * sizeof(int32_t));
+    int32_t *src = static_cast<int32_t*>(scratch.get()), *pages = src + T, *dst = pages + T / ps;
+    const ommx::PromptBlocks blocks{data<uint16_t>(K), data<uint16_t>(V), K->stride(0), K->stride(1), V->stride(0), V->stride(1),
+                                    data<uint16_t>(kh), data<uint16_t>(vh), kh->stride(0), static_cast<int>(H),
+                                    static_cast<int>(D), static_cast<int>(wsink), static_cast<int>(r.gt),
+                                    static_cast<int>(ps), static_cast<int>(per_seq)};
+    int rc, rc2 = 0;
+    Py_BEGIN_ALLOW_THREADS
+    rc = ommx::prompt_blocks(blocks, prompts.data(), static_cast<int>(B), static_cast<int32_t>(total), src, pages, dst, stream);
+    if (rc == 0 && total > 0) rc2 = launch_store(*K, *V, 0, p, r, T, ps, src, pages, dst, *table, data<int32_t>(err), {}, stream);
+    Py_END_ALLOW_THREADS
+    if (failed(rc, "prompt_blocks") || failed(rc2, "ommx_store_pack")) return nullptr;
+    Py_RETURN_TRUE;
+}
+
 // (q, planes, k_hist, v_hist, slots, seq, b_seq_len, req_to_token, req_to_group, out, sm_scale, page_size, max_seq_len,
 //  mean_seq_len, ring sink, ring span, window sink, window recent, plain kernel, err_flag, recipe x 8): decode over a
 // pool's planes with the tail rows read in place from its history; out bf16 or fp32.  An observed call is refused.
@@ -1004,7 +1060,7 @@ PyObject* guarded(PyObject* self, PyObject* const* a, Py_ssize_t n) {
 #define OMMX_FAST(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(guarded<py_##name>)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
     OMMX_FAST(auto_num_kv_splits), OMMX_FAST(plain), OMMX_FAST(rows_fit),
-    OMMX_FAST(decode), OMMX_FAST(decode_pool), OMMX_FAST(store_pack), OMMX_FAST(pack_block), OMMX_FAST(block_errors), OMMX_FAST(pack_groups), OMMX_FAST(ring_write),
+    OMMX_FAST(decode), OMMX_FAST(decode_pool), OMMX_FAST(store_pack), OMMX_FAST(pack_block), OMMX_FAST(block_errors), OMMX_FAST(pack_groups), OMMX_FAST(pack_prompts), OMMX_FAST(ring_write),
     OMMX_FAST(tail_gather), OMMX_FAST(rows_write), OMMX_FAST(upload), OMMX_FAST(prefill),
     {nullptr, nullptr, 0, nullptr},
 };

@@ -48,6 +48,23 @@ int store_pack(const void* K, const void* V, int in_dtype, int64_t k_ts, int64_t
 // The rows in one launch; fp32 is rounded as torch does.  The caller has checked that every slot lies inside the history.
 int rows_write(const BlockRows& rows, void* stream);
 
+// Prompts of several fresh requests that lie behind one another in K / V [rows, H, D] (bf16): every row into its request's
+// whole history (no ring), and the index tables of the one store launch that packs all their groups.
+struct PromptBlocks {
+    const uint16_t *K, *V;
+    int64_t k_ts, k_hs, v_ts, v_hs;
+    uint16_t *k_hist, *v_hist;
+    int64_t stride_req;             // elements between the histories of two requests
+    int H, D, window_sink, gt, ps, groups_per_seq;
+};
+constexpr int kPromptsPerLaunch = 240;
+// {first row in K, row behind the last, slot, groups before this request's} of each request
+struct PromptRow { int32_t first, end, slot, group0; };
+// prompts[n], in the order of their rows; groups[n] groups of each; src_rows / dst_pages / dst_groups as ommx_store_pack
+// takes them, all groups together.
+int prompt_blocks(const PromptBlocks& blocks, const PromptRow* prompts, int n, int32_t total_groups, int32_t* src_rows,
+                  int32_t* dst_pages, int32_t* dst_groups, void* stream);
+
 // Up to kUploadWords 32-bit words from the host to dst inside a kernel's own argument block: no staging buffer, no
 // copy engine, nothing to keep alive after the call.
 constexpr int kUploadWords = 960;

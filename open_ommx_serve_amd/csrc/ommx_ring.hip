@@ -141,6 +141,50 @@ int rows_write(const BlockRows& a, void* stream) {
     return 0;
 }
 
+// ---- prompts of several requests -------------------------------------------------------------
+// One workgroup per row: it finds its request in the table that came with the launch (a scalar search over the first
+// rows), copies the row, and its first thread notes where the row's token is packed from and to.  One launch for rows and
+// lists and one store launch of all groups, instead of a row copy and a store launch per request: these grids fill the chip
+// where eight prompts of 100 to 700 rows used to take 16 launches of 3.4 to 4.7 and 6.4 to 7.0 us one after another.
+struct PromptTable { PromptRow row[kPromptsPerLaunch]; };
+static_assert(sizeof(PromptTable) <= kUploadWords * sizeof(int32_t), "the argument block");
+
+__global__ void __launch_bounds__(128) prompt_rows_kernel(PromptBlocks a, int n, int32_t total_groups, int32_t* src_rows,
+                                                          int32_t* dst_pages, int32_t* dst_groups, int vec, PromptTable t) {
+    const int row = t.row[0].first + blockIdx.x;
+    int lo = 0, hi = n - 1;                        // the last request whose first row is not behind this one
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (t.row[mid].first <= row) lo = mid;
+        else hi = mid - 1;
+    }
+    const PromptRow r = t.row[lo];
+    const int pos = row - r.first;
+    const int64_t to = r.slot * a.stride_req + pos * static_cast<int64_t>(a.H * a.D);
+    copy_row_in(a.k_hist + to, a.K + row * a.k_ts, a.k_hs, a.H, a.D, vec);
+    copy_row_in(a.v_hist + to, a.V + row * a.v_ts, a.v_hs, a.H, a.D, vec);
+    const int p = pos - a.window_sink, groups = (lo + 1 < n ? t.row[lo + 1].group0 : total_groups) - r.group0;
+    if (threadIdx.x == 0 && p >= 0 && p < groups * a.gt) {
+        const int at = r.group0 * a.gt + p;
+        src_rows[at] = row;
+        if (p % a.ps == 0) dst_pages[at / a.ps] = r.slot * (a.groups_per_seq * (a.gt / a.ps)) + p / a.ps;
+        if (p % a.gt == 0) dst_groups[at / a.gt] = r.slot * a.groups_per_seq + p / a.gt;
+    }
+}
+
+int prompt_blocks(const PromptBlocks& a, const PromptRow* prompts, int n, int32_t total_groups, int32_t* src_rows,
+                  int32_t* dst_pages, int32_t* dst_groups, void* stream) {
+    if (n < 1 || n > kPromptsPerLaunch || a.gt < 1 || a.ps < 1 || a.gt % a.ps) { set_error("prompt_blocks: bad shape"); return -1; }
+    PromptTable t;
+    for (int i = 0; i < n; ++i) t.row[i] = prompts[i];
+    const int vec = a.D % 8 == 0 && aligned16(a.k_hist) && aligned16(a.v_hist) && aligned16(a.K) && aligned16(a.V) &&
+                    a.stride_req % 8 == 0 && (a.k_ts | a.k_hs | a.v_ts | a.v_hs) % 8 == 0;
+    hipLaunchKernelGGL(prompt_rows_kernel, dim3(prompts[n - 1].end - prompts[0].first), dim3(128), 0,
+                       static_cast<hipStream_t>(stream), a, n, total_groups, src_rows, dst_pages, dst_groups, vec, t);
+    if (hipGetLastError() != hipSuccess) { set_error("prompt_blocks: launch failed"); return -2; }
+    return 0;
+}
+
 // ---- small host-to-device blocks through the kernel argument buffer ----------------------------
 // A host-to-device copy of a few hundred bytes of pageable memory costs 10-15 us of host time and waits for its
 // staging; a launch that carries the words as its arguments costs 2 us and leaves nothing behind.

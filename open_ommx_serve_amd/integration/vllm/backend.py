@@ -323,6 +323,10 @@ class OMMXCanonicalImpl(_ImplBase):
             step = mgr.step_on_device(pool)
             pool.append_decode_rows(mgr.slots, step.sel, step.col, key, value)
             return
+        if B > 1 and all(seq == b - a for seq, a, b in zip(mgr.seq_lens, bounds, bounds[1:])):
+            prompts = getattr(pool, "append_prompts", None)          # every row belongs to a new request's prompt
+            if prompts is not None and prompts(mgr.slots, bounds, key, value):
+                return
         for i in range(B):
             slot = mgr.slots[i]
             t0, t1 = int(bounds[i]), int(bounds[i + 1])

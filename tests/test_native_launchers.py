@@ -145,3 +145,43 @@ def test_error_words_nobody_asks_for_stay_until_the_kernel_is_through():
     assert at not in [t.data_ptr() for t in others]
     torch.cuda.synchronize()
     del held
+
+
+@pytest.mark.parametrize("H,D,kw,lens", [
+    (8, 128, {}, [97, 1, 530, 39, 40, 71, 72, 73]), (1, 128, dict(outlier_repr="relidx7"), [700, 8, 104]),
+    (4, 64, {}, [72, 71]), (2, 128, dict(group_tokens=64, group_channels=64, outlier_repr="relidx7", kv_outlier_map=False), [300, 111]),
+    (3, 64, {}, [41, 200, 1, 1]), (2, 128, dict(outliers_per_vector=0), [260, 90]),
+])
+def test_prompts_of_several_requests_in_two_launches(H, D, kw, lens):
+    """Every row and group where one append_block per request puts them: bit for bit, whatever the slots, from rows of a
+    wider tensor that do not start at its first row; what the launches do not take is refused and leaves the pool alone."""
+    kw = dict(kw)
+    win = WindowSpec(group_tokens=kw.pop("group_tokens", 32))
+    kw.setdefault("group_channels", min(32, D))
+    g = torch.Generator(device="cuda").manual_seed(3)
+    slots = [(5 * i + 2) % (len(lens) + 3) for i in range(len(lens))] if (len(lens) + 3) % 5 else list(range(len(lens)))[::-1]
+    pools = [MultiSeqKVPool(D, H, len(lens) + 3, 720, window=win, device="cuda", **{"outlier_repr": "bitmap", **kw}) for _ in range(3)]
+    for p in pools:
+        for t in (p.k_hist, p.v_hist, *(v for k, v in p.pool_planes().items() if torch.is_tensor(v) and not k.startswith("req_"))):
+            t.zero_()
+    starts = [5]
+    for n in lens:
+        starts.append(starts[-1] + n)
+    wide = torch.randn(starts[-1] + 3, 2 * H, D, generator=g, device="cuda").to(torch.bfloat16)
+    K, V = wide[:, :H], wide[:, H:]
+    assert pools[0].append_prompts(slots, starts, K, V)
+    for r, a, b in zip(slots, starts, starts[1:]):
+        pools[1].append_block(r, K[a:b], V[a:b])
+    assert pools[0].seq_len == pools[1].seq_len and pools[0].packed_groups == pools[1].packed_groups
+    for name, t in pools[0].pool_planes().items():
+        if torch.is_tensor(t):
+            assert torch.equal(t.view(torch.uint8), pools[1].pool_planes()[name].view(torch.uint8)), name
+    assert torch.equal(pools[0].k_hist, pools[1].k_hist) and torch.equal(pools[0].v_hist, pools[1].v_hist)
+    pools[0].check_errors()
+    before = [list(pools[2].seq_len), pools[2].k_hist.clone()]
+    assert not pools[2].append_prompts(slots, starts, K.float(), V.float())
+    assert not pools[2].append_prompts(slots, [0, *[x + 721 for x in starts[1:]]], K, V)
+    assert not pools[2].append_prompts([slots[0]] * len(slots), starts, K, V)
+    rows = pools[2].k_hist.view(-1, H, D)
+    assert not pools[2].append_prompts(slots, [0, *[x - 5 for x in starts[1:]]], rows, rows)
+    assert before[0] == pools[2].seq_len and torch.equal(before[1], pools[2].k_hist)
