@@ -348,19 +348,35 @@ class MultiSeqKVPool:
         kept, gt = self.window.sink_tokens + self.window.recent_window, self.gt
         seq, packed = self.seq_len, self.packed_groups
         pend: List[Tuple[int, int, int]] = []
-        total = 0
         for r in slots:
             n = seq[r] + 1
             seq[r] = n
             target = (n - kept) // gt
             if target > packed[r]:
                 pend.append((r, packed[r], target))
-                total += target - packed[r]
+        return self._pack_completed(pend)
+
+    def _pack_completed(self, pend: Sequence[Tuple[int, int, int]]) -> int:
         if pend:
             self._regroup_pack_batched_device(pend)
             for r, _g0, g1 in pend:
-                packed[r] = g1
-        return total
+                self.packed_groups[r] = g1
+        return sum(g1 - g0 for _r, g0, g1 in pend)
+
+    def append_step(self, slots: List[int], seqs: List[int], rows: torch.Tensor, cols: torch.Tensor, K: torch.Tensor,
+                    V: torch.Tensor) -> bool:
+        """``append_decode_rows`` of a step after which slot ``slots[i]`` holds ``seqs[i]`` tokens, its checks and its
+        bookkeeping in one native call.  False, with nothing done, when a slot is not one token behind the step, has no
+        room, or the rows are not what the launch takes."""
+        w = self.window
+        full = self._host.append_rows(self.k_hist, self.v_hist, cols, K, V, self._ring_sink, self._ring_rec, rows,
+                                      self.err_flag, self.seq_len, self.packed_groups, slots, seqs,
+                                      w.sink_tokens + w.recent_window, self.gt,
+                                      None if self.kv_ring else self.max_seq_len)
+        if full is None:
+            return False
+        self._pack_completed(full)
+        return True
 
     def append_decode_batched(self, slots: Sequence[int], K: torch.Tensor, V: torch.Tensor) -> int:
         """B new rows ``[B, H, D]`` in one launch, then one pack launch for every group that

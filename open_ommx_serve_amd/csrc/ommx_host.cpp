@@ -768,7 +768,7 @@ PyObject* py_ring_write(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const c10::Device dev = kh->device();
     const int64_t B = k->size(0), N = kh->size(0), rows = kh->size(1), H = kh->size(2), D = kh->size(3);
     if (k->size(1) != H || k->size(2) != D || k->scalar_type() != at::kBFloat16 ||
-        v->scalar_type() != at::kBFloat16 || k->stride(2) != 1 || v->stride(2) != 1 ||
+        v->scalar_type() != at::kBFloat16 || k->stride(2) != 1 || v->stride(2) != 1 || !on(k, dev) || !on(v, dev) ||
         !is_index(pos, dev, at::kLong, B) || !is_index(slots, dev, at::kLong, B) ||
         !is_index(next, dev, at::kLong, B) || (!slots && B > N))
         Py_RETURN_FALSE;
@@ -1049,6 +1049,84 @@ PyObject* py_upload(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Py_RETURN_TRUE;
 }
 
+// ── one step's host bookkeeping ────────────────────────────────────────────────────────────────
+// A decode step of short contexts is some 20 us of GPU time a layer; the loops over its requests and the calls around its
+// launches took longer than that in Python.  Plain lists of ints only: anything else is refused, and served by the
+// caller's own loops.
+
+// Whether slot slots[i] holds seqs[i] - behind tokens for all i: 1 yes, 0 no, -1 not plain lists.
+int all_at(PyObject* seq_len, PyObject* slots, PyObject* seqs, int64_t behind) {
+    if (!PyList_CheckExact(seq_len) || !PyList_CheckExact(slots) || !PyList_CheckExact(seqs) ||
+        PyList_GET_SIZE(slots) != PyList_GET_SIZE(seqs))
+        return -1;
+    bool ok = true, all = true;
+    for (Py_ssize_t i = 0; i < PyList_GET_SIZE(slots); ++i) {
+        const int64_t slot = as_int(PyList_GET_ITEM(slots, i), ok), seq = as_int(PyList_GET_ITEM(seqs, i), ok);
+        if (!ok || slot < 0 || slot >= PyList_GET_SIZE(seq_len)) return -1;
+        const int64_t held = as_int(PyList_GET_ITEM(seq_len, slot), ok);
+        if (!ok) return -1;
+        all = all && held == seq - behind;
+    }
+    return all;
+}
+
+// (seq_len, slots, seqs, behind)
+PyObject* py_all_at(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    bool ok = n == 4;
+    const int64_t behind = ok ? as_int(a[3], ok) : 0;
+    const int r = ok ? all_at(a[0], a[1], a[2], behind) : -1;
+    if (r < 0) Py_RETURN_NONE;
+    return PyBool_FromLong(r);
+}
+
+// (the arguments of ring_write without pos_next) + (seq_len, packed_groups, slots, seqs, kept rows, group_tokens, capacity or
+// None): one row of every request of a step appended to a pool that is one token behind it.  Returns the list of
+// (slot, first, end) of the groups that are complete with it (packed_groups is the caller's to move, once they are
+// packed), or None with nothing done.
+PyObject* py_append_rows(PyObject* self, PyObject* const* a, Py_ssize_t n) {
+    if (n != 16) { PyErr_SetString(PyExc_TypeError, "append_rows: wrong number of arguments"); return nullptr; }
+    bool ok = true;
+    const int64_t kept = as_int(a[13], ok), gt = as_int(a[14], ok), cap = a[15] == Py_None ? INT32_MAX : as_int(a[15], ok);
+    PyObject *const lens = a[9], *const packed = a[10], *const slots = a[11];
+    if (!ok || gt < 1 || all_at(lens, slots, a[12], 1) != 1 || !PyList_CheckExact(packed) ||
+        PyList_GET_SIZE(packed) != PyList_GET_SIZE(lens))
+        Py_RETURN_NONE;
+    const Py_ssize_t B = PyList_GET_SIZE(slots), N = PyList_GET_SIZE(lens);
+    const at::Tensor* k = as_tensor(a[3], ok);
+    if (!ok || k->dim() != 3 || k->size(0) != B) Py_RETURN_NONE;
+    struct One { int64_t slot, len, done; };
+    std::vector<One> step(static_cast<size_t>(B));
+    std::vector<bool> taken(static_cast<size_t>(N), false);
+    for (Py_ssize_t i = 0; i < B; ++i) {
+        One& s = step[i];
+        s.slot = as_int(PyList_GET_ITEM(slots, i), ok);
+        s.len = as_int(PyList_GET_ITEM(lens, s.slot), ok) + 1;
+        s.done = as_int(PyList_GET_ITEM(packed, s.slot), ok);
+        if (!ok || s.len > cap || taken[s.slot]) Py_RETURN_NONE;
+        taken[s.slot] = true;
+    }
+    PyObject* const ring[] = {a[0], a[1], a[2], a[3], a[4], a[5], a[6], a[7], Py_None, a[8]};
+    PyObject* launched = py_ring_write(self, ring, 10);
+    if (!launched) return nullptr;
+    const bool done = launched == Py_True;
+    Py_DECREF(launched);
+    if (!done) Py_RETURN_NONE;
+    PyObject* full = PyList_New(0);
+    for (Py_ssize_t i = 0; i < B && full; ++i) {
+        const One& s = step[i];
+        const int64_t past = s.len - kept, target = past >= 0 ? past / gt : 0;
+        PyObject* item = nullptr;
+        bool put = PyList_SetItem(lens, s.slot, PyLong_FromLongLong(s.len)) == 0;
+        if (put && target > s.done) {
+            item = Py_BuildValue("(LLL)", static_cast<long long>(s.slot), static_cast<long long>(s.done), static_cast<long long>(target));
+            put = item && PyList_Append(full, item) == 0;
+        }
+        Py_XDECREF(item);
+        if (!put) Py_CLEAR(full);
+    }
+    return full;
+}
+
 // C++ exceptions (out of memory among them) become the Python exceptions torch raises for them.
 template <PyObject* (*F)(PyObject*, PyObject* const*, Py_ssize_t)>
 PyObject* guarded(PyObject* self, PyObject* const* a, Py_ssize_t n) {
@@ -1061,6 +1139,7 @@ PyObject* guarded(PyObject* self, PyObject* const* a, Py_ssize_t n) {
 PyMethodDef methods[] = {
     OMMX_FAST(auto_num_kv_splits), OMMX_FAST(plain), OMMX_FAST(rows_fit),
     OMMX_FAST(decode), OMMX_FAST(decode_pool), OMMX_FAST(store_pack), OMMX_FAST(pack_block), OMMX_FAST(block_errors), OMMX_FAST(pack_groups), OMMX_FAST(pack_prompts), OMMX_FAST(ring_write),
+    OMMX_FAST(all_at), OMMX_FAST(append_rows),
     OMMX_FAST(tail_gather), OMMX_FAST(rows_write), OMMX_FAST(upload), OMMX_FAST(prefill),
     {nullptr, nullptr, 0, nullptr},
 };

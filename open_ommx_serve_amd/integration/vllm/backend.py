@@ -256,10 +256,20 @@ class OMMXCanonicalImpl(_ImplBase):
     # ── write ────────────────────────────────────────────────────────────────────
 
     def do_kv_cache_update(self, layer, key, value, kv_cache=None, slot_mapping=None) -> None:
+        s, st = _STATE, _STATE.step
+        m = s.bmanager
+        if m is not None and st["batched_write"] and m.decode_rows and not (m.dead or m.graph):
+            # one token of every request: one native call writes the rows and moves the cursors, if the layer's pool is
+            # where the scheduler's lengths say (else the general way, which names what is wrong)
+            pool = m.pools.get(id(layer))
+            append = getattr(pool, "append_step", None)
+            if append is not None:
+                step = m.step_on_device(pool)
+                if append(m.slots, m.seq_lens, step.sel, step.col, key, value):
+                    return
         n = int(key.shape[0])
         if n == 0:
             return
-        s, st = _STATE, _STATE.step
         cfg = self._ommx_cfg()
         H, D = self.num_kv_heads, self.head_size
         if not _hip.host().rows_fit(key, value, H, D):
@@ -502,7 +512,9 @@ class OMMXCanonicalImpl(_ImplBase):
             raise RuntimeError("[ommx] batched decode before any write reached this layer's pool")
         B = len(mgr.slots)
         # (a pool that is not at the scheduler's lengths is read at its own, below)
-        in_step = self._reads_what_was_stored() and [pool.seq_len[x] for x in mgr.slots] == mgr.seq_lens
+        in_step = self._reads_what_was_stored() and _hip.host().all_at(pool.seq_len, mgr.slots, mgr.seq_lens, 0)
+        if in_step is None:
+            in_step = [pool.seq_len[x] for x in mgr.slots] == mgr.seq_lens
         step = mgr.step_on_device(pool) if in_step else None
         if step is not None and pool.decode_into(
                 q if q.shape[0] == B else q[:B], out if out.shape[0] == B else out[:B], step.sel, step.cur, step.packed, step.tables, sm_scale=self.scale,

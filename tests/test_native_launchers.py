@@ -185,3 +185,42 @@ def test_prompts_of_several_requests_in_two_launches(H, D, kw, lens):
     rows = pools[2].k_hist.view(-1, H, D)
     assert not pools[2].append_prompts(slots, [0, *[x - 5 for x in starts[1:]]], rows, rows)
     assert before[0] == pools[2].seq_len and torch.equal(before[1], pools[2].k_hist)
+
+
+@pytest.mark.parametrize("ring", [False, True])
+def test_a_step_of_rows_and_cursors_in_one_call(ring):
+    """append_step against append_decode_batched over steps that complete groups; a slot that is not one token behind,
+    without room, named twice, or rows of another type or device are refused and nothing moves."""
+    H, D, win, lens = 2, 64, WindowSpec(), [70, 9, 103, 71]
+    pools = [MultiSeqKVPool(D, H, 6, 110, window=win, device=DEV, kv_ring=ring, **RECIPE) for _ in range(2)]
+    slots = [3, 0, 5, 2]
+    for i, (r, n) in enumerate(zip(slots, lens)):
+        K, V = _block(n, H, D, torch.bfloat16, 10 + i), _block(n, H, D, torch.bfloat16, 20 + i)
+        for p in pools:
+            p.append_block(r, K, V)
+    sel = torch.tensor(slots, device=DEV)
+    for s in range(1, 6):
+        K, V = _block(4, H, D, torch.bfloat16, 30 + s), _block(4, H, D, torch.bfloat16, 40 + s)
+        seqs = [n + s for n in lens]
+        cols = torch.tensor([n - 1 for n in seqs], device=DEV)
+        assert pools[0].append_step(slots, seqs, sel, cols, K, V)
+        pools[1].append_decode_batched(slots, K, V)
+        assert pools[0].seq_len == pools[1].seq_len and pools[0].packed_groups == pools[1].packed_groups
+        assert torch.equal(pools[0].k_hist[sel], pools[1].k_hist[sel]) and torch.equal(pools[0].v_hist[sel], pools[1].v_hist[sel])
+    for r in slots:
+        a, b = pools[0].request_planes(r), pools[1].request_planes(r)
+        for n in ("k_base", "k_scale", "k_obmp", "k_oval", "v_main", "v_scale"):
+            assert torch.equal(a[n], b[n]), (r, n)
+    held, hist = list(pools[0].seq_len), pools[0].k_hist.clone()
+    nxt = [n + 6 for n in lens]
+    cols = torch.tensor([n - 1 for n in nxt], device=DEV)
+    refused = [(slots, [n + 1 for n in nxt], K, V), (slots, [*nxt[:3], nxt[3] - 1], K, V), ([3, 0, 5, 5], [*nxt[:3], nxt[2]], K, V),
+               (slots, nxt, K.float(), V.float()), (slots, nxt, K.cpu(), V.cpu()), (slots, nxt, K[:3], V[:3]),
+               (tuple(slots), nxt, K, V), ([3, 0, 5, 9], nxt, K, V)]
+    for sl, sq, k, v in refused:
+        assert not pools[0].append_step(sl, sq, sel, cols, k, v)
+    if not ring:
+        pools[0].seq_len[5] = 110
+        assert not pools[0].append_step(slots, [nxt[0], nxt[1], 111, nxt[3]], sel, cols, K, V)
+        pools[0].seq_len[5] = held[5]
+    assert held == pools[0].seq_len and torch.equal(hist, pools[0].k_hist)
