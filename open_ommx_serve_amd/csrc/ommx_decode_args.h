@@ -40,8 +40,8 @@ struct DecodeArgs {
     // set by the launcher of the serving-recipe kernel only: head_dim is 64 and Hkv counts PAIRS of kv
     // heads (the planes of two neighbouring 64-channel heads read like one 128-channel head)
     int half;
-    // The tail rows attended by this launch (ommx_decode_tail.h): that many slices of the grid, 0 none.  Slices of x
-    // behind the splits, or of y in front of the shares.
+    // The tail rows attended by this launch (ommx_decode_tail.h): that many workgroups more per head group, 0 none, at the
+    // end of the grid: slices of z behind the requests, or of y behind the shares.
     int t_slices;
     DecodeTail t;
 };

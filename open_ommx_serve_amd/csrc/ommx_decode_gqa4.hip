@@ -192,12 +192,13 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
     const int qh0 = kvh * heads;
     const int r_half = max(heads >> 1, 1);            // head_dim 64: q heads per kv head of the pair
     if (TAIL) {
-        // slices of the grid that attend the bf16 tail rows (head_dim 64: of either kv head of the pair)
-        const int slice = dealt ? static_cast<int>(blockIdx.y) : static_cast<int>(blockIdx.x) - a.S;
-        if (slice >= 0 && slice < a.t_slices) {
-            const int part = slice & (kTailParts - 1), rest = slice / kTailParts;
-            const int tb = dealt ? (half ? rest >> 1 : rest) : static_cast<int>(blockIdx.z);
-            const int sub = half ? rest & 1 : 0;
+        // the last workgroups of the grid attend the bf16 tail rows (head_dim 64: of either kv head of the pair)
+        const int past = dealt ? static_cast<int>(blockIdx.y) - a.shares : static_cast<int>(blockIdx.z) - a.B;
+        if (past >= 0) {
+            const int at = dealt ? past : past * a.S + static_cast<int>(blockIdx.x);
+            if (at >= a.t_slices) return;
+            const int part = at & (kTailParts - 1), rest = at / kTailParts;
+            const int tb = half ? rest >> 1 : rest, sub = half ? rest & 1 : 0;
             if ((GEN || HALF) && half) tail::attend_part<NH, 64>(a, sm, tb, 2 * kvh + sub, heads >> 1, part, lane);
             else if (!HALF) tail::attend_part<NH, 128>(a, sm, tb, kvh, heads, part, lane);
             return;
@@ -207,7 +208,7 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
     int b = ORDER == 0 ? 0 : static_cast<int>(blockIdx.z), L;      // ORDER 0 is launched for one request only
     if (dealt) {
         shares::Share mine;
-        if (!shares::find_share<(1 << UNIT_SH), ORDER == 2 ? 4 : 1>(a, blockIdx.y - (TAIL ? a.t_slices : 0), lane, mine)) return;
+        if (!shares::find_share<(1 << UNIT_SH), ORDER == 2 ? 4 : 1>(a, blockIdx.y, lane, mine)) return;
         b = mine.b; L = mine.L; sp = mine.sp; S = mine.n;
         if (TAIL && sp == 0) {
             // the merge then goes by the lse alone: the slots this request does not use say that nothing was attended
@@ -1177,9 +1178,9 @@ int OMMX_GQA4_LAUNCH(const DecodeArgs& a_in, int Dh, int R, const DecodeTail* ta
     a.t_slices = 0;
     if (TAIL) {
         a.t = *tail;
-        a.t_slices = kTailParts * (a.half ? 2 : 1) * (a.shares > 0 ? a.B : 1);
+        a.t_slices = kTailParts * (a.half ? 2 : 1) * a.B;
     }
-    const dim3 grid = a.shares > 0 ? dim3(a.Hkv / waves, a.t_slices + a.shares) : dim3(a.S + a.t_slices, a.Hkv / waves, a.B);
+    const dim3 grid = a.shares > 0 ? dim3(a.Hkv / waves, a.shares + a.t_slices) : dim3(a.S, a.Hkv / waves, a.B + (a.t_slices + a.S - 1) / a.S);
     const dim3 block(64 * waves);
     const size_t shm = (size_t)waves * (longer ? (nh == 8 ? LdsMap<8, true>::LDS_WAVE : LdsMap<4, true>::LDS_WAVE)
                                               : (nh == 8 ? LdsMap<8, false>::LDS_WAVE : LdsMap<4, false>::LDS_WAVE));

@@ -2,12 +2,14 @@
 // the splits' own: a wave takes a quarter of the rows of one kv head.
 //
 // Attending them in the merge put their whole chain -- length, rows, logits, softmax, P.V -- behind the split-KV kernel,
-// where it was most of the merge's time; here it runs on compute units that the splits leave free, in less time than one
-// split takes, and the merge (fold_kernel) is left with one round of loads: 4.6-5.0 -> 3.0-3.7 us at 1 K, 8.0 -> 3.7 us for
-// 8 short requests over a row history, whose length and slot are two more dependent loads.  Whole call at 1 K
-// 12.0 -> 10.5 us, 3 requests of 0.7 to 9 K with one kv head 14.6 -> 13.0.  Four waves a kv head: the quarter's rows and
-// its 8 or 16 output channels fit registers, and the slowest wave stays below a lone split's 6.4 us.  A launch whose
-// splits fill every wave slot keeps the tail in the merge (its rows would wait for, or delay, a split).
+// where it was most of the merge's time.  Here the last workgroups of that launch do it: on compute units that short
+// splits leave free, and in full batches while the last shares run out (their waves end 3 us apart).  The merge
+// (fold_kernel) is left with one round of loads: 4.6-5.0 -> 3.0-3.7 us at 1 K, 8.0 -> 3.7 us for 8 short requests over a row
+// history, whose length and slot are two more dependent loads.  Whole call: 1 K 12.0 -> 10.5 us, 3 requests of 0.7 to 9 K
+// with one kv head 14.6 -> 13.0, 32 of 1 to 16 K 101.6 -> 98.9, 8 of 32 K with 64 q heads 107.5 -> 105.9, 16 of 2 to 16 K
+// with 64 q heads 75.8 -> 66.5.  In front of the shares, or only where slots are free, the full batches gain nothing.
+// Four waves a kv head: the quarter's rows and its 8 or 16 output channels fit registers, and the slowest wave stays
+// below a lone split's 6.4 us.
 //
 // Precision is that of an fp32 softmax: q.k of bf16 operands on the matrix cores is exact in its products and summed in
 // fp32, the weights stay fp32 and P.V runs on the vector ALU.

@@ -102,7 +102,7 @@ def test_shares_over_a_row_history(lens):
 def test_tail_rows_beside_the_splits(hq, hkv, D, kw, recent):
     """The tail in four parts as states of its own: no rows, fewer rows than parts, parts of one and of two blocks of 16
     and one row more, several passes of 32; one request (fixed splits) and many (shares); rows that cannot be read 16
-    bytes at a time, and a launch whose splits leave no room, take the other merge."""
+    bytes at a time take the other merge."""
     win = WindowSpec(recent_window=recent, group_tokens=kw.get("group_tokens", 32))
     for seqs in ([2000], [2000, 900, 3000, 700, 2500, 1500]):
         case = build_decode_case(seqs, q_heads=hq, kv_heads=hkv, head_dim=D, seed=91, permute_tables=True,
