@@ -493,7 +493,9 @@ __global__ void __launch_bounds__(512) combine_grouped_kernel(CombineArgs a) {
 // The merge when the tail rows are among the states (ommx_decode_tail.h): o = sum w_i o_i / sum w_i over `slots` states
 // of every (request, q head), w_i = exp(lse_i - max).  A workgroup takes CH channels of one head, LPR lanes a state
 // (four channels each); every wave reads all the lse and works the maximum and the sum of weights out for itself, so
-// that between the one round of loads and the output lie one exchange through LDS and no other wait.
+// that between the one round of loads and the output lie one exchange through LDS and no other wait.  Latency bound, or
+// with many heads by how many of them are under way: 32-bit offsets and 47 registers let eight waves a SIMD (as 64-bit
+// addresses it took 120 to 130: 48 requests of 64 q heads 80.5 us in all instead of 85, one of 1 K 9.6 instead of 10.2).
 // An unused slot has lse -inf, and what it holds is not multiplied.
 struct FoldArgs {
     const float* al; int64_t al_b, al_h, al_s;
@@ -503,17 +505,21 @@ struct FoldArgs {
     int slots, sure;
 };
 template <int D, int Q, int NT>
-__global__ void __launch_bounds__(NT) fold_kernel(FoldArgs a) {
+__global__ void __launch_bounds__(NT, 8) fold_kernel(FoldArgs a) {
     constexpr int CH = D / Q, LPR = CH / 4, ROWS = NT / LPR, NW = NT / 64;
     constexpr int FIRST = 6;                       // states per thread of the first round of loads, upper bound
     constexpr int NL = 9;                          // 512 splits and the tail's parts, 64 a register
-    static_assert(LPR == 16 || LPR == 32, "lane layout of the sums");
+    static_assert(LPR == 8 || LPR == 16 || LPR == 32, "lane layout of the sums");
     __shared__ float s_acc[NW][CH];
     const int b = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int c4 = tid % LPR, row = tid / LPR;
-    const float* const base = a.al + b * a.al_b + (int64_t)h * a.al_h + blockIdx.z * CH + 4 * c4;
-    const float* const sl = a.sl + b * a.sl_b + (int64_t)h * a.sl_h;
+    // (uniform bases, 32-bit offsets behind them: a head's states span less than a megabyte)
+    const char* const base = reinterpret_cast<const char*>(a.al + b * a.al_b + (int64_t)h * a.al_h + blockIdx.z * CH);
+    const char* const sl = reinterpret_cast<const char*>(a.sl + b * a.sl_b + (int64_t)h * a.sl_h);
+    const uint32_t al_s = static_cast<uint32_t>(a.al_s) * 4u, sl_s = static_cast<uint32_t>(a.sl_s) * 4u;
     typedef float f32x4 __attribute__((ext_vector_type(4)));
+    auto state = [&](int s) { return *reinterpret_cast<const f32x4*>(base + (static_cast<uint32_t>(s) * al_s + 16u * c4)); };
+    auto lse_of = [&](int s) { return *reinterpret_cast<const float*>(sl + static_cast<uint32_t>(s) * sl_s); };
     const int N = a.slots;
     const int n_first = min((a.sure + ROWS - 1) / ROWS, FIRST);
     f32x4 v[FIRST];
@@ -524,17 +530,23 @@ __global__ void __launch_bounds__(NT) fold_kernel(FoldArgs a) {
         my[i] = -INFINITY;
         if (i < n_first) {
             const int s = min(row + ROWS * i, N - 1);
-            v[i] = *reinterpret_cast<const f32x4*>(base + (int64_t)s * a.al_s);
-            my[i] = sl[(int64_t)s * a.sl_s];
+            v[i] = state(s);
+            my[i] = lse_of(s);
         }
     }
     float top = -INFINITY;
+    int used = 0;                                  // slots up to the last one that holds something
 #pragma unroll
     for (int k = 0; k < NL; ++k) {
         all[k] = -INFINITY;
+        if (64 * k < N) all[k] = lse_of(min(64 * k + lane, N - 1));
+    }
+#pragma unroll
+    for (int k = 0; k < NL; ++k) {
         if (64 * k < N) {
-            all[k] = sl[(int64_t)min(64 * k + lane, N - 1) * a.sl_s];
             if (64 * k + lane >= N) all[k] = -INFINITY;
+            const uint64_t live = __ballot(all[k] != -INFINITY);
+            if (live) used = 64 * k + 64 - __builtin_clzll(live);
         }
         top = fmaxf(top, all[k]);
     }
@@ -548,10 +560,18 @@ __global__ void __launch_bounds__(NT) fold_kernel(FoldArgs a) {
             if (w > 0.0f) acc += w * v[i];
         }
     }
-    for (int s = row + ROWS * n_first; s < N; s += ROWS) {
-        const float l = sl[(int64_t)s * a.sl_s];
-        const float w = l == -INFINITY ? 0.0f : __expf(l - safe);
-        if (w > 0.0f) acc += w * *reinterpret_cast<const f32x4*>(base + (int64_t)s * a.al_s);
+    for (int s0 = row + ROWS * n_first; s0 < used; s0 += 4 * ROWS) {
+        float w[4];
+        f32x4 x[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) w[u] = lse_of(min(s0 + ROWS * u, used - 1));
+#pragma unroll
+        for (int u = 0; u < 4; ++u) x[u] = state(min(s0 + ROWS * u, used - 1));
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            w[u] = w[u] == -INFINITY || s0 + ROWS * u >= used ? 0.0f : __expf(w[u] - safe);
+            if (w[u] > 0.0f) acc += w[u] * x[u];
+        }
     }
     float W = 0.0f;
 #pragma unroll
@@ -573,7 +593,9 @@ __global__ void __launch_bounds__(NT) fold_kernel(FoldArgs a) {
         s_acc[wave][c + 1] = hi;
     } else {
         const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(lo), __float_as_uint(hi), false, false);
-        s_acc[wave][c + ((lane >> 4) & 1)] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        float one = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        if (LPR == 8) one += dpp_of<0x128>(one);          // row_ror:8
+        s_acc[wave][c + ((lane >> 4) & 1)] = one;
     }
     __syncthreads();
     if (tid < CH) {
@@ -592,22 +614,29 @@ int fold_states(const float* al, int64_t al_b, int64_t al_h, int64_t al_s, const
                 void* o, bool o_bf16, int64_t o_b, int64_t o_h, float* lse, int64_t lse_b, int B, int Hq, int D,
                 void* stream) {
     if (B <= 0 || Hq <= 0 || slots < 1 || slots > 512 + kTailParts || (D != 64 && D != 128) || !al || !o || !lse || !states.p ||
-        (reinterpret_cast<uintptr_t>(al) & 15) || al_b % 4 || al_h % 4 || al_s % 4) {
+        (reinterpret_cast<uintptr_t>(al) & 15) || al_b % 4 || al_h % 4 || al_s % 4 || al_s < 0 || al_s > 4096 || states.s < 0 ||
+        states.s > 4096) {
         set_error("fold_states: bad shape or misaligned states");
         return -1;
     }
     const FoldArgs a{al, al_b, al_h, al_s, states.p, states.b, states.h, states.s, o_bf16 ? nullptr : static_cast<float*>(o),
                      o_bf16 ? static_cast<uint16_t*>(o) : nullptr, o_b, o_h, lse, lse_b, slots, std::min(std::max(sure, 1), slots)};
     hipStream_t st = static_cast<hipStream_t>(stream);
-    // Few heads: two workgroups each, as many lanes as the states keep busy.
-    const bool halves = D == 128 && B * Hq <= 512, few = slots <= 96;
-    const dim3 grid(B, Hq, halves ? 2 : 1);
-    if (halves && few) hipLaunchKernelGGL((fold_kernel<128, 2, 256>), grid, dim3(256), 0, st, a);
-    else if (halves) hipLaunchKernelGGL((fold_kernel<128, 2, 1024>), grid, dim3(1024), 0, st, a);
-    else if (D == 128 && few) hipLaunchKernelGGL((fold_kernel<128, 1, 256>), grid, dim3(256), 0, st, a);
-    else if (D == 128) hipLaunchKernelGGL((fold_kernel<128, 1, 1024>), grid, dim3(1024), 0, st, a);
-    else if (few) hipLaunchKernelGGL((fold_kernel<64, 1, 256>), grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((fold_kernel<64, 1, 1024>), grid, dim3(1024), 0, st, a);
+    // Small workgroups once there is one head per compute unit (48 requests of 32 q heads 53.5 us as one of 256 threads a head,
+    // 54.7 / 57.4 as two / four, 65 with 1024 threads); below that two a head, and with many states four of 512 threads, so
+    // that no thread has more than a few loads (one request of 64 K 31.7 us; 32.2 as two of 1024, 33.4 as two of 256).
+    const int heads = B * Hq;
+#define OMMX_FOLD(DD, Q, NT) hipLaunchKernelGGL((fold_kernel<DD, Q, NT>), dim3(B, Hq, Q), dim3(NT), 0, st, a)
+    if (slots <= 96) {
+        if (D == 64) OMMX_FOLD(64, 1, 256);
+        else if (heads < 256) OMMX_FOLD(128, 2, 256);
+        else OMMX_FOLD(128, 1, 256);
+    } else {
+        if (D == 64) OMMX_FOLD(64, 2, 512);
+        else if (heads < 256) OMMX_FOLD(128, 4, 512);
+        else OMMX_FOLD(128, 2, 512);
+    }
+#undef OMMX_FOLD
     if (hipGetLastError() != hipSuccess) { set_error("fold_states: launch failed"); return -2; }
     return 0;
 }
