@@ -9,6 +9,9 @@
 //   V: thread x owns the vector "token x/(D/32), channels 32*(x%(D/32))..+31".
 // The K codes of 4 neighbouring channels share a byte of k_base, so they are transposed
 // through LDS and written as 8-byte pieces of the token-major rows.
+// While all workgroups fit the chip at once a group takes two, one for K and one for V: each of the two jobs is a chain of
+// its own (loads, 0.9 to 1.4 us of one wave's arithmetic, a table look-up, stores), and the two of them one after the
+// other are the kernel's time there.
 #include <limits.h>
 
 #include "ommx_store_common.h"
@@ -35,12 +38,14 @@ __device__ __forceinline__ int med3_i32(int a, int b, int c) {
     return max(min(a, b), min(max(a, b), c));          // v_med3_i32
 }
 
-// IDXT: index plane known at compile time (0 bitmap, 1 relidx7) or read from the arguments (2)
-template <bool F32, bool FAST6, int IDXT>
+// IDXT: index plane known at compile time (0 bitmap, 1 relidx7) or read from the arguments (2).  APART: K and V of a group
+// in workgroups of their own (blockIdx.z); an instantiation, as the two tests in the other one cost a full chip 1 %.
+template <bool F32, bool FAST6, int IDXT, bool APART>
 // (six waves per SIMD for the tuned bitmask instantiation, which fits their 80 registers without spilling)
 __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_kernel(StoreArgs a) {
     static_assert(!(F32 && FAST6), "the tuned path reads bf16 input");
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const bool do_k = !APART || blockIdx.z == 0, do_v = !APART || blockIdx.z == 1;
     if (copied_row(a)) return;
     // head_dim 128 is compiled in for the tuned instantiations (their launch checks it): row offsets
     // of the code tile become instruction immediates
@@ -61,7 +66,7 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
     int err = 0;
 
     // ------------------------------------------------------------------ K vector
-    {
+    if (do_k) {
         const int d = tid;
         float w[32];
         bool fin = true;
@@ -337,7 +342,7 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
     __syncthreads();
 
     // nibble plane: D frames of nval bytes, contiguous in memory
-    if (kout > 0) {
+    if (do_k && kout > 0) {
         const int64_t obase = (gs * a.H + h) * (int64_t)D * nval;
         // (D is a multiple of 32 and the plane is 8-byte aligned: whole dwords)
         for (int w = tid; w < D * nval / 4; w += D)
@@ -358,19 +363,21 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
         const int64_t page = a.dst_pages ? a.dst_pages[lp] : lp;
         const int64_t prow = page * a.ps + (tok % a.ps);  // physical token row
 
-        // 32 code bytes -> 64 bits: four codes of a dword fold into its low byte
-        uint64_t kb8 = 0;
-        const uint4* cr = reinterpret_cast<const uint4*>(s_codes + t * D + 32 * j);
+        if (do_k) {
+            // 32 code bytes -> 64 bits: four codes of a dword fold into its low byte
+            uint64_t kb8 = 0;
+            const uint4* cr = reinterpret_cast<const uint4*>(s_codes + t * D + 32 * j);
 #pragma unroll
-        for (int q4 = 0; q4 < 2; ++q4) {
-            const uint4 u = cr[q4];
-            const uint32_t uw[4] = {u.x, u.y, u.z, u.w};
+            for (int q4 = 0; q4 < 2; ++q4) {
+                const uint4 u = cr[q4];
+                const uint32_t uw[4] = {u.x, u.y, u.z, u.w};
 #pragma unroll
-            for (int k = 0; k < 4; ++k)      // bytes (c0, c1, c2, c3) . (1, 4, 16, 64): one dot product per byte of the row
-                kb8 |= static_cast<uint64_t>(__builtin_amdgcn_udot4(uw[k], 0x40100401u, 0u, false)) << (8 * (4 * q4 + k));
+                for (int k = 0; k < 4; ++k)      // bytes (c0, c1, c2, c3) . (1, 4, 16, 64): one dot product per byte of the row
+                    kb8 |= static_cast<uint64_t>(__builtin_amdgcn_udot4(uw[k], 0x40100401u, 0u, false)) << (8 * (4 * q4 + k));
+            }
+            reinterpret_cast<uint64_t*>(a.k_base)[(prow * a.H + h) * NGV + j] = kb8;
         }
-        reinterpret_cast<uint64_t*>(a.k_base)[(prow * a.H + h) * NGV + j] = kb8;
-
+        if (do_v) {
         const int64_t row = a.src_rows ? a.src_rows[tok] : tok;
         const int64_t vbase = row * a.v_ts + (int64_t)h * a.v_hs + 32 * j;
         float v[32];
@@ -442,8 +449,9 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
         if (scale_mode == 0) a.v_scale[vidx] = static_cast<int8_t>(st.e);
         else reinterpret_cast<uint16_t*>(a.v_scale)[vidx] = st.bits;
         a.v_zp[vidx] = zp_b;
+        }
     }
-    write_own_tables(a, g, tid);
+    if (do_k) write_own_tables(a, g, tid);
     if (err && a.err) report_store_bits(a, err);
 }
 
@@ -468,6 +476,18 @@ extern "C" void ommx_store_default_table(float* t) {
         t[256 + j] = c;
     }
 }
+
+namespace ommx {
+template <bool APART>
+static void launch_store_pack(int variant, const StoreArgs& a, hipStream_t st) {
+    const dim3 grid(store_grid_x(a), a.H, APART ? 2 : 1), block(a.D);
+    const size_t shm = 32 * (size_t)a.D + 4 * (size_t)a.D + (a.idx_repr ? 8 * (size_t)a.D : 0);
+    if (variant == 0) hipLaunchKernelGGL((store_pack_kernel<true, false, 2, APART>), grid, block, shm, st, a);
+    else if (variant == 1) hipLaunchKernelGGL((store_pack_kernel<false, true, 0, APART>), grid, block, shm, st, a);
+    else if (variant == 2) hipLaunchKernelGGL((store_pack_kernel<false, true, 1, APART>), grid, block, shm, st, a);
+    else hipLaunchKernelGGL((store_pack_kernel<false, false, 2, APART>), grid, block, shm, st, a);
+}
+}  // namespace ommx
 
 int ommx::store_pack(const void* K, const void* V, int in_dtype,
                      int64_t k_ts, int64_t k_hs, int64_t v_ts, int64_t v_hs,
@@ -525,16 +545,9 @@ int ommx::store_pack(const void* K, const void* V, int in_dtype,
             return 0;
         }
     }
-    const dim3 grid(store_grid_x(a), H), block(D);
-    const size_t shm = 32 * (size_t)D + 4 * (size_t)D + (index_repr ? 8 * (size_t)D : 0);
-    if (in_dtype == 1)
-        hipLaunchKernelGGL((store_pack_kernel<true, false, 2>), grid, block, shm, st, a);
-    else if (tuned && index_repr == 0)
-        hipLaunchKernelGGL((store_pack_kernel<false, true, 0>), grid, block, shm, st, a);
-    else if (tuned)
-        hipLaunchKernelGGL((store_pack_kernel<false, true, 1>), grid, block, shm, st, a);
-    else
-        hipLaunchKernelGGL((store_pack_kernel<false, false, 2>), grid, block, shm, st, a);
+    const int variant = in_dtype == 1 ? 0 : !tuned ? 3 : index_repr == 0 ? 1 : 2;
+    if (store_apart(a)) launch_store_pack<true>(variant, a, st);
+    else launch_store_pack<false>(variant, a, st);
     if (hipGetLastError() != hipSuccess) { set_error("ommx_store_pack: launch failed"); return -2; }
     return 0;
 }

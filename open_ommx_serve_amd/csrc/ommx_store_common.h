@@ -47,9 +47,14 @@ struct StoreArgs {
 __device__ __forceinline__ bool copied_row(const StoreArgs& a) {
     if (static_cast<int>(blockIdx.x) < a.groups) return false;
     const int n = (static_cast<int>(blockIdx.x) - a.groups) * a.H + static_cast<int>(blockIdx.y);
-    if (n < a.rows.rows) copy_block_row<false>(a.rows, n);
+    if (n < a.rows.rows && blockIdx.z == 0) copy_block_row<false>(a.rows, n);
     return true;
 }
+// A workgroup each for K and V of a group and head?  Two against one, 8 heads: 5.4 against 6.4 us (32 tokens), 5.5 / 6.7 (1024), 8.4 / 10.0
+// (4096), 13.4 / 14.0 (8192), 22.4 / 22.4 (16384), 52.9 / 48.0 (32 K tokens into a pool); fp32 rows 24.8 / 26.7 (4096).  Past
+// the line the chip is full either way, and the second workgroup is only one more to start.
+constexpr int kStoreApart = 2048;
+inline bool store_apart(const StoreArgs& a) { return a.groups * static_cast<int64_t>(a.H) <= kStoreApart; }
 inline unsigned store_grid_x(const StoreArgs& a) { return a.groups + (a.rows.rows + a.H - 1) / a.H; }
 
 // Entries of the identity tables that belong to K group g: the pages that begin in it, and its own.

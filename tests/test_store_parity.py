@@ -513,3 +513,20 @@ def test_store_randomised_tie_patterns_signed_zeros_and_extremes():
                 _hip(K, V)
             continue
         assert_planes_equal(_hip(K, V), want, what=what, zero_sign_free=True)
+
+
+@pytest.mark.parametrize("rep", ["bitmap", "relidx7"])
+@pytest.mark.parametrize("fp32", [False, True])
+def test_store_in_one_and_in_two_workgroups_a_group(rep, fp32):
+    """2048 workgroups are the most that pack K and V apart: 65 groups of 32 heads take one each, their first 64 two, and
+    every byte is the same; the last group against the oracle."""
+    K, V = synth_kv(65 * 32, 32, 128, seed=77, sparse_frac=0.01)
+    if fp32:
+        K, V = K.float(), V.float()
+    whole, first = _hip(K, V, outlier_repr=rep), _hip(K[:2048], V[:2048], outlier_repr=rep)
+    names = [n for n in PLANE_NAMES if n != "k_obmp"] + ["k_obmp" if rep == "bitmap" else "k_oidx"]
+    last = O.pack_kv(K[2048:], V[2048:], outliers_per_vector=6, outlier_repr=rep)
+    for n in names:
+        got = bits_of(whole[n])
+        assert np.array_equal(got[:len(bits_of(first[n]))], bits_of(first[n])), n
+        assert np.array_equal(got[len(bits_of(first[n])):], bits_of(last[n])), n
