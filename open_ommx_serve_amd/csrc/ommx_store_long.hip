@@ -5,7 +5,12 @@
 // keeps the recipes left over (other outlier counts, largest-magnitude selection, bf16 steps, fp32 rows, bf16 V).
 //
 // One workgroup of 2 D threads packs one (K group, kv head): the first D threads own one channel each and do K, the
-// others take the V vectors meanwhile.  The K tile comes in by 16-byte loads through LDS, and both passes over a
+// others take the V vectors meanwhile: 16 bytes a lane with the lanes of a load side by side, so that a vector lies in 4, 8
+// or 16 neighbouring lanes, which exchange its extremes (DPP) and, one lane a vector, its step.  One thread a vector instead
+// touched 64 cache lines a load and read each of them eight times, more than L1 holds: 32 K tokens of 64 x 64 vectors into a
+// pool 76 -> 57 us, 1024 tokens 11.1 -> 9.9, 16 K tokens at head_dim 64 19.7 -> 17.8.  (The V rows are asked for when the K
+// tile is there and are on their way during the selection; asked for before it they delay it, 57 -> 61 us.)
+// The K tile comes in by 16-byte loads through LDS, and both passes over a
 // channel (selection, codes) are loops that read it there: held in registers and unrolled, 128 tokens overrun the
 // register file, and a straight-line body of 20-30 KB that every wave runs once is bound by instruction
 // fetch.  Selection is what remains: the general kernel runs k passes of 5 instructions per element over
@@ -14,6 +19,8 @@
 // element and leaves the extremes of what stays as its last ranks.  The outliers come out of the network by
 // rank and are wanted by position: each thread sorts them through its own few bytes of LDS.
 #include <limits.h>
+
+#include <utility>
 
 #include "ommx_store_common.h"
 
@@ -44,9 +51,35 @@ __device__ __forceinline__ void keep_smallest(int (&t)[N], int key) {
     t[0] = min(t[0], key);
 }
 
-// k_vec: K rows allow 16-byte loads
+// The minimum (or maximum) over the L neighbouring lanes of a vector, in all of them.
+template <int CTRL, class F>
+__device__ __forceinline__ float with_lane(float x, F f) {
+    return f(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, x), __builtin_bit_cast(int, x),
+                                                                      CTRL, 0xF, 0xF, false)));
+}
+template <int L, class F>
+__device__ __forceinline__ float over_vector(float x, F f) {
+    x = with_lane<0xB1>(x, f);                          // quad_perm [1,0,3,2]
+    x = with_lane<0x4E>(x, f);                          // quad_perm [2,3,0,1]
+    if constexpr (L >= 8) x = with_lane<0x141>(x, f);   // row_half_mirror
+    if constexpr (L >= 16) x = with_lane<0x140>(x, f);  // row_mirror
+    return x;
+}
+// The value of lane N of the vector's L lanes.
+template <int L, int N>
+__device__ __forceinline__ float lane_of_vector(float x) {
+    static_assert(L == 4 || L == 8 || L == 16, "lanes of a vector");
+    return __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, x), (N << 5) | (0x1F & ~(L - 1))));
+}
+template <int N, class F, int... I>
+__device__ __forceinline__ void each_of(F&& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
+template <int N, class F>
+__device__ __forceinline__ void each(F&& f) { each_of<N>(f, std::make_integer_sequence<int, N>{}); }
+
+// k_vec: K rows allow 16-byte loads.  As many waves a SIMD as the LDS of head_dim 128 allows: left alone, the compiler takes
+// 78 to 150 registers (32 K tokens into a pool 72 us instead of 61).
 template <int GT, int GC, int KH>
-__global__ void __launch_bounds__(512) store_long_kernel(StoreArgs a, int k_vec) {
+__global__ void __launch_bounds__(512, GT < GC ? 1 : GT == 32 ? 8 : GT == 64 ? 5 : 2) store_long_kernel(StoreArgs a, int k_vec) {
     constexpr int K = 2 * KH, MW = GT / 32, TIE = GT - 1;      // GT is a power of two: the tie breaker is its low bits
     constexpr int SORT = K <= 8 ? 8 : 12;                      // LDS bytes per thread and sorted list
     constexpr int NVAL = K / 2, NIDX = (7 * K + 7) / 8;
@@ -65,20 +98,40 @@ __global__ void __launch_bounds__(512) store_long_kernel(StoreArgs a, int k_vec)
     const float* __restrict__ tab = a.table;
     int err = 0;
     auto src_row = [&](int i) -> int64_t { return a.src_rows ? a.src_rows[g * GT + i] : (int64_t)g * GT + i; };
-    auto phys_row = [&](int tok) {
-        const int lp = tok / a.ps;
-        const int64_t page = a.dst_pages ? a.dst_pages[lp] : lp;
-        return page * a.ps + (tok % a.ps);
+    const int ps_log2 = __ffs(a.ps) - 1;                       // a divisor of GT: a power of two
+    auto page_of = [&](int row) {
+        const int lp = (g * GT + row) >> ps_log2;
+        return a.dst_pages ? a.dst_pages[lp] : lp;
     };
+    auto phys_row = [&](int page, int row) { return static_cast<int64_t>(page) * a.ps + (row & (a.ps - 1)); };
 
-    if (k_vec) {
-        const int per_row = D / 8;
-#pragma unroll 4
-        for (int i = tid; i < GT * per_row; i += NT) {
-            const int r = i / per_row, c = i % per_row;
-            const uint16_t* src = static_cast<const uint16_t*>(a.K) + src_row(r) * a.k_ts + (int64_t)h * a.k_hs + 8 * c;
-            *reinterpret_cast<uint4*>(s_k + r * D + 8 * c) = *reinterpret_cast<const uint4*>(src);
+    // V: piece v_piece (8 channels) of rows v_row, v_row + 8, ... of the group
+    constexpr int VP = GT / 8, VL = GC / 8;
+    const int v = tid - D, v_row = v / (D / 8), v_piece = v % (D / 8);
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    typedef u32x4 u32x4_a2 __attribute__((aligned(2)));      // V rows need not be 16-byte aligned
+    u32x4 vu[VP];
+    const uint16_t* const v_base = static_cast<const uint16_t*>(a.V) + (int64_t)h * a.v_hs + 8 * v_piece;
+    auto load_v = [&]() {
+        int row[VP];
+#pragma unroll
+        for (int n = 0; n < VP; ++n) row[n] = g * GT + 8 * n + v_row;
+        if (a.src_rows) {
+#pragma unroll
+            for (int n = 0; n < VP; ++n) row[n] = a.src_rows[row[n]];
         }
+#pragma unroll
+        for (int n = 0; n < VP; ++n) vu[n] = *reinterpret_cast<const u32x4_a2*>(v_base + row[n] * a.v_ts);
+    };
+    if (k_vec) {
+        constexpr int KP = GT / 16;                // 16-byte pieces of the K tile a thread: rows k_row, k_row + 16, ...
+        const int k_row = tid / (D / 8), c = 8 * (tid % (D / 8));
+        const uint16_t* const base = static_cast<const uint16_t*>(a.K) + (int64_t)h * a.k_hs + c;
+        uint4 ku[KP];
+#pragma unroll
+        for (int n = 0; n < KP; ++n) ku[n] = *reinterpret_cast<const uint4*>(base + src_row(16 * n + k_row) * a.k_ts);
+#pragma unroll
+        for (int n = 0; n < KP; ++n) *reinterpret_cast<uint4*>(s_k + (16 * n + k_row) * D + c) = ku[n];
     } else {
         for (int i = tid; i < GT * D; i += NT)
             s_k[i] = static_cast<const uint16_t*>(a.K)[src_row(i / D) * a.k_ts + (int64_t)h * a.k_hs + i % D];
@@ -248,69 +301,91 @@ __global__ void __launch_bounds__(512) store_long_kernel(StoreArgs a, int k_vec)
         }
     } else {
         // -------------------------------------------- V vectors (pack.py:604-623)
-        const int ngv = D / GC;
-        for (int it = tid - D; it < GT * ngv; it += D) {
-            const int tk = it / ngv, j = it % ngv, tok = g * GT + tk;
-            const int64_t prow = phys_row(tok);
-            const int64_t row = a.src_rows ? a.src_rows[tok] : tok;
-            const uint16_t* const vp = static_cast<const uint16_t*>(a.V) + row * a.v_ts + (int64_t)h * a.v_hs + GC * j;
-            // eight channels a turn, read again (from L1 / L2) by the second pass
-            auto eight = [&](int q) {
-                if (a.v_vec) return reinterpret_cast<const uint4*>(vp)[q];
-                const uint16_t* e = vp + 8 * q;
-                return uint4{e[0] | (static_cast<uint32_t>(e[1]) << 16), e[2] | (static_cast<uint32_t>(e[3]) << 16),
-                             e[4] | (static_cast<uint32_t>(e[5]) << 16), e[6] | (static_cast<uint32_t>(e[7]) << 16)};
-            };
+        load_v();
+        // (minimum and maximum of a piece, then of its vector in all VL lanes)
+        float mn[VP], mx[VP];
+        bool fin = true;                        // no exponent field of all ones
+#pragma unroll
+        for (int n = 0; n < VP; ++n) {
             typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-            u16x2 e2 = {0, 0};                    // largest exponent field: all ones when a value is not finite
-            float mn = bf16_to_f32(vp[0]), mx = mn;
-#pragma unroll 4
-            for (int q = 0; q < GC / 8; ++q) {
-                const uint4 u = eight(q);
-                const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+            const u32x4 w = vu[n];
+            u16x2 e2 = {0, 0};
+            mn[n] = mx[n] = __uint_as_float(w[0] << 16);
 #pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    const float lo = __uint_as_float(w[c] << 16), hi = __uint_as_float(w[c] & 0xFFFF0000u);
-                    mn = fminf(fminf(mn, lo), hi);
-                    mx = fmaxf(fmaxf(mx, lo), hi);
-                    e2 = __builtin_elementwise_max(e2, __builtin_bit_cast(u16x2, w[c] & 0x7F807F80u));
-                }
+            for (int c = 0; c < 4; ++c) {
+                const float lo = __uint_as_float(w[c] << 16), hi = __uint_as_float(w[c] & 0xFFFF0000u);
+                mn[n] = fminf(fminf(mn[n], lo), hi);
+                mx[n] = fmaxf(fmaxf(mx[n], lo), hi);
+                e2 = __builtin_elementwise_max(e2, __builtin_bit_cast(u16x2, w[c] & 0x7F807F80u));
             }
-            if (e2[0] == 0x7F80 || e2[1] == 0x7F80) err |= OMMX_ERR_NONFINITE_V;
-            const Step st = make_step(__fdiv_rn(fmaxf(mx - mn, 1e-8f), 3.0f), 0, tab);
-            if (!st.in_range) err |= OMMX_ERR_EXP_RANGE;
-            if (st.e > 15) err |= OMMX_NOTE_WIDE_STEP;
-            const uint16_t zp_b = f32_to_bf16_rne(mn);
-            const float zp = bf16_to_f32(zp_b), zc = -zp * st.inv;
-            const bool fused = st.inv_ok && fabsf(zc) < INFINITY;
-            uint16_t* const dst = reinterpret_cast<uint16_t*>(a.v_main + (prow * H + h) * (D / 4) + j * (GC / 4));
-#pragma unroll 4
-            for (int q = 0; q < GC / 8; ++q) {
-                const uint4 u = eight(q);
-                const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+            fin = fin && e2[0] != 0x7F80 && e2[1] != 0x7F80;
+            mn[n] = over_vector<VL>(mn[n], [](float x, float y) { return fminf(x, y); });
+            mx[n] = over_vector<VL>(mx[n], [](float x, float y) { return fmaxf(x, y); });
+        }
+        if (!fin) err |= OMMX_ERR_NONFINITE_V;
+        // Lane i of a vector's VL lanes works out the step of the vector of turn VL r + i, for all of them.
+        const int me = v % VL, ngv = D / GC;
+        int page[VP];
+#pragma unroll
+        for (int n = 0; n < VP; ++n) page[n] = page_of(8 * n + v_row);
+        auto code_word = [&](int pg, int row) -> uint16_t& {
+            return reinterpret_cast<uint16_t*>(a.v_main + (phys_row(pg, row) * H + h) * (D / 4))[v_piece];
+        };
+#pragma unroll
+        for (int r = 0; r < VP; r += VL) {
+            float my_mn = mn[r], my_mx = mx[r];
+#pragma unroll
+            for (int n = 1; n < VL && r + n < VP; ++n) {
+                my_mn = me == n ? mn[r + n] : my_mn;
+                my_mx = me == n ? mx[r + n] : my_mx;
+            }
+            const Step st = make_step(__fdiv_rn(fmaxf(my_mx - my_mn, 1e-8f), 3.0f), 0, tab);
+            const uint16_t zp_b = f32_to_bf16_rne(my_mn);
+            const float zc = -bf16_to_f32(zp_b) * st.inv;
+            if (r + me < VP) {
+                if (!st.in_range) err |= OMMX_ERR_EXP_RANGE;
+                if (st.e > 15) err |= OMMX_NOTE_WIDE_STEP;
+                const int64_t vidx = (phys_row(page_of(8 * (r + me) + v_row), 8 * (r + me) + v_row) * H + h) * ngv + v_piece / VL;
+                a.v_scale[vidx] = static_cast<int8_t>(st.e);
+                a.v_zp[vidx] = zp_b;
+            }
+            const float my_inv = st.inv_ok && fabsf(zc) < INFINITY ? st.inv : 0.0f;       // 0: the long way, below
+            each<(VP < VL ? VP : VL)>([&](auto turn) {
+                constexpr int n = decltype(turn)::value;
+                const int at = r + n;
+                const float inv = lane_of_vector<VL, n>(my_inv), c0 = lane_of_vector<VL, n>(zc);
+                const u32x4 w = vu[at];
                 uint32_t bits = 0;
-                if (fused) {
 #pragma unroll
-                    for (int f = 0; f < 2; ++f) {
-                        uint32_t four = 0;
+                for (int f = 0; f < 2; ++f) {
+                    uint32_t four = 0;
 #pragma unroll
-                        for (int c = 0; c < 4; ++c) {
-                            const uint32_t x = w[2 * f + (c >> 1)];
-                            const float v = __uint_as_float((c & 1) ? x & 0xFFFF0000u : x << 16);
-                            four = __builtin_amdgcn_cvt_pk_u8_f32(fminf(__builtin_fmaf(v, st.inv, zc), 3.0f), c, four);
-                        }
-                        bits |= __builtin_amdgcn_udot4(four, 0x40100401u, 0u, false) << (8 * f);
+                    for (int c = 0; c < 4; ++c) {
+                        const uint32_t x = w[2 * f + (c >> 1)];
+                        const float val = __uint_as_float((c & 1) ? x & 0xFFFF0000u : x << 16);
+                        four = __builtin_amdgcn_cvt_pk_u8_f32(fminf(__builtin_fmaf(val, inv, c0), 3.0f), c, four);
                     }
-                } else {
+                    bits |= __builtin_amdgcn_udot4(four, 0x40100401u, 0u, false) << (8 * f);
+                }
+                if (inv != 0.0f) code_word(page[at], 8 * at + v_row) = static_cast<uint16_t>(bits);
+                asm volatile("" : : : "memory");       // addresses of the next turn: in the next turn
+            });
+            if (__ballot(my_inv == 0.0f) != 0) {       // steps or zero points at the ends of the range: read again, one by one
+#pragma unroll 1
+                for (int n = 0; n < VL && r + n < VP; ++n) {
+                    const int from = (static_cast<int>(threadIdx.x) & 63 & ~(VL - 1)) + n, row = 8 * (r + n) + v_row;
+                    const float lo = __shfl(my_mn, from), hi = __shfl(my_mx, from), inv = __shfl(my_inv, from);
+                    if (inv != 0.0f) continue;
+                    const Step s1 = make_step(__fdiv_rn(fmaxf(hi - lo, 1e-8f), 3.0f), 0, tab);
+                    const float zp = bf16_to_f32(f32_to_bf16_rne(lo));
+                    const uint16_t* const e = v_base + src_row(row) * a.v_ts;
+                    uint32_t bits = 0;
 #pragma unroll 1
                     for (int c = 0; c < 8; ++c)
-                        bits |= int2_code(bf16_to_f32(vp[8 * q + c]) - zp, st.scale, st.inv, st.inv_ok) << (2 * c);
+                        bits |= int2_code(bf16_to_f32(e[c]) - zp, s1.scale, s1.inv, s1.inv_ok) << (2 * c);
+                    code_word(page_of(row), row) = static_cast<uint16_t>(bits);
                 }
-                dst[q] = static_cast<uint16_t>(bits);
             }
-            const int64_t vidx = (prow * H + h) * ngv + j;
-            a.v_scale[vidx] = static_cast<int8_t>(st.e);
-            a.v_zp[vidx] = zp_b;
         }
     }
     __syncthreads();
@@ -337,7 +412,7 @@ __global__ void __launch_bounds__(512) store_long_kernel(StoreArgs a, int k_vec)
             for (int q = 0; q < 4; ++q)
                 kb8 |= static_cast<uint64_t>(__builtin_amdgcn_udot4(uw[q], 0x40100401u, 0u, false)) << (8 * (4 * q4 + q));
         }
-        reinterpret_cast<uint64_t*>(a.k_base)[(phys_row(g * GT + tk) * H + h) * pieces + j] = kb8;
+        reinterpret_cast<uint64_t*>(a.k_base)[(phys_row(page_of(tk), tk) * H + h) * pieces + j] = kb8;
     }
 
     write_own_tables(a, g, tid);

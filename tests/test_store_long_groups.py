@@ -71,3 +71,24 @@ def test_long_group_store_reports_values_that_are_not_finite(gt, k, where, error
     with pytest.raises(error):
         ommx_pack_kv_canonical_block(K.cuda(), V.cuda(), outliers_per_vector=k, outlier_repr="relidx7",
                                      outlier_select="signed", use_pow2=True, group_tokens=gt)
+
+
+@pytest.mark.parametrize("gt,gc,D,k", [(32, 32, 64, 6), (32, 128, 128, 6), (64, 64, 192, 10), (64, 128, 256, 6), (64, 32, 32, 6),
+                                       (128, 32, 96, 10), (128, 128, 128, 6)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_v_vectors_of_any_alignment_and_range(gt, gc, D, k, shift):
+    """V vectors shared by several lanes: rows that are not 16-byte aligned, zero points so far from their step that the
+    code takes the two-step way, and denormal vectors, beside ordinary ones in the same wave."""
+    T, H = 2 * gt, 2
+    K, V = synth_kv(T, H, D, seed=gt + gc + D, sparse_frac=0.01)
+    V[1::5, 0, :gc] = 3e38                               # 2^-e * zero point overflows
+    V[2::7, 1, D - gc:] = torch.linspace(0, 6e-39, gc).to(torch.bfloat16)
+    V[3, :, :gc] = torch.tensor([-0.0, 0.0, 2e-38, -2e-38]).repeat(gc // 4).to(torch.bfloat16)
+    recipe = dict(outliers_per_vector=k, outlier_repr="relidx7", outlier_select="signed", use_pow2=True,
+                  group_tokens=gt, group_channels=gc)
+    want = O.pack_kv(K, V, **recipe)
+    wide_k, wide_v = (torch.zeros(T, H, D + 2 * shift, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    k_in, v_in = wide_k[:, :, shift:shift + D], wide_v[:, :, shift:shift + D]
+    k_in.copy_(K)
+    v_in.copy_(V)
+    _same(ommx_pack_kv_canonical_block(k_in, v_in, **recipe), want, _names(recipe))
