@@ -14,7 +14,10 @@
 // the history is kept whole and the slot is the position.
 //
 // Both kernels are pure row copies (H*D bf16 per row), 16 bytes per thread when rows are
-// 16-byte aligned, one workgroup per row.
+// 16-byte aligned, one workgroup per row.  A step's write is a few rows: its time is a launch and a chain of memory
+// latencies, so the new row is asked for beside its position (8 heads of 128: one piece of K or V a thread).
+#include <algorithm>
+
 #include "ommx_ring_args.h"
 #include "ommx_rows.h"
 
@@ -35,10 +38,19 @@ __device__ __forceinline__ void copy_row_in(uint16_t* dst, const uint16_t* src, 
     }
 }
 
-__global__ void __launch_bounds__(256) ring_write_kernel(
+__global__ void __launch_bounds__(1024) ring_write_kernel(
     RingArgs a, const uint16_t* k, const uint16_t* v, int64_t k_bs, int64_t k_hs, int64_t v_bs,
     int64_t v_hs, const int64_t* pos, int64_t* pos_next, int vec) {
     const int b = blockIdx.x;
+    // pieces of eight: those of K, then those of V
+    const int per_head = a.D / 8, pieces = a.H * per_head;
+    auto piece = [&](int i) {
+        const bool is_v = i >= pieces;
+        const int n = is_v ? i - pieces : i, h = n / per_head, c = (n - h * per_head) * 8;
+        return *reinterpret_cast<const uint4*>((is_v ? v + b * v_bs + h * v_hs : k + b * k_bs + h * k_hs) + c);
+    };
+    uint4 first = {};
+    if (vec && static_cast<int>(threadIdx.x) < 2 * pieces) first = piece(threadIdx.x);
     const int64_t p = pos[b];
     const int64_t slot = a.slots ? a.slots[b] : b;
     const int64_t row = ring_slot(p, a.sink, a.span);
@@ -49,8 +61,15 @@ __global__ void __launch_bounds__(256) ring_write_kernel(
         return;
     }
     const int64_t off = slot * a.req_stride + row * (int64_t)(a.H * a.D);
-    copy_row_in(a.k_hist + off, k + b * k_bs, k_hs, a.H, a.D, vec);
-    copy_row_in(a.v_hist + off, v + b * v_bs, v_hs, a.H, a.D, vec);
+    if (vec) {
+        for (int i = threadIdx.x; i < 2 * pieces; i += blockDim.x) {
+            const uint4 x = i == static_cast<int>(threadIdx.x) ? first : piece(i);
+            reinterpret_cast<uint4*>((i < pieces ? a.k_hist : a.v_hist) + off)[i < pieces ? i : i - pieces] = x;
+        }
+        return;
+    }
+    copy_row_in(a.k_hist + off, k + b * k_bs, k_hs, a.H, a.D, false);
+    copy_row_in(a.v_hist + off, v + b * v_bs, v_hs, a.H, a.D, false);
 }
 
 __global__ void __launch_bounds__(256) tail_gather_kernel(
@@ -109,7 +128,8 @@ int launch_ring_write(const RingArgs& a, const uint16_t* k, const uint16_t* v, i
     const int vec = a.D % 8 == 0 && aligned16(a.k_hist) && aligned16(a.v_hist) && aligned16(k) &&
                     aligned16(v) && a.req_stride % 8 == 0 && k_bs % 8 == 0 && k_hs % 8 == 0 &&
                     v_bs % 8 == 0 && v_hs % 8 == 0;
-    const int threads = (a.H * a.D / (vec ? 8 : 1)) >= 256 ? 256 : 128;
+    const int pieces = a.H * a.D / (vec ? 4 : 1);        // of K and V, or elements of one of them
+    const int threads = vec ? std::min((pieces + 63) / 64 * 64, 1024) : (pieces >= 256 ? 256 : 128);
     hipLaunchKernelGGL(ring_write_kernel, dim3(B), dim3(threads), 0, st, a, k, v, k_bs, k_hs, v_bs,
                        v_hs, pos, pos_next, vec);
     return 0;

@@ -8,7 +8,9 @@ namespace ommx {
 
 __device__ __forceinline__ int64_t ring_slot(int64_t pos, int sink, int span) {
     if (span <= 0 || pos < sink) return pos;
-    return sink + (pos - sink) % span;
+    const int64_t past = pos - sink;
+    if (past >> 32 == 0) return sink + static_cast<uint32_t>(past) % static_cast<uint32_t>(span);    // a third of the steps
+    return sink + past % span;
 }
 
 template <bool F32>

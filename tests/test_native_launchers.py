@@ -224,3 +224,19 @@ def test_a_step_of_rows_and_cursors_in_one_call(ring):
         assert not pools[0].append_step(slots, [nxt[0], nxt[1], 111, nxt[3]], sel, cols, K, V)
         pools[0].seq_len[5] = held[5]
     assert held == pools[0].seq_len and torch.equal(hist, pools[0].k_hist)
+
+
+@pytest.mark.parametrize("H,D", [(1, 8), (3, 40), (8, 128), (16, 256), (32, 256), (7, 12)])
+def test_rows_of_any_width_reach_their_slot(H, D):
+    """One piece of K or V a thread up to 1024 of them, several beyond, and rows without 16-byte pieces; positions past 32
+    bits turn with the ring."""
+    sink, span = 4, 24
+    kh, vh = (torch.zeros(2, sink + span, H, D, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    for pos in ([3, 4], [27, 28], [2 ** 33 + 5, 2 ** 32 + 3]):
+        K, V = _block(2, H, D, torch.bfloat16, pos[0] % 97), _block(2, H, D, torch.bfloat16, 7)
+        at = torch.tensor(pos, dtype=torch.int64, device=DEV)
+        assert _hip.host().ring_write(kh, vh, at, K, V, sink, span, None, at, None)
+        assert at.tolist() == [p + 1 for p in pos]
+        for b, p in enumerate(pos):
+            slot = p if p < sink else sink + (p - sink) % span
+            assert torch.equal(kh[b, slot], K[b]) and torch.equal(vh[b, slot], V[b])
