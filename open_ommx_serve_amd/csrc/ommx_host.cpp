@@ -875,11 +875,30 @@ PyObject* py_pack_groups(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const c10::Device dev = kh->device();
     c10::hip::HIPGuard guard(dev.index());
     hipStream_t stream = stream_of(dev);
+    const at::Tensor K = kh->view({N * rows, kh->size(2), kh->size(3)}), V = vh->view({N * rows, kh->size(2), kh->size(3)});
+    int rc = 1;
+    // the groups as arguments of the store launch, where its kernel takes them: rows that turn around at most once
+    if (count <= ommx::kRingGroups && N * rows <= INT32_MAX && N * per_seq <= INT32_MAX && (span == 0 || (wsink >= sink && span >= r.gt))) {
+        ommx::RingGroups ring;
+        for (int64_t i = 0; i < count; ++i) {
+            const int64_t pos = wsink + pairs64[2 * i + 1] * r.gt, slot = span > 0 ? sink + (pos - sink) % span : pos;
+            ring.of[i] = {static_cast<int32_t>(pairs64[2 * i] * rows + slot), span > 0 ? static_cast<int32_t>(sink + span - slot) : INT32_MAX,
+                          static_cast<int32_t>(pairs64[2 * i] * per_seq + pairs64[2 * i + 1])};
+        }
+        ommx::StoreExtras extras;
+        extras.ring = &ring;
+        extras.ring_span = static_cast<int>(span);
+        Py_BEGIN_ALLOW_THREADS
+        rc = launch_store(K, V, 0, p, r, count * r.gt, ps, nullptr, nullptr, nullptr, *table, data<int32_t>(err), extras, stream);
+        Py_END_ALLOW_THREADS
+        if (rc != 1) {
+            if (failed(rc, "ommx_store_pack")) return nullptr;
+            Py_RETURN_TRUE;
+        }
+    }
     // index tables: stream-ordered scratch, given back to torch's allocator when this call returns
     c10::DataPtr scratch = c10::GetAllocator(c10::DeviceType::CUDA)->allocate(count * (r.gt + ppg + 1) * sizeof(int32_t));
     int32_t *src = static_cast<int32_t*>(scratch.get()), *pages = src + count * r.gt, *groups = pages + count * ppg;
-    const at::Tensor K = kh->view({N * rows, kh->size(2), kh->size(3)}), V = vh->view({N * rows, kh->size(2), kh->size(3)});
-    int rc;
     Py_BEGIN_ALLOW_THREADS
     rc = ommx::pack_list(pairs.data(), count, src, pages, groups, r.gt, ppg, rows, sink, span, wsink, per_seq,
                          per_seq * ppg, stream);

@@ -28,11 +28,19 @@ inline BlockRows block_rows(const void* K, const void* V, bool k_f32, bool v_f32
             n_head, lo, H, D, sink, span, n_head + (T - lo)};
 }
 
+// Groups whose rows lie in a ring history, as arguments of the store launch: the first row of each (of the flat history),
+// the token at which its rows continue at the start of the ring (32 or more: none does), its destination.
+struct RingGroup { int32_t row, turn, group; };
+constexpr int kRingGroups = 96;
+struct RingGroups { RingGroup of[kRingGroups]; };
+
 // What a store launch of the native launchers does besides packing.
 struct StoreExtras {
     bool err_words = false;               // err_flag is an array of OMMX_STORE_ERR_WORDS host-visible ints, one per error bit
     int32_t *own_pages = nullptr, *own_groups = nullptr;      // identity tables [T / page_size], [T / group_tokens] to
                                                               // fill (both or neither)
+    const RingGroups* ring = nullptr;     // where the groups lie; T / 32 of them, span rows in the ring.  store_pack returns 1,
+    int ring_span = 0;                    // with nothing launched, for a recipe or a number of groups that needs the tables
     const BlockRows* rows = nullptr;      // bf16 rows to copy into the history (head_dim a multiple of 8, every slot inside it)
 };
 

@@ -14,6 +14,8 @@
 // other are the kernel's time there.
 #include <limits.h>
 
+#include <type_traits>
+
 #include "ommx_store_common.h"
 
 namespace ommx {
@@ -40,9 +42,12 @@ __device__ __forceinline__ int med3_i32(int a, int b, int c) {
 
 // IDXT: index plane known at compile time (0 bitmap, 1 relidx7) or read from the arguments (2).  APART: K and V of a group
 // in workgroups of their own (blockIdx.z); an instantiation, as the two tests in the other one cost a full chip 1 %.
-template <bool F32, bool FAST6, int IDXT, bool APART>
+// RING: the groups come as arguments, rows in a ring history and destinations by group; completed groups of a decode step
+// need no tables written by a launch before (pack_list, 1.4 us and its gap).
+struct NoRing {};
+template <bool F32, bool FAST6, int IDXT, bool APART, bool RING = false>
 // (six waves per SIMD for the tuned bitmask instantiation, which fits their 80 registers without spilling)
-__global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_kernel(StoreArgs a) {
+__global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_kernel(StoreArgs a, std::conditional_t<RING, RingGroups, NoRing> ring) {
     static_assert(!(F32 && FAST6), "the tuned path reads bf16 input");
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const bool do_k = !APART || blockIdx.z == 0, do_v = !APART || blockIdx.z == 1;
@@ -57,7 +62,9 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
     const int NGV = D >> 5;
     const int kout = a.kout, kt = (kout + 1) >> 1, kb = kout - kt;
     const int nval = (kout + 1) >> 1;              // nibble bytes per frame
-    const int64_t gs = a.dst_groups ? a.dst_groups[g] : g;
+    RingGroup from = {0, INT_MAX, 0};
+    if constexpr (RING) from = ring.of[g];
+    const int64_t gs = RING ? from.group : a.dst_groups ? a.dst_groups[g] : g;
     const float* __restrict__ tab = a.table;
     // the tuned instantiation serves the serving recipe only: its variants are compile-time there
     const int scale_mode = FAST6 ? 0 : a.scale_mode;
@@ -70,7 +77,7 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
         const int d = tid;
         float w[32];
         bool fin = true;
-        if (a.src_rows) {
+        if (!RING && a.src_rows) {
 #pragma unroll
             for (int i = 0; i < 32; ++i) {
                 const int64_t row = a.src_rows[g * 32 + i];
@@ -82,7 +89,7 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
             // the 32 loads
             typedef const __attribute__((address_space(1))) char* gptr;      // a global-memory address
             uint64_t row = reinterpret_cast<uint64_t>(a.K) +
-                           static_cast<uint64_t>(((int64_t)g * 32 * a.k_ts + (int64_t)h * a.k_hs) * (F32 ? 4 : 2));
+                           static_cast<uint64_t>(((RING ? from.row : (int64_t)g * 32) * a.k_ts + (int64_t)h * a.k_hs) * (F32 ? 4 : 2));
             const uint64_t stride = static_cast<uint64_t>(a.k_ts * (F32 ? 4 : 2));
             const uint32_t off = static_cast<uint32_t>(d) * (F32 ? 4u : 2u);
 #pragma unroll
@@ -90,6 +97,7 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
                 if (F32) w[i] = *reinterpret_cast<const __attribute__((address_space(1))) float*>(reinterpret_cast<gptr>(row) + off);
                 else w[i] = bf16_to_f32(*reinterpret_cast<const __attribute__((address_space(1))) uint16_t*>(reinterpret_cast<gptr>(row) + off));
                 row += stride;
+                if (RING && i + 1 == from.turn) row -= stride * static_cast<uint64_t>(a.ring_span);
                 asm volatile("" : "+s"(row));        // keeps the row address a scalar of its own: folded into one
                                                      // vector expression it costs four vector instructions a load
             }
@@ -361,7 +369,7 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
         const int tok = g * 32 + t;
         const int lp = tok / a.ps;
         const int64_t page = a.dst_pages ? a.dst_pages[lp] : lp;
-        const int64_t prow = page * a.ps + (tok % a.ps);  // physical token row
+        const int64_t prow = RING ? gs * 32 + t : page * a.ps + (tok % a.ps);  // physical token row
 
         if (do_k) {
             // 32 code bytes -> 64 bits: four codes of a dword fold into its low byte
@@ -378,7 +386,7 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
             reinterpret_cast<uint64_t*>(a.k_base)[(prow * a.H + h) * NGV + j] = kb8;
         }
         if (do_v) {
-        const int64_t row = a.src_rows ? a.src_rows[tok] : tok;
+        const int64_t row = RING ? from.row + t - (t >= from.turn ? a.ring_span : 0) : a.src_rows ? a.src_rows[tok] : tok;
         const int64_t vbase = row * a.v_ts + (int64_t)h * a.v_hs + 32 * j;
         float v[32];
         bool fin = true;
@@ -482,10 +490,16 @@ template <bool APART>
 static void launch_store_pack(int variant, const StoreArgs& a, hipStream_t st) {
     const dim3 grid(store_grid_x(a), a.H, APART ? 2 : 1), block(a.D);
     const size_t shm = 32 * (size_t)a.D + 4 * (size_t)a.D + (a.idx_repr ? 8 * (size_t)a.D : 0);
-    if (variant == 0) hipLaunchKernelGGL((store_pack_kernel<true, false, 2, APART>), grid, block, shm, st, a);
-    else if (variant == 1) hipLaunchKernelGGL((store_pack_kernel<false, true, 0, APART>), grid, block, shm, st, a);
-    else if (variant == 2) hipLaunchKernelGGL((store_pack_kernel<false, true, 1, APART>), grid, block, shm, st, a);
-    else hipLaunchKernelGGL((store_pack_kernel<false, false, 2, APART>), grid, block, shm, st, a);
+    if (variant == 0) hipLaunchKernelGGL((store_pack_kernel<true, false, 2, APART>), grid, block, shm, st, a, NoRing{});
+    else if (variant == 1) hipLaunchKernelGGL((store_pack_kernel<false, true, 0, APART>), grid, block, shm, st, a, NoRing{});
+    else if (variant == 2) hipLaunchKernelGGL((store_pack_kernel<false, true, 1, APART>), grid, block, shm, st, a, NoRing{});
+    else hipLaunchKernelGGL((store_pack_kernel<false, false, 2, APART>), grid, block, shm, st, a, NoRing{});
+}
+static void launch_store_ring(const StoreArgs& a, const RingGroups& ring, hipStream_t st) {
+    const dim3 grid(store_grid_x(a), a.H, 2), block(a.D);
+    const size_t shm = 36 * (size_t)a.D + (a.idx_repr ? 8 * (size_t)a.D : 0);
+    if (a.idx_repr == 0) hipLaunchKernelGGL((store_pack_kernel<false, true, 0, true, true>), grid, block, shm, st, a, ring);
+    else hipLaunchKernelGGL((store_pack_kernel<false, true, 1, true, true>), grid, block, shm, st, a, ring);
 }
 }  // namespace ommx
 
@@ -531,10 +545,16 @@ int ommx::store_pack(const void* K, const void* V, int in_dtype,
                 err_flag, H, D, page_size, k_outliers,
                 (reinterpret_cast<uintptr_t>(V) % 16 == 0 && v_ts % 8 == 0 && v_hs % 8 == 0) ? 1 : 0,
                 index_repr, select_abs ? 1 : 0, scale_mode, gt, gc, v_bf16 ? 1 : 0, extras.err_words ? 1 : 0,
-                extras.own_pages, extras.own_groups, T / gt, extras.rows ? *extras.rows : BlockRows{}};
+                extras.own_pages, extras.own_groups, extras.ring_span, T / gt, extras.rows ? *extras.rows : BlockRows{}};
     hipStream_t st = static_cast<hipStream_t>(stream);
     const bool tuned = k_outliers == 6 && !select_abs && scale_mode == 0 && k_ms && D == 128 && gt == 32 && gc == 32 &&
                        32 % page_size == 0 && !v_bf16 && in_dtype == 0;   // the serving recipe
+    if (extras.ring) {
+        if (!tuned || !store_apart(a) || a.groups > kRingGroups) return 1;
+        launch_store_ring(a, *extras.ring, st);
+        if (hipGetLastError() != hipSuccess) { set_error("ommx_store_pack: launch failed"); return -2; }
+        return 0;
+    }
     if (!tuned) {
         int rc = launch_store_long(a, T, in_dtype, st);
         if (rc == 1 && (gt != 32 || gc != 32 || k_outliers > 8 || 32 % page_size || v_bf16))

@@ -38,6 +38,7 @@ struct StoreArgs {
                             // word of bits: the bus has no atomic OR, a store of 1 per bit needs none
     int32_t *own_pages, *own_groups;      // with a block of its own: its identity tables, written on the way instead of by a
                                           // launch of their own (4096-token block, whole call: 33.4 -> 31.9 us)
+    int ring_span;          // rows of the ring the groups lie in (RingGroups)
     int groups;             // T / gt; workgroups beyond them copy rows into the history (bf16), H rows per blockIdx.x
     BlockRows rows;
 };

@@ -7,7 +7,7 @@ import torch
 import oracle.ommx_oracle as O
 from open_ommx_serve_amd.attention import MultiSeqKVPool, WindowSpec, _hip, ommx_pack_kv_canonical_block
 from open_ommx_serve_amd.attention.kv_store_ops import ring_slot
-from open_ommx_serve_amd.attention.pack import store_table
+from open_ommx_serve_amd.attention.pack import alloc_planes, store_pack_into, store_table
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -224,6 +224,42 @@ def test_a_step_of_rows_and_cursors_in_one_call(ring):
         assert not pools[0].append_step(slots, [nxt[0], nxt[1], 111, nxt[3]], sel, cols, K, V)
         pools[0].seq_len[5] = held[5]
     assert held == pools[0].seq_len and torch.equal(hist, pools[0].k_hist)
+
+
+@pytest.mark.parametrize("sink,span,wsink,count,H,ps", [
+    (0, 0, 8, 3, 8, 16), (8, 96, 8, 3, 8, 16),            # whole history; groups that end where the ring turns
+    (8, 83, 8, 2, 3, 8), (8, 41, 13, 1, 8, 32),           # groups that turn with it
+    (8, 96, 8, 96, 2, 16), (8, 96, 8, 97, 2, 16), (0, 0, 8, 30, 70, 16)])   # as arguments, and through the tables
+@pytest.mark.parametrize("rep", ["bitmap", "relidx7"])
+def test_groups_of_a_history_as_arguments_of_their_store(sink, span, wsink, count, H, ps, rep):
+    """pack_groups against the general entry with index tables, for the newest groups of many requests."""
+    D, gt, per_seq, rows = 128, 32, 9, sink + span if span else 300
+    g = torch.Generator(device=DEV).manual_seed(count + span)
+    kh, vh = (torch.randn(count, rows, H, D, generator=g, device=DEV).to(torch.bfloat16) for _ in range(2))
+    pairs = [(r, (5 * r + 3) % per_seq) for r in range(count)]
+    pos = [[wsink + n * gt + i for i in range(gt)] for _, n in pairs]
+    src = [r * rows + (ring_slot(p, sink, span) if span else p) for (r, _), ps_ in zip(pairs, pos) for p in ps_]
+    pages = [(r * per_seq + n) * (gt // ps) + i for r, n in pairs for i in range(gt // ps)]
+    groups = [r * per_seq + n for r, n in pairs]
+    how = dict(outliers_per_vector=6, outlier_repr=rep)
+    planes = [alloc_planes(count * per_seq * (gt // ps), count * per_seq, H, D, page_size=ps, device=DEV, **how) for _ in range(2)]
+    for p in planes:
+        for t in p.values():
+            if torch.is_tensor(t):
+                t.fill_(0x5A if t.dtype == torch.uint8 else 1)
+    names = [n for n, t in planes[0].items() if torch.is_tensor(t)]
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    store_pack_into(kh.view(-1, H, D), vh.view(-1, H, D), planes[0], page_size=ps, src_rows=i32(src), dst_pages=i32(pages),
+                    dst_groups=i32(groups), **how)
+    err = torch.zeros(1, dtype=torch.int32, device=DEV)
+    assert _hip.host().pack_groups(kh, vh, {n: planes[1].get(n) for n in ("k_base", "k_scale", "k_zp", "k_fp4_mapscale",
+                                                                         "k_fp4_mapcenter", "k_obmp", "k_oidx", "k_oval",
+                                                                         "v_main", "v_scale", "v_zp")},
+                                   [x for pair in pairs for x in pair], ps, sink, span, wsink, per_seq, err,
+                                   store_table(kh.device), 6, gt, 32, rep, "signed", True, True, "i2")
+    assert int(err.item()) == 0
+    for n in names:
+        assert torch.equal(planes[0][n].view(torch.uint8), planes[1][n].view(torch.uint8)), n
 
 
 @pytest.mark.parametrize("H,D", [(1, 8), (3, 40), (8, 128), (16, 256), (32, 256), (7, 12)])
