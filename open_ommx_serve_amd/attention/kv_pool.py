@@ -266,6 +266,12 @@ class MultiSeqKVPool:
         if not self.kv_ring:
             if s + T > self.max_seq_len:
                 raise RuntimeError(f"MultiSeqKVPool req {r} capacity {self.max_seq_len} exceeded")
+            target = self.window.num_groups(T) if s == 0 and self.packed_groups[r] == 0 else 0
+            if target and K.shape == V.shape and K.dtype == V.dtype == torch.bfloat16:     # a fresh slot: rows and groups in one launch
+                if not self._pack_block_into_pool(r, K, V, 0, target, row0=self.window.sink_tokens, live=(0, 0)):
+                    self._write_rows(r, K, V, 0, 0, 0)
+                self.seq_len[r], self.packed_groups[r] = T, target
+                return target
             self._write_rows(r, K, V, s, 0, 0)
             self.seq_len[r] = s + T
             return self.regroup(r)
@@ -483,7 +489,7 @@ class MultiSeqKVPool:
                               row0: int = 0, live: Optional[Tuple[int, int]] = None) -> bool:
         """Pack the ``(g1-g0)*gt`` tokens from row ``row0`` of a source block into request ``req``'s group /
         page slots ``[g0, g1)`` with one store launch (kv_pool.py:677-734).  ``live = (n_head, lo)``: the same
-        launch may write the block's rows ``[0, n_head)`` and ``[lo, T)`` into the ring; True when it has."""
+        launch may write the block's rows ``[0, n_head)`` and ``[lo, T)`` into the history; True when it has."""
         r = int(req)
         n_tok = (g1 - g0) * self.gt
         if row0 + n_tok > int(K.shape[0]) or row0 + n_tok > int(V.shape[0]):

@@ -243,6 +243,14 @@ class CanonicalKVStore:
         if not self.kv_ring:
             if self.seq_len + T > self.kv_cap:
                 raise RuntimeError("CanonicalKVStore capacity exceeded (block)")
+            target = self.window.num_groups(T) if self.seq_len == 0 and self.packed_groups == 0 else 0
+            if (target and K.shape == V.shape == (T, self.H, self.D) and K.dtype == V.dtype == torch.bfloat16
+                    and K.device == V.device == self.device):
+                # a fresh sequence: rows and groups in one launch
+                if not self._pack_block_into_planes(K, V, 0, target, row0=self.window.sink_tokens, live=(0, 0)):
+                    self._write_rows(K, V, 0, 0, 0)
+                self.seq_len, self.packed_groups = T, target
+                return
             self._write_rows(K, V, self.seq_len, 0, 0)
             self.seq_len += T
             self.maybe_regroup()
@@ -300,15 +308,20 @@ class CanonicalKVStore:
         self._pack_block_into_planes(self.k_hist, self.v_hist, g0, g1, src_rows=rows)
 
     def _pack_block_into_planes(self, K: torch.Tensor, V: torch.Tensor, g0: int, g1: int, *, row0: int = 0,
-                                src_rows: Optional[torch.Tensor] = None) -> None:
+                                src_rows: Optional[torch.Tensor] = None,
+                                live: Optional[Tuple[int, int]] = None) -> bool:
         """Pack ``(g1-g0)*gt`` tokens (rows from ``row0`` on, or ``src_rows``) into group slots ``[g0, g1)``
-        with one store launch (kv_store.py:551-610)."""
+        with one store launch (kv_store.py:551-610).  ``live = (n_head, lo)``: the same launch may write the block's
+        rows ``[0, n_head)`` and ``[lo, T)`` into the history; True when it has."""
         n_tok = (g1 - g0) * self.gt
         ppg = self.pages_per_group
-        if self._host.store_pack(K, V, self._store_planes, self.ps, src_rows, self._req_to_token_full,
-                                 self._req_to_group_full, self.err_flag, n_tok, store_table(K.device), row0,
-                                 g0 * ppg, g0, *self._recipe):
-            return
+        call = (K, V, self._store_planes, self.ps, src_rows, self._req_to_token_full, self._req_to_group_full,
+                self.err_flag, n_tok, store_table(K.device), row0, g0 * ppg, g0, *self._recipe)
+        if live is not None and self._host.store_pack(*call, self._k_hist4, self._v_hist4, 0, *live, self._ring_sink,
+                                                      self._ring_rec):
+            return True
+        if self._host.store_pack(*call):
+            return False
         if src_rows is None:
             K, V = K[row0:row0 + n_tok], V[row0:row0 + n_tok]
         store_pack_into(K, V, self._store_planes, outliers_per_vector=self.k,
@@ -319,6 +332,7 @@ class CanonicalKVStore:
                         dst_pages=self._req_to_token_full.view(-1)[g0 * ppg:g1 * ppg],
                         dst_groups=self._req_to_group_full.view(-1)[g0:g1],
                         err_flag=self.err_flag, num_tokens=n_tok)
+        return False
 
     # ── read path ────────────────────────────────────────────────────────────────
 

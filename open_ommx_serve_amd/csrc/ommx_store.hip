@@ -51,7 +51,7 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
     static_assert(!(F32 && FAST6), "the tuned path reads bf16 input");
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const bool do_k = !APART || blockIdx.z == 0, do_v = !APART || blockIdx.z == 1;
-    if (copied_row(a)) return;
+    if (copied_row<APART>(a)) return;
     // head_dim 128 is compiled in for the tuned instantiations (their launch checks it): row offsets
     // of the code tile become instruction immediates
     const int D = FAST6 ? 128 : a.D;
@@ -488,7 +488,7 @@ extern "C" void ommx_store_default_table(float* t) {
 namespace ommx {
 template <bool APART>
 static void launch_store_pack(int variant, const StoreArgs& a, hipStream_t st) {
-    const dim3 grid(store_grid_x(a), a.H, APART ? 2 : 1), block(a.D);
+    const dim3 grid = store_grid<APART>(a), block(a.D);
     const size_t shm = 32 * (size_t)a.D + 4 * (size_t)a.D + (a.idx_repr ? 8 * (size_t)a.D : 0);
     if (variant == 0) hipLaunchKernelGGL((store_pack_kernel<true, false, 2, APART>), grid, block, shm, st, a, NoRing{});
     else if (variant == 1) hipLaunchKernelGGL((store_pack_kernel<false, true, 0, APART>), grid, block, shm, st, a, NoRing{});
@@ -496,7 +496,7 @@ static void launch_store_pack(int variant, const StoreArgs& a, hipStream_t st) {
     else hipLaunchKernelGGL((store_pack_kernel<false, false, 2, APART>), grid, block, shm, st, a, NoRing{});
 }
 static void launch_store_ring(const StoreArgs& a, const RingGroups& ring, hipStream_t st) {
-    const dim3 grid(store_grid_x(a), a.H, 2), block(a.D);
+    const dim3 grid = store_grid<true>(a), block(a.D);
     const size_t shm = 36 * (size_t)a.D + (a.idx_repr ? 8 * (size_t)a.D : 0);
     if (a.idx_repr == 0) hipLaunchKernelGGL((store_pack_kernel<false, true, 0, true, true>), grid, block, shm, st, a, ring);
     else hipLaunchKernelGGL((store_pack_kernel<false, true, 1, true, true>), grid, block, shm, st, a, ring);

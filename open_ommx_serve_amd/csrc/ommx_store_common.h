@@ -43,20 +43,30 @@ struct StoreArgs {
     BlockRows rows;
 };
 
-// Live rows of a prompt ride along with its packed groups: workgroups behind the last group copy a row each while that
-// one is still being packed.  True when the workgroup had no group.
+// Rows of a prompt ride along with its packed groups: workgroups behind those of the groups copy a row each while the
+// groups are still being packed.  They are slices of z when the groups take two workgroups each (z 0 and 1; at most
+// kStoreApart of them run empty), of y otherwise (a row slice of a full chip is mostly empty).  True when the workgroup had
+// no group.  A fresh prompt of 4096 rows, all of them kept: 7.3 + 9.1 us as two launches, 12.0 as one (13.8 with the rows'
+// slices between those of K and of V).
+template <bool APART>
 __device__ __forceinline__ bool copied_row(const StoreArgs& a) {
-    if (static_cast<int>(blockIdx.x) < a.groups) return false;
-    const int n = (static_cast<int>(blockIdx.x) - a.groups) * a.H + static_cast<int>(blockIdx.y);
-    if (n < a.rows.rows && blockIdx.z == 0) copy_block_row<false>(a.rows, n);
+    const int past = APART ? static_cast<int>(blockIdx.z) - 2 : static_cast<int>(blockIdx.y) - a.H;
+    if (past < 0) return false;
+    const int n = ((APART ? past * a.H + static_cast<int>(blockIdx.y) : past)) * a.groups + static_cast<int>(blockIdx.x);
+    if (n < a.rows.rows) copy_block_row<false>(a.rows, n);
     return true;
 }
+
 // A workgroup each for K and V of a group and head?  Two against one, 8 heads: 5.4 against 6.4 us (32 tokens), 5.5 / 6.7 (1024), 8.4 / 10.0
 // (4096), 13.4 / 14.0 (8192), 22.4 / 22.4 (16384), 52.9 / 48.0 (32 K tokens into a pool); fp32 rows 24.8 / 26.7 (4096).  Past
 // the line the chip is full either way, and the second workgroup is only one more to start.
 constexpr int kStoreApart = 2048;
 inline bool store_apart(const StoreArgs& a) { return a.groups * static_cast<int64_t>(a.H) <= kStoreApart; }
-inline unsigned store_grid_x(const StoreArgs& a) { return a.groups + (a.rows.rows + a.H - 1) / a.H; }
+template <bool APART>
+inline dim3 store_grid(const StoreArgs& a) {
+    const int each = APART ? a.groups * a.H : a.groups, slices = (a.rows.rows + each - 1) / each;
+    return APART ? dim3(a.groups, a.H, 2 + slices) : dim3(a.groups, a.H + slices);
+}
 
 // Entries of the identity tables that belong to K group g: the pages that begin in it, and its own.
 __device__ __forceinline__ void write_own_tables(const StoreArgs& a, int g, int tid) {

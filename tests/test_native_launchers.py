@@ -5,7 +5,7 @@ import pytest
 import torch
 
 import oracle.ommx_oracle as O
-from open_ommx_serve_amd.attention import MultiSeqKVPool, WindowSpec, _hip, ommx_pack_kv_canonical_block
+from open_ommx_serve_amd.attention import CanonicalKVStore, MultiSeqKVPool, WindowSpec, _hip, ommx_pack_kv_canonical_block
 from open_ommx_serve_amd.attention.kv_store_ops import ring_slot
 from open_ommx_serve_amd.attention.pack import alloc_planes, store_pack_into, store_table
 
@@ -276,3 +276,26 @@ def test_rows_of_any_width_reach_their_slot(H, D):
         for b, p in enumerate(pos):
             slot = p if p < sink else sink + (p - sink) % span
             assert torch.equal(kh[b, slot], K[b]) and torch.equal(vh[b, slot], V[b])
+
+
+@pytest.mark.parametrize("T,H,gt", [(105, 3, 32), (4096, 8, 32), (8300, 8, 32), (1100, 2, 64)])
+@pytest.mark.parametrize("single", [False, True])
+def test_rows_and_groups_of_a_fresh_block_in_one_launch(T, H, gt, single):
+    """A fresh block against the same rows in two pieces, which take a launch for the rows and one for the groups: a full
+    chip, one that is not, a block of one or two groups with more rows than that."""
+    D, how = 128, dict(window=WindowSpec(group_tokens=gt), device=DEV, kv_ring=False, outliers_per_vector=6,
+                       use_pow2=True, outlier_repr="bitmap" if gt == 32 else "relidx7")
+    K, V = _block(T, H, D, torch.bfloat16, 1), _block(T, H, D, torch.bfloat16, 2)
+    made = [CanonicalKVStore(D, H, T + 5, **how) if single else MultiSeqKVPool(D, H, 2, T + 5, **how) for _ in range(2)]
+    put = (lambda s, a, b: s.append_block(a, b)) if single else (lambda s, a, b: s.append_block(1, a, b))
+    for s in made:
+        for t in [s.k_hist, s.v_hist, *(t for t in s._store_planes.values() if torch.is_tensor(t))]:
+            t.zero_()
+    put(made[0], K, V)
+    put(made[1], K[:40], V[:40])
+    put(made[1], K[40:], V[40:])
+    assert made[0].seq_len == made[1].seq_len and made[0].packed_groups == made[1].packed_groups
+    assert torch.equal(made[0].k_hist, made[1].k_hist) and torch.equal(made[0].v_hist, made[1].v_hist)
+    for n, t in made[0]._store_planes.items():
+        if torch.is_tensor(t):
+            assert torch.equal(t.view(torch.uint8), made[1]._store_planes[n].view(torch.uint8)), n
