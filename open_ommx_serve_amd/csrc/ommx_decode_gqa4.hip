@@ -130,9 +130,13 @@ __device__ __forceinline__ uint32_t k_pair(uint32_t w, uint32_t w_up, uint32_t w
 }
 // V channel y of a merged dword (token a in the low 16 bits, token b in the high 16 bits) as
 // f16 (1 + c/16) * 2^e (even y, code at mantissa bits [7:6]) or (1 + c/4) * 2^e (odd y, bits
-// [9:8]); `step` holds the f16 2^e of the two tokens.
-template <int Y>
+// [9:8]); `step` holds the f16 2^e of the two tokens.  The epilogue takes the constant out of the sum and multiplies what is
+// left by 16 or 4, the fp32 sum's own rounding with it: longer groups take bits [9:8] for every channel (three more shifts a
+// dword), without which one split over 16 K tokens of 64 x 64 vectors came out 1.22 times as far from 64-bit sums as the
+// kernel that served them before.
+template <int Y, bool LONG>
 __device__ __forceinline__ uint32_t v_pair(uint32_t m, uint32_t step) {
+    if constexpr (LONG) return ((Y <= 4 ? m << (8 - 2 * Y) : m >> (2 * Y - 8)) & 0x03000300u) | step;
     const uint32_t sh = Y <= 1 ? (m << 6) : Y <= 3 ? (m << 2) : Y <= 5 ? (m >> 2) : (m >> 6);
     return (sh & ((Y & 1) ? 0x03000300u : 0x00C000C0u)) | step;
 }
@@ -1065,10 +1069,10 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
                 {                                                                                         \
                     const bool mine = (jp >> 2) == X;                                                     \
                     const u32x4 bx = {mine ? pw[0] : 0u, mine ? pw[1] : 0u, mine ? pw[2] : 0u, mine ? pw[3] : 0u}; \
-                    acc[0] = mfma_f16(u32x4{v_pair<X>(mg0, sw[0]), v_pair<X>(mg1, sw[1]),                 \
-                                            v_pair<X>(mg2, sw[2]), v_pair<X>(mg3, sw[3])}, bx, acc[0]);   \
-                    acc[1] = mfma_f16(u32x4{v_pair<4 + X>(mg0, sw[0]), v_pair<4 + X>(mg1, sw[1]),         \
-                                            v_pair<4 + X>(mg2, sw[2]), v_pair<4 + X>(mg3, sw[3])}, bx, acc[1]); \
+                    acc[0] = mfma_f16(u32x4{v_pair<X, LONG>(mg0, sw[0]), v_pair<X, LONG>(mg1, sw[1]),                 \
+                                            v_pair<X, LONG>(mg2, sw[2]), v_pair<X, LONG>(mg3, sw[3])}, bx, acc[0]);   \
+                    acc[1] = mfma_f16(u32x4{v_pair<4 + X, LONG>(mg0, sw[0]), v_pair<4 + X, LONG>(mg1, sw[1]),         \
+                                            v_pair<4 + X, LONG>(mg2, sw[2]), v_pair<4 + X, LONG>(mg3, sw[3])}, bx, acc[1]); \
                 }
                 OMMX_PVX(0) OMMX_PVX(1) OMMX_PVX(2) OMMX_PVX(3)
 #undef OMMX_PVX
@@ -1079,8 +1083,8 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
                 const u32x4 bx0 = {first ? pw[0] : 0u, first ? pw[1] : 0u, first ? pw[2] : 0u, first ? pw[3] : 0u};
                 const u32x4 bx1 = {first ? 0u : pw[0], first ? 0u : pw[1], first ? 0u : pw[2], first ? 0u : pw[3]};
 #define OMMX_PVY(Y)                                                                                       \
-                acc[(Y) >> 1] = mfma_f16(u32x4{v_pair<Y>(mg0, sw[0]), v_pair<Y>(mg1, sw[1]),              \
-                                               v_pair<Y>(mg2, sw[2]), v_pair<Y>(mg3, sw[3])},             \
+                acc[(Y) >> 1] = mfma_f16(u32x4{v_pair<Y, LONG>(mg0, sw[0]), v_pair<Y, LONG>(mg1, sw[1]),              \
+                                               v_pair<Y, LONG>(mg2, sw[2]), v_pair<Y, LONG>(mg3, sw[3])},             \
                                          ((Y) & 1) ? bx1 : bx0, acc[(Y) >> 1]);
                 OMMX_PVY(0) OMMX_PVY(1) OMMX_PVY(2) OMMX_PVY(3) OMMX_PVY(4) OMMX_PVY(5) OMMX_PVY(6) OMMX_PVY(7)
 #undef OMMX_PVY
@@ -1119,7 +1123,7 @@ __global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : O
                 const float pz = (r >> 1) ? ((kqe & 1) ? z4[3] : z4[1]) : ((kqe & 1) ? z4[2] : z4[0]);
                 const float psum = (r >> 1) ? ((kqe & 1) ? s4[3] : s4[1]) : ((kqe & 1) ? s4[2] : s4[0]);
                 const int ch = 64 * (kqe & 1) + 16 * r + 8 * (kqe >> 1) + (NH == 8 ? 2 : 4) * a2 + x;
-                const float f = (x & 1) ? 4.0f : 16.0f;
+                const float f = LONG || (x & 1) ? 4.0f : 16.0f;
                 const float val = (f * (acc[a2][r] - psum) + pz) * inv;
                 if (!half) dst[ch] = val;
                 else if ((kqe & 1) == h / r_half) dst[ch & 63] = val;     // the head's own 64 channels
