@@ -4,7 +4,8 @@
 // k_tail/v_tail; o = sum w_i o_i / sum w_i, lse = max + ln sum w_i; nothing attended gives
 // o = 0, lse = -inf.
 //
-// Two kernels.  combine_kernel: Q workgroups per (request, q head), one per piece of the head's
+// fold_kernel (at the end) merges when the split-KV launch has attended the tail already; two kernels attend it themselves.
+// combine_kernel: Q workgroups per (request, q head), one per piece of the head's
 // channels.  It is latency bound (few small workgroups, a few KB each), so every global load is
 // issued before the first wait: thread (d, sg) owns channel d of the splits sg, sg+NSG, ... and
 // of the tail rows sg, sg+NSG, ...; for the tail logits the same threads regroup as (row, 16

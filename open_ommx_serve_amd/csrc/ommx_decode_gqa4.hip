@@ -36,7 +36,7 @@
 //            (outlier - zp - code*2^e) / 2^(10-2m) as f16 into a [32 tokens][128 channels] tile
 //            that is the B operand of an f16 MFMA against the same A.  Entries whose f16 rounding
 //            could show on a logit add their rounding residual times q through LDS float atomics.
-//   P.V      A = (1 + code/4 | 1 + code/16) * 2^e_v as f16 for 8 tokens of one channel, B = p (f16).
+//   P.V      A = (1 + code/4 | 1 + code/16) * 2^e_v as f16 for 8 tokens of one channel (longer groups code/4), B = p (f16).
 #include <type_traits>
 
 #include "ommx_decode_shares.h"

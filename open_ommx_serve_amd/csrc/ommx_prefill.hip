@@ -22,9 +22,12 @@
 // so the weights never pass through LDS.  K rows and transposed V are double buffered in LDS (70 KB); the next tile's
 // rows are requested before a tile is worked on, through buffers that end with the request.
 //
-// Bound: matrix instructions and vector instructions share a SIMD's time (next to a wave that issues matrix
-// instructions back to back another one keeps about half its vector rate).  4096 tokens of 32 heads:
-// 203 K clocks of matrix instructions (85 us at 2.4 GHz) and 203 K of vector ones in 363 K (rocprofv3 counters).  That is
+// Bound: power, once the chip is full.  4096 tokens of 32 heads: 203 K clocks of matrix instructions and 203 K of vector
+// ones in 363 K (rocprofv3 counters), and those pass at 1.8 GHz: a tile step of a workgroup takes 3.03 us with 512 of
+// them and 1.93 us with 128 (8 heads), both alone on their compute units, and 1.05 PFLOP/s issued compares with 1.21 of a
+// large library product on the same card.  The two kinds of instructions hardly hold each other up (a vector instruction
+// 7.45 clocks beside a wave of matrix instructions, 6.8 without; the matrix ones the same), and dealing the staging out
+// evenly over both groups of waves changed nothing (206.7 -> 212.5 us).  That is
 // 191 to 200 us from card to card (HIP events around launches back to back; the kernel trace of rocprofv3 has 204 at least
 // and 207 on average).  Two groups of waves in one workgroup, one half a tile behind the other so that the matrix phase of
 // one meets the vector phase of the other, share the staged tiles as well: 264 -> 191 us (events, one card, with two pieces
