@@ -76,10 +76,11 @@ __device__ __forceinline__ void each_of(F&& f, std::integer_sequence<int, I...>)
 template <int N, class F>
 __device__ __forceinline__ void each(F&& f) { each_of<N>(f, std::make_integer_sequence<int, N>{}); }
 
-// k_vec: K rows allow 16-byte loads.  As many waves a SIMD as the LDS of head_dim 128 allows: left alone, the compiler takes
-// 78 to 150 registers (32 K tokens into a pool 72 us instead of 61).
+// k_vec: K rows allow 16-byte loads.  As many waves a SIMD as the LDS allows (128 tokens: of head_dim 64): left alone, the
+// compiler takes 78 to 256 registers (64 tokens, 32 K into a pool 72 us instead of 61; 128 tokens at head_dim 64, 24 K into
+// a block 40.6 instead of 36.7).
 template <int GT, int GC, int KH>
-__global__ void __launch_bounds__(512, GT < GC ? 1 : GT == 32 ? 8 : GT == 64 ? 5 : 2) store_long_kernel(StoreArgs a, int k_vec) {
+__global__ void __launch_bounds__(512, GT < GC ? 1 : GT == 32 ? 8 : GT == 64 ? 5 : 3) store_long_kernel(StoreArgs a, int k_vec) {
     constexpr int K = 2 * KH, MW = GT / 32, TIE = GT - 1;      // GT is a power of two: the tie breaker is its low bits
     constexpr int SORT = K <= 8 ? 8 : 12;                      // LDS bytes per thread and sorted list
     constexpr int NVAL = K / 2, NIDX = (7 * K + 7) / 8;
