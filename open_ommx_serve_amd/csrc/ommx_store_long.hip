@@ -51,18 +51,28 @@ __device__ __forceinline__ void keep_smallest(int (&t)[N], int key) {
     t[0] = min(t[0], key);
 }
 
-// The minimum (or maximum) over the L neighbouring lanes of a vector, in all of them.
-template <int CTRL, class F>
-__device__ __forceinline__ float with_lane(float x, F f) {
-    return f(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, x), __builtin_bit_cast(int, x),
-                                                                      CTRL, 0xF, 0xF, false)));
+// The extremes of bf16 values in packed 16-bit integers: b ^ (sign ? 0x7FFF : 0) orders them (-0 below +0, as v_min_f32 has
+// it; infinities and NaN at the ends), two at once.
+typedef int16_t s16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ s16x2 pair_image(uint32_t two) {
+    const s16x2 m = __builtin_bit_cast(s16x2, two) >> s16x2{15, 15};
+    return __builtin_bit_cast(s16x2, (__builtin_bit_cast(uint32_t, m) & 0x7FFF7FFFu) ^ two);
 }
-template <int L, class F>
-__device__ __forceinline__ float over_vector(float x, F f) {
-    x = with_lane<0xB1>(x, f);                          // quad_perm [1,0,3,2]
-    x = with_lane<0x4E>(x, f);                          // quad_perm [2,3,0,1]
-    if constexpr (L >= 8) x = with_lane<0x141>(x, f);   // row_half_mirror
-    if constexpr (L >= 16) x = with_lane<0x140>(x, f);  // row_mirror
+__device__ __forceinline__ float value_of_image(int img) {        // a sign-extended image
+    return __int_as_float((img ^ ((img >> 31) & 0x7FFF)) << 16);
+}
+// (minimum, complement of the maximum) of a vector from those of its L neighbouring lanes, in all of them.
+template <int CTRL>
+__device__ __forceinline__ uint32_t with_lane(uint32_t x) {
+    const uint32_t other = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), CTRL, 0xF, 0xF, true));
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(s16x2, x), __builtin_bit_cast(s16x2, other)));
+}
+template <int L>
+__device__ __forceinline__ uint32_t over_vector(uint32_t x) {
+    x = with_lane<0xB1>(x);                          // quad_perm [1,0,3,2]
+    x = with_lane<0x4E>(x);                          // quad_perm [2,3,0,1]
+    if constexpr (L >= 8) x = with_lane<0x141>(x);   // row_half_mirror
+    if constexpr (L >= 16) x = with_lane<0x140>(x);  // row_mirror
     return x;
 }
 // The value of lane N of the vector's L lanes.
@@ -76,9 +86,10 @@ __device__ __forceinline__ void each_of(F&& f, std::integer_sequence<int, I...>)
 template <int N, class F>
 __device__ __forceinline__ void each(F&& f) { each_of<N>(f, std::make_integer_sequence<int, N>{}); }
 
-// k_vec: K rows allow 16-byte loads.  As many waves a SIMD as the LDS allows (128 tokens: of head_dim 64): left alone, the
-// compiler takes 78 to 256 registers (64 tokens, 32 K into a pool 72 us instead of 61; 128 tokens at head_dim 64, 24 K into
-// a block 40.6 instead of 36.7).
+// k_vec: K rows allow 16-byte loads.  As many waves a SIMD as the LDS allows (128 tokens: of head_dim 64), which the compiler
+// has to be told: with the extremes of V in floats it took 78 to 256 registers by itself (64 tokens, 32 K into a pool 72 us
+// instead of 61; 128 tokens at head_dim 64, 24 K into a block 40.6 instead of 36.7).  In packed integers they take a third of
+// the registers and half of the instructions: 45 / 72 / 136, 11 K tokens at head_dim 64 14.4 -> 13.9 us.
 template <int GT, int GC, int KH>
 __global__ void __launch_bounds__(512, GT < GC ? 1 : GT == 32 ? 8 : GT == 64 ? 5 : 3) store_long_kernel(StoreArgs a, int k_vec) {
     constexpr int K = 2 * KH, MW = GT / 32, TIE = GT - 1;      // GT is a power of two: the tie breaker is its low bits
@@ -303,27 +314,23 @@ __global__ void __launch_bounds__(512, GT < GC ? 1 : GT == 32 ? 8 : GT == 64 ? 5
     } else {
         // -------------------------------------------- V vectors (pack.py:604-623)
         load_v();
-        // (minimum and maximum of a piece, then of its vector in all VL lanes)
-        float mn[VP], mx[VP];
-        bool fin = true;                        // no exponent field of all ones
+        // (minimum, complement of the maximum) of a piece, then of its vector in all VL lanes
+        uint32_t ends[VP];
 #pragma unroll
         for (int n = 0; n < VP; ++n) {
-            typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
             const u32x4 w = vu[n];
-            u16x2 e2 = {0, 0};
-            mn[n] = mx[n] = __uint_as_float(w[0] << 16);
+            s16x2 lo = pair_image(w[0]), hi = lo;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const float lo = __uint_as_float(w[c] << 16), hi = __uint_as_float(w[c] & 0xFFFF0000u);
-                mn[n] = fminf(fminf(mn[n], lo), hi);
-                mx[n] = fmaxf(fmaxf(mx[n], lo), hi);
-                e2 = __builtin_elementwise_max(e2, __builtin_bit_cast(u16x2, w[c] & 0x7F807F80u));
+            for (int c = 1; c < 4; ++c) {
+                const s16x2 img = pair_image(w[c]);
+                lo = __builtin_elementwise_min(lo, img);
+                hi = __builtin_elementwise_max(hi, img);
             }
-            fin = fin && e2[0] != 0x7F80 && e2[1] != 0x7F80;
-            mn[n] = over_vector<VL>(mn[n], [](float x, float y) { return fminf(x, y); });
-            mx[n] = over_vector<VL>(mx[n], [](float x, float y) { return fmaxf(x, y); });
+            const uint32_t l = __builtin_bit_cast(uint32_t, lo), h2 = ~__builtin_bit_cast(uint32_t, hi);
+            const s16x2 even = __builtin_bit_cast(s16x2, __builtin_amdgcn_perm(h2, l, 0x05040100u)),
+                        odd = __builtin_bit_cast(s16x2, __builtin_amdgcn_perm(h2, l, 0x07060302u));
+            ends[n] = over_vector<VL>(__builtin_bit_cast(uint32_t, __builtin_elementwise_min(even, odd)));
         }
-        if (!fin) err |= OMMX_ERR_NONFINITE_V;
         // Lane i of a vector's VL lanes works out the step of the vector of turn VL r + i, for all of them.
         const int me = v % VL, ngv = D / GC;
         int page[VP];
@@ -334,12 +341,11 @@ __global__ void __launch_bounds__(512, GT < GC ? 1 : GT == 32 ? 8 : GT == 64 ? 5
         };
 #pragma unroll
         for (int r = 0; r < VP; r += VL) {
-            float my_mn = mn[r], my_mx = mx[r];
+            uint32_t mine = ends[r];
 #pragma unroll
-            for (int n = 1; n < VL && r + n < VP; ++n) {
-                my_mn = me == n ? mn[r + n] : my_mn;
-                my_mx = me == n ? mx[r + n] : my_mx;
-            }
+            for (int n = 1; n < VL && r + n < VP; ++n) mine = me == n ? ends[r + n] : mine;
+            const float my_mn = value_of_image(static_cast<int16_t>(mine)), my_mx = value_of_image(static_cast<int16_t>(~mine >> 16));
+            if (!is_finite_f32(my_mn) || !is_finite_f32(my_mx)) err |= OMMX_ERR_NONFINITE_V;
             const Step st = make_step(__fdiv_rn(fmaxf(my_mx - my_mn, 1e-8f), 3.0f), 0, tab);
             const uint16_t zp_b = f32_to_bf16_rne(my_mn);
             const float zc = -bf16_to_f32(zp_b) * st.inv;
