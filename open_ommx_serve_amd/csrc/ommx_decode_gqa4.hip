@@ -10,8 +10,8 @@
 // a workgroup is 4 waves = 4 neighbouring kv heads.  Measured on MI355X this operator is bound
 // by how many instructions a SIMD can issue (vector ALU first, LDS second, a 16-byte LDS access
 // taking four issue slots), so the kernel is built for few instructions per token and to keep
-// THREE waves per SIMD resident: at most 168 vector registers, no scratch memory, 13.4 KB of LDS
-// per wave.  What that takes, against the kernel in ommx_decode.hip:
+// THREE waves per SIMD resident (two with longer groups): at most 168 vector registers, no scratch
+// memory, 13.4 KB of LDS per wave.  What that takes, against the kernel in ommx_decode.hip:
 //   * P.V runs transposed (rows = V channels, columns = q heads), the V step 2^e sits in the
 //     exponent field of the V operand, and the four column replicas of the q heads each take
 //     every fourth channel block, so the output accumulator is 8 registers instead of 32;
@@ -87,8 +87,14 @@ struct LdsMap {
     static constexpr int LDS_WAVE = OFF_ONES + 128;            // 13376 (4 heads) / 14464 (8 heads), LONG 272 more
     static_assert(OFF_KT % 16 == 0 && OFF_PT % 16 == 0 && OFF_VZ % 16 == 0 && OFF_LC % 16 == 0, "b128 alignment");
 };
-static_assert(3 * 4 * LdsMap<4, true>::LDS_WAVE <= 160 * 1024, "4 heads: three workgroups per compute unit");
-static_assert(2 * 4 * LdsMap<8, true>::LDS_WAVE <= 160 * 1024, "8 heads: two workgroups per compute unit");
+// LDS is handed out in pieces of 1280 bytes (768 workgroups of 53760 bytes on 256 compute units take one round, of 53776 two).
+// The 33rd row of longer groups is what makes a third workgroup not fit: 54592 bytes take 55040, three of them 165120 of 163840.
+constexpr int lds_of(int workgroup_bytes) { return (workgroup_bytes + 1279) / 1280 * 1280; }
+// Workgroups resident on a compute unit, by registers and LDS; the launcher deals out as many shares (`lean` in ommx_host.cpp).
+constexpr int resident(int nh, bool longer) { return nh == 4 && !longer ? OMMX_GQA4_WAVES : 2; }
+static_assert(resident(4, false) * lds_of(4 * LdsMap<4, false>::LDS_WAVE) <= 160 * 1024, "4 heads, 32-token groups");
+static_assert(resident(4, true) * lds_of(4 * LdsMap<4, true>::LDS_WAVE) <= 160 * 1024, "4 heads, longer groups");
+static_assert(resident(8, true) * lds_of(4 * LdsMap<8, true>::LDS_WAVE) <= 160 * 1024, "8 heads");
 
 // One f16 carries 11 bits: rounding an outlier delta d costs up to |d| * 2^-11, i.e. up to
 // |d| * max|q| * 2^-11 * sm_scale on a logit.  A delta with |d| * max|q| >= BIG_DELTA * 16
@@ -159,10 +165,10 @@ __device__ __forceinline__ uint32_t pk_u16(uint32_t lo, uint32_t hi) { return (l
 // and channel pair, against 24 in a 32-token recipe) but no branch.  The work is dealt out in those 64-token steps:
 // whole groups of 128 left a batch of 342 groups on 172 of 256 resident workgroups, four serial steps each.  Whole
 // call, ommx_decode.hip's kernel on whole groups -> this one: 128 tokens and 10 outliers, 4 requests of 2 to 20 K
-// 45.9 -> 34.7 us, one of 64 K 47.1 -> 40.0, 8 of 4 to 16 K with 64 q heads 84.7 -> 52.6; 64 tokens and 6 outliers,
-// 64 K 36.8 -> 32.3, 1.1 K 15.5 -> 14.5.
+// 45.8 -> 31.5 us, one of 64 K 47.7 -> 37.8, 32 of 1 to 16 K 165 -> 129, 8 of 4 to 16 K with 64 q heads 84.5 -> 48.8; 64
+// tokens and 6 outliers, 64 K 37.3 -> 32.2, 700 tokens 14.4 -> 11.5, 32 of 1 to 16 K 128 -> 107.
 template <int IDX, bool OWN_MAP, bool PARTIAL, int ORDER, int NH = 4, bool GEN = false, int KSLOTS = 6, int GTS = 0, bool HALF = false>
-__global__ void __launch_bounds__(256, (NH == 8 || (GEN && KSLOTS == 8)) ? 2 : OMMX_GQA4_WAVES) decode_gqa4_kernel(DecodeArgs a) {
+__global__ void __launch_bounds__(256, (GEN && KSLOTS == 8) ? 2 : resident(NH, GTS > 0)) decode_gqa4_kernel(DecodeArgs a) {
     static_assert(NH == 4 || (NH == 8 && !PARTIAL), "4 heads (or fewer, PARTIAL) or exactly 8");
     static_assert(!GEN || IDX == 0, "the general form reads bitmaps");
     // outlier slots walked per vector: the general form walks 4 or 8 whatever a.kout is (loads and
