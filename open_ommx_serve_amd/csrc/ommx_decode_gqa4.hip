@@ -105,8 +105,12 @@ static_assert(resident(8, true) * lds_of(4 * LdsMap<8, true>::LDS_WAVE) <= 160 *
 // large values then stay in the base codes, the steps grow, and so do the entries).
 constexpr float BIG_DELTA = 2.0f;
 constexpr float BIG_DELTA_SM_SCALE = 0.08838834764831845f;
-// the running maximum of the online softmax is refreshed when a logit (base 2) exceeds it by this
-constexpr float MAX_SLACK = 8.0f;
+// The running maximum of the online softmax is refreshed when a logit (base 2) exceeds it by this.  Under a maximum that lags,
+// the largest weight is no longer 1 but a number rounded to f16, and the lse takes over its rounding error (up to 2^-12).  Longer
+// groups are refreshed at once, as on the kernel that served them before: one split over 6001 tokens of 64 x 64 vectors, error of
+// the lse 3.5e-5 there, 1.07e-4 with a slack of 8 (rms), of the output 6.4e-5 and 8.1e-5 (2-norm).
+template <bool LONG>
+constexpr float MAX_SLACK = LONG ? 0.0f : 8.0f;
 // The base operand (1 + code*2^(2m-10)) * 2^e carries a constant A*2^e per channel, up to 2^6 times
 // the signal, which the bias MFMA takes out again: two large sums that cancel in fp32.  From steps
 // of 2^EXACT_STEP_EXP on (values a hundred or more wide inside one vector) that shows on the logits, and
@@ -932,7 +936,7 @@ __global__ void __launch_bounds__(256, (GEN && KSLOTS == 8) ? 2 : resident(NH, G
                     if (!tok_ok) { x[r] = -INFINITY; pe[r] = -INFINITY; }
                 }
             }
-            if (__any(fmaxf(fmaxf(pe[0], pe[1]), fmaxf(pe[2], pe[3])) > MAX_SLACK)) {
+            if (__any(fmaxf(fmaxf(pe[0], pe[1]), fmaxf(pe[2], pe[3])) > MAX_SLACK<LONG>)) {
                 // refresh the running maxima (always on the first step) and rescale what is summed so far
                 float mxs[4] = {x[0], x[1], x[2], x[3]};
                 wave_max4(mxs);
@@ -1004,7 +1008,7 @@ __global__ void __launch_bounds__(256, (GEN && KSLOTS == 8) ? 2 : resident(NH, G
                     pe[g][r] = x[g][r] - m_run[r];
                     over = fmaxf(over, pe[g][r]);
                 }
-            if (__any(over > MAX_SLACK)) {
+            if (__any(over > MAX_SLACK<LONG>)) {
                 // refresh the running maxima of the lane's four heads (rows kq and kq ^ 2 hold the same
                 // heads) and rescale what is summed so far
                 float mxs[4];

@@ -10,6 +10,7 @@ import torch
 import oracle.ommx_oracle as O
 from open_ommx_serve_amd.attention import _hip
 from open_ommx_serve_amd.attention.kv_window import WindowSpec
+from open_ommx_serve_amd.attention.pack import ommx_pack_kv_canonical_block
 from open_ommx_serve_amd.attention.paged_decode import (make_attn_logits,
                                                         ommx_paged_decode_attention_canonical)
 from open_ommx_serve_amd.synth import build_decode_case
@@ -357,6 +358,32 @@ def test_longer_groups_cut_into_pieces(gt, gc, k, hq, own_map):
         want = _oracle(case)
         for S in (None, 1, 3 * gt // 64):
             _check(_run(case, num_kv_splits=S), want, f"gt{gt} gc{gc} k{k} S{S}")
+
+
+@pytest.mark.parametrize("gt,k,hq", [(64, 6, 32), (64, 6, 64), (128, 10, 32), (128, 10, 64)])
+def test_the_largest_weight_of_a_longer_group_is_one(gt, k, hq):
+    """Weights are f16 and relative to the running maximum: the largest is 1 and exact only if that maximum is up to date.
+    Keys of 0..3 and then of 0..6 (all operands exact) against queries that put the second group's maximum 2^6.1 to 2^7.6
+    above the first's: the other weights sum to at most 8 % of the largest, so their rounding (2^-12) moves the lse by 2e-5
+    (that of the largest itself, were it not 1, by up to 2.4e-4), fp32 by some 1e-6."""
+    H, D, T = 8, 128, 2 * gt
+    t = torch.arange(T, device="cuda")
+    K = ((t % 4) << (t // gt)).to(torch.bfloat16).view(T, 1, 1).expand(T, H, D).contiguous()
+    V = torch.randn(T, H, D, generator=torch.Generator(device="cuda").manual_seed(3), device="cuda").to(torch.bfloat16)
+    p = ommx_pack_kv_canonical_block(K, V, outliers_per_vector=k, outlier_select="signed", outlier_repr="relidx7",
+                                     use_pow2=True, kv_outlier_map=False, page_size=16, group_tokens=gt, group_channels=gt,
+                                     device="cuda")
+    assert int(p["k_scale"].max()) == 1 and int(p["k_scale"].min()) == 0
+    q = torch.zeros(1, hq, D, device="cuda")
+    q[0, :, 5] = 16.0 + 4.0 * torch.arange(hq, device="cuda") / hq
+    q = q.to(torch.bfloat16)
+    o, lse = torch.empty(1, hq, D, device="cuda"), torch.empty(1, hq, device="cuda")
+    ommx_paged_decode_attention_canonical(
+        q, p["k_base"], p["k_scale"], p["k_zp"], p["k_oidx"], p["k_oval"], p["v_main"], p["v_scale"], p["v_zp"], None, None,
+        None, o, lse, p["req_to_token"], p["req_to_group"], torch.tensor([T], dtype=torch.int32, device="cuda"),
+        sm_scale=D ** -0.5, page_size=16, k_outliers_per_vector=k, kv_int8_scale=True, num_kv_splits=1, max_seq_len=T)
+    want = torch.logsumexp(q[0, :, 5].double().view(-1, 1) * D ** -0.5 * K[:, 0, 5].double(), 1)
+    assert (lse[0].double() - want).abs().max().item() <= 2.5e-5
 
 
 def test_randomised_recipes_against_the_oracle():
