@@ -56,7 +56,7 @@ extern "C" {
 #define OMMX_ERR_RING_RANGE   16   /* row outside the history (kv_store_ops.py:33-34,52-53) */
 /* error bits OR-ed into *err_flag by the decode entry points */
 #define OMMX_ERR_TABLE_RANGE  64   /* a page id or group slot outside the planes (kv_pool.py:526-550 guards these on the host) */
-#define OMMX_ERR_VALUE_RANGE 128   /* a K step above 2^15 (K values beyond some 1e5) does not fit the f16 operands of
+#define OMMX_ERR_VALUE_RANGE 128   /* a V step, or a K step of 32-token groups, above 2^15 does not fit the f16 operands of
                                       the matrix-core kernels; it is held at 2^15 and the result is off */
 /* not an error: OR-ed into *err_flag by ommx_store_pack when it writes a K step above 2^15, so that the owner
    of the cache can send its decodes to ommx_decode_splitkv_ref before OMMX_ERR_VALUE_RANGE ever happens */
@@ -163,8 +163,9 @@ int ommx_store_pack(const void* K, const void* V, int in_dtype,
  *                 both extents are given and every plane is below 4 GiB (pages * page_size * Hkv * 32
  *                 bytes of code rows, group slots * Hkv * D * 6 bytes of index plane); other calls run
  *                 on the matrix-core kernel with 64-bit addressing (same results, more time).
- *                 OMMX_ERR_VALUE_RANGE: a K or V step above 2^15 met by the serving-recipe kernel, whose
- *                 f16 operands end there (the step is held at 2^15: finite output, but off); the store
+ *                 OMMX_ERR_VALUE_RANGE: a V step, or a K step of 32-token groups, above 2^15 met by the
+ *                 serving-recipe kernel, whose f16 operands end there (the step is held at 2^15: finite
+ *                 output, but off; K steps of longer groups are served at any size); the store
  *                 announces such a cache with OMMX_NOTE_WIDE_STEP, and ommx_decode_splitkv_ref serves it.
  *                 Query elements of any size are served (a query with elements of 128 or more is taken
  *                 divided by a power of two, exactly, and the softmax scale carries the factor).

@@ -109,9 +109,9 @@ def ommx_paged_decode_attention_canonical(
     signature either): an int32 device tensor that receives ``_hip.ERR_TABLE_RANGE`` when a page id
     or group slot of the tables lies outside the planes (the kernels clamp such an entry, so nothing
     is read out of bounds; the reference leaves these checks to the pools, ``kv_pool.py:526-550``),
-    and ``_hip.ERR_VALUE_RANGE`` when a K step lies above 2^15 (K values beyond some 1e5), which the
-    f16 operands of the matrix-core kernel cannot carry: the output is finite but off, and
-    ``_force_reference_kernel=True`` serves such a cache.
+    and ``_hip.ERR_VALUE_RANGE`` when a V step, or a K step of 32-token groups, lies above 2^15 (values beyond
+    some 1e5), which the f16 operands of the matrix-core kernel cannot carry: the output is finite but off,
+    and ``_force_reference_kernel=True`` serves such a cache.  (K steps of longer groups are served at any size.)
     """
     if (_native or _load_native()).decode(
             q, k_base, k_scale, k_zp, k_oidx, k_oval, v_main, v_scale, v_zp, k_tail, v_tail, b_tail_len,

@@ -386,6 +386,95 @@ def test_the_largest_weight_of_a_longer_group_is_one(gt, k, hq):
     assert (lse[0].double() - want).abs().max().item() <= 2.5e-5
 
 
+@pytest.mark.parametrize("gt,gc,k,hq,own_map", [(64, 64, 6, 32, False), (128, 64, 6, 64, True), (128, 128, 10, 32, True),
+                                                (128, 32, 10, 64, False)])
+@pytest.mark.parametrize("kind", ["large", "small", "small, ordinary q", "zero points", "entries"])
+def test_longer_groups_take_k_steps_of_every_size(gt, gc, k, hq, own_map, kind):
+    """K times 2^16 or 2^-20 and q divided by it (the same logits), steps of 2^-16 under ordinary queries, zero points beyond
+    2^18 and outliers whose distance to the base code no f16 holds: nothing is held at a bound, so nothing is reported."""
+    case = build_decode_case([700, 333], q_heads=hq, kv_heads=8, seed=88, permute_tables=True, group_tokens=gt,
+                             group_channels=gc, outliers_per_vector=k, outlier_repr="relidx7", kv_outlier_map=own_map,
+                             outlier_gain=3.0e5 if kind == "entries" else 1.0)
+    p, up = case.planes, {"large": 16, "small": -20, "small, ordinary q": -16}.get(kind, 0)
+    p["k_scale"] += up
+    for name, by in (("k_zp", 2.0 ** up), ("k_fp4_mapcenter", 2.0 ** up), ("k_fp4_mapscale", 2.0 ** -up)):
+        if p[name] is not None:
+            p[name] *= by
+    case.k_tail *= 2.0 ** up
+    case.q *= 24.0 if kind == "small, ordinary q" else 2.0 ** -up
+    if kind == "zero points":
+        for name in ("k_zp", "k_fp4_mapcenter"):
+            if p[name] is not None:
+                p[name][..., 4] += 300000.0
+        case.q[..., 4] = 2.0 ** -16
+    if kind == "entries":
+        case.q *= 2.0 ** -16
+    assert (case.q.abs().max() < 128) == (kind != "small")
+    top = int(p["k_scale"].max())
+    assert {"large": top > 15, "entries": top > 15}.get(kind, top < 15), top
+    err = torch.zeros(1, dtype=torch.int32, device=case.q.device)
+    wo, wl = _oracle(case)
+    for S in (None, 1):
+        o, lse = _run(case, num_kv_splits=S, err_flag=err)
+        d = (o.double() - wo).abs()
+        assert d.max().item() <= MAX_ABS and d.mean().item() <= MEAN_ABS, f"S{S}: {d.max().item():.3e}"
+        # (logits of 1e-3: the f16 tile entries are subnormal, 2^-25 each times 16 times q, a dozen a token)
+        bound = 1e-4 if kind == "small, ordinary q" else 2e-3
+        assert (lse.double() - wl).abs().max().item() <= bound, f"S{S}: lse {(lse.double() - wl).abs().max().item():.3e}"
+    assert int(err.item()) == 0
+
+
+@pytest.mark.parametrize("gt,gc,k,hq,own_map", [(64, 64, 6, 32, False), (128, 64, 6, 64, True), (128, 128, 10, 32, True),
+                                                (128, 32, 10, 64, False)])
+@pytest.mark.parametrize("lo,hi", [(-22, -15), (-16, 3)])
+def test_longer_groups_take_v_steps_down_to_subnormal_f16(gt, gc, k, hq, own_map, lo, hi):
+    """V steps of 2^-22 (a quarter of which is the smallest f16) to 2^-15, alone and among ordinary ones: the output is as
+    exact as the steps allow, each weighted element to the f16 weight's 2^-12 and a zero point's 2^-25."""
+    case = build_decode_case([700, 333], q_heads=hq, kv_heads=8, seed=89, permute_tables=True, group_tokens=gt,
+                             group_channels=gc, outliers_per_vector=k, outlier_repr="relidx7", kv_outlier_map=own_map)
+    p = case.planes
+    g = torch.Generator(device="cuda").manual_seed(4)
+    p["v_scale"].copy_(torch.randint(lo, hi + 1, p["v_scale"].shape, generator=g, device="cuda"))
+    small = hi < 0
+    if small:
+        p["v_zp"] *= 2.0 ** -15
+        case.b_tail_len.zero_()
+    err = torch.zeros(1, dtype=torch.int32, device="cuda")
+    wo, _ = _oracle(case)
+    scale = 2.0 ** -15 if small else 2.0 ** 3
+    for S in (None, 1):
+        o, _ = _run(case, num_kv_splits=S, err_flag=err)
+        d = (o.double() - wo).abs()
+        assert d.max().item() <= MAX_ABS * scale + 2.0 ** -25 and d.mean().item() <= MEAN_ABS * scale, f"S{S}: {d.max().item():.3e}"
+    assert int(err.item()) == 0
+
+
+@pytest.mark.parametrize("gt,gc,k,hq,own_map", [(64, 64, 6, 32, False), (128, 64, 6, 64, True), (128, 128, 10, 32, True),
+                                                (128, 32, 10, 64, False)])
+@pytest.mark.parametrize("k_late,v_late,codes", [(True, False, True), (False, True, True), (True, True, True), (True, True, False)])
+def test_longer_groups_change_their_form_in_the_middle_of_a_split(gt, gc, k, hq, own_map, k_late, v_late, codes):
+    """A K group and two pages of V with steps of 2^-20 behind several ordinary steps: the split is walked again, all of it and
+    once, in the form that takes them.  Without codes (channels and rows that do not vary) the steps do not matter."""
+    case = build_decode_case([1500, 333], q_heads=hq, kv_heads=8, seed=90, permute_tables=True, sparse_frac=0.005,
+                             group_tokens=gt, group_channels=gc, outliers_per_vector=k, outlier_repr="relidx7",
+                             kv_outlier_map=own_map)
+    p = case.planes
+    if k_late:
+        g = case.req_to_group[0, 6 * 128 // gt].long()
+        p["k_scale"][g] = -20
+        p["k_zp"][g] *= 2.0 ** -20
+    if v_late:
+        pages = case.req_to_token[0, 41:43].long()
+        p["v_scale"][pages] = -20
+    if not codes:
+        p["v_main"][pages] = 0
+        first = 6 * 128 // 16
+        p["k_base"][case.req_to_token[0, first:first + gt // 16].long()] = 0
+    want = _oracle(case)
+    for S in (None, 1, 3):
+        _check(_run(case, num_kv_splits=S), want, f"S{S}")
+
+
 def test_randomised_recipes_against_the_oracle():
     """Forty random draws over the whole recipe space the kernels accept (group sizes, outlier
     count, index plane, outlier map, step mode, V format, head shapes, table dtype, splits,
