@@ -49,7 +49,10 @@ def auto_num_kv_splits(max_seq_len: int, batch: int, kv_heads: int, n_cu: int = 
     more splits are faster.  The kernel with ``resident`` 3 deals whole groups out evenly by itself;
     for the others the count is chosen so that their rounding leaves no split empty.  At most 512,
     the number of partial states the combine kernel keeps on chip.  Splits are whole K groups
-    (``group_tokens``), so longer groups mean coarser steps."""
+    (``group_tokens``), so longer groups mean coarser steps.
+
+    ``attn_logits`` for that many splits (``resident`` 2, the recipe's ``group_tokens``) is enough for a call that
+    leaves the split count to the launcher; in a workspace of its own it may take more."""
     mean = -1.0 if mean_seq_len is None else float(mean_seq_len)
     return _hip.host().auto_num_kv_splits(int(max_seq_len), int(batch), int(kv_heads), int(n_cu),
                                           int(group_tokens), mean, int(resident))

@@ -413,7 +413,13 @@ int run_decode(const DecodeCall& c) {
     }
     if (rc == 1) {
         int64_t S = c.splits;
-        if (S == 0) S = auto_splits(c.max_seq, B, wave_heads, cu_count(dev.index()), unit, c.mean, lean ? 3 : 2);
+        if (S == 0) {
+            S = auto_splits(c.max_seq, B, wave_heads, cu_count(dev.index()), unit, c.mean, lean ? 3 : 2);
+            // What this kernel likes best can be more than the public rule gives for the recipe's own groups and heads, by which a
+            // caller sizes its workspace (128-token groups, 8 kv heads, 4096 tokens: 64 against 32): that many then.
+            if (c.ws && c.ws->dim() == 4 && c.ws->size(2) < S)
+                S = std::min<int64_t>(S, auto_splits(c.max_seq, B, Hkv, cu_count(dev.index()), gt, c.mean, 2));
+        }
         if (c.ws && (c.ws->scalar_type() != at::kFloat || c.ws->dim() != 4 || c.ws->size(0) != B || c.ws->size(1) != Hq ||
                      c.ws->size(2) < S || c.ws->size(3) < D + 1 || c.ws->stride(3) != 1))
             return 0;

@@ -11,7 +11,7 @@ import oracle.ommx_oracle as O
 from open_ommx_serve_amd.attention import _hip
 from open_ommx_serve_amd.attention.kv_window import WindowSpec
 from open_ommx_serve_amd.attention.pack import ommx_pack_kv_canonical_block
-from open_ommx_serve_amd.attention.paged_decode import (make_attn_logits,
+from open_ommx_serve_amd.attention.paged_decode import (auto_num_kv_splits, make_attn_logits,
                                                         ommx_paged_decode_attention_canonical)
 from open_ommx_serve_amd.synth import build_decode_case
 
@@ -473,6 +473,30 @@ def test_longer_groups_change_their_form_in_the_middle_of_a_split(gt, gc, k, hq,
     want = _oracle(case)
     for S in (None, 1, 3):
         _check(_run(case, num_kv_splits=S), want, f"S{S}")
+
+
+@pytest.mark.parametrize("lens,hq,hkv,D,kw", [
+    ([1100], 32, 8, 128, dict(group_tokens=128, group_channels=128, outlier_repr="relidx7")),
+    ([4200], 64, 8, 128, dict(group_tokens=128, group_channels=128, outliers_per_vector=10, outlier_repr="relidx7")),
+    ([2100] * 4, 32, 8, 128, dict(group_tokens=64, group_channels=64, outlier_repr="relidx7")),
+    ([6300] * 16, 32, 8, 128, {}),                       # a third workgroup a compute unit
+    ([6300] * 16, 16, 8, 64, {}),                        # waves that take pairs of kv heads
+    ([700, 300], 32, 8, 128, {}),
+])
+def test_a_workspace_of_the_documented_size_is_taken(lens, hq, hkv, D, kw):
+    """``attn_logits`` sized by ``auto_num_kv_splits`` for the recipe, no split count given; one slot fewer is refused."""
+    case = build_decode_case(lens, q_heads=hq, kv_heads=hkv, head_dim=D, seed=92, **kw)
+    longest, gt = max(case.packed_lens), kw.get("group_tokens", 32)
+    mean = sum(case.packed_lens) / len(lens)
+    S = auto_num_kv_splits(longest, len(lens), hkv, torch.cuda.get_device_properties(0).multi_processor_count,
+                           group_tokens=gt, mean_seq_len=mean)
+    want, lse = _run(case, max_seq_len=longest)
+    ws = make_attn_logits(len(lens), hq, S, D, "cuda")
+    for w in (ws, ws[:, :, :S]):
+        got, glse = _run(case, max_seq_len=longest, mean_seq_len=mean, attn_logits=w)
+        assert (got - want).abs().max().item() <= MAX_ABS and (glse - lse).abs().max().item() <= 2e-3
+    with pytest.raises(ValueError, match="too small"):
+        _run(case, max_seq_len=longest, mean_seq_len=mean, attn_logits=ws[:, :, :S - 1])
 
 
 def test_randomised_recipes_against_the_oracle():
