@@ -624,7 +624,9 @@ PyObject* py_store_pack(PyObject*, PyObject* const* a, Py_ssize_t n) {
     ommx::BlockRows rows;
     if (n == 28) {
         // (rows that come out of the history itself: not while it is being written)
-        if (T == 0 || K->scalar_type() != at::kBFloat16 || !read_block_rows(*K, *V, a + 21, 0, rows)) Py_RETURN_FALSE;
+        if (T == 0 || K->scalar_type() != at::kBFloat16 || !read_block_rows(*K, *V, a + 21, 0, rows) ||
+            rows.rows > ommx::kRowSlices * (T / r.gt))
+            Py_RETURN_FALSE;
         for (PyObject* hist : {a[21], a[22]})
             if (K->is_alias_of(THPVariable_Unpack(hist)) || V->is_alias_of(THPVariable_Unpack(hist))) Py_RETURN_FALSE;
         extras.rows = &rows;

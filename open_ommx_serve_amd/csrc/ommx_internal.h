@@ -41,8 +41,12 @@ struct StoreExtras {
                                                               // fill (both or neither)
     const RingGroups* ring = nullptr;     // where the groups lie; T / 32 of them, span rows in the ring.  store_pack returns 1,
     int ring_span = 0;                    // with nothing launched, for a recipe or a number of groups that needs the tables
-    const BlockRows* rows = nullptr;      // bf16 rows to copy into the history (head_dim a multiple of 8, every slot inside it)
+    const BlockRows* rows = nullptr;      // bf16 rows to copy into the history (head_dim a multiple of 8, every slot inside it),
+                                          // at most kRowSlices for a group
 };
+// The rows of StoreExtras are slices of the grid's y or z behind those of the groups, a row for every group in a slice: few
+// groups under a long recent window would need more slices than a grid has (65 536).
+constexpr int64_t kRowSlices = 32768;
 
 // ommx_store_pack (the C ABI documents the arguments) with extras.
 int store_pack(const void* K, const void* V, int in_dtype, int64_t k_ts, int64_t k_hs, int64_t v_ts, int64_t v_hs,

@@ -42,6 +42,27 @@ def test_block_rows_reach_their_history_slots(ring, T, dtype, strided):
             assert torch.equal(got[n].cpu(), want[n]), n
 
 
+@pytest.mark.parametrize("ring", [False, True])
+@pytest.mark.parametrize("recent,D,gt", [(32600, 64, 32), (32800, 64, 32), (70000, 128, 32), (140000, 64, 32), (70000, 64, 128)])
+def test_one_group_under_a_long_window(ring, recent, D, gt):
+    """The rows that are copied along with a single group take a slice of the grid each: from as many slices on as a grid
+    does not hold, they are copied by a launch of their own."""
+    T, win = 8 + gt + recent, WindowSpec(recent_window=recent, group_tokens=gt)
+    recipe = dict(RECIPE, outlier_select="signed", kv_outlier_map=True)
+    if gt != 32:
+        recipe.update(outlier_repr="relidx7", group_channels=gt // 2)
+    assert win.num_groups(T) == 1
+    pool = MultiSeqKVPool(D, 1, 1, T + 100, window=win, device=DEV, kv_ring=ring, **recipe)
+    K, V = _block(T, 1, D, torch.bfloat16, 21), _block(T, 1, D, torch.bfloat16, 22)
+    assert pool.append_block(0, K, V) == 1
+    at = [ring_slot(p, pool._ring_sink, pool._ring_rec) if ring else p for p in range(T)]
+    assert torch.equal(pool.k_hist[0, at], K) and torch.equal(pool.v_hist[0, at], V)
+    want = ommx_pack_kv_canonical_block(K[8:8 + gt], V[8:8 + gt], page_size=16, device=DEV, group_tokens=gt, **recipe)
+    got = pool.request_planes(0)
+    for n in ("k_base", "k_scale", "k_oval", "v_main", "v_scale"):
+        assert torch.equal(got[n], want[n]), n
+
+
 @pytest.mark.parametrize("n", [1, 479, 480, 481, 960, 961, 2000])
 @pytest.mark.parametrize("dtype", [torch.int64, torch.int32])
 def test_uploads_of_one_launch_and_more(n, dtype):
