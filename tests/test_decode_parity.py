@@ -328,8 +328,8 @@ def test_bf16_v_rows(kw):
 @pytest.mark.parametrize("hq,own_map", [(32, False), (64, True), (32, True), (64, False)])
 def test_longer_groups_on_the_matrix_core_kernel(gt, gc, k, hq, own_map):
     """K groups of 64 / 128 tokens with position streams and 6 outliers (10 with 128-token
-    groups: the reference's 2.75-bit "paper-kv" recipe) run on the matrix-core kernel as
-    32-token pieces of a group: against the oracle and against the plain kernel, ragged
+    groups: the reference's 2.75-bit "paper-kv" recipe) run on the serving recipe's matrix-core kernel
+    as 64-token pieces of a group: against the oracle and against the plain kernel, ragged
     lengths, permuted tables, several split counts."""
     case = build_decode_case([2900, 700, 150], q_heads=hq, kv_heads=8, seed=81, permute_tables=True,
                              sparse_frac=0.005, group_tokens=gt, group_channels=gc, outliers_per_vector=k,

@@ -11,6 +11,8 @@ from open_ommx_serve_amd.synth import build_decode_case
 
 pytestmark = pytest.mark.gpu
 LEVER = dict(group_tokens=64, group_channels=64, outliers_per_vector=10, outlier_repr="relidx7")
+LEVER6 = dict(LEVER, outliers_per_vector=6, kv_outlier_map=False)
+PAPER10 = dict(group_tokens=128, group_channels=128, outliers_per_vector=10, outlier_repr="relidx7")
 PAPER = dict(group_tokens=128, group_channels=128, outlier_repr="relidx7")
 
 
@@ -54,8 +56,13 @@ def _oracle(case):
     (4, 4, 128, {}, [5000, 4000]),
     (32, 8, 64, {}, [72, 9000, 5000]),                                    # head_dim 64: pairs of kv heads
     (16, 4, 64, {}, [300 + i for i in range(65)]),
-    (32, 8, 128, LEVER, [5000, 9, 9000]),                                 # longer groups: the other kernel
-    (32, 8, 128, PAPER, [400 + 5 * i for i in range(66)]),
+    (32, 8, 128, LEVER, [5000, 9, 9000]),                                 # ten outliers of 64 tokens: the plain kernel
+    (32, 8, 128, PAPER, [400 + 5 * i for i in range(66)]),                # more requests than longer groups are dealt out for
+    (32, 8, 128, LEVER6, [5000, 9, 9000]),                                # pieces of longer groups
+    (64, 8, 128, LEVER6, [300 + 37 * i for i in range(64)]),
+    (8, 1, 128, PAPER10, [9000, 131, 20000]),
+    (32, 8, 128, PAPER10, [2100 + 67 * i for i in range(20)]),
+    (64, 8, 128, dict(PAPER10, group_channels=64), [6000, 9, 170, 4000]),
 ])
 def test_shares_against_the_oracle(hq, hkv, D, kw, lens):
     case = build_decode_case(lens, q_heads=hq, kv_heads=hkv, head_dim=D, seed=77, permute_tables=True,

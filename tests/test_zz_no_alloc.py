@@ -22,7 +22,7 @@ pytestmark = pytest.mark.gpu
 MAX_ABS, MEAN_ABS = 2e-3, 2e-4
 
 
-def _noalloc(case, S):
+def _noalloc(case, S, extents=True):
     B, Hq, D = case.q.shape
     dev = case.q.device
     o = torch.full((B, Hq, D), float("nan"), dtype=torch.float32, device=dev)
@@ -35,8 +35,8 @@ def _noalloc(case, S):
         rc = lib.ommx_decode_attention_noalloc(
             case.q.data_ptr(), case.q.stride(0), case.q.stride(1),
             p["k_base"].data_ptr(), p["k_scale"].data_ptr(), p["k_zp"].data_ptr(),
-            p["k_fp4_mapscale"].data_ptr(), p["k_fp4_mapcenter"].data_ptr(),
-            p["k_obmp"].data_ptr(), p["k_oval"].data_ptr(),
+            *(None if t is None else t.data_ptr() for t in (p["k_fp4_mapscale"], p["k_fp4_mapcenter"])),
+            p["k_obmp" if case.outlier_repr == "bitmap" else "k_oidx"].data_ptr(), p["k_oval"].data_ptr(),
             p["v_main"].data_ptr(), p["v_scale"].data_ptr(), p["v_zp"].data_ptr(),
             case.req_to_token.data_ptr(), case.req_to_token.stride(0),
             case.req_to_group.data_ptr(), case.req_to_group.stride(0),
@@ -46,8 +46,10 @@ def _noalloc(case, S):
             case.v_tail.stride(0), case.v_tail.stride(1), case.v_tail.stride(2),
             case.b_tail_len.data_ptr(),
             o.data_ptr(), o.stride(0), o.stride(1), lse.data_ptr(), lse.stride(0),
-            B, Hq, case.kv_heads, D, case.page_size, case.outliers_per_vector, _hip.INDEX_BITMAP, 0,
-            32, 32, 0, S, int(case.k_tail.shape[1]), float(case.sm_scale), 0.0, 0, int(p["k_base"].shape[0]), int(p["k_scale"].shape[0]), None,
+            B, Hq, case.kv_heads, D, case.page_size, case.outliers_per_vector,
+            _hip.INDEX_BITMAP if case.outlier_repr == "bitmap" else _hip.INDEX_RELIDX7, 0,
+            p["group_tokens"], p["group_channels"], 0, S, int(case.k_tail.shape[1]), float(case.sm_scale), 0.0, 0,
+            int(p["k_base"].shape[0]) if extents else 0, int(p["k_scale"].shape[0]) if extents else 0, None,
             _hip.current_stream_ptr(dev))
         torch.cuda.synchronize()
         _noalloc.taken = free_before - torch.cuda.mem_get_info()[0]
@@ -116,6 +118,26 @@ def test_head_dim_64_and_eight_q_heads_per_kv_head_through_the_same_entry_point(
         assert (o - wo).abs().max().item() <= 1e-5, f"{name}: same kernels, same split count"
         oo, ol = _oracle(case)
         _close(o, lse, oo, ol, f"{name} vs oracle")
+
+
+@pytest.mark.parametrize("gt,gc,k,hq,own_map", [(64, 64, 6, 32, False), (64, 128, 6, 32, True), (64, 32, 6, 64, False),
+                                                (64, 64, 6, 64, True), (128, 128, 6, 32, False), (128, 64, 6, 32, True),
+                                                (128, 128, 6, 64, False), (128, 32, 6, 64, True), (128, 128, 10, 32, False),
+                                                (128, 64, 10, 32, True), (128, 32, 10, 64, False), (128, 128, 10, 64, True),
+                                                (32, 32, 6, 32, True), (32, 32, 6, 64, False), (32, 32, 6, 8, True),
+                                                (32, 32, 6, 16, False)])
+def test_planes_of_unknown_extent_go_to_the_kernel_with_64_bit_addresses(gt, gc, k, hq, own_map):
+    """Without the extents of the planes (or from 4 GiB of them on) the matrix-core kernel with 64-bit addresses serves what the
+    one with 32-bit offsets takes otherwise; both against the oracle."""
+    case = build_decode_case([1500, 700, 150], q_heads=hq, kv_heads=8, seed=81, permute_tables=True, sparse_frac=0.005,
+                             group_tokens=gt, group_channels=gc, outliers_per_vector=k, outlier_repr="relidx7",
+                             kv_outlier_map=own_map)
+    want = _oracle(case)
+    for S in (1, 5):
+        for extents in (False, True):
+            rc, o, lse = _noalloc(case, S, extents)
+            assert rc == 0, _hip.load().ommx_last_error()
+            _close(o, lse, *want, f"S{S} extents {extents}")
 
 
 def test_sizes_beyond_the_built_in_array_are_refused():
