@@ -192,8 +192,8 @@ __device__ __forceinline__ uint32_t pk_u16(uint32_t lo, uint32_t hi) { return (l
 // and channel pair, against 24 in a 32-token recipe) but no branch.  The work is dealt out in those 64-token steps:
 // whole groups of 128 left a batch of 342 groups on 172 of 256 resident workgroups, four serial steps each.  Whole
 // call, ommx_decode.hip's kernel on whole groups -> this one: 128 tokens and 10 outliers, 4 requests of 2 to 20 K
-// 45.8 -> 31.5 us, one of 64 K 47.7 -> 37.8, 32 of 1 to 16 K 165 -> 129, 8 of 4 to 16 K with 64 q heads 84.5 -> 48.8; 64
-// tokens and 6 outliers, 64 K 37.3 -> 32.2, 700 tokens 14.4 -> 11.5, 32 of 1 to 16 K 128 -> 107.
+// 46.0 -> 31.4 us, one of 64 K 47.5 -> 37.2, 32 of 1 to 16 K 165 -> 125, 8 of 4 to 16 K with 64 q heads 84.4 -> 48.5; 64
+// tokens and 6 outliers, 64 K 37.3 -> 32.2, 700 tokens 14.6 -> 11.8, 32 of 1 to 16 K 128 -> 105.
 // Longer groups: a split that needs what f16 does not hold (MIN_STEP_EXP above), walked from its start; every output of the
 // wave is written here then.
 template <int ORDER, bool OWN_MAP, int NH, int KSLOTS, int GTS>

@@ -301,8 +301,8 @@ int run_decode(const DecodeCall& c) {
                         (k == 6 || (k == 10 && gt == 128));
     const int64_t unit = pieces ? 64 : gt;                       // tokens that a share is made of
     // Longer groups keep two workgroups a compute unit (a third does not fit their LDS, and the shares of a round that is not
-    // there made full batches slower than whole groups on the kernel before: 8 x 32 K tokens of 64 x 64 vectors 123 us with
-    // three, 113 on that kernel, 96 with two; 32 of 1 to 16 K 134 / 128 / 107; of 128 x 128 with ten outliers 173 / 165 / 129).
+    // there made full batches slower than whole groups on the kernel before: 8 x 32 K tokens of 64 x 64 vectors 124 us with
+    // three, 113 on that kernel, 95 with two; 32 of 1 to 16 K 134 / 128 / 105; of 128 x 128 with ten outliers 173 / 165 / 125).
     const bool lean = plain_planes && ((D == 128 && R <= 4 && k == 6) ||
                                        (c.bitmap && k >= 1 && k <= 6 && ((D == 128 && R <= 4) ||
                                                                          (D == 64 && R <= 2 && Hkv % 2 == 0))));
