@@ -125,7 +125,7 @@ constexpr int MAX_STEP_EXP = 15;
 // zero, or a zero point of K from 2^18 on, or that has a query of 2^12 or more, drops what it has and walks its split in a
 // second form (ANY): K codes and zero points as bf16, V codes times a step that may be subnormal, neither with a constant to
 // take out again, and outlier entries that no normal f16 holds settled exactly.  (V steps above 2^15 stay held and
-// reported.)  Steps that do not matter, of channels and rows that do not vary, stay in the first form (5 to 7 % slower).
+// reported.)  Steps that do not matter, of channels and rows that do not vary, stay in the first form (up to 9 % slower).
 // Whole call over a kernel without any of it 0.99 to 0.98; the same as branches of the one loop 0.96 to 0.92, as a second loop that
 // took over in the middle, with the sums so far, 0.99 to 0.93.  The looks go where the loop has a branch already: one
 // of its own where V is staged cost 4 to 8 %.

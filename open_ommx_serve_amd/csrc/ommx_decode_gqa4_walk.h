@@ -594,7 +594,8 @@
                     if (GEN && sidx >= kout) continue;
                     const float dl = dls[sidx];
                     bool matters = fabsf(dl) >= big_thr[u];
-                    if constexpr (ANY) matters |= q_down >= HUGE_Q_DOWN && fabsf(dl) < MIN_F16;
+                    if constexpr (ANY)
+                        matters |= q_down >= HUGE_Q_DOWN && fabsf(dl) < MIN_F16 && dl != static_cast<float>(static_cast<_Float16>(dl));
                     if (matters && (!LONG || pos[sidx] < 32)) {
                         float hi = static_cast<float>(static_cast<_Float16>(dl));
                         if constexpr (ANY) {
