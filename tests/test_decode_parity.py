@@ -655,6 +655,26 @@ def test_head_dim_64_eight_outliers_many_requests_stay_inside_the_tolerance():
     _check(_run(case, num_kv_splits=5), _oracle(case), "d64 k8 70 requests")
 
 
+@pytest.mark.parametrize("loud", [0, 1])
+@pytest.mark.parametrize("lens", [[1700], [333, 97, 1100]])
+def test_exact_residuals_at_head_dim_64_go_to_the_heads_of_their_own_kv_head(lens, loud):
+    """Two 64-channel kv heads are read as one of 128 channels, whose outlier residuals are added for the four q heads of
+    the channel's own kv head only.  With the queries of one of the two 8 times as large a dropped rounding is up to
+    24 * 2^-12 * 24 * 64^-0.5 = 1.8e-2 of a logit, and one that went to the other head the same: both far over the
+    tolerance of the lse (2e-3, and 1e-5 of logits in the hundreds for fp32)."""
+    case = build_decode_case(lens, q_heads=32, kv_heads=8, head_dim=64, seed=91 + loud, permute_tables=True,
+                             sparse_frac=0.005)
+    q = case.q.float().view(len(lens), 4, 2, 4, 64)
+    q[:, :, loud] *= 8.0
+    case.q.copy_(q.view(len(lens), 32, 64).to(case.q.dtype))
+    wo, wl = _oracle(case)
+    for S in (None, 3):
+        o, lse = _run(case, num_kv_splits=S)
+        d = (o.double() - wo).abs()
+        assert d.max().item() <= MAX_ABS and d.mean().item() <= MEAN_ABS, f"S{S}: {d.max().item():.3e}"
+        assert ((lse.double() - wl).abs() <= 2e-3 + 1e-5 * wl.abs()).all(), f"S{S}: lse"
+
+
 @pytest.mark.parametrize("hq,hkv,D,k,own_map", [(32, 8, 128, 6, True), (64, 8, 128, 6, True), (32, 8, 128, 5, False),
                                                  (8, 8, 128, 3, True), (16, 8, 64, 6, True)])
 def test_large_steps_take_the_operand_without_its_constant(hq, hkv, D, k, own_map):
