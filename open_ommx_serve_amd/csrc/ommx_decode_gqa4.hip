@@ -81,14 +81,14 @@ struct LdsMap {
     static constexpr int OFF_VZ = OFF_PT + NH * PT_ROW * 2;    // [4 channel groups][PT_ROW] f16 V zero points
     static constexpr int OFF_VS = OFF_VZ + 4 * PT_ROW * 2;     // [4 channel groups][PT_ROW] f16 2^e_v
     static constexpr int OFF_STAGE_END = (OFF_VS + 4 * PT_ROW * 2 > OFF_ZPP + 512) ? OFF_VS + 4 * PT_ROW * 2 : OFF_ZPP + 512;
-    static constexpr int OFF_LC = OFF_STAGE_END;               // [32 tokens][NH heads] f32 logit corrections of one group
-    static constexpr int OFF_ZERO = OFF_LC + 32 * NH * 4;      // 128 B of zeros, never written again
+    static constexpr int OFF_LC = OFF_STAGE_END;               // [tokens][NH heads] f32 logit corrections of one group (32), or of a step of a longer one (64)
+    static constexpr int OFF_ZERO = OFF_LC + (LONG ? 64 : 32) * NH * 4;      // 128 B of zeros, never written again
     static constexpr int OFF_ONES = OFF_ZERO + 128;            // 128 B of f16 1.0, never written again
     static constexpr int LDS_WAVE = OFF_ONES + 128;            // 13376 (4 heads) / 14464 (8 heads), LONG 272 more
     static_assert(OFF_KT % 16 == 0 && OFF_PT % 16 == 0 && OFF_VZ % 16 == 0 && OFF_LC % 16 == 0, "b128 alignment");
 };
 // LDS is handed out in pieces of 1280 bytes (768 workgroups of 53760 bytes on 256 compute units take one round, of 53776 two).
-// The 33rd row of longer groups is what makes a third workgroup not fit: 54592 bytes take 55040, three of them 165120 of 163840.
+// Longer groups (56640 bytes, and more than 168 registers) have two workgroups a compute unit, not three.
 constexpr int lds_of(int workgroup_bytes) { return (workgroup_bytes + 1279) / 1280 * 1280; }
 // Workgroups resident on a compute unit, by registers and LDS; the launcher deals out as many shares (`lean` in ommx_host.cpp).
 constexpr int resident(int nh, bool longer) { return nh == 4 && !longer ? OMMX_GQA4_WAVES : 2; }
@@ -186,14 +186,14 @@ __device__ __forceinline__ uint32_t pk_u16(uint32_t lo, uint32_t hi) { return (l
 // 128-channel head, so a wave takes the pair as one head whose q heads are those of both, each
 // zero on the other one's channels, and writes each q head only its own half of the output.
 // GTS: K groups of 32 << GTS tokens (position streams; V vectors then 32, 64 or 128 channels wide), 6 outliers, or
-// 10 with 128 tokens (KSLOTS).  The 64 tokens of a step lie in one group then, whose parameters are held once, and
-// each 32-token half of the step walks all of the group's outliers: the ones that lie elsewhere go to a row of the
-// tile that nobody reads, which costs their instructions (10 outliers per 128 tokens walked four times are 40 a step
-// and channel pair, against 24 in a 32-token recipe) but no branch.  The work is dealt out in those 64-token steps:
+// 10 with 128 tokens (KSLOTS).  The 64 tokens of a step lie in one group then, whose parameters are held once and whose
+// outliers are walked once a step; either half scatters all of them, the ones that lie elsewhere to a row of the tile
+// that nobody reads, which costs their instructions (10 outliers per 128 tokens walked twice are 20 a step and channel,
+// against 12 in a 32-token recipe) but no branch.  The work is dealt out in those 64-token steps:
 // whole groups of 128 left a batch of 342 groups on 172 of 256 resident workgroups, four serial steps each.  Whole
 // call, ommx_decode.hip's kernel on whole groups -> this one: 128 tokens and 10 outliers, 4 requests of 2 to 20 K
-// 46.0 -> 31.4 us, one of 64 K 47.5 -> 37.2, 32 of 1 to 16 K 165 -> 125, 8 of 4 to 16 K with 64 q heads 84.4 -> 48.5; 64
-// tokens and 6 outliers, 64 K 37.3 -> 32.2, 700 tokens 14.6 -> 11.8, 32 of 1 to 16 K 128 -> 105.
+// 46.0 -> 28.9 us, one of 64 K 47.5 -> 35.2, 32 of 1 to 16 K 165 -> 113; 64 tokens and 6 outliers, 64 K 37.3 -> 30.6, 700 tokens
+// 14.6 -> 10.9, 32 of 1 to 16 K 128 -> 99.
 // Longer groups: a split that needs what f16 does not hold (MIN_STEP_EXP above), walked from its start; every output of the
 // wave is written here then.
 template <int ORDER, bool OWN_MAP, int NH, int KSLOTS, int GTS>

@@ -314,7 +314,7 @@
     {
         u32x4* p = reinterpret_cast<u32x4*>(sm + OFF_TILE);
         for (int i = lane; i < 32 * TILE_ROW / 16; i += 64) p[i] = u32x4{0, 0, 0, 0};
-        if (lane < 8 * NH) reinterpret_cast<u32x4*>(sm + OFF_LC)[lane] = u32x4{0, 0, 0, 0};
+        for (int i = lane; i < (LONG ? 16 : 8) * NH; i += 64) reinterpret_cast<u32x4*>(sm + OFF_LC)[i] = u32x4{0, 0, 0, 0};
         if (lane < 16) reinterpret_cast<u32x4*>(sm + OFF_ZERO)[lane] =
             lane < 8 ? u32x4{0, 0, 0, 0} : u32x4{0x3C003C00u, 0x3C003C00u, 0x3C003C00u, 0x3C003C00u};
     }
@@ -439,41 +439,128 @@
         f32x4 dsel[NH / 4];
 #pragma unroll
         for (int i = 0; i < NH / 4; ++i) dsel[i] = f32x4{0, 0, 0, 0};
+        // Longer groups: both halves of the step lie in one group, whose outliers are walked once: what an outlier adds, as f16, and
+        // the tile row it goes to in half 0 (as an offset; half 1 lies 32 rows on, and what lies in neither half past both).
+        // Each half then takes the scatter alone.  Walked anew for every half, as before, the positions, code reads and entries
+        // are formed twice; vector instructions are what these kernels are nearest to a limit of.  Whole call, 32 requests of 1
+        // to 16 K: 64 x 64 with six outliers 105.8 -> 99.2 us, 128 x 128 with ten 125.5 -> 113.2; 4 of 2 to 20 K of those
+        // 31.3 -> 28.9, 64 K alone 37.1 -> 35.2, 16 of 2 to 16 K with 64 q heads 78.5 -> 71.9.
+        uint32_t l_at[LONG ? 2 : 1][KMAX];
+        uint16_t l_e[LONG ? 2 : 1][KMAX];
+        bool l_res = false;
+        constexpr uint32_t HALF_ROWS = 32u * TILE_ROW;
+        if constexpr (LONG) {
+            float dls[2][KMAX];
+            auto walk = [&](auto U) {
+                constexpr int u = decltype(U)::value;
+                // index bits and levels of the channel; 10 outliers: the lane's bytes start 0 or 2 bytes into the loaded dwords
+                uint32_t ixw[3] = {0, 0, 0}, o0, o1 = 0;
+                if constexpr (KMAX == 10) {
+                    const uint32_t sh = ((lane & 1) ? 16u : 0u) + (u ? 8u : 0u);
+#pragma unroll
+                    for (int i = 0; i < 3; ++i)
+                        ixw[i] = (i == 2 && u) ? g_ix10[4] >> sh : __builtin_amdgcn_alignbit(g_ix10[i + 1 + 2 * u], g_ix10[i + 2 * u], sh);
+                    o0 = __builtin_amdgcn_alignbit(g_ov10[1 + u], g_ov10[u], sh);
+                    o1 = u ? g_ov10[2] >> sh : __builtin_amdgcn_alignbit(g_ov10[2], g_ov10[1], sh);
+                } else {
+                    ixw[0] = u ? __builtin_amdgcn_alignbit(g_bx[0], g_bm[0][1], 16) : g_bm[0][0];
+                    ixw[1] = u ? (g_bx[0] >> 16) : g_bm[0][1];
+                    o0 = static_cast<uint32_t>(((static_cast<uint64_t>(g_ov[0][1]) << 32) | g_ov[0][0]) >> (nib_sh + 24 * u));
+                }
+                // 128 tokens: the upper bit of every position flipped in the second piece, so that those of the piece read below 64
+                if (GTS == 2 && (n0 & 64)) {
+#pragma unroll
+                    for (int i = 0; i < 3; ++i) {
+                        uint32_t two = 0;
+                        for (int s7 = 0; s7 < KMAX; ++s7)
+                            if ((7 * s7 + 6) >> 5 == i) two |= 1u << ((7 * s7 + 6) & 31);
+                        ixw[i] ^= two;
+                    }
+                }
+                uint32_t cb[KMAX];
+#pragma unroll
+                for (int sidx = 0; sidx < KMAX; ++sidx) {
+                    constexpr uint32_t PM = (1u << GT_SH) - 1;
+                    const int bit = 7 * sidx, wi = bit >> 5, bo = bit & 31;
+                    const uint32_t f = (bo + GT_SH <= 32 ? (ixw[wi] >> bo) : __builtin_amdgcn_alignbit(ixw[wi < 2 ? wi + 1 : 2], ixw[wi], bo)) & PM;
+                    const uint32_t pos = GTS == 2 ? min(f, 64u) : f;
+                    l_at[u][sidx] = pos * TILE_ROW;
+                    cb[sidx] = *(sm + kt_lane + pos * KT_ROW);        // (of a row past the 64 nothing is used)
+                }
+                const float zp = __uint_as_float(u ? (g_zp[0] & 0xFFFF0000u) : (g_zp[0] << 16));
+                const int e = static_cast<int8_t>((g_sc[0] >> (8 * u)) & 0xFFu);
+                // in units of the channel's A scale, as in the walk of 32-token groups below
+                const float cs = u ? cs1 : cs0;
+                const float sc = __uint_as_float(static_cast<uint32_t>(e + 127) << 23) * cs;
+                float a1 = sc, b1 = 0.0f;
+                if (OWN_MAP) {
+                    a1 = cs * __builtin_amdgcn_rcpf(__uint_as_float(u ? (g_ms[0] & 0xFFFF0000u) : (g_ms[0] << 16)));
+                    b1 = cs * (__uint_as_float(u ? (g_mc[0] & 0xFFFF0000u) : (g_mc[0] << 16)) - zp);
+                }
+                float lv[10];
+                const f32x2 l01 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(o0, 1.0f, 0);
+                const f32x2 l23 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(o0, 1.0f, 1);
+                const f32x2 l45 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(o0, 1.0f, 2);
+                lv[0] = l01[0]; lv[1] = l01[1]; lv[2] = l23[0]; lv[3] = l23[1]; lv[4] = l45[0]; lv[5] = l45[1];
+                if constexpr (KMAX == 10) {
+                    const f32x2 l67 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(o0, 1.0f, 3);
+                    const f32x2 l89 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(o1, 1.0f, 0);
+                    lv[6] = l67[0]; lv[7] = l67[1]; lv[8] = l89[0]; lv[9] = l89[1];
+                }
+                float dl_max = 0.0f;
+#pragma unroll
+                for (int sidx = 0; sidx < KMAX; ++sidx) {
+                    const float code = static_cast<float>((cb[sidx] >> (code_sh + 2 * u)) & 3u);
+                    float dl = fmaf(-code, sc, fmaf(lv[sidx], a1, b1));
+                    // (the entry as a value of its own: rounded to f16 here exactly as the residual pass rounds it)
+                    asm("" : "+v"(dl));
+                    dls[u][sidx] = dl;
+                    // (ANY: the tile takes the largest f16, the logits the rest)
+                    l_e[u][sidx] = __builtin_bit_cast(uint16_t, static_cast<_Float16>(
+                        ANY && fabsf(dl) > MAX_F16 ? copysignf(MAX_F16, dl) : dl));
+                    dl_max = fmaxf(dl_max, GTS == 1 || l_at[u][sidx] < 2 * HALF_ROWS ? fabsf(dl) : 0.0f);
+                }
+                return (ANY && q_down >= HUGE_Q_DOWN) || __any(dl_max >= big_thr[u]) != 0;
+            };
+            // Entries of the step whose f16 rounding matters add what the rounding dropped to the logits, exactly.
+            auto residuals = [&](auto U) {
+                constexpr int u = decltype(U)::value;
+                const float un = __builtin_amdgcn_rcpf(u ? cs1 : cs0);
+                float* lc = reinterpret_cast<float*>(sm + OFF_LC);
+#pragma unroll
+                for (int sidx = 0; sidx < KMAX; ++sidx) {
+                    const float dl = dls[u][sidx], hi = static_cast<float>(__builtin_bit_cast(_Float16, l_e[u][sidx]));
+                    bool matters = fabsf(dl) >= big_thr[u];
+                    if constexpr (ANY) matters |= q_down >= HUGE_Q_DOWN && fabsf(dl) < MIN_F16 && dl != hi;
+                    if (matters && (GTS == 1 || l_at[u][sidx] < 2 * HALF_ROWS)) {
+                        const float lo = (dl - hi) * un;
+                        float* at_pos = lc + l_at[u][sidx] / TILE_ROW * NH;
+#pragma unroll
+                        for (int r = 0; r < NH; ++r)
+                            __hip_atomic_fetch_add(at_pos + r, lo * q_of(u, r), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+                    }
+                }
+            };
+            const bool res0 = walk(std::integral_constant<int, 0>{});
+            if (res0) residuals(std::integral_constant<int, 0>{});
+            const bool res1 = walk(std::integral_constant<int, 1>{});
+            if (res1) residuals(std::integral_constant<int, 1>{});
+            l_res = res0 || res1;
+            if (more) fetch_params_g(0);
+        }
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
             if (g == 1 && !g1_live) break;
             const int pg = LONG ? 0 : g;           // the group's parameter set
-            float* lc = reinterpret_cast<float*>(sm + OFF_LC);
-            // (both halves of a step read the same group here: without these copies the compiler would carry what the
-            // halves have in common, positions and levels, in registers that are not there)
+            float* lc = reinterpret_cast<float*>(sm + OFF_LC) + (LONG ? 32 * NH * g : 0);
+            bool res_any = l_res;
             if constexpr (LONG) {
-                if (g == 1) {
-                    asm volatile("" : "+v"(g_sc[0]), "+v"(g_zp[0]), "+v"(g_ms[0]), "+v"(g_mc[0]));
-                    if constexpr (KMAX == 10) {
 #pragma unroll
-                        for (int i = 0; i < 5; ++i) asm volatile("" : "+v"(g_ix10[i]));
+                for (int u = 0; u < 2; ++u)
 #pragma unroll
-                        for (int i = 0; i < 3; ++i) asm volatile("" : "+v"(g_ov10[i]));
-                    } else {
-                        asm volatile("" : "+v"(g_bm[0]), "+v"(g_ov[0]), "+v"(g_bx[0]));
-                    }
-                }
-            }
-            // LONG: what flips the upper bits of every 7-bit position so that those of this half's tokens read below 32
-            uint32_t flip[3] = {0, 0, 0};
-            if constexpr (LONG) {
-                const uint32_t piece = (static_cast<uint32_t>(n0 >> 5) + g) & ((1u << GTS) - 1);      // uniform
-                // ones at bits 5, 12, 19, ... (bit 0 of a piece number) and 6, 13, 20, ... (bit 1)
-#pragma unroll
-                for (int i = 0; i < 3; ++i) {
-                    uint32_t one = 0, two = 0;
-                    for (int s7 = 0; s7 < KMAX; ++s7) {
-                        if ((7 * s7 + 5) >> 5 == i) one |= 1u << ((7 * s7 + 5) & 31);
-                        if ((7 * s7 + 6) >> 5 == i) two |= 1u << ((7 * s7 + 6) & 31);
-                    }
-                    flip[i] = ((piece & 1u) ? one : 0u) ^ ((piece & 2u) ? two : 0u);
-                }
-            }
+                    for (int sidx = 0; sidx < KMAX; ++sidx)
+                        *reinterpret_cast<uint16_t*>(sm + OFF_TILE + 2 * hw0 + 4 * u + min(l_at[u][sidx] - g * HALF_ROWS, HALF_ROWS)) = l_e[u][sidx];
+            } else {
             // The channel pass of a group in two halves, so that the code bytes of both channels are on their
             // way before either channel's entries need them: positions and code reads, then entries and scatter.
             // The base MFMA takes every position of the K rows as it is stored; the tile entry of an
@@ -483,34 +570,16 @@
             auto walk_read = [&](auto U, int (&pos)[KMAX], uint32_t (&cb)[KMAX]) {
                 constexpr int u = decltype(U)::value;
                 uint32_t bm = 0, ix_lo = 0, ix_hi = 0;
-                uint32_t ixw[3] = {0, 0, 0};             // 10 outliers: the channel's 70 index bits
-                if constexpr (KMAX == 10) {
-                    // the lane's bytes start 0 or 2 bytes into the loaded dwords; channel 1's stream 9 bytes on
-                    const uint32_t sh = ((lane & 1) ? 16u : 0u) + (u ? 8u : 0u);
-#pragma unroll
-                    for (int i = 0; i < 3; ++i)
-                        ixw[i] = (i == 2 && u) ? g_ix10[4] >> sh : __builtin_amdgcn_alignbit(g_ix10[i + 1 + 2 * u], g_ix10[i + 2 * u], sh);
-#pragma unroll
-                    for (int i = 0; i < 3; ++i) ixw[i] ^= flip[i];
-                } else if constexpr (IDX == 0) {
+                if constexpr (IDX == 0) {
                     bm = g_bm[pg][u];
                 } else {
                     ix_lo = u ? __builtin_amdgcn_alignbit(g_bx[pg], g_bm[pg][1], 16) : g_bm[pg][0];
                     ix_hi = u ? (g_bx[pg] >> 16) : g_bm[pg][1];
-                    if constexpr (LONG) { ix_lo ^= flip[0]; ix_hi ^= flip[1]; }
                 }
                 const uint8_t* kt = sm + kt_lane + g * 32 * KT_ROW;
 #pragma unroll
                 for (int sidx = 0; sidx < KMAX; ++sidx) {
-                    if constexpr (LONG) {
-                        // (the position with the half's own bits flipped to zero: below 32 when it lies here)
-                        constexpr uint32_t PM = (1u << GT_SH) - 1;
-                        const int bit = 7 * sidx, wi = bit >> 5, bo = bit & 31;
-                        const uint32_t lo = KMAX == 10 ? ixw[wi] : (wi ? ix_hi : ix_lo);
-                        const uint32_t hi = KMAX == 10 ? ixw[wi < 2 ? wi + 1 : 2] : ix_hi;
-                        const uint32_t f = (bo + GT_SH <= 32 ? (lo >> bo) : __builtin_amdgcn_alignbit(hi, lo, bo)) & PM;
-                        pos[sidx] = static_cast<int>(min(f, 32u));
-                    } else if constexpr (IDX == 0) {
+                    if constexpr (IDX == 0) {
                         pos[sidx] = __builtin_ctz(bm) & 31;
                         if (sidx < KMAX - 1) bm &= bm - 1;
                     } else {
@@ -540,20 +609,7 @@
                     a1 = sc;
                     b1 = 0.0f;
                 }
-                float lv[KMAX < 8 ? 8 : KMAX];
-                if constexpr (KMAX == 10) {
-                    // the lane's bytes start 0 or 2 bytes into the loaded dwords; channel u: bytes 5u .. 5u+4
-                    const uint32_t sh = ((lane & 1) ? 16u : 0u) + (u ? 8u : 0u);
-                    const uint32_t o0 = __builtin_amdgcn_alignbit(g_ov10[1 + u], g_ov10[u], sh);
-                    const uint32_t o1 = u ? g_ov10[2] >> sh : __builtin_amdgcn_alignbit(g_ov10[2], g_ov10[1], sh);
-                    const f32x2 l01 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(o0, 1.0f, 0);
-                    const f32x2 l23 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(o0, 1.0f, 1);
-                    const f32x2 l45 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(o0, 1.0f, 2);
-                    const f32x2 l67 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(o0, 1.0f, 3);
-                    const f32x2 l89 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(o1, 1.0f, 0);
-                    lv[0] = l01[0]; lv[1] = l01[1]; lv[2] = l23[0]; lv[3] = l23[1]; lv[4] = l45[0]; lv[5] = l45[1];
-                    lv[6] = l67[0]; lv[7] = l67[1]; lv[8] = l89[0]; lv[9] = l89[1];
-                } else {
+                float lv[8];
                 const uint64_t ov64 = (static_cast<uint64_t>(g_ov[pg][1]) << 32) | g_ov[pg][0];
                 const uint32_t nib = GEN ? static_cast<uint32_t>(ov64 >> (nib_sh + 8 * kbytes * u))
                                          : static_cast<uint32_t>(ov64 >> (nib_sh + 24 * u)) & 0xFFFFFFu;
@@ -563,7 +619,6 @@
                 const f32x2 l67 = KMAX > 6 ? __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(nib, 1.0f, 3) : f32x2{0.0f, 0.0f};
                 lv[0] = l01[0]; lv[1] = l01[1]; lv[2] = l23[0]; lv[3] = l23[1]; lv[4] = l45[0]; lv[5] = l45[1];
                 lv[6] = l67[0]; lv[7] = l67[1];
-                }
                 uint16_t* dt = reinterpret_cast<uint16_t*>(sm + OFF_TILE) + hw0 + 2 * u;      // pair order, like MAG
                 float dl_max = 0.0f;
 #pragma unroll
@@ -576,10 +631,7 @@
                     dls[sidx] = dl;
                     if (GEN && sidx >= kout) continue;          // an unused slot (uniform): nothing to write
                     dt[pos[sidx] * (TILE_ROW / 2)] = __builtin_bit_cast(uint16_t, static_cast<_Float16>(dl));
-                    // (longer groups: of the outliers that lie in this half; with those of the others, whose code byte is not their
-                    // own, most halves took the pass below for nothing: 32 requests of 1 to 16 K 109.5 -> 105.5 us with 64 x 64
-                    // vectors, 131 -> 126 with 128 x 128 and ten outliers, 136 -> 130 with 64 q heads)
-                    dl_max = fmaxf(dl_max, !LONG || pos[sidx] < 32 ? fabsf(dl) : 0.0f);
+                    dl_max = fmaxf(dl_max, fabsf(dl));
                 }
                 return dl_max;
             };
@@ -593,18 +645,8 @@
                 for (int sidx = 0; sidx < KMAX; ++sidx) {
                     if (GEN && sidx >= kout) continue;
                     const float dl = dls[sidx];
-                    bool matters = fabsf(dl) >= big_thr[u];
-                    if constexpr (ANY)
-                        matters |= q_down >= HUGE_Q_DOWN && fabsf(dl) < MIN_F16 && dl != static_cast<float>(static_cast<_Float16>(dl));
-                    if (matters && (!LONG || pos[sidx] < 32)) {
-                        float hi = static_cast<float>(static_cast<_Float16>(dl));
-                        if constexpr (ANY) {
-                            if (fabsf(dl) > MAX_F16) {           // the tile takes the largest f16, the logits the rest
-                                hi = copysignf(MAX_F16, dl);
-                                reinterpret_cast<uint16_t*>(sm + OFF_TILE)[hw0 + 2 * u + pos[sidx] * (TILE_ROW / 2)] =
-                                    __builtin_bit_cast(uint16_t, static_cast<_Float16>(hi));
-                            }
-                        }
+                    if (fabsf(dl) >= big_thr[u]) {
+                        const float hi = static_cast<float>(static_cast<_Float16>(dl));
                         const float lo = (dl - hi) * un;
                         if constexpr (HALF && !PARTIAL) {
                             // (the lane's channels belong to one kv head of the pair: the other's queries read zero there, and half
@@ -630,33 +672,20 @@
             int pos0[KMAX], pos1[KMAX];
             uint32_t cb0[KMAX], cb1[KMAX];
             float dls0[KMAX], dls1[KMAX];
-            // (the general form and longer groups have fewer registers to spare: one channel after the other there)
-            constexpr bool ONE_BY_ONE = GEN || LONG;
+            // (the general form has fewer registers to spare: one channel after the other there)
             walk_read(std::integral_constant<int, 0>{}, pos0, cb0);
-            if constexpr (!ONE_BY_ONE) walk_read(std::integral_constant<int, 1>{}, pos1, cb1);
+            if constexpr (!GEN) walk_read(std::integral_constant<int, 1>{}, pos1, cb1);
             const float dlm0 = walk_write(std::integral_constant<int, 0>{}, pos0, cb0, dls0);
-            // (longer groups: the first channel's residuals before the second's walk, whose entries take its registers)
-            constexpr bool SOON = LONG;
-            bool res_any = false;
-            if constexpr (SOON) {
-                res_any = (ANY && q_down >= HUGE_Q_DOWN) || __any(dlm0 >= big_thr[0]) != 0;
-                if (res_any) residuals(std::integral_constant<int, 0>{}, pos0, dls0);
-            }
-            if constexpr (ONE_BY_ONE) walk_read(std::integral_constant<int, 1>{}, pos1, cb1);
+            if constexpr (GEN) walk_read(std::integral_constant<int, 1>{}, pos1, cb1);
             const float dlm1 = walk_write(std::integral_constant<int, 1>{}, pos1, cb1, dls1);
-            if constexpr (SOON) {
-                const bool res1 = (ANY && q_down >= HUGE_Q_DOWN) || __any(dlm1 >= big_thr[1]) != 0;
-                if (res1) residuals(std::integral_constant<int, 1>{}, pos1, dls1);
-                res_any |= res1;
-            } else {
-                res_any = __any(dlm0 >= big_thr[0] || dlm1 >= big_thr[1]) != 0;
-                if (__builtin_expect(res_any, 0)) {
-                    residuals(std::integral_constant<int, 0>{}, pos0, dls0);
-                    residuals(std::integral_constant<int, 1>{}, pos1, dls1);
-                }
+            res_any = __any(dlm0 >= big_thr[0] || dlm1 >= big_thr[1]) != 0;
+            if (__builtin_expect(res_any, 0)) {
+                residuals(std::integral_constant<int, 0>{}, pos0, dls0);
+                residuals(std::integral_constant<int, 1>{}, pos1, dls1);
+            }
             }
             lds_fence();
-            if (more && (!LONG || g == 1)) fetch_params_g(pg);
+            if (more && !LONG) fetch_params_g(pg);
             // both 16-token blocks of the group go through the eight k-steps together (two independent
             // accumulation chains): tile rows (read, clear), then the base codes
             f32x4 d[2] = {f32x4{0, 0, 0, 0}, f32x4{0, 0, 0, 0}};
@@ -752,18 +781,18 @@
                 for (int t2 = 0; t2 < 2; ++t2)
                     if (kq == 2 * g + t2) dsel[0] = d[t2];
                 if (res_any) {       // exact residuals of this group's large deltas, then zero again
-                    const f32x4 corr = *reinterpret_cast<const f32x4*>(sm + OFF_LC + 16 * (lane & 31));
+                    const f32x4 corr = *reinterpret_cast<const f32x4*>(lc + 4 * (lane & 31));
                     if ((kq >> 1) == g) dsel[0] += corr;
                     lds_fence();
-                    *reinterpret_cast<u32x4*>(sm + OFF_LC + 16 * (lane & 31)) = u32x4{0, 0, 0, 0};
+                    *reinterpret_cast<u32x4*>(lc + 4 * (lane & 31)) = u32x4{0, 0, 0, 0};
                 }
             } else {
                 dsel[g] = (kq >> 1) ? d[1] : d[0];
                 if (res_any) {
                     // the lane's token of this group, its four heads
-                    dsel[g] += *reinterpret_cast<const f32x4*>(sm + OFF_LC + 32 * (16 * (kq >> 1) + j) + 16 * (kq & 1));
+                    dsel[g] += *reinterpret_cast<const f32x4*>(lc + 8 * (16 * (kq >> 1) + j) + 4 * (kq & 1));
                     lds_fence();
-                    *reinterpret_cast<u32x4*>(sm + OFF_LC + 16 * lane) = u32x4{0, 0, 0, 0};
+                    *reinterpret_cast<u32x4*>(lc + 4 * lane) = u32x4{0, 0, 0, 0};
                 }
             }
             lds_fence();

@@ -345,7 +345,7 @@ def test_longer_groups_on_the_matrix_core_kernel(gt, gc, k, hq, own_map):
 @pytest.mark.parametrize("gt,gc,k,hq,own_map", [(64, 64, 6, 32, False), (128, 64, 6, 64, True), (128, 128, 10, 32, True),
                                                 (128, 32, 10, 64, False)])
 def test_longer_groups_cut_into_pieces(gt, gc, k, hq, own_map):
-    """The kernel takes a longer group in pieces of 64 tokens and walks the group's outliers once per 32: lengths that
+    """The kernel takes a longer group in pieces of 64 tokens and scatters the group's outliers once per 32: lengths that
     end a piece after 1, 31, 32, 33, 63 and 64 tokens, in every quarter of a group, dealt out piece by piece, and
     steps of 2^5 and more (the operand without its constant, once per half of a piece)."""
     lens = [2 * gt + n for n in (1, 31, 32, 33, 63, 64, gt - 31, gt - 1, gt)]
@@ -473,6 +473,27 @@ def test_longer_groups_change_their_form_in_the_middle_of_a_split(gt, gc, k, hq,
     want = _oracle(case)
     for S in (None, 1, 3):
         _check(_run(case, num_kv_splits=S), want, f"S{S}")
+
+
+@pytest.mark.parametrize("gt,gc,k,hq,own_map", [(64, 64, 6, 32, False), (128, 64, 6, 64, True), (128, 128, 10, 32, True),
+                                                (128, 128, 10, 64, False)])
+def test_longer_groups_settle_the_rounding_of_either_half(gt, gc, k, hq, own_map):
+    """Queries 8 times as large (below the 2^12 that asks for the second form): the f16 rounding of an outlier's entry, some
+    24 * 2^-12 of it, is up to 24 * 24 * 2^-12 * 128^-0.5 = 1.2e-2 of a logit unless its residual is added, to the right token of
+    the 64 of a step, in the first piece of a group and in the last, which is cut inside its first half and inside its second."""
+    case = build_decode_case([1700, 1030], q_heads=hq, kv_heads=8, head_dim=128, seed=93, permute_tables=True, sparse_frac=0.005,
+                             outlier_repr="relidx7", outliers_per_vector=k, group_tokens=gt, group_channels=gc,
+                             kv_outlier_map=own_map)
+    case.q.mul_(8.0)
+    cut = case.b_seq_len.cpu() - torch.tensor([64 - 17, 64 - 45], dtype=torch.int32)
+    case.b_seq_len.copy_(cut)
+    case.extra["packed_lens"] = cut.tolist()
+    wo, wl = _oracle(case)
+    for S in (None, 3):
+        o, lse = _run(case, num_kv_splits=S)
+        d = (o.double() - wo).abs()
+        assert d.max().item() <= MAX_ABS and d.mean().item() <= MEAN_ABS, f"S{S}: {d.max().item():.3e}"
+        assert ((lse.double() - wl).abs() <= 2e-3 + 1e-5 * wl.abs()).all(), f"S{S}: lse"
 
 
 @pytest.mark.parametrize("lens,hq,hkv,D,kw", [
