@@ -41,7 +41,7 @@ __device__ __forceinline__ int med3_i32(int a, int b, int c) {
 }
 
 // IDXT: index plane known at compile time (0 bitmap, 1 relidx7) or read from the arguments (2).  APART: K and V of a group
-// in workgroups of their own (blockIdx.z); an instantiation, as the two tests in the other one cost a full chip 1 %.
+// in workgroups of their own; an instantiation, as the two tests in the other one cost a full chip 1 %.
 // RING: the groups come as arguments, rows in a ring history and destinations by group; completed groups of a decode step
 // need no tables written by a launch before (pack_list, 1.4 us and its gap).
 struct NoRing {};
@@ -50,15 +50,16 @@ template <bool F32, bool FAST6, int IDXT, bool APART, bool RING = false>
 __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_kernel(StoreArgs a, std::conditional_t<RING, RingGroups, NoRing> ring) {
     static_assert(!(F32 && FAST6), "the tuned path reads bf16 input");
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    const bool do_k = !APART || blockIdx.z == 0, do_v = !APART || blockIdx.z == 1;
-    if (copied_row<APART>(a)) return;
+    StorePlace at;
+    if (!store_place<APART>(a, at)) return;
+    const bool do_k = !at.second, do_v = !APART || at.second;
     // head_dim 128 is compiled in for the tuned instantiations (their launch checks it): row offsets
     // of the code tile become instruction immediates
     const int D = FAST6 ? 128 : a.D;
     uint8_t* s_codes = smem;                       // [32][D] one code per byte
     uint8_t* s_oval = smem + 32 * D;               // [D][nval] nibble bytes, packed as in memory
     uint8_t* s_oidx = smem + 36 * D;               // [D][nidx] position stream bytes (relidx7 only)
-    const int g = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+    const int g = at.g, h = at.h, tid = threadIdx.x;
     const int NGV = D >> 5;
     const int kout = a.kout, kt = (kout + 1) >> 1, kb = kout - kt;
     const int nval = (kout + 1) >> 1;              // nibble bytes per frame
@@ -459,7 +460,7 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
         a.v_zp[vidx] = zp_b;
         }
     }
-    if (do_k) write_own_tables(a, g, tid);
+    if (do_k) write_own_tables(a, g, h, tid);
     if (err && a.err) report_store_bits(a, err);
 }
 

@@ -39,22 +39,40 @@ struct StoreArgs {
     int32_t *own_pages, *own_groups;      // with a block of its own: its identity tables, written on the way instead of by a
                                           // launch of their own (4096-token block, whole call: 33.4 -> 31.9 us)
     int ring_span;          // rows of the ring the groups lie in (RingGroups)
-    int groups;             // T / gt; workgroups beyond them copy rows into the history (bf16), H rows per blockIdx.x
+    int groups;             // T / gt; workgroups beyond them copy rows into the history (bf16)
     BlockRows rows;
 };
 
+// Where a workgroup's place in the grid puts it.  Workgroups go to the eight dies (XCDs) in turn, each with an L2 of its own, and
+// a token's row of a plane holds all heads side by side: 32 bytes of codes, 4 and 8 of steps and zero points a head.
+// So the heads of eight groups are dispatched together, and the heads of one group to one die, whose L2 puts
+// the lines together before they leave: x is 8 h + g % 8, y (and z, past 32768 of them) counts eights of groups.
+// Groups side by side, as before, had the lines of a row written from eight dies one after the other, in pieces of 4 to
+// 32 bytes: 32 K tokens of 8 heads into a pool 47.3 -> 43.0 us, with position streams 16 K 24.8 -> 23.4, at head_dim 64 32 K
+// 31.8 -> 29.5, 64 x 64 vectors 32 K 52.7 -> 49.4; blocks that all run at once (8 K tokens and fewer) the same or 2 % faster.
 // Rows of a prompt ride along with its packed groups: workgroups behind those of the groups copy a row each while the
-// groups are still being packed.  They are slices of z when the groups take two workgroups each (z 0 and 1; at most
-// kStoreApart of them run empty), of y otherwise (a row slice of a full chip is mostly empty).  True when the workgroup had
-// no group.  A fresh prompt of 4096 rows, all of them kept: 7.3 + 9.1 us as two launches, 12.0 as one (13.8 with the rows'
-// slices between those of K and of V).
+// groups are still being packed.  A fresh prompt of 4096 rows, all of them kept: 7.3 + 9.1 us as two launches, 12.0 as one.
+constexpr int kStoreEights = 32768;
+struct StorePlace {
+    int g, h;
+    bool second;            // APART: the workgroup does V
+};
+// False when the workgroup has no group: it copied a row, or is beyond the last group.
 template <bool APART>
-__device__ __forceinline__ bool copied_row(const StoreArgs& a) {
-    const int past = APART ? static_cast<int>(blockIdx.z) - 2 : static_cast<int>(blockIdx.y) - a.H;
-    if (past < 0) return false;
-    const int n = ((APART ? past * a.H + static_cast<int>(blockIdx.y) : past)) * a.groups + static_cast<int>(blockIdx.x);
-    if (n < a.rows.rows) copy_block_row<false>(a.rows, n);
-    return true;
+__device__ __forceinline__ bool store_place(const StoreArgs& a, StorePlace& p) {
+    const int eights = (a.groups + 7) >> 3, x = blockIdx.x;
+    int e = static_cast<int>(blockIdx.z) * kStoreEights + static_cast<int>(blockIdx.y);
+    const int past = e - (APART ? 2 : 1) * eights;
+    if (past >= 0) {
+        const int n = past * 8 * a.H + x;
+        if (n < a.rows.rows) copy_block_row<false>(a.rows, n);
+        return false;
+    }
+    p.second = APART && e >= eights;
+    if (p.second) e -= eights;
+    p.g = 8 * e + (x & 7);
+    p.h = x >> 3;
+    return p.g < a.groups;
 }
 
 // A workgroup each for K and V of a group and head?  Two against one, 8 heads: 5.4 against 6.4 us (32 tokens), 5.5 / 6.7 (1024), 8.4 / 10.0
@@ -64,13 +82,13 @@ constexpr int kStoreApart = 2048;
 inline bool store_apart(const StoreArgs& a) { return a.groups * static_cast<int64_t>(a.H) <= kStoreApart; }
 template <bool APART>
 inline dim3 store_grid(const StoreArgs& a) {
-    const int each = APART ? a.groups * a.H : a.groups, slices = (a.rows.rows + each - 1) / each;
-    return APART ? dim3(a.groups, a.H, 2 + slices) : dim3(a.groups, a.H + slices);
+    const int64_t n = (APART ? 2 : 1) * ((a.groups + 7LL) / 8) + (a.rows.rows + 8LL * a.H - 1) / (8LL * a.H);
+    return dim3(8 * a.H, static_cast<unsigned>(n < kStoreEights ? n : kStoreEights), static_cast<unsigned>((n + kStoreEights - 1) / kStoreEights));
 }
 
 // Entries of the identity tables that belong to K group g: the pages that begin in it, and its own.
-__device__ __forceinline__ void write_own_tables(const StoreArgs& a, int g, int tid) {
-    if (!a.own_groups || blockIdx.y != 0) return;
+__device__ __forceinline__ void write_own_tables(const StoreArgs& a, int g, int h, int tid) {
+    if (!a.own_groups || h != 0) return;
     const int first = (g * a.gt + a.ps - 1) / a.ps, end = ((g + 1) * a.gt + a.ps - 1) / a.ps;
     for (int p = first + tid; p < end; p += blockDim.x) a.own_pages[p] = p;
     if (tid == 0) a.own_groups[g] = g;

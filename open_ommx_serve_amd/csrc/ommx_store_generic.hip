@@ -24,12 +24,13 @@ template <bool F32, int GT, int GC>
 __global__ void __launch_bounds__(256) store_generic_kernel(StoreArgs a) {
     constexpr int MW = (GT + 31) / 32;              // 32-bit words of a lane mask
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    if (copied_row<false>(a)) return;
+    StorePlace place;
+    if (!store_place<false>(a, place)) return;
     const int D = a.D, H = a.H;
     uint8_t* s_codes = smem;                        // [GT][D] one code per byte
     uint8_t* s_oval = smem + GT * D;                // [D][nval]
     uint8_t* s_oidx = s_oval + 8 * D;               // [D][nidx]
-    const int g = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+    const int g = place.g, h = place.h, tid = threadIdx.x;
     const int kout = a.kout;
     const int nval = (kout + 1) >> 1;
     const int nidx = kout == 0 ? 0 : (a.idx_repr == 0 ? (GT + 7) / 8 : (7 * kout + 7) / 8);
@@ -243,7 +244,7 @@ __global__ void __launch_bounds__(256) store_generic_kernel(StoreArgs a) {
         else reinterpret_cast<uint16_t*>(a.v_scale)[vidx] = st.bits;
         a.v_zp[vidx] = zp_b;
     }
-    write_own_tables(a, g, tid);
+    write_own_tables(a, g, h, tid);
     if (err && a.err) report_store_bits(a, err);
 }
 

@@ -96,7 +96,8 @@ __global__ void __launch_bounds__(512, GT < GC ? 1 : GT == 32 ? 8 : GT == 64 ? 5
     constexpr int SORT = K <= 8 ? 8 : 12;                      // LDS bytes per thread and sorted list
     constexpr int NVAL = K / 2, NIDX = (7 * K + 7) / 8;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    if (copied_row<false>(a)) return;
+    StorePlace place;
+    if (!store_place<false>(a, place)) return;
     const int D = a.D, H = a.H, pieces = D >> 5;
     uint16_t* const s_k = reinterpret_cast<uint16_t*>(smem);   // [GT][D] the K tile
     uint8_t* const s_codes = smem + 2 * GT * D;                // [GT][D] one code per byte
@@ -104,7 +105,7 @@ __global__ void __launch_bounds__(512, GT < GC ? 1 : GT == 32 ? 8 : GT == 64 ? 5
     uint8_t* const s_fp4 = s_pos + SORT * D;
     uint8_t* const s_oval = s_fp4 + SORT * D;                  // [D][NVAL] as in memory
     uint8_t* const s_oidx = s_oval + 8 * D;                    // [D][bytes of the index plane] as in memory
-    const int g = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, NT = 2 * D;
+    const int g = place.g, h = place.h, tid = threadIdx.x, NT = 2 * D;
     const int nidx = a.idx_repr == 0 ? GT / 8 : NIDX;
     const int64_t gs = a.dst_groups ? a.dst_groups[g] : g;
     const float* __restrict__ tab = a.table;
@@ -422,7 +423,7 @@ __global__ void __launch_bounds__(512, GT < GC ? 1 : GT == 32 ? 8 : GT == 64 ? 5
         reinterpret_cast<uint64_t*>(a.k_base)[(phys_row(page_of(tk), tk) * H + h) * pieces + j] = kb8;
     }
 
-    write_own_tables(a, g, tid);
+    write_own_tables(a, g, h, tid);
     if (err && a.err) report_store_bits(a, err);
 }
 

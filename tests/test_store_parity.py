@@ -530,3 +530,38 @@ def test_store_in_one_and_in_two_workgroups_a_group(rep, fp32):
         got = bits_of(whole[n])
         assert np.array_equal(got[:len(bits_of(first[n]))], bits_of(first[n])), n
         assert np.array_equal(got[len(bits_of(first[n])):], bits_of(last[n])), n
+
+
+@pytest.mark.parametrize("G,H,D,kw", [
+    (1, 1, 128, {}), (1, 8, 128, {}), (7, 3, 128, {}), (8, 8, 128, {}), (9, 2, 128, {}), (17, 5, 128, dict(outlier_repr="relidx7")),
+    (261, 8, 128, {}), (9, 3, 64, {}), (7, 1, 32, dict(outliers_per_vector=3)),
+    (9, 3, 128, dict(outlier_repr="relidx7", group_tokens=64, group_channels=64))])
+def test_every_group_and_head_has_its_workgroup(G, H, D, kw):
+    """Workgroups are handed out by eights of groups, all heads of an eight together: counts around a multiple of eight, one
+    head and odd numbers of them, K and V in one workgroup (261 x 8 groups and heads) and in two."""
+    K, V = synth_kv(G * kw.get("group_tokens", 32), H, D, 70 + G + H, outlier_channels=4, sparse_frac=0.01)
+    got, want = _hip(K, V, **kw), O.pack_kv(K, V, **{"outliers_per_vector": 6, **kw})
+    for n in ("k_base", "k_scale", "k_zp", "k_oval", "k_obmp", "k_oidx", "k_fp4_mapscale", "k_fp4_mapcenter",
+              "v_main", "v_scale", "v_zp"):
+        if want.get(n) is not None:
+            assert np.array_equal(bits_of(got[n]), bits_of(want[n])), n
+
+
+def test_more_eights_of_groups_than_one_dimension_of_a_grid():
+    """4.2 M tokens in 16-token groups are 32770 eights: the last of them and the first, against blocks of their own."""
+    T = 16 * (8 * 32769 + 3)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    K = torch.randn(T, 1, 32, generator=g, device="cuda", dtype=torch.bfloat16)
+    V = torch.randn(T, 1, 32, generator=g, device="cuda", dtype=torch.bfloat16)
+    kw = dict(outliers_per_vector=2, group_tokens=16, group_channels=16)
+    planes = alloc_planes(T // 16, T // 16, 1, 32, device="cuda", **kw)
+    err = torch.zeros(1, dtype=torch.int32, device="cuda")
+    store_pack_into(K, V, planes, err_flag=err, **kw)
+    assert int(err.item()) == 0
+    for t0 in (0, 16 * 8 * 32767, 16 * 8 * 32769 - 64):
+        t1 = min(T, t0 + 16 * 16)
+        own = alloc_planes((t1 - t0) // 16, (t1 - t0) // 16, 1, 32, device="cuda", **kw)
+        store_pack_into(K[t0:t1], V[t0:t1], own, err_flag=err, **kw)
+        for n, p in own.items():
+            if torch.is_tensor(p):
+                assert torch.equal(planes[n][t0 // 16:t1 // 16].view(torch.uint8), p.view(torch.uint8)), (n, t0)
