@@ -20,26 +20,6 @@
 
 namespace ommx {
 
-// Order-preserving integer image of a bf16 value held as fp32 bits, low 16 bits cleared.
-// -0 must have been turned into +0 before (they tie in the reference's sorts).
-__device__ __forceinline__ int ordered_bits(float x) {
-    const int b = __float_as_int(x);
-    return (b ^ ((b >> 31) & 0x7FFFFFFF)) & static_cast<int>(0xFFFF0000u);
-}
-// The same for a value whose low 16 bits are zero (a bf16 widened to fp32): nothing to clear.
-__device__ __forceinline__ int ordered_bits_bf16(float x) {
-    const int b = __float_as_int(x);
-    return b ^ ((b >> 31) & 0x7FFF0000);
-}
-__device__ __forceinline__ float from_ordered_bits(int k) {
-    const int s = k & static_cast<int>(0xFFFF0000u);
-    // the image is its own inverse: the sign bit stays, the others flip under a set sign
-    return __int_as_float(s ^ ((s >> 31) & 0x7FFF0000));
-}
-__device__ __forceinline__ int med3_i32(int a, int b, int c) {
-    return max(min(a, b), min(max(a, b), c));          // v_med3_i32
-}
-
 // IDXT: index plane known at compile time (0 bitmap, 1 relidx7) or read from the arguments (2).  APART: K and V of a group
 // in workgroups of their own; an instantiation, as the two tests in the other one cost a full chip 1 %.
 // RING: the groups come as arguments, rows in a ring history and destinations by group; completed groups of a decode step
@@ -61,7 +41,7 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
     uint8_t* s_oidx = smem + 36 * D;               // [D][nidx] position stream bytes (relidx7 only)
     const int g = at.g, h = at.h, tid = threadIdx.x;
     const int NGV = D >> 5;
-    const int kout = a.kout, kt = (kout + 1) >> 1, kb = kout - kt;
+    const int kout = FAST6 ? 6 : a.kout, kt = (kout + 1) >> 1, kb = kout - kt;
     const int nval = (kout + 1) >> 1;              // nibble bytes per frame
     RingGroup from = {0, INT_MAX, 0};
     if constexpr (RING) from = ring.of[g];
@@ -76,13 +56,30 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
     // ------------------------------------------------------------------ K vector
     if (do_k) {
         const int d = tid;
-        float w[32];
+        float w[FAST6 ? 1 : 32];
+        uint32_t pair[FAST6 ? 16 : 1];              // FAST6: tokens 2i and 2i + 1 as they are in memory
+        uint32_t even = 0;
+        auto take = [&](int i, auto v) {
+            if constexpr (FAST6) {
+                if (i & 1) pair[i >> 1] = even | static_cast<uint32_t>(v) << 16;
+                else even = v;
+            } else if constexpr (F32) {
+                w[i] = v;
+            } else {
+                w[i] = bf16_to_f32(v);
+            }
+        };
+        auto value = [&](int i) {                   // (i known at compile time)
+            if constexpr (FAST6) return __uint_as_float((i & 1) ? pair[i >> 1] & 0xFFFF0000u : pair[i >> 1] << 16);
+            else return w[i];
+        };
+        typedef std::conditional_t<F32, float, uint16_t> elem;
         bool fin = true;
         if (!RING && a.src_rows) {
 #pragma unroll
             for (int i = 0; i < 32; ++i) {
                 const int64_t row = a.src_rows[g * 32 + i];
-                w[i] = load_elem<F32>(a.K, row * a.k_ts + (int64_t)h * a.k_hs + d);
+                take(i, static_cast<const elem*>(a.K)[row * a.k_ts + (int64_t)h * a.k_hs + d]);
             }
         } else {
             // consecutive rows: the row address is the same for the whole workgroup (scalar registers,
@@ -95,8 +92,7 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
             const uint32_t off = static_cast<uint32_t>(d) * (F32 ? 4u : 2u);
 #pragma unroll
             for (int i = 0; i < 32; ++i) {
-                if (F32) w[i] = *reinterpret_cast<const __attribute__((address_space(1))) float*>(reinterpret_cast<gptr>(row) + off);
-                else w[i] = bf16_to_f32(*reinterpret_cast<const __attribute__((address_space(1))) uint16_t*>(reinterpret_cast<gptr>(row) + off));
+                take(i, *reinterpret_cast<const __attribute__((address_space(1))) elem*>(reinterpret_cast<gptr>(row) + off));
                 row += stride;
                 if (RING && i + 1 == from.turn) row -= stride * static_cast<uint64_t>(a.ring_span);
                 asm volatile("" : "+s"(row));        // keeps the row address a scalar of its own: folded into one
@@ -105,7 +101,7 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
         }
         if (!FAST6) {
 #pragma unroll
-            for (int i = 0; i < 32; ++i) fin = fin && is_finite_f32(w[i]);
+            for (int i = 0; i < 32; ++i) fin = fin && is_finite_f32(value(i));
         }
 
         uint32_t top = 0, bot = 0;
@@ -121,7 +117,7 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
     #pragma unroll
                     for (int i = 0; i < 32; ++i) {
                         const bool free_lane = !((top >> i) & 1u);
-                        if (free_lane && (bi < 0 || fabsf(w[i]) > best)) { best = fabsf(w[i]); bi = i; }
+                        if (free_lane && (bi < 0 || fabsf(value(i)) > best)) { best = fabsf(value(i)); bi = i; }
                     }
                     if (bi >= 0) top |= 1u << bi;
                 }
@@ -134,7 +130,7 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
     #pragma unroll
                 for (int i = 0; i < 32; ++i) {
                     const bool free_lane = !((top >> i) & 1u);
-                    if (free_lane && (bi < 0 || w[i] > best)) { best = w[i]; bi = i; }
+                    if (free_lane && (bi < 0 || value(i) > best)) { best = value(i); bi = i; }
                 }
                 if (bi >= 0) top |= 1u << bi;
             }
@@ -144,7 +140,7 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
                 float best = 0.0f; int bi = -1;
     #pragma unroll
                 for (int i = 0; i < 32; ++i) {
-                    const float v = ((top >> i) & 1u) ? 1e9f : w[i];
+                    const float v = ((top >> i) & 1u) ? 1e9f : value(i);
                     const bool free_lane = !((bot >> i) & 1u);
                     if (free_lane && (bi < 0 || v < best)) { best = v; bi = i; }
                 }
@@ -152,30 +148,33 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
             }
         };
         bool fast_done = false, ranks_clean = false;
-        if (FAST6) {
-            // bf16 inputs leave 16 free bits under the value: key = ordered value bits | tie
+        if constexpr (FAST6) {
+            // bf16 inputs leave 16 free bits under the value: key = rank of the value | tie
             // breaker.  Largest three: tie breaker 31-i with max (equal values: lower index
             // first, the stable descending sort).  Smallest three: tie breaker i with min.
             // One pass each through a three-deep max / median network.
             // (a fourth rank on either side: the largest and the smallest of the lanes that stay)
-            int t1 = INT_MIN, t2 = INT_MIN, t3 = INT_MIN;
-            int b1 = INT_MAX, b2 = INT_MAX, b3 = INT_MAX;
+            // The ranks are formed two at once in packed 16-bit integers and the keys in one instruction each, the medians are
+            // spelled out.  With that, the extremes of V below and a shorter x / 3 a wave issues some 1040 vector instructions,
+            // 1220 before (a SIMD's vector unit is busy for 94 % of the launch): 32 K tokens into a pool 43.0 -> 41.2 us, 16 K
+            // with position streams 23.3 -> 21.7, 8 K 13.4 -> 13.0.
+            int t[4], b[4];
 #pragma unroll
-            for (int i = 0; i < 32; ++i) {
-                const int ob = ordered_bits_bf16(w[i] + 0.0f);                   // FAST6 is a bf16-input instantiation
-                const int kt_i = ob | (31 - i), kb_i = ob | i;
-                const int n4 = med3_i32(t3, t4, kt_i), n3 = med3_i32(t2, t3, kt_i), n2 = med3_i32(t1, t2, kt_i);
-                t1 = max(t1, kt_i); t2 = n2; t3 = n3; t4 = n4;
-                const int m4 = med3_i32(b3, b4, kb_i), m3 = med3_i32(b2, b3, kb_i), m2 = med3_i32(b1, b2, kb_i);
-                b1 = min(b1, kb_i); b2 = m2; b3 = m3; b4 = m4;
+            for (int i = 0; i < 32; i += 2) {
+                const uint32_t y = ranks_of(pair[i >> 1]);
+                keep_largest(t, key_low(y, 31 - i), i);
+                keep_smallest(b, key_low(y, i), i);
+                keep_largest(t, key_high(y, 30 - i), i + 1);
+                keep_smallest(b, key_high(y, i + 1), i + 1);
             }
             // (the fourth ranks are pinned here: left to the compiler, their two chains of 32 steps
             // move down into the one branch that reads them, and all 64 keys stay live until then)
+            t4 = t[3]; b4 = b[3];
             asm volatile("" : "+v"(t4), "+v"(b4));
-            top = (1u << (31 - (t1 & 31))) | (1u << (31 - (t2 & 31))) | (1u << (31 - (t3 & 31)));
-            bot = (1u << (b1 & 31)) | (1u << (b2 & 31)) | (1u << (b3 & 31));
-            key_hi[0] = t1; key_hi[1] = t2; key_hi[2] = t3;
-            key_lo[0] = b1; key_lo[1] = b2; key_lo[2] = b3;
+            top = (1u << (31 - (t[0] & 31))) | (1u << (31 - (t[1] & 31))) | (1u << (31 - (t[2] & 31)));
+            bot = (1u << (b[0] & 31)) | (1u << (b[1] & 31)) | (1u << (b[2] & 31));
+#pragma unroll
+            for (int j = 0; j < 3; ++j) { key_hi[j] = t[j]; key_lo[j] = b[j]; }
             // The reference takes the smallest three of the vector with the top lanes moved
             // to +1e9.  That is the same set unless a top lane is among the overall smallest
             // three (heavy ties): then the bottom ranks are taken again with those lanes at +1e9.
@@ -184,18 +183,17 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
             // count.)
             ranks_clean = (top & bot) == 0u;
             if (!ranks_clean) {
-                b1 = INT_MAX; b2 = INT_MAX; b3 = INT_MAX;
+                int c[3] = {INT_MAX, INT_MAX, INT_MAX};
 #pragma unroll
                 for (int i = 0; i < 32; ++i) {
-                    float wi = w[i];
+                    uint32_t wi = __float_as_uint(value(i));
                     asm volatile("" : "+v"(wi));      // formed again here: 32 keys kept from the first pass would cost 32 registers
                     // (the reference's own sentinel, so that a vector it refuses is refused here too)
-                    const int kb_i = ordered_bits(((top >> i) & 1u) ? 1e9f : wi + 0.0f) | i;
-                    const int m3 = med3_i32(b2, b3, kb_i), m2 = med3_i32(b1, b2, kb_i);
-                    b1 = min(b1, kb_i); b2 = m2; b3 = m3;
+                    keep_smallest(c, (((top >> i) & 1u) ? static_cast<int>(__float_as_uint(1e9f) & 0xFFFF0000u) : rank_of(wi)) | i);
                 }
-                bot = (1u << (b1 & 31)) | (1u << (b2 & 31)) | (1u << (b3 & 31));
-                key_lo[0] = b1; key_lo[1] = b2; key_lo[2] = b3;
+                bot = (1u << (c[0] & 31)) | (1u << (c[1] & 31)) | (1u << (c[2] & 31));
+#pragma unroll
+                for (int j = 0; j < 3; ++j) key_lo[j] = c[j];
             }
             fast_done = true;
         }
@@ -204,10 +202,10 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
         if (FAST6 && fast_done) {
             // NaN / Inf sort to the ends of the ordered keys: the largest and the smallest
             // chosen value tell whether the whole vector is finite
-            fin = is_finite_f32(from_ordered_bits(key_hi[0])) && is_finite_f32(from_ordered_bits(key_lo[0]));
+            fin = is_finite_f32(value_of_rank(key_hi[0])) && is_finite_f32(value_of_rank(key_lo[0]));
         } else if (FAST6) {
 #pragma unroll
-            for (int i = 0; i < 32; ++i) fin = fin && is_finite_f32(w[i]);
+            for (int i = 0; i < 32; ++i) fin = fin && is_finite_f32(value(i));
         }
         if (!fin) err |= OMMX_ERR_NONFINITE_K;
         if (__popc(om) != kout) err |= OMMX_ERR_UNDERFILLED;
@@ -221,10 +219,10 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
         // takes depends on the lanes, not on the ranks.
         bool ranks_do = false;
         if (FAST6 && ranks_clean) {
-            mn = from_ordered_bits(b4);
-            mx = from_ordered_bits(t4);
-            omn = from_ordered_bits(key_lo[0]);
-            omx = from_ordered_bits(key_hi[0]);
+            mn = value_of_rank(b4);
+            mx = value_of_rank(t4);
+            omn = value_of_rank(key_lo[0]);
+            omx = value_of_rank(key_hi[0]);
             ranks_do = mn != 0.0f && (omn != 0.0f || omx != 0.0f);
         }
         if (!ranks_do) {
@@ -232,17 +230,17 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
 #pragma unroll
             for (int i = 0; i < 32; ++i) {
                 const bool o = (om >> i) & 1u;
-                mn = fminf(mn, o ? 1e9f : w[i]);
-                mx = fmaxf(mx, o ? -1e9f : w[i]);
-                omn = fminf(omn, o ? w[i] : 1e9f);
-                omx = fmaxf(omx, o ? w[i] : -1e9f);
+                mn = fminf(mn, o ? 1e9f : value(i));
+                mx = fmaxf(mx, o ? -1e9f : value(i));
+                omn = fminf(omn, o ? value(i) : 1e9f);
+                omx = fmaxf(omx, o ? value(i) : -1e9f);
             }
         }
         if (mn > 1e8f) mn = 0.0f;
         if (mx < -1e8f) mx = 0.0f;
         if (omn > 1e8f) omn = 0.0f;
         if (omx < -1e8f) omx = 0.0f;
-        const float raw = __fdiv_rn(fmaxf(mx - mn, 1e-8f), 3.0f);
+        const float raw = third(fmaxf(mx - mn, 1e-8f));
         const Step st = make_step(raw, scale_mode, tab);
         if (!st.in_range) err |= OMMX_ERR_EXP_RANGE;
         if (st.e > 15) err |= OMMX_NOTE_WIDE_STEP;      // beyond the f16 operands of the matrix-core decode
@@ -280,15 +278,15 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
             if (inv_ok && fabsf(zc) < INFINITY) {      // one branch per vector, not one per element
 #pragma unroll
                 for (int i = 0; i < 32; ++i)
-                    s_codes[i * D + d] = static_cast<uint8_t>(int2_code_fused(w[i], inv_scale, zc));
+                    s_codes[i * D + d] = static_cast<uint8_t>(int2_code_fused(value(i), inv_scale, zc));
             } else if (inv_ok) {
 #pragma unroll
                 for (int i = 0; i < 32; ++i)
-                    s_codes[i * D + d] = static_cast<uint8_t>(int2_code(w[i] - zp, scale, inv_scale, true));
+                    s_codes[i * D + d] = static_cast<uint8_t>(int2_code(value(i) - zp, scale, inv_scale, true));
             } else {
 #pragma unroll
                 for (int i = 0; i < 32; ++i)
-                    s_codes[i * D + d] = static_cast<uint8_t>(int2_code(w[i] - zp, scale, inv_scale, false));
+                    s_codes[i * D + d] = static_cast<uint8_t>(int2_code(value(i) - zp, scale, inv_scale, false));
             }
             // |(w - mc) * ms| is largest at the extreme lanes, which are outliers: they decide
             // whether every mapped value is finite (codec.py:55-57 checks all of them)
@@ -301,8 +299,8 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
             for (int r = 0; r < 6; ++r) {
                 const int key = r < 3 ? key_hi[r] : key_lo[r - 3];
                 const int pos = r < 3 ? 31 - (key & 31) : (key & 31);
-                const float mapped = fp4_input(from_ordered_bits(key));
-                mfin = mfin && is_finite_f32(mapped);
+                const float mapped = fp4_input(value_of_rank(key));
+                if (r % 3 == 0) mfin = mfin && is_finite_f32(mapped);
                 const int slot = __popc(om & ((1u << pos) - 1u));
                 nib |= fp4_encode_sorted(mapped, thr) << (4 * slot);
             }
@@ -310,9 +308,9 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
             int slot = 0;
 #pragma unroll
             for (int i = 0; i < 32; ++i) {
-                s_codes[i * D + d] = static_cast<uint8_t>(int2_code(w[i] - zp, scale, inv_scale, inv_ok));
+                s_codes[i * D + d] = static_cast<uint8_t>(int2_code(value(i) - zp, scale, inv_scale, inv_ok));
                 if (kout > 0) {
-                    const float mapped = fp4_input(w[i]);
+                    const float mapped = fp4_input(value(i));
                     mfin = mfin && is_finite_f32(mapped);
                     if ((om >> i) & 1u) {
                         nib |= fp4_encode(mapped, tab + 256) << (4 * slot);
@@ -390,11 +388,7 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
         const int64_t row = RING ? from.row + t - (t >= from.turn ? a.ring_span : 0) : a.src_rows ? a.src_rows[tok] : tok;
         const int64_t vbase = row * a.v_ts + (int64_t)h * a.v_hs + 32 * j;
         float v[32];
-        bool fin = true;
-        // finite <=> exponent field not all ones: the largest exponent field of the vector decides
         if (!F32 && a.v_vec) {                    // 64 contiguous bytes: four 16-byte loads
-            typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-            u16x2 e2 = {0, 0};                    // largest exponent field of the even / of the odd channels
             const uint4* vp = reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(a.V) + vbase);
 #pragma unroll
             for (int q4 = 0; q4 < 4; ++q4) {
@@ -404,27 +398,22 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
                 for (int k = 0; k < 4; ++k) {
                     v[8 * q4 + 2 * k] = __uint_as_float(uw[k] << 16);
                     v[8 * q4 + 2 * k + 1] = __uint_as_float(uw[k] & 0xFFFF0000u);
-                    e2 = __builtin_elementwise_max(e2, __builtin_bit_cast(u16x2, uw[k] & 0x7F807F80u));
                 }
             }
-            fin = e2[0] != 0x7F80 && e2[1] != 0x7F80;
         } else {
-            uint32_t emax = 0;
 #pragma unroll
-            for (int c = 0; c < 32; ++c) {
-                v[c] = load_elem<F32>(a.V, vbase + c);
-                emax = max(emax, __float_as_uint(v[c]) & 0x7F800000u);
-            }
-            fin = emax != 0x7F800000u;
+            for (int c = 0; c < 32; ++c) v[c] = load_elem<F32>(a.V, vbase + c);
         }
-        float mn = 0.0f, mx = 0.0f;
+        // (the IEEE minimum and maximum, which a NaN goes through: the two tell whether the whole vector is finite; -0 below +0)
+        float mn = v[0], mx = v[0];
 #pragma unroll
-        for (int c = 0; c < 32; ++c) {
-            mn = c == 0 ? v[c] : fminf(mn, v[c]);
-            mx = c == 0 ? v[c] : fmaxf(mx, v[c]);
+        for (int c = 1; c < 32; ++c) {
+            mn = __builtin_elementwise_minimum(mn, v[c]);
+            mx = __builtin_elementwise_maximum(mx, v[c]);
         }
+        const bool fin = is_finite_f32(mn) && is_finite_f32(mx);
         if (!fin) err |= OMMX_ERR_NONFINITE_V;
-        const float raw = __fdiv_rn(fmaxf(mx - mn, 1e-8f), 3.0f);
+        const float raw = third(fmaxf(mx - mn, 1e-8f));
         const Step st = make_step(raw, scale_mode, tab);
         if (!st.in_range) err |= OMMX_ERR_EXP_RANGE;
         if (st.e > 15) err |= OMMX_NOTE_WIDE_STEP;

@@ -167,6 +167,69 @@ __device__ __forceinline__ Step make_step(float raw, int mode, const float* tab)
     return s;
 }
 
+// x / 3 rounded once, for x >= 1e-8 or infinite: a quotient within one unit and one exact remainder step, four instructions
+// against the ten of a division by a variable (held against it for every mantissa).  The remainder of an infinity is NaN and
+// is taken as a finite number, which leaves the infinity.
+__device__ __forceinline__ float third(float x) {
+    constexpr float r = 1.0f / 3.0f;
+    const float q = x * r;
+    return __builtin_fmaf(fmaxf(__builtin_fmaf(-3.0f, q, x), -3.0e38f), r, q);
+}
+
+// Ranks.  A bf16 value (in the high half of a word, the low half zero) as a two's complement number in the same place: zeros of
+// both signs give 0, infinities and NaN lie at the ends.  Its inverse takes a key, whose low half holds a tie breaker.
+__device__ __forceinline__ int rank_of(uint32_t b) {
+    const int w = static_cast<int>(b), s = w >> 31;
+    return (w ^ (s & 0x7FFFFFFF)) - s;
+}
+__device__ __forceinline__ float value_of_rank(int key) {
+    const int v = key & static_cast<int>(0xFFFF0000u), s = v >> 31;
+    return __int_as_float((v + s) ^ (s & 0x7FFFFFFF));
+}
+// The same for two values at once.
+typedef int16_t s16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t ranks_of(uint32_t two) {
+    const s16x2 s = __builtin_bit_cast(s16x2, two) >> s16x2{15, 15};
+    const uint32_t x = (__builtin_bit_cast(uint32_t, s) & 0x7FFF7FFFu) ^ two;
+    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(s16x2, x) - s);
+}
+// Keys of the two: rank, and a tie breaker below 64 in the low half.  One instruction each, which the compiler would take
+// apart to share the shift and the mask.
+__device__ __forceinline__ int key_low(uint32_t two, int tie) {
+    int k;
+    asm("v_lshl_or_b32 %0, %1, 16, %2" : "=v"(k) : "v"(two), "n"(tie));
+    return k;
+}
+__device__ __forceinline__ int key_high(uint32_t two, int tie) {
+    int k;
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(k) : "v"(two), "s"(0xFFFF0000u), "n"(tie));
+    return k;
+}
+// Median, spelled out: where two of the three are known to be in order the compiler takes a minimum and a maximum instead.
+__device__ __forceinline__ int med3_i32(int a, int b, int c) {
+    int m;
+    asm("v_med3_i32 %0, %1, %2, %3" : "=v"(m) : "v"(a), "v"(b), "v"(c));
+    return m;
+}
+// N largest (smallest) keys in order from the end; the last one is the extreme of the rest.  `held` keys are there already
+// (known at compile time while there are fewer than N).
+template <int N>
+__device__ __forceinline__ void keep_largest(int (&t)[N], int key, int held = N) {
+    if (held > 0 && held < N) t[held] = min(t[held - 1], key);
+#pragma unroll
+    for (int j = N - 1; j > 0; --j)
+        if (j < held) t[j] = med3_i32(t[j - 1], t[j], key);
+    t[0] = held == 0 ? key : max(t[0], key);
+}
+template <int N>
+__device__ __forceinline__ void keep_smallest(int (&t)[N], int key, int held = N) {
+    if (held > 0 && held < N) t[held] = max(t[held - 1], key);
+#pragma unroll
+    for (int j = N - 1; j > 0; --j)
+        if (j < held) t[j] = med3_i32(t[j - 1], t[j], key);
+    t[0] = held == 0 ? key : min(t[0], key);
+}
+
 // INT2 code clamp(rint(x / 2^e), 0, 3) of a finite x.  v_cvt_pk_u8_f32 rounds to nearest even
 // and saturates below at 0; the upper clamp commutes with the rounding.
 __device__ __forceinline__ uint32_t int2_code(float x, float scale, float inv_scale, bool inv_ok) {

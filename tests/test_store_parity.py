@@ -8,6 +8,7 @@ import oracle.ommx_oracle as O
 from conftest import (GOLDEN_CASES, PLANE_NAMES, VARIANT_CASES, assert_planes_equal,
                       assert_variant_planes_equal, bits_of, load_golden, load_variant,
                       tensor_from_bits)
+from open_ommx_serve_amd.attention import _hip as _hip_lib
 from open_ommx_serve_amd.attention import pack as hip_pack
 from open_ommx_serve_amd.attention.pack import (alloc_planes, ommx_pack_kv_canonical_block,
                                                 store_pack_into)
@@ -565,3 +566,25 @@ def test_more_eights_of_groups_than_one_dimension_of_a_grid():
         for n, p in own.items():
             if torch.is_tensor(p):
                 assert torch.equal(planes[n][t0 // 16:t1 // 16].view(torch.uint8), p.view(torch.uint8)), (n, t0)
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), -float("inf")])
+@pytest.mark.parametrize("T", [64, 64 * 140])                 # K and V of a group in two workgroups, and in one
+def test_one_value_that_is_not_finite_is_found_wherever_it_lies(T, bad):
+    """The extremes of a V vector and the first ranks of a K vector tell whether all of it is finite: every place of a minimum or
+    maximum of three, every rank of a tie (a vector of equal values), first and last elements."""
+    K, V = synth_kv(T, 2, 128, 11)
+    K[:, :, 5] = 1.0
+    K, V = K.cuda(), V.cuda()
+    planes = alloc_planes(T // 16, T // 32, 2, 128, device="cuda")
+    for which, t, h, c in [("V", t, t & 1, c) for t in (0, 33) for c in (0, 1, 2, 30, 31, 32, 97, 127)] + \
+                          [("K", t, 1, c) for t in (0, 1, 15, 30, 31, T - 1) for c in (5, 127)]:
+        k, v = K.clone(), V.clone()
+        (k if which == "K" else v)[t, h, c] = bad
+        err = torch.zeros(1, dtype=torch.int32, device="cuda")
+        store_pack_into(k, v, planes, err_flag=err)
+        want = _hip_lib.ERR_NONFINITE_K if which == "K" else _hip_lib.ERR_NONFINITE_V
+        assert int(err.item()) & want, (which, t, h, c)
+        err.zero_()
+        store_pack_into(K, V, planes, err_flag=err)
+        assert int(err.item()) == 0
