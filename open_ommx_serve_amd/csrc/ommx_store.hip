@@ -20,19 +20,19 @@
 
 namespace ommx {
 
-// IDXT: index plane known at compile time (0 bitmap, 1 relidx7) or read from the arguments (2).  APART: K and V of a group
-// in workgroups of their own; an instantiation, as the two tests in the other one cost a full chip 1 %.
+// IDXT: index plane known at compile time (0 bitmap, 1 relidx7) or read from the arguments (2).  ORDER: K and V of a group
+// in one workgroup or in workgroups of their own; an instantiation, as the two tests in the other one cost a full chip 1 %.
 // RING: the groups come as arguments, rows in a ring history and destinations by group; completed groups of a decode step
 // need no tables written by a launch before (pack_list, 1.4 us and its gap).
 struct NoRing {};
-template <bool F32, bool FAST6, int IDXT, bool APART, bool RING = false>
+template <bool F32, bool FAST6, int IDXT, StoreOrder ORDER, bool RING = false>
 // (six waves per SIMD for the tuned bitmask instantiation, which fits their 80 registers without spilling)
 __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_kernel(StoreArgs a, std::conditional_t<RING, RingGroups, NoRing> ring) {
     static_assert(!(F32 && FAST6), "the tuned path reads bf16 input");
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     StorePlace at;
-    if (!store_place<APART>(a, at)) return;
-    const bool do_k = !at.second, do_v = !APART || at.second;
+    if (!store_place<ORDER>(a, at)) return;
+    const bool do_k = !at.second, do_v = ORDER == kByEights || at.second;
     // head_dim 128 is compiled in for the tuned instantiations (their launch checks it): row offsets
     // of the code tile become instruction immediates
     const int D = FAST6 ? 128 : a.D;
@@ -476,20 +476,26 @@ extern "C" void ommx_store_default_table(float* t) {
 }
 
 namespace ommx {
-template <bool APART>
 static void launch_store_pack(int variant, const StoreArgs& a, hipStream_t st) {
-    const dim3 grid = store_grid<APART>(a), block(a.D);
+    const bool apart = store_apart(a), in_line = variant == 0 || variant == 3 || a.groups * static_cast<int64_t>(a.H) <= kStoreInLine;
+    const StoreOrder order = !apart ? kByEights : in_line ? kApartInLine : kApartByEights;
+    const dim3 grid = store_grid(a, order), block(a.D);
     const size_t shm = 32 * (size_t)a.D + 4 * (size_t)a.D + (a.idx_repr ? 8 * (size_t)a.D : 0);
-    if (variant == 0) hipLaunchKernelGGL((store_pack_kernel<true, false, 2, APART>), grid, block, shm, st, a, NoRing{});
-    else if (variant == 1) hipLaunchKernelGGL((store_pack_kernel<false, true, 0, APART>), grid, block, shm, st, a, NoRing{});
-    else if (variant == 2) hipLaunchKernelGGL((store_pack_kernel<false, true, 1, APART>), grid, block, shm, st, a, NoRing{});
-    else hipLaunchKernelGGL((store_pack_kernel<false, false, 2, APART>), grid, block, shm, st, a, NoRing{});
+#define OMMX_GO(F32, FAST6, IDXT, ORDER) hipLaunchKernelGGL((store_pack_kernel<F32, FAST6, IDXT, ORDER>), grid, block, shm, st, a, NoRing{})
+#define OMMX_GO_APART(F32, FAST6, IDXT) do { if (apart) OMMX_GO(F32, FAST6, IDXT, kApartInLine); else OMMX_GO(F32, FAST6, IDXT, kByEights); } while (0)
+    if (variant == 0) OMMX_GO_APART(true, false, 2);
+    else if (variant == 3) OMMX_GO_APART(false, false, 2);
+    else if (order == kApartByEights) { if (variant == 1) OMMX_GO(false, true, 0, kApartByEights); else OMMX_GO(false, true, 1, kApartByEights); }
+    else if (variant == 1) OMMX_GO_APART(false, true, 0);
+    else OMMX_GO_APART(false, true, 1);
+#undef OMMX_GO_APART
+#undef OMMX_GO
 }
 static void launch_store_ring(const StoreArgs& a, const RingGroups& ring, hipStream_t st) {
-    const dim3 grid = store_grid<true>(a), block(a.D);
+    const dim3 grid = store_grid(a, kApartInLine), block(a.D);
     const size_t shm = 36 * (size_t)a.D + (a.idx_repr ? 8 * (size_t)a.D : 0);
-    if (a.idx_repr == 0) hipLaunchKernelGGL((store_pack_kernel<false, true, 0, true, true>), grid, block, shm, st, a, ring);
-    else hipLaunchKernelGGL((store_pack_kernel<false, true, 1, true, true>), grid, block, shm, st, a, ring);
+    if (a.idx_repr == 0) hipLaunchKernelGGL((store_pack_kernel<false, true, 0, kApartInLine, true>), grid, block, shm, st, a, ring);
+    else hipLaunchKernelGGL((store_pack_kernel<false, true, 1, kApartInLine, true>), grid, block, shm, st, a, ring);
 }
 }  // namespace ommx
 
@@ -556,8 +562,7 @@ int ommx::store_pack(const void* K, const void* V, int in_dtype,
         }
     }
     const int variant = in_dtype == 1 ? 0 : !tuned ? 3 : index_repr == 0 ? 1 : 2;
-    if (store_apart(a)) launch_store_pack<true>(variant, a, st);
-    else launch_store_pack<false>(variant, a, st);
+    launch_store_pack(variant, a, st);
     if (hipGetLastError() != hipSuccess) { set_error("ommx_store_pack: launch failed"); return -2; }
     return 0;
 }

@@ -49,17 +49,34 @@ struct StoreArgs {
 // the lines together before they leave: x is 8 h + g % 8, y (and z, past 32768 of them) counts eights of groups.
 // Groups side by side, as before, had the lines of a row written from eight dies one after the other, in pieces of 4 to
 // 32 bytes: 32 K tokens of 8 heads into a pool 47.3 -> 43.0 us, with position streams 16 K 24.8 -> 23.4, at head_dim 64 32 K
-// 31.8 -> 29.5, 64 x 64 vectors 32 K 52.7 -> 49.4; blocks that all run at once (8 K tokens and fewer) the same or 2 % faster.
+// 31.8 -> 29.5, 64 x 64 vectors 32 K 52.7 -> 49.4.
+// In line (x the group, y the head, z which of K and V): where the chip is half empty what counts is how soon the workgroups start,
+// and these need nothing but their numbers for that.  Kernel alone, 8 heads, in line against by eights: 1 K tokens 5.6 / 5.8 us,
+// 2 K 6.9 / 7.0, 4 K 7.3 / 7.6, but 6 K 11.4 / 11.1 and 8 K 13.6 / 13.3 (fp32 rows and other outlier counts: always); an instantiation of its own, as a test of which it is
+// waits for the arguments (4 K 7.6).
 // Rows of a prompt ride along with its packed groups: workgroups behind those of the groups copy a row each while the
 // groups are still being packed.  A fresh prompt of 4096 rows, all of them kept: 7.3 + 9.1 us as two launches, 12.0 as one.
 constexpr int kStoreEights = 32768;
+enum StoreOrder { kByEights, kApartInLine, kApartByEights };      // apart: K and V in workgroups of their own
+constexpr int kStoreInLine = 1024;                                 // groups and heads in line
 struct StorePlace {
     int g, h;
-    bool second;            // APART: the workgroup does V
+    bool second;            // apart: the workgroup does V
 };
 // False when the workgroup has no group: it copied a row, or is beyond the last group.
-template <bool APART>
+template <StoreOrder ORDER>
 __device__ __forceinline__ bool store_place(const StoreArgs& a, StorePlace& p) {
+    constexpr bool APART = ORDER != kByEights;
+    if constexpr (ORDER == kApartInLine) {
+        const int past = static_cast<int>(blockIdx.z) - 2;
+        if (past >= 0) {
+            const int n = (past * a.H + static_cast<int>(blockIdx.y)) * a.groups + static_cast<int>(blockIdx.x);
+            if (n < a.rows.rows) copy_block_row<false>(a.rows, n);
+            return false;
+        }
+        p = {static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y), blockIdx.z == 1};
+        return true;
+    }
     const int eights = (a.groups + 7) >> 3, x = blockIdx.x;
     int e = static_cast<int>(blockIdx.z) * kStoreEights + static_cast<int>(blockIdx.y);
     const int past = e - (APART ? 2 : 1) * eights;
@@ -80,9 +97,12 @@ __device__ __forceinline__ bool store_place(const StoreArgs& a, StorePlace& p) {
 // the line the chip is full either way, and the second workgroup is only one more to start.
 constexpr int kStoreApart = 2048;
 inline bool store_apart(const StoreArgs& a) { return a.groups * static_cast<int64_t>(a.H) <= kStoreApart; }
-template <bool APART>
-inline dim3 store_grid(const StoreArgs& a) {
-    const int64_t n = (APART ? 2 : 1) * ((a.groups + 7LL) / 8) + (a.rows.rows + 8LL * a.H - 1) / (8LL * a.H);
+inline dim3 store_grid(const StoreArgs& a, StoreOrder order) {
+    if (order == kApartInLine) {
+        const int each = a.groups * a.H;
+        return dim3(a.groups, a.H, 2 + (a.rows.rows + each - 1) / each);
+    }
+    const int64_t n = (order == kByEights ? 1 : 2) * ((a.groups + 7LL) / 8) + (a.rows.rows + 8LL * a.H - 1) / (8LL * a.H);
     return dim3(8 * a.H, static_cast<unsigned>(n < kStoreEights ? n : kStoreEights), static_cast<unsigned>((n + kStoreEights - 1) / kStoreEights));
 }
 

@@ -25,7 +25,7 @@ __global__ void __launch_bounds__(256) store_generic_kernel(StoreArgs a) {
     constexpr int MW = (GT + 31) / 32;              // 32-bit words of a lane mask
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     StorePlace place;
-    if (!store_place<false>(a, place)) return;
+    if (!store_place<kByEights>(a, place)) return;
     const int D = a.D, H = a.H;
     uint8_t* s_codes = smem;                        // [GT][D] one code per byte
     uint8_t* s_oval = smem + GT * D;                // [D][nval]
@@ -250,7 +250,7 @@ __global__ void __launch_bounds__(256) store_generic_kernel(StoreArgs a) {
 
 template <bool F32, int GT>
 int launch_gt(const StoreArgs& a, int T, hipStream_t st) {
-    const dim3 grid = store_grid<false>(a), block(a.D);
+    const dim3 grid = store_grid(a, kByEights), block(a.D);
     const size_t shm = (size_t)GT * a.D + 8 * (size_t)a.D + 16 * (size_t)a.D;
     switch (a.gc) {
         case 16: hipLaunchKernelGGL((store_generic_kernel<F32, GT, 16>), grid, block, shm, st, a); return 0;

@@ -97,7 +97,7 @@ __global__ void __launch_bounds__(512, GT < GC ? 1 : GT == 32 ? 8 : GT == 64 ? 5
     constexpr int NVAL = K / 2, NIDX = (7 * K + 7) / 8;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     StorePlace place;
-    if (!store_place<false>(a, place)) return;
+    if (!store_place<kByEights>(a, place)) return;
     const int D = a.D, H = a.H, pieces = D >> 5;
     uint16_t* const s_k = reinterpret_cast<uint16_t*>(smem);   // [GT][D] the K tile
     uint8_t* const s_codes = smem + 2 * GT * D;                // [GT][D] one code per byte
@@ -429,7 +429,7 @@ __global__ void __launch_bounds__(512, GT < GC ? 1 : GT == 32 ? 8 : GT == 64 ? 5
 
 template <int GT, int GC>
 int launch_k(const StoreArgs& a, int T, hipStream_t st) {
-    const dim3 grid = store_grid<false>(a), block(2 * a.D);
+    const dim3 grid = store_grid(a, kByEights), block(2 * a.D);
     const size_t shm = static_cast<size_t>(a.D) * (3 * GT + 2 * 12 + 8 + 16);
     if (shm > 64 * 1024) return 1;           // 128 tokens of a 256-channel head: the general kernel
     const int k_vec = reinterpret_cast<uintptr_t>(a.K) % 16 == 0 && a.k_ts % 8 == 0 && a.k_hs % 8 == 0;

@@ -535,11 +535,12 @@ def test_store_in_one_and_in_two_workgroups_a_group(rep, fp32):
 
 @pytest.mark.parametrize("G,H,D,kw", [
     (1, 1, 128, {}), (1, 8, 128, {}), (7, 3, 128, {}), (8, 8, 128, {}), (9, 2, 128, {}), (17, 5, 128, dict(outlier_repr="relidx7")),
-    (261, 8, 128, {}), (9, 3, 64, {}), (7, 1, 32, dict(outliers_per_vector=3)),
+    (129, 8, 128, {}), (171, 6, 128, dict(outlier_repr="relidx7")), (261, 8, 128, {}), (9, 3, 64, {}), (7, 1, 32, dict(outliers_per_vector=3)),
     (9, 3, 128, dict(outlier_repr="relidx7", group_tokens=64, group_channels=64))])
 def test_every_group_and_head_has_its_workgroup(G, H, D, kw):
-    """Workgroups are handed out by eights of groups, all heads of an eight together: counts around a multiple of eight, one
-    head and odd numbers of them, K and V in one workgroup (261 x 8 groups and heads) and in two."""
+    """Workgroups are handed out by eights of groups, all heads of an eight together, or group by group up to 1024 groups and
+    heads: counts around a multiple of eight, one head and odd numbers of them, K and V in one workgroup (261 x 8 groups
+    and heads) and in two."""
     K, V = synth_kv(G * kw.get("group_tokens", 32), H, D, 70 + G + H, outlier_channels=4, sparse_frac=0.01)
     got, want = _hip(K, V, **kw), O.pack_kv(K, V, **{"outliers_per_vector": 6, **kw})
     for n in ("k_base", "k_scale", "k_zp", "k_oval", "k_obmp", "k_oidx", "k_fp4_mapscale", "k_fp4_mapcenter",
