@@ -159,13 +159,15 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
             // 1220 before (a SIMD's vector unit is busy for 94 % of the launch): 32 K tokens into a pool 43.0 -> 41.2 us, 16 K
             // with position streams 23.3 -> 21.7, 8 K 13.4 -> 13.0.
             int t[4], b[4];
+            uint32_t upper = 0xFFFF0000u;
+            asm("" : "+v"(upper));
 #pragma unroll
             for (int i = 0; i < 32; i += 2) {
                 const uint32_t y = ranks_of(pair[i >> 1]);
                 keep_largest(t, key_low(y, 31 - i), i);
                 keep_smallest(b, key_low(y, i), i);
-                keep_largest(t, key_high(y, 30 - i), i + 1);
-                keep_smallest(b, key_high(y, i + 1), i + 1);
+                keep_largest(t, key_high(y, upper, 30 - i), i + 1);
+                keep_smallest(b, key_high(y, upper, i + 1), i + 1);
             }
             // (the fourth ranks are pinned here: left to the compiler, their two chains of 32 steps
             // move down into the one branch that reads them, and all 64 keys stay live until then)

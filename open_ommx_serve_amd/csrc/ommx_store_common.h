@@ -213,16 +213,27 @@ __device__ __forceinline__ uint32_t ranks_of(uint32_t two) {
     const uint32_t x = (__builtin_bit_cast(uint32_t, s) & 0x7FFF7FFFu) ^ two;
     return __builtin_bit_cast(uint32_t, __builtin_bit_cast(s16x2, x) - s);
 }
-// Keys of the two: rank, and a tie breaker below 64 in the low half.  One instruction each, which the compiler would take
-// apart to share the shift and the mask.
+// Keys of the two: rank, and a tie breaker in the low half: a number below 64 that is known at compile time, or (_s) in a scalar
+// register.  One instruction each, which the compiler would take apart to share the shift and the mask; `upper` is
+// 0xFFFF0000 in a vector register (an instruction reads one scalar).
 __device__ __forceinline__ int key_low(uint32_t two, int tie) {
     int k;
     asm("v_lshl_or_b32 %0, %1, 16, %2" : "=v"(k) : "v"(two), "n"(tie));
     return k;
 }
-__device__ __forceinline__ int key_high(uint32_t two, int tie) {
+__device__ __forceinline__ int key_high(uint32_t two, uint32_t upper, int tie) {
     int k;
-    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(k) : "v"(two), "s"(0xFFFF0000u), "n"(tie));
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(k) : "v"(two), "v"(upper), "n"(tie));
+    return k;
+}
+__device__ __forceinline__ int key_low_s(uint32_t two, int tie) {
+    int k;
+    asm("v_lshl_or_b32 %0, %1, 16, %2" : "=v"(k) : "v"(two), "s"(tie));
+    return k;
+}
+__device__ __forceinline__ int key_high_s(uint32_t two, uint32_t upper, int tie) {
+    int k;
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(k) : "v"(two), "v"(upper), "s"(tie));
     return k;
 }
 // Median, spelled out: where two of the three are known to be in order the compiler takes a minimum and a maximum instead.
@@ -263,8 +274,9 @@ __device__ __forceinline__ uint32_t int2_code(float x, float scale, float inv_sc
 // once, and scaling by a power of two commutes with rounding while nothing under- or overflows: an
 // underflowing quotient gives code 0 and an overflowing one code 3 either way.  The caller checks
 // that c is finite (a huge zero point over a tiny step would make it infinite).
-__device__ __forceinline__ uint32_t int2_code_fused(float w, float inv_scale, float c) {
-    return __builtin_amdgcn_cvt_pk_u8_f32(fminf(__builtin_fmaf(w, inv_scale, c), 3.0f), 0u, 0u);
+// (into byte `at` of `others`)
+__device__ __forceinline__ uint32_t int2_code_fused(float w, float inv_scale, float c, uint32_t at = 0u, uint32_t others = 0u) {
+    return __builtin_amdgcn_cvt_pk_u8_f32(fminf(__builtin_fmaf(w, inv_scale, c), 3.0f), at, others);
 }
 
 int launch_store_long(const StoreArgs& a, int T, int in_dtype, hipStream_t st);

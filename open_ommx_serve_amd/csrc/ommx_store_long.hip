@@ -10,14 +10,18 @@
 // touched 64 cache lines a load and read each of them eight times, more than L1 holds: 32 K tokens of 64 x 64 vectors into a
 // pool 76 -> 57 us, 1024 tokens 11.1 -> 9.9, 16 K tokens at head_dim 64 19.7 -> 17.8.  (The V rows are asked for when the K
 // tile is there and are on their way during the selection; asked for before it they delay it, 57 -> 61 us.)
-// The K tile comes in by 16-byte loads through LDS, and both passes over a
+// The K tile comes in by 16-byte loads through LDS, two tokens of a channel a word, and both passes over a
 // channel (selection, codes) are loops that read it there: held in registers and unrolled, 128 tokens overrun the
 // register file, and a straight-line body of 20-30 KB that every wave runs once is bound by instruction
 // fetch.  Selection is what remains: the general kernel runs k passes of 5 instructions per element over
 // the vector (64 tokens, 6 outliers: 1920); here one pass through two sorted networks of depth k/2 + 1
-// (max / median of three on keys that hold the ordered bf16 value and the tie breaker) takes k + 7 an
-// element and leaves the extremes of what stays as its last ranks.  The outliers come out of the network by
-// rank and are wanted by position: each thread sorts them through its own few bytes of LDS.
+// (max / median of three on keys that hold the rank of the bf16 value and the tie breaker; ranks of two tokens at
+// once) takes k + 5 an element and leaves the extremes of what stays as its last ranks.  The outliers come out of the
+// network by rank and are wanted by position: position and FP4 code go through a fixed sorting network as one number.
+// The codes of two tokens take the place of the tokens in the tile.  (32 K tokens into a pool, a token a halfword,
+// codes in a tile of their own and the outliers sorted through LDS -> this: 64 x 64 vectors with six outliers 49.4 ->
+// 45.7 us, 128 x 128 with ten 78.6 -> 54.1, which also has four workgroups a compute unit instead of two; 8 K tokens
+// 17.4 -> 16.2 and 24.3 -> 21.4; 11 K at head_dim 64 16.5 -> 15.1.)
 #include <limits.h>
 
 #include <utility>
@@ -27,33 +31,27 @@
 namespace ommx {
 namespace {
 
-__device__ __forceinline__ int ordered_pair_half(uint32_t b) {      // b: a bf16 in the high half, low half zero
-    const int s = static_cast<int>(b);
-    return s ^ ((s >> 31) & 0x7FFF0000);
+// Ascending order by a fixed network of compare-exchanges (12 for six, 29 for ten).
+__device__ __forceinline__ void in_order(int& a, int& b) {
+    const int lo = min(a, b);
+    b = max(a, b);
+    a = lo;
 }
-__device__ __forceinline__ float value_of_key(int k) {
-    const int s = k & static_cast<int>(0xFFFF0000u);
-    return __int_as_float(s ^ ((s >> 31) & 0x7FFF0000));
-}
-__device__ __forceinline__ int med3(int a, int b, int c) { return max(min(a, b), min(max(a, b), c)); }
-
-// N largest keys in descending order; the last one is the largest of the rest
-template <int N>
-__device__ __forceinline__ void keep_largest(int (&t)[N], int key) {
+__device__ __forceinline__ void sort_ascending(int (&x)[6]) {
+    constexpr int net[12][2] = {{0, 5}, {1, 3}, {2, 4}, {1, 2}, {3, 4}, {0, 3}, {2, 5}, {0, 1}, {2, 3}, {4, 5}, {1, 2}, {3, 4}};
 #pragma unroll
-    for (int j = N - 1; j > 0; --j) t[j] = med3(t[j - 1], t[j], key);
-    t[0] = max(t[0], key);
+    for (int i = 0; i < 12; ++i) in_order(x[net[i][0]], x[net[i][1]]);
 }
-template <int N>
-__device__ __forceinline__ void keep_smallest(int (&t)[N], int key) {
+__device__ __forceinline__ void sort_ascending(int (&x)[10]) {
+    constexpr int net[29][2] = {{0, 8}, {1, 9}, {2, 7}, {3, 5}, {4, 6}, {0, 2}, {1, 4}, {5, 8}, {7, 9}, {0, 3},
+                                {2, 4}, {5, 7}, {6, 9}, {0, 1}, {3, 6}, {8, 9}, {1, 5}, {2, 3}, {4, 8}, {6, 7},
+                                {1, 2}, {3, 5}, {4, 6}, {7, 8}, {2, 3}, {4, 5}, {6, 7}, {3, 4}, {5, 6}};
 #pragma unroll
-    for (int j = N - 1; j > 0; --j) t[j] = med3(t[j - 1], t[j], key);
-    t[0] = min(t[0], key);
+    for (int i = 0; i < 29; ++i) in_order(x[net[i][0]], x[net[i][1]]);
 }
 
 // The extremes of bf16 values in packed 16-bit integers: b ^ (sign ? 0x7FFF : 0) orders them (-0 below +0, as v_min_f32 has
 // it; infinities and NaN at the ends), two at once.
-typedef int16_t s16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ s16x2 pair_image(uint32_t two) {
     const s16x2 m = __builtin_bit_cast(s16x2, two) >> s16x2{15, 15};
     return __builtin_bit_cast(s16x2, (__builtin_bit_cast(uint32_t, m) & 0x7FFF7FFFu) ^ two);
@@ -86,24 +84,21 @@ __device__ __forceinline__ void each_of(F&& f, std::integer_sequence<int, I...>)
 template <int N, class F>
 __device__ __forceinline__ void each(F&& f) { each_of<N>(f, std::make_integer_sequence<int, N>{}); }
 
-// k_vec: K rows allow 16-byte loads.  As many waves a SIMD as the LDS allows (128 tokens: of head_dim 64), which the compiler
-// has to be told: with the extremes of V in floats it took 78 to 256 registers by itself (64 tokens, 32 K into a pool 72 us
-// instead of 61; 128 tokens at head_dim 64, 24 K into a block 40.6 instead of 36.7).  In packed integers they take a third of
-// the registers and half of the instructions: 45 / 72 / 136, 11 K tokens at head_dim 64 14.4 -> 13.9 us.
+// k_vec: K rows allow 16-byte loads.  As many waves a SIMD as the LDS allows (128 tokens: four, with up to nine registers in
+// scratch memory; with three and none 32 K tokens into a pool take 56.5 us instead of 54.1), which the compiler has to be
+// told: with the extremes of V in floats it took 78 to 256 registers by itself.  In packed integers they take a third of
+// the registers and half of the instructions.
 template <int GT, int GC, int KH>
-__global__ void __launch_bounds__(512, GT < GC ? 1 : GT == 32 ? 8 : GT == 64 ? 5 : 3) store_long_kernel(StoreArgs a, int k_vec) {
+__global__ void __launch_bounds__(512, GT < GC ? 1 : GT == 32 ? 8 : GT == 64 ? 7 : 4) store_long_kernel(StoreArgs a, int k_vec) {
     constexpr int K = 2 * KH, MW = GT / 32, TIE = GT - 1;      // GT is a power of two: the tie breaker is its low bits
-    constexpr int SORT = K <= 8 ? 8 : 12;                      // LDS bytes per thread and sorted list
     constexpr int NVAL = K / 2, NIDX = (7 * K + 7) / 8;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     StorePlace place;
     if (!store_place<kByEights>(a, place)) return;
     const int D = a.D, H = a.H, pieces = D >> 5;
-    uint16_t* const s_k = reinterpret_cast<uint16_t*>(smem);   // [GT][D] the K tile
-    uint8_t* const s_codes = smem + 2 * GT * D;                // [GT][D] one code per byte
-    uint8_t* const s_pos = s_codes + GT * D;                   // [D][SORT] positions, then FP4 codes, by slot
-    uint8_t* const s_fp4 = s_pos + SORT * D;
-    uint8_t* const s_oval = s_fp4 + SORT * D;                  // [D][NVAL] as in memory
+    uint32_t* const s_k = reinterpret_cast<uint32_t*>(smem);   // [GT / 2][D] the K tile, two tokens of a channel a word; then their
+                                                               // two codes in the word's lower bytes
+    uint8_t* const s_oval = smem + 2 * GT * D;                 // [D][NVAL] as in memory
     uint8_t* const s_oidx = s_oval + 8 * D;                    // [D][bytes of the index plane] as in memory
     const int g = place.g, h = place.h, tid = threadIdx.x, NT = 2 * D;
     const int nidx = a.idx_repr == 0 ? GT / 8 : NIDX;
@@ -137,34 +132,53 @@ __global__ void __launch_bounds__(512, GT < GC ? 1 : GT == 32 ? 8 : GT == 64 ? 5
         for (int n = 0; n < VP; ++n) vu[n] = *reinterpret_cast<const u32x4_a2*>(v_base + row[n] * a.v_ts);
     };
     if (k_vec) {
-        constexpr int KP = GT / 16;                // 16-byte pieces of the K tile a thread: rows k_row, k_row + 16, ...
+        constexpr int KP = GT / 32;                // 16-byte pieces of two rows a thread: pairs k_row, k_row + 16, ...
         const int k_row = tid / (D / 8), c = 8 * (tid % (D / 8));
         const uint16_t* const base = static_cast<const uint16_t*>(a.K) + (int64_t)h * a.k_hs + c;
-        uint4 ku[KP];
+        u32x4 ku[KP][2];
 #pragma unroll
-        for (int n = 0; n < KP; ++n) ku[n] = *reinterpret_cast<const uint4*>(base + src_row(16 * n + k_row) * a.k_ts);
+        for (int n = 0; n < KP; ++n)
 #pragma unroll
-        for (int n = 0; n < KP; ++n) *reinterpret_cast<uint4*>(s_k + (16 * n + k_row) * D + c) = ku[n];
+            for (int o = 0; o < 2; ++o) ku[n][o] = *reinterpret_cast<const u32x4*>(base + src_row(2 * (16 * n + k_row) + o) * a.k_ts);
+#pragma unroll
+        for (int n = 0; n < KP; ++n) {
+            u32x4* const to = reinterpret_cast<u32x4*>(s_k + (16 * n + k_row) * D + c);
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {          // channels c + 4q .. c + 4q + 3
+                u32x4 w;
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    w[2 * e] = __builtin_amdgcn_perm(ku[n][1][2 * q + e], ku[n][0][2 * q + e], 0x05040100u);
+                    w[2 * e + 1] = __builtin_amdgcn_perm(ku[n][1][2 * q + e], ku[n][0][2 * q + e], 0x07060302u);
+                }
+                to[q] = w;
+            }
+        }
     } else {
         for (int i = tid; i < GT * D; i += NT)
-            s_k[i] = static_cast<const uint16_t*>(a.K)[src_row(i / D) * a.k_ts + (int64_t)h * a.k_hs + i % D];
+            reinterpret_cast<uint16_t*>(s_k)[2 * ((i / D >> 1) * D + i % D) + (i / D & 1)] =
+                static_cast<const uint16_t*>(a.K)[src_row(i / D) * a.k_ts + (int64_t)h * a.k_hs + i % D];
     }
     __syncthreads();
 
     // ------------------------------------------------------------------ K vector
     if (tid < D) {
         const int d = tid;
-        auto one = [&](int i) { return bf16_to_f32(s_k[i * D + d]); };       // token i of this thread's channel
+        auto two = [&](int i) { return s_k[i * D + d]; };                    // tokens 2i and 2i + 1 of this thread's channel
+        auto one = [&](int i) { return bf16_to_f32(reinterpret_cast<const uint16_t*>(s_k)[2 * ((i >> 1) * D + d) + (i & 1)]); };
 
-        // (adding +0 turns -0 into +0: they tie in the reference's sorts)
         int t[KH + 1], b[KH + 1];
+        uint32_t upper = 0xFFFF0000u;
+        asm("" : "+v"(upper));
 #pragma unroll
         for (int j = 0; j <= KH; ++j) { t[j] = INT_MIN; b[j] = INT_MAX; }
-#pragma unroll 8
-        for (int i = 0; i < GT; ++i) {
-            const int ob = ordered_pair_half(__float_as_uint(one(i) + 0.0f));
-            keep_largest(t, ob | (TIE - i));           // equal values: the lower position first
-            keep_smallest(b, ob | i);
+#pragma unroll 4
+        for (int i = 0; i < GT; i += 2) {
+            const uint32_t y = ranks_of(two(i >> 1));  // (zeros of both signs have one rank: they tie in the reference's sorts)
+            keep_largest(t, key_low_s(y, TIE - i));      // equal values: the lower position first
+            keep_smallest(b, key_low_s(y, i));
+            keep_largest(t, key_high_s(y, upper, TIE - i - 1));
+            keep_smallest(b, key_high_s(y, upper, i + 1));
         }
 #pragma unroll
         for (int j = 0; j <= KH; ++j) asm volatile("" : "+v"(t[j]), "+v"(b[j]));
@@ -191,8 +205,8 @@ __global__ void __launch_bounds__(512, GT < GC ? 1 : GT == 32 ? 8 : GT == 64 ? 5
             for (int cc = 0; cc < MW; ++cc) {
 #pragma unroll 1
                 for (int i = 0; i < 32; ++i) {
-                    const uint32_t bits = ((top[cc] >> i) & 1u) ? __float_as_uint(1e9f) & 0xFFFF0000u : __float_as_uint(one(32 * cc + i) + 0.0f);
-                    keep_smallest(c, ordered_pair_half(bits) | i | (32 * cc));
+                    const uint32_t bits = ((top[cc] >> i) & 1u) ? __float_as_uint(1e9f) & 0xFFFF0000u : __float_as_uint(one(32 * cc + i));
+                    keep_smallest(c, rank_of(bits) | i | (32 * cc));
                 }
             }
 #pragma unroll
@@ -204,13 +218,13 @@ __global__ void __launch_bounds__(512, GT < GC ? 1 : GT == 32 ? 8 : GT == 64 ? 5
 #pragma unroll
         for (int w = 0; w < MW; ++w) { om[w] = top[w] | bot[w]; picked += __popc(om[w]); }
         // NaN / Inf sort to the ends of the ordered keys
-        if (!is_finite_f32(value_of_key(t[0])) || !is_finite_f32(value_of_key(b[0]))) err |= OMMX_ERR_NONFINITE_K;
+        if (!is_finite_f32(value_of_rank(t[0])) || !is_finite_f32(value_of_rank(b[0]))) err |= OMMX_ERR_NONFINITE_K;
         if (picked != K) err |= OMMX_ERR_UNDERFILLED;
 
         // affine base over the other lanes (pack.py:455-465): their extremes are the ranks after the chosen
         // ones.  A zero minimum, or zeros at both outlier ends, go the long way: which sign a zero result takes
         // depends on the lanes, not on the ranks.
-        float mn = value_of_key(b[KH]), mx = value_of_key(t[KH]), omn = value_of_key(b[0]), omx = value_of_key(t[0]);
+        float mn = value_of_rank(b[KH]), mx = value_of_rank(t[KH]), omn = value_of_rank(b[0]), omx = value_of_rank(t[0]);
         if (!(clean && mn != 0.0f && (omn != 0.0f || omx != 0.0f))) {
             mn = 1e9f; mx = -1e9f; omn = 1e9f; omx = -1e9f;
 #pragma unroll
@@ -229,7 +243,7 @@ __global__ void __launch_bounds__(512, GT < GC ? 1 : GT == 32 ? 8 : GT == 64 ? 5
         if (mx < -1e8f) mx = 0.0f;
         if (omn > 1e8f) omn = 0.0f;
         if (omx < -1e8f) omx = 0.0f;
-        const Step st = make_step(__fdiv_rn(fmaxf(mx - mn, 1e-8f), 3.0f), 0, tab);
+        const Step st = make_step(third(fmaxf(mx - mn, 1e-8f)), 0, tab);
         if (!st.in_range) err |= OMMX_ERR_EXP_RANGE;
         if (st.e > 15) err |= OMMX_NOTE_WIDE_STEP;      // beyond the f16 operands of the matrix-core decode
         const uint16_t zp_b = f32_to_bf16_rne(mn);
@@ -247,39 +261,39 @@ __global__ void __launch_bounds__(512, GT < GC ? 1 : GT == 32 ? 8 : GT == 64 ? 5
         const float zc = -zp * st.inv;
         const bool fused_k = st.inv_ok && fabsf(zc) < INFINITY;
         if (fused_k) {
-#pragma unroll 8
-            for (int i = 0; i < GT; ++i) s_codes[i * D + d] = static_cast<uint8_t>(int2_code_fused(one(i), st.inv, zc));
+#pragma unroll 4
+            for (int i = 0; i < GT / 2; ++i) {
+                const uint32_t w = two(i);
+                const uint32_t even = int2_code_fused(__uint_as_float(w << 16), st.inv, zc);
+                s_k[i * D + d] = int2_code_fused(__uint_as_float(w & 0xFFFF0000u), st.inv, zc, 1, even);
+            }
         } else {
 #pragma unroll 1
-            for (int i = 0; i < GT; ++i)
-                s_codes[i * D + d] = static_cast<uint8_t>(int2_code(one(i) - zp, st.scale, st.inv, st.inv_ok));
+            for (int i = 0; i < GT / 2; ++i)
+                s_k[i * D + d] = int2_code(one(2 * i) - zp, st.scale, st.inv, st.inv_ok) |
+                                 int2_code(one(2 * i + 1) - zp, st.scale, st.inv, st.inv_ok) << 8;
         }
 
-        // FP4 codes of the chosen lanes by slot = rank of their position.  |mapped| is largest at the extreme
-        // lanes, which are chosen ones, so these decide whether every mapped value is finite (codec.py:55-57).
+        // FP4 codes of the chosen lanes, in the order of their positions: position and code as one number, sorted.  |mapped| is
+        // largest at the extreme lanes, which are chosen ones, so these decide whether every mapped value is finite
+        // (codec.py:55-57).
         float thr[8];
 #pragma unroll
         for (int j = 1; j < 8; ++j)
             thr[j] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(tab[256 + j])));
         thr[0] = 0.0f;
         bool mfin = true;
+        int slot[K];
 #pragma unroll
         for (int r = 0; r < K; ++r) {
             const int key = r < KH ? t[r] : b[r - KH];
             const int pos = r < KH ? TIE - (key & TIE) : key & TIE;
-            const float wv = value_of_key(key);
+            const float wv = value_of_rank(key);
             const float mapped = own_map ? (wv - mc) * ms : (st.inv_ok ? (wv - zp) * st.inv : __fdiv_rn(wv - zp, st.scale));
-            mfin = mfin && is_finite_f32(mapped);
-            int slot = 0;
-#pragma unroll
-            for (int w = 0; w < MW; ++w) {
-                const uint32_t below = MW == 1 || (pos >> 5) == w ? (1u << (pos & 31)) - 1u : ((pos >> 5) > w ? 0xFFFFFFFFu : 0u);
-                slot += __popc(om[w] & below);
-            }
-            slot = min(slot, SORT - 1);             // (an under-filled set is refused; its slots may repeat)
-            s_pos[SORT * d + slot] = static_cast<uint8_t>(pos);
-            s_fp4[SORT * d + slot] = static_cast<uint8_t>(fp4_encode_sorted(mapped, thr));
+            if (r % KH == 0) mfin = mfin && is_finite_f32(mapped);
+            slot[r] = pos << 4 | static_cast<int>(fp4_encode_sorted(mapped, thr));
         }
+        sort_ascending(slot);
         if (!mfin) err |= OMMX_ERR_NONFINITE_K;
 
         const int64_t gidx = (gs * H + h) * D + d;
@@ -287,18 +301,11 @@ __global__ void __launch_bounds__(512, GT < GC ? 1 : GT == 32 ? 8 : GT == 64 ? 5
         a.k_zp[gidx] = zp_b;
         if (own_map) { a.k_ms[gidx] = ms_b; a.k_mc[gidx] = mc_b; }
 
-        // this thread's own bytes back in slot order (one wave writes and reads them: program order is enough)
-        uint32_t pw[SORT / 4], fw[SORT / 4];
-#pragma unroll
-        for (int w = 0; w < SORT / 4; ++w) {
-            pw[w] = *reinterpret_cast<const uint32_t*>(s_pos + SORT * d + 4 * w);
-            fw[w] = *reinterpret_cast<const uint32_t*>(s_fp4 + SORT * d + 4 * w);
-        }
         uint64_t nib = 0, lo = 0, hi = 0;           // position s at bits [7s, 7s+7) of hi:lo
 #pragma unroll
         for (int s = 0; s < K; ++s) {
-            const uint64_t pos = (pw[s >> 2] >> (8 * (s & 3))) & 0x7Fu;
-            nib |= static_cast<uint64_t>((fw[s >> 2] >> (8 * (s & 3))) & 0xFu) << (4 * s);
+            const uint64_t pos = static_cast<uint32_t>(slot[s]) >> 4;
+            nib |= static_cast<uint64_t>(slot[s] & 0xF) << (4 * s);
             if (7 * s < 64) lo |= pos << (7 * s);
             if (7 * s + 7 > 64) hi |= 7 * s >= 64 ? pos << (7 * s - 64) : pos >> (64 - 7 * s);
         }
@@ -347,7 +354,7 @@ __global__ void __launch_bounds__(512, GT < GC ? 1 : GT == 32 ? 8 : GT == 64 ? 5
             for (int n = 1; n < VL && r + n < VP; ++n) mine = me == n ? ends[r + n] : mine;
             const float my_mn = value_of_image(static_cast<int16_t>(mine)), my_mx = value_of_image(static_cast<int16_t>(~mine >> 16));
             if (!is_finite_f32(my_mn) || !is_finite_f32(my_mx)) err |= OMMX_ERR_NONFINITE_V;
-            const Step st = make_step(__fdiv_rn(fmaxf(my_mx - my_mn, 1e-8f), 3.0f), 0, tab);
+            const Step st = make_step(third(fmaxf(my_mx - my_mn, 1e-8f)), 0, tab);
             const uint16_t zp_b = f32_to_bf16_rne(my_mn);
             const float zc = -bf16_to_f32(zp_b) * st.inv;
             if (r + me < VP) {
@@ -384,7 +391,7 @@ __global__ void __launch_bounds__(512, GT < GC ? 1 : GT == 32 ? 8 : GT == 64 ? 5
                     const int from = (static_cast<int>(threadIdx.x) & 63 & ~(VL - 1)) + n, row = 8 * (r + n) + v_row;
                     const float lo = __shfl(my_mn, from), hi = __shfl(my_mx, from), inv = __shfl(my_inv, from);
                     if (inv != 0.0f) continue;
-                    const Step s1 = make_step(__fdiv_rn(fmaxf(hi - lo, 1e-8f), 3.0f), 0, tab);
+                    const Step s1 = make_step(third(fmaxf(hi - lo, 1e-8f)), 0, tab);
                     const float zp = bf16_to_f32(f32_to_bf16_rne(lo));
                     const uint16_t* const e = v_base + src_row(row) * a.v_ts;
                     uint32_t bits = 0;
@@ -407,20 +414,24 @@ __global__ void __launch_bounds__(512, GT < GC ? 1 : GT == 32 ? 8 : GT == 64 ? 5
             reinterpret_cast<uint32_t*>(a.k_obmp + ibase)[wd] = reinterpret_cast<const uint32_t*>(s_oidx)[wd];
     }
 
-    // ------------------------------------------------- k_base rows: 8 bytes = 32 channels a piece
-    for (int it = tid; it < GT * pieces; it += NT) {
-        const int tk = it / pieces, j = it % pieces;
-        uint64_t kb8 = 0;
-        const uint4* cr = reinterpret_cast<const uint4*>(s_codes + tk * D + 32 * j);
+    // ------------------------------------------------- k_base rows: 4 bytes = 16 channels a piece, of two tokens
+    for (int it = tid; it < GT / 2 * 2 * pieces; it += NT) {
+        const int tp = it / (2 * pieces), j = it % (2 * pieces), turn = (j >> 1) & 3;
+        // 16 words, four at a time; the pieces start in turn, so that neighbouring lanes read from different banks
+        const u32x4* const words = reinterpret_cast<const u32x4*>(s_k + tp * D + 16 * j);
+        uint32_t four[4];                          // bytes 0 and 1: four codes of either token
 #pragma unroll
-        for (int q4 = 0; q4 < 2; ++q4) {
-            const uint4 u = cr[q4];
-            const uint32_t uw[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-                kb8 |= static_cast<uint64_t>(__builtin_amdgcn_udot4(uw[q], 0x40100401u, 0u, false)) << (8 * (4 * q4 + q));
+        for (int q = 0; q < 4; ++q) {
+            const u32x4 w = words[(q + turn) & 3];
+            four[q] = w[0] | w[1] << 2 | w[2] << 4 | w[3] << 6;
         }
-        reinterpret_cast<uint64_t*>(a.k_base)[(phys_row(page_of(tk), tk) * H + h) * pieces + j] = kb8;
+        const uint32_t lo = __builtin_amdgcn_perm(four[1], four[0], 0x05010400u), hi = __builtin_amdgcn_perm(four[3], four[2], 0x05010400u);
+        const uint32_t even = __builtin_amdgcn_perm(hi, lo, 0x05040100u), odd = __builtin_amdgcn_perm(hi, lo, 0x07060302u);
+        const int back = (32 - 8 * turn) & 31;     // byte q is piece (q + turn) % 4
+        const int page = page_of(2 * tp);          // (a page holds an even number of tokens, or one)
+        reinterpret_cast<uint32_t*>(a.k_base)[(phys_row(page, 2 * tp) * H + h) * 2 * pieces + j] = __builtin_amdgcn_alignbit(even, even, back);
+        reinterpret_cast<uint32_t*>(a.k_base)[(phys_row(a.ps == 1 ? page_of(2 * tp + 1) : page, 2 * tp + 1) * H + h) * 2 * pieces + j] =
+            __builtin_amdgcn_alignbit(odd, odd, back);
     }
 
     write_own_tables(a, g, h, tid);
@@ -430,8 +441,8 @@ __global__ void __launch_bounds__(512, GT < GC ? 1 : GT == 32 ? 8 : GT == 64 ? 5
 template <int GT, int GC>
 int launch_k(const StoreArgs& a, int T, hipStream_t st) {
     const dim3 grid = store_grid(a, kByEights), block(2 * a.D);
-    const size_t shm = static_cast<size_t>(a.D) * (3 * GT + 2 * 12 + 8 + 16);
-    if (shm > 64 * 1024) return 1;           // 128 tokens of a 256-channel head: the general kernel
+    const size_t shm = static_cast<size_t>(a.D) * (2 * GT + 8 + 16);
+    if (GT == 128 && a.D > 128) return 1;    // (LDS: the general kernel)
     const int k_vec = reinterpret_cast<uintptr_t>(a.K) % 16 == 0 && a.k_ts % 8 == 0 && a.k_hs % 8 == 0;
     if (a.kout == 6) hipLaunchKernelGGL((store_long_kernel<GT, GC, 3>), grid, block, shm, st, a, k_vec);
     else hipLaunchKernelGGL((store_long_kernel<GT, GC, 5>), grid, block, shm, st, a, k_vec);

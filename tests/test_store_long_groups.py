@@ -92,3 +92,26 @@ def test_v_vectors_of_any_alignment_and_range(gt, gc, D, k, shift):
     k_in.copy_(K)
     v_in.copy_(V)
     _same(ommx_pack_kv_canonical_block(k_in, v_in, **recipe), want, _names(recipe))
+
+
+@pytest.mark.parametrize("gt,gc,D,k", [(32, 32, 64, 6), (64, 64, 128, 6), (64, 32, 96, 10), (128, 128, 128, 10), (128, 64, 64, 6)])
+@pytest.mark.parametrize("ps", [1, 2, 32])
+def test_tokens_of_a_pair_on_pages_of_any_size(gt, gc, D, k, ps):
+    """Codes of two tokens are written together: pages of one token, of one pair and of a whole 32-token group in a shuffled
+    order, K rows that cannot be read 16 bytes at a time (a view one element into its storage)."""
+    T, H = 3 * gt, 2
+    K, V = synth_kv(T, H, D, seed=gt + D + k + ps, sparse_frac=0.01)
+    recipe = dict(outliers_per_vector=k, outlier_repr="relidx7", kv_outlier_map=True, group_tokens=gt, group_channels=gc)
+    want = O.pack_kv(K, V, outlier_select="signed", use_pow2=True, **recipe)
+    pages = torch.randperm(T // ps, generator=torch.Generator().manual_seed(ps))
+    shifted = torch.empty(T * H * D + 1, dtype=torch.bfloat16, device="cuda")
+    shifted[1:] = K.cuda().flatten()
+    for rows in (K.cuda(), shifted[1:].view(T, H, D)):
+        planes = alloc_planes(T // ps, T // gt, H, D, device="cuda", page_size=ps, **recipe)
+        store_pack_into(rows, V.cuda(), planes, page_size=ps, dst_pages=pages.int().cuda(), outliers_per_vector=k,
+                        outlier_repr="relidx7", group_tokens=gt, group_channels=gc)
+        for n in ("k_base", "v_main", "v_scale", "v_zp"):
+            got = planes[n].cpu()[pages].reshape(T, H, -1)
+            assert np.array_equal(bits_of(got), bits_of(want[n].reshape(T, H, -1))), n
+        for n in ("k_scale", "k_zp", "k_oval", "k_oidx", "k_fp4_mapscale", "k_fp4_mapcenter"):
+            assert np.array_equal(bits_of(planes[n].cpu()), bits_of(want[n])), n
