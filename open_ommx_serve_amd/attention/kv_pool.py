@@ -384,6 +384,22 @@ class MultiSeqKVPool:
         self._pack_completed(full)
         return True
 
+    def append_step_rows(self, slots: List[int], seqs: List[int], K: torch.Tensor, V: torch.Tensor,
+                         block: Optional[torch.Tensor] = None) -> Optional[Tuple[int, int]]:
+        """``append_step`` for a caller that holds nothing on the device yet: slots and positions go with the launch, which
+        also fills ``block`` (int32 ``[7 B]``: slots, positions and lengths as int64, then packed lengths).  The largest
+        packed length and the sum of all; ``None``, with nothing done, where ``append_step`` says False, and for more
+        than 64 requests."""
+        w = self.window
+        done = self._host.append_step(self.k_hist, self.v_hist, K, V, self._ring_sink, self._ring_rec, self.err_flag,
+                                      self.seq_len, self.packed_groups, slots, seqs, w.sink_tokens + w.recent_window,
+                                      self.gt, None if self.kv_ring else self.max_seq_len, block)
+        if done is None:
+            return None
+        if done[0]:
+            self._pack_completed(done[0])
+        return done[1], done[2]
+
     def append_decode_batched(self, slots: Sequence[int], K: torch.Tensor, V: torch.Tensor) -> int:
         """B new rows ``[B, H, D]`` in one launch, then one pack launch for every group that
         completed this step (kv_pool.py:383-438).  Returns the number of groups packed."""

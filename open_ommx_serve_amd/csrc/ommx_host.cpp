@@ -1102,42 +1102,32 @@ PyObject* py_all_at(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return PyBool_FromLong(r);
 }
 
-// (the arguments of ring_write without pos_next) + (seq_len, packed_groups, slots, seqs, kept rows, group_tokens, capacity or
-// None): one row of every request of a step appended to a pool that is one token behind it.  Returns the list of
-// (slot, first, end) of the groups that are complete with it (packed_groups is the caller's to move, once they are
-// packed), or None with nothing done.
-PyObject* py_append_rows(PyObject* self, PyObject* const* a, Py_ssize_t n) {
-    if (n != 16) { PyErr_SetString(PyExc_TypeError, "append_rows: wrong number of arguments"); return nullptr; }
-    bool ok = true;
-    const int64_t kept = as_int(a[13], ok), gt = as_int(a[14], ok), cap = a[15] == Py_None ? INT32_MAX : as_int(a[15], ok);
-    PyObject *const lens = a[9], *const packed = a[10], *const slots = a[11];
-    if (!ok || gt < 1 || all_at(lens, slots, a[12], 1) != 1 || !PyList_CheckExact(packed) ||
-        PyList_GET_SIZE(packed) != PyList_GET_SIZE(lens))
-        Py_RETURN_NONE;
+// What one step does to a pool that is one token behind it.
+struct StepRow { int64_t slot, len, done; };         // length after the step, packed groups before it
+// False, with nothing done: not plain lists, a slot not one token behind, without room, or named twice.
+bool read_step(PyObject* lens, PyObject* packed, PyObject* slots, PyObject* seqs, int64_t cap, std::vector<StepRow>& step) {
+    if (all_at(lens, slots, seqs, 1) != 1 || !PyList_CheckExact(packed) || PyList_GET_SIZE(packed) != PyList_GET_SIZE(lens)) return false;
     const Py_ssize_t B = PyList_GET_SIZE(slots), N = PyList_GET_SIZE(lens);
-    const at::Tensor* k = as_tensor(a[3], ok);
-    if (!ok || k->dim() != 3 || k->size(0) != B) Py_RETURN_NONE;
-    struct One { int64_t slot, len, done; };
-    std::vector<One> step(static_cast<size_t>(B));
+    bool ok = true;
+    step.resize(static_cast<size_t>(B));
     std::vector<bool> taken(static_cast<size_t>(N), false);
     for (Py_ssize_t i = 0; i < B; ++i) {
-        One& s = step[i];
+        StepRow& s = step[i];
         s.slot = as_int(PyList_GET_ITEM(slots, i), ok);
         s.len = as_int(PyList_GET_ITEM(lens, s.slot), ok) + 1;
         s.done = as_int(PyList_GET_ITEM(packed, s.slot), ok);
-        if (!ok || s.len > cap || taken[s.slot]) Py_RETURN_NONE;
+        if (!ok || s.len > cap || taken[s.slot]) return false;
         taken[s.slot] = true;
     }
-    PyObject* const ring[] = {a[0], a[1], a[2], a[3], a[4], a[5], a[6], a[7], Py_None, a[8]};
-    PyObject* launched = py_ring_write(self, ring, 10);
-    if (!launched) return nullptr;
-    const bool done = launched == Py_True;
-    Py_DECREF(launched);
-    if (!done) Py_RETURN_NONE;
+    return true;
+}
+int64_t groups_after(const StepRow& s, int64_t kept, int64_t gt) { return s.len >= kept ? (s.len - kept) / gt : 0; }
+// The pool's lengths moved; the list of (slot, first, end) of the groups that are complete with the step.
+PyObject* finish_step(PyObject* lens, const std::vector<StepRow>& step, int64_t kept, int64_t gt) {
     PyObject* full = PyList_New(0);
-    for (Py_ssize_t i = 0; i < B && full; ++i) {
-        const One& s = step[i];
-        const int64_t past = s.len - kept, target = past >= 0 ? past / gt : 0;
+    for (size_t i = 0; i < step.size() && full; ++i) {
+        const StepRow& s = step[i];
+        const int64_t target = groups_after(s, kept, gt);
         PyObject* item = nullptr;
         bool put = PyList_SetItem(lens, s.slot, PyLong_FromLongLong(s.len)) == 0;
         if (put && target > s.done) {
@@ -1148,6 +1138,92 @@ PyObject* py_append_rows(PyObject* self, PyObject* const* a, Py_ssize_t n) {
         if (!put) Py_CLEAR(full);
     }
     return full;
+}
+
+// (the arguments of ring_write without pos_next) + (seq_len, packed_groups, slots, seqs, kept rows, group_tokens, capacity or
+// None): one row of every request of a step appended to a pool that is one token behind it.  Returns the list of
+// (slot, first, end) of the groups that are complete with it (packed_groups is the caller's to move, once they are
+// packed), or None with nothing done.
+PyObject* py_append_rows(PyObject* self, PyObject* const* a, Py_ssize_t n) {
+    if (n != 16) { PyErr_SetString(PyExc_TypeError, "append_rows: wrong number of arguments"); return nullptr; }
+    bool ok = true;
+    const int64_t kept = as_int(a[13], ok), gt = as_int(a[14], ok), cap = a[15] == Py_None ? INT32_MAX : as_int(a[15], ok);
+    std::vector<StepRow> step;
+    if (!ok || gt < 1 || !read_step(a[9], a[10], a[11], a[12], cap, step)) Py_RETURN_NONE;
+    const at::Tensor* k = as_tensor(a[3], ok);
+    if (!ok || k->dim() != 3 || k->size(0) != static_cast<int64_t>(step.size())) Py_RETURN_NONE;
+    PyObject* const ring[] = {a[0], a[1], a[2], a[3], a[4], a[5], a[6], a[7], Py_None, a[8]};
+    PyObject* launched = py_ring_write(self, ring, 10);
+    if (!launched) return nullptr;
+    const bool done = launched == Py_True;
+    Py_DECREF(launched);
+    if (!done) Py_RETURN_NONE;
+    return finish_step(a[9], step, kept, gt);
+}
+
+// (k_hist, v_hist, K, V, sink, span, err_flag, seq_len, packed_groups, slots, seqs, kept rows, group_tokens, capacity or None,
+// block or None): append_rows of up to kStepRows requests with slots and positions as arguments of the launch, which also
+// fills the int32 tensor block[7 B] (ommx::ring_step).  Returns (groups as append_rows, largest packed length, their
+// sum), or None with nothing done.
+PyObject* py_append_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 15) { PyErr_SetString(PyExc_TypeError, "append_step: wrong number of arguments"); return nullptr; }
+    bool ok = true;
+    const at::Tensor *kh = as_tensor(a[0], ok), *vh = as_tensor(a[1], ok), *k = as_tensor(a[2], ok), *v = as_tensor(a[3], ok),
+                     *err = as_tensor_or_none(a[6], ok), *block = as_tensor_or_none(a[14], ok);
+    const int64_t sink = as_int(a[4], ok), span = as_int(a[5], ok), kept = as_int(a[11], ok), gt = as_int(a[12], ok),
+                  cap = a[13] == Py_None ? INT32_MAX : as_int(a[13], ok);
+    std::vector<StepRow> step;
+    if (!ok || gt < 1 || !read_step(a[7], a[8], a[9], a[10], std::min<int64_t>(cap, INT32_MAX), step)) Py_RETURN_NONE;
+    const int64_t B = static_cast<int64_t>(step.size());
+    if (B < 1 || B > ommx::kStepRows || !is_history(*kh, *vh) || k->dim() != 3 || k->sizes() != v->sizes()) Py_RETURN_NONE;
+    const c10::Device dev = kh->device();
+    const int64_t N = kh->size(0), rows = kh->size(1), H = kh->size(2), D = kh->size(3);
+    if (k->size(0) != B || k->size(1) != H || k->size(2) != D || k->scalar_type() != at::kBFloat16 ||
+        v->scalar_type() != at::kBFloat16 || k->stride(2) != 1 || v->stride(2) != 1 || !on(k, dev) || !on(v, dev) ||
+        !is_index(block, dev, at::kInt, 7 * B) || (block && reinterpret_cast<uintptr_t>(block->data_ptr()) % 8))
+        Py_RETURN_NONE;
+    ommx::StepRows at_rows;
+    int64_t longest = 0, sum = 0;
+    for (int64_t i = 0; i < B; ++i) {
+        const StepRow& s = step[i];
+        if (s.slot >= N) Py_RETURN_NONE;
+        const int64_t packed = groups_after(s, kept, gt) * gt;
+        at_rows.slot[i] = static_cast<int32_t>(s.slot);
+        at_rows.pos[i] = static_cast<int32_t>(s.len - 1);
+        at_rows.packed[i] = static_cast<int32_t>(packed);
+        longest = std::max(longest, packed);
+        sum += packed;
+    }
+    c10::hip::HIPGuard guard(dev.index());
+    hipStream_t stream = stream_of(dev);
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = ommx::ring_step(data<uint16_t>(k), data<uint16_t>(v), k->stride(0), k->stride(1), v->stride(0), v->stride(1),
+                         data<uint16_t>(kh), data<uint16_t>(vh), kh->stride(0), rows, B, H, D, sink, span, at_rows,
+                         data<int32_t>(block), data<int32_t>(err), stream);
+    Py_END_ALLOW_THREADS
+    if (failed(rc, "append_step")) return nullptr;
+    PyObject* full = finish_step(a[7], step, kept, gt);
+    if (!full) return nullptr;
+    return Py_BuildValue("(NLL)", full, static_cast<long long>(longest), static_cast<long long>(sum));
+}
+
+// (table, B): column 0 of the first B rows of a 2-D table of int32 or int64 in host memory as a list; None for anything else.
+PyObject* py_first_column(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    bool ok = n == 2;
+    const at::Tensor* t = ok ? as_tensor(a[0], ok) : nullptr;
+    const int64_t B = ok ? as_int(a[1], ok) : 0;
+    if (!ok || t->dim() != 2 || !t->is_cpu() || t->size(0) < B || t->size(1) < 1 || B < 0 || !plain_call(a, 1) ||
+        (t->scalar_type() != at::kInt && t->scalar_type() != at::kLong))
+        Py_RETURN_NONE;
+    PyObject* out = PyList_New(B);
+    for (int64_t i = 0; i < B && out; ++i) {
+        const int64_t at = i * t->stride(0);
+        PyObject* x = PyLong_FromLongLong(t->scalar_type() == at::kInt ? t->data_ptr<int32_t>()[at] : t->data_ptr<int64_t>()[at]);
+        if (!x) Py_CLEAR(out);
+        else PyList_SET_ITEM(out, i, x);
+    }
+    return out;
 }
 
 // C++ exceptions (out of memory among them) become the Python exceptions torch raises for them.
@@ -1162,7 +1238,7 @@ PyObject* guarded(PyObject* self, PyObject* const* a, Py_ssize_t n) {
 PyMethodDef methods[] = {
     OMMX_FAST(auto_num_kv_splits), OMMX_FAST(plain), OMMX_FAST(rows_fit),
     OMMX_FAST(decode), OMMX_FAST(decode_pool), OMMX_FAST(store_pack), OMMX_FAST(pack_block), OMMX_FAST(block_errors), OMMX_FAST(pack_groups), OMMX_FAST(pack_prompts), OMMX_FAST(ring_write),
-    OMMX_FAST(all_at), OMMX_FAST(append_rows),
+    OMMX_FAST(all_at), OMMX_FAST(append_rows), OMMX_FAST(append_step), OMMX_FAST(first_column),
     OMMX_FAST(tail_gather), OMMX_FAST(rows_write), OMMX_FAST(upload), OMMX_FAST(prefill),
     {nullptr, nullptr, 0, nullptr},
 };

@@ -82,6 +82,15 @@ int prompt_blocks(const PromptBlocks& blocks, const PromptRow* prompts, int n, i
 constexpr int kUploadWords = 960;
 int upload_words(int32_t* dst, const int32_t* host_words, int n, void* stream);
 
+// One new row of every request of a step into its ring history, slots and positions as arguments of the launch; `block`
+// (may be NULL) receives what later launches of the step read on the device: int64 slots[B], positions[B], lengths after
+// the step[B], then int32 packed lengths[B].
+constexpr int kStepRows = 64;
+struct StepRows { int32_t slot[kStepRows], pos[kStepRows], packed[kStepRows]; };
+int ring_step(const uint16_t* k, const uint16_t* v, int64_t k_bs, int64_t k_hs, int64_t v_bs, int64_t v_hs, uint16_t* k_hist,
+              uint16_t* v_hist, int64_t stride_req, int rows, int B, int H, int D, int sink, int span, const StepRows& step,
+              int32_t* block, int32_t* err, void* stream);
+
 // Index tables of one store launch that packs `n` groups of a pool, from (request, group) pairs in host memory:
 // src_rows[n * gt] flat history rows through the ring map, dst_pages[n * ppg], dst_groups[n].
 int pack_list(const int32_t* host_pairs, int n, int32_t* src_rows, int32_t* dst_pages, int32_t* dst_groups, int gt,

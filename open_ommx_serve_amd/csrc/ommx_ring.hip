@@ -1,6 +1,6 @@
 // bf16 residual ring of the KV store: the rows that are not (yet) packed.
 //
-//   ring_write_kernel   one new K/V row per request into its ring slot; follows
+//   ring_write_kernel   one new K/V row per request into its ring slot (ring_step_kernel: places as arguments); follows
 //                       ommx_gpu_serve/attention/kv_store_ops.py:22-40 (_kv_write_token) and
 //                       the batched scatter of attention/kv_pool.py:407-419.
 //   tail_gather_kernel  sink + recent rows of every request into the fixed tail buffers,
@@ -38,24 +38,19 @@ __device__ __forceinline__ void copy_row_in(uint16_t* dst, const uint16_t* src, 
     }
 }
 
-__global__ void __launch_bounds__(1024) ring_write_kernel(
-    RingArgs a, const uint16_t* k, const uint16_t* v, int64_t k_bs, int64_t k_hs, int64_t v_bs,
-    int64_t v_hs, const int64_t* pos, int64_t* pos_next, int vec) {
-    const int b = blockIdx.x;
-    // pieces of eight: those of K, then those of V
+// The piece of eight of a new row (those of K, then those of V) that thread i copies.
+__device__ __forceinline__ uint4 new_row_piece(const RingArgs& a, const uint16_t* k, const uint16_t* v, int64_t k_bs,
+                                               int64_t k_hs, int64_t v_bs, int64_t v_hs, int b, int i) {
     const int per_head = a.D / 8, pieces = a.H * per_head;
-    auto piece = [&](int i) {
-        const bool is_v = i >= pieces;
-        const int n = is_v ? i - pieces : i, h = n / per_head, c = (n - h * per_head) * 8;
-        return *reinterpret_cast<const uint4*>((is_v ? v + b * v_bs + h * v_hs : k + b * k_bs + h * k_hs) + c);
-    };
-    uint4 first = {};
-    if (vec && static_cast<int>(threadIdx.x) < 2 * pieces) first = piece(threadIdx.x);
-    const int64_t p = pos[b];
-    const int64_t slot = a.slots ? a.slots[b] : b;
+    const bool is_v = i >= pieces;
+    const int n = is_v ? i - pieces : i, h = n / per_head, c = (n - h * per_head) * 8;
+    return *reinterpret_cast<const uint4*>((is_v ? v + b * v_bs + h * v_hs : k + b * k_bs + h * k_hs) + c);
+}
+// Row b of K and V to position p of history `slot`; `first` is the thread's first piece.
+__device__ __forceinline__ void put_new_row(const RingArgs& a, const uint16_t* k, const uint16_t* v, int64_t k_bs, int64_t k_hs,
+                                            int64_t v_bs, int64_t v_hs, int b, int64_t p, int64_t slot, bool vec, uint4 first) {
+    const int pieces = a.H * (a.D / 8);
     const int64_t row = ring_slot(p, a.sink, a.span);
-    __syncthreads();                       // every thread has read pos[b] before it moves
-    if (pos_next && threadIdx.x == 0) pos_next[b] = p + 1;
     if (row < 0 || row >= a.cap) {         // kv_store_ops.py:33-34 asserts here
         if (a.err && threadIdx.x == 0) atomicOr(a.err, OMMX_ERR_RING_RANGE);
         return;
@@ -63,13 +58,45 @@ __global__ void __launch_bounds__(1024) ring_write_kernel(
     const int64_t off = slot * a.req_stride + row * (int64_t)(a.H * a.D);
     if (vec) {
         for (int i = threadIdx.x; i < 2 * pieces; i += blockDim.x) {
-            const uint4 x = i == static_cast<int>(threadIdx.x) ? first : piece(i);
+            const uint4 x = i == static_cast<int>(threadIdx.x) ? first : new_row_piece(a, k, v, k_bs, k_hs, v_bs, v_hs, b, i);
             reinterpret_cast<uint4*>((i < pieces ? a.k_hist : a.v_hist) + off)[i < pieces ? i : i - pieces] = x;
         }
         return;
     }
     copy_row_in(a.k_hist + off, k + b * k_bs, k_hs, a.H, a.D, false);
     copy_row_in(a.v_hist + off, v + b * v_bs, v_hs, a.H, a.D, false);
+}
+
+__global__ void __launch_bounds__(1024) ring_write_kernel(
+    RingArgs a, const uint16_t* k, const uint16_t* v, int64_t k_bs, int64_t k_hs, int64_t v_bs,
+    int64_t v_hs, const int64_t* pos, int64_t* pos_next, int vec) {
+    const int b = blockIdx.x;
+    uint4 first = {};
+    if (vec && static_cast<int>(threadIdx.x) < 2 * a.H * (a.D / 8)) first = new_row_piece(a, k, v, k_bs, k_hs, v_bs, v_hs, b, threadIdx.x);
+    const int64_t p = pos[b];
+    const int64_t slot = a.slots ? a.slots[b] : b;
+    __syncthreads();                       // every thread has read pos[b] before it moves
+    if (pos_next && threadIdx.x == 0) pos_next[b] = p + 1;
+    put_new_row(a, k, v, k_bs, k_hs, v_bs, v_hs, b, p, slot, vec, first);
+}
+
+// The same with the places as arguments: no launch before this one has to bring them to the device; the step's other launches
+// read them from `block`, which the first layer's launch fills.  8 requests of 8 heads, kernel alone 2.6 us as the other, and the
+// upload's 1.4 are gone; the host's part of a step of two layers without its decodes 29 -> 20 us.
+__global__ void __launch_bounds__(1024) ring_step_kernel(RingArgs a, const uint16_t* k, const uint16_t* v, int64_t k_bs,
+                                                         int64_t k_hs, int64_t v_bs, int64_t v_hs, int32_t* block, int vec,
+                                                         StepRows step) {
+    const int b = blockIdx.x, B = gridDim.x, p = step.pos[b], slot = step.slot[b];
+    uint4 first = {};
+    if (vec && static_cast<int>(threadIdx.x) < 2 * a.H * (a.D / 8)) first = new_row_piece(a, k, v, k_bs, k_hs, v_bs, v_hs, b, threadIdx.x);
+    if (block && threadIdx.x == 0) {
+        int64_t* const wide = reinterpret_cast<int64_t*>(block);
+        wide[b] = slot;
+        wide[B + b] = p;
+        wide[2 * B + b] = p + 1LL;
+        block[6 * B + b] = step.packed[b];
+    }
+    put_new_row(a, k, v, k_bs, k_hs, v_bs, v_hs, b, p, slot, vec, first);
 }
 
 __global__ void __launch_bounds__(256) tail_gather_kernel(
@@ -122,16 +149,34 @@ __global__ void __launch_bounds__(256) tail_gather_kernel(
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
+static bool ring_rows_vec(const RingArgs& a, const uint16_t* k, const uint16_t* v, int64_t k_bs, int64_t k_hs, int64_t v_bs,
+                          int64_t v_hs) {
+    return a.D % 8 == 0 && aligned16(a.k_hist) && aligned16(a.v_hist) && aligned16(k) && aligned16(v) &&
+           a.req_stride % 8 == 0 && k_bs % 8 == 0 && k_hs % 8 == 0 && v_bs % 8 == 0 && v_hs % 8 == 0;
+}
+static int ring_row_threads(const RingArgs& a, bool vec) {
+    const int pieces = a.H * a.D / (vec ? 4 : 1);        // of K and V, or elements of one of them
+    return vec ? std::min((pieces + 63) / 64 * 64, 1024) : (pieces >= 256 ? 256 : 128);
+}
+
 int launch_ring_write(const RingArgs& a, const uint16_t* k, const uint16_t* v, int64_t k_bs,
                       int64_t k_hs, int64_t v_bs, int64_t v_hs, const int64_t* pos,
                       int64_t* pos_next, int B, hipStream_t st) {
-    const int vec = a.D % 8 == 0 && aligned16(a.k_hist) && aligned16(a.v_hist) && aligned16(k) &&
-                    aligned16(v) && a.req_stride % 8 == 0 && k_bs % 8 == 0 && k_hs % 8 == 0 &&
-                    v_bs % 8 == 0 && v_hs % 8 == 0;
-    const int pieces = a.H * a.D / (vec ? 4 : 1);        // of K and V, or elements of one of them
-    const int threads = vec ? std::min((pieces + 63) / 64 * 64, 1024) : (pieces >= 256 ? 256 : 128);
-    hipLaunchKernelGGL(ring_write_kernel, dim3(B), dim3(threads), 0, st, a, k, v, k_bs, k_hs, v_bs,
+    const bool vec = ring_rows_vec(a, k, v, k_bs, k_hs, v_bs, v_hs);
+    hipLaunchKernelGGL(ring_write_kernel, dim3(B), dim3(ring_row_threads(a, vec)), 0, st, a, k, v, k_bs, k_hs, v_bs,
                        v_hs, pos, pos_next, vec);
+    return 0;
+}
+
+int ring_step(const uint16_t* k, const uint16_t* v, int64_t k_bs, int64_t k_hs, int64_t v_bs, int64_t v_hs, uint16_t* k_hist,
+              uint16_t* v_hist, int64_t stride_req, int rows, int B, int H, int D, int sink, int span, const StepRows& step,
+              int32_t* block, int32_t* err, void* stream) {
+    if (B < 1 || B > kStepRows || H < 1 || D < 1 || rows < 1) { set_error("ring_step: bad shape"); return -1; }
+    const RingArgs a{k_hist, v_hist, stride_req, rows, sink, span, H, D, nullptr, err};
+    const bool vec = ring_rows_vec(a, k, v, k_bs, k_hs, v_bs, v_hs);
+    hipLaunchKernelGGL(ring_step_kernel, dim3(B), dim3(ring_row_threads(a, vec)), 0, static_cast<hipStream_t>(stream), a, k, v,
+                       k_bs, k_hs, v_bs, v_hs, block, vec, step);
+    if (hipGetLastError() != hipSuccess) { set_error("ring_step: launch failed"); return -2; }
     return 0;
 }
 

@@ -262,11 +262,8 @@ class OMMXCanonicalImpl(_ImplBase):
             # one token of every request: one native call writes the rows and moves the cursors, if the layer's pool is
             # where the scheduler's lengths say (else the general way, which names what is wrong)
             pool = m.pools.get(id(layer))
-            append = getattr(pool, "append_step", None)
-            if append is not None:
-                step = m.step_on_device(pool)
-                if append(m.slots, m.seq_lens, step.sel, step.col, key, value):
-                    return
+            if pool is not None and m.append_step(pool, key, value):
+                return
         n = int(key.shape[0])
         if n == 0:
             return

@@ -247,6 +247,59 @@ def test_a_step_of_rows_and_cursors_in_one_call(ring):
     assert held == pools[0].seq_len and torch.equal(hist, pools[0].k_hist)
 
 
+@pytest.mark.parametrize("ring,B,D,view", [(False, 1, 64, False), (True, 4, 128, False), (True, 64, 64, False), (False, 5, 64, True),
+                                           (True, 65, 64, False)])
+def test_a_step_whose_places_go_with_the_launch(ring, B, D, view):
+    """append_step_rows against append_step over steps that complete groups and turn the ring: histories, cursors, planes and
+    the block for the step's other launches; rows of a strided view; 65 requests and what append_step refuses change
+    nothing."""
+    H, win = 2, WindowSpec()
+    pools = [MultiSeqKVPool(D, H, B + 2, 210, window=win, device=DEV, kv_ring=ring, **RECIPE) for _ in range(2)]
+    slots = [(3 * i + 1) % (B + 2) if (B + 2) % 3 else i for i in range(B)]
+    lens = [60 + 7 * (i % 19) for i in range(B)]
+    for i, (r, n) in enumerate(zip(slots, lens)):
+        K, V = _block(n, H, D, torch.bfloat16, 10 + i), _block(n, H, D, torch.bfloat16, 200 + i)
+        for p in pools:
+            p.append_block(r, K, V)
+    sel, block = torch.tensor(slots, device=DEV), torch.full((7 * B,), -1, dtype=torch.int32, device=DEV)
+    for s in range(1, 9):
+        K, V = _block(B, H, D, torch.bfloat16, 30 + s), _block(B, H, D, torch.bfloat16, 40 + s)
+        if view:
+            both = torch.stack([K, V], 2)                       # [B, H, 2, D]: a head stride of 2 D
+            K, V = both[:, :, 0], both[:, :, 1]
+        seqs = [n + s for n in lens]
+        got = pools[0].append_step_rows(slots, seqs, K, V, block if s % 2 else None)
+        if B > 64:
+            assert got is None and pools[0].seq_len == pools[1].seq_len and bool((block == -1).all())
+            return
+        packed = [win.packed_len(n) for n in seqs]
+        assert got == (max(packed), sum(packed))
+        assert pools[1].append_step(slots, seqs, sel, torch.tensor([n - 1 for n in seqs], device=DEV), K, V)
+        assert pools[0].seq_len == pools[1].seq_len and pools[0].packed_groups == pools[1].packed_groups
+        assert torch.equal(pools[0].k_hist[sel], pools[1].k_hist[sel]) and torch.equal(pools[0].v_hist[sel], pools[1].v_hist[sel])
+        if s % 2:
+            wide = block[:6 * B].view(torch.int64).view(3, B)
+            assert wide.tolist() == [slots, [n - 1 for n in seqs], seqs] and block[6 * B:].tolist() == packed
+    for r in slots:
+        a, b = pools[0].request_planes(r), pools[1].request_planes(r)
+        for n in ("k_base", "k_scale", "k_obmp", "k_oval", "v_main", "v_scale"):
+            assert torch.equal(a[n], b[n]), (r, n)
+    held, hist, was = list(pools[0].seq_len), pools[0].k_hist.clone(), block.clone()
+    nxt = [n + 9 for n in lens]
+    refused = [(slots, [n + 1 for n in nxt], K, V, block), (slots, nxt, K.float(), V.float(), block), (slots, nxt, K.cpu(), V.cpu(), block),
+               (slots, nxt, K[:0], V[:0], block), (tuple(slots), nxt, K, V, block), ([B + 7, *slots[1:]], nxt, K, V, block),
+               (slots, nxt, K, V, block[:-1]), (slots, nxt, K, V, block.long()), (slots, nxt, K, V, block.cpu())]
+    for sl, sq, k, v, to in refused:
+        assert pools[0].append_step_rows(sl, sq, k, v, to) is None
+    if not ring:
+        pools[0].seq_len[slots[0]] = 210
+        assert pools[0].append_step_rows(slots, [211, *nxt[1:]], K, V, block) is None
+        pools[0].seq_len[slots[0]] = held[slots[0]]
+    torch.cuda.synchronize()
+    assert held == pools[0].seq_len and torch.equal(hist, pools[0].k_hist) and torch.equal(was, block)
+    pools[0].check_errors()
+
+
 @pytest.mark.parametrize("sink,span,wsink,count,H,ps", [
     (0, 0, 8, 3, 8, 16), (8, 96, 8, 3, 8, 16),            # whole history; groups that end where the ring turns
     (8, 83, 8, 2, 3, 8), (8, 41, 13, 1, 8, 32),           # groups that turn with it

@@ -13,7 +13,7 @@ from open_ommx_serve_amd.attention.kv_window import WindowSpec, packed_boundary
 from open_ommx_serve_amd.integration.vllm import backend as BK
 from open_ommx_serve_amd.integration.vllm.config import OMMXServingConfig, resolve_serving_config
 from open_ommx_serve_amd.integration.vllm.metadata import (
-    STEP_ROUTE_UNCLASSIFIED, OMMXBatchedStepManager, OMMXSlotAllocationError, OMMXStepManager,
+    STEP_ROUTE_UNCLASSIFIED, OMMXBatchedStepManager, OMMXSlotAllocationError, OMMXStepManager, StepShape,
     assign_slots, detect_full_prefill, detect_step_route)
 
 
@@ -336,6 +336,32 @@ def test_each_stream_has_its_own_block_and_tables_of_a_step(monkeypatch):
     for stream in range(3, 40):                # bounded however many streams come
         at(stream)
     assert len(m._stream_blocks) <= 8
+
+
+@pytest.mark.parametrize("table,rows", [
+    (torch.arange(12).view(4, 3), 3), (torch.arange(12, dtype=torch.int32).view(4, 3).flip(0), 4),
+    (torch.arange(24).view(4, 6)[:, ::2], 2), (torch.arange(12).view(3, 4).t(), 4), (torch.arange(4).view(4, 1), 0),
+    (torch.arange(12.0).view(4, 3), 3), (torch.arange(12, dtype=torch.int16).view(4, 3), 2), ([[7, 1], [9, 2]], 2)])
+def test_first_blocks_of_any_table(table, rows):
+    """Column 0 as the index expression gives it: views, orders, types that the native call takes and those it leaves."""
+    m, _ = _bmgr(graph=False)
+    whole = table.tolist() if torch.is_tensor(table) else table
+    assert m._first_blocks(table, rows) == [int(r[0]) for r in whole[:rows]]
+    if torch.is_tensor(table):
+        with pytest.raises((ValueError, IndexError)):
+            m._first_blocks(table, table.shape[0] + 1)
+
+
+@pytest.mark.parametrize("lengths,offsets", [
+    ([1, 1, 1], [0, 1, 2, 3]), ([5, 1, 9], [4, 5, 6, 7]), ([2, 3], [0, 2, 5]), ([2, 1], [0, 2, 3]), ([4, 4], [0, 1, 1]),
+    ([3], [0, 1]), ([1], [0, 1]), ([], [0]), ([7, 8], [0, 1]), ([7], None), (None, [0, 1]), ([2, 2], [0, 2, 1])])
+def test_step_shapes_by_their_counts(lengths, offsets):
+    counts = None
+    if lengths is not None and offsets is not None and len(offsets) == len(lengths) + 1:
+        counts = [b - a for a, b in zip(offsets, offsets[1:])]
+    s = StepShape(lengths, offsets)
+    assert s.one_token_each == (bool(counts) and all(c == 1 for c in counts))
+    assert s.whole_sequences == (bool(counts) and counts == lengths)
 
 
 # ── config and route decisions ───────────────────────────────────────────────────────────
