@@ -10,8 +10,8 @@
 // a workgroup is 4 waves = 4 neighbouring kv heads.  Measured on MI355X this operator is bound
 // by how many instructions a SIMD can issue (vector ALU first, LDS second, a 16-byte LDS access
 // taking four issue slots), so the kernel is built for few instructions per token and to keep
-// THREE waves per SIMD resident (two with longer groups): at most 168 vector registers, no scratch
-// memory, 13.4 KB of LDS per wave.  What that takes, against the kernel in ommx_decode.hip:
+// THREE waves per SIMD resident (two with longer groups): at most 168 vector registers (one of those of the bitmap
+// forms lies in scratch memory and is read on the path of large steps alone), 13.4 KB of LDS per wave.  What that takes, against the kernel in ommx_decode.hip:
 //   * P.V runs transposed (rows = V channels, columns = q heads), the V step 2^e sits in the
 //     exponent field of the V operand, and the four column replicas of the q heads each take
 //     every fourth channel block, so the output accumulator is 8 registers instead of 32;
@@ -173,6 +173,19 @@ __device__ __forceinline__ uint32_t v_op(uint32_t m, uint32_t step) {
     const f16x2 one = {1.0f, 1.0f};
     return __builtin_bit_cast(uint32_t, (__builtin_bit_cast(f16x2, v_pair<Y, LONG>(m, 0x3C003C00u)) - one) * __builtin_bit_cast(f16x2, step));
 }
+// Outlier positions of a bitmap from below: the lowest set bit, and the map without the bit at `pos`, one addition of
+// -1 << pos (m & (m - 1) takes two instructions).
+__device__ __forceinline__ int lowest_bit(uint32_t m) {
+    int pos;
+    asm("v_ffbl_b32 %0, %1" : "=v"(pos) : "v"(m));
+    return pos;
+}
+__device__ __forceinline__ uint32_t without_bit(uint32_t m, int pos) {
+    uint32_t r;
+    asm("v_lshl_add_u32 %0, -1, %1, %2" : "=v"(r) : "v"(pos), "v"(m));
+    return r;
+}
+__device__ __forceinline__ float f16_bits(uint32_t b) { return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(b))); }
 __device__ __forceinline__ uint32_t pk_u16(uint32_t lo, uint32_t hi) { return (lo & 0xFFFFu) | (hi << 16); }
 
 // IDX: 0 = outlier positions from 32-bit bitmaps, 1 = from 7-bit position streams.

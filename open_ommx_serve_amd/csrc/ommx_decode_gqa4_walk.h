@@ -118,7 +118,7 @@
 #pragma unroll
         for (int r = 0; r < NH; ++r)
             qa = fmaxf(qa, fmaxf(fabsf(__uint_as_float(qraw[r] << 16)), fabsf(__uint_as_float(qraw[r] & 0xFFFF0000u))));
-        if (__builtin_expect(__any(qa >= 128.0f) != 0, 0)) {
+        if (__builtin_expect(any_lane(qa >= 128.0f), 0)) {
             float m4[4] = {qa, qa, qa, qa};
             wave_max4(m4);
             q_down = min(static_cast<int>((__float_as_uint(m4[0]) >> 23) & 0xFFu) - 127 - 6, 100);
@@ -354,9 +354,10 @@
         if (LONG) big_thr[u] = fminf(big_thr[u], MAX_F16);     // (what no f16 holds is looked at whatever q is)
     }
     const uint32_t kt_lane = OFF_KT + (c0 >> 2);                   // code byte of the channel pair (4 channels a byte), row 0
-    const uint32_t code_sh = 2u * (c0 & 3u);                      // bit of channel c0's code in that byte; c0 + 1 sits two on
+    const uint32_t code_bits = 3u << (2u * (c0 & 3u));            // of channel c0's code in that byte; c0 + 1 sits two bits on
     const uint32_t kbytes = static_cast<uint32_t>(kout + 1) >> 1;            // nibble bytes per channel
     const uint32_t nib_sh = 8u * ((2u * kbytes * lane) & 3u);
+    const uint32_t nib_at = (lane & 1) ? 0x0C040302u : 0x0C020100u;          // 6 outliers: the bytes of channel c0's nibbles (c0 + 1: three on)
     const float c2 = sm_scale * 1.4426950408889634f;
     if constexpr (!FETCH_FIRST) first_fetch();
 
@@ -384,7 +385,7 @@
             e_from = __builtin_bit_cast(u16x2e, __builtin_amdgcn_perm(0u, g_sc[0], 0x010C000Cu)) + static_cast<uint16_t>(-MIN_STEP_EXP * 256);
             zp_over = __builtin_elementwise_sub_sat(__builtin_bit_cast(u16x2e, g_zp[0] & 0x7FFF7FFFu),
                                                     u16x2e{ANY_ZP_BF16 - 1, ANY_ZP_BF16 - 1});
-            exact_step = __any((e_from[0] > e_from[1] ? e_from[0] : e_from[1]) >= EXACT || __builtin_bit_cast(uint32_t, zp_over) != 0) != 0 ||
+            exact_step = any_lane((e_from[0] > e_from[1] ? e_from[0] : e_from[1]) >= EXACT || __builtin_bit_cast(uint32_t, zp_over) != 0) ||
                          q_down != 0;
         } else if constexpr (!ANY) {
             typedef short s16x2e __attribute__((ext_vector_type(2)));
@@ -393,6 +394,7 @@
                 __builtin_bit_cast(s16x2e, __builtin_amdgcn_perm(0u, g_sc[NG - 1], 0x010C000Cu)));
             const short e_top = top2[0] > top2[1] ? top2[0] : top2[1];
             // (a scaled-down query means operands near the top of f16: the same cancellation, the same remedy)
+            // (not any_lane: with this test in a scalar register up to 16 vector registers are spilled)
             exact_step = __any(e_top >= EXACT_STEP_EXP * 256) != 0 || q_down != 0;
             if (__builtin_expect(exact_step, 0)) over_step |= __any(e_top > MAX_STEP_EXP * 256) != 0;
         }
@@ -465,7 +467,7 @@
                 } else {
                     ixw[0] = u ? __builtin_amdgcn_alignbit(g_bx[0], g_bm[0][1], 16) : g_bm[0][0];
                     ixw[1] = u ? (g_bx[0] >> 16) : g_bm[0][1];
-                    o0 = static_cast<uint32_t>(((static_cast<uint64_t>(g_ov[0][1]) << 32) | g_ov[0][0]) >> (nib_sh + 24 * u));
+                    o0 = __builtin_amdgcn_perm(g_ov[0][1], g_ov[0][0], nib_at + (u ? 0x030303u : 0u));
                 }
                 // 128 tokens: the upper bit of every position flipped in the second piece, so that those of the piece read below 64
                 if (GTS == 2 && (n0 & 64)) {
@@ -491,11 +493,15 @@
                 const int e = static_cast<int8_t>((g_sc[0] >> (8 * u)) & 0xFFu);
                 // in units of the channel's A scale, as in the walk of 32-token groups below
                 const float cs = u ? cs1 : cs0;
-                const float sc = __uint_as_float(static_cast<uint32_t>(e + 127) << 23) * cs;
-                float a1 = sc, b1 = 0.0f;
+                // (the code is taken as the bits of a subnormal f16, 2^-24 each, where it lies in its byte: a mask and one mixed
+                // multiply-add, exact, in the place of a shift, a conversion and a multiply-add)
+                const float code_step = __builtin_ldexpf(cs, e + ((lane & 1) ? 20 : 24) - 2 * u);
+                float a1, b1 = 0.0f;
                 if (OWN_MAP) {
                     a1 = cs * __builtin_amdgcn_rcpf(__uint_as_float(u ? (g_ms[0] & 0xFFFF0000u) : (g_ms[0] << 16)));
                     b1 = cs * (__uint_as_float(u ? (g_mc[0] & 0xFFFF0000u) : (g_mc[0] << 16)) - zp);
+                } else {
+                    a1 = __builtin_ldexpf(cs, e);
                 }
                 float lv[10];
                 const f32x2 l01 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(o0, 1.0f, 0);
@@ -510,8 +516,7 @@
                 float dl_max = 0.0f;
 #pragma unroll
                 for (int sidx = 0; sidx < KMAX; ++sidx) {
-                    const float code = static_cast<float>((cb[sidx] >> (code_sh + 2 * u)) & 3u);
-                    float dl = fmaf(-code, sc, fmaf(lv[sidx], a1, b1));
+                    float dl = fmaf(-f16_bits(cb[sidx] & (code_bits << 2 * u)), code_step, fmaf(lv[sidx], a1, b1));
                     // (the entry as a value of its own: rounded to f16 here exactly as the residual pass rounds it)
                     asm("" : "+v"(dl));
                     dls[u][sidx] = dl;
@@ -520,7 +525,7 @@
                         ANY && fabsf(dl) > MAX_F16 ? copysignf(MAX_F16, dl) : dl));
                     dl_max = fmaxf(dl_max, GTS == 1 || l_at[u][sidx] < 2 * HALF_ROWS ? fabsf(dl) : 0.0f);
                 }
-                return (ANY && q_down >= HUGE_Q_DOWN) || __any(dl_max >= big_thr[u]) != 0;
+                return (ANY && q_down >= HUGE_Q_DOWN) || any_lane(dl_max >= big_thr[u]);
             };
             // Entries of the step whose f16 rounding matters add what the rounding dropped to the logits, exactly.
             auto residuals = [&](auto U) {
@@ -580,8 +585,8 @@
 #pragma unroll
                 for (int sidx = 0; sidx < KMAX; ++sidx) {
                     if constexpr (IDX == 0) {
-                        pos[sidx] = __builtin_ctz(bm) & 31;
-                        if (sidx < KMAX - 1) bm &= bm - 1;
+                        pos[sidx] = lowest_bit(bm);
+                        if (sidx < KMAX - 1) bm = without_bit(bm, pos[sidx]);
                     } else {
                         pos[sidx] = sidx < 4 ? ((ix_lo >> (7 * sidx)) & 31)
                                   : sidx == 4 ? (__builtin_amdgcn_alignbit(ix_hi, ix_lo, 28) & 31)
@@ -594,11 +599,17 @@
                 constexpr int u = decltype(U)::value;
                 const float zp = __uint_as_float(u ? (g_zp[pg] & 0xFFFF0000u) : (g_zp[pg] << 16));
                 const int e = static_cast<int8_t>((g_sc[pg] >> (8 * u)) & 0xFFu);
-                const float s = __uint_as_float(static_cast<uint32_t>(e + 127) << 23);
                 // everything below is in units of the channel's A scale: tile entry =
-                // (outlier - zp - code * 2^e) / 2^(10-2m) = level * a1 + b1 (less 3 * sc for code 3)
+                // (outlier - zp - code * 2^e) / 2^(10-2m) = level * a1 + b1 less the code's step times the code
                 const float cs = u ? cs1 : cs0;
-                const float sc = s * cs;
+                // (the code is taken as the bits of a subnormal f16, 2^-24 each, where it lies in its byte: a mask and one mixed
+                // multiply-add, exact, in the place of a shift, a conversion and a multiply-add)
+                // (a code is taken as the bits of a subnormal f16, 2^-24 each, where it lies in its byte: a mask and one mixed
+                // multiply-add, exact, in the place of a shift, a conversion and a multiply-add.  With positions by two
+                // instructions instead of three, one test a channel for residuals and nibbles by one permutation the pass over a
+                // group's outliers is 126 vector instructions, 157 before: 64 K 31.4 -> 30.8 us, 8 x 32 K with 64 q heads
+                // 103.5 -> 102.4, 32 of 1 to 16 K with position streams 100.3 -> 98.7.)
+                const float code_step = __builtin_ldexpf(cs, e + ((lane & 1) ? 20 : 24) - 2 * u);
                 float a1, b1;
                 if (OWN_MAP) {
                     const float ms = __uint_as_float(u ? (g_ms[pg] & 0xFFFF0000u) : (g_ms[pg] << 16));
@@ -606,13 +617,13 @@
                     a1 = cs * __builtin_amdgcn_rcpf(ms);
                     b1 = cs * (mc - zp);
                 } else {
-                    a1 = sc;
+                    a1 = __builtin_ldexpf(cs, e);
                     b1 = 0.0f;
                 }
                 float lv[8];
-                const uint64_t ov64 = (static_cast<uint64_t>(g_ov[pg][1]) << 32) | g_ov[pg][0];
-                const uint32_t nib = GEN ? static_cast<uint32_t>(ov64 >> (nib_sh + 8 * kbytes * u))
-                                         : static_cast<uint32_t>(ov64 >> (nib_sh + 24 * u)) & 0xFFFFFFu;
+                uint32_t nib;
+                if constexpr (GEN) nib = static_cast<uint32_t>(((static_cast<uint64_t>(g_ov[pg][1]) << 32) | g_ov[pg][0]) >> (nib_sh + 8 * kbytes * u));
+                else nib = __builtin_amdgcn_perm(g_ov[pg][1], g_ov[pg][0], nib_at + (u ? 0x030303u : 0u));
                 const f32x2 l01 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(nib, 1.0f, 0);
                 const f32x2 l23 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(nib, 1.0f, 1);
                 const f32x2 l45 = KMAX > 4 ? __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(nib, 1.0f, 2) : f32x2{0.0f, 0.0f};
@@ -624,8 +635,7 @@
 #pragma unroll
                 for (int sidx = 0; sidx < KMAX; ++sidx) {
                     const float dl0 = fmaf(lv[sidx], a1, b1);
-                    const float code = static_cast<float>((cb[sidx] >> (code_sh + 2 * u)) & 3u);
-                    float dl = fmaf(-code, sc, dl0);
+                    float dl = fmaf(-f16_bits(cb[sidx] & (code_bits << 2 * u)), code_step, dl0);
                     // (the entry as a value of its own: rounded to f16 here exactly as the residual pass rounds it)
                     asm("" : "+v"(dl));
                     dls[sidx] = dl;
@@ -678,11 +688,10 @@
             const float dlm0 = walk_write(std::integral_constant<int, 0>{}, pos0, cb0, dls0);
             if constexpr (GEN) walk_read(std::integral_constant<int, 1>{}, pos1, cb1);
             const float dlm1 = walk_write(std::integral_constant<int, 1>{}, pos1, cb1, dls1);
-            res_any = __any(dlm0 >= big_thr[0] || dlm1 >= big_thr[1]) != 0;
-            if (__builtin_expect(res_any, 0)) {
-                residuals(std::integral_constant<int, 0>{}, pos0, dls0);
-                residuals(std::integral_constant<int, 1>{}, pos1, dls1);
-            }
+            const bool res0 = any_lane(dlm0 >= big_thr[0]), res1 = any_lane(dlm1 >= big_thr[1]);
+            res_any = res0 || res1;
+            if (__builtin_expect(res0, 0)) residuals(std::integral_constant<int, 0>{}, pos0, dls0);
+            if (__builtin_expect(res1, 0)) residuals(std::integral_constant<int, 1>{}, pos1, dls1);
             }
             lds_fence();
             if (more && !LONG) fetch_params_g(pg);
@@ -748,7 +757,7 @@
                 if constexpr (LONG) {
                     if (g == 0) {
                         auto over = [&](uint16_t e) { return e > MOST && e < BELOW; };
-                        if (__any(over(e_from[0]) || over(e_from[1]) || __builtin_bit_cast(uint32_t, zp_over) != 0)) goto other_form;
+                        if (any_lane(over(e_from[0]) || over(e_from[1]) || __builtin_bit_cast(uint32_t, zp_over) != 0)) goto other_form;
                         // a step below the range is harmless where all codes are zero (a channel that does not vary)
                         const uint64_t lo = __ballot(e_from[0] >= BELOW), hi = __ballot(e_from[1] >= BELOW);
                         if (lo | hi) {
@@ -764,7 +773,7 @@
                             }
                         }
                     }
-                    if (__any((((kw[0][0] | kw[1][0]) & dead[0]) | ((kw[0][1] | kw[1][1]) & dead[1])) != 0)) goto other_form;
+                    if (any_lane((((kw[0][0] | kw[1][0]) & dead[0]) | ((kw[0][1] | kw[1][1]) & dead[1])) != 0)) goto other_form;
                 }
                 base_mfmas(std::true_type{});
                 // the bias MFMA must not take the constant out a second time: its 2^e column of this group reads zeros
@@ -779,7 +788,7 @@
                 // rows 4kq..4kq+3 of every result hold the four heads: the lane keeps its own token block
 #pragma unroll
                 for (int t2 = 0; t2 < 2; ++t2)
-                    if (kq == 2 * g + t2) dsel[0] = d[t2];
+                    if (kq == 2 * g + t2 || (g == 0 && t2 == 0)) dsel[0] = d[t2];      // (group 1's lanes: theirs comes, or is not wanted)
                 if (res_any) {       // exact residuals of this group's large deltas, then zero again
                     const f32x4 corr = *reinterpret_cast<const f32x4*>(lc + 4 * (lane & 31));
                     if ((kq >> 1) == g) dsel[0] += corr;
@@ -829,7 +838,7 @@
             }
             // a V step above 2^MAX_STEP_EXP (a signed exponent byte of 16 or more) is held there and reported
             if constexpr (!LONG || ANY) {
-                if (__builtin_expect(__any((((vsc & 0x7F7F7F7Fu) + 0x70707070u) & ~vsc & 0x80808080u) != 0u) != 0, 0)) over_step = true;
+                if (__builtin_expect(any_lane((((vsc & 0x7F7F7F7Fu) + 0x70707070u) & ~vsc & 0x80808080u) != 0u), 0)) over_step = true;
             }
             uint16_t* vs16 = reinterpret_cast<uint16_t*>(sm + OFF_VS) + lane;
             uint16_t* vz16 = reinterpret_cast<uint16_t*>(sm + OFF_VZ) + lane;
@@ -867,7 +876,7 @@
                 const uint32_t step = vs16[c * PT_ROW];
                 bad |= (step == 0x0400u || step == 0x7800u) && (vt[2 * c * VT_COL] | vt[(2 * c + 1) * VT_COL]) != 0;
             }
-            return __any(held && bad) != 0;
+            return any_lane(held && bad);
         };
 
         // ------------------------------------------------------------------ softmax
@@ -910,9 +919,9 @@
                 }
             }
             // (longer groups: a V step for the other form is seen to here, before it is summed)
-            if (__any(fmaxf(fmaxf(pe[0], pe[1]), fmaxf(pe[2], pe[3])) > MAX_SLACK<LONG> || (LONG && !ANY && v_out != 0))) {
+            if (any_lane(fmaxf(fmaxf(pe[0], pe[1]), fmaxf(pe[2], pe[3])) > MAX_SLACK<LONG> || (LONG && !ANY && v_out != 0))) {
                 if constexpr (LONG && !ANY) {
-                    if (__builtin_expect(__any(v_out != 0), 0)) {
+                    if (__builtin_expect(any_lane(v_out != 0), 0)) {
                         if (v_needs_other_form(v_out != 0)) goto other_form;
                     }
                 }
@@ -987,9 +996,9 @@
                     pe[g][r] = x[g][r] - m_run[r];
                     over = fmaxf(over, pe[g][r]);
                 }
-            if (__any(over > MAX_SLACK<LONG> || (LONG && !ANY && v_out != 0))) {
+            if (any_lane(over > MAX_SLACK<LONG> || (LONG && !ANY && v_out != 0))) {
                 if constexpr (LONG && !ANY) {
-                    if (__builtin_expect(__any(v_out != 0), 0)) {
+                    if (__builtin_expect(any_lane(v_out != 0), 0)) {
                         if (v_needs_other_form(v_out != 0)) goto other_form;
                     }
                 }

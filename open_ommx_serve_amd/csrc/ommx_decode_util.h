@@ -22,6 +22,8 @@ __device__ __forceinline__ f32x4 mfma_f16(u32x4 a, u32x4 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
                                                   __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
 }
+// Whether any lane says so; uniform.  (__any goes through an integer: two vector instructions and their wait states more.)
+__device__ __forceinline__ bool any_lane(bool p) { return __builtin_amdgcn_ballot_w64(p) != 0; }
 __device__ __forceinline__ void lds_fence() {
     // LDS traffic of one wave is executed in order; this only stops the compiler from
     // moving accesses across a point where lanes exchange data through LDS.
