@@ -155,8 +155,8 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
             // One pass each through a three-deep max / median network.
             // (a fourth rank on either side: the largest and the smallest of the lanes that stay)
             // The ranks are formed two at once in packed 16-bit integers and the keys in one instruction each, the medians are
-            // spelled out.  With that, the extremes of V below and a shorter x / 3 a wave issues some 1040 vector instructions,
-            // 1220 before (a SIMD's vector unit is busy for 94 % of the launch): 32 K tokens into a pool 43.0 -> 41.2 us, 16 K
+            // spelled out.  With that, the extremes of V below and a shorter x / 3 a wave issues 1095 vector instructions,
+            // 1220 before (a SIMD's vector unit is busy for 91 to 94 % of the launch): 32 K tokens into a pool 43.0 -> 41.2 us, 16 K
             // with position streams 23.3 -> 21.7, 8 K 13.4 -> 13.0.
             int t[4], b[4];
             uint32_t upper = 0xFFFF0000u;
