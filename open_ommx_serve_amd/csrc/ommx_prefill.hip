@@ -33,7 +33,10 @@
 // one meets the vector phase of the other, share the staged tiles as well: 264 -> 191 us (events, one card, with two pieces
 // and no second pass).  In lockstep, without the shift, the eight waves took 210 us, as two workgroups of four 233 us; any
 // register spilled in the loop costs more than all of this, because its reload waits for the loads on their way (285 us).
-// Short prompts are latency: one group per workgroup, two workgroups per compute unit (see prefill_attention).  The
+// Short prompts are latency: one group per workgroup, two workgroups per compute unit (see prefill_attention).  Where the
+// workgroups leave compute units idle beside the longest chain of tiles, two groups take the keys of the same rows, every
+// other tile each with staging of its own and half a tile apart, and their sums are put together through LDS (SPLIT): 1.4 us a
+// tile of the chain instead of 2.1.  In lockstep, without the shift, 1024 rows took 39.0 us instead of 36.3 (one group 42.5).  The
 // library's fp32 attention took 2.45 ms.
 #include <algorithm>
 
@@ -48,6 +51,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -117,19 +121,26 @@ constexpr unsigned short V_LOW = (104 + 1) << 7, V_HIGH = ((104 + 31) << 7) - 1;
 constexpr int k_stride(int D) { return 2 * D + 16; }
 constexpr int V_STRIDE = 2 * KEYS + 16;
 
-template <int D, int GROUPS>
-__global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a, TileList tiles) {
+// GROUPS 2: two groups of waves that share the staged tiles.  SPLIT: two that take the even and the odd tiles of the same rows.
+template <int D, int GROUPS, bool SPLIT = false>
+__global__ void __launch_bounds__(SPLIT ? 512 : 256 * GROUPS, 2) prefill_kernel(PrefillArgs a, TileList tiles) {
     constexpr int KB = D / 16;           // 16-channel blocks of QK
     constexpr int DB = D / 32;           // 32-channel blocks of the output
     constexpr int CHUNKS = D / 8;        // 16-byte chunks of a K row
     constexpr int KS = k_stride(D), VS = V_STRIDE;
     constexpr int KLOADS = KEYS * CHUNKS / 256;
-    __shared__ __attribute__((aligned(16))) uint8_t s_k[2][KEYS * KS], s_v[2][D * VS];
+    static_assert(!SPLIT || GROUPS == 1, "groups that split the keys stage for themselves, as one group does");
+    constexpr int STEP = SPLIT ? 2 : 1;              // tiles from one of a group's to its next
+    constexpr int K_BUF = KEYS * KS, V_BUF = D * VS, GROUP_LDS = 2 * (K_BUF + V_BUF);
+    __shared__ __attribute__((aligned(16))) uint8_t s_kv[STEP][GROUP_LDS];       // K rows and transposed V, two tiles each
     __shared__ uint32_t s_inexact[kPrefillMaxRows / KEYS / 32];          // bit per tile: some V element is no f16
     __shared__ uint32_t s_top, s_again;              // largest |V| of the other tiles; a row wants all tiles again
     __shared__ int s_first[3][D], s_special;         // first row with +inf, -inf, NaN in a channel of V; whether there is one
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int col = lane & 31, half = lane >> 5, group = GROUPS == 2 ? wave >> 2 : 0;
+    const int col = lane & 31, half = lane >> 5, group = GROUPS == 2 || SPLIT ? wave >> 2 : 0;
+    uint8_t* const lds = s_kv[SPLIT ? group : 0];
+    auto s_k = [&](int t) { return lds + (t / STEP & 1) * K_BUF; };
+    auto s_v = [&](int t) { return lds + 2 * K_BUF + (t / STEP & 1) * V_BUF; };
     const int t0 = tiles.w[3 * blockIdx.y], len = tiles.w[3 * blockIdx.y + 1], q0 = tiles.w[3 * blockIdx.y + 2];
     // (neighbouring workgroups take neighbouring kv heads, so with 8 kv heads an XCD keeps to one)
     const int kvh = blockIdx.x % a.Hkv, part = blockIdx.x / a.Hkv;
@@ -138,7 +149,7 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
     const uint16_t* const kp = a.k + t0 * a.k_t + kvh * a.k_h;
     const uint16_t* const vp = a.v + t0 * a.v_t + kvh * a.v_h;
 
-    const int row_first = q0 + 32 * (wave & 3) + (pair ? 0 : QROWS * group), row = row_first + col;   // of this wave, of this lane
+    const int row_first = q0 + 32 * (wave & 3) + (pair || SPLIT ? 0 : QROWS * group), row = row_first + col;   // of this wave, of this lane
     u32x4 qf[KB];
     {
         const uint16_t* qp = a.q + (t0 + min(row, len - 1)) * a.q_t + h * a.q_h + 8 * half;
@@ -154,7 +165,7 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
 
     // key tiles of the workgroup and of this wave (causal; a wave whose rows are past the end has none)
     const int n_tiles = (min(len, q0 + (pair ? QROWS : GROUPS * QROWS)) + KEYS - 1) / KEYS;
-    const int n_mine = row_first < len ? min(n_tiles, (row_first + 31) / KEYS + 1) : 0;
+    int n_mine = row_first < len ? min(n_tiles, (row_first + 31) / KEYS + 1) : 0;
 
     // ---- staging.  The first group brings V: channels 8*d8.. of four neighbouring rows per thread, sixteen lanes write a
     // whole row of transposed V (head_dim 64: half of the threads).  The second group brings K: chunk kc of rows kr, ...
@@ -184,9 +195,9 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
 #pragma unroll
         for (int i = 0; i < 4; ++i) nx[i] = load16(rows, v_at + i * v_row);
     };
-    auto write_v = [&](int buf, const u32x4* f) {
+    auto write_v = [&](int t, const u32x4* f) {
         // keys 4kg..4kg+3 are block kg / 4, half kg & 1 of it, first or second four slots of that chunk
-        uint8_t* const at = s_v[buf] + 8 * d8 * VS + 16 * (2 * (kg >> 2) + (kg & 1)) + 8 * ((kg >> 1) & 1);
+        uint8_t* const at = s_v(t) + 8 * d8 * VS + 16 * (2 * (kg >> 2) + (kg & 1)) + 8 * ((kg >> 1) & 1);
 #pragma unroll
         for (int w = 0; w < 4; ++w)
 #pragma unroll
@@ -200,7 +211,7 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
         if (t >= n_tiles) return;
 #pragma unroll
         for (int i = 0; i < KLOADS; ++i)
-            *reinterpret_cast<u32x4*>(s_k[t & 1] + (kr + i * (256 / CHUNKS)) * KS + 16 * kc) = nk[i];
+            *reinterpret_cast<u32x4*>(s_k(t) + (kr + i * (256 / CHUNKS)) * KS + 16 * kc) = nk[i];
     };
     auto stage_v = [&](int t) {
         if (d8 >= CHUNKS) return;
@@ -220,7 +231,7 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
             }
         if (min(low[0], low[1]) < V_LOW - 1 || max(high[0], high[1]) > V_HIGH) atomicOr(&s_inexact[t >> 5], 1u << (t & 31));
         else v_top = __builtin_elementwise_max(v_top, high);
-        write_v(t & 1, f);
+        write_v(t, f);
     };
     // Elements of V that are no number are taken out of the staged rows, where a weight of zero (a row before them, a
     // piece of a weight) would turn them into NaN, and noted: every row from theirs on gets them in the end.
@@ -247,10 +258,10 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
     f32x16 s[2];                 // scores of the tile, transposed: lane's row is the query
     u32x4 p0[4], p1[4];          // their weights in two f16 pieces, by 16-key block
 
-    auto v_operand = [&](int buf, int b, int d) {
-        return *reinterpret_cast<const u32x4*>(s_v[buf] + (32 * d + col) * VS + 32 * b + 16 * half);
+    auto v_operand = [&](int t, int b, int d) {
+        return *reinterpret_cast<const u32x4*>(s_v(t) + (32 * d + col) * VS + 32 * b + 16 * half);
     };
-    auto scores = [&](int buf) {
+    auto scores = [&](int t) {
 #pragma unroll
         for (int g = 0; g < 2; ++g)
 #pragma unroll
@@ -260,7 +271,7 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
 #pragma unroll
             for (int i = 0; i < 4; ++i)
                 kf[kb2 & 1][i >> 1][i & 1] =
-                    *reinterpret_cast<const u32x4*>(s_k[buf] + (32 * (i & 1) + col) * KS + 32 * (2 * kb2 + (i >> 1)) + 16 * half);
+                    *reinterpret_cast<const u32x4*>(s_k(t) + (32 * (i & 1) + col) * KS + 32 * (2 * kb2 + (i >> 1)) + 16 * half);
         };
         read(0);
 #pragma unroll
@@ -285,12 +296,12 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
         if (inexact(t)) return;              // (follows after the loop)
         u32x4 vf[2][DB];                     // operands one block ahead, no further: registers
 #pragma unroll
-        for (int d = 0; d < DB; ++d) vf[0][d] = v_operand(t & 1, 0, d);
+        for (int d = 0; d < DB; ++d) vf[0][d] = v_operand(t, 0, d);
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
 #pragma unroll
             for (int d = 0; d < DB; ++d)
-                if (b < 3) vf[(b + 1) & 1][d] = v_operand(t & 1, b + 1, d);
+                if (b < 3) vf[(b + 1) & 1][d] = v_operand(t, b + 1, d);
 #pragma unroll
             for (int d = 0; d < DB; ++d) acc[d] = mfma_f16(vf[b & 1][d], p0[b], acc[d]);
 #pragma unroll
@@ -298,11 +309,17 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
             __builtin_amdgcn_sched_barrier(0);
         }
     };
+    // a row none of whose keys in this group has had any weight so far (scores of -inf): SPLIT, where the first tile is not every row's
+    auto finite = [](float x) { return SPLIT && x == -INFINITY ? 0.0f : x; };
     // vector phase: staging, then the online softmax of one row per lane
     auto vector_phase = [&](int t) {
-        if (GROUPS == 1 || !group) { stage_v(t); request_v(t + 1); }
-        if (GROUPS == 1) { stage_k(t + 1); request_k(t + 2); }
+        if (GROUPS == 1 || !group) {
+            if (!SPLIT || t < n_tiles) stage_v(t);
+            request_v(t + STEP);
+        }
+        if (GROUPS == 1) { stage_k(t + STEP); request_k(t + 2 * STEP); }
         else if (group) { stage_k(t + 2); request_k(t + 3); }
+        if (SPLIT && t >= n_mine) return;        // (all keys masked: there may be no maximum yet)
         mask(t);
         float mx = s[0][0];
 #pragma unroll
@@ -312,7 +329,7 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
         mx = fmaf(fmaxf(mx, other_half(mx)), a.scale_log2, -P_SHIFT);      // (the scale is positive)
         if (__any(mx > m + MAX_SLACK)) {
             const float m_new = fmaxf(m, mx);
-            const float shrink = __builtin_amdgcn_exp2f(m - m_new);       // 0 on the first tile
+            const float shrink = __builtin_amdgcn_exp2f(m - finite(m_new));       // 0 on the first tile
             m = m_new;
             l *= shrink;
 #pragma unroll
@@ -320,13 +337,14 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
 #pragma unroll
                 for (int r = 0; r < 16; ++r) acc[d][r] *= shrink;
         }
+        const float less = finite(m);
         float tile_l = 0.0f;      // (of its own: next to a large weight small ones would be rounded off one by one)
 #pragma unroll
         for (int b = 0; b < 4; ++b)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const float x = __builtin_amdgcn_exp2f(fmaf(s[b >> 1][8 * (b & 1) + 2 * i], a.scale_log2, -m));
-                const float y = __builtin_amdgcn_exp2f(fmaf(s[b >> 1][8 * (b & 1) + 2 * i + 1], a.scale_log2, -m));
+                const float x = __builtin_amdgcn_exp2f(fmaf(s[b >> 1][8 * (b & 1) + 2 * i], a.scale_log2, -less));
+                const float y = __builtin_amdgcn_exp2f(fmaf(s[b >> 1][8 * (b & 1) + 2 * i + 1], a.scale_log2, -less));
                 tile_l += x + y;
                 const f16x2 hi = __builtin_convertvector((f32x2{x, y}), f16x2);
                 const f32x2 rest = {minus_low(x, hi), minus_high(y, hi)};
@@ -334,7 +352,7 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
                 p1[b][i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(rest, f16x2));
             }
         l += tile_l;
-        if (GROUPS == 2) {        // all of it here: the compiler would move the weights behind the barrier, to their use
+        if (GROUPS == 2 || SPLIT) {        // all of it here: the compiler would move the weights behind the barrier, to their use
 #pragma unroll
             for (int b = 0; b < 4; ++b) asm volatile("" : "+v"(p0[b]), "+v"(p1[b]));
             asm volatile("" : "+v"(l));
@@ -344,23 +362,51 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
     if (tid < kPrefillMaxRows / KEYS / 32) s_inexact[tid] = 0;
     if (tid < D) s_first[0][tid] = s_first[1][tid] = s_first[2][tid] = INT32_MAX;
     if (tid == 0) s_top = s_again = s_special = 0;
-    if (GROUPS == 1 || group) { request_k(0); stage_k(0); request_k(1); }
-    if (GROUPS == 1 || !group) request_v(0);
+    const int t_first = SPLIT ? group : 0;
+    if (GROUPS == 1 || group) { request_k(t_first); stage_k(t_first); request_k(t_first + STEP); }
+    if (GROUPS == 1 || !group) request_v(t_first);
     __syncthreads();
     if (group) {                  // one phase behind the first group
-        stage_k(1);
-        request_k(2);
+        if (GROUPS == 2) { stage_k(1); request_k(2); }
         __syncthreads();
     }
-    scores(0);
-    if (GROUPS == 2) __syncthreads();
-    for (int t = 0; t < n_tiles; ++t) {
+    if (!SPLIT || t_first < n_mine) scores(t_first);
+    if (GROUPS == 2 || SPLIT) __syncthreads();
+    for (int t0s = 0; t0s < n_tiles; t0s += STEP) {
+        const int t = t0s + t_first;
         vector_phase(t);
         __syncthreads();
-        add_pv(t);
-        if (t + 1 < n_tiles) scores((t + 1) & 1);
+        if (!SPLIT || t < n_mine) add_pv(t);
+        if (t + STEP < (SPLIT ? n_mine : n_tiles)) scores(t + STEP);
         else asm volatile("" : "=v"(s[0]), "=v"(s[1]));           // (keeps the scores out of the loop's registers)
-        if (GROUPS == 2 && (!group || t + 1 < n_tiles)) __syncthreads();
+        if ((GROUPS == 2 || SPLIT) && (!group || t0s + STEP < n_tiles)) __syncthreads();
+    }
+    if constexpr (SPLIT) {
+        // the second group's sums to the first, which goes on alone (the second keeps its barriers company)
+        static_assert(GROUP_LDS >= (4 * DB + 1) * 256 * 16, "sums of a group");
+        f32x4* const there = reinterpret_cast<f32x4*>(s_kv[1]) + st;
+        __syncthreads();
+        if (group) {
+#pragma unroll
+            for (int i = 0; i < 4 * DB; ++i)
+                there[256 * i] = f32x4{acc[i >> 2][4 * (i & 3)], acc[i >> 2][4 * (i & 3) + 1], acc[i >> 2][4 * (i & 3) + 2], acc[i >> 2][4 * (i & 3) + 3]};
+            there[256 * 4 * DB] = f32x4{m, l, 0.0f, 0.0f};
+            n_mine = 0;
+        }
+        __syncthreads();
+        if (!group && n_mine > 0) {
+            const f32x4 ml = there[256 * 4 * DB];
+            const float m_new = fmaxf(m, ml[0]);
+            const float mine = __builtin_amdgcn_exp2f(m - m_new), other = __builtin_amdgcn_exp2f(ml[0] - m_new);
+            m = m_new;
+            l = l * mine + ml[1] * other;
+#pragma unroll
+            for (int i = 0; i < 4 * DB; ++i) {
+                const f32x4 x = there[256 * i];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[i >> 2][4 * (i & 3) + r] = acc[i >> 2][4 * (i & 3) + r] * mine + x[r] * other;
+            }
+        }
     }
 
     // Second pass over tiles whose V is not exact in f16: scores once more, weights against the final maximum in three bf16
@@ -371,14 +417,14 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
         for (int w = 0; w <= (n_tiles - 1) >> 5; ++w)
             for (uint32_t left = tiles_of(w); left; left &= left - 1) {
                 const int t = 32 * w + __builtin_ctz(left);
-                if (GROUPS == 1 || group) {
+                if (SPLIT ? !group : GROUPS == 1 || group) {
                     request_k(t);
                     stage_k(t);
                 }
-                if ((GROUPS == 1 || !group) && d8 < CHUNKS) {
+                if ((SPLIT ? !group : GROUPS == 1 || !group) && d8 < CHUNKS) {
                     request_v(t);
                     take_special(t);
-                    write_v(t & 1, nx);
+                    write_v(t, nx);
                 }
                 if (first) {
 #pragma unroll
@@ -390,7 +436,7 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
                 }
                 __syncthreads();
                 if (t < n_mine) {
-                    scores(t & 1);
+                    scores(t);
                     mask(t);
 #pragma unroll
                     for (int b = 0; b < 4; ++b) {
@@ -406,7 +452,7 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
 #pragma unroll
                             for (int i = 0; i < 8; ++i) x[i] -= __uint_as_float(__float_as_uint(x[i]) & 0xFFFF0000u);
 #pragma unroll
-                            for (int d = 0; d < DB; ++d) acc[d] = mfma_bf16(v_operand(t & 1, b, d), p, acc[d]);
+                            for (int d = 0; d < DB; ++d) acc[d] = mfma_bf16(v_operand(t, b, d), p, acc[d]);
                         }
                     }
                 }
@@ -428,14 +474,14 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
             for (int r = 0; r < 16; ++r) most = fmaxf(most, fabsf(acc[d][r]));
         most = fmaxf(most, other_half(most));
         const float top = __uint_as_float(s_top << 16) * gain * AGAIN_BELOW;
-        if (row < len && most * most < top * top * static_cast<float>(row + 1)) s_again = 1;
+        if (row < len && !(SPLIT && group) && most * most < top * top * static_cast<float>(row + 1)) s_again = 1;
     }
     __syncthreads();
     if (__builtin_amdgcn_readfirstlane(s_again))
         second_pass([&](int w) { return n_tiles - 32 * w >= 32 ? ~0u : (1u << (n_tiles - 32 * w)) - 1; }, 0.0f);
 
     const bool special = __builtin_amdgcn_readfirstlane(s_special);
-    if (row >= len) return;
+    if (row >= len || (SPLIT && group)) return;
     l += other_half(l);
     const float inv = 1.0f / (l * gain);
     const int64_t at = (t0 + row) * a.o_t + h * a.o_h;
@@ -463,10 +509,13 @@ __global__ void __launch_bounds__(256 * GROUPS, 2) prefill_kernel(PrefillArgs a,
         }
 }
 
+enum class Form { one_group, split_keys, two_groups };
 template <int D>
-void launch(const PrefillArgs& a, const TileList& list, int n, bool two_groups, hipStream_t st) {
-    if (two_groups)
+void launch(const PrefillArgs& a, const TileList& list, int n, Form form, hipStream_t st) {
+    if (form == Form::two_groups)
         hipLaunchKernelGGL((prefill_kernel<D, 2>), dim3(a.R % 2 ? a.Hkv * a.R : a.Hkv * a.R / 2, n), dim3(512), 0, st, a, list);
+    else if (form == Form::split_keys)
+        hipLaunchKernelGGL((prefill_kernel<D, 1, true>), dim3(a.Hkv * a.R, n), dim3(512), 0, st, a, list);
     else
         hipLaunchKernelGGL((prefill_kernel<D, 1>), dim3(a.Hkv * a.R, n), dim3(256), 0, st, a, list);
 }
@@ -506,12 +555,20 @@ int prefill_attention(const uint16_t* q, int64_t q_t, int64_t q_h, const uint16_
             key_tiles += (std::min(len, q0 + QROWS) + KEYS - 1) / KEYS;
         }
     const bool two_groups = groups * Hq >= 2 * 256 && key_tiles >= 8 * groups;
+    // One group a workgroup leaves compute units idle, or half empty, while the longest tiles are at their keys: then those are
+    // split.  Kernel alone, one group -> split, us, 32 q / 8 kv heads: 100 rows 11.8 -> 13.4, 200 15.4 -> 15.5, 300 17.6 -> 16.9, 433 21.7 ->
+    // 20.0, 622 29.7 -> 26.0, 1024 42.5 -> 36.3, head_dim 64 35.5 -> 30.6; 4000 rows of 8 heads 131.8 -> 99.7.  Two rounds of
+    // workgroups with their keys split pay where the tiles of the first are long: 1100 rows 49.3 -> 39.4, 1488 63.6 -> 52.9, 1900 82.9 -> 75.2,
+    // but 2 x 622 32.9 -> 32.2, 2 x 768 37.8 -> 38.8, 3 x 512 29.6 -> 35.0, 8 x 256 24.8 -> 35.9.
+    const int64_t workgroups = groups * Hq, longest = (most + KEYS - 1) / KEYS;
+    const bool split = !two_groups && ((workgroups <= 256 && longest >= 5) || (workgroups <= 512 && longest > 16));
+    const Form form = two_groups ? Form::two_groups : split ? Form::split_keys : Form::one_group;
     TileList list;
     int n = 0;
     hipStream_t st = static_cast<hipStream_t>(stream);
     auto flush = [&]() {
         if (n == 0) return;
-        if (D == 128) launch<128>(a, list, n, two_groups, st); else launch<64>(a, list, n, two_groups, st);
+        if (D == 128) launch<128>(a, list, n, form, st); else launch<64>(a, list, n, form, st);
         n = 0;
     };
     const int step = two_groups && a.R % 2 ? 2 * QROWS : QROWS;

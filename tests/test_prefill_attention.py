@@ -84,6 +84,43 @@ def test_long_prompts_in_two_wave_groups(D, hq, hkv, starts):
     assert bool((out[:starts[0]] == 7).all()) and bool((out[starts[-1]:] == 7).all())
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("starts", [[0, 257], [0, 321], [3, 387, 388, 700], [0, 1, 64, 449]])
+@pytest.mark.parametrize("case", ["plain", "no f16", "weightless", "infinite"])
+def test_keys_split_between_two_wave_groups(D, starts, case):
+    """Few workgroups with tiles of five and more: odd and even numbers of 64-key tiles, requests of one among them, and in
+    the second group's tiles V that is no f16, keys without weight (a row may have no other there), V that is no number."""
+    n, hq, hkv = starts[-1] + 3, 8, 2
+    q, k, v = _rows(n, hq, D, 1), _rows(n, hkv, D, 2), _rows(n, hkv, D, 3)
+    k[:, :, :3] *= 12
+    for a, b in zip(starts, starts[1:]):
+        if case == "no f16":
+            v[a + 64:b:2, :, 5] = 1e4
+        elif case == "weightless":
+            q[a:b, :, 7], k[a:b, :, 7] = 1e20, 0.0
+            for t in range(a + 64, b, 128):
+                k[t:min(t + 64, b), :, 7] = -1e20              # scores of -1e40, -inf in fp32
+        elif case == "infinite" and b - a > 70:
+            v[a + 70, :, 9] = float("inf")
+    out = torch.full((n, hq, D), 7.0, device=DEV)
+    assert _hip.host().prefill(q, k, v, out, starts, D ** -0.5)
+    if case == "infinite":
+        for a, b in zip(starts, starts[1:]):
+            if b - a > 70:
+                assert bool((out[a + 70:b, :, 9] == float("inf")).all())
+                v[a + 70, :, 9] = out[a + 70:b, :, 9] = 0.0
+    live = slice(starts[0], starts[-1])
+    want = _reference(q, k, v, starts, D ** -0.5)
+    if case == "infinite":
+        for a, b in zip(starts, starts[1:]):
+            if b - a > 70:
+                want[a + 70:b, :, 9] = 0.0
+    # fp32 sums of up to n weights, relative to the largest value of the channel
+    bound = 1e-5 * max(1.0, v[live].abs().max().item() / 8)
+    assert (out[live].double() - want[live]).abs().max().item() <= bound
+    assert bool((out[:starts[0]] == 7).all()) and bool((out[starts[-1]:] == 7).all())
+
+
 @pytest.mark.parametrize("hq,hkv,n", [(4, 2, 201), (64, 8, 1025)])       # one wave group, two
 @pytest.mark.parametrize("case", ["tiny", "huge", "some", "edges"])
 def test_values_that_are_no_f16(case, hq, hkv, n):
