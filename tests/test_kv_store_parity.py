@@ -81,6 +81,22 @@ def test_strided_source_rows_take_the_elementwise_path():
     assert torch.equal(vh[0, 7], v[0]) and torch.equal(vh[1, 39], v[1])
 
 
+@pytest.mark.parametrize("H,D", [(1, 8), (3, 24), (8, 128), (32, 128), (40, 128), (513, 8), (2, 8192), (1, 8200)])
+def test_written_rows_of_every_head_count_and_width(H, D):
+    """One piece of 16 bytes a thread, more heads than a workgroup has threads for, widths that no workgroup holds."""
+    kh = torch.zeros(2, 5, H, D, dtype=torch.bfloat16, device=DEV)
+    vh = torch.zeros_like(kh)
+    both = _rows(2, 2 * H, D, 6).to(DEV)         # K and V heads side by side: strides of their own
+    k, v = both[:, :H], both[:, H:]
+    pos = torch.tensor([4, 1], dtype=torch.int64, device=DEV)
+    write_tokens(kh, vh, pos, k, v, 0, 0, pos_next=pos)
+    assert pos.tolist() == [5, 2]
+    for got, new in ((kh, k), (vh, v)):
+        assert torch.equal(got[0, 4], new[0]) and torch.equal(got[1, 1], new[1])
+        got[0, 4] = got[1, 1] = 0
+        assert not got.any()
+
+
 @pytest.mark.parametrize("ring", [False, True])
 def test_gather_window_arithmetic_matches_the_host_closed_forms(ring):
     win = WindowSpec()
