@@ -84,7 +84,7 @@ __global__ void __launch_bounds__(1024) ring_write_kernel(
 }
 
 // The same with the places as arguments: no launch before this one has to bring them to the device; the step's other launches
-// read them from `block`, which the first layer's launch fills.  8 requests of 8 heads, kernel alone 2.6 us as the other, and the
+// read them from `block`, which the first layer's launch fills.  8 requests of 8 heads, kernel alone 2.4 us as the other, and the
 // upload's 1.4 are gone; the host's part of a step of two layers without its decodes 29 -> 20 us.
 __global__ void __launch_bounds__(1024) ring_step_kernel(RingArgs a, const uint16_t* k, const uint16_t* v, int64_t k_bs,
                                                          int64_t k_hs, int64_t v_bs, int64_t v_hs, int32_t* block, int vec,
