@@ -67,12 +67,20 @@ constexpr int TILE_ROW = 272;                       // bytes per row of the outl
 constexpr int KT_ROW = 40;                          // bytes per staged K code row (32 used): 16 rows read as b64 spread over all banks
 constexpr int VT_COL = 68;                          // dwords per V dword column (64 used)
 constexpr int PT_ROW = 72;                          // halfwords per row of the f16 [row][64 tokens] arrays
-constexpr int OFF_TILE = 0;                         // [32 tokens][TILE_ROW] f16 outlier deltas of one group
-// The rest depends on the number of q heads per kv head (NH = 4 or 8) and, with groups longer than 32 tokens, on one
+// Regions, in an order that makes row -1 of the tile, of the corrections and of the K codes harmless: the lowest bit of an empty
+// bitmap is -1 (lowest_bit), and a map with fewer bits than outlier slots is something a caller's planes can hold (the store
+// writes one, and reports it, for a K vector without enough distinct values; a converted index plane has zeros for a bad
+// vector).  A code row -1 is read from the wave's own constant rows, a tile row -1 is written over staged V that nobody reads
+// any more, corrections of a row -1 go to the unused end of the tile's last row: the neighbouring wave, another kv head, is not
+// touched, and no position needs an instruction for it (a test where corrections are added, which most groups do for some
+// entry, cost 1 % at 64 K).
+// They depend on the number of q heads per kv head (NH = 4 or 8) and, with groups longer than 32 tokens, on one
 // more row of the tile: where the outliers of the group's other tokens go.
 template <int NH, bool LONG>
 struct LdsMap {
-    static constexpr int OFF_KT = OFF_TILE + (LONG ? 33 : 32) * TILE_ROW;    // [64 tokens][KT_ROW] K code rows
+    static constexpr int OFF_ZERO = 0;                         // 128 B of zeros, never written again
+    static constexpr int OFF_ONES = OFF_ZERO + 128;            // 128 B of f16 1.0, never written again
+    static constexpr int OFF_KT = OFF_ONES + 128;              // [64 tokens][KT_ROW] K code rows
     static constexpr int OFF_MAG = OFF_KT + 64 * KT_ROW;       // [2 groups][128] f16 2^e, channels (p, p+8) adjacent
     static constexpr int OFF_ZPP = OFF_MAG + 512;              // same order, f16 zero points over the A scale
     // after QK the same bytes hold what P.V needs
@@ -80,12 +88,14 @@ struct LdsMap {
     static constexpr int OFF_PT = OFF_VT + 8 * VT_COL * 4;     // [NH heads][PT_ROW] f16 softmax weights
     static constexpr int OFF_VZ = OFF_PT + NH * PT_ROW * 2;    // [4 channel groups][PT_ROW] f16 V zero points
     static constexpr int OFF_VS = OFF_VZ + 4 * PT_ROW * 2;     // [4 channel groups][PT_ROW] f16 2^e_v
-    static constexpr int OFF_STAGE_END = (OFF_VS + 4 * PT_ROW * 2 > OFF_ZPP + 512) ? OFF_VS + 4 * PT_ROW * 2 : OFF_ZPP + 512;
-    static constexpr int OFF_LC = OFF_STAGE_END;               // [tokens][NH heads] f32 logit corrections of one group (32), or of a step of a longer one (64)
-    static constexpr int OFF_ZERO = OFF_LC + (LONG ? 64 : 32) * NH * 4;      // 128 B of zeros, never written again
-    static constexpr int OFF_ONES = OFF_ZERO + 128;            // 128 B of f16 1.0, never written again
-    static constexpr int LDS_WAVE = OFF_ONES + 128;            // 13376 (4 heads) / 14464 (8 heads), LONG 272 more
-    static_assert(OFF_KT % 16 == 0 && OFF_PT % 16 == 0 && OFF_VZ % 16 == 0 && OFF_LC % 16 == 0, "b128 alignment");
+    static constexpr int OFF_TILE = OFF_VS + 4 * PT_ROW * 2;   // [32 tokens][TILE_ROW] f16 outlier deltas of one group
+    static constexpr int TILE_END = OFF_TILE + (LONG ? 33 : 32) * TILE_ROW;
+    static constexpr int OFF_LC = TILE_END + (NH == 8 ? 16 : 0);             // [tokens][NH heads] f32 logit corrections of one group (32), or of a step of a longer one (64)
+    static constexpr int LDS_WAVE = OFF_LC + (LONG ? 64 : 32) * NH * 4;      // 13376 (4 heads) / 14480 (8 heads), LONG 784 / 1296 more
+    static_assert(OFF_KT % 16 == 0 && OFF_PT % 16 == 0 && OFF_VZ % 16 == 0 && OFF_TILE % 16 == 0 && OFF_LC % 16 == 0, "b128 alignment");
+    static_assert(OFF_KT - KT_ROW >= OFF_ZERO, "code row -1: the constant rows");
+    static_assert(OFF_TILE - TILE_ROW >= OFF_ZPP + 512, "tile row -1: behind what is staged for K");
+    static_assert(OFF_LC - NH * 4 >= TILE_END - (TILE_ROW - 256), "corrections of row -1: behind the tile's last channel");
 };
 // LDS is handed out in pieces of 1280 bytes (768 workgroups of 53760 bytes on 256 compute units take one round, of 53776 two).
 // Longer groups (56640 bytes, and more than 168 registers) have two workgroups a compute unit, not three.
@@ -173,8 +183,8 @@ __device__ __forceinline__ uint32_t v_op(uint32_t m, uint32_t step) {
     const f16x2 one = {1.0f, 1.0f};
     return __builtin_bit_cast(uint32_t, (__builtin_bit_cast(f16x2, v_pair<Y, LONG>(m, 0x3C003C00u)) - one) * __builtin_bit_cast(f16x2, step));
 }
-// Outlier positions of a bitmap from below: the lowest set bit, and the map without the bit at `pos`, one addition of
-// -1 << pos (m & (m - 1) takes two instructions).
+// Outlier positions of a bitmap from below: the lowest set bit (-1 of an empty map, see LdsMap), and the map without the bit at
+// `pos`, one addition of -1 << pos (m & (m - 1) takes two instructions).
 __device__ __forceinline__ int lowest_bit(uint32_t m) {
     int pos;
     asm("v_ffbl_b32 %0, %1" : "=v"(pos) : "v"(m));

@@ -15,7 +15,7 @@
     const int kout = GEN ? a.kout : KMAX;
     const bool half = GEN ? a.half != 0 : HALF;
     using Lds = LdsMap<NH, LONG>;
-    constexpr int OFF_KT = Lds::OFF_KT, OFF_MAG = Lds::OFF_MAG, OFF_ZPP = Lds::OFF_ZPP, OFF_VT = Lds::OFF_VT,
+    constexpr int OFF_TILE = Lds::OFF_TILE, OFF_KT = Lds::OFF_KT, OFF_MAG = Lds::OFF_MAG, OFF_ZPP = Lds::OFF_ZPP, OFF_VT = Lds::OFF_VT,
                   OFF_PT = Lds::OFF_PT, OFF_VZ = Lds::OFF_VZ, OFF_VS = Lds::OFF_VS, OFF_LC = Lds::OFF_LC, OFF_ZERO = Lds::OFF_ZERO,
                   OFF_ONES = Lds::OFF_ONES, LDS_WAVE = Lds::LDS_WAVE;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem_all[];

@@ -10,7 +10,7 @@ import torch
 import oracle.ommx_oracle as O
 from open_ommx_serve_amd.attention import _hip
 from open_ommx_serve_amd.attention.kv_window import WindowSpec
-from open_ommx_serve_amd.attention.pack import ommx_pack_kv_canonical_block
+from open_ommx_serve_amd.attention.pack import ommx_pack_kv_canonical_block, store_pack_into
 from open_ommx_serve_amd.attention.paged_decode import (auto_num_kv_splits, make_attn_logits,
                                                         ommx_paged_decode_attention_canonical)
 from open_ommx_serve_amd.synth import build_decode_case
@@ -694,6 +694,56 @@ def test_exact_residuals_at_head_dim_64_go_to_the_heads_of_their_own_kv_head(len
         d = (o.double() - wo).abs()
         assert d.max().item() <= MAX_ABS and d.mean().item() <= MEAN_ABS, f"S{S}: {d.max().item():.3e}"
         assert ((lse.double() - wl).abs() <= 2e-3 + 1e-5 * wl.abs()).all(), f"S{S}: lse"
+
+
+@pytest.mark.parametrize("hq,hkv,D,k,own_map,how", [
+    (32, 8, 128, 6, True, "emptied"), (64, 8, 128, 6, False, "emptied"), (8, 8, 128, 6, True, "emptied"), (32, 8, 128, 3, False, "emptied"),
+    (64, 8, 128, 5, True, "emptied"), (16, 8, 128, 8, True, "emptied"), (32, 8, 64, 6, True, "emptied"), (16, 8, 64, 6, False, "emptied"),
+    (16, 8, 64, 5, True, "emptied"), (32, 8, 128, 6, True, "nan"), (64, 8, 128, 6, False, "nan"), (32, 8, 128, 5, True, "nan"),
+    (32, 8, 128, 6, True, "2e9"), (64, 8, 128, 8, False, "2e9")])
+def test_maps_with_fewer_bits_than_outliers_concern_their_own_head_alone(hq, hkv, D, k, own_map, how):
+    """Four kv heads share a workgroup and its LDS.  Heads 0, 1 and 7 (the first, one between two others and the last of a
+    workgroup) get bitmaps with 0 .. k bits, emptied by the caller or stored from a channel without k distinct values: the
+    other heads' results keep their bits.  Queries of 8 times the size have roundings of the entries settled, too.  (At
+    head_dim 64 a wave has two kv heads and refreshes the running maximum of both at once: head 6, beside head 7, takes weights
+    against another maximum, each rounded to f16 as before, and stays within the tolerance of any decode.)"""
+    case = build_decode_case([1700, 333], q_heads=hq, kv_heads=hkv, head_dim=D, seed=94, permute_tables=True, sparse_frac=0.005,
+                             outliers_per_vector=k, kv_outlier_map=own_map, keep_source=True)
+    case.q.mul_(8.0)
+    want = {S: _run(case, num_kv_splits=S) for S in (None, 1, 3)}
+    bad, p = [0, 1, 7], case.planes
+    if how == "emptied":
+        maps = p["k_obmp"].view(torch.int32)                     # [groups, heads, channels, 1]
+        channel = torch.arange(D, device=maps.device)
+        for h in bad:
+            m = maps[:, h, :, 0].clone()
+            for i in range(k):                                   # channel c keeps its lowest c % (k + 1) bits
+                low = m & -m
+                maps[:, h, :, 0] ^= torch.where(channel % (k + 1) <= i, low, 0)
+                m ^= low
+    else:
+        err = torch.zeros(1, dtype=torch.int32, device=case.q.device)
+        for b, n in enumerate(case.packed_lens):
+            K, V = (x[8:8 + n].cuda() for x in case.extra["source"][b])
+            for h in bad:
+                K[:64, h, 5] = K[-32:, h, 64:70] = float(how)
+            store_pack_into(K, V, p, outliers_per_vector=k, page_size=16, err_flag=err,
+                            dst_pages=case.req_to_token[b, :n // 16].int(), dst_groups=case.req_to_group[b, :n // 32].int())
+        assert int(err.item()) & _hip.ERR_UNDERFILLED
+    heads = torch.ones(hkv, hq // hkv, dtype=torch.bool)
+    heads[bad] = False
+    sound = heads.flatten().clone()
+    if D == 64:
+        heads[6] = False
+    alone = heads.flatten()
+    for S, (wo, wl) in want.items():
+        for _ in range(3):
+            o, lse = _run(case, num_kv_splits=S)
+            assert torch.equal(o[:, alone], wo[:, alone]) and torch.equal(lse[:, alone], wl[:, alone]), f"S{S}"
+            assert (o - wo)[:, sound].abs().max().item() <= MAX_ABS, f"S{S}"
+            assert ((lse - wl).abs() <= 2e-3 + 2e-6 * wl.abs())[:, sound].all(), f"S{S}"
+        if how == "emptied":
+            assert torch.isfinite(o).all() and not torch.equal(o[:, ~sound], wo[:, ~sound])
 
 
 @pytest.mark.parametrize("hq,hkv,D,k,own_map", [(32, 8, 128, 6, True), (64, 8, 128, 6, True), (32, 8, 128, 5, False),
