@@ -130,6 +130,8 @@ constexpr int EXACT_STEP_EXP = 5;
 // f16 operands: steps above 2^15 do not fit (K or V values beyond some 1e5); such a step is held at 2^15
 // and OMMX_ERR_VALUE_RANGE is reported
 constexpr int MAX_STEP_EXP = 15;
+// largest step whose 2^24-fold over the smallest A scale, 4, is an fp32 number
+constexpr int CODE_STEP_EXP = 105;
 // Longer groups were served before by a kernel with bf16 operands for K, which hold every step, and steps of V down to 2^-24.
 // They keep that range.  A wave that meets a step of K or V outside 2^-14..2^15 (normal f16 numbers) with a code that is not
 // zero, or a zero point of K from 2^18 on, or that has a query of 2^12 or more, drops what it has and walks its split in a

@@ -355,6 +355,10 @@
     }
     const uint32_t kt_lane = OFF_KT + (c0 >> 2);                   // code byte of the channel pair (4 channels a byte), row 0
     const uint32_t code_bits = 3u << (2u * (c0 & 3u));            // of channel c0's code in that byte; c0 + 1 sits two bits on
+    // A code is taken where it lies in its byte, as the bits of a subnormal f16, 2^-24 each: a mask and one mixed multiply-add, in
+    // the place of a shift, a conversion and a multiply-add.  Exact, as long as its step times 2^24 is an fp32 number; ANY, where
+    // steps of every size come by, takes the masked byte as a number.  This is the exponent of the unit that it counts.
+    auto code_unit = [&](int u) { return (ANY ? 0 : 24) - ((lane & 1) ? 4 : 0) - 2 * u; };
     const uint32_t kbytes = static_cast<uint32_t>(kout + 1) >> 1;            // nibble bytes per channel
     const uint32_t nib_sh = 8u * ((2u * kbytes * lane) & 3u);
     const uint32_t nib_at = (lane & 1) ? 0x0C040302u : 0x0C020100u;          // 6 outliers: the bytes of channel c0's nibbles (c0 + 1: three on)
@@ -396,7 +400,16 @@
             // (a scaled-down query means operands near the top of f16: the same cancellation, the same remedy)
             // (not any_lane: with this test in a scalar register up to 16 vector registers are spilled)
             exact_step = __any(e_top >= EXACT_STEP_EXP * 256) != 0 || q_down != 0;
-            if (__builtin_expect(exact_step, 0)) over_step |= __any(e_top > MAX_STEP_EXP * 256) != 0;
+            if (__builtin_expect(exact_step, 0)) {
+                over_step |= __any(e_top > MAX_STEP_EXP * 256) != 0;
+                // (the walk below takes such a step times 2^24, past the largest fp32 if it is not held here: far outside f16, as it was)
+#pragma unroll
+                for (int g = 0; g < NG; ++g) {
+                    const uint32_t held = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(
+                        __builtin_bit_cast(s16x2e, __builtin_amdgcn_perm(0u, g_sc[g], 0x010C000Cu)), s16x2e{CODE_STEP_EXP * 256, CODE_STEP_EXP * 256}));
+                    g_sc[g] = __builtin_amdgcn_perm(0u, held, 0x0C0C0301u);
+                }
+            }
         }
         {
             u32x2* krow = reinterpret_cast<u32x2*>(sm + OFF_KT + lane * KT_ROW);
@@ -493,9 +506,7 @@
                 const int e = static_cast<int8_t>((g_sc[0] >> (8 * u)) & 0xFFu);
                 // in units of the channel's A scale, as in the walk of 32-token groups below
                 const float cs = u ? cs1 : cs0;
-                // (the code is taken as the bits of a subnormal f16, 2^-24 each, where it lies in its byte: a mask and one mixed
-                // multiply-add, exact, in the place of a shift, a conversion and a multiply-add)
-                const float code_step = __builtin_ldexpf(cs, e + ((lane & 1) ? 20 : 24) - 2 * u);
+                const float code_step = __builtin_ldexpf(cs, e + code_unit(u));
                 float a1, b1 = 0.0f;
                 if (OWN_MAP) {
                     a1 = cs * __builtin_amdgcn_rcpf(__uint_as_float(u ? (g_ms[0] & 0xFFFF0000u) : (g_ms[0] << 16)));
@@ -516,7 +527,8 @@
                 float dl_max = 0.0f;
 #pragma unroll
                 for (int sidx = 0; sidx < KMAX; ++sidx) {
-                    float dl = fmaf(-f16_bits(cb[sidx] & (code_bits << 2 * u)), code_step, fmaf(lv[sidx], a1, b1));
+                    const uint32_t code = cb[sidx] & (code_bits << 2 * u);
+                    float dl = fmaf(ANY ? -static_cast<float>(code) : -f16_bits(code), code_step, fmaf(lv[sidx], a1, b1));
                     // (the entry as a value of its own: rounded to f16 here exactly as the residual pass rounds it)
                     asm("" : "+v"(dl));
                     dls[u][sidx] = dl;
@@ -602,14 +614,10 @@
                 // everything below is in units of the channel's A scale: tile entry =
                 // (outlier - zp - code * 2^e) / 2^(10-2m) = level * a1 + b1 less the code's step times the code
                 const float cs = u ? cs1 : cs0;
-                // (the code is taken as the bits of a subnormal f16, 2^-24 each, where it lies in its byte: a mask and one mixed
-                // multiply-add, exact, in the place of a shift, a conversion and a multiply-add)
-                // (a code is taken as the bits of a subnormal f16, 2^-24 each, where it lies in its byte: a mask and one mixed
-                // multiply-add, exact, in the place of a shift, a conversion and a multiply-add.  With positions by two
-                // instructions instead of three, one test a channel for residuals and nibbles by one permutation the pass over a
-                // group's outliers is 126 vector instructions, 157 before: 64 K 31.4 -> 30.8 us, 8 x 32 K with 64 q heads
-                // 103.5 -> 102.4, 32 of 1 to 16 K with position streams 100.3 -> 98.7.)
-                const float code_step = __builtin_ldexpf(cs, e + ((lane & 1) ? 20 : 24) - 2 * u);
+                // (With codes by two instructions, positions by two instead of three, one test a channel for residuals and nibbles
+                // by one permutation the pass over a group's outliers is 126 vector instructions, 157 before: 64 K 31.4 -> 30.8 us,
+                // 8 x 32 K with 64 q heads 103.5 -> 102.4, 32 of 1 to 16 K with position streams 100.3 -> 98.7.)
+                const float code_step = __builtin_ldexpf(cs, e + code_unit(u));
                 float a1, b1;
                 if (OWN_MAP) {
                     const float ms = __uint_as_float(u ? (g_ms[pg] & 0xFFFF0000u) : (g_ms[pg] << 16));
@@ -635,7 +643,8 @@
 #pragma unroll
                 for (int sidx = 0; sidx < KMAX; ++sidx) {
                     const float dl0 = fmaf(lv[sidx], a1, b1);
-                    float dl = fmaf(-f16_bits(cb[sidx] & (code_bits << 2 * u)), code_step, dl0);
+                    const uint32_t code = cb[sidx] & (code_bits << 2 * u);
+                    float dl = fmaf(-f16_bits(code), code_step, dl0);
                     // (the entry as a value of its own: rounded to f16 here exactly as the residual pass rounds it)
                     asm("" : "+v"(dl));
                     dls[sidx] = dl;

@@ -388,14 +388,14 @@ def test_the_largest_weight_of_a_longer_group_is_one(gt, k, hq):
 
 @pytest.mark.parametrize("gt,gc,k,hq,own_map", [(64, 64, 6, 32, False), (128, 64, 6, 64, True), (128, 128, 10, 32, True),
                                                 (128, 32, 10, 64, False)])
-@pytest.mark.parametrize("kind", ["large", "small", "small, ordinary q", "zero points", "entries"])
+@pytest.mark.parametrize("kind", ["large", "largest", "small", "small, ordinary q", "zero points", "entries"])
 def test_longer_groups_take_k_steps_of_every_size(gt, gc, k, hq, own_map, kind):
-    """K times 2^16 or 2^-20 and q divided by it (the same logits), steps of 2^-16 under ordinary queries, zero points beyond
+    """K times 2^16, 2^110 or 2^-20 and q divided by it (the same logits), steps of 2^-16 under ordinary queries, zero points beyond
     2^18 and outliers whose distance to the base code no f16 holds: nothing is held at a bound, so nothing is reported."""
     case = build_decode_case([700, 333], q_heads=hq, kv_heads=8, seed=88, permute_tables=True, group_tokens=gt,
                              group_channels=gc, outliers_per_vector=k, outlier_repr="relidx7", kv_outlier_map=own_map,
                              outlier_gain=3.0e5 if kind == "entries" else 1.0)
-    p, up = case.planes, {"large": 16, "small": -20, "small, ordinary q": -16}.get(kind, 0)
+    p, up = case.planes, {"large": 16, "largest": 110, "small": -20, "small, ordinary q": -16}.get(kind, 0)
     p["k_scale"] += up
     for name, by in (("k_zp", 2.0 ** up), ("k_fp4_mapcenter", 2.0 ** up), ("k_fp4_mapscale", 2.0 ** -up)):
         if p[name] is not None:
@@ -411,7 +411,7 @@ def test_longer_groups_take_k_steps_of_every_size(gt, gc, k, hq, own_map, kind):
         case.q *= 2.0 ** -16
     assert (case.q.abs().max() < 128) == (kind != "small")
     top = int(p["k_scale"].max())
-    assert {"large": top > 15, "entries": top > 15}.get(kind, top < 15), top
+    assert {"large": top > 15, "largest": 127 > top >= 110, "entries": top > 15}.get(kind, top < 15), top
     err = torch.zeros(1, dtype=torch.int32, device=case.q.device)
     wo, wl = _oracle(case)
     for S in (None, 1):
@@ -744,6 +744,28 @@ def test_maps_with_fewer_bits_than_outliers_concern_their_own_head_alone(hq, hkv
             assert ((lse - wl).abs() <= 2e-3 + 2e-6 * wl.abs())[:, sound].all(), f"S{S}"
         if how == "emptied":
             assert torch.isfinite(o).all() and not torch.equal(o[:, ~sound], wo[:, ~sound])
+
+
+@pytest.mark.parametrize("hq,D,k,rep,own_map", [(32, 128, 6, "bitmap", True), (64, 128, 6, "bitmap", False), (32, 128, 6, "relidx7", True),
+                                                (64, 128, 6, "relidx7", False), (32, 128, 5, "bitmap", True), (8, 128, 3, "bitmap", False),
+                                                (32, 64, 6, "bitmap", True), (16, 64, 8, "bitmap", False)])
+@pytest.mark.parametrize("exp", [105, 106, 120, 127])
+def test_a_step_of_any_size_over_codes_of_zero_adds_nothing(hq, D, k, rep, own_map, exp):
+    """Channels that do not vary (codes and outlier levels zero, K the zero point) under exponent bytes up to the largest:
+    the step is reported, and zero times it stays zero."""
+    case = build_decode_case([700, 333], q_heads=hq, kv_heads=8, head_dim=D, seed=95, permute_tables=True, sparse_frac=0.005,
+                             outliers_per_vector=k, outlier_repr=rep, kv_outlier_map=own_map)
+    p = case.planes
+    for c in (0, 3, 13, D - 2):
+        p["k_scale"][..., c] = exp
+        p["k_base"][..., c // 4] &= 0xFF ^ (3 << 2 * (c % 4))
+        p["k_oval"][:, :, c] = 0
+        if own_map:
+            p["k_fp4_mapcenter"][..., c] = p["k_zp"][..., c]
+    want, err = _oracle(case), torch.zeros(1, dtype=torch.int32, device=case.q.device)
+    for S in (None, 3):
+        _check(_run(case, num_kv_splits=S, err_flag=err), want, f"S{S}")
+    assert int(err.item()) & _hip.ERR_VALUE_RANGE
 
 
 @pytest.mark.parametrize("hq,hkv,D,k,own_map", [(32, 8, 128, 6, True), (64, 8, 128, 6, True), (32, 8, 128, 5, False),
