@@ -413,8 +413,13 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
             mn = __builtin_elementwise_minimum(mn, v[c]);
             mx = __builtin_elementwise_maximum(mx, v[c]);
         }
-        const bool fin = is_finite_f32(mn) && is_finite_f32(mx);
-        if (!fin) err |= OMMX_ERR_NONFINITE_V;
+        if (!(is_finite_f32(mn) && is_finite_f32(mx))) {
+            err |= OMMX_ERR_NONFINITE_V;
+            // a vector with a NaN is packed between the extremes of its other elements
+            mn = v[0]; mx = v[0];
+#pragma unroll
+            for (int c = 1; c < 32; ++c) { mn = fminf(mn, v[c]); mx = fmaxf(mx, v[c]); }
+        }
         const float raw = third(fmaxf(mx - mn, 1e-8f));
         const Step st = make_step(raw, scale_mode, tab);
         if (!st.in_range) err |= OMMX_ERR_EXP_RANGE;

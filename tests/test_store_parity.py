@@ -589,3 +589,30 @@ def test_one_value_that_is_not_finite_is_found_wherever_it_lies(T, bad):
         err.zero_()
         store_pack_into(K, V, planes, err_flag=err)
         assert int(err.item()) == 0
+
+
+@pytest.mark.parametrize("T", [64, 64 * 140])                 # K and V of a group in two workgroups, and in one
+@pytest.mark.parametrize("D,fp32,kw", [(128, False, {}), (128, False, dict(outlier_repr="relidx7")), (128, True, {}),
+                                       (64, False, dict(outliers_per_vector=3))])
+def test_a_nan_in_v_leaves_the_extremes_to_the_other_elements(T, D, fp32, kw):
+    """A vector with a NaN is reported, and packed between the smallest and the largest of its other elements, the NaN as code
+    3: the zero point and the step are those of the vector with its smallest element in that place.  One NaN at every place of a
+    vector (head 0), all but one element (head 1)."""
+    K, V = (x.float() if fp32 else x for x in synth_kv(T, 2, D, 12))
+    v = V.view(T, 2, D // 32, 32)
+    t, j, c = torch.arange(T), torch.arange(T) % (D // 32), torch.arange(T) % 32
+    nan = torch.zeros(v.shape, dtype=torch.bool)
+    nan[t, 0, j, c] = True
+    nan[t, 1, j] = True
+    nan[t, 1, j, c] = False
+    least = torch.where(nan, float("inf"), v.float()).amin(-1, keepdim=True).to(v.dtype)
+    got = []
+    for fill in (torch.full_like(v, float("nan")), least.expand_as(v)):
+        planes = alloc_planes(T // 16, T // 32, 2, D, device="cuda", **{"outliers_per_vector": 6, **kw})
+        err = torch.zeros(1, dtype=torch.int32, device="cuda")
+        store_pack_into(K.cuda(), torch.where(nan, fill, v).view(T, 2, D).cuda(), planes, err_flag=err, **kw)
+        assert bool(int(err.item()) & _hip_lib.ERR_NONFINITE_V) == (not got)
+        codes = planes["v_main"].cpu().view(T, 2, D // 4, 1) >> torch.tensor([0, 2, 4, 6], dtype=torch.uint8) & 3
+        got.append((planes["v_zp"].cpu().view(torch.int16), planes["v_scale"].cpu(), codes.view(nan.shape)))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    assert torch.equal(got[0][2][~nan], got[1][2][~nan]) and bool((got[0][2][nan] == 3).all())
