@@ -291,9 +291,18 @@ __global__ void __launch_bounds__(512, GT < GC ? 1 : GT == 32 ? 8 : GT == 64 ? 7
             const float wv = value_of_rank(key);
             const float mapped = own_map ? (wv - mc) * ms : (st.inv_ok ? (wv - zp) * st.inv : __fdiv_rn(wv - zp, st.scale));
             if (r % KH == 0) mfin = mfin && is_finite_f32(mapped);
-            slot[r] = pos << 4 | static_cast<int>(fp4_encode_sorted(mapped, thr));
+            slot[r] = pos << 5 | (r < KH ? 0 : 16) | static_cast<int>(fp4_encode_sorted(mapped, thr));
         }
         sort_ascending(slot);
+        if (picked != K) {          // positions taken from both ends (reported): each once, with its code from the lower end; then the last again
+#pragma unroll
+            for (int s = 0; s + 1 < K; ++s)
+                if (slot[s] >> 5 == slot[s + 1] >> 5) slot[s] = INT_MAX;
+            sort_ascending(slot);
+#pragma unroll
+            for (int s = 1; s < K; ++s)
+                if (slot[s] == INT_MAX) slot[s] = slot[s - 1];
+        }
         if (!mfin) err |= OMMX_ERR_NONFINITE_K;
 
         const int64_t gidx = (gs * H + h) * D + d;
@@ -304,7 +313,7 @@ __global__ void __launch_bounds__(512, GT < GC ? 1 : GT == 32 ? 8 : GT == 64 ? 7
         uint64_t nib = 0, lo = 0, hi = 0;           // position s at bits [7s, 7s+7) of hi:lo
 #pragma unroll
         for (int s = 0; s < K; ++s) {
-            const uint64_t pos = static_cast<uint32_t>(slot[s]) >> 4;
+            const uint64_t pos = static_cast<uint32_t>(slot[s]) >> 5;
             nib |= static_cast<uint64_t>(slot[s] & 0xF) << (4 * s);
             if (7 * s < 64) lo |= pos << (7 * s);
             if (7 * s + 7 > 64) hi |= 7 * s >= 64 ? pos << (7 * s - 64) : pos >> (64 - 7 * s);

@@ -8,7 +8,7 @@ import torch
 
 import oracle.ommx_oracle as O
 from conftest import bits_of
-from open_ommx_serve_amd.attention import ommx_pack_kv_canonical_block
+from open_ommx_serve_amd.attention import _hip, ommx_pack_kv_canonical_block
 from open_ommx_serve_amd.attention.pack import alloc_planes, store_pack_into
 from open_ommx_serve_amd.synth import synth_kv
 
@@ -115,3 +115,27 @@ def test_tokens_of_a_pair_on_pages_of_any_size(gt, gc, D, k, ps):
             assert np.array_equal(bits_of(got), bits_of(want[n].reshape(T, H, -1))), n
         for n in ("k_scale", "k_zp", "k_oval", "k_oidx", "k_fp4_mapscale", "k_fp4_mapcenter"):
             assert np.array_equal(bits_of(planes[n].cpu()), bits_of(want[n])), n
+
+
+@pytest.mark.parametrize("gt,gc,D,k,rep", [(32, 32, 64, 6, "bitmap"), (64, 64, 128, 6, "bitmap"), (64, 32, 96, 10, "bitmap"),
+                                           (32, 32, 64, 6, "relidx7"), (64, 64, 128, 6, "relidx7"), (128, 128, 128, 10, "relidx7")])
+def test_positions_taken_from_both_ends_keep_codes_and_positions_together(gt, gc, D, k, rep):
+    """A channel of 3e9 but for k/2 - 1 tokens: the lanes of the largest count as 1e9 for the smallest, so one of them is taken
+    twice and a slot is left over, which is reported.  Codes stay beside the positions they belong to."""
+    half, low = k // 2, [7, 19, 20, 31][:k // 2 - 1]
+    K, V = synth_kv(gt, 2, D, seed=5)
+    K[:, 1, 3] = 3e9
+    K[low, 1, 3] = -3e9
+    planes = alloc_planes(gt // 16, 1, 2, D, device="cuda", outliers_per_vector=k, outlier_repr=rep, group_tokens=gt, group_channels=gc)
+    err = torch.zeros(1, dtype=torch.int32, device="cuda")
+    store_pack_into(K.cuda(), V.cuda(), planes, err_flag=err, outliers_per_vector=k, outlier_repr=rep, group_tokens=gt, group_channels=gc)
+    assert int(err.item()) & _hip.ERR_UNDERFILLED
+    index = planes["k_obmp" if rep == "bitmap" else "k_oidx"][0, 1, 3].tolist()
+    bits = sum(b << (8 * i) for i, b in enumerate(index))
+    want = [*range(half), *low]
+    if rep == "bitmap":
+        assert [i for i in range(gt) if bits >> i & 1] == want
+    else:
+        assert [bits >> (7 * s) & 127 for s in range(k)] == [*want, want[-1]]
+    codes = [planes["k_oval"][0, 1, 3, s // 2].item() >> (4 * (s & 1)) & 15 for s in range(k)]
+    assert len(set(codes[1:half])) == 1 and len(set(codes[half:k - 1])) == 1 and codes[1] != codes[half]
