@@ -201,6 +201,7 @@ class MultiSeqKVPool:
         self._dbuf: Optional[Dict[str, object]] = None
         self._planes_cache: Optional[dict] = None
         self._host = _hip.host()
+        self.step_rows = self._host.STEP_ROWS
         # what every store launch of this pool is told (argument order of the native launchers)
         self._recipe = (self.k, self.gt, self.gc, self.outlier_repr, self.outlier_select, self.use_pow2,
                         self.kv_int8_scale, "i2")
@@ -389,7 +390,7 @@ class MultiSeqKVPool:
         """``append_step`` for a caller that holds nothing on the device yet: slots and positions go with the launch, which
         also fills ``block`` (int32 ``[7 B]``: slots, positions and lengths as int64, then packed lengths).  The largest
         packed length and the sum of all; ``None``, with nothing done, where ``append_step`` says False, and for more
-        than 64 requests."""
+        than ``step_rows`` requests."""
         w = self.window
         done = self._host.append_step(self.k_hist, self.v_hist, K, V, self._ring_sink, self._ring_rec, self.err_flag,
                                       self.seq_len, self.packed_groups, slots, seqs, w.sink_tokens + w.recent_window,

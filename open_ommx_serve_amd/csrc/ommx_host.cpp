@@ -1173,9 +1173,12 @@ PyObject* py_append_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const int64_t sink = as_int(a[4], ok), span = as_int(a[5], ok), kept = as_int(a[11], ok), gt = as_int(a[12], ok),
                   cap = a[13] == Py_None ? INT32_MAX : as_int(a[13], ok);
     std::vector<StepRow> step;
-    if (!ok || gt < 1 || !read_step(a[7], a[8], a[9], a[10], std::min<int64_t>(cap, INT32_MAX), step)) Py_RETURN_NONE;
+    // (a larger batch is refused before its lists are read: the caller's other way reads them)
+    if (!ok || gt < 1 || !PyList_CheckExact(a[9]) || PyList_GET_SIZE(a[9]) > ommx::kStepRows ||
+        !read_step(a[7], a[8], a[9], a[10], std::min<int64_t>(cap, INT32_MAX), step))
+        Py_RETURN_NONE;
     const int64_t B = static_cast<int64_t>(step.size());
-    if (B < 1 || B > ommx::kStepRows || !is_history(*kh, *vh) || k->dim() != 3 || k->sizes() != v->sizes()) Py_RETURN_NONE;
+    if (B < 1 || !is_history(*kh, *vh) || k->dim() != 3 || k->sizes() != v->sizes()) Py_RETURN_NONE;
     const c10::Device dev = kh->device();
     const int64_t N = kh->size(0), rows = kh->size(1), H = kh->size(2), D = kh->size(3);
     if (k->size(0) != B || k->size(1) != H || k->size(2) != D || k->scalar_type() != at::kBFloat16 ||
@@ -1253,5 +1256,7 @@ PyMODINIT_FUNC PyInit__ommx_host(void) {
     for (int i = 0; i < 11; ++i)
         if (!(g_names[i] = PyUnicode_InternFromString(names[i]))) return nullptr;
     if (!(g_bitmap = PyUnicode_InternFromString("bitmap"))) return nullptr;
-    return PyModule_Create(&module);
+    PyObject* m = PyModule_Create(&module);
+    if (m && PyModule_AddIntConstant(m, "STEP_ROWS", ommx::kStepRows) < 0) Py_CLEAR(m);
+    return m;
 }

@@ -269,6 +269,7 @@ def test_a_step_whose_places_go_with_the_launch(ring, B, D, view):
             K, V = both[:, :, 0], both[:, :, 1]
         seqs = [n + s for n in lens]
         got = pools[0].append_step_rows(slots, seqs, K, V, block if s % 2 else None)
+        assert pools[0].step_rows == 64
         if B > 64:
             assert got is None and pools[0].seq_len == pools[1].seq_len and bool((block == -1).all())
             return

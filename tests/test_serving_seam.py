@@ -338,6 +338,31 @@ def test_each_stream_has_its_own_block_and_tables_of_a_step(monkeypatch):
     assert len(m._stream_blocks) <= 8
 
 
+@pytest.mark.parametrize("B,route", [(64, ["rows", "rows"]), (65, ["upload", "step", "step"])])
+def test_a_batch_past_one_launch_is_not_offered_to_it(monkeypatch, B, route):
+    """Rows of up to 64 requests carry their places with the launch; a larger batch uploads them once and is appended by them
+    in every layer, without being walked for a launch that refuses it first."""
+    m, _ = _bmgr(num_seqs=B, graph=False)
+    calls = []
+
+    def rows(slots, seqs, key, value, block=None):
+        calls.append("rows")
+        if block is not None:
+            block.zero_()
+        return (200, 200 * B) if len(slots) <= 64 else None
+
+    pool = NS(k_hist=torch.empty(1), _req_to_token=torch.zeros(B, 10), _req_to_group=torch.zeros(B, 5), step_rows=64,
+              append_step_rows=rows, append_step=lambda *a: calls.append("step") or True)
+    seam = "open_ommx_serve_amd.integration.vllm.metadata."
+    monkeypatch.setattr(seam + "_current_stream", lambda index: 1)
+    monkeypatch.setattr(seam + "_hip.host", lambda: NS(upload=lambda block, *a: calls.append("upload") or block.zero_() is block))
+    m.on_build(_md([300] * B, range(11, 11 + B)))
+    assert len(m.slots) == B
+    for _ in range(2):                                            # two layers
+        assert m.append_step(pool, None, None)
+    assert calls == route
+
+
 @pytest.mark.parametrize("table,rows", [
     (torch.arange(12).view(4, 3), 3), (torch.arange(12, dtype=torch.int32).view(4, 3).flip(0), 4),
     (torch.arange(24).view(4, 6)[:, ::2], 2), (torch.arange(12).view(3, 4).t(), 4), (torch.arange(4).view(4, 1), 0),
