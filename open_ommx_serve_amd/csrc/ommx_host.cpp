@@ -1048,6 +1048,16 @@ PyObject* py_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Py_RETURN_TRUE;
 }
 
+// (starts, q heads, head_dim): the form of the kernel such prompts take, 0 to 2 in the order of ommx::PrefillForm.
+PyObject* py_prefill_form(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    bool ok = n == 3;
+    std::vector<int64_t> starts;
+    if (!ok || !read_ints(a[0], starts) || starts.size() < 2) { PyErr_SetString(PyExc_TypeError, "prefill_form: starts, heads and head_dim expected"); return nullptr; }
+    const int64_t Hq = as_int(a[1], ok), D = as_int(a[2], ok);
+    if (!ok) { PyErr_SetString(PyExc_ValueError, "prefill_form: integers expected"); return nullptr; }
+    return PyLong_FromLong(static_cast<long>(ommx::prefill_form(starts.data(), static_cast<int>(starts.size()) - 1, Hq, D)));
+}
+
 // (dst, values, n64 = all or none): a contiguous GPU tensor filled from a list of ints by a launch.  int64 and int32
 // tensors take one entry per value; an int32 tensor with n64 given holds n64 int64 values first, then int32 ones.
 PyObject* py_upload(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -1242,7 +1252,7 @@ PyMethodDef methods[] = {
     OMMX_FAST(auto_num_kv_splits), OMMX_FAST(plain), OMMX_FAST(rows_fit),
     OMMX_FAST(decode), OMMX_FAST(decode_pool), OMMX_FAST(store_pack), OMMX_FAST(pack_block), OMMX_FAST(block_errors), OMMX_FAST(pack_groups), OMMX_FAST(pack_prompts), OMMX_FAST(ring_write),
     OMMX_FAST(all_at), OMMX_FAST(append_rows), OMMX_FAST(append_step), OMMX_FAST(first_column),
-    OMMX_FAST(tail_gather), OMMX_FAST(rows_write), OMMX_FAST(upload), OMMX_FAST(prefill),
+    OMMX_FAST(tail_gather), OMMX_FAST(rows_write), OMMX_FAST(upload), OMMX_FAST(prefill), OMMX_FAST(prefill_form),
     {nullptr, nullptr, 0, nullptr},
 };
 #undef OMMX_FAST

@@ -174,6 +174,9 @@ int decode_combine(const float* attn_logits, int64_t al_b, int64_t al_h, int64_t
 // offsets, which bounds their row strides; a bit per tile of the longest request fits the kernel's LDS.
 constexpr int64_t kPrefillMaxStride = 1 << 24;
 constexpr int kPrefillMaxRows = 1 << 18;
+// The form of the kernel that a batch takes: a group of waves a workgroup, two that share the keys of its rows, two with rows each.
+enum class PrefillForm { one_group, split_keys, two_groups };
+PrefillForm prefill_form(const int64_t* host_starts, int B, int Hq, int D);
 int prefill_attention(const uint16_t* q, int64_t q_t, int64_t q_h, const uint16_t* k, int64_t k_t, int64_t k_h,
                       const uint16_t* v, int64_t v_t, int64_t v_h, void* o, bool o_bf16, int64_t o_t, int64_t o_h,
                       const int64_t* host_starts, int B, int Hq, int Hkv, int D, float scale, void* stream);

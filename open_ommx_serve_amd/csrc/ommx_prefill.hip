@@ -509,18 +509,48 @@ __global__ void __launch_bounds__(SPLIT ? 512 : 256 * GROUPS, 2) prefill_kernel(
         }
 }
 
-enum class Form { one_group, split_keys, two_groups };
 template <int D>
-void launch(const PrefillArgs& a, const TileList& list, int n, Form form, hipStream_t st) {
-    if (form == Form::two_groups)
+void launch(const PrefillArgs& a, const TileList& list, int n, PrefillForm form, hipStream_t st) {
+    if (form == PrefillForm::two_groups)
         hipLaunchKernelGGL((prefill_kernel<D, 2>), dim3(a.R % 2 ? a.Hkv * a.R : a.Hkv * a.R / 2, n), dim3(512), 0, st, a, list);
-    else if (form == Form::split_keys)
+    else if (form == PrefillForm::split_keys)
         hipLaunchKernelGGL((prefill_kernel<D, 1, true>), dim3(a.Hkv * a.R, n), dim3(512), 0, st, a, list);
     else
         hipLaunchKernelGGL((prefill_kernel<D, 1>), dim3(a.Hkv * a.R, n), dim3(256), 0, st, a, list);
 }
 
 }  // namespace
+
+// Two wave groups per workgroup pay when the tiles are long and fill the chip: they halve the vector work of staging
+// and overlap matrix and vector work, but a workgroup is twice as large and runs half a tile longer.  One group -> two
+// groups, us, 32 q / 8 kv heads: 4096 rows 246 -> 208, 2048 80.5 -> 79.3, 8 x 1024 141 -> 137; 1024 38.5 -> 42.1
+// (half the chip), 16 x 512 95 -> 126 (five key tiles a workgroup on average), 100 rows 9.8 -> 13.0.
+// One group a workgroup leaves compute units idle, or half empty, while the longest tiles are at their keys: then those are
+// split.  Kernel alone, one group -> split, us, 32 q / 8 kv heads: 100 rows 11.8 -> 13.4, 200 15.4 -> 15.5, 300 17.6 -> 16.9, 433 21.7 ->
+// 20.0, 622 29.7 -> 26.0, 1024 42.5 -> 36.3, head_dim 64 35.5 -> 30.6; 4000 rows of 8 heads 131.8 -> 99.7.
+// A compute unit holds one workgroup with its keys split, two of one group.  Two rounds of the former pay where what a compute
+// unit has to do in all, key_tiles * Hq / 256 tiles, is little beside the longest chain: 1100 rows (18 tiles, 11 a unit) 46.5 ->
+// 36.4, 1900 (30, 30) 73.1 -> 64.0, beside short prompts 1100 + 7 x 100 (13) 43.8 -> 41.4, 1100 + 600 (15) 44.5 -> 41.0, 1500 + 3 x 128 (24, 20)
+// 57.7 -> 53.3, 4000 + 30 x 100 of 8 heads 122.9 -> 89.6; equal prompts of 8 heads 6 x 1100 (16.9) 45.2 -> 44.3, 5 x 1500 (24, 24.4) 59.0 ->
+// 55.5, but 7 x 1030 (17, 19.5) 44.5 -> 47.6, head_dim 64 34.4 -> 40.6, 6 x 1200 (19, 20.4) 47.3 -> 48.9 and 38.0 -> 41.0; shorter chains 2 x 768 37.8 -> 38.8,
+// 3 x 512 29.6 -> 35.0, 8 x 256 24.8 -> 35.9.  The line lies where the two meet over 122 batches of 17 tiles and more, 4 to 32
+// heads (at head_dim 64 tiles are shorter beside what a workgroup does once): the other form would be better by 2.7 % for one of
+// them, by at most 1.4 % for the rest.
+PrefillForm prefill_form(const int64_t* host_starts, int B, int Hq, int D) {
+    int64_t groups = 0, key_tiles = 0, longest = 0;
+    for (int b = 0; b < B; ++b)
+        for (int64_t q0 = 0, len = host_starts[b + 1] - host_starts[b]; q0 < len; q0 += QROWS) {
+            const int64_t keys = (std::min<int64_t>(len, q0 + QROWS) + KEYS - 1) / KEYS;
+            ++groups;
+            key_tiles += keys;
+            longest = std::max(longest, keys);
+        }
+    const int64_t workgroups = groups * Hq;
+    if (workgroups >= 2 * 256 && key_tiles >= 8 * groups) return PrefillForm::two_groups;
+    if (workgroups <= 256) return longest >= 5 ? PrefillForm::split_keys : PrefillForm::one_group;
+    const bool two_rounds = workgroups <= 2 * 256 && longest > 16 && 2 * key_tiles * Hq <= 256 * (3 * longest - (D == 128 ? 18 : 20));
+    return two_rounds ? PrefillForm::split_keys : PrefillForm::one_group;
+}
 
 int prefill_attention(const uint16_t* q, int64_t q_t, int64_t q_h, const uint16_t* k, int64_t k_t, int64_t k_h,
                       const uint16_t* v, int64_t v_t, int64_t v_h, void* o, bool o_bf16, int64_t o_t, int64_t o_h,
@@ -544,25 +574,7 @@ int prefill_attention(const uint16_t* q, int64_t q_t, int64_t q_h, const uint16_
         const int64_t n = host_starts[b + 1] - host_starts[b];
         if (n > most) most = static_cast<int>(n);
     }
-    // Two wave groups per workgroup pay when the tiles are long and fill the chip: they halve the vector work of staging
-    // and overlap matrix and vector work, but a workgroup is twice as large and runs half a tile longer.  One group -> two
-    // groups, us, 32 q / 8 kv heads: 4096 rows 246 -> 208, 2048 80.5 -> 79.3, 8 x 1024 141 -> 137; 1024 38.5 -> 42.1
-    // (half the chip), 16 x 512 95 -> 126 (five key tiles a workgroup on average), 100 rows 9.8 -> 13.0.
-    int64_t groups = 0, key_tiles = 0;
-    for (int b = 0; b < B; ++b)
-        for (int64_t q0 = 0, len = host_starts[b + 1] - host_starts[b]; q0 < len; q0 += QROWS) {
-            ++groups;
-            key_tiles += (std::min(len, q0 + QROWS) + KEYS - 1) / KEYS;
-        }
-    const bool two_groups = groups * Hq >= 2 * 256 && key_tiles >= 8 * groups;
-    // One group a workgroup leaves compute units idle, or half empty, while the longest tiles are at their keys: then those are
-    // split.  Kernel alone, one group -> split, us, 32 q / 8 kv heads: 100 rows 11.8 -> 13.4, 200 15.4 -> 15.5, 300 17.6 -> 16.9, 433 21.7 ->
-    // 20.0, 622 29.7 -> 26.0, 1024 42.5 -> 36.3, head_dim 64 35.5 -> 30.6; 4000 rows of 8 heads 131.8 -> 99.7.  Two rounds of
-    // workgroups with their keys split pay where the tiles of the first are long: 1100 rows 49.3 -> 39.4, 1488 63.6 -> 52.9, 1900 82.9 -> 75.2,
-    // but 2 x 622 32.9 -> 32.2, 2 x 768 37.8 -> 38.8, 3 x 512 29.6 -> 35.0, 8 x 256 24.8 -> 35.9.
-    const int64_t workgroups = groups * Hq, longest = (most + KEYS - 1) / KEYS;
-    const bool split = !two_groups && ((workgroups <= 256 && longest >= 5) || (workgroups <= 512 && longest > 16));
-    const Form form = two_groups ? Form::two_groups : split ? Form::split_keys : Form::one_group;
+    const PrefillForm form = prefill_form(host_starts, B, Hq, D);
     TileList list;
     int n = 0;
     hipStream_t st = static_cast<hipStream_t>(stream);
@@ -571,7 +583,7 @@ int prefill_attention(const uint16_t* q, int64_t q_t, int64_t q_h, const uint16_
         if (D == 128) launch<128>(a, list, n, form, st); else launch<64>(a, list, n, form, st);
         n = 0;
     };
-    const int step = two_groups && a.R % 2 ? 2 * QROWS : QROWS;
+    const int step = form == PrefillForm::two_groups && a.R % 2 ? 2 * QROWS : QROWS;
     for (int q0 = (most - 1) / step * step; q0 >= 0; q0 -= step)
         for (int b = 0; b < B; ++b) {
             const int len = static_cast<int>(host_starts[b + 1] - host_starts[b]);

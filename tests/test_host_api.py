@@ -320,3 +320,20 @@ def test_table_id_clamp_arithmetic():
         got = lib.ommx_clamp_table_id(ident, extent, ctypes.byref(flag))
         assert (got, flag.value) == (want, bad), (ident, extent, got, flag.value)
         assert extent == 0 or 0 <= got < extent
+
+
+@pytest.mark.parametrize("lens,heads,D,form", [
+    ([100], 32, 128, 0), ([256], 32, 128, 0), ([257], 32, 128, 1), ([1024], 32, 128, 1), ([1024], 32, 64, 1),       # one round
+    ([1100], 32, 128, 1), ([1900], 32, 64, 1), ([8000], 8, 128, 1), ([1100] + [100] * 7, 32, 128, 1),                # two, of long tiles
+    ([1100, 600], 32, 64, 1), ([1500, 128, 128, 128], 32, 128, 1), ([4000] + [100] * 30, 8, 128, 1),
+    ([1100] * 6, 8, 64, 1), ([1500] * 5, 8, 128, 1), ([1030, 1030, 900], 16, 128, 1),
+    ([1030] * 7, 8, 128, 0), ([1030] * 7, 8, 64, 0), ([1100] * 7, 8, 128, 0), ([1200] * 3, 16, 128, 0), ([1030] * 14, 4, 128, 0),
+    ([1030, 1030, 900], 16, 64, 0), ([1030, 700], 32, 64, 0), ([768, 768], 32, 128, 0), ([512] * 3, 32, 128, 0),
+    ([2048], 32, 128, 2), ([4096], 32, 64, 2), ([1030, 896], 32, 128, 2), ([512] * 16, 32, 128, 0), ([100, 0, 0], 32, 128, 0)])
+def test_the_form_that_prompts_take(lens, heads, D, form):
+    """Keys split between two wave groups (1) where compute units would idle beside the longest chain of key tiles; not in
+    batches whose second round of workgroups is as long as their first (0), nor in those that fill the chip (2)."""
+    starts = [5]
+    for n in lens:
+        starts.append(starts[-1] + n)
+    assert _hip.host().prefill_form(starts, heads, D) == form

@@ -85,6 +85,27 @@ def test_long_prompts_in_two_wave_groups(D, hq, hkv, starts):
 
 
 @pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("hq,hkv,lens", [(32, 8, [1100] + [100] * 7), (16, 4, [1500, 300, 1, 300, 128]), (8, 1, [33, 4000, 100])])
+def test_a_long_prompt_beside_short_ones(D, hq, hkv, lens):
+    """More workgroups than compute units, the long prompt's first, keys split between two wave groups in all of them."""
+    starts = [2]
+    for n in lens:
+        starts.append(starts[-1] + n)
+    n = starts[-1] + 3
+    assert _hip.host().prefill_form(starts, hq, D) == 1 and sum(-(-x // 128) for x in lens) * hq > 256
+    q, k, v = _rows(n, hq, D, 1), _rows(n, hkv, D, 2), _rows(n, hkv, D, 3)
+    k[:, :, :3] *= 12
+    out = torch.full((n, hq, D), 7.0, device=DEV)
+    assert _hip.host().prefill(q, k, v, out, starts, D ** -0.5)
+    live = slice(starts[0], starts[-1])
+    for h in range(0, hq, hq // hkv):
+        heads, kv = slice(h, h + hq // hkv), slice(h // (hq // hkv), h // (hq // hkv) + 1)
+        want = _reference(q[:, heads], k[:, kv], v[:, kv], starts, D ** -0.5)
+        assert (out[live, heads].double() - want[live]).abs().max().item() <= 1e-5
+    assert bool((out[:starts[0]] == 7).all()) and bool((out[starts[-1]:] == 7).all())
+
+
+@pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("starts", [[0, 257], [0, 321], [3, 387, 388, 700], [0, 1, 64, 449]])
 @pytest.mark.parametrize("case", ["plain", "no f16", "weightless", "infinite"])
 def test_keys_split_between_two_wave_groups(D, starts, case):
