@@ -200,7 +200,7 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
             fast_done = true;
         }
         if (!fast_done) select_generic();
-        const uint32_t om = top | bot;
+        uint32_t om = top | bot;
         if (FAST6 && fast_done) {
             // NaN / Inf sort to the ends of the ordered keys: the largest and the smallest
             // chosen value tell whether the whole vector is finite
@@ -308,6 +308,10 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
             }
         } else {
             int slot = 0;
+            // (as a value of its own: the tests of the extremes above, kept for the ones here, are 32 masks of a wave, 64 scalar
+            // registers, which went to vector lanes and back 75 to 229 times.  Launches back to back, 8 heads, bf16 rows with three outliers: 1 K
+            // tokens 14.7 -> 13.65 us, 4 K 17.2 -> 16.4, 32 K 86.7 -> 83.1; fp32 rows 4 K 20.6 -> 17.4, 8 K at head_dim 64 20.4 -> 17.5)
+            asm("" : "+v"(om));
 #pragma unroll
             for (int i = 0; i < 32; ++i) {
                 s_codes[i * D + d] = static_cast<uint8_t>(int2_code(value(i) - zp, scale, inv_scale, inv_ok));
