@@ -275,6 +275,8 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
         };
         uint32_t nib = 0;
         bool mfin = true;
+        float thr[8];
+        fp4_boundaries(tab, thr);
         if (FAST6 && fast_done) {
             const float zc = -zp * inv_scale;
             if (inv_ok && fabsf(zc) < INFINITY) {      // one branch per vector, not one per element
@@ -292,11 +294,6 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
             }
             // |(w - mc) * ms| is largest at the extreme lanes, which are outliers: they decide
             // whether every mapped value is finite (codec.py:55-57 checks all of them)
-            float thr[8];      // the FP4 boundaries, the same for every thread: scalar registers
-#pragma unroll
-            for (int j2 = 1; j2 < 8; ++j2)
-                thr[j2] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(tab[256 + j2])));
-            thr[0] = 0.0f;
 #pragma unroll
             for (int r = 0; r < 6; ++r) {
                 const int key = r < 3 ? key_hi[r] : key_lo[r - 3];
@@ -304,13 +301,14 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
                 const float mapped = fp4_input(value_of_rank(key));
                 if (r % 3 == 0) mfin = mfin && is_finite_f32(mapped);
                 const int slot = __popc(om & ((1u << pos) - 1u));
-                nib |= fp4_encode_sorted(mapped, thr) << (4 * slot);
+                nib |= fp4_encode(mapped, thr) << (4 * slot);
             }
         } else {
             int slot = 0;
             // (as a value of its own: the tests of the extremes above, kept for the ones here, are 32 masks of a wave, 64 scalar
-            // registers, which went to vector lanes and back 75 to 229 times.  Launches back to back, 8 heads, bf16 rows with three outliers: 1 K
-            // tokens 14.7 -> 13.65 us, 4 K 17.2 -> 16.4, 32 K 86.7 -> 83.1; fp32 rows 4 K 20.6 -> 17.4, 8 K at head_dim 64 20.4 -> 17.5)
+            // registers, which went to vector lanes and back 75 to 229 times.  Launches back to back, 8 heads, without that and the
+            // boundaries in registers -> with both: bf16 rows with three outliers 1 K tokens 14.7 -> 11.8 us, 4 K 17.4 -> 14.6, 16 K
+            // 49.1 -> 41.2; magnitude selection 16 K 58.0 -> 50.8; fp32 rows with six outliers 4 K 21.3 -> 18.4, 16 K 61.3 -> 52.7)
             asm("" : "+v"(om));
 #pragma unroll
             for (int i = 0; i < 32; ++i) {
@@ -319,7 +317,7 @@ __global__ void __launch_bounds__(256, (FAST6 && IDXT == 0) ? 6 : 1) store_pack_
                     const float mapped = fp4_input(value(i));
                     mfin = mfin && is_finite_f32(mapped);
                     if ((om >> i) & 1u) {
-                        nib |= fp4_encode(mapped, tab + 256) << (4 * slot);
+                        nib |= fp4_encode(mapped, thr) << (4 * slot);
                         ++slot;
                     }
                 }

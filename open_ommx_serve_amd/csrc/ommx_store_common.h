@@ -139,18 +139,18 @@ __device__ __forceinline__ float exp2_int(int e) {   // exact 2^e, e in [-126,12
     return __uint_as_float(static_cast<uint32_t>(e + 127) << 23);
 }
 
-// FP4 code of m: sign bit and the number of magnitude thresholds fthr[1..7] (ascending) that |m| has
-// reached.
-__device__ __forceinline__ uint32_t fp4_encode(float m, const float* __restrict__ fthr) {
-    const float a = fabsf(m);
-    uint32_t idx = 0;
+// The magnitude thresholds t[1..7] of the FP4 codes (ascending), the same for every thread, in scalar registers: left to the
+// compiler they are read from memory again for every element of the general kernels, behind the copy of a row by vector loads.
+// Launches back to back, 8 heads, with seven compares of values read again -> this, and the masks kept apart: 16 x 16
+// vectors of four outliers 32 K tokens 111.6 -> 98.3 us, 64 x 32 of four 202 -> 166, 128 x 64 of eight 579 -> 538; small blocks of the
+// tuned form as well, whose reads now start before the codes: 500 tokens into a pool, whole call, 17.4 -> 15.5.
+__device__ __forceinline__ void fp4_boundaries(const float* __restrict__ tab, float (&t)[8]) {
+    t[0] = 0.0f;
 #pragma unroll
-    for (int j = 1; j <= 7; ++j) idx += (a >= fthr[j]) ? 1u : 0u;
-    return ((m < 0.0f) ? 8u : 0u) | idx;
+    for (int j = 1; j < 8; ++j) t[j] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(tab[256 + j])));
 }
-// The same with the seven thresholds in (scalar) registers t[1..7]: three compares down the sorted
-// thresholds instead of seven.
-__device__ __forceinline__ uint32_t fp4_encode_sorted(float m, const float (&t)[8]) {
+// FP4 code of m: sign bit and the number of thresholds that |m| has reached, by three compares down the sorted ones.
+__device__ __forceinline__ uint32_t fp4_encode(float m, const float (&t)[8]) {
     const float a = fabsf(m);
     const bool c4 = a >= t[4];
     const bool c2 = a >= (c4 ? t[6] : t[2]);

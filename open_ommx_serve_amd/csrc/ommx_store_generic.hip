@@ -130,6 +130,11 @@ __global__ void __launch_bounds__(256) store_generic_kernel(StoreArgs a) {
         uint64_t stream[2] = {0, 0};        // relidx7: position s at bits [7s, 7s+7)
         int slot = 0;
         bool mfin = true;
+        float thr[8];
+        fp4_boundaries(tab, thr);
+        // (as values of their own: the tests of the extremes above, kept for the ones here, are GT masks of a wave in scalar registers)
+#pragma unroll
+        for (int m = 0; m < MW; ++m) asm("" : "+v"(om[m]));
 #pragma unroll
         for (int i = 0; i < GT; ++i) {
             s_codes[i * D + d] = static_cast<uint8_t>(int2_code(w[i] - zp, st.scale, st.inv, st.inv_ok));
@@ -138,7 +143,7 @@ __global__ void __launch_bounds__(256) store_generic_kernel(StoreArgs a) {
                                              : (st.inv_ok ? (w[i] - zp) * st.inv : __fdiv_rn(w[i] - zp, st.scale));
                 mfin = mfin && is_finite_f32(mapped);
                 if (taken(om, i)) {
-                    nib |= static_cast<uint64_t>(fp4_encode(mapped, tab + 256)) << (4 * slot);
+                    nib |= static_cast<uint64_t>(fp4_encode(mapped, thr)) << (4 * slot);
                     const int bit = 7 * slot;
                     stream[bit >> 6] |= static_cast<uint64_t>(i) << (bit & 63);
                     if ((bit & 63) > 57) stream[1] |= static_cast<uint64_t>(i) >> (64 - (bit & 63));

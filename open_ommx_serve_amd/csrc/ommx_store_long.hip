@@ -278,10 +278,7 @@ __global__ void __launch_bounds__(512, GT < GC ? 1 : GT == 32 ? 8 : GT == 64 ? 7
         // largest at the extreme lanes, which are chosen ones, so these decide whether every mapped value is finite
         // (codec.py:55-57).
         float thr[8];
-#pragma unroll
-        for (int j = 1; j < 8; ++j)
-            thr[j] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(tab[256 + j])));
-        thr[0] = 0.0f;
+        fp4_boundaries(tab, thr);
         bool mfin = true;
         int slot[K];
 #pragma unroll
@@ -291,7 +288,7 @@ __global__ void __launch_bounds__(512, GT < GC ? 1 : GT == 32 ? 8 : GT == 64 ? 7
             const float wv = value_of_rank(key);
             const float mapped = own_map ? (wv - mc) * ms : (st.inv_ok ? (wv - zp) * st.inv : __fdiv_rn(wv - zp, st.scale));
             if (r % KH == 0) mfin = mfin && is_finite_f32(mapped);
-            slot[r] = pos << 5 | (r < KH ? 0 : 16) | static_cast<int>(fp4_encode_sorted(mapped, thr));
+            slot[r] = pos << 5 | (r < KH ? 0 : 16) | static_cast<int>(fp4_encode(mapped, thr));
         }
         sort_ascending(slot);
         if (picked != K) {          // positions taken from both ends (reported): each once, with its code from the lower end; then the last again
