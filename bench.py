@@ -39,7 +39,7 @@ HBM_PEAK_GBPS = 8000.0
 # HBM bytes per launch of the split-KV kernel at the default workload (ctx 65536, 256
 # splits), from rocprofv3 FETCH_SIZE + WRITE_SIZE scaled by a 256 MiB copy kernel
 # (profiles/decode_ctx64k_hbm_traffic.txt); counters cannot be read from inside this script.
-TRAFFIC_BYTES_CTX64K = 74.56e6
+TRAFFIC_BYTES_CTX64K = 74.00e6
 STAGE1_REP = 20
 STORE_REP = 8
 LAYERS = 32                  # decode steps (layers) per graph replay

@@ -10,8 +10,8 @@
 // a workgroup is 4 waves = 4 neighbouring kv heads.  Measured on MI355X this operator is bound
 // by how many instructions a SIMD can issue (vector ALU first, LDS second, a 16-byte LDS access
 // taking four issue slots), so the kernel is built for few instructions per token and to keep
-// THREE waves per SIMD resident (two with longer groups): at most 168 vector registers (one of those of the bitmap
-// forms lies in scratch memory and is read on the path of large steps alone), 13.4 KB of LDS per wave.  What that takes, against the kernel in ommx_decode.hip:
+// THREE waves per SIMD resident (two with longer groups or eight outlier slots): at most 168 vector registers, no scratch memory,
+// 13.4 KB of LDS per wave.  What that takes, against the kernel in ommx_decode.hip:
 //   * P.V runs transposed (rows = V channels, columns = q heads), the V step 2^e sits in the
 //     exponent field of the V operand, and the four column replicas of the q heads each take
 //     every fourth channel block, so the output accumulator is 8 registers instead of 32;
@@ -21,7 +21,7 @@
 //   * the V staging area of LDS is the K staging area of the same step, reused once QK is done.
 // With 8 q heads per kv head (NH = 8) the sixteen matrix rows / columns are two replicas of the
 // heads instead of four: a lane then keeps four heads of one token of either group, the output
-// takes four accumulators, and two workgroups fit a compute unit (190 registers, 14.1 KB of LDS
+// takes four accumulators, and two workgroups fit a compute unit (184 to 197 registers, 14.1 KB of LDS
 // per wave); everything up to the logits is the same code.
 // Arithmetic: exact 16-bit operands, fp32 accumulation, as in ommx_decode.hip.
 //   A (QK)   q * 2^(10-2m) as f16 in pair order, m = 2..4 (3 or 4 with longer groups) fixed per channel pair; this one operand

@@ -93,8 +93,9 @@ __device__ __forceinline__ bool store_place(const StoreArgs& a, StorePlace& p) {
 }
 
 // A workgroup each for K and V of a group and head?  Kernel alone, two against one, 8 heads: 5.9 against 6.5 us (1024 tokens), 6.8 / 8.1
-// (2 K), 7.6 / 9.6 (4 K), 11.8 / 13.9 (6 K), 13.7 / 14.3 (8 K), 23.3 / 24.0 (16 K), 23.4 / 22.1 (16 K tokens into a pool); fp32
-// rows 24.8 / 26.7 (4096).  Past the line the chip is full either way, and the second workgroup is only one more to start.
+// (2 K), 7.6 / 9.6 (4 K), 11.8 / 13.9 (6 K), 13.7 / 14.3 (8 K), 23.3 / 24.0 (16 K), 23.4 / 22.1 (16 K tokens into a pool); launches
+// back to back fp32 rows 14.2 / 15.2 (1 K), 18.3 / 18.3 (4 K), 28.8 / 29.3 (8 K).  Past the line the chip is full either way, and the
+// second workgroup is only one more to start.
 constexpr int kStoreApart = 2048;
 inline bool store_apart(const StoreArgs& a) { return a.groups * static_cast<int64_t>(a.H) <= kStoreApart; }
 inline dim3 store_grid(const StoreArgs& a, StoreOrder order) {

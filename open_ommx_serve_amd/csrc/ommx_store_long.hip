@@ -31,7 +31,8 @@
 namespace ommx {
 namespace {
 
-// Ascending order by a fixed network of compare-exchanges (12 for six, 29 for ten).
+// Ascending order by a fixed network of compare-exchanges: the smallest known ones, 12 for six and 29 for ten (Knuth, The Art of
+// Computer Programming, vol. 3, 5.3.4), in the layers that Bert Dobbelaere's list of sorting networks gives.
 __device__ __forceinline__ void in_order(int& a, int& b) {
     const int lo = min(a, b);
     b = max(a, b);
