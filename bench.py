@@ -13,12 +13,12 @@ capture fails), so K is rounded up to a multiple of 32 (``steps_requested`` /
 copy of the cache, query, tail and workspace, at its own addresses, as the layers of a model
 do: 32 x 69 MB at the headline context, far beyond the 256 MB last-level cache, so every
 step reads its planes from HBM.  Before anything is timed the outputs are filled with NaN,
-every layer is run once and compared with the CPU checker (``parity_before_timing``); a
+every layer is run once and compared with the oracle (``parity_before_timing``); a
 mismatch ends the run.  Prints ONE JSON line.  ``value`` is the p50 over the K timed steps
 at the headline context; ``roofline`` is the split-KV kernel alone (algorithmic bytes of the
 packed planes it must read over its average duration, against 8 TB/s); ``store`` is the
 quantize-on-store kernel over the same cache (its own roofline figures); ``cpu_baseline``
-is the CPU checker (dequantise-then-attend, torch on the host cores) timed on the same
+is the oracle (dequantise-then-attend, torch on the host cores) timed on the same
 workload for a bounded number of runs, and on the 1024-token configuration.
 """
 from __future__ import annotations
@@ -147,7 +147,7 @@ def _make_runner(cases, splits=None):
 
 
 def _parity_gate(case, outs, run_layer, want=None):
-    """NaN-fill the outputs, run every layer once, compare each with the CPU checker's result for
+    """NaN-fill the outputs, run every layer once, compare each with the oracle's result for
     the (shared) inputs.  Returns ``(figures, want)``; raises on a mismatch."""
     import torch
     for o, lse in outs:
@@ -208,7 +208,7 @@ def _pool_step(batch, ctx, q_heads, steps, warmup, splits=0):
     completed (one store launch, outside the timed replay), so the gather is told that the planes
     lag the sequence by one token.  Every request gets the same synthetic rows (the kernels do not
     care).  The outputs of the first replay whose token completes a group, and of the last replay,
-    are compared with the CPU checker.  Returns the JSON object."""
+    are compared with the oracle.  Returns the JSON object."""
     import torch
     from open_ommx_serve_amd.attention import MultiSeqKVPool, WindowSpec, gather_tails, write_tokens
     from open_ommx_serve_amd.attention.paged_decode import (auto_num_kv_splits, make_attn_logits,
@@ -263,7 +263,7 @@ def _pool_step(batch, ctx, q_heads, steps, warmup, splits=0):
     torch.cuda.current_stream().wait_stream(stream)
     d["seq_dev"].copy_(seq0)                      # capture ran no kernel
     def check(s):
-        """Replay s has run and the host has not packed yet: request 0 against the CPU checker."""
+        """Replay s has run and the host has not packed yet: request 0 against the oracle."""
         import oracle.ommx_oracle as O
         n = ctx + s + 1
         edge = win.boundary(n - 1)                 # what the planes hold

@@ -51,7 +51,7 @@ def synth_q(batch: int, q_heads: int, head_dim: int, seed: int):
 
 @dataclass
 class DecodeCase:
-    """All operands of one batched decode call, on ``device``, plus what a checker needs."""
+    """All operands of one batched decode call, on ``device``, plus what the oracle needs."""
     q: torch.Tensor
     planes: Dict[str, Any]
     k_tail: torch.Tensor

@@ -1,6 +1,6 @@
 """CPU restatement of the OMMX paged decode-attention path.  TEST INFRASTRUCTURE ONLY.
 
-This module is the checker the HIP kernels are compared against.  Nothing in the
+This module is the oracle that the HIP kernels are compared against.  Nothing in the
 shipped package may import it: only ``tests/``, ``__graft_entry__.smoke()`` and the
 ``cpu_baseline`` leg of ``bench.py`` do.  It runs on torch-CPU because the reference's
 own packer is torch-CPU code whose results depend on torch's fp32 ``log2`` / ``log`` /
