@@ -28,6 +28,7 @@ SOURCES = {
     "ommx_decode.hip": [],
     "ommx_decode_gqa4.hip": [],
     "ommx_decode_gqa4_tail.hip": [],
+    "ommx_decode_team.hip": [],
     "ommx_combine.hip": [],
     "ommx_ring.hip": [],
     "ommx_merge.hip": [],

@@ -15,6 +15,7 @@ void set_error(const char* msg) { g_error = msg; }
 int launch_decode_fast(const DecodeArgs& a, int D, int R, hipStream_t st);
 int launch_decode_gqa4(const DecodeArgs& a, int D, int R, const DecodeTail* tail, hipStream_t st);
 int launch_decode_gqa4_tail(const DecodeArgs& a, int D, int R, const DecodeTail* tail, hipStream_t st);
+int launch_decode_team(const DecodeArgs& a, int D, int R, const DecodeTail& tail, const TeamMerge& merge, hipStream_t st);
 
 }  // namespace ommx
 
@@ -109,7 +110,7 @@ static void set_error2(const char* where, const char* what) { g_error = std::str
 }  // namespace ommx
 
 int ommx::decode_splitkv(OMMX_DECODE_PARAMS, bool plain, const StateLse* lse, const Shares* shares, const DecodeTail* tail,
-                         bool* tail_done) {
+                         bool* tail_done, const TeamMerge* team) {
     if (tail_done) *tail_done = false;
     const char* where = plain ? "ommx_decode_splitkv_ref" : "ommx_decode_splitkv";
     if (const char* bad = check_decode(OMMX_DECODE_ARGS)) { set_error2(where, bad); return -1; }
@@ -128,7 +129,11 @@ int ommx::decode_splitkv(OMMX_DECODE_PARAMS, bool plain, const StateLse* lse, co
     const int R = Hq / Hkv;
     hipStream_t st = static_cast<hipStream_t>(stream);
     int rc = 1;
-    if (!plain) {
+    if (team) {
+        rc = tail && !plain ? launch_decode_team(a, D, R, *tail, *team, st) : 1;
+        if (rc == 1) return 1;
+        if (tail_done) *tail_done = true;
+    } else if (!plain) {
         rc = tail ? launch_decode_gqa4_tail(a, D, R, tail, st) : launch_decode_gqa4(a, D, R, nullptr, st);
         if (rc == 0 && tail_done) *tail_done = tail != nullptr;
         if (rc == 1) rc = launch_decode_fast(a, D, R, st);

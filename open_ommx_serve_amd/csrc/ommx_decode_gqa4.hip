@@ -39,6 +39,7 @@
 //   P.V      A = (1 + code/4 | 1 + code/16) * 2^e_v as f16 for 8 tokens of one channel (longer groups code/4), B = p (f16).
 #include <type_traits>
 
+#include "ommx_decode_recipe.h"
 #include "ommx_decode_shares.h"
 #include "ommx_decode_tail.h"
 #include "ommx_decode_util.h"
@@ -106,32 +107,12 @@ static_assert(resident(4, false) * lds_of(4 * LdsMap<4, false>::LDS_WAVE) <= 160
 static_assert(resident(4, true) * lds_of(4 * LdsMap<4, true>::LDS_WAVE) <= 160 * 1024, "4 heads, longer groups");
 static_assert(resident(8, true) * lds_of(4 * LdsMap<8, true>::LDS_WAVE) <= 160 * 1024, "8 heads");
 
-// One f16 carries 11 bits: rounding an outlier delta d costs up to |d| * 2^-11, i.e. up to
-// |d| * max|q| * 2^-11 * sm_scale on a logit.  A delta with |d| * max|q| >= BIG_DELTA * 16
-// (at most 1.4e-3 on a logit at sm_scale = 128^-0.5) gets its residual added exactly; smaller
-// ones stay below that and average a quarter of it.  The bound is held at other sm_scale values
-// (head_dim 64: 64^-0.5) by dividing the threshold by sm_scale / 128^-0.5; the general form, with
-// up to 8 entries per vector, takes three quarters of it, and half with fewer than 6 outlier slots (more
-// large values then stay in the base codes, the steps grow, and so do the entries).
-constexpr float BIG_DELTA = 2.0f;
-constexpr float BIG_DELTA_SM_SCALE = 0.08838834764831845f;
 // The running maximum of the online softmax is refreshed when a logit (base 2) exceeds it by this.  Under a maximum that lags,
 // the largest weight is no longer 1 but a number rounded to f16, and the lse takes over its rounding error (up to 2^-12).  Longer
 // groups are refreshed at once, as on the kernel that served them before: one split over 6001 tokens of 64 x 64 vectors, error of
 // the lse 3.5e-5 there, 1.07e-4 with a slack of 8 (rms), of the output 6.4e-5 and 8.1e-5 (2-norm).
 template <bool LONG>
 constexpr float MAX_SLACK = LONG ? 0.0f : 8.0f;
-// The base operand (1 + code*2^(2m-10)) * 2^e carries a constant A*2^e per channel, up to 2^6 times
-// the signal, which the bias MFMA takes out again: two large sums that cancel in fp32.  From steps
-// of 2^EXACT_STEP_EXP on (values a hundred or more wide inside one vector) that shows on the logits, and
-// the step's two groups take the operand code*2^(2m-10+e) instead (one packed subtraction more per operand
-// register, exact: both terms share the exponent) and drops the 2^e bias column.
-constexpr int EXACT_STEP_EXP = 5;
-// f16 operands: steps above 2^15 do not fit (K or V values beyond some 1e5); such a step is held at 2^15
-// and OMMX_ERR_VALUE_RANGE is reported
-constexpr int MAX_STEP_EXP = 15;
-// largest step whose 2^24-fold over the smallest A scale, 4, is an fp32 number
-constexpr int CODE_STEP_EXP = 105;
 // Longer groups were served before by a kernel with bf16 operands for K, which hold every step, and steps of V down to 2^-24.
 // They keep that range.  A wave that meets a step of K or V outside 2^-14..2^15 (normal f16 numbers) with a code that is not
 // zero, or a zero point of K from 2^18 on, or that has a query of 2^12 or more, drops what it has and walks its split in a
@@ -185,19 +166,6 @@ __device__ __forceinline__ uint32_t v_op(uint32_t m, uint32_t step) {
     const f16x2 one = {1.0f, 1.0f};
     return __builtin_bit_cast(uint32_t, (__builtin_bit_cast(f16x2, v_pair<Y, LONG>(m, 0x3C003C00u)) - one) * __builtin_bit_cast(f16x2, step));
 }
-// Outlier positions of a bitmap from below: the lowest set bit (-1 of an empty map, see LdsMap), and the map without the bit at
-// `pos`, one addition of -1 << pos (m & (m - 1) takes two instructions).
-__device__ __forceinline__ int lowest_bit(uint32_t m) {
-    int pos;
-    asm("v_ffbl_b32 %0, %1" : "=v"(pos) : "v"(m));
-    return pos;
-}
-__device__ __forceinline__ uint32_t without_bit(uint32_t m, int pos) {
-    uint32_t r;
-    asm("v_lshl_add_u32 %0, -1, %1, %2" : "=v"(r) : "v"(pos), "v"(m));
-    return r;
-}
-__device__ __forceinline__ float f16_bits(uint32_t b) { return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(b))); }
 __device__ __forceinline__ uint32_t pk_u16(uint32_t lo, uint32_t hi) { return (lo & 0xFFFFu) | (hi << 16); }
 
 // IDX: 0 = outlier positions from 32-bit bitmaps, 1 = from 7-bit position streams.

@@ -56,8 +56,10 @@ __device__ __forceinline__ uint32_t wave_cost(uint32_t g, bool third) {
 // The share `f` of the batch; false when the batch has fewer.  GT: tokens per group, PER_LANE: requests per lane
 // (B <= 64 * PER_LANE).  The launcher sees to shares >= shares_few >= B, so the search ends at the latest when g is
 // the longest request.
-template <int GT, int PER_LANE>
-__device__ __forceinline__ bool find_share(const DecodeArgs& a, uint32_t f, int lane, Share& out) {
+// OF_REQUEST: f is a request, of which only L and n are looked up.
+// (Args: DecodeArgs, or what else has its fields)
+template <int GT, int PER_LANE, bool OF_REQUEST = false, class Args>
+__device__ __forceinline__ bool find_share(const Args& a, uint32_t f, int lane, Share& out) {
     int len[PER_LANE];
     uint32_t G[PER_LANE], total = 0, top = 0;
 #pragma unroll
@@ -106,6 +108,14 @@ __device__ __forceinline__ bool find_share(const DecodeArgs& a, uint32_t f, int 
         const uint32_t g3 = smallest(a.shares, g0);
         if (wave_cost<GT>(g3, true) < wave_cost<GT>(g, false)) g = g3;
         else deal(g);
+    }
+    if constexpr (OF_REQUEST) {
+        static_assert(PER_LANE == 1, "one request a lane");
+        out.b = static_cast<int>(f);
+        out.n = __builtin_amdgcn_readlane(static_cast<int>(n[0]), f);
+        out.sp = 0;
+        out.L = __builtin_amdgcn_readlane(len[0], f);
+        return true;
     }
     if (f >= lane_top(incl[PER_LANE - 1])) return false;
 #pragma unroll

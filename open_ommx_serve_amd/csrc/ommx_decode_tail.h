@@ -49,9 +49,27 @@ __device__ __forceinline__ float fold16(float x, float y) {
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// RT: q head slots (4 or 8; slots from R on repeat the last head and are not written).  LDS: 32 * RT + 2 * RT floats.
-template <int RT, int D>
-__device__ __forceinline__ void attend_part(const DecodeArgs& a, uint8_t* sm, int b, int kvh, int R, int part, int lane) {
+// A store that other workgroups of the same launch may read: it goes past this die's cache.
+template <bool SHARED>
+__device__ __forceinline__ void put2(float* p, float x, float y) {
+    if constexpr (SHARED) {
+        const uint64_t v = static_cast<uint64_t>(__float_as_uint(y)) << 32 | __float_as_uint(x);
+        __hip_atomic_store(reinterpret_cast<uint64_t*>(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } else {
+        *reinterpret_cast<f32x2*>(p) = f32x2{x, y};
+    }
+}
+template <bool SHARED>
+__device__ __forceinline__ void put1(float* p, float x) {
+    if constexpr (SHARED) __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else *p = x;
+}
+
+// RT: q head slots (4 or 8; slots from R on repeat the last head and are not written).  LDS: 32 * RT + 2 * RT floats.  SHARED: the states are
+// read by another workgroup of this launch.
+// (Args: DecodeArgs, or what else has its fields)
+template <int RT, int D, bool SHARED = false, class Args>
+__device__ __forceinline__ void attend_part(const Args& a, uint8_t* sm, int b, int kvh, int R, int part, int lane) {
     constexpr int CHUNK = 32;                      // rows per pass: two blocks of 16
     constexpr int KS = D / 32;                     // k-steps of a logit
     constexpr int LPR = D / 8;                     // lanes that read a V row
@@ -78,7 +96,7 @@ __device__ __forceinline__ void attend_part(const DecodeArgs& a, uint8_t* sm, in
     typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
     u32x4 aq[KS];
     {
-        const uint16_t* qp = a.q + b * a.q_sb + (int64_t)(qh0 + min(j & (RT - 1), R - 1)) * a.q_sh + 8 * kq;
+        const uint16_t* qp = a.q + (int64_t)b * a.q_sb + (int64_t)(qh0 + min(j & (RT - 1), R - 1)) * a.q_sh + 8 * kq;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) aq[ks] = *reinterpret_cast<const u32x4_a4*>(qp + 32 * ks);
     }
@@ -167,15 +185,15 @@ __device__ __forceinline__ void attend_part(const DecodeArgs& a, uint8_t* sm, in
         decode_util::lds_fence();
     }
     // ---- the state: sums over the lanes, normalised ----------------------------------------------
-    float* const al = a.al + b * a.al_b + (int64_t)qh0 * a.al_h + (int64_t)(part - kTailParts) * a.al_s;
-    float* const sl = a.sl + b * a.sl_b + (int64_t)qh0 * a.sl_h + (int64_t)(part - kTailParts) * a.sl_s;
+    float* const al = a.al + (int64_t)b * a.al_b + (int64_t)qh0 * a.al_h + (int64_t)(part - kTailParts) * a.al_s;
+    float* const sl = a.sl + (int64_t)b * a.sl_b + (int64_t)qh0 * a.sl_h + (int64_t)(part - kTailParts) * a.sl_s;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const float l = row16_sum(l_run[r]);
         const int h = 4 * kq + r;
         if (j == 0 && kq < RT / 4) {
             s_l[h] = l;
-            if (h < R) sl[h * a.sl_h] = l > 0.0f ? m_run[r] + __logf(l) : -INFINITY;
+            if (h < R) put1<SHARED>(sl + h * a.sl_h, l > 0.0f ? m_run[r] + __logf(l) : -INFINITY);
         }
     }
     if (lo >= hi) return;                           // (nothing attended: the lse says so, the state is not read)
@@ -196,8 +214,13 @@ __device__ __forceinline__ void attend_part(const DecodeArgs& a, uint8_t* sm, in
             float* dst = al + h * a.al_h + 8 * c8;
 #pragma unroll
             for (int e = 0; e < 8; ++e) o[e] *= inv;
-            *reinterpret_cast<f32x4*>(dst) = f32x4{o[0], o[1], o[2], o[3]};
-            *reinterpret_cast<f32x4*>(dst + 4) = f32x4{o[4], o[5], o[6], o[7]};
+            if constexpr (SHARED) {
+#pragma unroll
+                for (int e = 0; e < 8; e += 2) put2<true>(dst + e, o[e], o[e + 1]);
+            } else {
+                *reinterpret_cast<f32x4*>(dst) = f32x4{o[0], o[1], o[2], o[3]};
+                *reinterpret_cast<f32x4*>(dst + 4) = f32x4{o[4], o[5], o[6], o[7]};
+            }
         }
     }
 }

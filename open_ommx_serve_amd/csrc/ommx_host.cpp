@@ -378,15 +378,96 @@ int run_decode(const DecodeCall& c) {
         c.bitmap ? OMMX_INDEX_BITMAP : OMMX_INDEX_RELIDX7, scale_bf16, gt, gc, v_bf16, SPLITS, c.sm_scale, c.cap, c.off, \
         c.gbase, pages, slots, data<int32_t>(c.err), stream
 
+    // (max_seq bounds how many units there can be; were it too small, the shares would be longer, nothing else)
+    const int64_t longest = std::max<int64_t>(1, (c.max_seq + unit - 1) / unit);
     int rc = 1, rc2 = 0;
-    if (c.splits == 0 && !c.ws && !c.force && B > 1) {
+    const int64_t front = tail_rows ? ommx::kTailParts : 0;
+    // the merge inside the launch: its words lie behind the `used` bytes of the scratch, on a line of their own
+    const size_t words = static_cast<size_t>(B * wave_heads + 1) * 64;
+    auto team_merge = [&](void* scratch, int64_t used, float* lse, int64_t per, bool fused) {
+        static std::atomic<uint64_t> calls{ommx::kFirstCall};
+        ommx::TeamMerge m{static_cast<int>(std::min<int64_t>(rt.size(1), INT32_MAX)), static_cast<int>(std::min<int64_t>(rg.size(1), INT32_MAX)),
+                          static_cast<int>(per)};
+        if (!fused) return m;
+        (o_bf16 ? reinterpret_cast<void*&>(m.o16) : reinterpret_cast<void*&>(m.o)) = data(c.o);
+        m.o_b = c.o->stride(0); m.o_h = c.o->stride(1);
+        m.lse = lse; m.lse_b = c.lse ? c.lse->stride(0) : Hq;
+        m.arrivals = reinterpret_cast<unsigned long long*>((reinterpret_cast<uintptr_t>(scratch) + used + 63) / 64 * 64);
+        m.number = calls.fetch_add(1, std::memory_order_relaxed);
+        return m;
+    };
+    // the work in equal shares, at most `most` of them for one request
+    auto dealt_out = [&](int64_t shares, int64_t few, int64_t singles, int64_t most, bool team, bool fused) {
+        const int64_t row = most + front, n = B * Hq * row;
+        c10::DataPtr scratch = allocator->allocate(static_cast<size_t>(n * (D + 1) + B * Hq + B) * sizeof(float) + words);
+        float *al = static_cast<float*>(scratch.get()), *lse = c.lse ? data<float>(c.lse) : al + n * (D + 1);
+        const ommx::StateLse states{al + n * D + front, Hq * row, row, 1};
+        const ommx::Shares dealt{static_cast<int>(shares), static_cast<int>(few), static_cast<int>(singles),
+                                 static_cast<int>((std::min(shares, B * longest > singles ? B * longest / 2 : shares) + B - 1) / B),
+                                 reinterpret_cast<int32_t*>(al + n * (D + 1) + B * Hq)};
+        al += front * D;
+        const ommx::TeamMerge tm = team_merge(scratch.get(), (n * (D + 1) + B * Hq + B) * 4, lse, 0, fused);
+        Py_BEGIN_ALLOW_THREADS
+        rc = ommx::decode_splitkv(OMMX_SPLITKV_ARGS(al, Hq * row * D, row * D, D, most), false, &states, &dealt,
+                                  tail_rows ? &tl : nullptr, &tail_done, team ? &tm : nullptr);
+        if (rc == 0 && !fused) rc2 = merge(al, Hq * row * D, row * D, D, lse, most, states, &dealt);
+        Py_END_ALLOW_THREADS
+    };
+    // S splits of every request
+    auto split_up = [&](int64_t S, bool team, int64_t per, bool fused) {
+        const int64_t row = S + front, n = B * Hq * row;
+        int64_t al_b = Hq * row * D, al_h = row * D, al_s = D;
+        c10::DataPtr scratch;
+        float *al, *lse = data<float>(c.lse);
+        ommx::StateLse states;
+        if (c.ws && c.lse) {
+            al = c.ws->data_ptr<float>();
+            al_b = c.ws->stride(0); al_h = c.ws->stride(1); al_s = c.ws->stride(2);
+            states = {al + D, al_b, al_h, al_s};
+        } else {
+            scratch = allocator->allocate(static_cast<size_t>(n * (D + 1) + B * Hq) * sizeof(float) + words);
+            al = static_cast<float*>(scratch.get());
+            states = {al + n * D + front, Hq * row, row, 1};
+            if (!lse) lse = al + n * (D + 1);
+            al += front * D;
+        }
+        const ommx::TeamMerge tm = team_merge(scratch.get(), (n * (D + 1) + B * Hq) * 4, lse, per, fused);
+        Py_BEGIN_ALLOW_THREADS
+        rc = ommx::decode_splitkv(OMMX_SPLITKV_ARGS(al, al_b, al_h, al_s, S), c.force, &states, nullptr,
+                                  tail_rows ? &tl : nullptr, &tail_done, team ? &tm : nullptr);
+        if (rc == 0 && !fused) rc2 = merge(al, al_b, al_h, al_s, lse, S, states, nullptr);
+        Py_END_ALLOW_THREADS
+    };
+    // Short calls: four waves on one kv head of one split (csrc/ommx_decode_team.hip), in 64-token steps, while there are few of
+    // those for a compute unit (counted by the longest request).  From there on that kernel's quarter more instructions count: 8 K tokens
+    // of 8 kv heads 14.0 us against 14.3, 12 K 17.6 against 15.8; 8 K with 64 q heads 16.6 / 19.8, 16 K 22.8 / 21.3; with 64 channels, whose
+    // heads it does not read in pairs of which one is zero, 16 K 13.6 / 18.0, 2 x 12 K (six steps) 15.7 / 17.8; with one kv head, where a
+    // workgroup of the other kernel is a single wave, 16 of 1 to 16 K (16 steps) 20.3 / 22.2, but 8 of 20 to 32 K 24.0 / 23.2.
+    if (c.splits == 0 && tail_rows && plain_planes && k == 6 && B <= 64 && (D == 128 || paired)) {
+        const int64_t cus = cu_count(dev.index()), steps = (longest + 1) / 2, all = B * steps * wave_heads;
+        if (all <= cus * (paired || wave_heads == 1 ? 8 : 4)) {
+            // The merge inside the launch while its one workgroup has little to read, instead of a launch of its own (3.5 us of host
+            // time; 1 K tokens 8.5 us against 9.1 to 10).  Not under capture: see TeamMerge.
+            hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+            const bool eager = hipStreamIsCapturing(stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone;
+            auto merged = [&](int64_t states) { return eager && states <= ommx::kTeamMerged && states * (Hq / wave_heads) * D <= ommx::kTeamMerged * 512; };
+            // one request: up to three workgroups a compute unit (two with 8 heads); several: two, or a split a step where all of those fit
+            const int64_t room = std::clamp<int64_t>((B == 1 && R <= 4 ? 3 : 2) * cus / wave_heads, 1, 508);
+            if (B == 1 || B * steps <= room) {
+                const int64_t each = (steps + room - 1) / room, S = (steps + each - 1) / each;
+                split_up(S, true, 2 * each, merged(S));
+            } else if (B <= room) {
+                const int64_t most = std::min<int64_t>({508, steps, std::max<int64_t>(8, 4 * room / B)});
+                dealt_out(room, room, 0, most, true, merged(most));
+            }
+        }
+    }
+    if (rc == 1 && c.splits == 0 && !c.ws && !c.force && B > 1) {
         // Several requests and nobody asked for a split count: the kernels deal the groups out in equal shares, as many
         // as are resident at once (a wave per kv head and share).  One request gets at most 256 of them (its states
         // are merged on chip), 64 with many (request, head) pairs, where the combine's small form serves, and no
         // more than four times its even part, which bounds the workspace.
         const int64_t fit = cu_count(dev.index()) * 4 / wave_heads;
-        // (max_seq bounds how many groups there can be; were it too small, the shares would be longer, nothing else)
-        const int64_t longest = std::max<int64_t>(1, (c.max_seq + unit - 1) / unit);
         const int64_t shares = std::min({int64_t{2048}, fit * (lean ? 3 : 2), B * longest});
         const int64_t few = std::min(shares, fit * 2);
         const int64_t most = std::min({int64_t{B * Hq >= 256 ? 64 : (shares > 256 * B && longest > 512 ? 512 : 256)}, longest,
@@ -394,22 +475,7 @@ int run_decode(const DecodeCall& c) {
         // A batch that cannot have more groups than SIMDs is left to fixed splits of one group: those need not find their
         // share (0.3 us).  From there on a split per group of the longest request would put two workgroups on some
         // compute units, empty ones among them: 8 requests of 97 to 701 tokens 9.9 us as 23 splits each, 8.5 dealt out.
-        if (few >= B && B * longest > fit) {
-            const int64_t singles = paired ? 2 * fit : fit;
-            const int64_t front = tail_rows ? ommx::kTailParts : 0, row = most + front, n = B * Hq * row;
-            c10::DataPtr scratch = allocator->allocate(static_cast<size_t>(n * (D + 1) + B * Hq + B) * sizeof(float));
-            float *al = static_cast<float*>(scratch.get()), *lse = c.lse ? data<float>(c.lse) : al + n * (D + 1);
-            const ommx::StateLse states{al + n * D + front, Hq * row, row, 1};
-            const ommx::Shares dealt{static_cast<int>(shares), static_cast<int>(few), static_cast<int>(singles),
-                                     static_cast<int>((std::min(shares, B * longest > singles ? B * longest / 2 : shares) + B - 1) / B),
-                                     reinterpret_cast<int32_t*>(al + n * (D + 1) + B * Hq)};
-            al += front * D;
-            Py_BEGIN_ALLOW_THREADS
-            rc = ommx::decode_splitkv(OMMX_SPLITKV_ARGS(al, Hq * row * D, row * D, D, most), false, &states, &dealt,
-                                      tail_rows ? &tl : nullptr, &tail_done);
-            if (rc == 0) rc2 = merge(al, Hq * row * D, row * D, D, lse, most, states, &dealt);
-            Py_END_ALLOW_THREADS
-        }
+        if (few >= B && B * longest > fit) dealt_out(shares, few, paired ? 2 * fit : fit, most, false, false);
     }
     if (rc == 1) {
         int64_t S = c.splits;
@@ -423,27 +489,7 @@ int run_decode(const DecodeCall& c) {
         if (c.ws && (c.ws->scalar_type() != at::kFloat || c.ws->dim() != 4 || c.ws->size(0) != B || c.ws->size(1) != Hq ||
                      c.ws->size(2) < S || c.ws->size(3) < D + 1 || c.ws->stride(3) != 1))
             return 0;
-        const int64_t front = tail_rows ? ommx::kTailParts : 0, row = S + front, n = B * Hq * row;
-        int64_t al_b = Hq * row * D, al_h = row * D, al_s = D;
-        c10::DataPtr scratch;
-        float *al, *lse = data<float>(c.lse);
-        ommx::StateLse states;
-        if (c.ws && c.lse) {
-            al = c.ws->data_ptr<float>();
-            al_b = c.ws->stride(0); al_h = c.ws->stride(1); al_s = c.ws->stride(2);
-            states = {al + D, al_b, al_h, al_s};
-        } else {
-            scratch = allocator->allocate(static_cast<size_t>(n * (D + 1) + B * Hq) * sizeof(float));
-            al = static_cast<float*>(scratch.get());
-            states = {al + n * D + front, Hq * row, row, 1};
-            if (!lse) lse = al + n * (D + 1);
-            al += front * D;
-        }
-        Py_BEGIN_ALLOW_THREADS
-        rc = ommx::decode_splitkv(OMMX_SPLITKV_ARGS(al, al_b, al_h, al_s, S), c.force, &states, nullptr,
-                                  tail_rows ? &tl : nullptr, &tail_done);
-        if (rc == 0) rc2 = merge(al, al_b, al_h, al_s, lse, S, states, nullptr);
-        Py_END_ALLOW_THREADS
+        split_up(S, false, 0, false);
     }
 #undef OMMX_SPLITKV_ARGS
     if (failed(rc, "ommx_decode_splitkv") || failed(rc2, "ommx_decode_combine")) return -1;

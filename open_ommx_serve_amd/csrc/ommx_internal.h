@@ -142,8 +142,24 @@ int fold_states(const float* al, int64_t al_b, int64_t al_h, int64_t al_s, const
                 void* o, bool o_bf16, int64_t o_b, int64_t o_h, float* lse, int64_t lse_b, int B, int Hq, int D,
                 void* stream);
 
+// What the kernel for short calls (csrc/ommx_decode_team.hip) is told beyond the common arguments: entries of a row of either table,
+// 32-token groups of a split (fixed splits), and the merge, when the launch does it itself (up to kTeamMerged splits or shares of a
+// request): `arrivals`, a word every 64 bytes for each (request, kv head or pair of 64-channel ones), memory that only this call uses,
+// whatever it holds; `number` of this call, from kFirstCall on and below 2^56, no two the same (so not in a launch that is replayed).
+constexpr uint64_t kFirstCall = 0xFF000000000000ull;
+constexpr int kTeamMerged = 32;
+struct TeamMerge {
+    int rt_n, rg_n, per_split;
+    float* o; uint16_t* o16;        // one of them
+    int64_t o_b, o_h;
+    float* lse; int64_t lse_b;
+    unsigned long long* arrivals;   // NULL: states only
+    uint64_t number;
+};
+
 // ommx_decode_splitkv / _ref (plain) with these choices (each may be NULL).  Returns 1, with nothing done, when shares
-// are asked for and no kernel with shares serves the call.  *tail_done tells whether the launch attends the tail.
+// are asked for and no kernel with shares serves the call.  *tail_done tells whether the launch attends the tail.  team: by the
+// kernel for short calls (csrc/ommx_decode_team.hip), which needs a tail; returns 1, with nothing done, for what it does not serve.
 #define OMMX_DECODE_DECL                                                                            \
     const uint16_t* q, int64_t q_stride_b, int64_t q_stride_h, const uint8_t* k_base,               \
     const void* k_scale, const uint16_t* k_zp, const uint16_t* k_ms, const uint16_t* k_mc,          \
@@ -156,7 +172,7 @@ int fold_states(const float* al, int64_t al_b, int64_t al_h, int64_t al_s, const
     int packed_start_offset, int seg_group_base, int num_pages, int num_group_slots,                \
     int32_t* err_flag, void* stream
 int decode_splitkv(OMMX_DECODE_DECL, bool plain, const StateLse* lse, const Shares* shares, const DecodeTail* tail,
-                   bool* tail_done);
+                   bool* tail_done, const TeamMerge* team = nullptr);
 #undef OMMX_DECODE_DECL
 
 // ommx_decode_combine with the lse of the states elsewhere (NULL: column D) and the shares they come from (NULL:

@@ -1,0 +1,135 @@
+"""Short decode calls, served by four waves on one kv head of one split (csrc/ommx_decode_team.hip), with their merge inside the
+launch or as one of its own: edges of groups, steps, shares and states, against the oracle; the same call again, from a graph and
+beside others on its own bits."""
+import pytest
+import torch
+
+import oracle.ommx_oracle as O
+from open_ommx_serve_amd.attention import _hip
+from open_ommx_serve_amd.attention.paged_decode import ommx_paged_decode_attention_canonical
+from open_ommx_serve_amd.synth import build_decode_case
+
+pytestmark = pytest.mark.gpu
+
+
+def _outputs(case):
+    B, Hq, D = case.q.shape
+    return (torch.full((B, Hq, D), float("nan"), dtype=torch.float32, device=case.q.device),
+            torch.full((B, Hq), float("nan"), dtype=torch.float32, device=case.q.device))
+
+
+def _run(case, **over):
+    o, lse = _outputs(case)
+    ommx_paged_decode_attention_canonical(*case.decode_args(o, lse), **{**case.decode_kwargs(), **over})
+    return o.cpu(), lse.cpu()
+
+
+def _oracle(case):
+    planes = {k: (v.cpu() if torch.is_tensor(v) else v) for k, v in case.planes.items()}
+    return O.decode_reference(case.q.cpu(), planes | {"outliers_per_vector": case.outliers_per_vector},
+                              case.k_tail.cpu(), case.v_tail.cpu(), case.b_tail_len.tolist(), case.req_to_token.cpu(),
+                              case.req_to_group.cpu(), case.b_seq_len.tolist(), sm_scale=case.sm_scale,
+                              page_size=case.page_size)
+
+
+def _close(got, want, what):
+    # the bounds of every decode test: f16 rounding of weights and outlier entries, fp32 sums
+    (o, lse), (wo, wl) = got, want
+    assert torch.isfinite(o).all(), what
+    err = (o.double() - wo.double()).abs()
+    assert err.max().item() <= 2e-3 and err.mean().item() <= 2e-4, (what, err.max().item())
+    fin = torch.isfinite(wl)
+    assert torch.equal(torch.isfinite(lse), fin), what
+    assert (lse.double()[fin] - wl.double()[fin]).abs().max().item() <= 2e-3, what
+
+
+SHAPES = [(32, 8, 128, {}), (64, 8, 128, {}), (8, 1, 128, dict(outlier_repr="relidx7")), (16, 8, 128, dict(outlier_repr="relidx7")),
+          (4, 4, 128, {}), (32, 8, 64, {}), (4, 2, 64, {}), (32, 8, 128, dict(kv_outlier_map=False)),
+          (64, 8, 128, dict(kv_outlier_map=False, outlier_repr="relidx7")), (8, 8, 64, dict(kv_outlier_map=False))]
+
+
+@pytest.mark.parametrize("hq,hkv,D,kw", SHAPES)
+@pytest.mark.parametrize("lens", [[7], [72], [104], [105], [136], [167], [2072], [4136], [9, 72, 100], [72, 9, 136, 700, 40],
+                                  [40 + 33 * i for i in range(17)], [72] * 63 + [1]], ids=lambda l: f"{len(l)}x{max(l)}")
+def test_edges_of_groups_and_shares(hq, hkv, D, kw, lens):
+    """No packed token, one group, a step of one and of two groups, 32 steps and more; requests without any beside others."""
+    case = build_decode_case(lens, q_heads=hq, kv_heads=hkv, head_dim=D, seed=len(lens) + max(lens), permute_tables=True,
+                             sparse_frac=0.005, **kw)
+    want = _oracle(case)
+    _close(_run(case), want, "as told")
+    _close(_run(case, max_seq_len=int(case.b_seq_len.max()) + 1000), want, "longer than it is")
+    # a hint that says too little: splits take more groups each
+    _close(_run(case, max_seq_len=64), want, "shorter than it is")
+
+
+def test_tables_are_not_read_past_their_rows():
+    """The hint says more groups than the tables have entries: what lies behind a row is another request's, or nobody's."""
+    case = build_decode_case([700, 135], seed=3, permute_tables=True)
+    err = torch.zeros(1, dtype=torch.int32, device=case.q.device)
+    _close(_run(case, max_seq_len=3000, err_flag=err), _oracle(case), "")
+    one = build_decode_case([700], seed=3, permute_tables=True)
+    _close(_run(one, max_seq_len=2000, err_flag=err), _oracle(one), "")
+    assert int(err.item()) == 0
+
+
+@pytest.mark.parametrize("hq,hkv,D", [(32, 8, 128), (64, 8, 128), (32, 8, 64)])
+def test_the_same_bits_again_in_memory_of_other_calls(hq, hkv, D):
+    """The merge counts in scratch that holds whatever calls before left there, of this shape or another; bits stay."""
+    cases = [build_decode_case(l, q_heads=hq, kv_heads=hkv, head_dim=D, seed=5, permute_tables=True, sparse_frac=0.005)
+             for l in ([1000], [300, 90, 500], [72], [9], [100 + 40 * i for i in range(8)])]
+    first = [_run(c) for c in cases]
+    for c, f in zip(cases, first):
+        _close(f, _oracle(c), "")
+    for turn in range(30):
+        junk = torch.full((1 << 20,), [0, -1, 0x7F][turn % 3], dtype=torch.int8, device="cuda")
+        del junk
+        for i in ((turn * 7 + k) % len(cases) for k in range(len(cases))):
+            o, lse = _run(cases[i])
+            assert torch.equal(o, first[i][0]) and torch.equal(lse, first[i][1]), (turn, i)
+
+
+def test_captured_calls_replay_like_eager_ones():
+    """Under capture the merge is a launch of its own: the same states in another order of sums (fp32 rounding)."""
+    cases = [build_decode_case(l, seed=6, permute_tables=True, sparse_frac=0.005) for l in ([1000], [300, 90, 500])]
+    eager = [_run(c) for c in cases]
+    outs = [_outputs(c) for c in cases]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for c, (o, lse) in zip(cases, outs):
+            ommx_paged_decode_attention_canonical(*c.decode_args(o, lse), **c.decode_kwargs())
+    for turn in range(4):
+        for o, lse in outs:
+            o.fill_(float("nan"))
+            lse.fill_(float("nan"))
+        graph.replay()
+        again = [_run(c) for c in cases]                     # eager work between the replays
+        for (o, lse), (wo, wl), a in zip(outs, eager, again):
+            assert (o.cpu() - wo).abs().max().item() <= 2e-6 * max(1.0, wo.abs().max().item()), turn
+            assert (lse.cpu() - wl).abs().max().item() <= 1e-5
+            assert torch.equal(a[0], wo)
+
+
+def test_two_streams_at_once():
+    """Calls under way together have scratch of their own."""
+    cases = [build_decode_case(l, seed=8, permute_tables=True) for l in ([1000], [400, 90, 600])]
+    want = [_run(c) for c in cases]
+    streams = [torch.cuda.Stream() for _ in cases]
+    outs = [[_outputs(c) for _ in range(25)] for c in cases]
+    torch.cuda.synchronize()
+    for i in range(25):
+        for c, s, os in zip(cases, streams, outs):
+            with torch.cuda.stream(s):
+                ommx_paged_decode_attention_canonical(*c.decode_args(*os[i]), **c.decode_kwargs())
+    torch.cuda.synchronize()
+    for os, (wo, wl) in zip(outs, want):
+        for o, lse in os:
+            assert torch.equal(o.cpu(), wo) and torch.equal(lse.cpu(), wl)
+
+
+def test_an_id_outside_its_plane_is_reported():
+    case = build_decode_case([700], seed=9, permute_tables=True)
+    err = torch.zeros(1, dtype=torch.int32, device=case.q.device)
+    case.req_to_group[0, 5] = 1 << 20
+    _run(case, err_flag=err)
+    torch.cuda.synchronize()
+    assert int(err.item()) == _hip.ERR_TABLE_RANGE
