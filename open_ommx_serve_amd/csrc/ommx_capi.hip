@@ -15,7 +15,7 @@ void set_error(const char* msg) { g_error = msg; }
 int launch_decode_fast(const DecodeArgs& a, int D, int R, hipStream_t st);
 int launch_decode_gqa4(const DecodeArgs& a, int D, int R, const DecodeTail* tail, hipStream_t st);
 int launch_decode_gqa4_tail(const DecodeArgs& a, int D, int R, const DecodeTail* tail, hipStream_t st);
-int launch_decode_team(const DecodeArgs& a, int D, int R, const DecodeTail& tail, const TeamMerge& merge, hipStream_t st);
+int launch_decode_team(const DecodeArgs& a, int D, int R, const DecodeTail* tail, const TeamMerge& merge, hipStream_t st);
 
 }  // namespace ommx
 
@@ -130,9 +130,9 @@ int ommx::decode_splitkv(OMMX_DECODE_PARAMS, bool plain, const StateLse* lse, co
     hipStream_t st = static_cast<hipStream_t>(stream);
     int rc = 1;
     if (team) {
-        rc = tail && !plain ? launch_decode_team(a, D, R, *tail, *team, st) : 1;
+        rc = plain ? 1 : launch_decode_team(a, D, R, tail, *team, st);
         if (rc == 1) return 1;
-        if (tail_done) *tail_done = true;
+        if (tail_done) *tail_done = tail != nullptr;
     } else if (!plain) {
         rc = tail ? launch_decode_gqa4_tail(a, D, R, tail, st) : launch_decode_gqa4(a, D, R, nullptr, st);
         if (rc == 0 && tail_done) *tail_done = tail != nullptr;

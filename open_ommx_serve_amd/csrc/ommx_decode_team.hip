@@ -94,6 +94,7 @@ struct TeamArgs {
     float sm_scale, cap;
     int B, shares, shares_few, singles;
     int32_t* share_count;
+    int tails;                               // workgroups of a kv head (HALF: of a pair) that attend its tail rows; 0 without any
     DecodeTail t;
 };
 // The kernel's arguments read again from where they lie, for parts that come late or that only some workgroups run: kept for
@@ -588,12 +589,13 @@ template <int DH>
 __device__ __forceinline__ void merge_states(const TeamArgs& a, int b, int qh0, int heads, int n, int lane, int wave) {
     constexpr int LPR = DH / 4, ROWS = 64 / LPR, LOADS = MOST_STATES / ROWS, HP = DH == 64 ? 2 : 1;
     static_assert(MOST_STATES <= 64 && MOST_STATES % ROWS == 0, "a state a lane");
-    const uint32_t N = min(n + kTailParts, MOST_STATES);
+    const int front = a.tails ? kTailParts : 0;           // states of the tail, before the others
+    const uint32_t N = min(n + front, MOST_STATES);
     const int c4 = lane % LPR, row = lane / LPR;
     // (bytes; a request's states span less than 2^32 of them)
     const uint32_t al_h = 4u * a.al_h, al_s = 4u * a.al_s, sl_h = 4u * a.sl_h, sl_s = 4u * a.sl_s;
-    const char* const al = reinterpret_cast<const char*>(a.al) + b * 4u * a.al_b - kTailParts * static_cast<int64_t>(al_s);
-    const char* const sl = reinterpret_cast<const char*>(a.sl) + b * 4u * a.sl_b - kTailParts * static_cast<int64_t>(sl_s);
+    const char* const al = reinterpret_cast<const char*>(a.al) + b * 4u * a.al_b - front * static_cast<int64_t>(al_s);
+    const char* const sl = reinterpret_cast<const char*>(a.sl) + b * 4u * a.sl_b - front * static_cast<int64_t>(sl_s);
     for (int h0 = wave; h0 < heads; h0 += WAVES * HP) {
         float lse[HP];
         uint64_t v[HP][LOADS][2];
@@ -664,15 +666,14 @@ __device__ __forceinline__ void merge_states(const TeamArgs& a, int b, int qh0, 
 
 // IDX, OWN_MAP: as in ommx_decode_gqa4.hip.  NH: q heads of a kv head the matrix rows are laid out for, 4 (1, 2 or 4 of them) or
 // 8.  HALF: head_dim 64, a workgroup takes a pair of kv heads, two waves each.  DEALT: the work of several requests in equal
-// shares (ommx_decode_shares.h), else a.S splits each.  The first workgroups of a kv head (HALF: two) attend its bf16 tail rows.
+// shares (ommx_decode_shares.h), else a.S splits each.  The first workgroups of a kv head (HALF: two) attend its bf16 tail rows, if there are any.
 template <int IDX, bool OWN_MAP, int NH, bool HALF, bool DEALT>
 __global__ void __launch_bounds__(64 * WAVES, team_resident(NH)) decode_team_kernel(TeamArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    constexpr int TAILS = HALF ? 2 : 1;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int unit = DEALT ? blockIdx.x : blockIdx.y;
-    const int first = DEALT ? TAILS * a.B : TAILS;
+    const int first = DEALT ? a.tails * a.B : a.tails;
     const int at = DEALT ? blockIdx.y : blockIdx.x;
     int b, page = 0, slot = 0;
     uint32_t n;                                     // splits of the request that hold something
@@ -684,10 +685,10 @@ __global__ void __launch_bounds__(64 * WAVES, team_resident(NH)) decode_team_ker
     };
     if (at < first) {
         const TeamArgs& t = args_again();
-        b = DEALT ? at / TAILS : blockIdx.z;
+        b = DEALT ? (HALF ? at >> 1 : at) : blockIdx.z;
         announce();
         uint8_t* const sm = smem + wave * TeamLds<NH, !OWN_MAP>::LDS_WAVE;
-        if constexpr (HALF) tail::attend_part<NH, 64, true>(t, sm, b, 2 * unit + at % TAILS, t.heads >> 1, wave, lane);
+        if constexpr (HALF) tail::attend_part<NH, 64, true>(t, sm, b, 2 * unit + (at & 1), t.heads >> 1, wave, lane);
         else tail::attend_part<NH, 128, true>(t, sm, b, unit, t.heads, wave, lane);
         if (!t.arrivals) return;
         if constexpr (DEALT) {
@@ -732,6 +733,7 @@ __global__ void __launch_bounds__(64 * WAVES, team_resident(NH)) decode_team_ker
                 slot = *reinterpret_cast<const int*>(a.rg + b * a.rg_b + ((uint32_t)min(g_first + (lane >> 5), G - 1) << a.tsh));
             }
             n = (G + per - 1) / per;
+            if (n == 0 && a.tails == 0) n = 1;      // (somebody has to say that nothing was attended)
             g_count = g_first < G ? min(per, G - g_first) : 0u;
         }
         if (L < 0) {                                // a negative length: nothing packed, reported
@@ -741,7 +743,12 @@ __global__ void __launch_bounds__(64 * WAVES, team_resident(NH)) decode_team_ker
         if (g_count == 0) {                         // an empty split: nothing attended (what the state holds is not read then)
             for (int r = threadIdx.x; r < a.heads; r += 64 * WAVES)
                 tail::put1<true>(a.sl + b * a.sl_b + (unit * a.heads + r) * a.sl_h + sp * a.sl_s, -INFINITY);
-            if (!DEALT) return;                     // (one of a fixed number is not waited for)
+            if (a.tails == 0 && !a.arrivals) {      // (a merge of its own without a tail multiplies it by its weight, zero)
+                const int width = HALF ? D / 2 : D;
+                for (int i = threadIdx.x; i < a.heads * width; i += 64 * WAVES)
+                    a.al[b * a.al_b + (unit * a.heads + i / width) * a.al_h + sp * a.al_s + i % width] = 0.0f;
+            }
+            if (!DEALT && !(a.tails == 0 && sp == 0)) return;      // (one of a fixed number is not waited for)
         } else {
             walk<IDX, OWN_MAP, NH, HALF>(a, smem, unit, b, L, sp, g_first, g_count, page, slot, !DEALT, lane, wave);
         }
@@ -754,7 +761,7 @@ __global__ void __launch_bounds__(64 * WAVES, team_resident(NH)) decode_team_ker
     uint32_t* const s_arrived = reinterpret_cast<uint32_t*>(smem);
     if (threadIdx.x == 0) *s_arrived = static_cast<uint32_t>(arrive(t.arrivals + 8 * (b * t.Hkv + unit), t.number, seen));
     team_barrier();
-    const bool last = *s_arrived == n + TAILS - 1;
+    const bool last = *s_arrived == n + t.tails - 1;
     if (!last) return;
     merge_states<HALF ? 64 : 128>(t, b, unit * heads, heads, n, lane, wave);
 }
@@ -762,7 +769,7 @@ __global__ void __launch_bounds__(64 * WAVES, team_resident(NH)) decode_team_ker
 }  // namespace
 
 // Returns 0 when launched, 1 when the shape belongs to another kernel (the same bounds as launch_decode_gqa4's).
-int launch_decode_team(const DecodeArgs& a, int Dh, int R, const DecodeTail& tail, const TeamMerge& merge, hipStream_t st) {
+int launch_decode_team(const DecodeArgs& a, int Dh, int R, const DecodeTail* tail, const TeamMerge& merge, hipStream_t st) {
     if (a.scale_bf16 || a.v_bf16 || a.gt != 32 || a.gc != 32 || a.kout != 6) return 1;
     if ((reinterpret_cast<uintptr_t>(a.q) & 3) || (a.q_sb & 1) || (a.q_sh & 1)) return 1;
     const bool half = Dh == 64;
@@ -784,6 +791,7 @@ int launch_decode_team(const DecodeArgs& a, int Dh, int R, const DecodeTail& tai
     // (states are written and merged eight bytes at a time and more)
     if ((reinterpret_cast<uintptr_t>(a.al) & 15) || a.al_b % 4 || a.al_h % 4 || a.al_s % 4) return 1;
     if (merge.arrivals && (a.S > kTeamMerged || !merge.lse || merge.number < kFirstCall)) return 1;
+    const int nh = R == 8 ? 8 : 4, tails = !tail ? 0 : half ? 2 : 1;
     auto u = [](int64_t v) { return static_cast<uint32_t>(v); };
     const TeamArgs t{merge.arrivals, merge.number, merge.o, merge.o16, merge.lse, merge.o_b, merge.o_h, merge.lse_b,
                      a.seq, a.q, a.k_base, a.k_scale, a.k_zp, a.k_ms, a.k_mc, a.k_obmp, a.k_oval, a.v_main, a.v_scale, a.v_zp,
@@ -791,8 +799,7 @@ int launch_decode_team(const DecodeArgs& a, int Dh, int R, const DecodeTail& tai
                      u(a.rt_s << tsh), u(a.rg_s << tsh), merge.rt_n, merge.rg_n - a.gbase,
                      u(a.q_sb), u(a.q_sh), u(a.al_b), u(a.al_h), u(a.al_s), u(a.sl_b), u(a.sl_h), u(a.sl_s),
                      a.Hq / Hk, Hk, __builtin_ctz(a.ps), tsh, a.gbase * 32 + a.off, a.n_pages, a.n_gslots, a.S, merge.per_split,
-                     a.sm_scale, a.cap, a.B, a.shares, a.shares_few, a.singles, a.share_count, tail};
-    const int nh = R == 8 ? 8 : 4, tails = half ? 2 : 1;
+                     a.sm_scale, a.cap, a.B, a.shares, a.shares_few, a.singles, a.share_count, tails, tail ? *tail : DecodeTail{}};
     const dim3 grid = a.shares > 0 ? dim3(Hk, a.shares + tails * a.B) : dim3(a.S + tails, Hk, a.B);
     const size_t shm = nh == 8 ? (a.k_ms ? TeamLds<8, false>::BYTES : TeamLds<8, true>::BYTES) : a.k_ms ? TeamLds<4, false>::BYTES : TeamLds<4, true>::BYTES;
 #define OMMX_TEAM(IDX, MAP, NH, HALF)                                                                                            \

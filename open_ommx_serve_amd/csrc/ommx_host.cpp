@@ -30,6 +30,7 @@
 #include <cstring>
 #include <initializer_list>
 #include <mutex>
+#include <random>
 #include <vector>
 
 #include "../../include/ommx_hip.h"
@@ -385,7 +386,8 @@ int run_decode(const DecodeCall& c) {
     // the merge inside the launch: its words lie behind the `used` bytes of the scratch, on a line of their own
     const size_t words = static_cast<size_t>(B * wave_heads + 1) * 64;
     auto team_merge = [&](void* scratch, int64_t used, float* lse, int64_t per, bool fused) {
-        static std::atomic<uint64_t> calls{ommx::kFirstCall};
+        // (from a number of this process' own on: memory handed on by the driver may hold another one's words)
+        static std::atomic<uint64_t> calls{ommx::kFirstCall + (static_cast<uint64_t>(std::random_device{}()) << 14)};
         ommx::TeamMerge m{static_cast<int>(std::min<int64_t>(rt.size(1), INT32_MAX)), static_cast<int>(std::min<int64_t>(rg.size(1), INT32_MAX)),
                           static_cast<int>(per)};
         if (!fused) return m;
@@ -443,7 +445,9 @@ int run_decode(const DecodeCall& c) {
     // of 8 kv heads 14.0 us against 14.3, 12 K 17.6 against 15.8; 8 K with 64 q heads 16.6 / 19.8, 16 K 22.8 / 21.3; with 64 channels, whose
     // heads it does not read in pairs of which one is zero, 16 K 13.6 / 18.0, 2 x 12 K (six steps) 15.7 / 17.8; with one kv head, where a
     // workgroup of the other kernel is a single wave, 16 of 1 to 16 K (16 steps) 20.3 / 22.2, but 8 of 20 to 32 K 24.0 / 23.2.
-    if (c.splits == 0 && tail_rows && plain_planes && k == 6 && B <= 64 && (D == 128 || paired)) {
+    // (a range of groups without a tail, of which the caller merges the states, has the rounding of the whole then)
+    const bool no_tail = !hist && !tail && !c.ws && !c.force;
+    if (c.splits == 0 && (tail_rows || no_tail) && plain_planes && k == 6 && B <= 64 && (D == 128 || paired)) {
         const int64_t cus = cu_count(dev.index()), steps = (longest + 1) / 2, all = B * steps * wave_heads;
         if (all <= cus * (paired || wave_heads == 1 ? 8 : 4)) {
             // The merge inside the launch while its one workgroup has little to read, instead of a launch of its own (3.5 us of host

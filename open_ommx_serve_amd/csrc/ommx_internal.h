@@ -159,7 +159,7 @@ struct TeamMerge {
 
 // ommx_decode_splitkv / _ref (plain) with these choices (each may be NULL).  Returns 1, with nothing done, when shares
 // are asked for and no kernel with shares serves the call.  *tail_done tells whether the launch attends the tail.  team: by the
-// kernel for short calls (csrc/ommx_decode_team.hip), which needs a tail; returns 1, with nothing done, for what it does not serve.
+// kernel for short calls (csrc/ommx_decode_team.hip); returns 1, with nothing done, for what it does not serve.
 #define OMMX_DECODE_DECL                                                                            \
     const uint16_t* q, int64_t q_stride_b, int64_t q_stride_h, const uint8_t* k_base,               \
     const void* k_scale, const uint16_t* k_zp, const uint16_t* k_ms, const uint16_t* k_mc,          \
