@@ -152,6 +152,8 @@ int ommx_store_pack(const void* K, const void* V, int in_dtype,
  *   the same with 1..8 outliers on the bitmap plane, also at head_dim 64 (r in {1,2,4}, Hkv even);
  *   64- or 128-token groups with 32/64/128-channel V vectors and 6 outliers, relidx7 plane;
  *   128-token groups with 10 outliers, relidx7 plane (4 or 8 q heads per kv head).
+ * 64-channel heads with position streams and 1, 2 or 4 q heads per kv head (32-token groups with up to 6
+ * outliers, 64 / 128-token ones with up to 10) run on a kernel of their own in fp32.
  * Every other supported shape or recipe (k_outliers up to 16) runs on the plain fp32 kernel.
  *   num_pages, num_group_slots   extents of the planes the tables index (k_base / v_main pages,
  *                 k_scale group slots); the reference guards table entries on the host

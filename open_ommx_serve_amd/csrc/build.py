@@ -29,6 +29,7 @@ SOURCES = {
     "ommx_decode_gqa4.hip": [],
     "ommx_decode_gqa4_tail.hip": [],
     "ommx_decode_team.hip": [],
+    "ommx_decode_fp32.hip": [],
     "ommx_combine.hip": [],
     "ommx_ring.hip": [],
     "ommx_merge.hip": [],

@@ -15,6 +15,7 @@ void set_error(const char* msg) { g_error = msg; }
 int launch_decode_fast(const DecodeArgs& a, int D, int R, hipStream_t st);
 int launch_decode_gqa4(const DecodeArgs& a, int D, int R, const DecodeTail* tail, hipStream_t st);
 int launch_decode_gqa4_tail(const DecodeArgs& a, int D, int R, const DecodeTail* tail, hipStream_t st);
+int launch_decode_fp32(const DecodeArgs& a, int D, int R, const DecodeTail* tail, hipStream_t st);
 int launch_decode_team(const DecodeArgs& a, int D, int R, const DecodeTail* tail, const TeamMerge& merge, hipStream_t st);
 
 }  // namespace ommx
@@ -137,6 +138,10 @@ int ommx::decode_splitkv(OMMX_DECODE_PARAMS, bool plain, const StateLse* lse, co
         rc = tail ? launch_decode_gqa4_tail(a, D, R, tail, st) : launch_decode_gqa4(a, D, R, nullptr, st);
         if (rc == 0 && tail_done) *tail_done = tail != nullptr;
         if (rc == 1) rc = launch_decode_fast(a, D, R, st);
+        if (rc == 1) {
+            rc = launch_decode_fp32(a, D, R, tail, st);
+            if (rc == 0 && tail_done) *tail_done = tail != nullptr;
+        }
         if (rc == 1 && shares) return 1;                  // (the plain kernel knows fixed splits only)
     }
     if (rc == 1) rc = launch_decode_ref(a, D, R, st);     // shapes the matrix-core kernels leave out

@@ -2,8 +2,8 @@
 // the FP4 outliers, attend, accumulate P.V from the INT2 V rows.  One workgroup per
 // (request, kv head, split); 256 threads.  This is the straightforward formulation of
 // ommx_gpu_serve/attention/paged_decode.py:1657-2284 (production branch), used as the
-// on-device cross-check of the tuned kernel and for head shapes the tuned kernel does
-// not cover.
+// on-device cross-check of the tuned kernels and for what they do not cover (ommx_decode.hip, ommx_decode_gqa4.hip,
+// ommx_decode_team.hip, ommx_decode_fp32.hip).
 //
 // Bound by the vector instructions and waits around its loads at five to seven waves per SIMD.  The outlier frames of a
 // channel come in whole dwords and are walked in registers (byte by byte from memory, each slot waited for its

@@ -300,13 +300,16 @@ int run_decode(const DecodeCall& c) {
     // with the same numbers).
     const bool pieces = gt >= 64 && !scale_bf16 && !v_bf16 && !c.force && D == 128 && R >= 4 && gc >= 32 && !c.bitmap &&
                         (k == 6 || (k == 10 && gt == 128));
-    const int64_t unit = pieces ? 64 : gt;                       // tokens that a share is made of
+    // 64-channel heads with position streams (csrc/ommx_decode_fp32.hip): longer groups in pieces as well
+    const bool fp32 = D == 64 && R <= 4 && !c.bitmap && !scale_bf16 && !v_bf16 && !c.force && gt >= 32 && gc >= 32 && k >= 1 &&
+                      k <= (gt == 32 ? 6 : 10);
+    const int64_t unit = pieces || (fp32 && gt >= 64) ? 64 : gt;           // tokens that a share is made of
     // Longer groups keep two workgroups a compute unit (a third does not fit their LDS, and the shares of a round that is not
     // there made full batches slower than whole groups on the kernel before: 8 x 32 K tokens of 64 x 64 vectors 124 us with
     // three, 113 on that kernel, 95 with two; 32 of 1 to 16 K 134 / 128 / 105; of 128 x 128 with ten outliers 173 / 165 / 125).
-    const bool lean = plain_planes && ((D == 128 && R <= 4 && k == 6) ||
+    const bool lean = fp32 || (plain_planes && ((D == 128 && R <= 4 && k == 6) ||
                                        (c.bitmap && k >= 1 && k <= 6 && ((D == 128 && R <= 4) ||
-                                                                         (D == 64 && R <= 2 && Hkv % 2 == 0))));
+                                                                         (D == 64 && R <= 2 && Hkv % 2 == 0)))));
     const bool paired = plain_planes && D == 64 && c.bitmap && k >= 1 && k <= 8 && R <= 4 && Hkv % 2 == 0;
     const int64_t wave_heads = paired ? Hkv / 2 : Hkv;           // waves that one share of the tokens takes
 
