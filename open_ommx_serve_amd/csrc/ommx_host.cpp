@@ -22,6 +22,7 @@
 #include <c10/hip/HIPGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
+#include <torch/csrc/Device.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -718,6 +719,90 @@ at::Tensor take_flags() {
     return t;
 }
 
+// A block packed into planes of its own with identity tables: the launch is under way when this returns; `t` takes the planes and the
+// error words.  0 launched, 1 not for this path (nothing done), -1 failed.
+enum { FLAGS, KBASE, KSCALE, KZP, INDEX, OVAL, MS, MC, VMAIN, VSCALE, VZP, TOK, GRP, COUNT };
+int launch_block(const at::Tensor& K, const at::Tensor& V, int64_t ps, bool own_map, const at::Tensor& table, const Recipe& r,
+                 hipStream_t stream, at::Tensor (&t)[COUNT]) {
+    const int64_t T = K.size(0), H = K.size(1), D = K.size(2), G = T / r.gt, P = T / ps;
+    c10::Allocator* const allocator = c10::hip::HIPCachingAllocatorMasqueradingAsCUDA::get();
+    // (a dozen tensors: their memory from the allocator directly, the dispatcher would cost a microsecond for each, and what holds it
+    // is made while the kernel runs)
+    struct Part {
+        int64_t shape[4];
+        int dims;
+        at::ScalarType type;
+        size_t bytes = 0;
+        c10::DataPtr mem;
+    } part[COUNT];
+    auto make = [&](int i, std::initializer_list<int64_t> shape, at::ScalarType type) {
+        Part& x = part[i];
+        std::copy(shape.begin(), shape.end(), x.shape);
+        x.dims = static_cast<int>(shape.size());
+        x.type = type;
+        x.bytes = c10::elementSize(type);
+        for (int64_t n : shape) x.bytes *= static_cast<size_t>(n);
+        x.mem = allocator->allocate(x.bytes);
+        return x.mem.get();
+    };
+    const at::ScalarType step = r.mode == OMMX_SCALE_POW2_INT8 ? at::kChar : at::kBFloat16;
+    t[FLAGS] = take_flags();
+    void *index = nullptr, *oval = nullptr, *ms = nullptr, *mc = nullptr;
+    void* const k_base = make(KBASE, {P, ps, H, D / 4}, at::kByte);
+    void* const k_scale = make(KSCALE, {G, H, D}, step);
+    void* const k_zp = make(KZP, {G, H, D}, at::kBFloat16);
+    if (r.k > 0) {
+        index = make(INDEX, {G, H, D, r.bitmap ? (r.gt + 7) / 8 : (7 * r.k + 7) / 8}, at::kByte);
+        oval = make(OVAL, {G, H, D, (r.k + 1) / 2}, at::kByte);
+        if (own_map) {
+            ms = make(MS, {G, H, D}, at::kBFloat16);
+            mc = make(MC, {G, H, D}, at::kBFloat16);
+        }
+    }
+    void* const v_main = r.v_bf16 ? make(VMAIN, {P, ps, H, D}, at::kBFloat16) : make(VMAIN, {P, ps, H, D / 4}, at::kByte);
+    void* const v_scale = make(VSCALE, {P, ps, H, D / r.gc}, step);
+    void* const v_zp = make(VZP, {P, ps, H, D / r.gc}, at::kBFloat16);
+    void* const tok = make(TOK, {1, P}, at::kInt);
+    void* const grp = make(GRP, {1, G}, at::kInt);
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = ommx::store_pack(K.data_ptr(), V.data_ptr(), K.scalar_type() == at::kFloat, K.stride(0), K.stride(1), V.stride(0), V.stride(1),
+                          nullptr, T, H, D, ps, r.k, r.bitmap ? OMMX_INDEX_BITMAP : OMMX_INDEX_RELIDX7, r.abs, r.mode, r.gt, r.gc, r.v_bf16,
+                          nullptr, nullptr, table.data_ptr<float>(), static_cast<uint8_t*>(k_base), k_scale, static_cast<uint16_t*>(k_zp),
+                          static_cast<uint16_t*>(ms), static_cast<uint16_t*>(mc), static_cast<uint8_t*>(index), static_cast<uint8_t*>(oval),
+                          static_cast<uint8_t*>(v_main), v_scale, static_cast<uint16_t*>(v_zp), t[FLAGS].data_ptr<int32_t>(),
+                          {true, static_cast<int32_t*>(tok), static_cast<int32_t*>(grp)}, stream);
+    Py_END_ALLOW_THREADS
+    for (int i = 0; i < COUNT; ++i) {
+        Part& x = part[i];
+        if (x.bytes == 0) continue;
+        t[i] = at::detail::make_tensor_base<c10::TensorImpl>(
+            c10::make_intrusive<c10::StorageImpl>(c10::StorageImpl::use_byte_size_t(), x.bytes, std::move(x.mem), allocator, true),
+            c10::DispatchKeySet(c10::DispatchKey::CUDA), c10::scalarTypeToTypeMeta(x.type));
+        t[i].unsafeGetTensorImpl()->generic_set_sizes_contiguous(at::IntArrayRef(x.shape, x.dims));
+    }
+    return rc;
+}
+// Should nobody ask for the errors of a block, its words must not be handed on before the kernel is through with them.
+void keep_flags_for(const at::Tensor& flags, c10::Device dev) {
+    at::getHostAllocator(c10::DeviceType::CUDA)->record_event(flags.data_ptr(), flags.storage().data_ptr().get_context(),
+                                                              c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index()).unwrap());
+}
+// The error bits, once the launch has ended; the words go back to those kept idle.
+long take_errors(const at::Tensor& flags) {
+    const int32_t* words = flags.data_ptr<int32_t>();
+    long bits = 0;
+    for (int i = 0; i < OMMX_STORE_ERR_WORDS; ++i) bits |= (words[i] ? 1L : 0L) << i;
+    FlagPool& pool = flag_pool();
+    std::lock_guard<std::mutex> hold(pool.lock);
+    if (pool.idle.size() < kKeptFlags) pool.idle.push_back(flags);
+    return bits;
+}
+bool is_block(const at::Tensor& K, const at::Tensor& V, int64_t ps, const Recipe& r) {
+    return is_rows(K) && is_rows(V) && K.sizes() == V.sizes() && ps >= 1 && K.scalar_type() == V.scalar_type() &&
+           K.device() == V.device() && K.is_cuda() && K.size(0) >= 1 && K.size(0) % ps == 0 && K.size(0) % r.gt == 0 && K.size(2) % r.gc == 0;
+}
+
 // (K, V, page_size, kv_outlier_map, table, recipe x 8) -> (flags, k_base, k_scale, k_zp, k_index, k_oval, k_mapscale,
 // k_mapcenter, v_main, v_scale, v_zp, req_to_token, req_to_group), or False.  Launches the packing of a block into planes
 // of its own with identity tables.  The caller does its own work and then asks block_errors(flags), the one host
@@ -730,49 +815,12 @@ PyObject* py_pack_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const int64_t ps = as_int(a[2], ok);
     const bool own_map = as_bool(a[3], ok);
     Recipe r;
-    if (!ok || !read_recipe(a + 5, r) || !is_rows(*K) || !is_rows(*V) || K->sizes() != V->sizes() || ps < 1 ||
-        K->scalar_type() != V->scalar_type() || K->device() != V->device() || !K->is_cuda() || K->size(0) < 1 ||
-        K->size(0) % ps || K->size(0) % r.gt || K->size(2) % r.gc)
-        Py_RETURN_FALSE;
+    if (!ok || !read_recipe(a + 5, r) || !is_block(*K, *V, ps, r)) Py_RETURN_FALSE;
     const c10::Device dev = K->device();
     c10::hip::HIPGuard guard(dev.index());
-    hipStream_t stream = stream_of(dev);
-    const int64_t T = K->size(0), H = K->size(1), D = K->size(2), G = T / r.gt, P = T / ps;
-    c10::Allocator* const allocator = c10::hip::HIPCachingAllocatorMasqueradingAsCUDA::get();
-    // (a dozen tensors: taken from the allocator directly, the dispatcher would cost a microsecond for each)
-    auto make = [&](at::IntArrayRef shape, at::ScalarType type) {
-        return at::detail::empty_generic(shape, allocator, c10::DispatchKeySet(c10::DispatchKey::CUDA), type, std::nullopt);
-    };
-    const at::ScalarType step = r.mode == OMMX_SCALE_POW2_INT8 ? at::kChar : at::kBFloat16;
-    enum { FLAGS, KBASE, KSCALE, KZP, INDEX, OVAL, MS, MC, VMAIN, VSCALE, VZP, TOK, GRP, COUNT };
     at::Tensor t[COUNT];
-    t[FLAGS] = take_flags();
-    t[KBASE] = make({P, ps, H, D / 4}, at::kByte);
-    t[KSCALE] = make({G, H, D}, step);
-    t[KZP] = make({G, H, D}, at::kBFloat16);
-    if (r.k > 0) {
-        t[INDEX] = make({G, H, D, r.bitmap ? (r.gt + 7) / 8 : (7 * r.k + 7) / 8}, at::kByte);
-        t[OVAL] = make({G, H, D, (r.k + 1) / 2}, at::kByte);
-        if (own_map) {
-            t[MS] = make({G, H, D}, at::kBFloat16);
-            t[MC] = make({G, H, D}, at::kBFloat16);
-        }
-    }
-    t[VMAIN] = r.v_bf16 ? make({P, ps, H, D}, at::kBFloat16) : make({P, ps, H, D / 4}, at::kByte);
-    t[VSCALE] = make({P, ps, H, D / r.gc}, step);
-    t[VZP] = make({P, ps, H, D / r.gc}, at::kBFloat16);
-    t[TOK] = make({1, P}, at::kInt);
-    t[GRP] = make({1, G}, at::kInt);
-    auto opt = [&](int i) { return t[i].defined() ? &t[i] : nullptr; };
-    const Planes p{&t[KBASE], &t[KSCALE], &t[KZP], opt(MS), opt(MC), opt(INDEX), opt(OVAL), &t[VMAIN], &t[VSCALE], &t[VZP]};
-    int rc;
-    Py_BEGIN_ALLOW_THREADS
-    rc = launch_store(*K, *V, 0, p, r, T, ps, nullptr, nullptr, nullptr, *table, t[FLAGS].data_ptr<int32_t>(),
-                      {true, t[TOK].data_ptr<int32_t>(), t[GRP].data_ptr<int32_t>()}, stream);
-    Py_END_ALLOW_THREADS
-    // Should the caller never ask for the errors, the block must not be handed on before the kernel is through with it.
-    at::getHostAllocator(c10::DeviceType::CUDA)->record_event(t[FLAGS].data_ptr(), t[FLAGS].storage().data_ptr().get_context(),
-                                                              c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index()).unwrap());
+    const int rc = launch_block(*K, *V, ps, own_map, *table, r, stream_of(dev), t);
+    keep_flags_for(t[FLAGS], dev);
     if (failed(rc, "ommx_store_pack")) return nullptr;
     PyObject* out = PyTuple_New(COUNT);
     for (int i = 0; i < COUNT; ++i) {
@@ -780,6 +828,83 @@ PyObject* py_pack_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
         else PyTuple_SET_ITEM(out, i, THPVariable_Wrap(std::move(t[i])));
     }
     return out;
+}
+
+// The whole of a block's call for arguments in their plain form: (K, V, table, page_size, device, kv_outlier_map, k_format, outliers,
+// group_tokens, group_channels, outlier_repr, outlier_select, use_pow2, kv_int8_scale, v_format), None for either flag that may be
+// left out.  -> the plane dict, the error bits of a block that has any, or False with nothing done.
+constexpr const char* kBlockKeys[] = {
+    "k_base", "k_scale", "k_zp", "k_oidx", "k_oval", "k_crank", "k_obmp", "k_fp4_mapscale", "k_fp4_mapcenter", "k_field_bytes",
+    "v_main", "v_scale", "v_zp", "req_to_token", "req_to_group", "head_dim", "n_kv_heads", "num_tokens", "n_groups", "page_size",
+    "outliers_per_vector", "outlier_repr", "outlier_select", "group_tokens", "group_channels", "k_format", "v_format", "k_base_bits",
+    "oval_bits", "use_pow2", "kv_outlier_map", "kv_int8_scale"};
+constexpr int kBlockKeyCount = sizeof(kBlockKeys) / sizeof(kBlockKeys[0]);
+PyObject* g_block_keys[kBlockKeyCount];
+
+PyObject* py_pack_whole_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 15) { PyErr_SetString(PyExc_TypeError, "pack_whole_block: wrong number of arguments"); return nullptr; }
+    if (!plain_call(a, 2)) Py_RETURN_FALSE;
+    bool ok = true;
+    const at::Tensor *K = as_tensor(a[0], ok), *V = as_tensor(a[1], ok), *table = as_tensor(a[2], ok);
+    const int64_t ps = as_int(a[3], ok);
+    PyObject* const recipe[8] = {a[7], a[8], a[9], a[10], a[11], a[12], a[13] == Py_None ? Py_True : a[13], a[14]};
+    const bool map = a[5] == Py_None || as_bool(a[5], ok);
+    Recipe r;
+    if (!ok || !(is_word(a[6], "i2f4") || is_word(a[6], "itf4")) || !read_recipe(recipe, r) || !is_block(*K, *V, ps, r) ||
+        K->size(2) % 32 || K->size(2) > 256 || r.k > r.gt)
+        Py_RETURN_FALSE;
+    const c10::Device dev = K->device();
+    if (THPDevice_Check(a[4])) {
+        const c10::Device& want = reinterpret_cast<THPDevice*>(a[4])->device;
+        if (!want.is_cuda() || (want.has_index() ? want.index() : c10::hip::current_device()) != dev.index()) Py_RETURN_FALSE;
+    } else if (!is_word(a[4], "cuda") || c10::hip::current_device() != dev.index()) {
+        Py_RETURN_FALSE;
+    }
+    c10::hip::HIPGuard guard(dev.index());
+    hipStream_t stream = stream_of(dev);
+    at::Tensor t[COUNT];
+    if (failed(launch_block(*K, *V, ps, map, *table, r, stream, t), "ommx_store_pack")) { keep_flags_for(t[FLAGS], dev); return nullptr; }
+    // (put together while the kernel runs)
+    const at::Tensor flags = t[FLAGS];
+    PyObject* const out = PyDict_New();
+    int key = 0;
+    bool good = out != nullptr;
+    auto put = [&](PyObject* value) {          // takes the reference
+        good = good && value && PyDict_SetItem(out, g_block_keys[key], value) == 0;
+        ++key;
+        Py_XDECREF(value);
+    };
+    auto tensor = [&](int i) { put(t[i].defined() ? THPVariable_Wrap(std::move(t[i])) : Py_NewRef(Py_None)); };
+    auto none = [&]() { put(Py_NewRef(Py_None)); };
+    auto number = [&](int64_t v) { put(PyLong_FromLongLong(v)); };
+    auto flag = [&](bool v) { put(Py_NewRef(v ? Py_True : Py_False)); };
+    auto same = [&](PyObject* o) { put(Py_NewRef(o)); };
+    const int64_t T = K->size(0);
+    tensor(KBASE); tensor(KSCALE); tensor(KZP);
+    if (r.bitmap) none(); else tensor(INDEX);
+    tensor(OVAL); none();
+    if (r.bitmap) tensor(INDEX); else none();
+    tensor(MS); tensor(MC);
+    number(r.bitmap && r.k > 0 ? (r.gt + 7) / 8 : 0);
+    tensor(VMAIN); tensor(VSCALE); tensor(VZP); tensor(TOK); tensor(GRP);
+    number(K->size(2)); number(K->size(1)); number(T); number(T / r.gt); number(ps); number(r.k);
+    same(recipe[3]); same(recipe[4]); number(r.gt); number(r.gc); same(a[6]); same(recipe[7]);
+    number(2); number(4);
+    flag(recipe[5] == Py_True); flag(map && r.k > 0); flag(recipe[5] == Py_True && recipe[6] == Py_True);
+    hipError_t waited;
+    Py_BEGIN_ALLOW_THREADS
+    waited = hipStreamSynchronize(stream);
+    Py_END_ALLOW_THREADS
+    if (waited != hipSuccess) {
+        keep_flags_for(flags, dev);
+        Py_XDECREF(out);
+        PyErr_Format(PyExc_RuntimeError, "ommx_store_pack: %s", hipGetErrorString(waited));
+        return nullptr;
+    }
+    const long bits = take_errors(flags) & ~static_cast<long>(OMMX_NOTE_WIDE_STEP);
+    if (good && bits == 0) return out;
+    Py_XDECREF(out);
+    return good ? PyLong_FromLong(bits) : nullptr;
 }
 
 // (flags, tensor of the packing device): waits for the current stream of that device and returns the error bits
@@ -800,15 +925,7 @@ PyObject* py_block_errors(PyObject*, PyObject* const* a, Py_ssize_t n) {
         PyErr_Format(PyExc_RuntimeError, "ommx_store_pack: %s", hipGetErrorString(waited));
         return nullptr;
     }
-    const int32_t* words = flags->data_ptr<int32_t>();
-    long bits = 0;
-    for (int i = 0; i < OMMX_STORE_ERR_WORDS; ++i) bits |= (words[i] ? 1L : 0L) << i;
-    {
-        FlagPool& pool = flag_pool();
-        std::lock_guard<std::mutex> hold(pool.lock);
-        if (pool.idle.size() < kKeptFlags) pool.idle.push_back(*flags);
-    }
-    return PyLong_FromLong(bits);
+    return PyLong_FromLong(take_errors(*flags));
 }
 
 // ── bf16 row history ───────────────────────────────────────────────────────────────────────────
@@ -1303,7 +1420,7 @@ PyObject* guarded(PyObject* self, PyObject* const* a, Py_ssize_t n) {
 #define OMMX_FAST(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(guarded<py_##name>)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
     OMMX_FAST(auto_num_kv_splits), OMMX_FAST(plain), OMMX_FAST(rows_fit),
-    OMMX_FAST(decode), OMMX_FAST(decode_pool), OMMX_FAST(store_pack), OMMX_FAST(pack_block), OMMX_FAST(block_errors), OMMX_FAST(pack_groups), OMMX_FAST(pack_prompts), OMMX_FAST(ring_write),
+    OMMX_FAST(decode), OMMX_FAST(decode_pool), OMMX_FAST(store_pack), OMMX_FAST(pack_block), OMMX_FAST(pack_whole_block), OMMX_FAST(block_errors), OMMX_FAST(pack_groups), OMMX_FAST(pack_prompts), OMMX_FAST(ring_write),
     OMMX_FAST(all_at), OMMX_FAST(append_rows), OMMX_FAST(append_step), OMMX_FAST(first_column),
     OMMX_FAST(tail_gather), OMMX_FAST(rows_write), OMMX_FAST(upload), OMMX_FAST(prefill), OMMX_FAST(prefill_form),
     {nullptr, nullptr, 0, nullptr},
@@ -1319,6 +1436,8 @@ PyMODINIT_FUNC PyInit__ommx_host(void) {
     for (int i = 0; i < 11; ++i)
         if (!(g_names[i] = PyUnicode_InternFromString(names[i]))) return nullptr;
     if (!(g_bitmap = PyUnicode_InternFromString("bitmap"))) return nullptr;
+    for (int i = 0; i < kBlockKeyCount; ++i)
+        if (!(g_block_keys[i] = PyUnicode_InternFromString(kBlockKeys[i]))) return nullptr;
     PyObject* m = PyModule_Create(&module);
     if (m && PyModule_AddIntConstant(m, "STEP_ROWS", ommx::kStepRows) < 0) Py_CLEAR(m);
     return m;

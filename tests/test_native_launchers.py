@@ -374,3 +374,34 @@ def test_rows_and_groups_of_a_fresh_block_in_one_launch(T, H, gt, single):
     for n, t in made[0]._store_planes.items():
         if torch.is_tensor(t):
             assert torch.equal(t.view(torch.uint8), made[1]._store_planes[n].view(torch.uint8)), n
+
+
+@pytest.mark.parametrize("kw", [
+    {}, dict(outlier_repr="relidx7", kv_outlier_map=False), dict(group_tokens=64, group_channels=64, outliers_per_vector=10, outlier_repr="relidx7"),
+    dict(outliers_per_vector=0), dict(v_format="bf16", k_format="itf4"), dict(use_pow2=False, outlier_select="abs"),
+    dict(kv_int8_scale=False, kv_outlier_map=None), dict(kv_int8_scale=True, outliers_per_vector=3)], ids=lambda k: "-".join(map(str, k.values())) or "serving")
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_the_one_call_of_a_block_gives_what_the_steps_give(kw, dtype):
+    """Same keys in the same order, same values of the same types, same bits as arguments that take the way through Python
+    (a device by its full name), and the same error for the same block."""
+    call = dict(outliers_per_vector=6, outlier_repr="bitmap", outlier_select="signed", use_pow2=True, page_size=16) | kw
+    K, V = _block(128, 2, 64, dtype, 31), _block(128, 2, 64, dtype, 32, strided=True)
+    store_table(K.device)
+    assert _hip.host().pack_whole_block(K, V, store_table(K.device), 16, "cuda:0", None, "i2f4", 6, 32, 32, "bitmap", "signed", True, None, "i2") is False
+    want = ommx_pack_kv_canonical_block(K, V, device="cuda:0", **call)
+    for device in ("cuda", torch.device("cuda"), torch.device("cuda", 0), K.device):
+        got = ommx_pack_kv_canonical_block(K, V, device=device, **call)
+        assert list(got) == list(want)
+        for name, value in want.items():
+            assert type(got[name]) is type(value), name
+            if torch.is_tensor(value):
+                assert got[name].dtype == value.dtype and got[name].device == value.device and got[name].is_contiguous(), name
+                assert torch.equal(got[name].view(torch.uint8), value.view(torch.uint8)), name
+            else:
+                assert got[name] == value, name
+    if kw.get("v_format") != "bf16":
+        V = V.clone()
+        V[5, 1, 3] = float("nan")
+        for device in ("cuda", "cuda:0"):
+            with pytest.raises(ValueError, match="V pack: non-finite"):
+                ommx_pack_kv_canonical_block(K, V, device=device, **call)
