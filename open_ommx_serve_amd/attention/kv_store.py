@@ -204,8 +204,11 @@ class CanonicalKVStore:
     def write_token(self, pos: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> None:
         """Write one K/V row at the absolute position held in the device tensor ``pos``
         ([1] int64); launch-only, ``seq_len`` is not touched (kv_store.py:361-385)."""
-        if self._host.ring_write(self._k_hist4, self._v_hist4, pos, k.reshape(1, self.H, self.D),
-                                 v.reshape(1, self.H, self.D), self._ring_sink, self._ring_rec, None, None,
+        self.write_row(pos, k.reshape(1, self.H, self.D), v.reshape(1, self.H, self.D))
+
+    def write_row(self, pos: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> None:
+        """``write_token`` of rows ``[1, H, D]`` as a step has them."""
+        if self._host.ring_write(self._k_hist4, self._v_hist4, pos, k, v, self._ring_sink, self._ring_rec, None, None,
                                  self.err_flag):
             return
         kb = k.reshape(self.H, self.D)

@@ -1252,6 +1252,23 @@ PyObject* py_upload(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Py_RETURN_TRUE;
 }
 
+// (block, length, boundary, sink rows, tail rows, packed length): the block of a one-request step (ommx::step_block)
+PyObject* py_step_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 6) { PyErr_SetString(PyExc_TypeError, "step_block: wrong number of arguments"); return nullptr; }
+    bool ok = true;
+    const at::Tensor* block = as_tensor(a[0], ok);
+    const int64_t seq = as_int(a[1], ok), boundary = as_int(a[2], ok), sink = as_int(a[3], ok), tail = as_int(a[4], ok),
+                  packed = as_int(a[5], ok);
+    if (!ok || !block->is_cuda() || !block->is_contiguous() || block->scalar_type() != at::kInt || block->numel() < 6 ||
+        block->numel() % 2 || reinterpret_cast<uintptr_t>(block->data_ptr()) % 8)
+        Py_RETURN_FALSE;
+    c10::hip::HIPGuard guard(block->device().index());
+    if (failed(ommx::step_block(block->data_ptr<int32_t>(), static_cast<int>(block->numel() / 2 - 1), seq, boundary, sink, tail, packed,
+                                stream_of(block->device())), "step_block"))
+        return nullptr;
+    Py_RETURN_TRUE;
+}
+
 // ── one step's host bookkeeping ────────────────────────────────────────────────────────────────
 // A decode step of short contexts is some 20 us of GPU time a layer; the loops over its requests and the calls around its
 // launches took longer than that in Python.  Plain lists of ints only: anything else is refused, and served by the
@@ -1422,7 +1439,7 @@ PyMethodDef methods[] = {
     OMMX_FAST(auto_num_kv_splits), OMMX_FAST(plain), OMMX_FAST(rows_fit),
     OMMX_FAST(decode), OMMX_FAST(decode_pool), OMMX_FAST(store_pack), OMMX_FAST(pack_block), OMMX_FAST(pack_whole_block), OMMX_FAST(block_errors), OMMX_FAST(pack_groups), OMMX_FAST(pack_prompts), OMMX_FAST(ring_write),
     OMMX_FAST(all_at), OMMX_FAST(append_rows), OMMX_FAST(append_step), OMMX_FAST(first_column),
-    OMMX_FAST(tail_gather), OMMX_FAST(rows_write), OMMX_FAST(upload), OMMX_FAST(prefill), OMMX_FAST(prefill_form),
+    OMMX_FAST(tail_gather), OMMX_FAST(rows_write), OMMX_FAST(upload), OMMX_FAST(step_block), OMMX_FAST(prefill), OMMX_FAST(prefill_form),
     {nullptr, nullptr, 0, nullptr},
 };
 #undef OMMX_FAST

@@ -81,6 +81,8 @@ int prompt_blocks(const PromptBlocks& blocks, const PromptRow* prompts, int n, i
 // copy engine, nothing to keep alive after the call.
 constexpr int kUploadWords = 960;
 int upload_words(int32_t* dst, const int32_t* host_words, int n, void* stream);
+// int64 [write position | length | tail positions], n64 of them, then int32 [packed length | tail rows]
+int step_block(int32_t* block, int n64, int64_t seq, int64_t boundary, int sink, int tail, int packed, void* stream);
 
 // One new row of every request of a step into its ring history, slots and positions as arguments of the launch; `block`
 // (may be NULL) receives what later launches of the step read on the device: int64 slots[B], positions[B], lengths after

@@ -274,6 +274,25 @@ int upload_words(int32_t* dst, const int32_t* host_words, int n, void* stream) {
     return 0;
 }
 
+// The block of a one-request step: int64 write position, length and positions of the tail rows (the first `sink`, then those from
+// `boundary` on, `tail` in all, zeros behind them), int32 packed length and tail count.  The positions follow from four numbers: as a list
+// made on the host and sent as words they were 5 us of a step's 11 there (3.2 of them the launch, which takes as long on the GPU).
+__global__ void __launch_bounds__(256) step_block_kernel(int64_t* wide, int n64, int64_t seq, int64_t boundary, int sink, int tail, int packed) {
+    for (int i = threadIdx.x; i < n64; i += 256) {
+        const int t = i - 2;
+        wide[i] = i == 0 ? (seq > 0 ? seq - 1 : 0) : i == 1 ? seq : t >= tail ? 0 : t < sink ? t : boundary + (t - sink);
+    }
+    if (threadIdx.x < 2) reinterpret_cast<int32_t*>(wide + n64)[threadIdx.x] = threadIdx.x ? tail : packed;
+}
+
+int step_block(int32_t* block, int n64, int64_t seq, int64_t boundary, int sink, int tail, int packed, void* stream) {
+    if (n64 < 2 || tail < 0 || tail > n64 - 2) { set_error("step_block: bad shape"); return -1; }
+    hipLaunchKernelGGL(step_block_kernel, dim3(1), dim3(256), 0, static_cast<hipStream_t>(stream), reinterpret_cast<int64_t*>(block), n64,
+                       seq, boundary, sink, tail, packed);
+    if (hipGetLastError() != hipSuccess) { set_error("step_block: launch failed"); return -2; }
+    return 0;
+}
+
 // One workgroup per group of the list.
 constexpr int kPackPairs = kUploadWords / 2;
 __global__ void __launch_bounds__(128) pack_list_kernel(int32_t* src_rows, int32_t* dst_pages, int32_t* dst_groups,

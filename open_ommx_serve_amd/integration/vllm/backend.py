@@ -157,7 +157,7 @@ class OMMXCanonicalMetadataBuilder(_BuilderBase):
         st["batched_write"] = in_batched
         st["batched_read"] = bool(in_batched and uniform and B >= 1)
         if not in_batched and s.manager is not None and B == 1:
-            s.manager.on_build(common, new_request=st["full_prefill"])
+            s.manager.on_build(common, new_request=st["full_prefill"], shape=shape if shape.lengths is not None else None)
             if s.manager.dead:
                 raise RuntimeError("OMMX refuses to decode with stale KV metadata: "
                                    f"{s.manager.dead_reason}")
@@ -296,7 +296,7 @@ class OMMXCanonicalImpl(_ImplBase):
             mgr.register(id(layer), store)
             if mgr.cur_seq <= 0:                       # manager created after this step's build
                 mgr.on_build(s.last_common, new_request=False)
-            store.write_token(mgr.write_pos, key[0], value[0])
+            store.write_row(mgr.write_pos, key, value)
         else:
             raise RuntimeError("OMMX single-sequence route does not support chunked prefill")
 
@@ -484,7 +484,7 @@ class OMMXCanonicalImpl(_ImplBase):
         T = mgr.max_tail_cap
         # outside graph capture the split count may follow the actual length
         if self._reads_what_was_stored() and store.decode_into(
-                q[:1], out[:1], mgr.seq_dev, mgr.b_seq_len, sm_scale=self.scale,
+                q if q.shape[0] == 1 else q[:1], out if out.shape[0] == 1 else out[:1], mgr.seq_dev, mgr.b_seq_len, sm_scale=self.scale,
                 max_seq_len=mgr.max_seq_len if _STATE.graph else max(1, mgr.cur_packed)):
             _STATE.fires["single"] += 1
             return

@@ -170,6 +170,20 @@ def test_single_manager_buffers_follow_the_window_arithmetic():
     assert st.calls[-1] == "reset" and int(m.b_seq_len) == win.packed_len(77)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("kw", [{}, dict(sink_tokens=0), dict(sink_tokens=100, recent_window=64), dict(recent_window=1)])
+def test_single_manager_block_on_the_device_is_the_one_worked_out_here(kw):
+    """The launch that fills the block gives what the host's lists say, and a prompt's block is there for whoever asks."""
+    cfg = _cfg(**kw)
+    here, there = OMMXStepManager(cfg, "cpu"), OMMXStepManager(cfg, "cuda")
+    for seq in [1, 2, 7, 8, 9, 39, 40, 41, 71, 72, 73, 104, 105, 300, 511, 5]:
+        for new in (False, True):
+            for m in (here, there):
+                m.on_build(NS(seq_lens_cpu=[seq], query_start_loc_cpu=[0, seq if new else 1]), new_request=new)
+            for name in ("write_pos", "seq_dev", "tail_idx", "b_seq_len", "b_tail_len"):
+                assert torch.equal(getattr(there, name).cpu(), getattr(here, name)), (seq, new, name)
+
+
 def test_single_manager_records_why_it_died_and_strict_reraises():
     m = OMMXStepManager(_cfg(), "cpu")
     m.on_build(NS())
