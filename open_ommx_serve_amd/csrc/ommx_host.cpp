@@ -449,11 +449,17 @@ int run_decode(const DecodeCall& c) {
     // of 8 kv heads 14.0 us against 14.3, 12 K 17.6 against 15.8; 8 K with 64 q heads 16.6 / 19.8, 16 K 22.8 / 21.3; with 64 channels, whose
     // heads it does not read in pairs of which one is zero, 16 K 13.6 / 18.0, 2 x 12 K (six steps) 15.7 / 17.8; with one kv head, where a
     // workgroup of the other kernel is a single wave, 16 of 1 to 16 K (16 steps) 20.3 / 22.2, but 8 of 20 to 32 K 24.0 / 23.2.
+    // Several requests go a step further, their shares being dealt out either way: 3 of 1 to 3.4 K 14.0 / 12.3, 16 of 100 to 620 13.8 / 12.8, 2 x 5 K
+    // 15.6 / 14.7, 16 x 600 16.0 / 15.4 (the other kernel's time first), 6 of 200 to 1600 with 64 q heads 14.5 / 13.3.  Not where the
+    // workgroups of their tails crowd the ones of the shares: 24 of 40 to 400 13.2 / 13.7, 48 of 40 to 300 16.2 / 19.8, 8 x 1250
+    // with 64 q heads 18.3 / 19.6.  (At six and eight steps ragged batches still gain, 4 of 1 to 4 K 16.3 / 14.9, and equal ones lose, 24 of 1.0 to
+    // 1.4 K with 4 heads 17.1 / 18.7; how long they are beside the longest is not known here.)
     // (a range of groups without a tail, of which the caller merges the states, has the rounding of the whole then)
     const bool no_tail = !hist && !tail && !c.ws && !c.force;
     if (c.splits == 0 && (tail_rows || no_tail) && plain_planes && k == 6 && B <= 64 && (D == 128 || paired)) {
         const int64_t cus = cu_count(dev.index()), steps = (longest + 1) / 2, all = B * steps * wave_heads;
-        if (all <= cus * (paired || wave_heads == 1 ? 8 : 4)) {
+        const bool few = B > 1 && B * wave_heads * (R <= 4 ? 4 : 10) <= 2 * cus;
+        if (all <= cus * (paired || wave_heads == 1 ? 8 : few ? 5 : 4)) {
             // The merge inside the launch while its one workgroup has little to read, instead of a launch of its own (3.5 us of host
             // time; 1 K tokens 8.5 us against 9.1 to 10).  Not under capture: see TeamMerge.
             hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
