@@ -202,6 +202,7 @@ class MultiSeqKVPool:
         self._planes_cache: Optional[dict] = None
         self._host = _hip.host()
         self.step_rows = self._host.STEP_ROWS
+        self._step_how: Optional[tuple] = None
         # what every store launch of this pool is told (argument order of the native launchers)
         self._recipe = (self.k, self.gt, self.gc, self.outlier_repr, self.outlier_select, self.use_pow2,
                         self.kv_int8_scale, "i2")
@@ -394,12 +395,24 @@ class MultiSeqKVPool:
         w = self.window
         done = self._host.append_step(self.k_hist, self.v_hist, K, V, self._ring_sink, self._ring_rec, self.err_flag,
                                       self.seq_len, self.packed_groups, slots, seqs, w.sink_tokens + w.recent_window,
-                                      self.gt, None if self.kv_ring else self.max_seq_len, block)
+                                      self.gt, None if self.kv_ring else self.max_seq_len, block, self._step_store())
         if done is None:
             return None
-        if done[0]:
-            self._pack_completed(done[0])
-        return done[1], done[2]
+        full, longest, total, packed = done
+        if packed:
+            for r, _g0, g1 in full:
+                self.packed_groups[r] = g1
+        elif full:
+            self._pack_completed(full)
+        return longest, total
+
+    def _step_store(self) -> tuple:
+        """What the launch of a step's rows is told to pack completed groups along with them."""
+        how = self._step_how
+        if how is None:
+            how = self._step_how = (self._store_planes, self.ps, self.window.sink_tokens, self.G_per_seq,
+                                    store_table(self.k_hist.device), *self._recipe)
+        return how
 
     def append_decode_batched(self, slots: Sequence[int], K: torch.Tensor, V: torch.Tensor) -> int:
         """B new rows ``[B, H, D]`` in one launch, then one pack launch for every group that

@@ -633,6 +633,30 @@ int launch_store(const at::Tensor& K, const at::Tensor& V, int64_t row0, const P
         data<uint8_t>(p.oval), data<uint8_t>(p.v_main), data(p.v_scale), data<uint16_t>(p.v_zp), err, extras, stream);
 }
 
+// Groups of a pool's history (contiguous, [slots, rows, heads, head_dim]) as arguments of one store launch, where its kernel takes
+// them: 1 with nothing done otherwise.  Rows that turn around at most once.
+int launch_ring_groups(const at::Tensor& kh, const at::Tensor& vh, const std::vector<int64_t>& pairs, const Planes& p, const Recipe& r, int64_t ps,
+                       int64_t sink, int64_t span, int64_t wsink, int64_t per_seq, const at::Tensor& table, int32_t* err,
+                       const ommx::StepWrite* step, hipStream_t stream) {
+    const int64_t count = static_cast<int64_t>(pairs.size()) / 2, N = kh.size(0), rows = kh.size(1), H = kh.size(2), D = kh.size(3);
+    if (count > ommx::kRingGroups || N * rows > INT32_MAX || N * per_seq > INT32_MAX || (span != 0 && (wsink < sink || span < r.gt))) return 1;
+    ommx::RingGroups ring;
+    for (int64_t i = 0; i < count; ++i) {
+        const int64_t pos = wsink + pairs[2 * i + 1] * r.gt, slot = span > 0 ? sink + (pos - sink) % span : pos;
+        ring.of[i] = {static_cast<int32_t>(pairs[2 * i] * rows + slot), span > 0 ? static_cast<int32_t>(sink + span - slot) : INT32_MAX,
+                      static_cast<int32_t>(pairs[2 * i] * per_seq + pairs[2 * i + 1])};
+    }
+    ommx::StoreExtras extras;
+    extras.ring = &ring;
+    extras.ring_span = static_cast<int>(span);
+    extras.step = step;
+    return ommx::store_pack(
+        kh.data_ptr(), vh.data_ptr(), 0, H * D, D, H * D, D, nullptr, count * r.gt, H, D, ps, r.k, r.bitmap ? OMMX_INDEX_BITMAP : OMMX_INDEX_RELIDX7,
+        r.abs, r.mode, r.gt, r.gc, r.v_bf16, nullptr, nullptr, table.data_ptr<float>(), data<uint8_t>(p.k_base), data(p.k_scale),
+        data<uint16_t>(p.k_zp), data<uint16_t>(p.ms), data<uint16_t>(p.mc), data<uint8_t>(p.index), data<uint8_t>(p.oval),
+        data<uint8_t>(p.v_main), data(p.v_scale), data<uint16_t>(p.v_zp), err, extras, stream);
+}
+
 bool is_history(const at::Tensor& k, const at::Tensor& v) {
     return k.dim() == 4 && k.sizes() == v.sizes() && k.scalar_type() == at::kBFloat16 &&
            v.scalar_type() == at::kBFloat16 && k.is_contiguous() && v.is_contiguous() && k.is_cuda();
@@ -1061,27 +1085,15 @@ PyObject* py_pack_groups(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const c10::Device dev = kh->device();
     c10::hip::HIPGuard guard(dev.index());
     hipStream_t stream = stream_of(dev);
-    const at::Tensor K = kh->view({N * rows, kh->size(2), kh->size(3)}), V = vh->view({N * rows, kh->size(2), kh->size(3)});
-    int rc = 1;
-    // the groups as arguments of the store launch, where its kernel takes them: rows that turn around at most once
-    if (count <= ommx::kRingGroups && N * rows <= INT32_MAX && N * per_seq <= INT32_MAX && (span == 0 || (wsink >= sink && span >= r.gt))) {
-        ommx::RingGroups ring;
-        for (int64_t i = 0; i < count; ++i) {
-            const int64_t pos = wsink + pairs64[2 * i + 1] * r.gt, slot = span > 0 ? sink + (pos - sink) % span : pos;
-            ring.of[i] = {static_cast<int32_t>(pairs64[2 * i] * rows + slot), span > 0 ? static_cast<int32_t>(sink + span - slot) : INT32_MAX,
-                          static_cast<int32_t>(pairs64[2 * i] * per_seq + pairs64[2 * i + 1])};
-        }
-        ommx::StoreExtras extras;
-        extras.ring = &ring;
-        extras.ring_span = static_cast<int>(span);
-        Py_BEGIN_ALLOW_THREADS
-        rc = launch_store(K, V, 0, p, r, count * r.gt, ps, nullptr, nullptr, nullptr, *table, data<int32_t>(err), extras, stream);
-        Py_END_ALLOW_THREADS
-        if (rc != 1) {
-            if (failed(rc, "ommx_store_pack")) return nullptr;
-            Py_RETURN_TRUE;
-        }
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = launch_ring_groups(*kh, *vh, pairs64, p, r, ps, sink, span, wsink, per_seq, *table, data<int32_t>(err), nullptr, stream);
+    Py_END_ALLOW_THREADS
+    if (rc != 1) {
+        if (failed(rc, "ommx_store_pack")) return nullptr;
+        Py_RETURN_TRUE;
     }
+    const at::Tensor K = kh->view({N * rows, kh->size(2), kh->size(3)}), V = vh->view({N * rows, kh->size(2), kh->size(3)});
     // index tables: stream-ordered scratch, given back to torch's allocator when this call returns
     c10::DataPtr scratch = c10::GetAllocator(c10::DeviceType::CUDA)->allocate(count * (r.gt + ppg + 1) * sizeof(int32_t));
     int32_t *src = static_cast<int32_t*>(scratch.get()), *pages = src + count * r.gt, *groups = pages + count * ppg;
@@ -1365,11 +1377,12 @@ PyObject* py_append_rows(PyObject* self, PyObject* const* a, Py_ssize_t n) {
 }
 
 // (k_hist, v_hist, K, V, sink, span, err_flag, seq_len, packed_groups, slots, seqs, kept rows, group_tokens, capacity or None,
-// block or None): append_rows of up to kStepRows requests with slots and positions as arguments of the launch, which also
-// fills the int32 tensor block[7 B] (ommx::ring_step).  Returns (groups as append_rows, largest packed length, their
-// sum), or None with nothing done.
+// block or None, store): append_rows of up to kStepRows requests with slots and positions as arguments of the launch, which also
+// fills the int32 tensor block[7 B] (ommx::ring_step).  `store`: what pack_groups takes for this pool, (planes, page_size, window_sink,
+// groups_per_seq, table, recipe x 8); the groups that are complete with the step are packed by the same launch, where that takes both.
+// Returns (groups as append_rows, largest packed length, their sum, whether the groups are packed), or None with nothing done.
 PyObject* py_append_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
-    if (n != 15) { PyErr_SetString(PyExc_TypeError, "append_step: wrong number of arguments"); return nullptr; }
+    if (n != 16) { PyErr_SetString(PyExc_TypeError, "append_step: wrong number of arguments"); return nullptr; }
     bool ok = true;
     const at::Tensor *kh = as_tensor(a[0], ok), *vh = as_tensor(a[1], ok), *k = as_tensor(a[2], ok), *v = as_tensor(a[3], ok),
                      *err = as_tensor_or_none(a[6], ok), *block = as_tensor_or_none(a[14], ok);
@@ -1388,7 +1401,9 @@ PyObject* py_append_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
         v->scalar_type() != at::kBFloat16 || k->stride(2) != 1 || v->stride(2) != 1 || !on(k, dev) || !on(v, dev) ||
         !is_index(block, dev, at::kInt, 7 * B) || (block && reinterpret_cast<uintptr_t>(block->data_ptr()) % 8))
         Py_RETURN_NONE;
-    ommx::StepRows at_rows;
+    ommx::StepWrite write;
+    ommx::StepRows& at_rows = write.at;
+    std::vector<int64_t> pairs;
     int64_t longest = 0, sum = 0;
     for (int64_t i = 0; i < B; ++i) {
         const StepRow& s = step[i];
@@ -1399,19 +1414,57 @@ PyObject* py_append_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
         at_rows.packed[i] = static_cast<int32_t>(packed);
         longest = std::max(longest, packed);
         sum += packed;
+        for (int64_t g = s.done; g < packed / gt; ++g) { pairs.push_back(s.slot); pairs.push_back(g); }
     }
     c10::hip::HIPGuard guard(dev.index());
     hipStream_t stream = stream_of(dev);
-    int rc;
-    Py_BEGIN_ALLOW_THREADS
-    rc = ommx::ring_step(data<uint16_t>(k), data<uint16_t>(v), k->stride(0), k->stride(1), v->stride(0), v->stride(1),
-                         data<uint16_t>(kh), data<uint16_t>(vh), kh->stride(0), rows, B, H, D, sink, span, at_rows,
-                         data<int32_t>(block), data<int32_t>(err), stream);
-    Py_END_ALLOW_THREADS
-    if (failed(rc, "append_step")) return nullptr;
+    int rc = 1;
+    bool together = false;
+    if (!pairs.empty() && PyTuple_CheckExact(a[15]) && PyTuple_GET_SIZE(a[15]) == 13) {
+        PyObject* how[13];
+        for (int i = 0; i < 13; ++i) how[i] = PyTuple_GET_ITEM(a[15], i);
+        Recipe r;
+        Planes p;
+        const int64_t ps = as_int(how[1], ok), wsink = as_int(how[2], ok), per_seq = as_int(how[3], ok);
+        const at::Tensor* table = as_tensor(how[4], ok);
+        auto rows16 = [](const at::Tensor* t) {
+            return reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0 && t->stride(0) % 8 == 0 && t->stride(1) % 8 == 0;
+        };
+        bool fits = ok && read_recipe(how + 5, r) && read_planes(how[0], r, p) && r.gt == gt && ps >= 1 && gt % ps == 0 && (span == 0 || sink + span <= rows) &&
+                    rows16(k) && rows16(v) && rows16(kh) && rows16(vh) && !k->is_alias_of(*kh) && !k->is_alias_of(*vh) && !v->is_alias_of(*kh) && !v->is_alias_of(*vh);
+        // The workgroups of one launch run in any order: no group may hold the step's own token (a window without recent rows), nor a row whose place in
+        // the ring that token takes.
+        for (int64_t i = 0; i < B && fits; ++i) {
+            const int64_t pos = step[i].len - 1, first = wsink + step[i].done * gt, end = wsink + at_rows.packed[i];
+            if (step[i].done * gt >= at_rows.packed[i]) continue;
+            fits = step[i].done >= 0 && at_rows.packed[i] / gt <= per_seq && end <= pos && (span == 0 ? end <= rows : first + span > pos);
+        }
+        if (fits) {
+            write.k = data<uint16_t>(k); write.v = data<uint16_t>(v);
+            write.k_bs = k->stride(0); write.k_hs = k->stride(1); write.v_bs = v->stride(0); write.v_hs = v->stride(1);
+            write.k_hist = data<uint16_t>(kh); write.v_hist = data<uint16_t>(vh);
+            write.stride_req = kh->stride(0);
+            write.block = data<int32_t>(block); write.err = data<int32_t>(err);
+            write.B = static_cast<int>(B); write.H = static_cast<int>(H); write.rows = static_cast<int>(rows);
+            write.sink = static_cast<int>(sink); write.span = static_cast<int>(span);
+            Py_BEGIN_ALLOW_THREADS
+            rc = launch_ring_groups(*kh, *vh, pairs, p, r, ps, sink, span, wsink, per_seq, *table, data<int32_t>(err), &write, stream);
+            Py_END_ALLOW_THREADS
+            if (rc != 1 && failed(rc, "append_step")) return nullptr;
+            together = rc == 0;
+        }
+    }
+    if (!together) {
+        Py_BEGIN_ALLOW_THREADS
+        rc = ommx::ring_step(data<uint16_t>(k), data<uint16_t>(v), k->stride(0), k->stride(1), v->stride(0), v->stride(1),
+                             data<uint16_t>(kh), data<uint16_t>(vh), kh->stride(0), rows, B, H, D, sink, span, at_rows,
+                             data<int32_t>(block), data<int32_t>(err), stream);
+        Py_END_ALLOW_THREADS
+        if (failed(rc, "append_step")) return nullptr;
+    }
     PyObject* full = finish_step(a[7], step, kept, gt);
     if (!full) return nullptr;
-    return Py_BuildValue("(NLL)", full, static_cast<long long>(longest), static_cast<long long>(sum));
+    return Py_BuildValue("(NLLO)", full, static_cast<long long>(longest), static_cast<long long>(sum), together ? Py_True : Py_False);
 }
 
 // (table, B): column 0 of the first B rows of a 2-D table of int32 or int64 in host memory as a list; None for anything else.

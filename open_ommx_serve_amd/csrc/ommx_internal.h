@@ -34,11 +34,27 @@ struct RingGroup { int32_t row, turn, group; };
 constexpr int kRingGroups = 96;
 struct RingGroups { RingGroup of[kRingGroups]; };
 
+// The new rows of a decode step (ring_step below): pool slots, positions and packed lengths of its requests.
+constexpr int kStepRows = 64;
+struct StepRows { int32_t slot[kStepRows], pos[kStepRows], packed[kStepRows]; };
+// The same rows written by the store launch that packs the groups complete with them: rows of K and V, histories [slots, rows, H, D],
+// all 16 bytes at a time.  None of the groups reads a row that the step writes.
+struct StepWrite {
+    const uint16_t *k, *v;
+    int64_t k_bs, k_hs, v_bs, v_hs;
+    uint16_t *k_hist, *v_hist;
+    int64_t stride_req;
+    int32_t *block, *err;
+    int B, H, rows, sink, span;
+    StepRows at;
+};
+
 // What a store launch of the native launchers does besides packing.
 struct StoreExtras {
     bool err_words = false;               // err_flag is an array of OMMX_STORE_ERR_WORDS host-visible ints, one per error bit
     int32_t *own_pages = nullptr, *own_groups = nullptr;      // identity tables [T / page_size], [T / group_tokens] to
                                                               // fill (both or neither)
+    const StepWrite* step = nullptr;      // with `ring`: rows to write beside them
     const RingGroups* ring = nullptr;     // where the groups lie; T / 32 of them, span rows in the ring.  store_pack returns 1,
     int ring_span = 0;                    // with nothing launched, for a recipe or a number of groups that needs the tables
     const BlockRows* rows = nullptr;      // bf16 rows to copy into the history (head_dim a multiple of 8, every slot inside it),
@@ -87,8 +103,6 @@ int step_block(int32_t* block, int n64, int64_t seq, int64_t boundary, int sink,
 // One new row of every request of a step into its ring history, slots and positions as arguments of the launch; `block`
 // (may be NULL) receives what later launches of the step read on the device: int64 slots[B], positions[B], lengths after
 // the step[B], then int32 packed lengths[B].
-constexpr int kStepRows = 64;
-struct StepRows { int32_t slot[kStepRows], pos[kStepRows], packed[kStepRows]; };
 int ring_step(const uint16_t* k, const uint16_t* v, int64_t k_bs, int64_t k_hs, int64_t v_bs, int64_t v_hs, uint16_t* k_hist,
               uint16_t* v_hist, int64_t stride_req, int rows, int B, int H, int D, int sink, int span, const StepRows& step,
               int32_t* block, int32_t* err, void* stream);

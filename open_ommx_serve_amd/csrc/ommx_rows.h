@@ -43,4 +43,31 @@ __device__ __forceinline__ void copy_block_row(const BlockRows& a, int n) {
     }
 }
 
+// Row b of a step to its place, and the step's numbers of request b to the block that its other launches read, as ring_step_kernel
+// (ommx_ring.hip) does.
+template <int D>
+__device__ __forceinline__ void copy_step_row(const StepWrite& s, int b) {
+    const int p = s.at.pos[b], slot = s.at.slot[b], B = s.B;
+    if (s.block && threadIdx.x == 0) {
+        int64_t* const wide = reinterpret_cast<int64_t*>(s.block);
+        wide[b] = slot;
+        wide[B + b] = p;
+        wide[2 * B + b] = p + 1LL;
+        s.block[6 * B + b] = s.at.packed[b];
+    }
+    const int64_t row = ring_slot(p, s.sink, s.span);
+    if (row < 0 || row >= s.rows) {
+        if (s.err && threadIdx.x == 0) atomicOr(s.err, OMMX_ERR_RING_RANGE);
+        return;
+    }
+    const int64_t to = slot * s.stride_req + row * static_cast<int64_t>(s.H * D);
+    for (int i = threadIdx.x; i < s.H * (D / 8); i += blockDim.x) {
+        const int h = i / (D / 8), c = 8 * (i % (D / 8));
+        const uint4 x = *reinterpret_cast<const uint4*>(s.k + b * s.k_bs + h * s.k_hs + c);
+        const uint4 y = *reinterpret_cast<const uint4*>(s.v + b * s.v_bs + h * s.v_hs + c);
+        *reinterpret_cast<uint4*>(s.k_hist + to + h * D + c) = x;
+        *reinterpret_cast<uint4*>(s.v_hist + to + h * D + c) = y;
+    }
+}
+
 }  // namespace ommx

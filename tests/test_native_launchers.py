@@ -405,3 +405,47 @@ def test_the_one_call_of_a_block_gives_what_the_steps_give(kw, dtype):
         for device in ("cuda", "cuda:0"):
             with pytest.raises(ValueError, match="V pack: non-finite"):
                 ommx_pack_kv_canonical_block(K, V, device=device, **call)
+
+
+@pytest.mark.parametrize("ring,B,H,win,repr_,form", [
+    (False, 1, 1, {}, "bitmap", "plain"), (True, 1, 8, {}, "bitmap", "plain"), (False, 5, 8, {}, "relidx7", "view"), (True, 64, 2, {}, "bitmap", "plain"),
+    (False, 64, 1, {}, "relidx7", "plain"), (True, 3, 2, {}, "relidx7", "odd"), (False, 4, 2, dict(recent_window=0), "bitmap", "plain"),
+    (False, 4, 2, dict(sink_tokens=0, recent_window=1), "bitmap", "plain"), (True, 4, 2, dict(recent_window=1), "bitmap", "plain")])
+def test_a_step_whose_rows_go_with_its_groups(ring, B, H, win, repr_, form, monkeypatch):
+    """Steps that complete groups, rows and groups in one launch where that takes both, against rows first and groups behind them: histories,
+    planes, cursors and the step's block are the same bits, step after step.  Not in one launch: a group that ends with the step's own token (no recent
+    rows), rows that cannot be read 16 bytes at a time."""
+    D, w = 128, WindowSpec(**win)
+    pools = [MultiSeqKVPool(D, H, B + 2, 330, window=w, device=DEV, kv_ring=ring, outliers_per_vector=6, outlier_repr=repr_, use_pow2=True) for _ in range(2)]
+    slots = [(3 * i + 1) % (B + 2) if (B + 2) % 3 else i for i in range(B)]
+    lens = [35 + 11 * (i % 17) for i in range(B)]
+    for i, (r, n) in enumerate(zip(slots, lens)):
+        K, V = _block(n, H, D, torch.bfloat16, 10 + i), _block(n, H, D, torch.bfloat16, 200 + i)
+        for p in pools:
+            p.append_block(r, K, V)
+    blocks = [torch.full((7 * B,), -1, dtype=torch.int32, device=DEV) for _ in pools]
+    pools[1]._step_how = ()                                     # (nothing to pack with: a launch for the rows)
+    groups_behind = []
+    behind = pools[0]._pack_completed
+    monkeypatch.setattr(pools[0], "_pack_completed", lambda full: groups_behind.append(full) or behind(full))
+    completed = 0
+    for s in range(1, 71):
+        K, V = _block(B, H, D, torch.bfloat16, 30 + s), _block(B, H, D, torch.bfloat16, 140 + s)
+        if form == "view":
+            both = torch.stack([K, V], 2)
+            K, V = both[:, :, 0], both[:, :, 1]
+        elif form == "odd":
+            K = torch.cat([K.flatten(), K.new_zeros(1)])[1:].view(B, H, D)
+        seqs = [n + s for n in lens]
+        was = list(pools[0].packed_groups)
+        got = [p.append_step_rows(slots, seqs, K, V, t if s % 3 else None) for p, t in zip(pools, blocks)]
+        assert got[0] == got[1] and got[0] is not None
+        completed += pools[0].packed_groups != was
+        assert pools[0].seq_len == pools[1].seq_len and pools[0].packed_groups == pools[1].packed_groups
+        assert pools[0].packed_groups[slots[0]] == w.num_groups(seqs[0])
+        for a, b in zip([*pools[0]._store_planes.values(), pools[0].k_hist, pools[0].v_hist, blocks[0]],
+                        [*pools[1]._store_planes.values(), pools[1].k_hist, pools[1].v_hist, blocks[1]]):
+            assert a is b is None or torch.equal(a.view(torch.uint8), b.view(torch.uint8)), s
+    assert completed >= 2 and len(groups_behind) == (completed if form == "odd" or win.get("recent_window") == 0 else 0)
+    for p in pools:
+        p.check_errors()
