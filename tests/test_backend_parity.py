@@ -156,6 +156,53 @@ def test_unservable_steps_raise():
     BK.reset_worker_state()
 
 
+def test_single_graph_route_replays_across_requests():
+    """One captured step of the single-request route: replayed for the request it was captured in, for one that starts with a single
+    token (the shape of a decode step, so nothing but the replay runs) and for one behind a prompt."""
+    eng = _Engine(600, graph=True, batched=False, batched_graph=False)
+    key = [torch.zeros(1, HKV, D, dtype=torch.bfloat16, device=DEV) for _ in range(LAYERS)]
+    val = [torch.zeros_like(k) for k in key]
+    qry = torch.zeros(1, HQ, D, dtype=torch.bfloat16, device=DEV)
+    out = [torch.zeros(1, HQ, D, dtype=torch.float32, device=DEV) for _ in range(LAYERS)]
+
+    def forward_all():
+        for l, (layer, impl) in enumerate(zip(eng.layers, eng.impls)):
+            impl.do_kv_cache_update(layer, key[l], val[l], None, None)
+            impl.forward(layer, qry, key[l], val[l], None, None, out[l])
+
+    graph = None
+    for r, steps in ((_Request(1, 300, 320, 21), 12), (_Request(2, 1, 90, 22), 90), (_Request(3, 40, 80, 23), 36)):
+        if r.prompt > 1:
+            eng.step([r], check=False)
+            if graph is None:
+                eng.step([r], check=False)                  # an eager step allocates every workspace
+        for s in range(steps):
+            md = NS(seq_lens_cpu=[r.seq + 1], query_start_loc_cpu=[0, 1], block_table_tensor=torch.tensor([[r.key, r.key + 1]]))
+            eng.builder.build(0, md)
+            for l in range(LAYERS):
+                key[l].copy_(r.K[l][r.seq:r.seq + 1])
+                val[l].copy_(r.V[l][r.seq:r.seq + 1])
+            qry.copy_(r.q[r.seq:r.seq + 1])
+            if graph is None:
+                stream = torch.cuda.Stream()
+                stream.wait_stream(torch.cuda.current_stream())
+                graph = torch.cuda.CUDAGraph()
+                with torch.cuda.stream(stream):
+                    with torch.cuda.graph(graph, stream=stream):
+                        forward_all()
+                torch.cuda.current_stream().wait_stream(stream)
+            graph.replay()
+            torch.cuda.synchronize()
+            r.seq += 1
+            if s % 6 == 0 or s == steps - 1:
+                for l in range(LAYERS):
+                    want, _ = _oracle_decode(r.q[r.seq - 1:r.seq], [r.K[l][:r.seq]], [r.V[l][:r.seq]], eng.win, SCALE)
+                    err = (out[l].cpu()[0].double() - want[0]).abs()
+                    assert err.max().item() <= MAX_ABS and err.mean().item() <= MEAN_ABS, (r.key, s, l)
+    assert not eng.state.manager.dead
+    BK.reset_worker_state()
+
+
 def test_batched_graph_route_replays_from_a_hip_graph():
     """The launch-only write + read of every layer captured once and replayed for 40 steps; the
     host seam (slots, packing, the one control-block upload) runs between replays, and the row

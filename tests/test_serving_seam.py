@@ -170,18 +170,38 @@ def test_single_manager_buffers_follow_the_window_arithmetic():
     assert st.calls[-1] == "reset" and int(m.b_seq_len) == win.packed_len(77)
 
 
+BLOCK = ("write_pos", "seq_dev", "tail_idx", "b_seq_len", "b_tail_len")
+
+
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+def test_every_build_brings_the_fixed_addresses_up_to_date(device):
+    """A replayed step reads the block where it lay at capture and asks nobody: tensors taken once hold the numbers of the last
+    build, whether that one went on with a request or started one, by a prompt or by a single token."""
+    cfg = _cfg()
+    win, m = cfg.window(), OMMXStepManager(cfg, device)
+    held = {name: getattr(m, name) for name in BLOCK}
+    for seq, queries in [(300, 1), (301, 1), (302, 1), (1, 1), (2, 1), (450, 450), (451, 1), (7, 7), (1, 1)]:
+        m.on_build(NS(seq_lens_cpu=[seq], query_start_loc_cpu=[0, queries]))
+        tail = win.tail_indices(seq)
+        got = {name: t.tolist() for name, t in held.items()}
+        want = dict(write_pos=[seq - 1], seq_dev=[seq], tail_idx=tail + [0] * (m.max_tail_len - len(tail)),
+                    b_seq_len=[win.packed_len(seq)], b_tail_len=[len(tail)])
+        assert got == want, (seq, queries)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("kw", [{}, dict(sink_tokens=0), dict(sink_tokens=100, recent_window=64), dict(recent_window=1)])
 def test_single_manager_block_on_the_device_is_the_one_worked_out_here(kw):
-    """The launch that fills the block gives what the host's lists say, and a prompt's block is there for whoever asks."""
+    """The launch that fills the block gives what the host's lists say, a prompt's as well."""
     cfg = _cfg(**kw)
     here, there = OMMXStepManager(cfg, "cpu"), OMMXStepManager(cfg, "cuda")
+    held = [(name, getattr(here, name), getattr(there, name)) for name in BLOCK]
     for seq in [1, 2, 7, 8, 9, 39, 40, 41, 71, 72, 73, 104, 105, 300, 511, 5]:
         for new in (False, True):
             for m in (here, there):
                 m.on_build(NS(seq_lens_cpu=[seq], query_start_loc_cpu=[0, seq if new else 1]), new_request=new)
-            for name in ("write_pos", "seq_dev", "tail_idx", "b_seq_len", "b_tail_len"):
-                assert torch.equal(getattr(there, name).cpu(), getattr(here, name)), (seq, new, name)
+            for name, a, b in held:
+                assert torch.equal(b.cpu(), a), (seq, new, name)
 
 
 def test_single_manager_records_why_it_died_and_strict_reraises():
