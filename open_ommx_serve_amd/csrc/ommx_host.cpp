@@ -96,16 +96,20 @@ void written(const at::Tensor& t) {
     if (!t.is_inference()) t.unsafeGetTensorImpl()->bump_version();
 }
 
-// Whether the memory that two tensors span has bytes in common (strides are never negative).
-bool share_memory(const at::Tensor& a, const at::Tensor& b) {
-    auto end = [](const at::Tensor& t) {
+// The memory that a tensor spans (strides are never negative), empty without elements.
+struct Span {
+    const char *begin = nullptr, *end = nullptr;
+    explicit Span(const at::Tensor& t) {
+        if (t.numel() == 0) return;
         int64_t last = 0;
         for (int64_t d = 0; d < t.dim(); ++d) last += (t.size(d) - 1) * t.stride(d);
-        return static_cast<const char*>(t.data_ptr()) + (last + 1) * static_cast<int64_t>(t.element_size());
-    };
-    if (a.numel() == 0 || b.numel() == 0) return false;
-    return static_cast<const char*>(a.data_ptr()) < end(b) && static_cast<const char*>(b.data_ptr()) < end(a);
-}
+        begin = static_cast<const char*>(t.data_ptr());
+        end = begin + (last + 1) * static_cast<int64_t>(t.element_size());
+    }
+    bool meets(const Span& o) const { return begin < o.end && o.begin < end; }
+};
+// Whether the memory that two tensors span has bytes in common.
+bool share_memory(const at::Tensor& a, const at::Tensor& b) { return Span(a).meets(Span(b)); }
 
 bool failed(int rc, const char* what) {
     if (rc == 0) return false;
@@ -464,7 +468,20 @@ int run_decode(const DecodeCall& c) {
             // time; 1 K tokens 8.5 us against 9.1 to 10).  Not under capture: see TeamMerge.
             hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
             const bool eager = hipStreamIsCapturing(stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone;
-            auto merged = [&](int64_t states) { return eager && states <= ommx::kTeamMerged && states * (Hq / wave_heads) * D <= ommx::kTeamMerged * 512; };
+            // Nor where a result lies in what the call reads: the last workgroup of one head writes it while those of others still read.
+            auto apart = [&] {
+                const Span o(*c.o), lse = c.lse ? Span(*c.lse) : o;
+                for (const at::Tensor* t : {c.q, c.k_base, c.k_scale, c.k_zp, c.k_index, c.k_oval, c.v_main, c.v_scale, c.v_zp, c.ms, c.mc, c.k_tail,
+                                            c.v_tail, c.b_tail, c.hist_seq, c.hist_slots, c.rt, c.rg, c.seq}) {
+                    if (!t) continue;
+                    const Span in(*t);
+                    if (in.meets(o) || in.meets(lse)) return false;
+                }
+                return true;
+            };
+            auto merged = [&](int64_t states) {
+                return eager && states <= ommx::kTeamMerged && states * (Hq / wave_heads) * D <= ommx::kTeamMerged * 512 && apart();
+            };
             // one request: up to three workgroups a compute unit (two with 8 heads); several: two, or a split a step where all of those fit
             const int64_t room = std::clamp<int64_t>((B == 1 && R <= 4 ? 3 : 2) * cus / wave_heads, 1, 508);
             if (B == 1 || B * steps <= room) {

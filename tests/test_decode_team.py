@@ -130,6 +130,47 @@ def test_captured_calls_replay_like_eager_ones():
             assert torch.equal(a[0], wo)
 
 
+@pytest.mark.parametrize("where", ["o in q", "lse in q", "o in the tail rows", "o in a plane", "o around q"])
+@pytest.mark.parametrize("lens,hq,hkv,D", [([1000], 32, 8, 128), ([300, 90, 500], 64, 8, 128), ([700, 330], 8, 4, 64)])
+def test_results_that_lie_in_what_the_call_reads(where, lens, hq, hkv, D):
+    """The merge is a launch of its own then, behind everything that reads: on the bits of one under capture, which the merge
+    inside the launch (sums in another order) does not have."""
+    case = build_decode_case(lens, q_heads=hq, kv_heads=hkv, head_dim=D, seed=10, permute_tables=True, sparse_frac=0.005)
+    apart, outs = _run(case), _outputs(case)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        ommx_paged_decode_attention_canonical(*case.decode_args(*outs), **case.decode_kwargs())
+    graph.replay()
+    want = [t.cpu() for t in outs]
+    assert not torch.equal(apart[0], want[0])
+    B = len(lens)
+    o, lse = _outputs(case)
+    floats = torch.zeros(4 * B * hq * D, device="cuda")
+    if where == "o around q":                            # rows of one buffer, each head's q behind its result
+        rows = floats[:B * hq * 2 * D].view(B, hq, 2, D)
+        o, q = rows[:, :, 0], rows[:, :, 1].view(torch.bfloat16)[..., :D]
+        case.q = q.copy_(case.q)
+    elif where in ("o in q", "lse in q"):
+        q = floats[:B * hq * D].view(torch.bfloat16)[:B * hq * D].view(B, hq, D)
+        if where == "o in q":
+            o = floats[:B * hq * D].view(B, hq, D)
+        else:
+            lse = floats[:B * hq].view(B, hq)
+        case.q = q.copy_(case.q)
+    else:
+        name = "k_tail" if where == "o in the tail rows" else "k_base"
+        source = case.k_tail if name == "k_tail" else case.planes[name]
+        assert source.nbytes >= o.nbytes
+        held = source.clone()
+        o = held.view(-1).view(torch.float32)[:o.numel()].view(B, hq, D)
+        if name == "k_tail":
+            case.k_tail = held
+        else:
+            case.planes[name] = held
+    ommx_paged_decode_attention_canonical(*case.decode_args(o, lse), **case.decode_kwargs())
+    assert torch.equal(o.cpu(), want[0]) and torch.equal(lse.cpu(), want[1])
+
+
 def test_two_streams_at_once():
     """Calls under way together have scratch of their own."""
     cases = [build_decode_case(l, seed=8, permute_tables=True) for l in ([1000], [400, 90, 600])]
