@@ -95,7 +95,7 @@ def test_tables_are_not_read_past_their_rows():
 
 @pytest.mark.parametrize("hq,hkv,D", [(32, 8, 128), (64, 8, 128), (32, 8, 64)])
 def test_the_same_bits_again_in_memory_of_other_calls(hq, hkv, D):
-    """The merge counts in scratch that holds whatever calls before left there, of this shape or another; bits stay."""
+    """Calls of several shapes one behind another, in scratch that calls before or other tensors had; bits stay."""
     cases = [build_decode_case(l, q_heads=hq, kv_heads=hkv, head_dim=D, seed=5, permute_tables=True, sparse_frac=0.005)
              for l in ([1000], [300, 90, 500], [72], [9], [100 + 40 * i for i in range(8)])]
     first = [_run(c) for c in cases]
@@ -107,6 +107,80 @@ def test_the_same_bits_again_in_memory_of_other_calls(hq, hkv, D):
         for i in ((turn * 7 + k) % len(cases) for k in range(len(cases))):
             o, lse = _run(cases[i])
             assert torch.equal(o, first[i][0]) and torch.equal(lse, first[i][1]), (turn, i)
+
+
+@pytest.mark.parametrize("lens,mib", [([1000], 1), ([300, 90, 500], 1), ([97 + 86 * i for i in range(8)], 4)])
+def test_the_merge_counts_over_whatever_its_scratch_holds(lens, mib):
+    """A pool of its own holds one free block, so a call's scratch is cut from its front: filled beforehand with zeros, ones, words
+    above the call's number, which have to come down to it, and words of an earlier call.  Read back, the counts lie there, a word on
+    a line of 64 bytes for each request and kv head, all under one number, the lines' other words as they were filled."""
+    case = build_decode_case(lens, q_heads=32, kv_heads=8, head_dim=128, seed=5, permute_tables=True, sparse_frac=0.005)
+    want = _run(case)
+    pool, number = torch.cuda.MemPool(), 0
+    for left in ("zeros", "ones", "just above", "far above", "an earlier call's"):
+        fill = {"zeros": 0, "ones": 2 ** 64 - 1, "just above": (number + 2) << 8 | 3, "far above": (number + 2 ** 20) << 8 | 17,
+                "an earlier call's": number << 8 | 255}[left]
+        o, lse = _outputs(case)
+        with torch.cuda.use_mem_pool(pool):
+            block = torch.empty(mib << 17, dtype=torch.int64, device="cuda")
+            at = block.data_ptr()
+            block.fill_(fill - 2 ** 64 if fill >= 2 ** 63 else fill)
+            del block
+            ommx_paged_decode_attention_canonical(*case.decode_args(o, lse), **case.decode_kwargs())
+            block = torch.empty(mib << 17, dtype=torch.int64, device="cuda")
+        assert block.data_ptr() == at, left
+        lines = block.cpu().numpy().view("uint64").reshape(-1, 8)
+        first = lines[:, 0]
+        # (a call's number has 0xFF and zeros on top: no state or lse looks like it)
+        found = first[(lines[:, 1:] == fill).all(1) & (first != fill) & (first >> 48 >= 0xFF00) & (first >> 48 < 0xFF80)]
+        assert len(found) == len(lens) * 8 and len(set(found.tolist())) <= len(lens), left
+        numbers = set((found >> 8).tolist())
+        assert len(numbers) == 1 and min(numbers) > number, left
+        number = int(min(numbers))
+        assert torch.equal(o.cpu(), want[0]) and torch.equal(lse.cpu(), want[1]), left
+        del block
+
+
+OPTIONS = [(32, 8, 128, {}), (64, 8, 128, dict(outlier_repr="relidx7")), (32, 8, 64, {}), (64, 8, 128, dict(kv_outlier_map=False))]
+
+
+@pytest.mark.parametrize("hq,hkv,D,kw", OPTIONS)
+@pytest.mark.parametrize("lens", [[1000], [900, 40, 330]], ids=lambda l: f"{len(l)}x{max(l)}")
+def test_caps_large_queries_and_large_steps(hq, hkv, D, kw, lens):
+    """Options that take a branch of their own: a cap, query elements of several hundred in some waves' channels (the bounds of the same
+    test of the one-wave kernel), steps beyond the f16 operands, held and reported."""
+    def case_of(**over):
+        return build_decode_case(lens, q_heads=hq, kv_heads=hkv, head_dim=D, seed=31, permute_tables=True,
+                                 **{"sparse_frac": 0.005, **kw, **over})
+    case = case_of()
+    err = torch.zeros(1, dtype=torch.int32, device="cuda")
+    plain = _run(case, logit_cap=4.0, _force_reference_kernel=True)
+    assert not torch.allclose(plain[0], _run(case, _force_reference_kernel=True)[0], atol=1e-2)
+    _close(_run(case, logit_cap=4.0, err_flag=err), (plain[0], plain[1]), "cap")
+    q = case.q.float().cpu()
+    where = torch.randperm(q.numel(), generator=torch.Generator().manual_seed(7))[:20]
+    q.view(-1)[where] = torch.tensor([300.0, -512.0, 1000.0, -776.0, 256.0] * 4)
+    case.q.copy_(q.to(case.q.dtype))
+    want = _oracle(case)
+    (o, lse), (wo, wl) = _run(case, err_flag=err), want
+    d = (o.double() - wo).abs()
+    assert d.max().item() <= 2e-3 and d.mean().item() <= 2e-4, d.max().item()
+    assert ((lse.double() - wl).abs() <= 2e-3 + 1e-5 * wl.abs()).all()
+    assert int(err.item()) == 0
+    case = case_of(sparse_frac=0.02, sparse_gain=40.0, outlier_gain=150.0)
+    exps = case.planes["k_scale"].to(torch.int32)
+    assert int((exps >= 6).sum()) > 50 and int(exps.max()) <= 15
+    (o, lse), (wo, wl) = _run(case, err_flag=err), _oracle(case)
+    d = (o.double() - wo).abs()
+    assert d.max().item() <= 2e-3 and d.mean().item() <= 2e-4, d.max().item()
+    assert ((lse.double() - wl).abs() <= 2e-3 + 2e-6 * wl.abs()).all()
+    assert int(err.item()) == 0
+    for name in ("k_scale", "v_scale"):
+        case = case_of()
+        case.planes[name].view(-1)[5::97] = 17
+        err.zero_()
+        o, _ = _run(case, err_flag=err)
+        assert torch.isfinite(o).all() and int(err.item()) & _hip.ERR_VALUE_RANGE, name
 
 
 def test_captured_calls_replay_like_eager_ones():
