@@ -15,7 +15,8 @@
 // of 8 heads, one step each) the walk takes 4 us -- arguments 0.6, length and tables together 0.5, rows 0.7, the step 1.6, the state 0.4 --,
 // hand-over and merge 2.7.  Whole call, one wave a head and a merge of its own -> this: 1 K tokens 9.5 -> 8.2 us, 3 requests of 0.7 to
 // 9 K with one kv head 12.1 -> 9.9, 2 x 12 K of 64 channels 18.3 -> 15.9, 6 K 13.9 -> 11.9, 8 K with 64 q heads 19.8 -> 16.6; a batch of
-// eight served token by token 1.70 -> 1.42 ms for 80 steps of a layer.  38 to 50 KB of LDS a workgroup.
+// eight served token by token 1.70 -> 1.42 ms for 80 steps of a layer.  38 to 53 KB of LDS a workgroup.
+// (walk repeats the channel pass, QK, softmax and P.V of ommx_decode_gqa4_walk.h for 32 channels: a correction there is one here too.)
 #include <type_traits>
 
 #include "ommx_decode_recipe.h"
@@ -59,7 +60,7 @@ struct TeamLds {
     static constexpr int OFF_VS = OFF_VZ + PT_ROW * 2;              // [PT_ROW] f16 2^e_v
     static constexpr int OFF_TILE = OFF_VS + PT_ROW * 2;            // [2][TILE_GROUP][TILE_ROW] f16 outlier entries
     static constexpr int LDS_WAVE = OFF_TILE + 2 * TILE_GROUP * TILE_ROW;
-    static constexpr int BYTES = OFF_WAVES + WAVES * LDS_WAVE;      // 38272 (4 heads) / 48768 (8)
+    static constexpr int BYTES = OFF_WAVES + WAVES * LDS_WAVE;      // 38272 (4 heads) / 48768 (8), FINE 40576 / 53376
     static_assert(OFF_PT % 16 == 0 && OFF_VZ % 16 == 0 && OFF_TILE % 16 == 0 && LDS_WAVE % 16 == 0, "b128 alignment");
     static_assert(LDS_WAVE >= (32 * NH + 2 * NH) * 4, "the tail rows' share of it");
 };
